@@ -4,6 +4,7 @@
 #include "cq_launch.h"
 #include "../../include/candle_hip_nn.h"
 
+#include <algorithm>
 #include <mutex>
 
 // Workspace of cq_qmatmul_forward_static: device memory that belongs to the library's code object, so the entry point
@@ -179,8 +180,8 @@ int cq_matmul(int w_dtype, const void *w_dev, const void *act_scratch_dev, float
     return cq_matmul_launch(w_dtype, w_dev, act_scratch_dev, dst_dev, k, n, rows, stride_dst, (hipStream_t)stream);
 }
 
-int64_t cq_qmatmul_workspace_bytes(int w_dtype, int64_t m, int64_t k, int64_t n) {
-    if (check_mm_shape(w_dtype, k, n, m)) return -1;
+// What a call cannot do without.
+static int64_t workspace_least(int w_dtype, int64_t m, int64_t k, int64_t n) {
     int64_t bytes = cq_act_layout(w_dtype, k, m).total;
     // the batched matvec lays the rows out as matrix operands, 16 row slots whatever the batch
     const int64_t batch_ws = cq_matvec_batch_workspace(w_dtype, k, m);
@@ -197,6 +198,32 @@ int64_t cq_qmatmul_workspace_bytes(int w_dtype, int64_t m, int64_t k, int64_t n)
     return bytes;
 }
 
+// The kernels of cq_qtile.h write f16 / bf16 themselves but can use more planes: as many as the static workspace has room for, if the call fits
+// into that without them.
+int64_t cq_qmatmul_workspace_bytes(int w_dtype, int64_t m, int64_t k, int64_t n) {
+    if (check_mm_shape(w_dtype, k, n, m)) return -1;
+    const int64_t least = workspace_least(w_dtype, m, k, n);
+    if (m <= CQ_MATVEC_MAX_ROWS && !cq_use_mfma(w_dtype, m, k)) return least;
+    const int64_t planes = cq_act_layout(w_dtype, k, m).total + cq_qtile_plane_bytes(w_dtype, k, n, m);
+    return std::max(least, least <= CQ_STATIC_WORKSPACE_BYTES ? std::min<int64_t>(planes, CQ_STATIC_WORKSPACE_BYTES) : planes);
+}
+
+// The matrix-core product of m rows that the workspace holds quantized; what lies behind them is free.
+static int forward_quantized(int w_dtype, const void *w_dev, void *dst_dev, int dst_dtype, int64_t m, int64_t k, int64_t n, void *workspace_dev,
+                             int64_t workspace_bytes, hipStream_t s) {
+    const int64_t act = cq_act_layout(w_dtype, k, m).total;
+    float *tmp = (float *)((uint8_t *)workspace_dev + act);
+    if (cq_use_mfma(w_dtype, m, k) && cq_qtile_takes(w_dtype, w_dev, k, n)) {
+        // the split is one of the shape alone, whatever else the caller has to spare: the results of all entry points are the same bits
+        const int64_t room = std::min(workspace_bytes, cq_qmatmul_workspace_bytes(w_dtype, m, k, n)) - act;
+        return cq_qtile_launch(w_dtype, w_dev, cq_act_view(workspace_dev, w_dtype, k, m), dst_dev, dst_dtype, k, n, m, n, tmp, room, s);
+    }
+    float *split_ws = cq_qmm_splits(k, n, m) > 1 ? (float *)((uint8_t *)tmp + cq_align256(m * n * 4)) : nullptr;
+    if (dst_dtype == CQ_F32) return cq_matmul_launch(w_dtype, w_dev, workspace_dev, (float *)dst_dev, k, n, m, n, s, split_ws);
+    int rc = cq_matmul_launch(w_dtype, w_dev, workspace_dev, tmp, k, n, m, n, s, split_ws);
+    return rc ? rc : cq_convert_f32_launch(tmp, dst_dev, dst_dtype, m * n, s);
+}
+
 int cq_qmatmul_forward(int w_dtype, const void *w_dev, const void *x_dev, int x_dtype, void *dst_dev, int dst_dtype,
                        int64_t m, int64_t k, int64_t n, void *workspace_dev, int64_t workspace_bytes, void *stream) {
     int rc = check_mm_shape(w_dtype, k, n, m);
@@ -206,7 +233,7 @@ int cq_qmatmul_forward(int w_dtype, const void *w_dev, const void *x_dev, int x_
     if ((rc = check_weight_ptr(w_dtype, w_dev))) return rc;
     if (!x_dev || !dst_dev || !workspace_dev) return CQ_ERR_NULL;
     if (!aligned(x_dev, 16) || !aligned(workspace_dev, 256) || !aligned(dst_dev, float_size(dst_dtype))) return CQ_ERR_ALIGN;
-    if (workspace_bytes < cq_qmatmul_workspace_bytes(w_dtype, m, k, n)) return CQ_ERR_WORKSPACE;
+    if (workspace_bytes < workspace_least(w_dtype, m, k, n)) return CQ_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     // decode: one kernel quantizes the activations into LDS and streams W (no scratch traffic)
     // (Q4_1, Q5_0, Q5_1, Q2K, Q3K have the fused instance for f32 activations only)
@@ -225,12 +252,7 @@ int cq_qmatmul_forward(int w_dtype, const void *w_dev, const void *x_dev, int x_
         return cq_matvec_launch(w_dtype, w_dev, workspace_dev, dst_dev, dst_dtype, k, n, m, n, s);
     }
     if ((rc = cq_quantize_act_launch(w_dtype, x_dev, x_dtype, workspace_dev, k, m, s))) return rc;
-    float *tmp = (float *)((uint8_t *)workspace_dev + cq_act_layout(w_dtype, k, m).total);
-    float *split_ws = cq_qmm_splits(k, n, m) > 1 ? (float *)((uint8_t *)tmp + cq_align256(m * n * 4)) : nullptr;
-    if (dst_dtype == CQ_F32)
-        return cq_matmul_launch(w_dtype, w_dev, workspace_dev, (float *)dst_dev, k, n, m, n, s, split_ws);
-    if ((rc = cq_matmul_launch(w_dtype, w_dev, workspace_dev, tmp, k, n, m, n, s, split_ws))) return rc;
-    return cq_convert_f32_launch(tmp, dst_dev, dst_dtype, m * n, s);
+    return forward_quantized(w_dtype, w_dev, dst_dev, dst_dtype, m, k, n, workspace_dev, workspace_bytes, s);
 }
 
 int64_t cq_static_workspace_bytes(void) {
@@ -265,7 +287,7 @@ int cq_nn_qmatmul_swiglu_rows(int w_dtype, const void *w_dev, const float *gate_
     if ((rc = check_weight_ptr(w_dtype, w_dev))) return rc;
     if (!gate_dev || !up_dev || !dst_dev || !workspace_dev) return CQ_ERR_NULL;
     if (!aligned(gate_dev, 16) || !aligned(up_dev, 16) || !aligned(workspace_dev, 256) || !aligned(dst_dev, 4)) return CQ_ERR_ALIGN;
-    if (workspace_bytes < cq_qmatmul_workspace_bytes(w_dtype, m, k, n)) return CQ_ERR_WORKSPACE;
+    if (workspace_bytes < workspace_least(w_dtype, m, k, n)) return CQ_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     if (m >= 3 && cq_matvec_batch_takes(w_dtype, w_dev, k, n, m))          // the kernel cq_qmatmul_forward takes for these shapes
         return cq_matvec_batch_swiglu_launch(w_dtype, w_dev, gate_dev, up_dev, gate_stride, up_stride, workspace_dev, dst_dev, CQ_F32, k, n, m, n, s);
@@ -273,9 +295,7 @@ int cq_nn_qmatmul_swiglu_rows(int w_dtype, const void *w_dev, const float *gate_
         return cq_matvec_batch_mid_launch(w_dtype, w_dev, gate_dev, up_dev, gate_stride, up_stride, workspace_dev, dst_dev, k, n, m, s);
     if ((rc = cq_quantize_act_swiglu_launch(w_dtype, gate_dev, up_dev, gate_stride, up_stride, workspace_dev, k, m, s))) return rc;
     if (m <= CQ_MATVEC_MAX_ROWS && !cq_use_mfma(w_dtype, m, k)) return cq_matvec_launch(w_dtype, w_dev, workspace_dev, dst_dev, CQ_F32, k, n, m, n, s);
-    float *tmp = (float *)((uint8_t *)workspace_dev + cq_act_layout(w_dtype, k, m).total);
-    float *split_ws = cq_qmm_splits(k, n, m) > 1 ? (float *)((uint8_t *)tmp + cq_align256(m * n * 4)) : nullptr;
-    return cq_matmul_launch(w_dtype, w_dev, workspace_dev, dst_dev, k, n, m, n, s, split_ws);
+    return forward_quantized(w_dtype, w_dev, dst_dev, CQ_F32, m, k, n, workspace_dev, workspace_bytes, s);
 }
 
 int64_t cq_indexed_moe_workspace_bytes(int w_dtype, int64_t num_experts, int64_t n, int64_t k, int64_t batch, int64_t topk,

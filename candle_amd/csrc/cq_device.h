@@ -68,6 +68,12 @@ __device__ __forceinline__ uint16_t f2h_bits(float f) {
     return (uint16_t)(r & 0xffffu);
 }
 
+// f32 -> bf16 bit pattern, round to nearest even, NaNs quiet
+__device__ __forceinline__ uint16_t f2bf_bits(float f) {
+    const uint32_t b = __float_as_uint(f), r = (b & 0x7fffffffu) > 0x7f800000u ? (b | 0x00400000u) : b + 0x7fffu + ((b >> 16) & 1u);
+    return (uint16_t)(r >> 16);
+}
+
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }

@@ -53,6 +53,12 @@ int cq_matvec_norm_pair_merge_launch(int dta, const void *wa, int64_t na, float 
 int cq_matmul_launch(int w_dtype, const void *w, const void *scratch, float *dst, int64_t k, int64_t n, int64_t rows,
                      int64_t stride_dst, hipStream_t s, float *split_ws = nullptr);
 int cq_qmm_splits(int64_t k, int64_t n, int64_t rows);
+// Q4_K, Q5_K, Q6_K, Q4_0 and Q8_0 (cq_qtile.hip, cq_qtile0.hip): results in any float type; planes: optional workspace for K splits (cq_qtile_plane_bytes of it serves any number of
+// rows up to the given one; fewer bytes: fewer splits).  rows_of_w: rows of the whole tensor (of all experts)
+bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w);
+int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows);
+int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst, void *planes,
+                    int64_t plane_bytes, hipStream_t s);
 bool cq_use_mfma(int w_dtype, int64_t rows, int64_t k);
 int cq_embedding_launch(int dtype, const void *blocks, const uint32_t *ids, float *out, int64_t n_ids, int64_t rows, int64_t hidden, hipStream_t s);
 int cq_convert_f32_launch(const float *src, void *dst, int dst_dtype, int64_t count, hipStream_t s);
@@ -175,5 +181,6 @@ int cq_moe_stream_launch(int w_dtype, const void *w_a, const void *w_b, float *o
 // more than one large one)
 #define CQ_MOE_TILE_SMALL 32
 #define CQ_MOE_TILE_LARGE 128
-int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t k, int64_t n,
-                         int tile_rows, hipStream_t s);
+int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s);
+int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,
+                         int64_t n, int tile_rows, hipStream_t s);

@@ -5,19 +5,20 @@
 // candle-kernels/src/mmq_gguf/).  The arithmetic follows the CPU path instead of the CUDA one:
 // activations are the Q8_K / Q8_0 quantization written by cq_quantize_act.
 //
-// Q5_K, Q6_K, Q2_K, Q3_K — integer-exact formulation on the f16 matrix cores (qmm_kernel):
+// Q4_K, Q5_K and Q6_K go to the kernels of cq_qtile.hip where cq_qtile_takes allows it; here are the other formats, and what that
+// refuses: Q6_K tensors that do not begin and end on a dword.
+//
+// Q6_K, Q2_K, Q3_K — integer-exact formulation on the f16 matrix cores (qmm_kernel):
 //   per 256-element super-block kb      S[m,n] = sum_k q8[m,k] * (sc[n,sub(k)] * q[n,k])
-//   operands are small integers held exactly in f16 (|q8| <= 128, |sc*q| <= 1953 for Q5_K),
+//   operands are small integers held exactly in f16 (|q8| <= 128, |sc*q| <= 128 for Q3_K),
 //   products accumulate in f32, and once per super-block
 //       acc[m,n] += d8[m,kb] * ( d[n,kb] * S[m,n] - dmin[n,kb] * M[m,n] ),
-//       M[m,n] = sum_{j<16} bsums16[m,j] * min[n, group j]     (one extra K=16 MFMA; Q5_K: min of sub-block j / 2, Q2_K: of group j)
-//   — the same integers the CPU vec_dot sums (k_quants.rs:1714-1801, 2035-2092).  For Q6_K
+//       M[m,n] = sum_{j<16} bsums16[m,j] * min[n, group j]     (one extra K=16 MFMA; Q2_K's mins)
+//   — the same integers the CPU vec_dot sums (k_quants.rs:2035-2092).  For Q6_K
 //   the product sc*(q-32) can reach 4096, beyond the exact-integer range of f16, so it is fed as two
 //   terms: its f16 rounding and the exact remainder in {-1, 0, 1} (a second MFMA per k-slice).  This
 //   matters: a 1e-4 perturbation of one matmul is amplified to ~1e-2 in a decoder's logits by the
 //   activation quantizers downstream, an exact one is not.
-// Q4_K — the same sums on the int8 matrix cores (qmm_q4k_i8_kernel, k_quants.rs:1460-1540): the 6-bit sub-block scale
-//   is split into two 3-bit halves so that scale * weight fits int8; S is exact in int32.
 // Q4_0 / Q8_0 / Q4_1 / Q5_0 / Q5_1 — the per-32 sums of the CPU vec_dot (k_quants.rs:294-311, 720-738, 323-351,
 //   434-455, 530-562) on the int8 matrix cores (qmm_q0_i8_kernel): one v_mfma_i32_32x32x32_i8 per 32-element block gives
 //   the exact int32 sum of q8 * q (q - 8, q - 16 for Q4_0, Q5_0), and the vector units add
@@ -39,8 +40,7 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int BM = 128, BK = 64;
-constexpr int CQ_QMM_SMALL_ROWS = 32;      // up to here the 32-row block tile is used (measured, 14336 x 4096 Q4_K: 16 / 32 rows
-                                           // 37 / 38 us against 62 us on the 128-row tile; 64 rows as two tiles 73 us)
+constexpr int CQ_QMM_SMALL_ROWS = 32;      // up to here the 32-row block tile is used
 constexpr int LDK = BK + 8;            // padded row stride in halves (144 bytes)
 
 // ---- integer bytes -> f16 pairs ------------------------------------------------------------------
@@ -67,63 +67,11 @@ __device__ __forceinline__ uint32_t h2_splat(float v) {          // v exactly re
     return h | (h << 16);
 }
 
-// 6-bit scale / min of sub-block j (utils.rs:50-60) from the 12 packed bytes held in three dwords
-__device__ __forceinline__ void k4_sub_scale_min(uint32_t u0, uint32_t u1, uint32_t u2, int j, int &sc, int &mn) {
-    int sh = 8 * (j & 3);
-    if (j < 4) {
-        sc = (u0 >> sh) & 63;
-        mn = (u1 >> sh) & 63;
-    } else {
-        sc = ((u2 >> sh) & 0xF) | (((u0 >> sh) >> 6 & 3) << 4);
-        mn = ((u2 >> sh) >> 4 & 0xF) | (((u1 >> sh) >> 6 & 3) << 4);
-    }
-}
-
 // ---- per-format staging of NW = 32 or 16 consecutive weights of one row into NW / 2 dwords of f16 pairs -------
 // A 64-element stage (kb, g) of a row is split between 64 / NW threads; thread `part` takes elements
 // 256 kb + 64 g + NW part + [0, NW).  jh = the 32-element half of the stage these lie in, sx = which 16 of that half
 // (NW = 16 only).  Raw<NW>: what the thread loads for them.
 template <int DT> struct Stage;
-
-template <> struct Stage<CQ_Q5K> {
-    static constexpr bool HAS_MIN = true;
-    static constexpr int TERMS = 1;
-    template <int NW> struct Raw { u32x4 hdr, h[NW / 16], q[NW / 16]; };
-    template <int NW> static __device__ __forceinline__ void load(Raw<NW> &r, const uint8_t *row, int kb, int g, int part) {
-        const uint8_t *blk = row + (int64_t)kb * 176;
-        const int sx = NW == 16 ? part & 1 : 0;
-        r.hdr = *reinterpret_cast<const u32x4 *>(blk);
-#pragma unroll
-        for (int i = 0; i < NW / 16; i++) {
-            r.h[i] = *reinterpret_cast<const u32x4 *>(blk + 16 + 16 * (sx + i));
-            r.q[i] = *reinterpret_cast<const u32x4 *>(blk + 48 + 32 * g + 16 * (sx + i));
-        }
-    }
-    template <int NW> static __device__ __forceinline__ void header(const Raw<NW> &r, float &d, float &dmin) {
-        d = h2f(r.hdr.x);
-        dmin = h2f(r.hdr.x >> 16);
-    }
-    // the mins of the 16-element groups 2 jp and 2 jp + 1 in bits 0-7 and 16-23: both the min of sub-block jp (utils.rs:50-60)
-    template <int NW> static __device__ __forceinline__ uint32_t min_pair(const Raw<NW> &r, int jp) {
-        const uint32_t m4 = jp >= 4 ? ((r.hdr.w >> 4) & 0x0f0f0f0fu) | ((r.hdr.z >> 2) & 0x30303030u) : r.hdr.z & 0x3f3f3f3fu;
-        return ((m4 >> (8 * (jp & 3))) & 0xffu) * 0x00010001u;
-    }
-    template <int NW> static __device__ __forceinline__ void convert(const Raw<NW> &r, int g, int part, uint32_t out[NW / 2]) {
-        const int jh = NW == 16 ? part >> 1 : part;
-        int sc, mn;
-        k4_sub_scale_min(r.hdr.y, r.hdr.z, r.hdr.w, 2 * g + jh, sc, mn);
-        const uint32_t s2 = h2_splat((float)sc), c2 = h2_splat(-1024.0f * (float)sc);
-#pragma unroll
-        for (int i = 0; i < NW / 4; i++) {
-            const uint32_t hb = (r.h[i >> 2][i & 3] >> (2 * g + jh)) & 0x01010101u;
-            const uint32_t v = ((r.q[i >> 2][i & 3] >> (4 * jh)) & 0x0f0f0f0fu) | (hb << 4);
-            uint32_t lo, hi;
-            bytes_to_h1024(v, lo, hi);
-            out[2 * i] = pk_fma(lo, s2, c2);        // (1024 + q) * sc - 1024 * sc = sc * q, one exact rounding
-            out[2 * i + 1] = pk_fma(hi, s2, c2);
-        }
-    }
-};
 
 template <> struct Stage<CQ_Q6K> {
     static constexpr bool HAS_MIN = false;
@@ -519,238 +467,8 @@ __global__ __launch_bounds__(256, NJ == 1 && !(SM && Stage<DT>::TERMS == 2) ? 2 
         }
 }
 
-// ---- Q4_K on the int8 matrix cores ----------------------------------------------------------------------------------
-// The 6-bit sub-block scale is split as sc = 8 hi + lo (hi, lo < 8): lo * q and hi * q stay below 128, so they are int8
-// operands, and     S[m,n] = sum_k q8[m,k] * sc * q[n,k] = 8 * sum_k q8 (hi q) + sum_k q8 (lo q)
-// is two v_mfma_i32_32x32x32_i8 chains with exact int32 sums over the super-block — the integer the CPU vec_dot forms
-// (k_quants.rs:1460-1540) — followed by the same f32 step as above: acc += d8 * (d * S - dmin * M).  Against the f16
-// formulation: the activations go to LDS as the raw int8 (no conversion, half the bytes), four weights take one
-// v_pk_mul_lo_u16 per term, and a k-slice of 32 needs as many LDS bytes as a k-slice of 16 did.
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_mul_u16(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
-}
-
-// Same tiling and template parameters as qmm_kernel; a stage is 128 elements of k (half a super-block), held twice in
-// LDS: while the matrix cores work on one copy the threads fill the other (one barrier per stage).  What goes through
-// LDS is raw: the int8 activations, and the weight rows' packed nibbles and 16-byte headers as they lie in memory, both
-// copied with fully used cache lines (8 lanes per 128-byte activation row, 4 per 64-byte weight row) because the
-// address path of the vector cache, not the matrix cores, is what the tile loads saturate first.  Each lane then builds
-// its own MFMA B operands: lane (n, kg) of a 32 x 32 x 32 MFMA wants 16 consecutive k of row n, which for Q4_K are the
-// nibbles of one 16-byte piece — low nibbles for the even sub-block of a 64-element pair, high nibbles for the odd
-// one — times the two halves of the sub-block scale.  16-byte pieces are XOR-swizzled inside their rows so that eight
-// neighbouring lanes always touch eight different bank groups.
-template <int NJ, bool MOE = false, bool SM = false>
-__global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void qmm_q4k_i8_kernel(const uint8_t *__restrict__ w, ActView av, float *__restrict__ dst,
-                                                                            int k, int n, int rows, int64_t stride_dst, MoeChunks mc,
-                                                                            int64_t expert_bytes, int64_t split_stride) {
-    static_assert(!SM || NJ == 1, "the small-m tile has one 32-column MFMA tile per wave");
-    constexpr int BMT = SM ? 32 : BM, MI = SM ? 1 : 2;
-    constexpr int BN = SM ? 128 : 64 * NJ, WN = 32 * NJ;
-    constexpr int NA = BMT / 32, NB = BN / 64;                 // 16-byte pieces a thread copies per stage: activations, weights
-    __shared__ __align__(16) int8_t As[2][BMT * 128];          // [row][8 pieces], piece p of row r at p ^ (r & 7)
-    __shared__ __align__(16) uint8_t Bq[2][BN * 64];           // [row][4 pieces], piece p of row r at p ^ ((r >> 1) & 3)
-    __shared__ __align__(16) uint8_t Bhd[2][BN * 16];          // block headers (d, dmin, scales), per super-block parity
-    __shared__ __align__(16) _Float16 Am[2][BMT * 24];         // bsums16 of the super-block, as f16 (row stride 24 halves)
-    __shared__ float sD8[2][BMT];
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = SM ? 0 : wv >> 1, wn = SM ? wv : wv & 1;
-    int m0 = blockIdx.x * BMT;
-    const int n0 = blockIdx.y * BN;
-    if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;           // uniform over the workgroup
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
-    }
-    const int nsb_all = k >> 8;
-    const int kb0 = (int)(((int64_t)nsb_all * blockIdx.z) / gridDim.z), nsb = (int)(((int64_t)nsb_all * (blockIdx.z + 1)) / gridDim.z);
-    dst += (int64_t)blockIdx.z * split_stride;
-    const int64_t row_bytes = (int64_t)(k / 256) * 144;
-
-    // ---- copy roles.  Rows past the end of the tile are clamped to a valid row: an output row depends on its own
-    // activation row only, and the rows past the end are not stored ----
-    const int ra = tid >> 3, pa = tid & 7;                       // activations: piece pa of rows ra + 32 i
-    const int rb = tid >> 2, pb = tid & 3;                       // weights: piece pb of rows rb + 64 i
-    const int rh = tid & (BN - 1);                               // header of weight row rh
-    const int rs = (tid >> 1) & (BMT - 1), half = tid & 1;       // d8 and eight of the sixteen bsums of activation row rs
-    const int8_t *a_src[NA];
-#pragma unroll
-    for (int i = 0; i < NA; i++) a_src[i] = av.qs + (int64_t)min(m0 + ra + 32 * i, rows - 1) * k + 16 * pa;
-    const uint8_t *b_src[NB];
-#pragma unroll
-    for (int i = 0; i < NB; i++) b_src[i] = w + (int64_t)min(n0 + rb + 64 * i, n - 1) * row_bytes + 16 + 16 * pb;
-    const uint8_t *h_src = w + (int64_t)min(n0 + rh, n - 1) * row_bytes;
-    const int srow = min(m0 + rs, rows - 1);
-    const int a_dst = ra * 128 + 16 * (pa ^ (ra & 7)), b_dst = rb * 64 + 16 * (pb ^ ((rb >> 1) & 3));
-    // ---- MFMA operand roles ----
-    const int kg = lane >> 5, swz_a = lane & 7, swz_b = (lane >> 1) & 3;
-
-    f32x16 acc[MI][NJ];
-    i32x16 sl[MI][NJ], sh[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) { acc[i][j][e] = 0.0f; sl[i][j][e] = 0; sh[i][j][e] = 0; }
-
-    // registers of the stage in flight.  Stage (kb, s2) covers k = 256 kb + 128 s2 + [0, 128).  Positions past the end of
-    // this split's range are clamped to its last super-block: what they bring lands in an LDS copy that nobody reads.
-    u32x4 ga[NA], gb[NB], ghdr = u32x4{0, 0, 0, 0}, gbs = u32x4{0, 0, 0, 0};
-    float gd8 = 0.0f;
-    auto load_stage = [&](int kb, int s2) {
-        kb = min(kb, nsb - 1);
-#pragma unroll
-        for (int i = 0; i < NA; i++) ga[i] = *reinterpret_cast<const u32x4 *>(a_src[i] + kb * 256 + 128 * s2);
-#pragma unroll
-        for (int i = 0; i < NB; i++) gb[i] = *reinterpret_cast<const u32x4 *>(b_src[i] + (int64_t)kb * 144 + 64 * s2);
-        if (s2 == 0) {
-            ghdr = *reinterpret_cast<const u32x4 *>(h_src + (int64_t)kb * 144);
-            gd8 = av.d[(int64_t)srow * (k >> 8) + kb];
-            gbs = *reinterpret_cast<const u32x4 *>(av.bsums + (int64_t)srow * (k >> 4) + kb * 16 + 8 * half);
-        }
-    };
-    // buf: LDS copy of the stage (s2); hb: copy of the per-super-block arrays (parity of the super-block)
-    auto store_stage = [&](int s2, int hb) {
-#pragma unroll
-        for (int i = 0; i < NA; i++) *reinterpret_cast<u32x4 *>(As[s2] + a_dst + 32 * 128 * i) = ga[i];
-#pragma unroll
-        for (int i = 0; i < NB; i++) *reinterpret_cast<u32x4 *>(Bq[s2] + b_dst + 64 * 64 * i) = gb[i];
-        if (s2 == 0) {
-            // threads that share a row write the same values
-            *reinterpret_cast<u32x4 *>(Bhd[hb] + 16 * rh) = ghdr;
-            sD8[hb][rs] = gd8;
-            const uint32_t b4[4] = {gbs.x, gbs.y, gbs.z, gbs.w};
-            u32x4 bv;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t lo = f2h_bits((float)(int16_t)(b4[i] & 0xffff)), hi = f2h_bits((float)(int16_t)(b4[i] >> 16));
-                bv[i] = lo | (hi << 16);
-            }
-            *reinterpret_cast<u32x4 *>(Am[hb] + rs * 24 + 8 * half) = bv;
-        }
-    };
-    load_stage(kb0, 0);
-    store_stage(0, kb0 & 1);
-    load_stage(kb0, 1);
-    __syncthreads();
-
-    for (int kb = kb0; kb < nsb; kb++) {
-        const int hb = kb & 1;
-#pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
-            const int8_t *Ab = As[s2];
-            const uint8_t *Bb = Bq[s2];
-            u32x4 hdr[NJ];
-#pragma unroll
-            for (int t = 0; t < NJ; t++) hdr[t] = *reinterpret_cast<const u32x4 *>(Bhd[hb] + 16 * (wn * WN + t * 32 + (lane & 31)));
-#pragma unroll
-            for (int gg = 0; gg < 2; gg++) {
-                const int g = 2 * s2 + gg;
-                // ---- weights of sub-blocks 2 g (low nibbles) and 2 g + 1 (high nibbles) ----
-                i32x4 bl[2][NJ], bh[2][NJ];
-#pragma unroll
-                for (int t = 0; t < NJ; t++) {
-                    const u32x4 q = *reinterpret_cast<const u32x4 *>(Bb + (wn * WN + t * 32 + (lane & 31)) * 64 + 16 * ((2 * gg + kg) ^ swz_b));
-                    const u32x4 h = hdr[t];
-#pragma unroll
-                    for (int ks = 0; ks < 2; ks++) {
-                        // 6-bit scale of sub-block j = 2 g + ks (utils.rs:50-60); j < 4 exactly when g < 2
-                        const int sft = 16 * (g & 1) + 8 * ks;
-                        const uint32_t sc = g < 2 ? (h.y >> sft) & 63u : ((h.w >> sft) & 0xFu) | (((h.y >> sft) >> 2) & 0x30u);
-                        const uint32_t lo2 = (sc & 7u) * 0x00010001u, hi2 = (sc >> 3) * 0x00010001u;
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const uint32_t v = (ks ? q[i] >> 4 : q[i]) & 0x0f0f0f0fu;    // four weights, one per byte
-                            bl[ks][t][i] = (int)pk_mul_u16(v, lo2);                         // bytes stay below 128: no carries
-                            bh[ks][t][i] = (int)pk_mul_u16(v, hi2);
-                        }
-                    }
-                }
-                // ---- 2 k-slices of 32: MI x NJ tiles, two MFMA chains each ----
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    i32x4 af[MI];
-#pragma unroll
-                    for (int t = 0; t < MI; t++)
-                        af[t] = *reinterpret_cast<const i32x4 *>(Ab + (wm * 64 + t * 32 + (lane & 31)) * 128 + 16 * ((4 * gg + 2 * ks + kg) ^ swz_a));
-#pragma unroll
-                    for (int i = 0; i < MI; i++)
-#pragma unroll
-                        for (int j = 0; j < NJ; j++) {
-                            if (g == 0 && ks == 0) {                    // first slice of the super-block: the sums start from zero
-                                i32x16 z;
-#pragma unroll
-                                for (int e = 0; e < 16; e++) z[e] = 0;
-                                sl[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bl[ks][j], z, 0, 0, 0);
-                                sh[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bh[ks][j], z, 0, 0, 0);
-                            } else {
-                                sl[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bl[ks][j], sl[i][j], 0, 0, 0);
-                                sh[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bh[ks][j], sh[i][j], 0, 0, 0);
-                            }
-                        }
-                }
-            }
-            // ---- the stage in flight goes to the other LDS copy; its registers take the stage after it ----
-            store_stage(s2 ^ 1, s2 ? hb ^ 1 : hb);
-            load_stage(kb + 1, s2);
-            if (s2 == 1) {
-                // ---- end of the super-block: mins term and the f32 scales ----
-                half8 am[MI];
-#pragma unroll
-                for (int t = 0; t < MI; t++)
-                    am[t] = *reinterpret_cast<const half8 *>(Am[hb] + (wm * 64 + t * 32 + (lane & 31)) * 24 + 8 * kg);
-#pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    const u32x4 h = hdr[j];
-                    const float d = h2f(h.x), dmin = h2f(h.x >> 16);
-                    // B operand of the mins MFMA: element 2 i, 2 i + 1 of this lane = min of sub-block 4 kg + i, one per
-                    // byte first (sub-blocks 0-3: low 6 bits of h.z; 4-7: high nibbles of h.w | top bits of h.z)
-                    const uint32_t mine = kg ? ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u) : h.z & 0x3f3f3f3fu;
-                    u32x4 mv;
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        mv[i] = pk_add((0x6400u | ((mine >> (8 * i)) & 0xffu)) * 0x00010001u, 0xe400e400u);   // (1024 + min) - 1024, twice
-                    const half8 bm = __builtin_bit_cast(half8, mv);
-#pragma unroll
-                    for (int i = 0; i < MI; i++) {
-                        f32x16 z;
-#pragma unroll
-                        for (int e = 0; e < 16; e++) z[e] = 0.0f;
-                        const f32x16 mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am[i], bm, z, 0, 0, 0);
-#pragma unroll
-                        for (int e = 0; e < 16; e++) {
-                            const int ml = wm * 64 + i * 32 + 8 * (e >> 2) + 4 * kg + (e & 3);
-                            float t = d * (float)(8 * sh[i][j][e] + sl[i][j][e]);
-                            t = fmaf(-dmin, mt[e], t);
-                            acc[i][j][e] = fmaf(sD8[hb][ml], t, acc[i][j][e]);
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const int nn = n0 + wn * WN + j * 32 + (lane & 31);
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int mm = m0 + wm * 64 + i * 32 + 8 * (e >> 2) + 4 * kg + (e & 3);
-                if (mm < rows && nn < n) {
-                    if (MOE) dst[(int64_t)mc.pair_out[mm] * stride_dst + nn] = acc[i][j][e] * mc.pair_scale[mm];
-                    else dst[(int64_t)mm * stride_dst + nn] = acc[i][j][e];
-                }
-            }
-        }
-}
 
 // ---- Q4_0 / Q8_0 / Q4_1 / Q5_0 / Q5_1 on the int8 matrix cores --------------------------------------------------------
 // Same tiling and template parameters as above.  Both operands carry an f16 scale per 32 elements, so a 32 x 32 x 32 int8
@@ -759,7 +477,7 @@ __global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void qmm_q4k_i8_kernel(const 
 // (float(S) * d[n]) * d8[m], plus m[n] * s[m] for the formats with a block minimum (s = the Q8_1 block sum, k_quants.rs:770-799),
 // block after block in k order like the CPU loop.  That scaling is three or four vector instructions per result and
 // bounds the kernel; the matrix cores idle most of the time.  A stage is 128 elements of k (four blocks), held twice in
-// LDS (one barrier per stage): the int8 activations as in the Q4_K kernel, the four d8 (and s) per activation row, and
+// LDS (one barrier per stage): the int8 activations, the four d8 (and s) per activation row, and
 // the weight rows' four blocks as they lie in memory (72 .. 136 contiguous bytes per row), copied in 8-byte pieces by
 // neighbouring lanes so that a load instruction touches a handful of cache lines, not one per lane.  Lane (n, kg) of the
 // B operand wants 16 consecutive k of row n: the 16 quant bytes of the block (4- and 5-bit formats: low nibbles for
@@ -955,11 +673,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 }
 
 typedef void (*QmmFn)(const uint8_t *, ActView, float *, int, int, int, int64_t, MoeChunks, int64_t, int64_t);
-// the kernel of a format and tile shape: Q4_K and the 32-element formats run on the int8 matrix cores, the others on the f16 ones
+// the kernel of a format and tile shape: the 32-element formats run on the int8 matrix cores, the others on the f16 ones
 template <int DT, int NJ, bool MOE, bool SM>
 QmmFn qmm_fn() {
-    if constexpr (DT == CQ_Q4K) return qmm_q4k_i8_kernel<NJ, MOE, SM>;
-    else if constexpr (DT == CQ_Q4_0 || DT == CQ_Q8_0 || DT == CQ_Q4_1 || DT == CQ_Q5_0 || DT == CQ_Q5_1)
+    if constexpr (DT == CQ_Q4_0 || DT == CQ_Q8_0 || DT == CQ_Q4_1 || DT == CQ_Q5_0 || DT == CQ_Q5_1)
         return qmm_q0_i8_kernel<DT, NJ, MOE, SM>;
     else return qmm_kernel<DT, NJ, MOE, SM>;
 }
@@ -1007,9 +724,7 @@ __global__ __launch_bounds__(256) void convert_f32_kernel(const float *__restric
     if (dst_dtype == CQ_F16) {
         ((uint16_t *)dst)[i] = f2h_bits(v);
     } else {
-        uint32_t b = __float_as_uint(v);
-        uint32_t r = (b & 0x7fffffffu) > 0x7f800000u ? (b | 0x00400000u) : b + 0x7fffu + ((b >> 16) & 1u);
-        ((uint16_t *)dst)[i] = (uint16_t)(r >> 16);
+        ((uint16_t *)dst)[i] = f2bf_bits(v);
     }
 }
 
@@ -1043,17 +758,16 @@ int launch_qmm_moe(const void *w, const ActView &av, float *out, const MoeChunks
 }  // namespace
 
 // tile_rows: rows of one chunk of the table, CQ_MOE_TILE_SMALL (32) or CQ_MOE_TILE_LARGE (128)
-int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t k, int64_t n,
-                         int tile_rows, hipStream_t s) {
+int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,
+                         int64_t n, int tile_rows, hipStream_t s) {
     if (mc.max_chunks == 0 || n == 0) return CQ_OK;
     if (k % 256) return CQ_ERR_SHAPE;
     if (tile_rows != CQ_MOE_TILE_SMALL && tile_rows != CQ_MOE_TILE_LARGE) return CQ_ERR_RANGE;
     ActView av = cq_act_view(scratch, w_dtype, k, rows_alloc);
+    if (cq_qtile_takes(w_dtype, w, k, num_experts * n)) return cq_qtile_moe_launch(w_dtype, w, av, out, mc, k, n, tile_rows, s);
     switch (w_dtype) {
         case CQ_Q4_0: return launch_qmm_moe<CQ_Q4_0>(w, av, out, mc, k, n, tile_rows, s);
         case CQ_Q8_0: return launch_qmm_moe<CQ_Q8_0>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q4K: return launch_qmm_moe<CQ_Q4K>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q5K: return launch_qmm_moe<CQ_Q5K>(w, av, out, mc, k, n, tile_rows, s);
         case CQ_Q6K: return launch_qmm_moe<CQ_Q6K>(w, av, out, mc, k, n, tile_rows, s);
         case CQ_Q2K: return launch_qmm_moe<CQ_Q2K>(w, av, out, mc, k, n, tile_rows, s);
         case CQ_Q3K: return launch_qmm_moe<CQ_Q3K>(w, av, out, mc, k, n, tile_rows, s);
@@ -1094,6 +808,8 @@ int cq_matmul_launch(int w_dtype, const void *w, const void *scratch, float *dst
     // the matrix-core kernel of the 32-element formats copies weight rows in 8-byte pieces; weights at another alignment
     // take the loop below
     const bool q0_unaligned = !cq_is_kquant(w_dtype) && ((uintptr_t)w & 7) != 0;
+    if (cq_use_mfma(w_dtype, rows, k) && cq_qtile_takes(w_dtype, w, k, n))
+        return cq_qtile_launch(w_dtype, w, av, dst, CQ_F32, k, n, rows, stride_dst, nullptr, 0, s);
     if (cq_use_mfma(w_dtype, rows, k) && !q0_unaligned) {
         switch (w_dtype) {
             case CQ_Q4_0: return launch_qmm<CQ_Q4_0>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
@@ -1101,8 +817,6 @@ int cq_matmul_launch(int w_dtype, const void *w, const void *scratch, float *dst
             case CQ_Q4_1: return launch_qmm<CQ_Q4_1>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
             case CQ_Q5_0: return launch_qmm<CQ_Q5_0>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
             case CQ_Q5_1: return launch_qmm<CQ_Q5_1>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
-            case CQ_Q4K: return launch_qmm<CQ_Q4K>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
-            case CQ_Q5K: return launch_qmm<CQ_Q5K>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
             case CQ_Q6K: return launch_qmm<CQ_Q6K>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
             case CQ_Q2K: return launch_qmm<CQ_Q2K>(w, av, dst, k, n, rows, stride_dst, s, split_ws);
             case CQ_Q3K: return launch_qmm<CQ_Q3K>(w, av, dst, k, n, rows, stride_dst, s, split_ws);

@@ -274,7 +274,7 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
     int rc = cq_quantize_act_swiglu_gather_launch(w_dtype, gate, up, pout, n_valid, topk_weights, pscale, b + ws.act_off, k, n_pairs, ws.rows_alloc, s);
     if (rc) return rc;
     MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
-    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, k, n, moe_tile_rows(n_pairs, num_experts), s);
+    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, num_experts, k, n, moe_tile_rows(n_pairs, num_experts), s);
 }
 
 int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
@@ -330,8 +330,8 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     if (mfma) {
         if ((rc = cq_quantize_act_gather_launch(a.w_dtype, a.x, pin, b + ws.act_off, a.k, a.n_pairs, ws.rows_alloc, s))) return rc;
         MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
-        rc = cq_matmul_moe_launch(a.w_dtype, a.w, b + ws.act_off, ws.rows_alloc, a.out, mc, a.k, a.n, tile_rows, s);
-        if (!rc && a.w_b) rc = cq_matmul_moe_launch(a.w_dtype, a.w_b, b + ws.act_off, ws.rows_alloc, a.out_b, mc, a.k, a.n, tile_rows, s);
+        rc = cq_matmul_moe_launch(a.w_dtype, a.w, b + ws.act_off, ws.rows_alloc, a.out, mc, a.num_experts, a.k, a.n, tile_rows, s);
+        if (!rc && a.w_b) rc = cq_matmul_moe_launch(a.w_dtype, a.w_b, b + ws.act_off, ws.rows_alloc, a.out_b, mc, a.num_experts, a.k, a.n, tile_rows, s);
         return rc;
     }
     if (a.k % 256 == 0) {

@@ -1,0 +1,61 @@
+// Prefill kernels over quantized weights (cq_qtile.hip): the workgroup's shape, the way results go out, the launch.
+#pragma once
+#include "cq_device.h"
+#include "cq_fmt.h"
+#include "cq_launch.h"
+#include "cq_stream.h"
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int QT_NW = 8;                                 // waves of a workgroup, side by side along n
+
+// everything that goes into these sums is worked out before what follows (the scheduler would rather work on all tiles at once, out of
+// registers that are not there)
+__device__ __forceinline__ void qt_pin(f32x16 &v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(v) :: "memory");
+#endif
+}
+
+// Results of a wave: column nn of rows m0 .., in the layout of the 32 x 32 matrix instructions (row 8 (e / 4) + 4 kg + e % 4 of each tile).
+// MOE: rows of the expert-sorted list, scattered to their pairs' rows and scaled.  Splits of K after the first write f32 planes [rows, n].
+template <int MI, bool MOE>
+__device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int dst_dtype, int m0, int rows, int nn, int n, int kg, int64_t stride_dst, float *planes,
+                                         const MoeChunks &mc) {
+    auto store = [&](auto put) {
+#pragma unroll
+        for (int t = 0; t < MI; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int mm = m0 + t * 32 + 8 * (e >> 2) + 4 * kg + (e & 3);
+                if (mm < rows && nn < n) put(mm, acc[t][e]);
+                if ((e & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    if constexpr (MOE) {
+        store([&](int mm, float v) { ((float *)dst)[(int64_t)mc.pair_out[mm] * stride_dst + nn] = v * mc.pair_scale[mm]; });
+    } else {
+        if (dst_dtype == CQ_F32 || blockIdx.z > 0) {
+            float *const out = (blockIdx.z > 0 ? planes + (int64_t)(blockIdx.z - 1) * rows * n : (float *)dst) + nn;
+            const int64_t ld = blockIdx.z > 0 ? n : stride_dst;
+            store([&](int mm, float v) { out[mm * ld] = v; });
+        } else if (dst_dtype == CQ_F16) store([&](int mm, float v) { ((uint16_t *)dst)[nn + mm * stride_dst] = f2h_bits(v); });
+        else store([&](int mm, float v) { ((uint16_t *)dst)[nn + mm * stride_dst] = f2bf_bits(v); });
+    }
+}
+
+typedef void (*QtFn)(const uint8_t *, ActView, void *, int, int, int, int, int64_t, MoeChunks, int64_t, float *);
+
+inline int qtile_go(QtFn fn, int lds_bytes, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
+                    const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
+    hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(fn, grid, dim3(QT_NW * 64), lds_bytes, s, (const uint8_t *)w, av, dst, dst_dtype, (int)k, (int)n, (int)rows, stride_dst, mc, expert_bytes, planes);
+    return (int)hipGetLastError();
+}
+
+}  // namespace

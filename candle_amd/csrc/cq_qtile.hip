@@ -1,0 +1,508 @@
+// Prefill matmul of Q4_K, Q5_K and Q6_K over pre-quantized activations (Q8_K blocks) on the int8 matrix cores of gfx950:   dst[m, n] = sum_k x^[m, k] * W^[n, k]
+//
+// Per super-block of 256 elements the exact integer S[m,n] = sum_k q8[m,k] * (scale[n, sub(k)] * q[n,k]) of the CPU's dot products (k_quants.rs:1460-1540,
+// 1714-1801, 2035-2092), then acc += d8 * (d * S - dmin * M), M the products of the 16-element sums with the mins (one f16 MFMA, exact).  scale * q has up to
+// 13 bits, so it goes through the int8 cores as two operands in two chains: Q4_K as scale % 8 * q and scale / 8 * q (S = lo + 8 hi), Q5_K and Q6_K as the
+// low byte less 128 and the high byte of scale * q + 128 (S = lo + 256 hi).
+//
+// What bounds it: at many rows the matrix cores at the clock that the power limit leaves (16 + 1 MFMAs of 32 x 32 x 32 per 32 rows, super-block and wave, about
+// 20 ns each with all units busy, 14.5 at the full clock), with the conversion of the weights behind it; at few rows the weights' way from memory.  So:
+//  - a workgroup is eight waves side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
+//    multiplies it, straight into its operand registers (the kernels before this one staged converted weights in LDS, and the conversion
+//    of Q5_K and Q6_K was to f16, Q6_K as two f16 terms: twice the matrix time of int8);
+//  - weights go by copies to LDS into a ring of the wave's own, three stages of 64 elements ahead, with counted waits and no barrier; activations into a ring of
+//    three super-blocks shared by the workgroup, one barrier per super-block.  Q6_K blocks begin on 2 bytes: its pieces are brought from the dword below and
+//    shifted on reading, two half super-blocks at a time;
+//  - waves 4 - 7 (the second on each SIMD) run half a super-block behind, so that the vector work at the end of a super-block lies under the other wave's
+//    matrix work (7 % at 2048 rows; Q6_K, whose waves take part in fewer barriers, gains nothing and does without);
+//  - fragments, conversions and products of one step are interleaved by hand, the sums of a tile pinned before the next one's: left to itself the
+//    scheduler spills.
+// f16 / bf16 results are written by the product; the f32 copy and its conversion went (12 us of 154 for 512 rows of Q5_K).
+//
+// [4096 x 14336], us, before / now, quantizing the activations included:    17 rows   131 rows   512 rows   2048 rows
+//   Q4_K                                                                  20.3 19.1  53.6 42.8  103 92.1   360 298
+//   Q5_K                                                                  36.8 22.1  73.4 47.2  144 101    514 324
+//   Q6_K                                                                  37.2 26.3  80.6 52.4  161 109    584 357
+// 2048 rows of Q4_K are 810 TOP/s of products asked for and 1620 done.
+#include "cq_qtile.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t qt_pk_add(uint32_t a, uint32_t b) {
+    half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
+    return __builtin_bit_cast(uint32_t, r);
+}
+__device__ __forceinline__ uint32_t qt_pk_mul(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t qt_pk_mad(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
+}
+
+// The lane's number, worked out where it is asked for (what follows from threadIdx.x is kept in registers over the whole main loop, which needs all of them).
+__device__ __forceinline__ int qt_lane() {
+    int l = 0;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+#endif
+    return l;
+}
+
+// A wave's weights: 32 rows, lane (row = lane % 32, kg = lane / 32) holds elements 16 kg .. 16 kg + 15 of every 32-element sub-block.
+// EXTRA: 16-byte pieces per lane and super-block beside the four of the quants.  HI: factor of the hi chain.
+template <int DT> struct QTile;
+template <> struct QTile<CQ_Q4K> {
+    static constexpr int EXTRA = 1, HI = 8, QS = 16;
+    static constexpr bool HAS_MIN = true;
+};
+template <> struct QTile<CQ_Q5K> {
+    static constexpr int EXTRA = 2, HI = 256, QS = 48;
+    static constexpr bool HAS_MIN = true;
+};
+
+// Q6_K blocks (210 bytes) begin on 2 bytes: a lane brings the four dwords that its 16 bytes begin in and, separately, the one after them.
+// Its ring holds two half super-blocks of three pieces (ql[0 .. 31], ql[32 .. 63], qh of the half), and a piece of the scales with d behind them.
+template <> struct QTile<CQ_Q6K> {
+    static constexpr int EXTRA = 0, HI = 256, QS = 0;
+    static constexpr bool HAS_MIN = false;
+};
+
+constexpr int QT_R = 4, QT_L = QT_R - 1;                 // stages (64 elements) in a wave's ring of weights, stages requested ahead
+// RA: super-blocks in the ring of activations
+template <int DT, int MI> struct QtLds {
+    static constexpr int PIECE = 1024 + 256, RA = DT == CQ_Q6K ? 2 : 3;
+    static constexpr int A = MI * 8192, B = DT == CQ_Q6K ? 7 * PIECE : 1024 * (QT_R + QTile<DT>::EXTRA), AM = QTile<DT>::HAS_MIN ? MI * 1024 : 0, D8 = (MI + 1) / 2 * 256;
+    static constexpr int A_OFF = 0, B_OFF = RA * A, AM_OFF = B_OFF + QT_NW * B, D8_OFF = AM_OFF + RA * AM, BYTES = D8_OFF + RA * D8;
+};
+
+template <int DT, int MI, bool MOE>
+__global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
+                                                              int rows, int64_t stride_dst, MoeChunks mc, int64_t expert_bytes, float *__restrict__ planes) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler has no use for the body, and does not know its buffer accesses)
+    typedef QTile<DT> T;
+    typedef QtLds<DT, MI> LD;
+    constexpr int BB = BlockInfo<DT>::bytes, EX = T::EXTRA, BM = 32 * MI, BN = 32 * QT_NW;
+    constexpr int NA = MI;                                 // copy instructions per wave and super-block of activations
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nr = lane & 31, kg = lane >> 5;
+    int m0 = blockIdx.x * BM;
+    const int n0 = blockIdx.y * BN + 32 * wv;
+    if (MOE) {
+        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
+        m0 = mc.first[blockIdx.x];
+        rows = m0 + mc.count[blockIdx.x];
+        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+    }
+    const int nsb_all = k >> 8;
+    const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
+    const int64_t row_bytes = (int64_t)nsb_all * BB;
+
+    // ---- weights: rows past the end repeat the last one (their results are not stored) ----
+    const int wbase = min(n0, n - 1);
+    const uint8_t *const wrow = w + wbase * row_bytes;
+    const uint32_t w_odd = DT == CQ_Q6K ? (uint32_t)(uintptr_t)wrow & 2u : 0u;       // (the descriptor begins on a dword)
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(wrow - w_odd), 0, -1, 0x00020000);
+    const uint32_t w_off = (uint32_t)(min(nr, n - 1 - wbase) * row_bytes) + 16 * kg + w_odd;
+    // ---- activations: 64 bytes of 16 rows per instruction, piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
+    // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + 8 i of its 8 MI KB)
+    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
+    constexpr int NAO = MI == 4 ? 1 : NA;                  // (four row blocks of two: the instructions of a wave are whole stages apart)
+    uint32_t a_off[NAO];
+#pragma unroll
+    for (int i = 0; i < NAO; i++) {
+        const int blk = wv + QT_NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
+        a_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)k + 64 * st + 16 * p;
+    }
+    uint8_t *const myB = lds + LD::B_OFF + wv * LD::B;
+    // ---- scales and 16-element sums of the activations: waves 0 - 3 bring the sums of 32 rows each, the others the scales of 64 ----
+    const bool x_sums = T::HAS_MIN && wv < 4;
+    const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = min(x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane, rows - 1 - m0);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        x_sums ? (void *)(av.bsums + (int64_t)m0 * (k >> 4)) : (void *)(av.d + (int64_t)m0 * nsb_all), 0, -1, 0x00020000);
+    const uint32_t x_off = x_sums ? (uint32_t)x_r * (uint32_t)(32 * nsb_all) + 16 * (lane & 1) : (uint32_t)x_r * (uint32_t)(4 * nsb_all);
+    // weights of stage u = 4 (kb - kb0) + q into slot q of this wave's ring; past the end the last super-block again, into slots nobody reads
+    // (Q6_K: half q of the super-block)
+    auto issue_w = [&](int kb, int q) {
+        kb = min(kb, kb1 - 1);
+        if constexpr (DT == CQ_Q6K) {
+            const int at0 = kb * BB & ~3;                  // (210 kb is 2 past a dword for odd kb, and so are odd rows of an odd number of blocks)
+            const uint32_t off = (w_off + (uint32_t)(kb * BB & 2)) & ~2u;
+            auto piece = [&](int at, int slot) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::PIECE), 16, off, at0 + at, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::PIECE + 1024), 4, off, at0 + at + 16, 0, 0);
+            };
+            piece(64 * q, 3 * q);
+            piece(64 * q + 32, 3 * q + 1);
+            piece(128 + 32 * q, 3 * q + 2);
+            if (q == 0) {                                  // scales and d, for both halves of the wave
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 6 * LD::PIECE), 16, off - 16 * kg, at0 + 192, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 6 * LD::PIECE + 1024), 4, off - 16 * kg, at0 + 208, 0, 0);
+            }
+            return;
+        }
+        if (q == 0) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 1024 * QT_R), 16, w_off, kb * BB, 0, 0);      // (the upper lanes bring the 16 bytes behind it)
+            if constexpr (EX == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 1024 * (QT_R + 1)), 16, w_off, kb * BB + 16, 0, 0);
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 1024 * q), 16, w_off, kb * BB + T::QS + 32 * q, 0, 0);
+    };
+    // this wave's part of the activations of super-block j of this workgroup's range
+    auto issue_a = [&](int j, int slot) {
+        const int kb = min(kb0 + j, kb1 - 1);
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (cq_lds_void *)(lds + LD::A_OFF + slot * LD::A + 1024 * (wv + QT_NW * i)), 16, a_off[NAO == 1 ? 0 : i], kb * 256 + (NAO == 1 ? 64 * i : 0), 0, 0);
+    };
+    auto issue_x = [&](int j, int slot) {
+        const int kb = min(kb0 + j, kb1 - 1);
+        if (x_sums) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (cq_lds_void *)(lds + LD::AM_OFF + slot * LD::AM + 1024 * x_blk), 16, x_off, 32 * kb, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (cq_lds_void *)(lds + LD::D8_OFF + slot * LD::D8 + 256 * x_blk), 4, x_off, 4 * kb, 0, 0);
+    };
+
+    f32x16 acc[MI];
+    i32x16 sl[MI], sh[MI];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
+
+    issue_a(0, 0);
+    issue_x(0, 0);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < (DT == CQ_Q6K ? 1 : QT_L); t++) issue_w(kb0, t);
+    const int nsb = kb1 - kb0;
+    const int live = MOE ? (rows - m0 + 31) / 32 : MI;     // 32-row tiles that hold rows: an expert rarely fills its last ones
+
+    auto body = [&](auto late) {
+    constexpr bool LATE = decltype(late)::value;
+    int slot = 0, slot1 = 1;                               // ring slots of super-blocks j and j + 1
+    auto request = [&](int j1, int sl1) {                  // behind barrier j1 - 1: what super-block j1 needs of the activations
+        issue_a(j1, sl1);
+        issue_x(j1, sl1);
+        asm volatile("" ::: "memory");
+    };
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(DT == CQ_Q6K ? 0 : QT_L + EX) : "memory");
+    if constexpr (LATE) request(1, 1);
+    u32x4 hdr = u32x4{0, 0, 0, 0}, qh = u32x4{0, 0, 0, 0}, raw;
+    uint32_t shift = 0, d6 = 0;                            // Q6_K: bytes by which this super-block's pieces are off their dwords; d
+    i32x4 af[MI], bl, bh;
+    // operands of step s = 2 q + ks (32 elements): dword i of this lane's weights, tile t of the activations
+    uint32_t m_lo, m_hi;
+    auto scales = [&](int s) {
+        if constexpr (DT == CQ_Q6K) {
+            // int8 scale of the 16 elements 32 s + 16 kg (hdr is shifted by kg bytes)
+            const int sc = (int)(hdr[s >> 1] << (24 - 16 * (s & 1))) >> 24;
+            m_lo = __builtin_amdgcn_perm(0, (uint32_t)sc, 0x01000100u);
+            m_hi = __builtin_amdgcn_perm(0, (uint32_t)(128 - 32 * sc), 0x01000100u);
+            return;
+        }
+        // 6-bit scale of sub-block s (utils.rs:50-60)
+        const int sft = 8 * (s & 3);
+        const uint32_t sc = s < 4 ? (hdr.y >> sft) & 63u : ((hdr.w >> sft) & 0xFu) | (((hdr.y >> sft) >> 2) & 0x30u);
+        if constexpr (DT == CQ_Q4K) { m_lo = (sc & 7u) * 0x00010001u; m_hi = (sc >> 3) * 0x00010001u; }
+        else m_lo = sc * 0x00010001u;
+    };
+    auto convert = [&](int s, int i, i32x4 &lo, i32x4 &hi) {
+        if constexpr (DT == CQ_Q6K) {
+            // sc (q - 32) + 128 in 16 bits: high byte, and low byte less 128
+            const uint32_t v6 = ((s & 2 ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu) | (((qh[i] >> (2 * (s & 3))) & 0x03030303u) << 4);
+            const uint32_t e = qt_pk_mad(v6 & 0x00ff00ffu, m_lo, m_hi), o = qt_pk_mad((v6 >> 8) & 0x00ff00ffu, m_lo, m_hi);
+            lo[i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+            hi[i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+            return;
+        }
+        uint32_t v = (s & 1 ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu;
+        if constexpr (DT == CQ_Q4K) {
+            lo[i] = (int)qt_pk_mul(v, m_lo);
+            hi[i] = (int)qt_pk_mul(v, m_hi);
+        } else {
+            v |= ((qh[i] >> s) & 0x01010101u) << 4;
+            const uint32_t e = qt_pk_mad(v & 0x00ff00ffu, m_lo, 0x00800080u), o = qt_pk_mad((v >> 8) & 0x00ff00ffu, m_lo, 0x00800080u);
+            lo[i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+            hi[i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+        }
+    };
+    const uint8_t *const a_lane = lds + LD::A_OFF + nr * 64;
+    const int a_x0 = 16 * (kg ^ ((nr >> 2) & 3)), a_x1 = a_x0 ^ 32;
+    auto a_frag = [&](int s, int t) { return *reinterpret_cast<const i32x4 *>(a_lane + slot * LD::A + (s >> 1) * (MI * 2048) + t * 2048 + (s & 1 ? a_x1 : a_x0)); };
+    auto weights = [&](int q) { return *reinterpret_cast<const u32x4 *>(myB + 1024 * q + 16 * lane); };
+    // Q6_K: a piece, moved onto its dwords
+    auto piece6 = [&](int slot, uint32_t *last) {
+        u32x4 v = *reinterpret_cast<const u32x4 *>(myB + slot * LD::PIECE + 16 * lane);
+        const uint32_t behind = *reinterpret_cast<const uint32_t *>(myB + slot * LD::PIECE + 1024 + 4 * lane);
+#pragma unroll
+        for (int i = 0; i < 3; i++) v[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], shift);
+        v[3] = __builtin_amdgcn_alignbyte(behind, v[3], shift);
+        if (last) *last = behind >> (8 * shift);
+        return v;
+    };
+    auto weights6 = [&](int s) {                           // of step s
+        raw = piece6(3 * (s >> 2) + (s & 1), nullptr);
+        qh = piece6(3 * (s >> 2) + 2, nullptr);
+    };
+    // what this wave has requested behind its weights of stage q when it asks for them
+    constexpr int NX = NA + 1, W0[4] = {2, 2 + NX, 2 + NX + EX, 2 + EX}, W1[4] = {2 + NX, 2, 2 + EX, 2 + EX + NX};
+    for (int j = 0; j < nsb; j++) {
+        const int kb = kb0 + j;
+        // ---- first step of a super-block: nothing of it is in registers yet ----
+        if constexpr (DT == CQ_Q6K) {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            if (j > 0) asm volatile("s_barrier" ::: "memory");
+            issue_w(kb, 1);
+            request(j + 1, slot1);
+            shift = (w_off + (uint32_t)(kb * BB)) & 2u;
+            hdr = piece6(6, &d6);
+#pragma unroll
+            for (int i = 0; i < 4; i++) hdr[i] >>= 8 * kg;
+            weights6(0);
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LATE ? W1[0] : W0[0]) : "memory");
+            if constexpr (!LATE) {
+                if (j > 0) asm volatile("s_barrier" ::: "memory");
+                request(j + 1, slot1);
+            }
+            issue_w(kb, 3);
+            hdr = *reinterpret_cast<const u32x4 *>(myB + 1024 * QT_R + 16 * (qt_lane() & 31));
+            if constexpr (EX == 2) qh = *reinterpret_cast<const u32x4 *>(myB + 1024 * (QT_R + 1) + 16 * lane);
+            raw = weights(0);
+        }
+#pragma unroll
+        for (int t = 0; t < MI; t++) af[t] = a_frag(0, t);
+        scales(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) convert(0, i, bl, bh);
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int q = s >> 1, ns = s + 1;
+            i32x4 nl, nh;
+            if constexpr (DT == CQ_Q6K) {
+                if (s == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NX) : "memory");
+                if (s == 4) issue_w(kb + 1, 0);
+                if (ns < 8) weights6(ns);
+            } else if (s & 1) {
+                if (q < 3) {
+                    // the weights of the next stage, and a request for those three stages on
+                    if (q == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATE ? W1[1] : W0[1]) : "memory");
+                    if (q == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATE ? W1[2] : W0[2]) : "memory");
+                    if (q == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATE ? W1[3] : W0[3]) : "memory");
+                    raw = weights(q + 1);
+                }
+            } else if (q > 0) {
+                if (LATE && q == 2) {
+                    asm volatile("s_barrier" ::: "memory");
+                    request(j + 2, slot1 == 2 ? 0 : slot1 + 1);
+                }
+                issue_w(kb + 1, q - 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < MI; t++) {
+                if (!MOE || t < live) {
+                if (s == 0) {
+                    i32x16 z;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) z[e] = 0;
+                    sl[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[t], bl, z, 0, 0, 0);
+                    sh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[t], bh, z, 0, 0, 0);
+                } else {
+                    sl[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[t], bl, sl[t], 0, 0, 0);
+                    sh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[t], bh, sh[t], 0, 0, 0);
+                }
+                if (ns < 8) af[t] = a_frag(ns, t);
+                }
+                if (ns < 8) {
+                    if (t == 0) scales(ns);
+#pragma unroll
+                    for (int i = 4 * t / MI; i < 4 * (t + 1) / MI; i++) convert(ns, i, nl, nh);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (ns < 8) { bl = nl; bh = nh; }
+            if (s == 7) {
+                const float d = h2f(DT == CQ_Q6K ? d6 : hdr.x), dmin = h2f(hdr.x >> 16);
+                half8 bm;
+                if (T::HAS_MIN) {
+                    const uint32_t mlo = hdr.z & 0x3f3f3f3fu, mhi = ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u);
+                    const uint32_t kmask = 0u - (uint32_t)(qt_lane() >> 5), mine = (mhi & kmask) | (mlo & ~kmask);
+                    u32x4 mv;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) mv[i] = qt_pk_add((0x6400u | ((mine >> (8 * i)) & 0xffu)) * 0x00010001u, 0xe400e400u);
+                    bm = __builtin_bit_cast(half8, mv);
+                }
+#pragma unroll
+                for (int t = 0; t < MI; t++) {
+                    if (MOE && t >= live) break;
+                    __builtin_amdgcn_sched_barrier(0);
+                    f32x16 mt;
+                    if (T::HAS_MIN) {
+                        const s16x8 ai = *reinterpret_cast<const s16x8 *>(lds + LD::AM_OFF + slot * LD::AM + (t * 32 + nr) * 32 + 16 * kg);
+                        const half8 am = __builtin_convertvector(ai, half8);       // sums of 16 int8: exact
+                        f32x16 z;
+#pragma unroll
+                        for (int e = 0; e < 16; e++) z[e] = 0.0f;
+                        mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; e4++) {
+                        const f32x4 d8 = *reinterpret_cast<const f32x4 *>(lds + LD::D8_OFF + slot * LD::D8 + 4 * (t * 32 + 8 * e4 + 4 * kg));
+#pragma unroll
+                        for (int e1 = 0; e1 < 4; e1++) {
+                            const int e = 4 * e4 + e1;
+                            float v = d * (float)(T::HI * sh[t][e] + sl[t][e]);
+                            if (T::HAS_MIN) v = fmaf(-dmin, mt[e], v);
+                            acc[t][e] = fmaf(d8[e1], v, acc[t][e]);
+                        }
+                    }
+                    qt_pin(acc[t]);
+                }
+            }
+        }
+        slot = slot1;
+        slot1 = slot1 == LD::RA - 1 ? 0 : slot1 + 1;
+    }
+    if constexpr (!LATE && DT != CQ_Q6K) asm volatile("s_barrier" ::: "memory");       // the others' last one
+    };
+    if constexpr (DT == CQ_Q6K) body(std::false_type{});
+    else if (wv < QT_NW / 2) body(std::false_type{});
+    else body(std::true_type{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    const int lane_out = qt_lane();
+    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
+#endif
+}
+
+// The splits of K added in order, the first one from `first` (dst itself or a plane), the others from planes; n % 4 == 0.  Bound by the latency of the reads at
+// the sizes that are split: four planes are on their way at a time, and a workgroup is small enough that 32 x 4096 results fill the chip.
+constexpr int QT_RT = 128;
+template <int ODT>
+__global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first, int64_t ld_first, const float *__restrict__ planes, void *dst, int splits, int64_t n,
+                                                             int64_t stride_dst, int64_t count) {
+    const int64_t i = ((int64_t)blockIdx.x * QT_RT + threadIdx.x) * 4;
+    if (i >= count) return;
+    const int64_t r = i / n, c0 = i - r * n, o = r * stride_dst + c0;
+    float a[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) a[c] = first[r * ld_first + c0 + c];
+    for (int p = 0; p < splits - 1; p += 4) {
+        f32x4 b[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) b[u] = *reinterpret_cast<const f32x4 *>(planes + min(p + u, splits - 2) * count + i);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (p + u < splits - 1)
+#pragma unroll
+                for (int c = 0; c < 4; c++) a[c] += b[u][c];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        if (ODT == CQ_F32) ((float *)dst)[o + c] = a[c];
+        else ((uint16_t *)dst)[o + c] = ODT == CQ_F16 ? f2h_bits(a[c]) : f2bf_bits(a[c]);
+    }
+}
+
+template <int DT>
+int qtile_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
+             const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
+#define QT_GO(M, E)                                                                                                                                  \
+    static_assert(QtLds<DT, M>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                 \
+    return qtile_go(qtile_kernel<DT, M, E>, QtLds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+    if (moe) {
+        if (mi == 1) { QT_GO(1, true); }
+        QT_GO(4, true);
+    }
+    switch (mi) {
+        case 1: { QT_GO(1, false); }
+        case 2: { QT_GO(2, false); }
+        case 3: { QT_GO(3, false); }
+        default: { QT_GO(4, false); }
+    }
+#undef QT_GO
+}
+
+int qtile_any(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
+              int64_t stride_dst, const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
+    switch (w_dtype) {
+        case CQ_Q4K: return qtile_mi<CQ_Q4K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+        case CQ_Q5K: return qtile_mi<CQ_Q5K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+        case CQ_Q6K: return qtile_mi<CQ_Q6K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+    }
+    return CQ_ERR_DTYPE;
+}
+
+}  // namespace
+
+bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
+    if (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K) return k % 256 == 0;
+    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one
+    return w_dtype == CQ_Q6K && k % 256 == 0 && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
+}
+
+// Bytes of split planes that a call may use, not falling with the rows.
+static constexpr int64_t QT_PLANE_FLOATS = 12 << 20;
+int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
+    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K) || n % 4 || k < 512 || k % 256) return 0;
+    return cq_align256(std::min<int64_t>(16 * rows * n, QT_PLANE_FLOATS) * 4);
+}
+
+// Rows of the tile (32 mi) and K splits: the pair for which the model
+//   rounds * (super-blocks per split * (a + b mi) + 1.3) us,  + 6.8 us and the planes at 4.5 TB/s where K is split
+// is least.  A round is 256 workgroups (a tenth slower when all compute units are busy: the clock falls), a the conversion of the weights, b the products
+// and sums of 32 rows.  Fitted to 3800 launches of 17 - 2048 rows against [14336 x 4096], [4096 x 14336], [1024 x 4096] and [5120 x 4096] (6 % rms); the choice it makes is 0.2 - 1.2 % slower than the best of all pairs on average, at most 16 % (100 rows of Q4_K: 39.1 against 33.8 us).
+struct QtPlan { int mi, splits; };
+static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_t most_splits) {
+    const int64_t nsb = k / 256, nt = (n + 32 * QT_NW - 1) / (32 * QT_NW);
+    const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : 2.4;
+    const double b = w_dtype == CQ_Q6K ? 0.65 : 0.79, plane = (double)rows * n * 4;
+    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({16, nsb / 2, most_splits}));
+    QtPlan best{4, 1};
+    double least = 1e30;
+    for (int mi = 1; mi <= 4; mi++)
+        for (int sp = 1; sp <= most; sp++) {
+            const int64_t wgs = (rows + 32 * mi - 1) / (32 * mi) * nt * sp, rounds = (wgs + 255) / 256;
+            const double load = 1.1 * (rounds - 1) + 1.0 + 0.1 * (double)(wgs - 256 * (rounds - 1)) / 256;
+            const double t = load * ((double)((nsb + sp - 1) / sp) * (a + b * mi) + 1.3) + (sp > 1 ? 6.8 + (sp + 1) * plane / 4.5e6 : 0.0);
+            if (t < least) { least = t; best = {mi, sp}; }
+        }
+    return best;
+}
+
+int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst, void *planes,
+                    int64_t plane_bytes, hipStream_t s) {
+    // an f32 dst takes the first split itself
+    const bool f32 = dst_dtype == CQ_F32;
+    const QtPlan plan = qtile_plan(w_dtype, k, n, rows, planes ? (f32 ? 1 : 0) + plane_bytes / (4 * rows * n) : 1);
+    const int splits = plan.splits;
+    const dim3 grid((unsigned)((rows + 32 * plan.mi - 1) / (32 * plan.mi)), (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)), (unsigned)splits);
+    if (grid.y > 65535) return CQ_ERR_RANGE;
+    const int64_t count = rows * n;
+    const bool direct = splits == 1 || f32;
+    void *const first = direct ? dst : planes;
+    const int64_t ld = direct ? stride_dst : n;
+    float *const others = direct ? (float *)planes : (float *)planes + count;
+    const MoeChunks none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+    const int rc = qtile_any(w_dtype, plan.mi, false, grid, w, av, first, direct ? dst_dtype : CQ_F32, k, n, rows, ld, none, 0, others, s);
+    if (rc || splits == 1) return rc;
+    const dim3 rg((unsigned)((count / 4 + QT_RT - 1) / QT_RT));
+    if (f32) hipLaunchKernelGGL(qtile_reduce_kernel<CQ_F32>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
+    else if (dst_dtype == CQ_F16) hipLaunchKernelGGL(qtile_reduce_kernel<CQ_F16>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
+    else hipLaunchKernelGGL(qtile_reduce_kernel<CQ_BF16>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
+    return (int)hipGetLastError();
+}
+
+// tile_rows: rows of one chunk of the table, 32 or 128
+int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s) {
+    const dim3 grid((unsigned)mc.max_chunks, (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)));
+    if (grid.y > 65535) return CQ_ERR_RANGE;
+    return qtile_any(w_dtype, tile_rows / 32, true, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
+}

@@ -1,0 +1,98 @@
+"""The prefill kernels of cq_qtile.hip where they can go wrong, against the CPU oracle.
+
+Bound: the sums of 256 elements are exact integers on both sides; what differs is f32 rounding of three operations per block and the
+order of a split, nblocks <= 448 of them: below sqrt(448) * 3 * 2^-24 = 3.8e-6 of the terms' norm.  That norm is ||x|| ||w|| / sqrt(k), what a dot product
+of such vectors has on average: a single result may cancel to far less, and its error does not with it.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from candle_amd import _lib
+from tests.util import normal
+
+pytestmark = pytest.mark.gpu
+BOUND = 4e-6
+FMT = {"q4k": (12, oracle.Q4K), "q5k": (13, oracle.Q5K), "q6k": (14, oracle.Q6K)}
+OUT = {0: torch.float32, 1: torch.float16, 30: torch.bfloat16}
+
+
+def run(code, blocks, x, n, out=0, shift=0):
+    """cq_qmatmul_forward of x [m, k] with the weights `shift` bytes past a 256-byte boundary, the result between two rows of canaries."""
+    L = _lib.lib()
+    m, k = x.shape
+    raw = torch.zeros(len(blocks) + 512, dtype=torch.uint8, device="cuda")
+    raw[shift:shift + len(blocks)] = torch.from_numpy(blocks).cuda()
+    xd = torch.from_numpy(x).cuda()
+    y = torch.full((m + 2, n), 77.0, dtype=OUT[out], device="cuda")
+    nb = L.cq_qmatmul_workspace_bytes(code, m, k, n)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    rc = L.cq_qmatmul_forward(code, raw.data_ptr() + shift, ctypes.c_void_p(xd.data_ptr()), 0, ctypes.c_void_p(y[1].data_ptr()), out, m, k, n,
+                              ctypes.c_void_p(ws.data_ptr()), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    _lib.check("cq_qmatmul_forward", rc)
+    torch.cuda.synchronize()
+    y = y.float().cpu().numpy()
+    assert (y[0] == 77).all() and (y[-1] == 77).all()
+    return y[1:-1]
+
+
+def row_error(got, want, x, w, k):
+    """Largest error of a row [m, n] relative to the norm that rows x against the weights w have on average."""
+    size = np.linalg.norm(x.astype(np.float64), axis=1) * np.linalg.norm(w.astype(np.float64)) / np.sqrt(k)
+    return float((np.linalg.norm(got.astype(np.float64) - want, axis=1) / size).max())
+
+
+def check(fmt, m, n, k, out=0, shift=0):
+    print(f"case {fmt} m={m} n={n} k={k} out={out} shift={shift}", flush=True)
+    code, odt = FMT[fmt]
+    w = normal(7 + m, (n, k), 0.02)
+    blocks = oracle.from_float(odt, w.reshape(-1))
+    x = normal(9 + n, (m, k))
+    got, want = run(code, blocks, x, n, out, shift), oracle.matmul(odt, x, blocks, n)
+    eps = {0: 0.0, 1: 2.0 ** -11, 30: 2.0 ** -8}[out]                # one rounding to the output type
+    excess = np.maximum(np.abs(got - want) - eps * np.abs(want) - (2.0 ** -25 if out == 1 else 0), 0)        # (f16 results below 2^-14 are multiples of 2^-24)
+    assert row_error(excess, 0, x, w, k) <= BOUND
+
+
+@pytest.mark.parametrize("fmt", FMT)
+@pytest.mark.parametrize("m,n,k", [(66, 256, 256), (65, 1, 512), (97, 257, 768), (128, 31, 2304), (129, 260, 1280), (70, 292, 14336), (300, 510, 512)])
+def test_tile_edges(fmt, m, n, k):
+    # one row past a 32-row tile, one column past a workgroup's 256, one super-block, odd numbers of them, k split over workgroups (n % 4 == 0) and not;
+    # Q6_K with an odd number of blocks (n k / 256 odd) takes the general kernel
+    check(fmt, m, n, k)
+
+
+@pytest.mark.parametrize("fmt", FMT)
+@pytest.mark.parametrize("out", [1, 30])
+@pytest.mark.parametrize("n,k", [(130, 512), (260, 4096)])
+def test_half_results(fmt, out, n, k):
+    check(fmt, 67, n, k, out)                              # written by the product itself, and by the sum over the splits
+
+
+@pytest.mark.parametrize("fmt,shift", [("q6k", 2), ("q6k", 4), ("q4k", 16), ("q5k", 48)])
+def test_weights_at_other_addresses(fmt, shift):
+    check(fmt, 66, 96, 768, shift=shift)                   # Q6_K off 4 bytes: the general kernel
+
+
+@pytest.mark.parametrize("fmt", ["q6k", "q5k"])
+@pytest.mark.parametrize("tokens", [70, 1200])
+def test_grouped_experts(fmt, tokens):
+    """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row."""
+    import candle_amd as ca
+    code, odt = FMT[fmt]
+    E, n, k, topk = 5, 268, 768, 2
+    w = normal(21, (E, n, k), 0.02)
+    blocks = oracle.from_float(odt, w.reshape(-1))
+    qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(odt)), (E, n, k))
+    x = normal(22, (tokens, 1, k))
+    ids = np.random.default_rng(5).integers(0, E, (tokens, topk)).astype(np.uint32)
+    ids[: tokens // 2, 0] = 3
+    got = qt.indexed_moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids.astype(np.int32)).cuda()).cpu().numpy()
+    per = len(blocks) // E
+    for e in range(E):
+        t, s = np.nonzero(ids == e)
+        want = oracle.matmul(odt, x[t, 0], blocks[e * per:(e + 1) * per], n)
+        assert row_error(got[t, s], want, x[t, 0], w[e], k) <= BOUND
