@@ -26,7 +26,7 @@ LIB = os.path.join(HERE, "libcandle_hip_quant.so")
 LIB_MIXER = os.path.join(HERE, "libcandle_hip_mixer.so")
 LIB_BENCH = os.path.join(HERE, "libcq_bench.so")
 
-SOURCES = ["cq_api.hip", "cq_dequant.hip", "cq_actquant.hip", "cq_matvec.hip", "cq_matmul.hip", "cq_qtile.hip", "cq_moe.hip", "cq_quantize.hip", "cq_nn.hip", "cq_layer.hip", "cq_matvec_batch.hip", "cq_status.hip"]
+SOURCES = ["cq_api.hip", "cq_dequant.hip", "cq_actquant.hip", "cq_matvec.hip", "cq_matmul.hip", "cq_qtile.hip", "cq_qtile0.hip", "cq_moe.hip", "cq_quantize.hip", "cq_nn.hip", "cq_layer.hip", "cq_matvec_batch.hip", "cq_status.hip"]
 # models with bfloat16 weights: dense products and sequence mixers, with the glue of cq_nn.hip; complete without the library above, so
 # that such a model can run without compiling the quantized kernels
 MIXER_SOURCES = ["cq_nn.hip", "cq_status.hip", "cq_dense.hip", "cq_mix_glue.hip", "cq_mix_attention.hip", "cq_mix_state.hip", "cq_mix_latent.hip", "cq_mix_moe.hip"]

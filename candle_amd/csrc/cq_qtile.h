@@ -1,4 +1,4 @@
-// Prefill kernels over quantized weights (cq_qtile.hip): the workgroup's shape, the way results go out, the launch.
+// What the prefill kernels over quantized weights share (cq_qtile.hip: K-quants, cq_qtile0.hip: Q4_0 and Q8_0): the workgroup's shape, the way results go out, the launch.
 #pragma once
 #include "cq_device.h"
 #include "cq_fmt.h"
@@ -59,3 +59,7 @@ inline int qtile_go(QtFn fn, int lds_bytes, dim3 grid, const void *w, const ActV
 }
 
 }  // namespace
+
+// Q4_0 and Q8_0 (cq_qtile0.hip): one launch with tiles of 32 mi rows, K split over grid.z
+int cq_qtile0_launch(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
+                     int64_t stride_dst, const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s);

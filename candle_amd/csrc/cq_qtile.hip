@@ -1,4 +1,5 @@
-// Prefill matmul of Q4_K, Q5_K and Q6_K over pre-quantized activations (Q8_K blocks) on the int8 matrix cores of gfx950:   dst[m, n] = sum_k x^[m, k] * W^[n, k]
+// Prefill matmul of Q4_K, Q5_K and Q6_K over pre-quantized activations (Q8_K blocks) on the int8 matrix cores of gfx950, and the choice of tile and split
+// that Q4_0 and Q8_0 (cq_qtile0.hip) share:   dst[m, n] = sum_k x^[m, k] * W^[n, k]
 //
 // Per super-block of 256 elements the exact integer S[m,n] = sum_k q8[m,k] * (scale[n, sub(k)] * q[n,k]) of the CPU's dot products (k_quants.rs:1460-1540,
 // 1714-1801, 2035-2092), then acc += d8 * (d * S - dmin * M), M the products of the 16-element sums with the mins (one f16 MFMA, exact).  scale * q has up to
@@ -437,13 +438,14 @@ int qtile_any(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const Act
         case CQ_Q5K: return qtile_mi<CQ_Q5K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
         case CQ_Q6K: return qtile_mi<CQ_Q6K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
     }
-    return CQ_ERR_DTYPE;
+    return cq_qtile0_launch(w_dtype, mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
 }
 
 }  // namespace
 
 bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
     if (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K) return k % 256 == 0;
+    if (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) return k % 256 == 0 && ((uintptr_t)w & 15) == 0;      // (rows are multiples of 16 bytes)
     // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one
     return w_dtype == CQ_Q6K && k % 256 == 0 && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
 }
@@ -451,19 +453,20 @@ bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
 // Bytes of split planes that a call may use, not falling with the rows.
 static constexpr int64_t QT_PLANE_FLOATS = 12 << 20;
 int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
-    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K) || n % 4 || k < 512 || k % 256) return 0;
+    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K && w_dtype != CQ_Q4_0 && w_dtype != CQ_Q8_0) || n % 4 || k < 512 || k % 256) return 0;
     return cq_align256(std::min<int64_t>(16 * rows * n, QT_PLANE_FLOATS) * 4);
 }
 
 // Rows of the tile (32 mi) and K splits: the pair for which the model
 //   rounds * (super-blocks per split * (a + b mi) + 1.3) us,  + 6.8 us and the planes at 4.5 TB/s where K is split
 // is least.  A round is 256 workgroups (a tenth slower when all compute units are busy: the clock falls), a the conversion of the weights, b the products
-// and sums of 32 rows.  Fitted to 3800 launches of 17 - 2048 rows against [14336 x 4096], [4096 x 14336], [1024 x 4096] and [5120 x 4096] (6 % rms); the choice it makes is 0.2 - 1.2 % slower than the best of all pairs on average, at most 16 % (100 rows of Q4_K: 39.1 against 33.8 us).
+// and sums of 32 rows.  Fitted to 3800 launches of 17 - 2048 rows against [14336 x 4096], [4096 x 14336], [1024 x 4096] and [5120 x 4096] (6 % rms, 10 % for
+// Q4_0); the choice it makes is 0.2 - 1.2 % slower than the best of all pairs on average, at most 16 % (100 rows of Q4_K: 39.1 against 33.8 us).
 struct QtPlan { int mi, splits; };
 static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_t most_splits) {
     const int64_t nsb = k / 256, nt = (n + 32 * QT_NW - 1) / (32 * QT_NW);
-    const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : 2.4;
-    const double b = w_dtype == CQ_Q6K ? 0.65 : 0.79, plane = (double)rows * n * 4;
+    const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : w_dtype == CQ_Q6K ? 2.4 : 1.6;
+    const double b = w_dtype == CQ_Q6K ? 0.65 : cq_is_kquant(w_dtype) ? 0.79 : 1.23, plane = (double)rows * n * 4;
     const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({16, nsb / 2, most_splits}));
     QtPlan best{4, 1};
     double least = 1e30;

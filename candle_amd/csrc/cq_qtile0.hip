@@ -1,0 +1,243 @@
+// Prefill matmul of Q4_0 and Q8_0 over pre-quantized activations (Q8_0 blocks) on the int8 matrix cores of gfx950:
+//   dst[m, n] = sum over blocks b of (sum of 32 q8[m, k] * q[n, k]) * d[n, b] * d8[m, b]
+//
+// Both operands carry a scale per 32 elements, so one v_mfma_i32_32x32x32_i8 is one block of 32 x 32 results, each of which the vector units scale and
+// add: they are the bound (two instructions per result and block, against one matrix instruction per 1024).  The usual three are convert, times d[n], fma with
+// d8[m].  Here the sums start from 0x4b400000 instead of zero: read as f32 that is F = 12582912 + S exactly (|S| < 2^22), and
+// fma(F, d, -12582912 d) rounds S * d once, like the product of the converted sum: 12582912 = 3 * 2^22 and d has 11 bits, so the offset is exact.  The
+// results are those of the CPU's order of operations (k_quants.rs:294-311, 720-738).
+//
+// A workgroup's eight waves lie side by side along n and share 32 MI rows of activations in LDS (two super-blocks of 256, swizzled so that fragments are read
+// without bank conflicts); a wave owns 32 weight rows, brings their blocks for itself by copies to LDS, half a super-block at a time, and converts each
+// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  (The kernel that this
+// replaces for these formats shared weights and activations between 2 x 2 waves, converted every weight twice or four times and waited at two barriers per 64
+// elements.)  K is split over grid.z where that fills the chip better; see qtile_plan.
+//
+// [14336 x 4096], us, before / now, quantizing the activations included:   17 rows   131 rows   512 rows   2048 rows
+//   Q4_0                                                                  27.7 23.7  84.5 57.0  155 111    548 415
+//   Q8_0                                                                  27.1 23.9  82.0 61.0  144 121    515 468
+// 2048 rows of Q4_0 are 580 TOP/s: the two vector instructions per result and block take 1.1 us per super-block and 32 rows, the matrix cores half of that.
+#include "cq_qtile.h"
+
+namespace {
+
+// PPR: 16-byte pieces that cover four blocks of a row (128 elements, half a super-block) and the 8 bytes behind the first half, before the second
+template <int DT> struct Q0Tile;
+template <> struct Q0Tile<CQ_Q4_0> { static constexpr int BB = 18, PPR = 5; };
+template <> struct Q0Tile<CQ_Q8_0> { static constexpr int BB = 34, PPR = 9; };
+
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));       // (LDS reads on 2 bytes)
+
+constexpr uint32_t Q0_MAGIC = 0x4b400000u;                 // 12582912.0f
+template <int DT, int MI> struct Q0Lds {
+    static constexpr int NI = (32 * Q0Tile<DT>::PPR + 63) / 64;          // copy instructions per wave and half of weights
+    static constexpr int A = MI * 8192, B = NI * 1024, D8 = 8 * 32 * MI * 4;
+    static constexpr int A_OFF = 0, B_OFF = 2 * A, D8_OFF = B_OFF + 2 * QT_NW * B, BYTES = D8_OFF + 2 * D8;
+};
+
+template <int DT, int MI, bool MOE>
+__global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
+                                                               int rows, int64_t stride_dst, MoeChunks mc, int64_t expert_bytes, float *__restrict__ planes) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler has no use for the body, and does not know its buffer accesses)
+    typedef Q0Tile<DT> T;
+    typedef Q0Lds<DT, MI> LD;
+    constexpr int BB = T::BB, NI = LD::NI, RS = 16 * T::PPR, BM = 32 * MI, BN = 32 * QT_NW, NA = MI, ND = (8 * MI * 32 / 64 + QT_NW - 1) / QT_NW;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nr = lane & 31, kg = lane >> 5;
+    int m0 = blockIdx.x * BM;
+    const int n0 = blockIdx.y * BN + 32 * wv;
+    if (MOE) {
+        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
+        m0 = mc.first[blockIdx.x];
+        rows = m0 + mc.count[blockIdx.x];
+        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+    }
+    const int nsb_all = k >> 8;
+    const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
+    const int64_t row_bytes = (int64_t)nsb_all * (8 * BB);
+
+    // ---- weights: piece p of a half is 16-byte piece p % PPR of row p / PPR; rows past the end repeat the last one, pieces past the end the last piece.
+    // The first half's pieces begin where the super-block begins, the second's end where it ends: nothing outside it is read ----
+    const int wbase = min(n0, n - 1), wrows = min(32, n - wbase);
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(w + wbase * row_bytes), 0, -1, 0x00020000);
+    uint32_t w_off[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int p = min(64 * i + lane, 32 * T::PPR - 1), r = p / T::PPR;
+        w_off[i] = (uint32_t)(min(r, wrows - 1) * row_bytes) + 16 * (p - r * T::PPR);
+    }
+    uint8_t *const myB = lds + LD::B_OFF + wv * (2 * LD::B);
+    // (where this lane's row begins, with nothing known of its alignment: pieces at multiples of four bytes would be read as pairs of dwords)
+    uint32_t my_row = LD::B_OFF + wv * (2 * LD::B) + nr * RS;
+    asm volatile("" : "+v"(my_row));
+    auto issue_w = [&](int kb, int h) {
+        kb = min(kb, kb1 - 1);
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + h * LD::B + 1024 * i), 16, w_off[i], kb * (8 * BB) + h * (4 * BB - 8), 0, 0);
+    };
+    // ---- activations: [4 stages][32 MI rows][64 bytes], piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
+    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
+    uint32_t a_off[NA];
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+        const int blk = wv + QT_NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
+        a_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)k + 64 * st + 16 * p;
+    }
+    // ---- their scales: [8 blocks][32 MI rows], instruction i of a wave brings 64 of them ----
+    const __amdgpu_buffer_rsrc_t drs = __builtin_amdgcn_make_buffer_rsrc((void *)(av.d + (int64_t)m0 * (16 * nsb_all)), 0, -1, 0x00020000);
+    uint32_t d_off[ND];
+    int d_dst[ND];
+#pragma unroll
+    for (int i = 0; i < ND; i++) {
+        const int first = 64 * min(wv + QT_NW * i, 8 * BM / 64 - 1), at = first + lane, b = at / BM, r = at - b * BM;
+        d_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)(64 * nsb_all) + 8 * b;
+        d_dst[i] = 4 * first;
+    }
+    auto request = [&](int j) {
+        const int kb = min(kb0 + j, kb1 - 1), slot = j & 1;
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (cq_lds_void *)(lds + LD::A_OFF + slot * LD::A + 1024 * (wv + QT_NW * i)), 16, a_off[i], kb * 256, 0, 0);
+#pragma unroll
+        for (int i = 0; i < ND; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(drs, (cq_lds_void *)(lds + LD::D8_OFF + slot * LD::D8 + d_dst[i]), 4, d_off[i], kb * 64, 0, 0);
+        asm volatile("" ::: "memory");
+    };
+
+    f32x16 acc[MI];
+    i32x16 magic;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) magic[e] = (int)Q0_MAGIC;
+    asm volatile("" : "+v"(magic));                       // (in registers, not rebuilt for every block)
+
+    request(0);
+    issue_w(kb0, 0);
+    const int nsb = kb1 - kb0;
+    bool wild = false;
+    const int live = MOE ? (rows - m0 + 31) / 32 : MI;
+    const uint32_t nib = 4 - 4 * kg;                       // Q4_0: the lower lanes take the low nibbles
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    for (int j = 0; j < nsb; j++) {
+        const int kb = kb0 + j, slot = j & 1;
+        if (j > 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        issue_w(kb, 1);
+        request(j + 1);
+        const uint8_t *const Aj = lds + LD::A_OFF + slot * LD::A + nr * 64, *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 16 * kg;
+        // this lane's 16 weights of block b, and the block's scale
+        auto operand = [&](int b, i32x4 &op, float &dw) {
+            const uint8_t *const blk = lds + my_row + ((b >> 2) * (LD::B + 8) + (b & 3) * BB);
+            dw = h2f(*reinterpret_cast<const uint16_t *>(blk));
+            if constexpr (DT == CQ_Q4_0) {
+                // nibbles as 16 (q - 8): the high ones where they are, the low ones moved up
+                const u32x4 q = *reinterpret_cast<const u32x4_at2 *>(blk + 2);
+                dw *= 0.0625f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) op[i] = (int)(((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u);
+            } else {
+                op = __builtin_bit_cast(i32x4, (u32x4)*reinterpret_cast<const u32x4_at2 *>(blk + 2 + 16 * kg));
+            }
+        };
+        auto a_frag = [&](int b, int t) {
+            return *reinterpret_cast<const i32x4 *>(Aj + (b >> 1) * (MI * 2048) + t * 2048 + 16 * ((2 * (b & 1) + kg) ^ ((nr >> 2) & 3)));
+        };
+        // The sums of block b + 1 are on their way in the matrix cores while those of block b are scaled, tile by tile.
+        i32x4 op;
+        float dw;
+        i32x16 S[MI];
+        operand(0, op, dw);
+#pragma unroll
+        for (int t = 0; t < MI; t++)
+            if (!MOE || t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_frag(0, t), op, magic, 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
+            if (b == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+            if (b == 4) issue_w(kb + 1, 0);
+            const float c = -12582912.0f * dw;
+            wild |= !(__builtin_fabsf(dw) < __builtin_inff());
+            i32x4 op_n;
+            float dw_n = 0.0f;
+            if (b < 7) operand(b + 1, op_n, dw_n);
+#pragma unroll
+            for (int t = 0; t < MI; t++) {
+                if (MOE && t >= live) break;
+                f32x4 d8[4];
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) d8[e4] = *reinterpret_cast<const f32x4 *>(Dj + 4 * (b * BM + t * 32 + 8 * e4));
+                i32x4 af;
+                if (b < 7) af = a_frag(b + 1, t);
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw, c), d8[e >> 2][e & 3], acc[t][e]);
+                qt_pin(acc[t]);
+                if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, op_n, magic, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            op = op_n;
+            dw = dw_n;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // A scale that is not finite (a file's: no quantizer of finite values writes one) spoils the offset: once more, with the sums themselves, which may be
+    // zero or negative.
+    if (__builtin_amdgcn_ballot_w64(wild) != 0) {
+        const uint8_t *const wr = w + (int64_t)min(n0 + nr, n - 1) * row_bytes;
+#pragma unroll 1
+        for (int t = 0; t < live; t++) {
+            f32x16 a[1];
+#pragma unroll
+            for (int e = 0; e < 16; e++) a[0][e] = 0.0f;
+#pragma unroll 1
+            for (int g = 8 * kb0; g < 8 * kb1; g++) {
+                const uint8_t *const blk = wr + (int64_t)g * BB;
+                const float dg = h2f(ld_u<uint16_t>(blk)) * (DT == CQ_Q4_0 ? 0.0625f : 1.0f);
+                u32x4 q = ld_u<u32x4>(blk + 2 + (DT == CQ_Q4_0 ? 0 : 16 * kg));
+                if (DT == CQ_Q4_0) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) q[i] = ((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u;
+                }
+                const i32x4 af = *reinterpret_cast<const i32x4 *>(av.qs + (int64_t)min(m0 + 32 * t + nr, rows - 1) * k + 32 * g + 16 * kg);
+                i32x16 S;
+#pragma unroll
+                for (int e = 0; e < 16; e++) S[e] = 0;
+                S = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(i32x4, q), S, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int64_t mm = min(m0 + t * 32 + 8 * (e >> 2) + 4 * kg + (e & 3), rows - 1);
+                    a[0][e] = fmaf((float)S[e] * dg, av.d[2 * (mm * (8 * nsb_all) + g)], a[0][e]);
+                }
+            }
+            qt_store<1, MOE>(a, dst, dst_dtype, m0 + 32 * t, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+        }
+        return;
+    }
+    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+#endif
+}
+
+}  // namespace
+
+template <int DT>
+static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
+                     const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
+#define Q0_GO(M, E) return qtile_go(qtile0_kernel<DT, M, E>, Q0Lds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+    if (moe) { if (mi == 1) Q0_GO(1, true); else Q0_GO(4, true); }
+    switch (mi) {
+        case 1: Q0_GO(1, false);
+        case 2: Q0_GO(2, false);
+        case 3: Q0_GO(3, false);
+        default: Q0_GO(4, false);
+    }
+#undef Q0_GO
+}
+
+int cq_qtile0_launch(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
+                     int64_t stride_dst, const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
+    return w_dtype == CQ_Q4_0 ? launch_mi<CQ_Q4_0>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+                              : launch_mi<CQ_Q8_0>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+}

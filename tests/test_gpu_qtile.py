@@ -1,6 +1,6 @@
-"""The prefill kernels of cq_qtile.hip where they can go wrong, against the CPU oracle.
+"""The prefill kernels of cq_qtile.hip and cq_qtile0.hip where they can go wrong, against the CPU oracle.
 
-Bound: the sums of 256 elements are exact integers on both sides; what differs is f32 rounding of three operations per block and the
+Bound: the sums of 32 (Q4_0, Q8_0) and 256 elements are exact integers on both sides; what differs is f32 rounding of 1.5 - 2.5 operations per block and the
 order of a split, nblocks <= 448 of them: below sqrt(448) * 3 * 2^-24 = 3.8e-6 of the terms' norm.  That norm is ||x|| ||w|| / sqrt(k), what a dot product
 of such vectors has on average: a single result may cancel to far less, and its error does not with it.
 """
@@ -12,11 +12,11 @@ import torch
 
 import oracle
 from candle_amd import _lib
-from tests.util import normal
+from tests.util import normal, rel_l2
 
 pytestmark = pytest.mark.gpu
 BOUND = 4e-6
-FMT = {"q4k": (12, oracle.Q4K), "q5k": (13, oracle.Q5K), "q6k": (14, oracle.Q6K)}
+FMT = {"q4_0": (2, oracle.Q4_0), "q8_0": (8, oracle.Q8_0), "q4k": (12, oracle.Q4K), "q5k": (13, oracle.Q5K), "q6k": (14, oracle.Q6K)}
 OUT = {0: torch.float32, 1: torch.float16, 30: torch.bfloat16}
 
 
@@ -72,12 +72,30 @@ def test_half_results(fmt, out, n, k):
     check(fmt, 67, n, k, out)                              # written by the product itself, and by the sum over the splits
 
 
-@pytest.mark.parametrize("fmt,shift", [("q6k", 2), ("q6k", 4), ("q4k", 16), ("q5k", 48)])
+@pytest.mark.parametrize("fmt,shift", [("q4_0", 2), ("q4_0", 8), ("q8_0", 6), ("q8_0", 16), ("q6k", 2), ("q6k", 4), ("q4k", 16), ("q5k", 48)])
 def test_weights_at_other_addresses(fmt, shift):
-    check(fmt, 66, 96, 768, shift=shift)                   # Q6_K off 4 bytes: the general kernel
+    check(fmt, 66, 96, 768, shift=shift)                   # Q4_0 / Q8_0 off 16 bytes, Q6_K off 4: the general kernels
 
 
-@pytest.mark.parametrize("fmt", ["q6k", "q5k"])
+@pytest.mark.parametrize("fmt,bb", [("q4_0", 18), ("q8_0", 34)])
+@pytest.mark.parametrize("d", [np.inf, -np.inf, np.nan, 65504.0, 6e-8])
+def test_extreme_block_scales(fmt, bb, d):
+    """The scale of one block infinite, NaN, the largest and the smallest: the same values, infinities and NaN as the oracle's sums."""
+    code, odt = FMT[fmt]
+    n, k, m = 96, 512, 70
+    blocks = oracle.from_float(odt, normal(3, (n, k), 0.02).reshape(-1)).reshape(n, k // 32, bb)
+    blocks[[0, 40, 95], [0, 7, 15], :2] = np.frombuffer(np.float16(d).tobytes(), dtype=np.uint8)
+    x = normal(4, (m, k))
+    x[5, :32] = 0.0                                        # a sum of zero times an infinite scale
+    want = oracle.matmul(odt, x, blocks.reshape(-1), n)
+    got = run(code, blocks.reshape(-1), x, n)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.array_equal(got[~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)])
+    assert rel_l2(got[ok], want[ok]) <= BOUND
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q6k", "q5k"])
 @pytest.mark.parametrize("tokens", [70, 1200])
 def test_grouped_experts(fmt, tokens):
     """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row."""
