@@ -218,6 +218,135 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
     }
 }
 
+// ---- bf16 tiles of 256 activation rows x 256 weight rows, for products that fill the chip with them ------------------------------
+// The 128 x 128 tile reads a byte of LDS for every 64 multiply-adds and one of L2 for every 128: both are as slow as the matrix cores at 60 % of their rate.  Here
+// eight waves, 2 x 4, of 128 x 64 results each need two thirds and half of that.  LDS holds two stages of 64 of k: weights and bf16 activations go there by
+// copies that no register sees, f32 activations through registers, rounded on the way.  One barrier a stage, taken between the third and the last quarter of
+// its products: their operands are in registers by then, and those of the next stage's first quarter arrive under them.
+// LDS rows are 128 bytes in eight 16-byte chunks, chunk c of row r at c ^ (r / 2) % 8: 16 rows of a chunk lie in all 64 banks (c ^ r % 8 takes twice as long).
+// 2048 x 7168 x 2048: bf16 activations 80 -> 59 us (1020 TFLOP/s), f32 90 -> 72; 4096 x 4096 x 4096: 154 -> 113 (1220) and 176 -> 138.  Of the 59 about 11 are
+// the way to the first products and the stores; with f32 activations the loads that are to be rounded wait behind those of the stage before.
+// The copies are buffer loads: beside copies by address the compiler waits for all LDS reads at once.
+constexpr int DT_B = 256, DT_A = DT_B * 128, DT_STAGE = 2 * DT_A;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void dt_lds;
+
+template <bool XB>
+__global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tm, tn;
+    tile_at(xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
+    const int64_t m0 = (int64_t)tm * DT_B;
+    const int n0 = tn * DT_B, nst = K >> 6, wm = (wv >> 2) * 128, wn = (wv & 3) * 64, lr = lane & 31, kg = lane >> 5;
+
+    // ---- instruction i of a wave brings the eight rows 8 (wv + 8 i) .. of a stage, one 16-byte chunk (of bf16) a lane; rows past the end repeat the last ----
+    const uint8_t *const xbase = reinterpret_cast<const uint8_t *>(src.x) + m0 * src.ldx * (XB ? 2 : 4);
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(src.w + (int64_t)n0 * src.ldw), 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *)xbase, 0, -1, 0x00020000);
+    uint32_t w_off[4], x_off[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int row = 8 * (wv + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        w_off[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)(2 * src.ldw) + 16 * c;
+        // (f32 activations: chunk lane % 8, swizzled when it is written)
+        x_off[i] = (uint32_t)min((int64_t)row, M - 1 - m0) * (uint32_t)((XB ? 2 : 4) * src.ldx) + (XB ? 16 * c : 32 * (lane & 7));
+    }
+    auto copy = [&](int st) {                              // what goes by copies, of stage st (past the last one: that one again, into a place nobody reads)
+        uint8_t *const to = lds + (st & 1) * DT_STAGE + 1024 * wv;
+        const int at = 128 * min(st, nst - 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (XB) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (dt_lds *)(to + 8192 * i), 16, x_off[i], at, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (dt_lds *)(to + DT_A + 8192 * i), 16, w_off[i], at, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    };
+    f32x4 xr[4][2];                                        // f32 activations of the stage after the next
+    auto fetch = [&](int st) {
+        if constexpr (!XB) {
+            const uint8_t *const from = xbase + 256 * min(st, nst - 1);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) xr[i][j] = *reinterpret_cast<const f32x4 *>(from + x_off[i] + 16 * j);
+        }
+    };
+    auto put_x = [&](int st) {
+        if constexpr (!XB) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int row = 8 * (wv + 8 * i) + (lane >> 3);
+                *reinterpret_cast<bf16x8 *>(lds + (st & 1) * DT_STAGE + row * 128 + 16 * ((lane & 7) ^ ((row >> 1) & 7))) = round_bf16(xr[i][0], xr[i][1]);
+            }
+        }
+    };
+    // Barrier b: stage b is there for everybody, and nobody reads stage b - 1 any more: stage b + 1 may take its place.
+    auto sync = [&]() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    auto request = [&](int b) {
+        put_x(b + 1);
+        fetch(b + 2);
+        copy(b + 1);
+    };
+    f32x16 acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+    const uint32_t a_at = (wm + lr) * 128 + 16 * (kg ^ ((lr >> 1) & 7)), b_at = DT_A + (wn + lr) * 128 + 16 * (kg ^ ((lr >> 1) & 7));
+    bf16x8 fa[2][4], fb[2][2];
+    auto operands = [&](int st, int s) {                   // of quarter s of the stage, into set s % 2
+        const uint8_t *const from = lds + (st & 1) * DT_STAGE;
+#pragma unroll
+        for (int i = 0; i < 2; i++) fb[s & 1][i] = *reinterpret_cast<const bf16x8 *>(from + ((b_at + 4096 * i) ^ (32 * s)));
+#pragma unroll
+        for (int i = 0; i < 4; i++) fa[s & 1][i] = *reinterpret_cast<const bf16x8 *>(from + ((a_at + 4096 * i) ^ (32 * s)));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[s & 1][j], fa[s & 1][i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    fetch(0);
+    copy(0);
+    put_x(0);
+    fetch(1);
+    sync();
+    operands(0, 0);
+    request(0);
+    for (int st = 0; st < nst; st++) {
+#pragma unroll
+        for (int s = 0; s < 3; s++) {
+            operands(st, s + 1);
+            multiply(s);
+        }
+        sync();
+        operands(st + 1, 0);
+        request(st + 1);
+        multiply(3);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (copies may not outlive the workgroup)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int64_t m = m0 + wm + 32 * i + lr;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int n = n0 + wn + 32 * j + 8 * v + 4 * kg;
+                if (n < N) emit4(out, f32x4{acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]}, m, n, M, N, 0);
+            }
+    }
+#endif
+}
+
 // ---- f32 tiles: 64 x 64, k in steps of 32, weights widened on the way into LDS; a lane's float4 along k feeds four steps of
 // v_mfma_f32_16x16x4 (both operands use the same k order) ------------------------------------------------------------------
 constexpr int DF_ROW = 36;               // floats per LDS row: 32 + 4, 16 rows of a 16-byte read fall on distinct banks
@@ -355,6 +484,15 @@ Plan plan(int precision, int64_t m, int64_t n, int64_t k) {
     p.k_split = (int)((k / 64 + s - 1) / s) * 64;
     p.splits = (int)((k + p.k_split - 1) / p.k_split);
     return p;
+}
+
+// Where the 256 x 256 tile takes the place of the 128 x 128 one: from 1024 of k on (1500 x 8192 x 512: 30.1 us against 28.6), where one round of workgroups
+// fills five eighths of the chip (1500 x 7168 x 2048, 168 tiles: 52 against 65) or several fill three quarters (4096 x 7168 x 2048, 448 tiles: 114 against
+// 142; 2048 x 10368 x 2048 of f32, 328 tiles: 136 against 131).
+bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
+    if (k < 1024 || ldw > (1 << 20) || ldx > (1 << 20)) return false;      // (its offsets have 32 bits: 256 rows of up to 4-byte elements)
+    const int64_t t = ((m + DT_B - 1) / DT_B) * ((n + DT_B - 1) / DT_B), rounds = (t + 255) / 256;
+    return rounds == 1 ? t >= 160 : 4 * t >= 3 * 256 * rounds;
 }
 
 // ---- one row --------------------------------------------------------------------------------------------------------------
@@ -534,6 +672,13 @@ int cq_dense_product(int precision, const cq_dense_args *args, void *workspace_d
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.splits, (unsigned)a.batch);
 #define CQ_DM(K_) hipLaunchKernelGGL(K_, grid, dim3(256), 0, s, src, o, m, (int)n, (int)k, p.tiles_m, p.tiles_n, p.k_split)
     if (precision == CQ_DENSE_F32) CQ_DM(dense_f32_kernel);
+    else if (p.bm == 128 && p.splits == 1 && a.batch == 1 && !a.tiles_dev && !a.src_rows_dev && large_tile(m, n, k, a.ldw, a.ldx)) {
+        auto *const fn = a.x_bf16 ? dense_tile_kernel<true> : dense_tile_kernel<false>;
+        const hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * DT_STAGE);
+        if (e != hipSuccess) return (int)e;
+        const int tm = (int)((m + DT_B - 1) / DT_B), tn = (int)((n + DT_B - 1) / DT_B);
+        hipLaunchKernelGGL(fn, dim3((unsigned)(tm * tn)), dim3(512), 2 * DT_STAGE, s, src, o, m, (int)n, (int)k, tm, tn);
+    }
     else if (p.bm == 128 && a.x_bf16) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, true>));
     else if (p.bm == 128) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, false>));
     else if (p.bm == 64 && a.x_bf16) CQ_DM((dense_bf16_kernel<64, 64, 2, 2, true>));

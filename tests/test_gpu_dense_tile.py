@@ -1,0 +1,53 @@
+"""The 256 x 256 tile of the bfloat16 product (cq_dense.hip) at its edges, against float64 products of the rounded operands.
+
+Bound: the products of bfloat16 operands are exact in f32; a sum of k of them in f32, k / 16 at a time, rounds k / 16 times (and within the matrix
+instruction): below 2^-24 * sqrt(k / 16) * 4 = 4e-6 of the norm for k = 4160.
+"""
+import ctypes
+
+import pytest
+import torch
+
+from candle_amd._lib import DenseArgs
+from candle_amd import _lib
+
+pytestmark = pytest.mark.gpu
+BOUND = 4e-6
+
+
+@pytest.mark.parametrize("x_bf16", [0, 1])
+@pytest.mark.parametrize("m,n,k,pad", [(257, 20475, 1024, 0), (2300, 4610, 1088, 64), (2048, 5120, 4160, 0), (255, 40964, 1024, 128)])
+@pytest.mark.parametrize("form", ["plain", "add", "swiglu", "bf16", "rows"])
+def test_edges(m, n, k, pad, x_bf16, form):
+    print(f"case {m} {n} {k} {pad} {x_bf16} {form}", flush=True)
+    if form == "swiglu":
+        n &= ~1
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = torch.randn((n, k + pad), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k + pad), generator=g, device="cuda")
+    xd = x.bfloat16() if x_bf16 else x
+    cols = n // 2 if form == "swiglu" else n
+    y = torch.full((m + 2, cols + 3), 5.0, device="cuda", dtype=torch.bfloat16 if form == "bf16" else torch.float32)
+    add = torch.randn((m, n), generator=g, device="cuda") if form == "add" else None
+    perm = torch.randperm(m, generator=g, device="cuda").int() if form == "rows" else None
+    a = DenseArgs(w_dev=w.data_ptr(), ldw=k + pad, x_dev=xd.data_ptr(), ldx=k + pad, x_bf16=x_bf16, dst_dev=y[1].data_ptr(), ldd=cols + 3, m=m, n=n, k=k, batch=1,
+                  dst_bf16=int(form == "bf16"), act=2 if form == "swiglu" else 0, add_dev=add.data_ptr() if form == "add" else None, ld_add=n if form == "add" else 0,
+                  dst_rows_dev=perm.data_ptr() if form == "rows" else None)
+    L = _lib.mixer_lib()
+    assert L.cq_dense_matmul_workspace_bytes(0, m, n, k) == 0
+    _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), None, 0, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    want = x[:, :k].bfloat16().double() @ w[:, :k].double().t()
+    size = want.norm(dim=1, keepdim=True)
+    if form == "add":
+        want += add
+    if form == "swiglu":
+        want = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]
+    got = y[1:m + 1, :cols].double()
+    if form == "rows":
+        got = got[perm.long()]
+    err = (got - want).abs()
+    if form == "bf16":
+        err = (err - want.abs() * 2.0 ** -8).clamp(min=0)
+    assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * (4 if form == "swiglu" else 1)      # (silu and the gate: slopes up to 1.1, values to 4)
+    assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, cols:] == 5).all()
