@@ -6,7 +6,7 @@
 // activations are the Q8_K / Q8_0 quantization written by cq_quantize_act.
 //
 // Q4_K, Q5_K, Q6_K, Q4_0 and Q8_0 go to the kernels of cq_qtile.hip and cq_qtile0.hip where cq_qtile_takes allows it; here are the other formats, and what those
-// refuse: Q6_K tensors that do not begin and end on a dword, Q4_0 and Q8_0 rows that do not begin on 16 bytes.
+// refuse: Q6_K tensors that do not begin and end on a dword or have short rows, Q4_0 and Q8_0 rows that do not begin on 16 bytes.
 //
 // Q6_K, Q2_K, Q3_K — integer-exact formulation on the f16 matrix cores (qmm_kernel):
 //   per 256-element super-block kb      S[m,n] = sum_k q8[m,k] * (sc[n,sub(k)] * q[n,k])

@@ -15,7 +15,7 @@
 //    three super-blocks shared by the workgroup, one barrier per super-block.  Q6_K blocks begin on 2 bytes: its pieces are brought from the dword below and
 //    shifted on reading, two half super-blocks at a time;
 //  - waves 4 - 7 (the second on each SIMD) run half a super-block behind, so that the vector work at the end of a super-block lies under the other wave's
-//    matrix work (7 % at 2048 rows; Q6_K, whose waves take part in fewer barriers, gains nothing and does without);
+//    matrix work (Q6_K gains nothing from it and does without);
 //  - fragments, conversions and products of one step are interleaved by hand, the sums of a tile pinned before the next one's: left to itself the
 //    scheduler spills.
 // f16 / bf16 results are written by the product; the f32 copy and its conversion went (12 us of 154 for 512 rows of Q5_K).
@@ -443,17 +443,19 @@ int qtile_any(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const Act
 
 }  // namespace
 
+static constexpr int64_t QT_Q6K_MIN_K = 1536;
 bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
     if (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K) return k % 256 == 0;
     if (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) return k % 256 == 0 && ((uintptr_t)w & 15) == 0;      // (rows are multiples of 16 bytes)
-    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one
-    return w_dtype == CQ_Q6K && k % 256 == 0 && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
+    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one.  Its two half super-blocks in flight need some of k to pay (67 / 300 rows
+    // of [4096 x 768] 17.6 / 18.9 us against 16.8 / 17.6 of the general kernel, of [8192 x 1024] 21.3 at 67 against 20.2; from 2048 on it is the faster one)
+    return w_dtype == CQ_Q6K && k % 256 == 0 && k >= QT_Q6K_MIN_K && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
 }
 
 // Bytes of split planes that a call may use, not falling with the rows.
 static constexpr int64_t QT_PLANE_FLOATS = 12 << 20;
 int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
-    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K && w_dtype != CQ_Q4_0 && w_dtype != CQ_Q8_0) || n % 4 || k < 512 || k % 256) return 0;
+    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K && w_dtype != CQ_Q4_0 && w_dtype != CQ_Q8_0) || n % 4 || k < (w_dtype == CQ_Q6K ? QT_Q6K_MIN_K : 512) || k % 256) return 0;
     return cq_align256(std::min<int64_t>(16 * rows * n, QT_PLANE_FLOATS) * 4);
 }
 
@@ -467,7 +469,7 @@ static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_
     const int64_t nsb = k / 256, nt = (n + 32 * QT_NW - 1) / (32 * QT_NW);
     const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : w_dtype == CQ_Q6K ? 2.4 : 1.6;
     const double b = w_dtype == CQ_Q6K ? 0.65 : cq_is_kquant(w_dtype) ? 0.79 : 1.23, plane = (double)rows * n * 4;
-    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({16, nsb / 2, most_splits}));
+    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({16, nsb, most_splits}));
     QtPlan best{4, 1};
     double least = 1e30;
     for (int mi = 1; mi <= 4; mi++)

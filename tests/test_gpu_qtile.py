@@ -58,10 +58,11 @@ def check(fmt, m, n, k, out=0, shift=0):
 
 
 @pytest.mark.parametrize("fmt", FMT)
-@pytest.mark.parametrize("m,n,k", [(66, 256, 256), (65, 1, 512), (97, 257, 768), (128, 31, 2304), (129, 260, 1280), (70, 292, 14336), (300, 510, 512)])
+@pytest.mark.parametrize("m,n,k", [(66, 256, 256), (65, 1, 512), (97, 257, 768), (128, 31, 2304), (129, 260, 1280), (70, 292, 14336), (300, 510, 512), (65, 2, 1536), (97, 257, 2048), (129, 260, 1792),
+                                   (300, 512, 1536)])
 def test_tile_edges(fmt, m, n, k):
     # one row past a 32-row tile, one column past a workgroup's 256, one super-block, odd numbers of them, k split over workgroups (n % 4 == 0) and not;
-    # Q6_K with an odd number of blocks (n k / 256 odd) takes the general kernel
+    # Q6_K of less than 1536 of k or with an odd number of blocks (n k / 256 odd) takes the general kernel
     check(fmt, m, n, k)
 
 
@@ -74,7 +75,7 @@ def test_half_results(fmt, out, n, k):
 
 @pytest.mark.parametrize("fmt,shift", [("q4_0", 2), ("q4_0", 8), ("q8_0", 6), ("q8_0", 16), ("q6k", 2), ("q6k", 4), ("q4k", 16), ("q5k", 48)])
 def test_weights_at_other_addresses(fmt, shift):
-    check(fmt, 66, 96, 768, shift=shift)                   # Q4_0 / Q8_0 off 16 bytes, Q6_K off 4: the general kernels
+    check(fmt, 66, 96, 1792, shift=shift)                   # Q4_0 / Q8_0 off 16 bytes, Q6_K off 4: the general kernels
 
 
 @pytest.mark.parametrize("fmt,bb", [("q4_0", 18), ("q8_0", 34)])
@@ -101,7 +102,7 @@ def test_grouped_experts(fmt, tokens):
     """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row."""
     import candle_amd as ca
     code, odt = FMT[fmt]
-    E, n, k, topk = 5, 268, 768, 2
+    E, n, k, topk = 5, 268, 1792, 2
     w = normal(21, (E, n, k), 0.02)
     blocks = oracle.from_float(odt, w.reshape(-1))
     qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(odt)), (E, n, k))
