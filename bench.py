@@ -68,7 +68,7 @@ WDTYPES = {"q4_0": (2, 18, 32), "q8_0": (8, 34, 32), "q4k": (12, 144, 256), "q5k
 FMT_NAMES = {"q4_0": "Q4_0", "q8_0": "Q8_0", "q4k": "Q4_K", "q5k": "Q5_K", "q6k": "Q6_K", "q4_1": "Q4_1", "q5_0": "Q5_0", "q5_1": "Q5_1",
              "q2k": "Q2_K", "q3k": "Q3_K"}
 # formats whose prefill kernel runs on the int8 matrix cores (the others use the f16 ones)
-I8_PREFILL = ("q4k", "q4_0", "q8_0", "q4_1", "q5_0", "q5_1")
+I8_PREFILL = ("q4k", "q4_0", "q8_0", "q4_1", "q5_0", "q5_1", "q5k", "q6k")
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "q4k_decode_matvec_1x4096x14336_pmc.txt")
 
 
@@ -210,7 +210,7 @@ def prefill_record(L, torch, fmt, n, k, m, steps=20, warmup=5, pmc=False):
     def quantize_only():
         _lib.check("cq_quantize_act", L.cq_quantize_act(dt, x.data_ptr(), 0, ws.data_ptr(), k, m, sp))
 
-    # small grids split K into partial planes that a second kernel adds up (the workspace then holds those planes too)
+    # whether the workspace has room for planes of a split K, which a second kernel adds up (the library splits where that fills the chip better)
     act_bytes = L.cq_act_scratch_bytes(dt, k, m)
     split_k = ws_bytes > act_bytes + ((m * n * 4 + 255) // 256) * 256
 
@@ -255,7 +255,7 @@ def prefill_record(L, torch, fmt, n, k, m, steps=20, warmup=5, pmc=False):
     peak = MFMA_I8_PEAK_TOPS if i8 else MFMA_F16_PEAK_TFLOPS
     achieved = flops / (kern_us * 1e-6) / 1e12
     return {"fmt": fmt, "n": n, "k": k, "m": m, "steps": steps, "warmup": warmup, "forward_ms": round(ms, 5),
-            "forward_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1), "kernel": "qmm_q4k_i8_kernel" if fmt == "q4k" else ("qmm_q0_i8_kernel<%s>" if i8 else "qmm_kernel<%s>") % fmt,
+            "forward_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1), "kernel": ("qtile_kernel<%s>" if fmt in ("q4k", "q5k", "q6k") else "qtile0_kernel<%s>" if fmt in ("q4_0", "q8_0") else "qmm_q0_i8_kernel<%s>" if i8 else "qmm_kernel<%s>") % fmt,
             "split_k": bool(split_k), "quantize_us": round(q_us, 2),
             "kernel_us": round(kern_us, 2), "kernel_median_us": round(kst["median"], 2), "kernel_p10_us": round(kst["p10"], 2),
             "kernel_p90_us": round(kst["p90"], 2), "kernel_TFLOPs": round(achieved, 1), "mfma": "i8" if i8 else "f16", "peak": peak,
