@@ -194,3 +194,13 @@ def test_rust_ffi_declarations_match_the_headers():
     assert declared == set(_lib.SIGNATURES)
     used = set(re.findall(r"ffi::(cq_\w+)", open(os.path.join(crate, "src", "lib.rs")).read()))
     assert used and used <= declared
+
+
+def test_rust_build_script_compiles_the_sources_of_the_library():
+    """build.rs names every source of the library, and declares as many as it names (an array type of another length does not compile)."""
+    from candle_amd.build import SOURCES
+    text = open(os.path.join(ROOT, "rust", "candle-hip-quant", "build.rs")).read()
+    kind, names = re.search(r"const SOURCES: (\S+(?: \d+\])?)\s*=\s*&?\[(.*?)\];", text, re.S).groups()
+    names = re.findall(r'"(\w+)"', names)
+    assert [n + ".hip" for n in names] == SOURCES
+    assert kind in ("&[&str]", f"[&str; {len(names)}]")
