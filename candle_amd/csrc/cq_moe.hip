@@ -51,8 +51,11 @@ inline MoeWorkspace moe_workspace(int w_dtype, int64_t num_experts, int64_t n_pa
 // offsets[e] .. offsets[e+1] is expert e's segment of pair_in / pair_out / pair_scale.
 // LC: the per-expert counters live in LDS (up to GROUP_LDS_EXPERTS experts) instead of the global `cursor` array: the
 // two passes of atomics are then LDS atomics, not trips of one workgroup to the L2.
-constexpr int GROUP_LDS_EXPERTS = 4096;
-template <bool LC>
+// The first KEEP pairs of every thread stay in registers between the two passes.  Decoding a pair is two dependent loads.  MANY: all first ones are asked for
+// before any is used, then all second ones, whether a thread has that many pairs or not.  12000 pairs on 128 experts: 26 us, 30 pair by pair; but what threads
+// without pairs go through, divisions by topk above all, costs a call of 300 - 3000 pairs 2.3 us, one of 4800 1.1, one of 6000 0.4; 8000 gain 0.5.
+constexpr int GROUP_LDS_EXPERTS = 4096, GROUP_MANY_PAIRS = 6144;
+template <bool LC, bool MANY>
 __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__restrict__ offsets, int *__restrict__ cursor,
                                                          int *__restrict__ pair_in, int *__restrict__ pair_out,
                                                          float *__restrict__ pair_scale, float *__restrict__ out, int n, int *__restrict__ chunks,
@@ -65,14 +68,15 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
     const int E = ps.num_experts;
     for (int e = tid; e < E; e += 1024) cur[e] = 0;
     __syncthreads();
-    // The first KEEP pairs of every thread stay in registers between the two sweeps.  Decoding a pair is two dependent loads: all first ones are asked for
-    // before any is used, then all second ones (12000 pairs on 128 experts: 26 us, 30 for one pair at a time and 4 of them kept).
-    constexpr int KEEP = 12;
+    constexpr int KEEP = MANY ? 12 : 4;
     int ke[KEEP], kin[KEEP], kout[KEEP];
     float ksc[KEEP];
     bool kok[KEEP];
     const int last = ps.n_pairs - 1;
-    if (ps.mode == MOE_INDEXED) {
+    if (!MANY) {
+#pragma unroll
+        for (int i = 0; i < KEEP; i++) kok[i] = tid + i * 1024 <= last && pair_decode(ps, tid + i * 1024, ke[i], kin[i], kout[i], ksc[i]);
+    } else if (ps.mode == MOE_INDEXED) {
 #pragma unroll
         for (int i = 0; i < KEEP; i++) ke[i] = (int)ps.ids_u32[min(tid + i * 1024, last)];
 #pragma unroll
@@ -337,12 +341,11 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     // Hundreds of pairs per call: the expert-sorted rows go through the MFMA prefill kernel of the format in tiles of up to
     // 128 rows of one expert (integer-exact like the dense paths).  Otherwise 8 pairs per matvec pass.
     const int tile_rows = moe_tile_rows(a.n_pairs, a.num_experts);
-    if (a.num_experts <= GROUP_LDS_EXPERTS)
-        hipLaunchKernelGGL(moe_group_kernel<true>, dim3(1), dim3(1024), 0, s, ps, offsets, cursor, pin, pout, pscale, a.out, (int)a.n, chunks,
-                           (int)ws.max_chunks, stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK, stream ? extra : nullptr);
-    else
-        hipLaunchKernelGGL(moe_group_kernel<false>, dim3(1), dim3(1024), 0, s, ps, offsets, cursor, pin, pout, pscale, a.out, (int)a.n, chunks,
-                           (int)ws.max_chunks, stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK, stream ? extra : nullptr);
+    const bool many = a.n_pairs > GROUP_MANY_PAIRS;
+    auto *const group = a.num_experts <= GROUP_LDS_EXPERTS ? (many ? moe_group_kernel<true, true> : moe_group_kernel<true, false>)
+                                                           : (many ? moe_group_kernel<false, true> : moe_group_kernel<false, false>);
+    hipLaunchKernelGGL(group, dim3(1), dim3(1024), 0, s, ps, offsets, cursor, pin, pout, pscale, a.out, (int)a.n, chunks, (int)ws.max_chunks,
+                       stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK, stream ? extra : nullptr);
     if ((rc = (int)hipGetLastError())) return rc;
     if (stream) {
         // every expert a batched matvec over its own pairs: the weights of an expert are streamed once per 32 pairs

@@ -45,3 +45,27 @@ def test_grouping_many_pairs(tokens):
         t, s = np.nonzero(ids == e)
         assert rel_l2(got[t, s], oracle.matmul(oracle.Q8_0, x[t, 0], blocks[e * per:(e + 1) * per], n)) <= 2e-6
     assert (got[ids == E] == 0).all()
+
+
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("tokens", [140, 3072, 3073])                   # two pairs a token: up to 6144 are decoded pair by pair, more by loads asked for together
+def test_grouping_at_the_change_of_form(tokens, weights):
+    import candle_amd as ca
+    E, n, k, top = 7, 20, 256, 2
+    blocks = oracle.from_float(oracle.Q8_0, normal(5, (E, n, k), 0.02).reshape(-1))
+    qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(oracle.Q8_0)), (E, n, k))
+    pairs = tokens * top
+    rng = np.random.default_rng(pairs)
+    experts, order = rng.integers(0, E, pairs).astype(np.int32), rng.permutation(pairs).astype(np.int32)
+    x = normal(6, (pairs if weights else tokens, k))
+    tw = rng.uniform(0.1, 1, pairs).astype(np.float32) if weights else None
+    cuda = lambda a: torch.from_numpy(a).cuda()
+    got = ca.moe_gemm_gguf(cuda(x), qt, cuda(tw) if weights else None, cuda(order), cuda(experts), top, True).cpu().numpy()
+    assert rel_l2(got, oracle.moe_gemm_gguf(oracle.Q8_0, x, blocks, (E, n, k), order, experts, tw, top)) <= 2e-6
+    ids = rng.integers(0, E + 1, (tokens, top)).astype(np.int32)        # E: no such expert, a row of zeros
+    x = normal(7, (tokens, k))
+    got = qt.indexed_moe_forward(cuda(x[:, None]), cuda(ids)).cpu().numpy()
+    for e in range(E):
+        t, s = np.nonzero(ids == e)
+        assert rel_l2(got[t, s], oracle.matmul(oracle.Q8_0, x[t], blocks[e * len(blocks) // E:(e + 1) * len(blocks) // E], n)) <= 2e-6
+    assert (got[ids == E] == 0).all()
