@@ -383,32 +383,42 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__r
 #endif
 }
 
-// The splits of K added in order, the first one from `first` (dst itself or a plane), the others from planes; n % 4 == 0.  Bound by the latency of the reads at
-// the sizes that are split: four planes are on their way at a time, and a workgroup is small enough that 32 x 4096 results fill the chip.
-constexpr int QT_RT = 128;
+// The sum of the splits of K in a fixed order, in pairs and pairs of pairs: sixteen sums added one after the other round more than the chain of super-blocks
+// that they were cut from (Q6_K rows of 4096: 8.5e-8 of the results' norm against 6.2e-8 in four splits; in pairs 6.2e-8).  The first split comes from
+// `first` (dst itself or a plane), the others from planes; n % 4 == 0.  Bound by the latency of the reads at the sizes that are split: four planes are on their way at
+// a time, and a workgroup is small enough that 32 x 4096 results fill the chip.
+constexpr int QT_RT = 128, QT_MAX_SPLITS = 16;
 template <int ODT>
 __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first, int64_t ld_first, const float *__restrict__ planes, void *dst, int splits, int64_t n,
                                                              int64_t stride_dst, int64_t count) {
     const int64_t i = ((int64_t)blockIdx.x * QT_RT + threadIdx.x) * 4;
     if (i >= count) return;
     const int64_t r = i / n, c0 = i - r * n, o = r * stride_dst + c0;
-    float a[4];
+    const float none = -0.0f;                              // (x + -0 is x)
+    f32x4 sum[QT_MAX_SPLITS / 4];
 #pragma unroll
-    for (int c = 0; c < 4; c++) a[c] = first[r * ld_first + c0 + c];
-    for (int p = 0; p < splits - 1; p += 4) {
+    for (int g = 0; g < QT_MAX_SPLITS / 4; g++) {
+        sum[g] = f32x4{none, none, none, none};
+        if (4 * g >= splits) continue;
         f32x4 b[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) b[u] = *reinterpret_cast<const f32x4 *>(planes + min(p + u, splits - 2) * count + i);
+        for (int u = 0; u < 4; u++) {
+            if (4 * g + u == 0) {
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (p + u < splits - 1)
+                for (int c = 0; c < 4; c++) b[u][c] = first[r * ld_first + c0 + c];
+            } else b[u] = *reinterpret_cast<const f32x4 *>(planes + (min(4 * g + u, splits - 1) - 1) * count + i);
+        }
 #pragma unroll
-                for (int c = 0; c < 4; c++) a[c] += b[u][c];
+        for (int u = 1; u < 4; u++)
+            if (4 * g + u >= splits) b[u] = f32x4{none, none, none, none};
+#pragma unroll
+        for (int c = 0; c < 4; c++) sum[g][c] = (b[0][c] + b[1][c]) + (b[2][c] + b[3][c]);
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        if (ODT == CQ_F32) ((float *)dst)[o + c] = a[c];
-        else ((uint16_t *)dst)[o + c] = ODT == CQ_F16 ? f2h_bits(a[c]) : f2bf_bits(a[c]);
+        const float a = (sum[0][c] + sum[1][c]) + (sum[2][c] + sum[3][c]);
+        if (ODT == CQ_F32) ((float *)dst)[o + c] = a;
+        else ((uint16_t *)dst)[o + c] = ODT == CQ_F16 ? f2h_bits(a) : f2bf_bits(a);
     }
 }
 
@@ -464,16 +474,40 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
 // is least.  A round is 256 workgroups (a tenth slower when all compute units are busy: the clock falls), a the conversion of the weights, b the products
 // and sums of 32 rows.  Fitted to 3800 launches of 17 - 2048 rows against [14336 x 4096], [4096 x 14336], [1024 x 4096] and [5120 x 4096] (6 % rms, 10 % for
 // Q4_0); the choice it makes is 0.2 - 1.2 % slower than the best of all pairs on average, at most 16 % (100 rows of Q4_K: 39.1 against 33.8 us).
+// Only splits whose sums round no more than those of the general kernels (qt_roundings).
 struct QtPlan { int mi, splits; };
+// What the f32 sums of one result round, as twice a variance in units of one term's: a chain of c terms takes c fma's, which round partial sums of 1 .. c terms
+// (the first one, a product alone, like one and a half), and every addition of two splits rounds a sum of as many terms as both have.  in_pairs: as
+// qtile_reduce_kernel adds them, else one after the other like the general kernels (cq_qmm_splits).  More splits shorten the chains, but each begins with a
+// rounding that a longer chain does not have.  Q6_K, of the results' norm: rows of 2048 in eight splits 5.95e-8, in two 5.47e-8; rows of 4096 in 16 splits
+// 6.55e-8, in eight 6.22e-8, in the four of the general kernel 6.26e-8; 131 rows of Q8_0 [11008 x 4096] unsplit 2.05e-7, in the general kernel's two 1.49e-7.
+static int64_t qt_roundings(int64_t nsb, int terms, int splits, bool in_pairs) {
+    int64_t total = 0, sum[QT_MAX_SPLITS];
+    for (int z = 0; z < splits; z++) {
+        const int64_t c = terms * (nsb * (z + 1) / splits - nsb * z / splits);
+        total += c * (c + 1) + 1;
+        sum[z] = c;
+    }
+    for (int step = 1; in_pairs && step < splits; step *= 2)
+        for (int z = 0; z + step < splits; z += 2 * step) total += 2 * (sum[z] += sum[z + step]);
+    for (int z = 1; !in_pairs && z < splits; z++) total += 2 * (sum[z] += sum[z - 1]);
+    return total;
+}
 static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_t most_splits) {
     const int64_t nsb = k / 256, nt = (n + 32 * QT_NW - 1) / (32 * QT_NW);
     const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : w_dtype == CQ_Q6K ? 2.4 : 1.6;
     const double b = w_dtype == CQ_Q6K ? 0.65 : cq_is_kquant(w_dtype) ? 0.79 : 1.23, plane = (double)rows * n * 4;
-    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({16, nsb, most_splits}));
-    QtPlan best{4, 1};
+    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({QT_MAX_SPLITS, nsb, most_splits}));
+    const int terms = cq_is_kquant(w_dtype) ? 1 : 8;
+    const int general = std::min(most, cq_qmm_splits(k, n, rows));
+    bool rounds_less[QT_MAX_SPLITS + 1];
+    for (int sp = 1; sp <= most; sp++)
+        rounds_less[sp] = sp == general || qt_roundings(nsb, terms, sp, true) < qt_roundings(nsb, terms, general, false);
+    QtPlan best{4, general};
     double least = 1e30;
     for (int mi = 1; mi <= 4; mi++)
         for (int sp = 1; sp <= most; sp++) {
+            if (!rounds_less[sp]) continue;
             const int64_t wgs = (rows + 32 * mi - 1) / (32 * mi) * nt * sp, rounds = (wgs + 255) / 256;
             const double load = 1.1 * (rounds - 1) + 1.0 + 0.1 * (double)(wgs - 256 * (rounds - 1)) / 256;
             const double t = load * ((double)((nsb + sp - 1) / sp) * (a + b * mi) + 1.3) + (sp > 1 ? 6.8 + (sp + 1) * plane / 4.5e6 : 0.0);

@@ -115,3 +115,24 @@ def test_grouped_experts(fmt, tokens):
         t, s = np.nonzero(ids == e)
         want = oracle.matmul(odt, x[t, 0], blocks[e * per:(e + 1) * per], n)
         assert row_error(got[t, s], want, x[t, 0], w[e], k) <= BOUND
+
+
+@pytest.mark.parametrize("fmt,m,n,k,splits", [("q8_0", 131, 8192, 2304, 2), ("q4_0", 777, 2048, 2048, 2), ("q8_0", 131, 11008, 4096, 2), ("q6k", 24, 256, 4096, 4), ("q6k", 65, 1024, 4096, 4),
+                                              ("q6k", 300, 512, 2048, 2)])
+def test_split_sums_round_no_more_than_the_general_kernels(fmt, m, n, k, splits):
+    """Against 64 bits: however K is split, f32 sums may round no more than in the general kernels' `splits` chains, added one after the other.
+
+    An f32 rounding has an rms of 0.425 * 2^-24 of its value (half an ulp, uniform, over mantissas of 1 to 2).  A chain of c terms rounds partial sums of 1 .. c
+    terms, the sum of the chains those of all terms so far, and each term itself rounds once or twice before it is added (1.5 units); 5 % for the rest.
+    """
+    from perf import cases
+    name = {"q4k": "q4_k", "q5k": "q5_k", "q6k": "q6_k"}.get(fmt, fmt)
+    b = cases.blocks(name, 3, "w", n, k)
+    x = normal(9 + n, (m, k))
+    want = cases.product(name, torch.from_numpy(x).cuda(), cases.values(name, b, n, k)).cpu().numpy()
+    got = run(FMT[fmt][0], b.reshape(-1).cpu().numpy(), x, n)
+    terms, nsb = (8 if fmt in ("q4_0", "q8_0") else 1), k // 256
+    ends = [nsb * z // splits * terms for z in range(splits + 1)]
+    total = ends[-1]
+    variance = sum((e - s) * (e - s + 1) / 2 for s, e in zip(ends, ends[1:])) + sum(ends[2:]) + 1.5 * total
+    assert rel_l2(got, want) <= 1.05 * 0.425 * 2.0 ** -24 * np.sqrt(variance / total)
