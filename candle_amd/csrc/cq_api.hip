@@ -180,7 +180,7 @@ int cq_matmul(int w_dtype, const void *w_dev, const void *act_scratch_dev, float
     return cq_matmul_launch(w_dtype, w_dev, act_scratch_dev, dst_dev, k, n, rows, stride_dst, (hipStream_t)stream);
 }
 
-// What a call cannot do without.
+// What a call cannot do without: the general kernels' planes, which callers may have reserved before there were others.
 static int64_t workspace_least(int w_dtype, int64_t m, int64_t k, int64_t n) {
     int64_t bytes = cq_act_layout(w_dtype, k, m).total;
     // the batched matvec lays the rows out as matrix operands, 16 row slots whatever the batch
@@ -214,7 +214,8 @@ static int forward_quantized(int w_dtype, const void *w_dev, void *dst_dev, int 
     const int64_t act = cq_act_layout(w_dtype, k, m).total;
     float *tmp = (float *)((uint8_t *)workspace_dev + act);
     if (cq_use_mfma(w_dtype, m, k) && cq_qtile_takes(w_dtype, w_dev, k, n)) {
-        // the split is one of the shape alone, whatever else the caller has to spare: the results of all entry points are the same bits
+        // with the whole of cq_qmatmul_workspace_bytes the split is one of the shape alone, whatever else the caller has to spare; with less, down to
+        // workspace_least, it is the best of those that there is room for, and f32 sums may differ in their last bits
         const int64_t room = std::min(workspace_bytes, cq_qmatmul_workspace_bytes(w_dtype, m, k, n)) - act;
         return cq_qtile_launch(w_dtype, w_dev, cq_act_view(workspace_dev, w_dtype, k, m), dst_dev, dst_dtype, k, n, m, n, tmp, room, s);
     }

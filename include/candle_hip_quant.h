@@ -137,8 +137,9 @@ int cq_matmul(int w_dtype, const void *w_dev, const void *act_scratch_dev, float
  * up to 6144 elements quantized inside that kernel; Q4K / Q5K with 17 <= m <= 64 f32 rows of up to 4096 elements to an f32 dst: the
  * same with the rows in sets of 16, one pass over the weights per 32 rows) or MFMA matmul
  * (split over k with an ordered reduction when the grid would be small).  x is [m, k] contiguous (f32 / f16 / bf16), dst is [m, n] contiguous in dst_dtype
- * (CUDA keeps the input dtype: fast_mmvq.rs:161-323).  workspace_dev: 256-byte aligned,
- * at least cq_qmatmul_workspace_bytes(w_dtype, m, k, n) bytes.
+ * (CUDA keeps the input dtype: fast_mmvq.rs:161-323).  workspace_dev: 256-byte aligned, cq_qmatmul_workspace_bytes(w_dtype, m, k, n)
+ * bytes; with any more the results are the same bits.  Somewhat less is accepted too, as long as the quantized rows, the f32 results and
+ * the planes of the general kernels' split fit (CQ_ERR_WORKSPACE otherwise): k is then split less, and f32 sums may differ in their last bits.
  * ------------------------------------------------------------------------------------------- */
 int64_t cq_qmatmul_workspace_bytes(int w_dtype, int64_t m, int64_t k, int64_t n);
 /* Bytes of one wave step of the single-row decode kernel over a [n, k] weight of this format, or 0 when the shape does not take

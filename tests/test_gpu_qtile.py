@@ -20,20 +20,23 @@ FMT = {"q4_0": (2, oracle.Q4_0), "q8_0": (8, oracle.Q8_0), "q4k": (12, oracle.Q4
 OUT = {0: torch.float32, 1: torch.float16, 30: torch.bfloat16}
 
 
-def run(code, blocks, x, n, out=0, shift=0):
-    """cq_qmatmul_forward of x [m, k] with the weights `shift` bytes past a 256-byte boundary, the result between two rows of canaries."""
+def run(code, blocks, x, n, out=0, shift=0, room=None):
+    """cq_qmatmul_forward of x [m, k] with the weights `shift` bytes past a 256-byte boundary, the result between two rows of canaries.
+    room: bytes of workspace, less than cq_qmatmul_workspace_bytes asks for, with canaries behind them."""
     L = _lib.lib()
     m, k = x.shape
     raw = torch.zeros(len(blocks) + 512, dtype=torch.uint8, device="cuda")
     raw[shift:shift + len(blocks)] = torch.from_numpy(blocks).cuda()
     xd = torch.from_numpy(x).cuda()
     y = torch.full((m + 2, n), 77.0, dtype=OUT[out], device="cuda")
-    nb = L.cq_qmatmul_workspace_bytes(code, m, k, n)
-    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    full = L.cq_qmatmul_workspace_bytes(code, m, k, n)
+    nb = full if room is None else room
+    ws = torch.full((full + 256,), 173, dtype=torch.uint8, device="cuda")
     rc = L.cq_qmatmul_forward(code, raw.data_ptr() + shift, ctypes.c_void_p(xd.data_ptr()), 0, ctypes.c_void_p(y[1].data_ptr()), out, m, k, n,
                               ctypes.c_void_p(ws.data_ptr()), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     _lib.check("cq_qmatmul_forward", rc)
     torch.cuda.synchronize()
+    assert (ws[nb:] == 173).all()
     y = y.float().cpu().numpy()
     assert (y[0] == 77).all() and (y[-1] == 77).all()
     return y[1:-1]
@@ -45,13 +48,13 @@ def row_error(got, want, x, w, k):
     return float((np.linalg.norm(got.astype(np.float64) - want, axis=1) / size).max())
 
 
-def check(fmt, m, n, k, out=0, shift=0):
+def check(fmt, m, n, k, out=0, shift=0, room=None):
     print(f"case {fmt} m={m} n={n} k={k} out={out} shift={shift}", flush=True)
     code, odt = FMT[fmt]
     w = normal(7 + m, (n, k), 0.02)
     blocks = oracle.from_float(odt, w.reshape(-1))
     x = normal(9 + n, (m, k))
-    got, want = run(code, blocks, x, n, out, shift), oracle.matmul(odt, x, blocks, n)
+    got, want = run(code, blocks, x, n, out, shift, room), oracle.matmul(odt, x, blocks, n)
     eps = {0: 0.0, 1: 2.0 ** -11, 30: 2.0 ** -8}[out]                # one rounding to the output type
     excess = np.maximum(np.abs(got - want) - eps * np.abs(want) - (2.0 ** -25 if out == 1 else 0), 0)        # (f16 results below 2^-14 are multiples of 2^-24)
     assert row_error(excess, 0, x, w, k) <= BOUND
@@ -71,6 +74,21 @@ def test_tile_edges(fmt, m, n, k):
 @pytest.mark.parametrize("n,k", [(130, 512), (260, 4096)])
 def test_half_results(fmt, out, n, k):
     check(fmt, 67, n, k, out)                              # written by the product itself, and by the sum over the splits
+
+
+@pytest.mark.parametrize("fmt", FMT)
+@pytest.mark.parametrize("out", [0, 1])
+@pytest.mark.parametrize("m,n,k,splits", [(67, 260, 1536, 1), (67, 260, 4096, 4)])
+def test_least_workspace(fmt, out, m, n, k, splits):
+    """The quantized rows, one plane of results and the general kernels' `splits` of them: enough for a call, with canaries right behind; less is refused."""
+    L = _lib.lib()
+    code = FMT[fmt][0]
+    up = lambda b: (b + 255) // 256 * 256
+    least = L.cq_act_scratch_bytes(code, k, m) + up(4 * m * n) + (up(4 * splits * m * n) if splits > 1 else 0)
+    assert least < L.cq_qmatmul_workspace_bytes(code, m, k, n)
+    p = ctypes.c_void_p(4096)                              # (refused before anything is read)
+    assert L.cq_qmatmul_forward(code, p, p, 0, p, out, m, k, n, p, least - 1, None) == -5      # CQ_ERR_WORKSPACE
+    check(fmt, m, n, k, out, room=least)
 
 
 @pytest.mark.parametrize("fmt,shift", [("q4_0", 2), ("q4_0", 8), ("q8_0", 6), ("q8_0", 16), ("q6k", 2), ("q6k", 4), ("q4k", 16), ("q5k", 48)])
