@@ -114,13 +114,33 @@ def test_extreme_block_scales(fmt, bb, d):
     assert rel_l2(got[ok], want[ok]) <= BOUND
 
 
+@pytest.mark.parametrize("fmt,bb,at", [("q4k", 144, 0), ("q4k", 144, 2), ("q5k", 176, 0), ("q5k", 176, 2), ("q6k", 210, 208)])
+@pytest.mark.parametrize("d", [np.inf, -np.inf, np.nan, 65504.0, 6e-8])
+def test_extreme_super_block_scales(fmt, bb, at, d):
+    """d or dmin of a super-block: results that are not finite where the oracle's are not.  Its eight partial sums may make NaN of an infinity, never the reverse."""
+    code, odt = FMT[fmt]
+    n, k, m = 96, 1536, 70
+    blocks = oracle.from_float(odt, normal(3, (n, k), 0.02).reshape(-1)).reshape(n, k // 256, bb)
+    blocks[[0, 40, 95], [0, 3, 5], at:at + 2] = np.frombuffer(np.float16(d).tobytes(), dtype=np.uint8)
+    x = normal(4, (m, k))
+    x[5, :256] = 0.0                                       # sums of zero times an infinite scale
+    want = oracle.matmul(odt, x, blocks.reshape(-1), n)
+    got = run(code, blocks.reshape(-1), x, n)
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), ok)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]) and (not np.isnan(d) or np.isnan(got[~ok]).all())
+    assert rel_l2(got[ok], want[ok]) <= BOUND
+
+
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q6k", "q5k"])
 @pytest.mark.parametrize("tokens", [70, 1200])
-def test_grouped_experts(fmt, tokens):
-    """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row."""
+@pytest.mark.parametrize("E,n", [(5, 268), (4, 267)])
+def test_grouped_experts(fmt, tokens, E, n):
+    """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row, and of
+    rows too: every second expert begins 2 bytes past a dword."""
     import candle_amd as ca
     code, odt = FMT[fmt]
-    E, n, k, topk = 5, 268, 1792, 2
+    k, topk = 1792, 2
     w = normal(21, (E, n, k), 0.02)
     blocks = oracle.from_float(odt, w.reshape(-1))
     qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(odt)), (E, n, k))
