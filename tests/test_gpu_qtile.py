@@ -174,3 +174,23 @@ def test_split_sums_round_no_more_than_the_general_kernels(fmt, m, n, k, splits)
     total = ends[-1]
     variance = sum((e - s) * (e - s + 1) / 2 for s, e in zip(ends, ends[1:])) + sum(ends[2:]) + 1.5 * total
     assert rel_l2(got, want) <= 1.05 * 0.425 * 2.0 ** -24 * np.sqrt(variance / total)
+
+
+@pytest.mark.parametrize("fmt", FMT)
+@pytest.mark.parametrize("rows,n,k", [(9, 31, 1536), (17, 260, 4096), (33, 520, 512), (67, 257, 2304), (131, 260, 1280)])
+def test_matmul_of_quantized_rows(fmt, rows, n, k):
+    """cq_matmul, which has no planes to split k with, into rows of a larger stride: nothing between them is written."""
+    L = _lib.lib()
+    code, odt = FMT[fmt]
+    w = normal(31, (n, k), 0.02)
+    blocks = oracle.from_float(odt, w.reshape(-1))
+    x = normal(32, (rows, k))
+    wd, xd = torch.from_numpy(blocks).cuda(), torch.from_numpy(x).cuda()
+    scratch = torch.empty(L.cq_act_scratch_bytes(code, k, rows), dtype=torch.uint8, device="cuda")
+    y = torch.full((rows, n + 3), 77.0, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    _lib.check("cq_quantize_act", L.cq_quantize_act(code, xd.data_ptr(), 0, scratch.data_ptr(), k, rows, s))
+    _lib.check("cq_matmul", L.cq_matmul(code, wd.data_ptr(), scratch.data_ptr(), y.data_ptr(), k, n, rows, n + 3, s))
+    y = y.cpu().numpy()
+    assert (y[:, n:] == 77).all()
+    assert row_error(y[:, :n], oracle.matmul(odt, x, blocks, n), x, w, k) <= BOUND
