@@ -12,6 +12,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int QT_NW = 8;                                 // waves of a workgroup, side by side along n
+constexpr int QT_NW_NARROW = 4;                          // of a narrow one
 
 // everything that goes into these sums is worked out before what follows (the scheduler would rather work on all tiles at once, out of
 // registers that are not there)
@@ -50,11 +51,11 @@ __device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int
 
 typedef void (*QtFn)(const uint8_t *, ActView, void *, int, int, int, int, int64_t, MoeChunks, int64_t, float *);
 
-inline int qtile_go(QtFn fn, int lds_bytes, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
+inline int qtile_go(QtFn fn, int nw, int lds_bytes, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                     const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
     hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(fn, grid, dim3(QT_NW * 64), lds_bytes, s, (const uint8_t *)w, av, dst, dst_dtype, (int)k, (int)n, (int)rows, stride_dst, mc, expert_bytes, planes);
+    hipLaunchKernelGGL(fn, grid, dim3(nw * 64), lds_bytes, s, (const uint8_t *)w, av, dst, dst_dtype, (int)k, (int)n, (int)rows, stride_dst, mc, expert_bytes, planes);
     return (int)hipGetLastError();
 }
 

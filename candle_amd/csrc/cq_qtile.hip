@@ -8,7 +8,7 @@
 //
 // What bounds it: at many rows the matrix cores at the clock that the power limit leaves (16 + 1 MFMAs of 32 x 32 x 32 per 32 rows, super-block and wave, about
 // 20 ns each with all units busy, 14.5 at the full clock), with the conversion of the weights behind it; at few rows the weights' way from memory.  So:
-//  - a workgroup is eight waves side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
+//  - a workgroup is eight waves (or four: qtile_plan) side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
 //    multiplies it, straight into its operand registers (the kernels before this one staged converted weights in LDS, and the conversion
 //    of Q5_K and Q6_K was to f16, Q6_K as two f16 terms: twice the matrix time of int8);
 //  - weights go by copies to LDS into a ring of the wave's own, three stages of 64 elements ahead, with counted waits and no barrier; activations into a ring of
@@ -21,10 +21,10 @@
 // f16 / bf16 results are written by the product; the f32 copy and its conversion went (12 us of 154 for 512 rows of Q5_K).
 //
 // [4096 x 14336], us, before / now, quantizing the activations included:    17 rows   131 rows   512 rows   2048 rows
-//   Q4_K                                                                  20.3 19.1  53.6 42.8  103 92.1   360 298
-//   Q5_K                                                                  36.8 22.1  73.4 47.2  144 101    514 324
-//   Q6_K                                                                  37.2 26.3  80.6 52.4  161 109    584 357
-// 2048 rows of Q4_K are 810 TOP/s of products asked for and 1620 done.
+//   Q4_K                                                                  20.9 18.3  59.3 45.2  113 95.5   386 305
+//   Q5_K                                                                  38.4 21.8  80.3 50.1  160 103    559 324
+//   Q6_K                                                                  38.8 28.6  87.0 55.5  175 112    619 368
+// 2048 rows of Q4_K are 790 TOP/s of products asked for and 1580 done.
 #include "cq_qtile.h"
 
 #include <algorithm>
@@ -78,20 +78,21 @@ template <> struct QTile<CQ_Q6K> {
 
 constexpr int QT_R = 4, QT_L = QT_R - 1;                 // stages (64 elements) in a wave's ring of weights, stages requested ahead
 // RA: super-blocks in the ring of activations
-template <int DT, int MI> struct QtLds {
+template <int DT, int MI, int NW> struct QtLds {
     static constexpr int PIECE = 1024 + 256, RA = DT == CQ_Q6K ? 2 : 3;
     static constexpr int A = MI * 8192, B = DT == CQ_Q6K ? 7 * PIECE : 1024 * (QT_R + QTile<DT>::EXTRA), AM = QTile<DT>::HAS_MIN ? MI * 1024 : 0, D8 = (MI + 1) / 2 * 256;
-    static constexpr int A_OFF = 0, B_OFF = RA * A, AM_OFF = B_OFF + QT_NW * B, D8_OFF = AM_OFF + RA * AM, BYTES = D8_OFF + RA * D8;
+    static constexpr int A_OFF = 0, B_OFF = RA * A, AM_OFF = B_OFF + NW * B, D8_OFF = AM_OFF + RA * AM, BYTES = D8_OFF + RA * D8;
 };
 
-template <int DT, int MI, bool MOE>
-__global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
+template <int DT, int MI, bool MOE, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
                                                               int rows, int64_t stride_dst, MoeChunks mc, int64_t expert_bytes, float *__restrict__ planes) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler has no use for the body, and does not know its buffer accesses)
     typedef QTile<DT> T;
-    typedef QtLds<DT, MI> LD;
-    constexpr int BB = BlockInfo<DT>::bytes, EX = T::EXTRA, BM = 32 * MI, BN = 32 * QT_NW;
-    constexpr int NA = MI;                                 // copy instructions per wave and super-block of activations
+    typedef QtLds<DT, MI, NW> LD;
+    static_assert(NW == 8 || (NW == 4 && MI <= 2), "two waves bring the sums and two the scales of 64 rows at most");
+    constexpr int BB = BlockInfo<DT>::bytes, EX = T::EXTRA, BM = 32 * MI, BN = 32 * NW;
+    constexpr int NA = 8 * MI / NW;                                 // copy instructions per wave and super-block of activations
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nr = lane & 31, kg = lane >> 5;
@@ -114,18 +115,18 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__r
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(wrow - w_odd), 0, -1, 0x00020000);
     const uint32_t w_off = (uint32_t)(min(nr, n - 1 - wbase) * row_bytes) + 16 * kg + w_odd;
     // ---- activations: 64 bytes of 16 rows per instruction, piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
-    // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + 8 i of its 8 MI KB)
+    // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + NW i of its 8 MI KB)
     const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
-    constexpr int NAO = MI == 4 ? 1 : NA;                  // (four row blocks of two: the instructions of a wave are whole stages apart)
+    constexpr int NAO = NW == 2 * MI ? 1 : NA;             // (as many waves as row blocks: the instructions of a wave are whole stages apart)
     uint32_t a_off[NAO];
 #pragma unroll
     for (int i = 0; i < NAO; i++) {
-        const int blk = wv + QT_NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
+        const int blk = wv + NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
         a_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)k + 64 * st + 16 * p;
     }
     uint8_t *const myB = lds + LD::B_OFF + wv * LD::B;
-    // ---- scales and 16-element sums of the activations: waves 0 - 3 bring the sums of 32 rows each, the others the scales of 64 ----
-    const bool x_sums = T::HAS_MIN && wv < 4;
+    // ---- scales and 16-element sums of the activations: the first half of the waves brings the sums of 32 rows each, the others the scales of 64 ----
+    const bool x_sums = T::HAS_MIN && wv < NW / 2;
     const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = min(x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane, rows - 1 - m0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         x_sums ? (void *)(av.bsums + (int64_t)m0 * (k >> 4)) : (void *)(av.d + (int64_t)m0 * nsb_all), 0, -1, 0x00020000);
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__r
         const int kb = min(kb0 + j, kb1 - 1);
 #pragma unroll
         for (int i = 0; i < NA; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (cq_lds_void *)(lds + LD::A_OFF + slot * LD::A + 1024 * (wv + QT_NW * i)), 16, a_off[NAO == 1 ? 0 : i], kb * 256 + (NAO == 1 ? 64 * i : 0), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (cq_lds_void *)(lds + LD::A_OFF + slot * LD::A + 1024 * (wv + NW * i)), 16, a_off[NAO == 1 ? 0 : i], kb * 256 + (NAO == 1 ? 64 * i : 0), 0, 0);
     };
     auto issue_x = [&](int j, int slot) {
         const int kb = min(kb0 + j, kb1 - 1);
@@ -184,6 +185,7 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__r
     const int nsb = kb1 - kb0;
     const int live = MOE ? (rows - m0 + 31) / 32 : MI;     // 32-row tiles that hold rows: an expert rarely fills its last ones
 
+    constexpr bool STAGGER = DT != CQ_Q6K && NW == 8;      // (four waves have a SIMD each)
     auto body = [&](auto late) {
     constexpr bool LATE = decltype(late)::value;
     int slot = 0, slot1 = 1;                               // ring slots of super-blocks j and j + 1
@@ -371,10 +373,10 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile_kernel(const uint8_t *__r
         slot = slot1;
         slot1 = slot1 == LD::RA - 1 ? 0 : slot1 + 1;
     }
-    if constexpr (!LATE && DT != CQ_Q6K) asm volatile("s_barrier" ::: "memory");       // the others' last one
+    if constexpr (!LATE && STAGGER) asm volatile("s_barrier" ::: "memory");       // the others' last one
     };
-    if constexpr (DT == CQ_Q6K) body(std::false_type{});
-    else if (wv < QT_NW / 2) body(std::false_type{});
+    if constexpr (!STAGGER) body(std::false_type{});
+    else if (wv < NW / 2) body(std::false_type{});
     else body(std::true_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -423,30 +425,34 @@ __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first,
 }
 
 template <int DT>
-int qtile_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
+int qtile_mi(int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
              const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
-#define QT_GO(M, E)                                                                                                                                  \
-    static_assert(QtLds<DT, M>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                 \
-    return qtile_go(qtile_kernel<DT, M, E>, QtLds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+#define QT_GO(M, E, NW)                                                                                                                                \
+    static_assert(QtLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                               \
+    return qtile_go(qtile_kernel<DT, M, E, NW>, NW, QtLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
     if (moe) {
-        if (mi == 1) { QT_GO(1, true); }
-        QT_GO(4, true);
+        if (mi == 1) { QT_GO(1, true, QT_NW); }
+        QT_GO(4, true, QT_NW);
+    }
+    if (nw == QT_NW_NARROW) {
+        if (mi == 1) { QT_GO(1, false, QT_NW_NARROW); }
+        QT_GO(2, false, QT_NW_NARROW);
     }
     switch (mi) {
-        case 1: { QT_GO(1, false); }
-        case 2: { QT_GO(2, false); }
-        case 3: { QT_GO(3, false); }
-        default: { QT_GO(4, false); }
+        case 1: { QT_GO(1, false, QT_NW); }
+        case 2: { QT_GO(2, false, QT_NW); }
+        case 3: { QT_GO(3, false, QT_NW); }
+        default: { QT_GO(4, false, QT_NW); }
     }
 #undef QT_GO
 }
 
-int qtile_any(int w_dtype, int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
+int qtile_any(int w_dtype, int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
               int64_t stride_dst, const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
     switch (w_dtype) {
-        case CQ_Q4K: return qtile_mi<CQ_Q4K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
-        case CQ_Q5K: return qtile_mi<CQ_Q5K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
-        case CQ_Q6K: return qtile_mi<CQ_Q6K>(mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+        case CQ_Q4K: return qtile_mi<CQ_Q4K>(mi, nw, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+        case CQ_Q5K: return qtile_mi<CQ_Q5K>(mi, nw, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
+        case CQ_Q6K: return qtile_mi<CQ_Q6K>(mi, nw, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
     }
     return cq_qtile0_launch(w_dtype, mi, moe, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s);
 }
@@ -469,13 +475,16 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
     return cq_align256(std::min<int64_t>(16 * rows * n, QT_PLANE_FLOATS) * 4);
 }
 
-// Rows of the tile (32 mi) and K splits: the pair for which the model
-//   rounds * (super-blocks per split * (a + b mi) + 1.3) us,  + 6.8 us and the planes at 4.5 TB/s where K is split
-// is least.  A round is 256 workgroups (a tenth slower when all compute units are busy: the clock falls), a the conversion of the weights, b the products
-// and sums of 32 rows.  Fitted to 3800 launches of 17 - 2048 rows against [14336 x 4096], [4096 x 14336], [1024 x 4096] and [5120 x 4096] (6 % rms, 10 % for
-// Q4_0); the choice it makes is 0.2 - 1.2 % slower than the best of all pairs on average, at most 16 % (100 rows of Q4_K: 39.1 against 33.8 us).
+// Rows of the tile (32 mi), waves of a workgroup and K splits: the choice for which the model
+//   rounds * super-blocks per split * (a + b mi) us,  + split + planes / rate where K is split
+// is least.  A round is 256 workgroups, a the conversion of the weights, b the products and sums of 32 rows.  Workgroups of the K formats may have four waves
+// instead of eight if their rows are at most 64: each SIMD then converts and multiplies for one wave, and a small product takes up twice as many
+// compute units (131 rows of Q6_K [4096 x 4096] unsplit: 56 us in eight waves, 41 in four; 65 rows of Q4_K [4096 x 4096] 20.6 -> 17.5).
+// Costs of the K formats: fitted to the choice among 9000 forwards of 9 - 1200 rows against 90 shapes each of 1024 - 16384 by 1024 - 14336, cold weights; it
+// is 0.2 - 0.7 % slower than the best on average, at most 11 %.  Q4_0 and Q8_0 (rounds that leave compute units idle run at a higher clock
+// there, and a workgroup has 1.3 us of its own): 3800 launches of 17 - 2048 rows, 0.2 - 1.2 %.
 // Only splits whose sums round no more than those of the general kernels (qt_roundings).
-struct QtPlan { int mi, splits; };
+struct QtPlan { int mi, nw, splits; };
 // What the f32 sums of one result round, as twice a variance in units of one term's: a chain of c terms takes c fma's, which round partial sums of 1 .. c terms
 // (the first one, a product alone, like one and a half), and every addition of two splits rounds a sum of as many terms as both have.  in_pairs: as
 // qtile_reduce_kernel adds them, else one after the other like the general kernels (cq_qmm_splits).  More splits shorten the chains, but each begins with a
@@ -494,25 +503,32 @@ static int64_t qt_roundings(int64_t nsb, int terms, int splits, bool in_pairs) {
     return total;
 }
 static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_t most_splits) {
-    const int64_t nsb = k / 256, nt = (n + 32 * QT_NW - 1) / (32 * QT_NW);
-    const double a = w_dtype == CQ_Q4K ? 0.7 : w_dtype == CQ_Q5K ? 1.35 : w_dtype == CQ_Q6K ? 2.4 : 1.6;
-    const double b = w_dtype == CQ_Q6K ? 0.65 : cq_is_kquant(w_dtype) ? 0.79 : 1.23, plane = (double)rows * n * 4;
+    const int64_t nsb = k / 256;
+    struct Cost { double a, b, a_narrow, b_narrow, start, split, rate; };                   // us, bytes per us
+    static constexpr Cost q4k{1.25, 0.88, 0.69, 0.39, 0, 2.71, 1.90e6}, q5k{1.80, 0.99, 0.99, 0.53, 0, 3.31, 2.42e6}, q6k{3.12, 1.00, 1.83, 0.65, 0, 5.15, 3.94e6},
+        q0{1.6, 1.23, 0, 0, 1.3, 6.8, 4.5e6};
+    const bool kq = cq_is_kquant(w_dtype);
+    const Cost &c = w_dtype == CQ_Q4K ? q4k : w_dtype == CQ_Q5K ? q5k : w_dtype == CQ_Q6K ? q6k : q0;
+    const double plane = (double)rows * n * 4;
     const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({QT_MAX_SPLITS, nsb, most_splits}));
-    const int terms = cq_is_kquant(w_dtype) ? 1 : 8;
+    const int terms = kq ? 1 : 8;
     const int general = std::min(most, cq_qmm_splits(k, n, rows));
     bool rounds_less[QT_MAX_SPLITS + 1];
     for (int sp = 1; sp <= most; sp++)
         rounds_less[sp] = sp == general || qt_roundings(nsb, terms, sp, true) < qt_roundings(nsb, terms, general, false);
-    QtPlan best{4, general};
+    QtPlan best{4, QT_NW, general};
     double least = 1e30;
-    for (int mi = 1; mi <= 4; mi++)
-        for (int sp = 1; sp <= most; sp++) {
-            if (!rounds_less[sp]) continue;
-            const int64_t wgs = (rows + 32 * mi - 1) / (32 * mi) * nt * sp, rounds = (wgs + 255) / 256;
-            const double load = 1.1 * (rounds - 1) + 1.0 + 0.1 * (double)(wgs - 256 * (rounds - 1)) / 256;
-            const double t = load * ((double)((nsb + sp - 1) / sp) * (a + b * mi) + 1.3) + (sp > 1 ? 6.8 + (sp + 1) * plane / 4.5e6 : 0.0);
-            if (t < least) { least = t; best = {mi, sp}; }
-        }
+    for (int nw : {QT_NW, QT_NW_NARROW})
+        for (int mi = 1; mi <= (nw == QT_NW ? 4 : 2); mi++)
+            for (int sp = 1; sp <= most; sp++) {
+                const int64_t wgs = (rows + 32 * mi - 1) / (32 * mi) * ((n + 32 * nw - 1) / (32 * nw)) * sp, rounds = (wgs + 255) / 256;
+                const bool narrow = nw == QT_NW_NARROW;
+                if (!rounds_less[sp] || (narrow && (!kq || (n + 32 * nw - 1) / (32 * nw) > 65535))) continue;
+                const double load = kq ? (double)rounds : 1.1 * (rounds - 1) + 1.0 + 0.1 * (double)(wgs - 256 * (rounds - 1)) / 256;
+                const double block = narrow ? c.a_narrow + c.b_narrow * mi : c.a + c.b * mi;
+                const double t = load * ((double)((nsb + sp - 1) / sp) * block + c.start) + (sp > 1 ? c.split + (sp + 1) * plane / c.rate : 0.0);
+                if (t < least) { least = t; best = {mi, nw, sp}; }
+            }
     return best;
 }
 
@@ -522,7 +538,7 @@ int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, in
     const bool f32 = dst_dtype == CQ_F32;
     const QtPlan plan = qtile_plan(w_dtype, k, n, rows, planes ? (f32 ? 1 : 0) + plane_bytes / (4 * rows * n) : 1);
     const int splits = plan.splits;
-    const dim3 grid((unsigned)((rows + 32 * plan.mi - 1) / (32 * plan.mi)), (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)), (unsigned)splits);
+    const dim3 grid((unsigned)((rows + 32 * plan.mi - 1) / (32 * plan.mi)), (unsigned)((n + 32 * plan.nw - 1) / (32 * plan.nw)), (unsigned)splits);
     if (grid.y > 65535) return CQ_ERR_RANGE;
     const int64_t count = rows * n;
     const bool direct = splits == 1 || f32;
@@ -530,7 +546,7 @@ int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, in
     const int64_t ld = direct ? stride_dst : n;
     float *const others = direct ? (float *)planes : (float *)planes + count;
     const MoeChunks none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-    const int rc = qtile_any(w_dtype, plan.mi, false, grid, w, av, first, direct ? dst_dtype : CQ_F32, k, n, rows, ld, none, 0, others, s);
+    const int rc = qtile_any(w_dtype, plan.mi, plan.nw, false, grid, w, av, first, direct ? dst_dtype : CQ_F32, k, n, rows, ld, none, 0, others, s);
     if (rc || splits == 1) return rc;
     const dim3 rg((unsigned)((count / 4 + QT_RT - 1) / QT_RT));
     if (f32) hipLaunchKernelGGL(qtile_reduce_kernel<CQ_F32>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
@@ -543,5 +559,5 @@ int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, in
 int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s) {
     const dim3 grid((unsigned)mc.max_chunks, (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)));
     if (grid.y > 65535) return CQ_ERR_RANGE;
-    return qtile_any(w_dtype, tile_rows / 32, true, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
+    return qtile_any(w_dtype, tile_rows / 32, QT_NW, true, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
 }

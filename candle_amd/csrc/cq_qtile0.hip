@@ -225,7 +225,7 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
 template <int DT>
 static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                      const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
-#define Q0_GO(M, E) return qtile_go(qtile0_kernel<DT, M, E>, Q0Lds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+#define Q0_GO(M, E) return qtile_go(qtile0_kernel<DT, M, E>, QT_NW, Q0Lds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
     if (moe) { if (mi == 1) Q0_GO(1, true); else Q0_GO(4, true); }
     switch (mi) {
         case 1: Q0_GO(1, false);

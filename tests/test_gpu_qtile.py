@@ -69,6 +69,20 @@ def test_tile_edges(fmt, m, n, k):
     check(fmt, m, n, k)
 
 
+@pytest.mark.parametrize("fmt", ["q4k", "q5k", "q6k"])
+@pytest.mark.parametrize("m,n,k", [(33, 129, 1536), (64, 127, 1792), (140, 9002, 1536), (17, 33030, 1536), (300, 9002, 1536), (600, 9002, 1536), (800, 9002, 1536)])
+def test_workgroups_of_four_and_eight_waves(fmt, m, n, k):
+    """The shapes that qtile_plan gives workgroups of four waves with tiles of 32, 32 and 64 rows, then of eight with 32, 64 (Q4_K: of four), 96 and 128.
+    Against 64 bits on the same rounded activations."""
+    from perf import cases
+    name = {"q4k": "q4_k", "q5k": "q5_k", "q6k": "q6_k"}[fmt]
+    b = cases.blocks(name, 3, "w", n, k)
+    w, x = cases.values(name, b, n, k), normal(9 + n, (m, k))
+    want = cases.product(name, torch.from_numpy(x).cuda(), w).cpu().numpy()
+    got = run(FMT[fmt][0], b.reshape(-1).cpu().numpy(), x, n)
+    assert row_error(got, want, x, w.cpu().numpy(), k) <= BOUND
+
+
 @pytest.mark.parametrize("fmt", FMT)
 @pytest.mark.parametrize("out", [1, 30])
 @pytest.mark.parametrize("n,k", [(130, 512), (260, 4096)])
