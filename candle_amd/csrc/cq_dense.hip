@@ -106,13 +106,14 @@ __device__ __forceinline__ void tile_at(int t, int tiles_m, int tiles_n, int &tm
 // eight 16-byte chunks, chunk c of row r at c ^ (r / 2) % 8, without bank conflicts; c ^ r % 8, with two lanes to a bank, for the large tile of f32 activations,
 // where it is all the same 2 % faster (1500 x 5632 x 2048: 75.7 us against 77.2).
 // Three stages are on their way for the large tile of bf16 activations (the cold weights of a model's experts and layers: 1500 tokens of Kudurax 2347 -> 2270 us;
-// on warm operands 1500 x 5632 x 2048 66 -> 63), one for the others: f32 activations and small tiles gain nothing from more (40 x 4096 x 4096: 13.3 -> 14.2).
-// XB: the activations are bfloat16.  With a table of tiles (grouped products) the rows of a tile share the weights of one group.
-template <int BM, int BN, int WGM, int WGN, bool XB>
+// on warm operands 1500 x 5632 x 2048 66 -> 63), one for the others: f32 activations and small tiles gain nothing from more (40 x 4096 x 4096: 13.3 -> 14.2), and
+// workgroups of up to 12 stages (a split of k, short rows) lose by it: the three past the end are brought all the same (700 x 2048 x 2048 in six splits 26.4 us
+// with one, 28.1 with three; 4 - 11 stages 4 % slower on average, 13 - 16 none, from 18 on faster).
+// XB: the activations are bfloat16; PF: stages on their way.  With a table of tiles (grouped products) the rows of a tile share the weights of one group.
+template <int BM, int BN, int WGM, int WGN, bool XB, int PF = 1>
 __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n, int k_split) {
     constexpr int XV = XB ? 1 : 2;                         // 16-byte loads per eight activations
     constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, CA = BM * 8 / 256, CB = BN * 8 / 256;
-    constexpr int PF = BM == 128 && XB ? 3 : 1;            // stages on their way
     constexpr int SW = BM == 128 && !XB ? 0 : 1;
     __shared__ bf16x8 lds[2][(BM + BN) * 8];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -703,6 +704,7 @@ int cq_dense_product(int precision, const cq_dense_args *args, void *workspace_d
         const int tm = (int)((m + DT_B - 1) / DT_B), tn = (int)((n + DT_B - 1) / DT_B);
         hipLaunchKernelGGL(fn, dim3((unsigned)(tm * tn)), dim3(512), 2 * DT_STAGE, s, src, o, m, (int)n, (int)k, tm, tn);
     }
+    else if (p.bm == 128 && a.x_bf16 && p.k_split > 12 * 64) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, true, 3>));
     else if (p.bm == 128 && a.x_bf16) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, true>));
     else if (p.bm == 128) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, false>));
     else if (p.bm == 64 && a.x_bf16) CQ_DM((dense_bf16_kernel<64, 64, 2, 2, true>));

@@ -51,3 +51,26 @@ def test_edges(m, n, k, pad, x_bf16, form):
         err = (err - want.abs() * 2.0 ** -8).clamp(min=0)
     assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * (4 if form == "swiglu" else 1)      # (silu and the gate: slopes up to 1.1, values to 4)
     assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, cols:] == 5).all()
+
+
+@pytest.mark.parametrize("k", [512, 768, 832, 896, 960])
+@pytest.mark.parametrize("splits", [False, True])
+def test_stages_on_their_way(k, splits):
+    """The 128 x 128 tile of bfloat16 rows: up to 12 stages of k a workgroup with one of them on its way, beyond with three; all remainders of three."""
+    m, n = (2000, 3201) if not splits else (700, 1157)
+    k = k if not splits else 9 * k                         # 60 tiles: nine splits
+    g = torch.Generator(device="cuda").manual_seed(k)
+    w = torch.randn((n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k), generator=g, device="cuda").bfloat16()
+    y = torch.full((m + 2, n + 3), 5.0, device="cuda")
+    L = _lib.mixer_lib()
+    nb = L.cq_dense_matmul_workspace_bytes(0, m, n, k)
+    assert (nb > 0) == splits
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    a = DenseArgs(w_dev=w.data_ptr(), ldw=k, x_dev=x.data_ptr(), ldx=k, x_bf16=1, dst_dev=y[1].data_ptr(), ldd=n + 3, m=m, n=n, k=k, batch=1)
+    _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    want = x.double() @ w.double().t()
+    err = (y[1:m + 1, :n].double() - want).norm(dim=1) / want.norm(dim=1)
+    assert float(err.max()) <= BOUND
+    assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, n:] == 5).all()
