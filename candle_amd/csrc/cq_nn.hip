@@ -1103,7 +1103,7 @@ constexpr int ROUTE_MAX_EXPERTS = 1024, ROUTE_MAX_TOPK = 64;
 // T: tokens per wave (blockIdx.y is a group of T tokens): with hundreds of tokens the router rows a wave has loaded serve T
 // tokens instead of one (one token per wave re-reads the 1 MB router matrix once per token: 14 us for 256 tokens).  What bounds it there is the L2: <4, 2, 2>
 // asks for 48 KB of a 2048-element row set per eight logits, <8, 1, 8> for 128 KB per 64 (1500 tokens, 128 experts: 45 -> 24 us).  That one needs 1024 waves'
-// worth of logits, 65536 of them, to fill the chip.
+// worth of logits, 65536 of them, to fill the chip, and of short rows some more (rows of 1024: 76800 logits 14.2 -> 15.1 us, 96000 16.0 -> 15.1).
 template <int R, int C, int T = 1>
 __global__ __launch_bounds__(256) void moe_logits_kernel(const float *__restrict__ x, const float *__restrict__ router_w, float *__restrict__ logits,
                                                          int hidden, int n_experts, int tokens) {
@@ -1594,7 +1594,7 @@ int cq_nn_moe_route(const float *x_dev, const float *router_w_dev, uint32_t *top
     else if (tokens * num_experts <= 16384)
         hipLaunchKernelGGL((moe_logits_kernel<4, 2>), dim3((unsigned)((num_experts + 15) / 16), (unsigned)tokens), dim3(256), 0, (hipStream_t)stream, x_dev,
                            router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
-    else if (tokens * num_experts < 65536)
+    else if (tokens * num_experts < (hidden < 2048 ? 90112 : 65536))
         hipLaunchKernelGGL((moe_logits_kernel<4, 2, 2>), dim3((unsigned)((num_experts + 15) / 16), (unsigned)((tokens + 1) / 2)), dim3(256), 0,
                            (hipStream_t)stream, x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
     else

@@ -12,7 +12,7 @@ from tests.util import normal, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,experts,hidden", [(1027, 64, 516), (513, 128, 2048), (700, 100, 260), (8200, 8, 64)])
+@pytest.mark.parametrize("tokens,experts,hidden", [(1027, 64, 516), (513, 128, 2048), (700, 100, 260), (8200, 8, 64), (1407, 64, 516), (1409, 64, 516), (1001, 100, 260), (12300, 8, 64), (511, 128, 2048)])
 def test_router_logits(tokens, experts, hidden):
     """Against float64.  hidden products summed lane by lane (hidden / 64 in a row) and over 64 lanes: below 2^-24 * (hidden / 64 + 6) of the terms' sum."""
     print(f"case {tokens} {experts} {hidden}", flush=True)
