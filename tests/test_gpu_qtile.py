@@ -148,10 +148,10 @@ def test_extreme_super_block_scales(fmt, bb, at, d):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q6k", "q5k"])
 @pytest.mark.parametrize("tokens", [70, 1200])
-@pytest.mark.parametrize("E,n", [(5, 268), (4, 267)])
+@pytest.mark.parametrize("E,n", [(5, 268), (4, 267), (3, 1028)])
 def test_grouped_experts(fmt, tokens, E, n):
     """A few experts with tiles of 32 and of 128 rows, the last ones part full, columns past the last workgroup's; Q6_K: an odd number of blocks a row, and of
-    rows too: every second expert begins 2 bytes past a dword."""
+    rows too: every second expert begins 2 bytes past a dword; Q4_0: 32-row tiles of up to 1024 columns are the general kernel's."""
     import candle_amd as ca
     code, odt = FMT[fmt]
     k, topk = 1792, 2
