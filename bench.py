@@ -210,9 +210,10 @@ def prefill_record(L, torch, fmt, n, k, m, steps=20, warmup=5, pmc=False):
     def quantize_only():
         _lib.check("cq_quantize_act", L.cq_quantize_act(dt, x.data_ptr(), 0, ws.data_ptr(), k, m, sp))
 
-    # whether the workspace has room for planes of a split K, which a second kernel adds up (the library splits where that fills the chip better)
+    # small grids split K into partial planes that a second kernel adds up (the workspace then holds those planes too); the kernels of the formats
+    # below always have room for planes and choose by themselves: not known here
     act_bytes = L.cq_act_scratch_bytes(dt, k, m)
-    split_k = ws_bytes > act_bytes + ((m * n * 4 + 255) // 256) * 256
+    split_k = None if fmt in ("q4k", "q5k", "q6k", "q4_0", "q8_0") else ws_bytes > act_bytes + ((m * n * 4 + 255) // 256) * 256
 
     if pmc:
         with torch.cuda.stream(stream):
@@ -256,7 +257,7 @@ def prefill_record(L, torch, fmt, n, k, m, steps=20, warmup=5, pmc=False):
     achieved = flops / (kern_us * 1e-6) / 1e12
     return {"fmt": fmt, "n": n, "k": k, "m": m, "steps": steps, "warmup": warmup, "forward_ms": round(ms, 5),
             "forward_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1), "kernel": ("qtile_kernel<%s>" if fmt in ("q4k", "q5k", "q6k") else "qtile0_kernel<%s>" if fmt in ("q4_0", "q8_0") else "qmm_q0_i8_kernel<%s>" if i8 else "qmm_kernel<%s>") % fmt,
-            "split_k": bool(split_k), "quantize_us": round(q_us, 2),
+            "split_k": split_k, "quantize_us": round(q_us, 2),
             "kernel_us": round(kern_us, 2), "kernel_median_us": round(kst["median"], 2), "kernel_p10_us": round(kst["p10"], 2),
             "kernel_p90_us": round(kst["p90"], 2), "kernel_TFLOPs": round(achieved, 1), "mfma": "i8" if i8 else "f16", "peak": peak,
             "frac": round(achieved / peak, 4)}
