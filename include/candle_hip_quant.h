@@ -119,10 +119,11 @@ int cq_matvec(int w_dtype, const void *w_dev, const void *act_scratch_dev, void 
 
 /* ---------------------------------------------------------------------------------------------
  * Prefill matmul over pre-quantized activations (any rows >= 1): more than CQ_MATVEC_MAX_ROWS rows (Q4K: from 6 rows) with k a
- * multiple of 256 run on the matrix cores, every format integer-exact: Q4K, Q4_0, Q8_0, Q4_1, Q5_0, Q5_1 on the int8 cores (the
- * 32-element formats as one int8 MFMA per block, whose int32 result is the block sum the CPU forms; their weights must be 8-byte
- * aligned), Q2K, Q3K, Q5K, Q6K on the f16 cores with operands that are exact small integers.  Other shapes take 8 rows per
- * matvec pass.
+ * multiple of 256 run on the matrix cores, every format integer-exact: Q4K, Q5K, Q6K, Q4_0, Q8_0 on the int8 cores; Q4_1, Q5_0, Q5_1 there
+ * too, in a slower kernel; Q2K, Q3K on the f16 cores with operands that are exact small integers.  Where weights lie matters: Q4_0 and Q8_0
+ * that are not 16-byte aligned take the slower kernel of Q4_1, and any 32-element format that is not 8-byte aligned 8 rows per matvec pass, as
+ * other k do; Q6K takes the f16 cores if k < 1536, if the tensor is not 4-byte aligned, or if it has an odd number of blocks (n k / 256).
+ * cq_matmul has no room to split k in: cq_qmatmul_forward, which has, is the faster call where n and rows are small.
  * Counterpart of launch_mmq_gguf_<t> (candle-core/src/quantized/fast_mmq.rs:71-111, candle-kernels/src/mmq_gguf/).
  * Same buffers as cq_matvec; dst is f32.
  * ------------------------------------------------------------------------------------------- */
