@@ -787,8 +787,8 @@ int cq_qmm_splits(int64_t k, int64_t n, int64_t rows) {
     const int64_t base = rows <= CQ_QMM_SMALL_ROWS ? ((rows + 31) / 32) * ((n + 127) / 128) : ((rows + BM - 1) / BM) * ((n + 63) / 64);
     const int64_t nsb = k / 256;
     // about two workgroups per CU: one converts operands while the other feeds the matrix cores (measured against a target
-    // of one per CU: Q6_K 4096 x 14336 at 128 / 256 / 512 rows 69 / 131 / 248 -> 57 / 105 / 200 us, Q4_K 4096 x 4096 at 512
-    // rows 67 -> 54 us; three per CU is no better)
+    // of one per CU, Q6_K 4096 x 14336, which now comes here unaligned only, at 128 / 256 / 512 rows 69 / 131 / 248 -> 57 / 105 / 200 us;
+    // three per CU is no better).  The kernels of cq_qtile.h split as it suits them, but with no more rounding than this split has
     const int64_t target = 512;
     if (base >= target * 3 / 4 || nsb < 8) return 1;
     int64_t sp = (target + base - 1) / base;
@@ -797,9 +797,9 @@ int cq_qmm_splits(int64_t k, int64_t n, int64_t rows) {
     return sp < 2 ? 1 : (int)sp;
 }
 
-// Which row counts go to the matrix cores: everything beyond the matvec kernel's 8 rows, and for Q4_K, whose int8 kernel is
-// the faster one, from 6 rows (measured, Q4_K 14336 x 4096 / 4096 x 14336 in us: matvec at 4 / 5 / 6 / 8 rows 19.4 / 21.6 /
-// 23.4 / 27.5 and 18.3 / 20.8 / 23.6 / 29.9, the 32-row MFMA tile 20.7 and 22.3 at any of them, 21.3 / 23.0 at 16 / 32 rows).
+// Which row counts go to the matrix cores: everything beyond the matvec kernel's 8 rows, and Q4_K from 6 rows.  Of cq_qmatmul_forward that line concerns what
+// the batched matvec does not take, rows of more than 16384: 4096 x 20480 at 5 rows 25.1 us on the matvec kernel, at 6 / 8 rows 21.2 / 21.6 on the matrix cores
+// (matvec and quantizing 28.8 / 38.6).  cq_matmul, which splits no k, pays for it: 6 / 8 rows of 4096 x 4096 18.6 / 18.7 us, cq_matvec 9.4 / 11.1.
 constexpr int CQ_Q4K_MFMA_MIN_ROWS = 6;
 bool cq_use_mfma(int w_dtype, int64_t rows, int64_t k) {
     if (k % 256 || !cq_has_mfma(w_dtype)) return false;

@@ -463,8 +463,9 @@ static constexpr int64_t QT_Q6K_MIN_K = 1536;
 bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
     if (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K) return k % 256 == 0;
     if (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) return k % 256 == 0 && ((uintptr_t)w & 15) == 0;      // (rows are multiples of 16 bytes)
-    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one.  Its two half super-blocks in flight need some of k to pay (67 / 300 rows
-    // of [4096 x 768] 17.6 / 18.9 us against 16.8 / 17.6 of the general kernel, of [8192 x 1024] 21.3 at 67 against 20.2; from 2048 on it is the faster one)
+    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one.  Its two half super-blocks in flight need some of k to pay (in eight
+    // waves 67 / 300 rows of [4096 x 768] took 17.6 / 18.9 us against 16.8 / 17.6 of the general kernel, of [8192 x 1024] 21.3 at 67 against 20.2).  From 1536 on it is
+    // the faster one whatever the rows (9 / 131 / 300 / 2048 rows of [4096 x 1536] 12.9 / 20.6 / 24.0 / 49.8 us against 26.9 / 25.5 / 26.3 / 77.3)
     return w_dtype == CQ_Q6K && k % 256 == 0 && k >= QT_Q6K_MIN_K && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
 }
 
