@@ -6,8 +6,10 @@
 // 13 bits, so it goes through the int8 cores as two operands in two chains: Q4_K as scale % 8 * q and scale / 8 * q (S = lo + 8 hi), Q5_K and Q6_K as the
 // low byte less 128 and the high byte of scale * q + 128 (S = lo + 256 hi).
 //
-// What bounds it: at many rows the matrix cores at the clock that the power limit leaves (16 + 1 MFMAs of 32 x 32 x 32 per 32 rows, super-block and wave, about
-// 20 ns each with all units busy, 14.5 at the full clock), with the conversion of the weights behind it; at few rows the weights' way from memory.  So:
+// What bounds it: at many rows matrix and vector instructions together, at the 1.9 GHz that the power limit leaves.  Of the SIMDs' cycles at 2048 rows the matrix
+// cores take 39 % with Q4_K and 35 % with Q5_K and Q6_K (16 + 1 MFMAs of 32 x 32 x 32 per 32 rows, super-block and wave), the vector units 43, 55 and 54 %
+// (conversion, and the sums of a super-block), and the two waves of a SIMD overlap them only in part.  At few rows the weights' way from memory, and
+// in unsplit small products the chain of one wave a SIMD.  So:
 //  - a workgroup is eight waves (or four: qtile_plan) side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
 //    multiplies it, straight into its operand registers (the kernels before this one staged converted weights in LDS, and the conversion
 //    of Q5_K and Q6_K was to f16, Q6_K as two f16 terms: twice the matrix time of int8);
