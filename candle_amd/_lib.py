@@ -149,6 +149,8 @@ MIXER_SIGNATURES.update({
     "cq_mix_moe_step_fits": (_int, [_moe]),
     "cq_mix_moe_step": (_int, [_moe, _vp, _int, _vp, _f32, _i64, _vp, _vp, _vp, _vp, _vp]),
 })
+# the same calls with results in bfloat16
+MIXER_SIGNATURES.update({f"cq_mix_{n}_bf16": MIXER_SIGNATURES[f"cq_mix_{n}"] for n in ("rms_norm_rows", "poly_norm", "tanh", "head_norm_gate", "talk_attention")})
 # glue that the mixer library carries as well
 _MIXER_GLUE = ("cq_status_string", "cq_nn_embedding", "cq_nn_argmax")
 

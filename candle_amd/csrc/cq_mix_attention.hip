@@ -20,10 +20,10 @@ template <typename T> __device__ __forceinline__ T ld_at(const float *base, uint
 // query rows to fill the chip; a split leaves unnormalized outputs with their maximum and sum, talk_combine_kernel merges them.
 // LDS strides: query rows of KT + 4 floats (16 rows x 4 keys of an operand read fall on 64 banks), head blocks of 16 rows + 16
 // (4 heads x 16 keys likewise).
-template <int NW, int NHW, bool SHARED_K, int U, int VS, int KT>
+template <int NW, int NHW, bool SHARED_K, int U, int VS, int KT, typename OT>
 __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__restrict__ q, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
                                                              const float *__restrict__ talk, float scale, int window, int keep_first, float out_scale,
-                                                             float *__restrict__ out, int64_t out_stride, float *__restrict__ part, int pos, int rows, int H, int G,
+                                                             OT *__restrict__ out, int64_t out_stride, float *__restrict__ part, int pos, int rows, int H, int G,
                                                              int dp, int vdim, int vp, int ctx) {
     constexpr int NHT = (NW * NHW + 15) / 16, HP = 16 * NHT, NT = 64 * NW, RW = 16 / NW;       // heads padded to tiles of 16; queries per wave
     constexpr int RS = KT + 4, HS = 16 * RS + 16, TS = HP + 4, KTL = KT / 16;
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__
             for (int e = 0; e < 4; e++) {
                 const int row = 4 * lk + e;
                 if (row >= nr) continue;
-                if (nz == 1) out[(int64_t)(r0 + row) * out_stride + (int64_t)h * vdim + col] = out_scale * o[u][n][e] / l_run[h * 16 + row];
+                if (nz == 1) out[(int64_t)(r0 + row) * out_stride + (int64_t)h * vdim + col] = (OT)(out_scale * o[u][n][e] / l_run[h * 16 + row]);
                 else part[((int64_t)(z * rows + r0 + row) * H + h) * vdim + col] = o[u][n][e];
             }
         }
@@ -223,8 +223,9 @@ __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__
 }
 
 // one wave per (row, head)
+template <typename OT>
 __global__ __launch_bounds__(256) void talk_combine_kernel(const float *__restrict__ part, int nz, int64_t rows, int H, int vdim, float out_scale,
-                                                           float *__restrict__ out, int64_t out_stride) {
+                                                           OT *__restrict__ out, int64_t out_stride) {
     const int lane = threadIdx.x & 63, h = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (h >= H) return;
     const int64_t r = blockIdx.x, id = r * H + h, n = rows * H;
@@ -232,14 +233,14 @@ __global__ __launch_bounds__(256) void talk_combine_kernel(const float *__restri
     float m = -INFINITY, l = 0.0f;
     for (int z = 0; z < nz; z++) m = fmaxf(m, ml[2 * n * z]);
     for (int z = 0; z < nz; z++) l = fmaf(ml[2 * n * z] > -INFINITY ? __expf(ml[2 * n * z] - m) : 0.0f, ml[2 * n * z + 1], l);
-    float *o = out + r * out_stride + (int64_t)h * vdim;
+    OT *o = out + r * out_stride + (int64_t)h * vdim;
     for (int e = lane; e < vdim; e += 64) {
         float a = 0.0f;
         for (int z = 0; z < nz; z++) {
             const float w = ml[2 * n * z] > -INFINITY ? __expf(ml[2 * n * z] - m) : 0.0f;
             a = fmaf(w, part[(n * z + id) * vdim + e], a);
         }
-        o[e] = out_scale * a / l;
+        o[e] = (OT)(out_scale * a / l);
     }
 }
 
@@ -255,21 +256,21 @@ int talk_unit_blocks(int64_t H, int64_t vp) {               // units a launch ta
     return (int)((H * ((vp + 63) / 64) + per - 1) / per);
 }
 
-template <int NW, int NHW, bool SHARED_K, int U, int VS, int KT>
-int talk_launch(const float *q, const float *kc, const float *vc, const float *talk, float scale, int window, int keep, float out_scale, float *out,
+template <int NW, int NHW, bool SHARED_K, int U, int VS, int KT, typename OT>
+int talk_launch(const float *q, const float *kc, const float *vc, const float *talk, float scale, int window, int keep, float out_scale, OT *out,
                 int64_t out_stride, float *part, int nz, int pos, int rows, int H, int G, int dp, int vdim, int vp, int ctx, hipStream_t s) {
     constexpr int HP = (NW * NHW + 15) / 16 * 16;
     constexpr size_t lds = (size_t)(HP * (16 * (KT + 4) + 16) + HP * (HP + 4) + 3 * HP * 16) * sizeof(float);
     if (lds > 64 * 1024) {
-        const int e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(talk_attention_kernel<NW, NHW, SHARED_K, U, VS, KT>),
+        const int e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(talk_attention_kernel<NW, NHW, SHARED_K, U, VS, KT, OT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e) return e;
     }
     const int units = H * ((vp + 63) / 64);
-    hipLaunchKernelGGL((talk_attention_kernel<NW, NHW, SHARED_K, U, VS, KT>), dim3((rows + 15) / 16, (units + NW * U - 1) / (NW * U), nz), dim3(64 * NW), lds,
+    hipLaunchKernelGGL((talk_attention_kernel<NW, NHW, SHARED_K, U, VS, KT, OT>), dim3((rows + 15) / 16, (units + NW * U - 1) / (NW * U), nz), dim3(64 * NW), lds,
                        s, q, kc, vc, talk, scale, window, keep, out_scale, out, out_stride, part, pos, rows, H, G, dp, vdim, vp, ctx);
     if (nz > 1)
-        hipLaunchKernelGGL(talk_combine_kernel, dim3((unsigned)rows, (unsigned)((H + 3) / 4)), dim3(256), 0, s, (const float *)part, nz, (int64_t)rows, H, vdim, out_scale,
+        hipLaunchKernelGGL(talk_combine_kernel<OT>, dim3((unsigned)rows, (unsigned)((H + 3) / 4)), dim3(256), 0, s, (const float *)part, nz, (int64_t)rows, H, vdim, out_scale,
                            out, out_stride);
     return (int)hipGetLastError();
 }
@@ -507,19 +508,16 @@ int talk_decode_launch(const float *row, const cq_mix_heads *g, float eps, const
     return (int)hipGetLastError();
 }
 
-}  // namespace
-
-extern "C" {
-
-int64_t cq_mix_talk_attention_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos) {
+int64_t talk_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos) {
     if (rows <= 0 || n_head <= 0 || vdim <= 0 || window < 1 || keep_first < 0 || pos < 0) return 0;
     const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, (vdim + 15) / 16 * 16), talk_max_keys(window, keep_first, pos + rows));
     return nz > 1 ? nz * rows * n_head * (vdim + 2) * 4 : 0;
 }
 
-int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,
-                          int64_t keep_first, float out_scale, float *out_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
-                          int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes, void *stream) {
+template <typename OT>
+int talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,
+                   int64_t keep_first, float out_scale, OT *out_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
+                   int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes, void *stream) {
     if (rows < 0 || pos < 0 || n_head <= 0 || n_kv_head <= 0 || n_head % n_kv_head || dim_pad <= 0 || dim_pad % 16 || vdim <= 0 || 
         vdim_pad != (vdim + 15) / 16 * 16 || ctx <= 0 || window < 1 || keep_first < 0 || out_stride < n_head * vdim)
         return CQ_ERR_SHAPE;
@@ -531,7 +529,7 @@ int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const fl
     const int w = (int)(window < ctx ? window : ctx), keep = (int)(keep_first < ctx ? keep_first : ctx);
     const int H = (int)n_head, G = (int)n_kv_head, R = H / G;
     const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vdim_pad), talk_max_keys(window, keep_first, pos + rows));
-    if (nz > 1 && (!workspace_dev || workspace_bytes < cq_mix_talk_attention_workspace_bytes(rows, n_head, vdim, window, keep_first, pos))) return CQ_ERR_WORKSPACE;
+    if (nz > 1 && (!workspace_dev || workspace_bytes < talk_workspace_bytes(rows, n_head, vdim, window, keep_first, pos))) return CQ_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
 #define CQ_TA(NW_, NHW_, SH_, U_, VS_, KT_)                                                                                                            \
     talk_launch<NW_, NHW_, SH_, U_, VS_, KT_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride,      \
@@ -541,6 +539,28 @@ int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const fl
     if (H <= 32) return R % 2 ? CQ_TA(16, 2, false, 4, 1, 32) : (R % 4 ? CQ_TA(16, 2, true, 4, 2, 32) : CQ_TA(16, 2, true, 4, 4, 32));
     return R % 4 ? CQ_TA(16, 4, false, 4, 1, 16) : CQ_TA(16, 4, true, 4, 4, 16);
 #undef CQ_TA
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t cq_mix_talk_attention_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos) {
+    return talk_workspace_bytes(rows, n_head, vdim, window, keep_first, pos);
+}
+
+int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,
+                          int64_t keep_first, float out_scale, float *out_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
+                          int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes, void *stream) {
+    return talk_attention(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, window, keep_first, out_scale, out_dev, out_stride, pos, rows, n_head, n_kv_head, dim_pad, vdim,
+                          vdim_pad, ctx, workspace_dev, workspace_bytes, stream);
+}
+
+int cq_mix_talk_attention_bf16(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,
+                               int64_t keep_first, float out_scale, void *out_bf16_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
+                               int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes, void *stream) {
+    return talk_attention(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, window, keep_first, out_scale, (__bf16 *)out_bf16_dev, out_stride, pos, rows, n_head, n_kv_head,
+                          dim_pad, vdim, vdim_pad, ctx, workspace_dev, workspace_bytes, stream);
 }
 
 int64_t cq_mix_talk_decode_workspace_bytes(int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t ctx) {

@@ -1,5 +1,6 @@
 // Row operations around the sequence mixers: norms of rows and heads, the normalized polynomial activation, rotation of head
 // groups on their way into packed buffers and caches.
+#include "cq_dense.h"
 #include "cq_mix.h"
 
 namespace {
@@ -12,15 +13,23 @@ __device__ __forceinline__ float block_sum(float v, float *red) {        // 256 
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-template <bool VEC>
+// Results are f32, or bfloat16 where only a bf16 product reads them: the product would round them to the same values on their way into LDS, but reads half as
+// many bytes (each row once per column tile) and can bring them there by copies.  2048 rows x 2048: product with 7168 weight rows 98 -> 82 us, with 2048 48 -> 40,
+// with 10368 148 -> 133; a prompt of 2048 tokens of the width-2048 decoder 3981 -> 3710 us (the poly norm, its row kept in registers, 30 -> 18 a layer).
+__device__ __forceinline__ void store4(float *o, const f32x4 &v) { *reinterpret_cast<f32x4 *>(o) = v; }
+__device__ __forceinline__ void store4(__bf16 *o, const f32x4 &v) {
+    *reinterpret_cast<bf16x4 *>(o) = bf16x4{(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+}
+
+template <bool VEC, typename T>
 __global__ __launch_bounds__(256) void rms_norm_rows_kernel(float *x, int64_t x_stride, const int32_t *__restrict__ index, const float *__restrict__ delta,
-                                                            int64_t delta_stride, const float *__restrict__ w, float *__restrict__ out,
+                                                            int64_t delta_stride, const float *__restrict__ w, T *__restrict__ out,
                                                             int64_t out_stride, int dim, float eps) {
     __shared__ float red[4];
     const int64_t r = blockIdx.x;
     float *xr = x + (index ? (int64_t)index[r] : r) * x_stride;
     const float *dr = delta ? delta + r * delta_stride : nullptr;
-    float *o = out + r * out_stride;
+    T *o = out + r * out_stride;
     constexpr int KEEP = 4;                        // float4 per thread kept in registers (dim <= 4096)
     if (VEC) {
         const int n4 = dim >> 2;
@@ -47,7 +56,7 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(float *x, int64_t x_
         const float m = sqrtf(block_sum(acc, red) / (float)dim + eps);
         auto emit = [&](int i, const f32x4 &v) {
             const f32x4 a = reinterpret_cast<const f32x4 *>(w)[i];
-            reinterpret_cast<f32x4 *>(o)[i] = f32x4{v.x / m * a.x, v.y / m * a.y, v.z / m * a.z, v.w / m * a.w};
+            store4(o + 4 * i, f32x4{v.x / m * a.x, v.y / m * a.y, v.z / m * a.z, v.w / m * a.w});
         };
 #pragma unroll
         for (int c = 0; c < KEEP; c++) {
@@ -63,7 +72,7 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(float *x, int64_t x_
             acc = fmaf(v, v, acc);
         }
         const float m = sqrtf(block_sum(acc, red) / (float)dim + eps);
-        for (int i = threadIdx.x; i < dim; i += 256) o[i] = xr[i] / m * w[i];
+        for (int i = threadIdx.x; i < dim; i += 256) o[i] = (T)(xr[i] / m * w[i]);
     }
 }
 
@@ -104,34 +113,52 @@ __global__ __launch_bounds__(256) void layer_norm_rows_kernel(const float *__res
     for (int i = threadIdx.x + 256 * KEEP; i < dim; i += 256) emit(i, xr[i]);
 }
 
-// sum over n = 1..3 of coef[n-1] z^n / rms(z^n), plus coef[3]: one workgroup per row, the row re-read after its three sums
-__global__ __launch_bounds__(256) void poly_norm_kernel(const float *z, int64_t z_stride, const float *__restrict__ coef, float *out, int64_t out_stride,
+// sum over n = 1..3 of coef[n-1] z^n / rms(z^n), plus coef[3]: one workgroup per row.  The bound is memory: the first KEEP * 256 values are requested together and
+// stay in registers between the three sums and the result, so that a row is read once.
+template <typename T>
+__global__ __launch_bounds__(256) void poly_norm_kernel(const float *z, int64_t z_stride, const float *__restrict__ coef, T *out, int64_t out_stride,
                                                         int dim, float eps) {
     __shared__ float red[4];
     const float *zr = z + (int64_t)blockIdx.x * z_stride;
-    float *o = out + (int64_t)blockIdx.x * out_stride;
-    float s2 = 0.0f, s4 = 0.0f, s6 = 0.0f;
-    for (int i = threadIdx.x; i < dim; i += 256) {
-        const float v = zr[i], q = v * v;
+    T *o = out + (int64_t)blockIdx.x * out_stride;
+    constexpr int KEEP = 32;
+    float keep[KEEP], s2 = 0.0f, s4 = 0.0f, s6 = 0.0f;
+    auto count = [&](float v) {
+        const float q = v * v;
         s2 += q;
         s4 = fmaf(q, q, s4);
         s6 = fmaf(q * q, q, s6);
+    };
+#pragma unroll
+    for (int c = 0; c < KEEP; c++) {
+        const int i = threadIdx.x + 256 * c;
+        keep[c] = i < dim ? zr[i] : 0.0f;
     }
+#pragma unroll
+    for (int c = 0; c < KEEP; c++) count(keep[c]);
+    for (int i = threadIdx.x + 256 * KEEP; i < dim; i += 256) count(zr[i]);
     const float inv = 1.0f / (float)dim;
     const float i1 = coef[0] / sqrtf(block_sum(s2, red) * inv + eps);
     const float i2 = coef[1] / sqrtf(block_sum(s4, red) * inv + eps);
     const float i3 = coef[2] / sqrtf(block_sum(s6, red) * inv + eps);
     const float e = coef[3];
-    for (int i = threadIdx.x; i < dim; i += 256) {
-        const float v = zr[i], q = v * v;
-        o[i] = fmaf(i1, v, fmaf(i2, q, fmaf(i3, q * v, e)));
+    auto value = [&](float v) {
+        const float q = v * v;
+        return (T)fmaf(i1, v, fmaf(i2, q, fmaf(i3, q * v, e)));
+    };
+#pragma unroll
+    for (int c = 0; c < KEEP; c++) {
+        const int i = threadIdx.x + 256 * c;
+        if (i < dim) o[i] = value(keep[c]);
     }
+    for (int i = threadIdx.x + 256 * KEEP; i < dim; i += 256) o[i] = value(zr[i]);
 }
 
-__global__ __launch_bounds__(256) void tanh_kernel(const float *x, int64_t x_stride, float *out, int64_t out_stride, int dim) {
+template <typename T>
+__global__ __launch_bounds__(256) void tanh_kernel(const float *x, int64_t x_stride, T *out, int64_t out_stride, int dim) {
     const float *xr = x + (int64_t)blockIdx.x * x_stride;
-    float *o = out + (int64_t)blockIdx.x * out_stride;
-    for (int i = threadIdx.x; i < dim; i += 256) o[i] = tanhf(xr[i]);
+    T *o = out + (int64_t)blockIdx.x * out_stride;
+    for (int i = threadIdx.x; i < dim; i += 256) o[i] = (T)tanhf(xr[i]);
 }
 
 struct Groups {
@@ -176,16 +203,16 @@ __device__ __forceinline__ float gated(float v, float g, int kind) {
 }
 
 // One wave per (row, NH heads) of up to 64 NE dimensions, everything requested before the first sum.
-template <int NE, int NH>
+template <int NE, int NH, typename T>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float *__restrict__ o, int64_t o_stride, const float *__restrict__ gate, int64_t g_stride,
-                                                             const float *__restrict__ w, int kind, float scale, float *__restrict__ out, int64_t out_stride,
+                                                             const float *__restrict__ w, int kind, float scale, T *__restrict__ out, int64_t out_stride,
                                                              int heads, int dim, float eps) {
     const int lane = threadIdx.x & 63;
     const int h0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * NH;
     if (h0 >= heads) return;
     const int64_t r = blockIdx.x;
     const float *orow = o + r * o_stride, *grow = gate + r * g_stride;
-    float *dst = out + r * out_stride;
+    T *dst = out + r * out_stride;
     float v[NH][NE], g[NH][NE];
 #pragma unroll
     for (int i = 0; i < NH; i++)
@@ -204,14 +231,15 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float *__rest
 #pragma unroll
         for (int e = 0; e < NE; e++) {
             const int d = lane + 64 * e, at = (h0 + i) * dim + d;
-            if (h0 + i < heads && d < dim) dst[at] = scale * gated(v[i][e] * inv * (w ? w[at] : 1.0f), g[i][e], kind);
+            if (h0 + i < heads && d < dim) dst[at] = (T)(scale * gated(v[i][e] * inv * (w ? w[at] : 1.0f), g[i][e], kind));
         }
     }
 }
 
 // heads of any size
+template <typename T>
 __global__ __launch_bounds__(256) void head_norm_gate_long_kernel(const float *__restrict__ o, int64_t o_stride, const float *__restrict__ gate, int64_t g_stride,
-                                                                  const float *__restrict__ w, int kind, float scale, float *__restrict__ out,
+                                                                  const float *__restrict__ w, int kind, float scale, T *__restrict__ out,
                                                                   int64_t out_stride, int heads, int dim, float eps) {
     const int lane = threadIdx.x & 63;
     const int h = blockIdx.y * 4 + (threadIdx.x >> 6);
@@ -219,7 +247,62 @@ __global__ __launch_bounds__(256) void head_norm_gate_long_kernel(const float *_
     const int64_t r = blockIdx.x, hd = (int64_t)h * dim;
     const float *s = o + r * o_stride + hd;
     const float inv = head_inv_rms(s, dim, eps, lane);
-    for (int i = lane; i < dim; i += 64) out[r * out_stride + hd + i] = scale * gated(s[i] * inv * (w ? w[hd + i] : 1.0f), gate[r * g_stride + hd + i], kind);
+    for (int i = lane; i < dim; i += 64) out[r * out_stride + hd + i] = (T)(scale * gated(s[i] * inv * (w ? w[hd + i] : 1.0f), gate[r * g_stride + hd + i], kind));
+}
+
+template <typename T>
+int rms_norm_rows(float *x, int64_t x_stride, const int32_t *index, const float *delta, int64_t delta_stride, const float *weight, T *out, int64_t out_stride,
+                  int64_t rows, int64_t dim, float eps, void *stream) {
+    if (rows < 0 || dim <= 0 || x_stride < dim || out_stride < dim || (delta && delta_stride < dim)) return CQ_ERR_SHAPE;
+    if (rows == 0) return CQ_OK;
+    if (!x || !weight || !out) return CQ_ERR_NULL;
+    if (index && delta) return CQ_ERR_SHAPE;            // selected rows are only read
+    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
+    const bool vec = dim % 4 == 0 && x_stride % 4 == 0 && out_stride % 4 == 0 && (!delta || delta_stride % 4 == 0) && !mix_misaligned(x, 16) &&
+                     !mix_misaligned(delta, 16) && !mix_misaligned(weight, 16) && !mix_misaligned(out, 4 * sizeof(T));
+    auto *const fn = vec ? rms_norm_rows_kernel<true, T> : rms_norm_rows_kernel<false, T>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, x, x_stride, index, delta, delta_stride, weight, out, out_stride, (int)dim, eps);
+    return (int)hipGetLastError();
+}
+
+template <typename T>
+int poly_norm(const float *z, int64_t z_stride, const float *coef, T *out, int64_t out_stride, int64_t rows, int64_t dim, float eps, void *stream) {
+    if (rows < 0 || dim <= 0 || z_stride < dim || out_stride < dim) return CQ_ERR_SHAPE;
+    if (rows == 0) return CQ_OK;
+    if (!z || !coef || !out) return CQ_ERR_NULL;
+    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
+    hipLaunchKernelGGL(poly_norm_kernel<T>, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, z, z_stride, coef, out, out_stride, (int)dim, eps);
+    return (int)hipGetLastError();
+}
+
+template <typename T>
+int tanh_rows(const float *x, int64_t x_stride, T *out, int64_t out_stride, int64_t rows, int64_t dim, void *stream) {
+    if (rows < 0 || dim <= 0 || x_stride < dim || out_stride < dim) return CQ_ERR_SHAPE;
+    if (rows == 0) return CQ_OK;
+    if (!x || !out) return CQ_ERR_NULL;
+    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
+    hipLaunchKernelGGL(tanh_kernel<T>, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, x, x_stride, out, out_stride, (int)dim);
+    return (int)hipGetLastError();
+}
+
+template <typename T>
+int head_norm_gate(const float *o, int64_t o_stride, const float *g, int64_t g_stride, const float *weight, int gate, float scale, T *out, int64_t out_stride,
+                   int64_t rows, int64_t heads, int64_t dim, float eps, void *stream) {
+    if (rows < 0 || heads <= 0 || dim <= 0 || o_stride < heads * dim || g_stride < heads * dim || out_stride < heads * dim) return CQ_ERR_SHAPE;
+    if (gate != CQ_GATE_SILU && gate != CQ_GATE_SIGMOID) return CQ_ERR_DTYPE;
+    if (rows == 0) return CQ_OK;
+    if (!o || !g || !out) return CQ_ERR_NULL;
+    if (heads * dim > (1 << 24) || heads > 4 * 65535 || rows > 0x7fffffffLL) return CQ_ERR_RANGE;
+    hipStream_t s = (hipStream_t)stream;
+#define CQ_HG(K_, NH_)                                                                                                                                 \
+    hipLaunchKernelGGL(K_, dim3((unsigned)rows, (unsigned)((heads + 4 * NH_ - 1) / (4 * NH_))), dim3(256), 0, s, o, o_stride, g, g_stride, weight, gate, scale, out, \
+                       out_stride, (int)heads, (int)dim, eps)
+    if (dim <= 64) CQ_HG((head_norm_gate_kernel<1, 8, T>), 8);
+    else if (dim <= 128) CQ_HG((head_norm_gate_kernel<2, 4, T>), 4);
+    else if (dim <= 256) CQ_HG((head_norm_gate_kernel<4, 2, T>), 2);
+    else CQ_HG(head_norm_gate_long_kernel<T>, 1);
+#undef CQ_HG
+    return (int)hipGetLastError();
 }
 
 }  // namespace
@@ -228,21 +311,12 @@ extern "C" {
 
 int cq_mix_rms_norm_rows(float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *delta_dev, int64_t delta_stride, const float *weight_dev,
                          float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps, void *stream) {
-    if (rows < 0 || dim <= 0 || x_stride < dim || out_stride < dim || (delta_dev && delta_stride < dim)) return CQ_ERR_SHAPE;
-    if (rows == 0) return CQ_OK;
-    if (!x_dev || !weight_dev || !out_dev) return CQ_ERR_NULL;
-    if (index_dev && delta_dev) return CQ_ERR_SHAPE;            // selected rows are only read
-    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
-    const bool vec = dim % 4 == 0 && x_stride % 4 == 0 && out_stride % 4 == 0 && (!delta_dev || delta_stride % 4 == 0) && !mix_misaligned(x_dev, 16) &&
-                     !mix_misaligned(delta_dev, 16) && !mix_misaligned(weight_dev, 16) && !mix_misaligned(out_dev, 16);
-    hipStream_t s = (hipStream_t)stream;
-    if (vec)
-        hipLaunchKernelGGL(rms_norm_rows_kernel<true>, dim3((unsigned)rows), dim3(256), 0, s, x_dev, x_stride, index_dev, delta_dev, delta_stride, weight_dev,
-                           out_dev, out_stride, (int)dim, eps);
-    else
-        hipLaunchKernelGGL(rms_norm_rows_kernel<false>, dim3((unsigned)rows), dim3(256), 0, s, x_dev, x_stride, index_dev, delta_dev, delta_stride, weight_dev,
-                           out_dev, out_stride, (int)dim, eps);
-    return (int)hipGetLastError();
+    return rms_norm_rows(x_dev, x_stride, index_dev, delta_dev, delta_stride, weight_dev, out_dev, out_stride, rows, dim, eps, stream);
+}
+
+int cq_mix_rms_norm_rows_bf16(float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *delta_dev, int64_t delta_stride, const float *weight_dev,
+                              void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps, void *stream) {
+    return rms_norm_rows(x_dev, x_stride, index_dev, delta_dev, delta_stride, weight_dev, (__bf16 *)out_bf16_dev, out_stride, rows, dim, eps, stream);
 }
 
 int cq_mix_layer_norm_rows(const float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *vec_dev, float *out_dev, void *out_bf16_dev,
@@ -258,21 +332,20 @@ int cq_mix_layer_norm_rows(const float *x_dev, int64_t x_stride, const int32_t *
 
 int cq_mix_poly_norm(const float *z_dev, int64_t z_stride, const float *coef_dev, float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps,
                      void *stream) {
-    if (rows < 0 || dim <= 0 || z_stride < dim || out_stride < dim) return CQ_ERR_SHAPE;
-    if (rows == 0) return CQ_OK;
-    if (!z_dev || !coef_dev || !out_dev) return CQ_ERR_NULL;
-    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
-    hipLaunchKernelGGL(poly_norm_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, z_dev, z_stride, coef_dev, out_dev, out_stride, (int)dim, eps);
-    return (int)hipGetLastError();
+    return poly_norm(z_dev, z_stride, coef_dev, out_dev, out_stride, rows, dim, eps, stream);
+}
+
+int cq_mix_poly_norm_bf16(const float *z_dev, int64_t z_stride, const float *coef_dev, void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps,
+                          void *stream) {
+    return poly_norm(z_dev, z_stride, coef_dev, (__bf16 *)out_bf16_dev, out_stride, rows, dim, eps, stream);
 }
 
 int cq_mix_tanh(const float *x_dev, int64_t x_stride, float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, void *stream) {
-    if (rows < 0 || dim <= 0 || x_stride < dim || out_stride < dim) return CQ_ERR_SHAPE;
-    if (rows == 0) return CQ_OK;
-    if (!x_dev || !out_dev) return CQ_ERR_NULL;
-    if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
-    hipLaunchKernelGGL(tanh_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, x_dev, x_stride, out_dev, out_stride, (int)dim);
-    return (int)hipGetLastError();
+    return tanh_rows(x_dev, x_stride, out_dev, out_stride, rows, dim, stream);
+}
+
+int cq_mix_tanh_bf16(const float *x_dev, int64_t x_stride, void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, void *stream) {
+    return tanh_rows(x_dev, x_stride, (__bf16 *)out_bf16_dev, out_stride, rows, dim, stream);
 }
 
 int cq_mix_pack_heads(const float *src_dev, int64_t src_stride, const cq_mix_heads *groups, int n_groups, float eps, const int32_t *pos_dev, int64_t pos,
@@ -305,21 +378,12 @@ int cq_mix_pack_heads(const float *src_dev, int64_t src_stride, const cq_mix_hea
 
 int cq_mix_head_norm_gate(const float *o_dev, int64_t o_stride, const float *g_dev, int64_t g_stride, const float *weight_dev, int gate, float scale,
                           float *out_dev, int64_t out_stride, int64_t rows, int64_t heads, int64_t dim, float eps, void *stream) {
-    if (rows < 0 || heads <= 0 || dim <= 0 || o_stride < heads * dim || g_stride < heads * dim || out_stride < heads * dim) return CQ_ERR_SHAPE;
-    if (gate != CQ_GATE_SILU && gate != CQ_GATE_SIGMOID) return CQ_ERR_DTYPE;
-    if (rows == 0) return CQ_OK;
-    if (!o_dev || !g_dev || !out_dev) return CQ_ERR_NULL;
-    if (heads * dim > (1 << 24) || heads > 4 * 65535 || rows > 0x7fffffffLL) return CQ_ERR_RANGE;
-    hipStream_t s = (hipStream_t)stream;
-#define CQ_HG(K_, NH_)                                                                                                                                 \
-    hipLaunchKernelGGL(K_, dim3((unsigned)rows, (unsigned)((heads + 4 * NH_ - 1) / (4 * NH_))), dim3(256), 0, s, o_dev, o_stride, g_dev, g_stride, weight_dev, gate, \
-                       scale, out_dev, out_stride, (int)heads, (int)dim, eps)
-    if (dim <= 64) CQ_HG((head_norm_gate_kernel<1, 8>), 8);
-    else if (dim <= 128) CQ_HG((head_norm_gate_kernel<2, 4>), 4);
-    else if (dim <= 256) CQ_HG((head_norm_gate_kernel<4, 2>), 2);
-    else CQ_HG(head_norm_gate_long_kernel, 1);
-#undef CQ_HG
-    return (int)hipGetLastError();
+    return head_norm_gate(o_dev, o_stride, g_dev, g_stride, weight_dev, gate, scale, out_dev, out_stride, rows, heads, dim, eps, stream);
+}
+
+int cq_mix_head_norm_gate_bf16(const float *o_dev, int64_t o_stride, const float *g_dev, int64_t g_stride, const float *weight_dev, int gate, float scale,
+                               void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t heads, int64_t dim, float eps, void *stream) {
+    return head_norm_gate(o_dev, o_stride, g_dev, g_stride, weight_dev, gate, scale, (__bf16 *)out_bf16_dev, out_stride, rows, heads, dim, eps, stream);
 }
 
 }  // extern "C"

@@ -151,6 +151,12 @@ class Dense:
                                                           add, int(accumulate), self.n, self.kp, sp))
 
 
+def mix(rt: Runtime, name: str, bf16: bool) -> Callable[..., None]:
+    """A row operation, with results in f32 or in bfloat16 (for a product that would round them)."""
+    name = f"cq_mix_{name}_bf16" if bf16 else f"cq_mix_{name}"
+    return lambda *args: check(name, getattr(rt.L, name)(*args))
+
+
 def dense_product(rt: Runtime, precision: int, sp, workspace=None, workspace_bytes: int = 0, **fields) -> None:
     check("cq_dense_product", rt.L.cq_dense_product(precision, DenseArgs(**fields), workspace, workspace_bytes, sp))
 
@@ -182,9 +188,10 @@ class RmsNorm:
 
     def rows(self, x: int, ldx: int, out: Normed, ldo: int, rows: int, sp, index: Optional[int] = None, delta: Optional[int] = None) -> None:
         """Rows of x (those that `index` names) into out; `delta` [rows, ldx] is added to x first."""
-        if out.f32 is None or (out.typed is not None and out.typed != out.f32):
-            raise ValueError("this norm writes f32 only")
-        check("cq_mix_rms_norm_rows", self.rt.L.cq_mix_rms_norm_rows(x, ldx, index, delta, ldx, self.vec.data_ptr(), out.f32, ldo, rows, self.dim, self.eps, sp))
+        if out.f32 is not None and out.typed is not None and out.typed != out.f32:
+            raise ValueError("this norm writes rows of one type")
+        bf16 = out.f32 is None and self.rt.t_bf16
+        mix(self.rt, "rms_norm_rows", bf16)(x, ldx, index, delta, ldx, self.vec.data_ptr(), out.typed if out.f32 is None else out.f32, ldo, rows, self.dim, self.eps, sp)
 
 
 class LayerNorm:
@@ -269,9 +276,9 @@ class TalkingAttention:
         L = self.rt.L
         need = L.cq_mix_talk_attention_workspace_bytes(rows, self.heads, self.vdim, self.window, self.keep_first, pos)
         ws = self.rt.scratch("attention_splits", need // 4) if need else None
-        check("cq_mix_talk_attention", L.cq_mix_talk_attention(
+        mix(self.rt, "talk_attention", self.rt.t_bf16)(
             q, kv[0].data_ptr(), kv[1].data_ptr(), self.talk.data_ptr(), self.scale, self.window, self.keep_first, out_scale, out, out_stride, pos, rows, self.heads,
-            self.kv_heads, self.dp, self.vdim, self.vp, self.rt.ctx, ws, need, sp))
+            self.kv_heads, self.dp, self.vdim, self.vp, self.rt.ctx, ws, need, sp)
 
     def records(self):
         n = self.rt.L.cq_mix_talk_decode_workspace_bytes(self.heads, self.vdim, self.window, self.keep_first, self.rt.ctx)
@@ -322,8 +329,7 @@ class Retention:
         raw, w = rt.scratch("mixer_raw", rows * self.width_out()), self.width_out()
         check("cq_mix_retention", L.cq_mix_retention(q, k, row + 4 * v_off, row_stride, self.log2_decay.data_ptr(), state.data_ptr(), raw, w, rows, self.heads, self.dim,
                                                      self.dp, self.vdim, ws, need, sp))
-        check("cq_mix_head_norm_gate", L.cq_mix_head_norm_gate(raw, w, row + 4 * g_off, row_stride, None, SILU, out_scale, out, out_stride, rows, self.heads, self.vdim,
-                                                               self.eps, sp))
+        mix(rt, "head_norm_gate", rt.t_bf16)(raw, w, row + 4 * g_off, row_stride, None, SILU, out_scale, out, out_stride, rows, self.heads, self.vdim, self.eps, sp)
 
 
 class Mixer:
@@ -349,6 +355,8 @@ class Parallel(Mixer):
     """Attention and retention side by side on the same input, left_scale * left + right_scale * right.  One product projects for both, one takes
     their outputs, side by side and already scaled, back to the residual stream."""
 
+    INPUT = AS_TYPED
+
     def __init__(self, rt: Runtime, cfg: dict, get: Callable[[str], torch.Tensor], eps: float):
         self.rt, self.eps = rt, eps
         self.left = TalkingAttention(rt, cfg["left"], lambda n: get("left." + n), eps)
@@ -370,17 +378,17 @@ class Parallel(Mixer):
     def prefill(self, h, ldh, x, ldx, kept, pos, rows, sp):
         rt, lt, rg = self.rt, self.left, self.right
         kv, state = kept
-        ldp, ldo = pad_to(self.w_in.n, 4), self.w_out.kp
+        ldp, ldo, bf = pad_to(self.w_in.n, 4), self.w_out.kp, int(rt.t_bf16)
         row = rt.scratch("projection", rows * ldp)
         q = rt.scratch("attention_q", rows * lt.heads * lt.dp)
         rq, rk = rt.scratch("retention_q", rows * rg.heads * rg.dp), rt.scratch("retention_k", rows * rg.heads * rg.dp)
-        out = rt.scratch("mixer_out", rows * ldo)
-        self.w_in.rows(h.f32, ldh, row, ldp, rows, sp)
+        out = rt.typed("mixer_out_typed", rows * ldo)
+        self.w_in.rows(h.typed, ldh, row, ldp, rows, sp, x_bf16=bf)
         groups = _group_array(lt.groups(kv, 0, q) + rg.groups(self.off, rq, rk))
         check("cq_mix_pack_heads", rt.L.cq_mix_pack_heads(row, ldp, groups, len(groups), self.eps, None, pos, rows, sp))
         lt.attend(q, kv, out, ldo, self.left_scale, pos, rows, sp)
-        rg.attend(rq, rk, row, ldp, self.off, state, out + 4 * lt.width_out(), ldo, self.right_scale, rows, sp)
-        self.w_out.rows(out, ldo, x, ldx, rows, sp, accumulate=True)
+        rg.attend(rq, rk, row, ldp, self.off, state, out + (2 if bf else 4) * lt.width_out(), ldo, self.right_scale, rows, sp)
+        self.w_out.rows(out, ldo, x, ldx, rows, sp, accumulate=True, x_bf16=bf)
 
     def step(self, x, norm, kept, pos_dev, pos, add, sp):
         rt, lt, rg = self.rt, self.left, self.right
@@ -399,6 +407,8 @@ class Parallel(Mixer):
 
 class GeneralDelta(Mixer):
     """The generalized delta rule: a decay and a removal rate per head and key channel, the decay through a low-rank projection."""
+
+    INPUT = AS_TYPED
 
     def __init__(self, rt: Runtime, cfg: dict, get: Callable[[str], torch.Tensor], eps: float):
         self.rt, self.eps = rt, eps
@@ -422,20 +432,19 @@ class GeneralDelta(Mixer):
 
     def prefill(self, h, ldh, x, ldx, kept, pos, rows, sp):
         rt, L, w = self.rt, self.rt.L, self.width
-        ldp, ldw, ldo = pad_to(self.w_in.n, 4), pad_to(w, 4), self.w_out.kp
+        ldp, ldw, ldo, bf = pad_to(self.w_in.n, 4), pad_to(w, 4), self.w_out.kp, int(rt.t_bf16)
         row = rt.scratch("projection", rows * ldp)
-        low, wl = rt.scratch("delta_low", rows * self.w2.kp), rt.scratch("delta_decay", rows * ldw)
+        low, wl = rt.typed("delta_low", rows * self.w2.kp), rt.scratch("delta_decay", rows * ldw)
         packed = rt.scratch("delta_packed", rows * self.heads * (4 * L.cq_mix_state_pad(self.dim) + 1))
-        raw, out = rt.scratch("mixer_raw", rows * w), rt.scratch("mixer_out", rows * ldo)
-        self.w_in.rows(h.f32, ldh, row, ldp, rows, sp)
-        check("cq_mix_tanh", L.cq_mix_tanh(row + 4 * self.low_off, ldp, low, self.w2.kp, rows, self.rank, sp))
-        self.w2.rows(low, self.w2.kp, wl, ldw, rows, sp)
+        raw, out = rt.scratch("mixer_raw", rows * w), rt.typed("mixer_out_typed", rows * ldo)
+        self.w_in.rows(h.typed, ldh, row, ldp, rows, sp, x_bf16=bf)
+        mix(rt, "tanh", rt.t_bf16)(row + 4 * self.low_off, ldp, low, self.w2.kp, rows, self.rank, sp)
+        self.w2.rows(low, self.w2.kp, wl, ldw, rows, sp, x_bf16=bf)
         check("cq_mix_delta_prep", L.cq_mix_delta_prep(row, ldp, self.r_off, self.k_off, self.a_off, wl, ldw, self.w0.data_ptr(), self.a_bias.data_ptr(), packed, rows,
                                                        self.heads, self.dim, sp))
         check("cq_mix_delta_scan", L.cq_mix_delta_scan(packed, row + 4 * self.v_off, ldp, kept.data_ptr(), raw, w, rows, self.heads, self.dim, sp))
-        check("cq_mix_head_norm_gate", L.cq_mix_head_norm_gate(raw, w, row + 4 * self.g_off, ldp, self.norm.data_ptr(), SIGMOID, 1.0, out, ldo, rows, self.heads,
-                                                               self.dim, self.eps, sp))
-        self.w_out.rows(out, ldo, x, ldx, rows, sp, accumulate=True)
+        mix(rt, "head_norm_gate", rt.t_bf16)(raw, w, row + 4 * self.g_off, ldp, self.norm.data_ptr(), SIGMOID, 1.0, out, ldo, rows, self.heads, self.dim, self.eps, sp)
+        self.w_out.rows(out, ldo, x, ldx, rows, sp, accumulate=True, x_bf16=bf)
 
     def step(self, x, norm, kept, pos_dev, pos, add, sp):
         rt = self.rt
@@ -465,6 +474,8 @@ class FeedForward:
 class PolyFeedForward(FeedForward):
     """down(PolyNorm(up(norm(x)))): the activation is a polynomial whose powers are each divided by the row's root mean square."""
 
+    INPUT = AS_TYPED
+
     def __init__(self, rt: Runtime, cfg: dict, get: Callable[[str], torch.Tensor], eps: float):
         self.rt, self.eps = rt, eps
         self.up, self.down = Dense(rt, [get("up")]), Dense(rt, [get("down")])
@@ -477,11 +488,11 @@ class PolyFeedForward(FeedForward):
         return [self.up, self.down]
 
     def prefill(self, h, ldh, x, ldx, rows, sp):
-        rt, ld = self.rt, self.down.kp
-        z = rt.scratch("feed_forward", rows * ld)
-        self.up.rows(h.f32, ldh, z, ld, rows, sp)
-        check("cq_mix_poly_norm", rt.L.cq_mix_poly_norm(z, ld, self.coef.data_ptr(), z, ld, rows, self.ff, self.eps, sp))
-        self.down.rows(z, ld, x, ldx, rows, sp, accumulate=True)
+        rt, ld, bf = self.rt, self.down.kp, int(self.rt.t_bf16)
+        z, a = rt.scratch("feed_forward", rows * ld), rt.typed("activation", rows * ld)
+        self.up.rows(h.typed, ldh, z, ld, rows, sp, x_bf16=bf)
+        mix(rt, "poly_norm", rt.t_bf16)(z, ld, self.coef.data_ptr(), a, ld, rows, self.ff, self.eps, sp)
+        self.down.rows(a, ld, x, ldx, rows, sp, accumulate=True, x_bf16=bf)
 
     def step(self, x, norm, add, sp):
         z = self.rt.scratch("feed_forward", self.down.kp)

@@ -75,6 +75,9 @@ int cq_dense_matvec(const void *w_dev, int64_t ldw, const float *x_dev, int prol
  * delta, s also replaces the row of x.  Any dim; strides in floats. */
 int cq_mix_rms_norm_rows(float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *delta_dev, int64_t delta_stride, const float *weight_dev,
                          float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps, void *stream);
+/* The same with results in bfloat16, as the bf16 product that reads them would round them (strides in elements); here and below. */
+int cq_mix_rms_norm_rows_bf16(float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *delta_dev, int64_t delta_stride, const float *weight_dev,
+                              void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps, void *stream);
 /* Layer norm of (selected) rows: out[r] = (s - mean(s)) / sqrt(var(s) + eps) * vec[0..dim) + vec[dim..2 dim), s = x[index ? index[r] : r], as f32,
  * as bfloat16 or both (out_dev, out_bf16_dev: one may be NULL). */
 int cq_mix_layer_norm_rows(const float *x_dev, int64_t x_stride, const int32_t *index_dev, const float *vec_dev, float *out_dev, void *out_bf16_dev,
@@ -82,7 +85,10 @@ int cq_mix_layer_norm_rows(const float *x_dev, int64_t x_stride, const int32_t *
 /* out = coef[0] N(z) + coef[1] N(z^2) + coef[2] N(z^3) + coef[3], N(z) = z / sqrt(mean(z^2) + eps), row by row (out may be z). */
 int cq_mix_poly_norm(const float *z_dev, int64_t z_stride, const float *coef_dev, float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps,
                      void *stream);
+int cq_mix_poly_norm_bf16(const float *z_dev, int64_t z_stride, const float *coef_dev, void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, float eps,
+                          void *stream);
 int cq_mix_tanh(const float *x_dev, int64_t x_stride, float *out_dev, int64_t out_stride, int64_t rows, int64_t dim, void *stream);
+int cq_mix_tanh_bf16(const float *x_dev, int64_t x_stride, void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t dim, void *stream);
 
 /* A group of heads inside a projection row, for the calls below.  Element d of head h of row r is read at
  * src[r * src_stride + src_off + h * dim + d]; an optional RMS norm per head (norm_dev [dim], eps of the call), an optional
@@ -107,6 +113,8 @@ int cq_mix_pack_heads(const float *src_dev, int64_t src_stride, const cq_mix_hea
 enum cq_gate { CQ_GATE_SILU = 0, CQ_GATE_SIGMOID = 1 };
 int cq_mix_head_norm_gate(const float *o_dev, int64_t o_stride, const float *g_dev, int64_t g_stride, const float *weight_dev, int gate, float scale,
                           float *out_dev, int64_t out_stride, int64_t rows, int64_t heads, int64_t dim, float eps, void *stream);
+int cq_mix_head_norm_gate_bf16(const float *o_dev, int64_t o_stride, const float *g_dev, int64_t g_stride, const float *weight_dev, int gate, float scale,
+                               void *out_bf16_dev, int64_t out_stride, int64_t rows, int64_t heads, int64_t dim, float eps, void *stream);
 
 /* ---- attention with scores mixed across heads, a sliding window and kept first tokens --------------------------------
  * score_h = sum_g talk[h, g] * scale * (q_g . k_g), key j visible to position i when j <= i and (i - j < window or j < keep_first), softmax
@@ -120,6 +128,10 @@ int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const fl
                           int64_t keep_first, float out_scale, float *out_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
                           int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes,
                           void *stream);
+int cq_mix_talk_attention_bf16(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,
+                               int64_t keep_first, float out_scale, void *out_bf16_dev, int64_t out_stride, int64_t pos, int64_t rows, int64_t n_head,
+                               int64_t n_kv_head, int64_t dim_pad, int64_t vdim, int64_t vdim_pad, int64_t ctx, void *workspace_dev, int64_t workspace_bytes,
+                               void *stream);
 
 /* The same for one new token straight from its projection row: the three groups (q; k and v with their caches as dst, by_position
  * set) are normalized, rotated and appended as cq_mix_pack_heads would, then attended, in one launch that leaves a record per split of

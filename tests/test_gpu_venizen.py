@@ -128,6 +128,34 @@ def test_head_norm_gate(heads, dim, kind, weight):
     assert rel(out, want) < 3e-6
 
 
+@pytest.mark.parametrize("dim", [4, 7, 66, 1024, 5000, 9001])
+def test_rows_in_bfloat16(dim):
+    """The calls that leave bfloat16 rows give the f32 results, rounded: with 8-byte stores and one by one, heads of every size, keys split or not."""
+    L, ld, heads = _lib.mixer_lib(), mixers.pad_to(dim, 4) + 4, 3
+    x, w, z = up(rnd(1, 9, ld)), rnd(2, dim), rnd(3, 9, heads * dim)
+    coef = ptr(np.array([0.5, -0.7, 0.9, -0.2], dtype=np.float32))
+    calls = [("rms_norm_rows", ld, lambda out, n: (x.data_ptr(), ld, None, None, 0, ptr(w), out, n, 9, dim, EPS, sp())),
+             ("poly_norm", ld, lambda out, n: (x.data_ptr(), ld, coef, out, n, 9, dim, EPS, sp())),
+             ("tanh", ld, lambda out, n: (x.data_ptr(), ld, out, n, 9, dim, sp())),
+             ("head_norm_gate", heads * dim, lambda out, n: (ptr(z), heads * dim, ptr(z), heads * dim, None, mixers.SILU, 0.7, out, n, 9, heads, dim, EPS, sp()))]
+    for rows, pos in ((40, 0), (6, 300)):
+        T, d = rows + pos, 32
+        q, kc, vc_ = up(rnd(4, rows, 2, d)), up(rnd(5, 1, T, d)), up(rnd(6, 1, T, d))
+        need = L.cq_mix_talk_attention_workspace_bytes(rows, 2, d, T, 0, pos)
+        assert (need > 0) == (pos > 0)
+        ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=DEV)
+        _alive.extend((q, kc, vc_, ws))
+        a = (q.data_ptr(), kc.data_ptr(), vc_.data_ptr(), ptr(np.eye(2, dtype=np.float32)), 0.2, T, 0, 0.6)
+        b = (pos, rows, 2, 1, d, d, d, T, ws.data_ptr(), need, sp())
+        calls.append(("talk_attention", 64, lambda out, n, a=a, b=b: (*a, out, n, *b)))
+    for name, width, args in calls:
+        for n in (mixers.pad_to(width, 4), width + 5):
+            want, got = torch.zeros((48, n), device=DEV), torch.zeros((48, n), dtype=torch.bfloat16, device=DEV)
+            mixers.check(name, getattr(L, "cq_mix_" + name)(*args(want.data_ptr(), n)))
+            mixers.check(name, getattr(L, f"cq_mix_{name}_bf16")(*args(got.data_ptr(), n)))
+            assert bool(want.any()) and torch.equal(got, want.to(torch.bfloat16)), (name, n)
+
+
 @pytest.mark.parametrize("dim,rot", [(6, 2), (40, 40), (64, 20), (200, 128), (256, 0)])
 def test_pack_heads(dim, rot):
     """Norm, rotation and factor of two groups in one launch, one of them into a cache by position."""
