@@ -180,10 +180,19 @@ def _load(path: str, signatures: dict) -> ctypes.CDLL:
     return L
 
 
+qmatmul = None                 # QTensor.fwd of an ordinary call (csrc/cq_host.cpp), once the library is loaded
+
+
 def lib() -> ctypes.CDLL:
-    global _lib
+    global _lib, qmatmul
     if _lib is None:
-        _lib = _load(LIB_PATH, SIGNATURES)
+        L = _load(LIB_PATH, SIGNATURES)
+        try:
+            from . import _host
+        except ImportError as e:
+            raise ImportError("candle_amd/_host.so is missing or does not fit this PyTorch: build it first (python -m candle_amd.build)") from e
+        _host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (L.cq_qmatmul_workspace_bytes, L.cq_qmatmul_forward)))
+        _lib, qmatmul = L, _host.qmatmul
     return _lib
 
 

@@ -1,4 +1,4 @@
-"""Builds libcandle_hip_quant.so (gfx950) in-tree with hipcc.
+"""Builds libcandle_hip_quant.so (gfx950) in-tree with hipcc, and the native host path (_host.so) with the host compiler.
 
     python -m candle_amd.build            # compile what changed, link
     python -m candle_amd.build --force    # recompile everything
@@ -33,6 +33,9 @@ MIXER_SOURCES = ["cq_nn.hip", "cq_status.hip", "cq_dense.hip", "cq_mix_glue.hip"
 MIXER_HEADERS = ("candle_hip_mixer.h", "cq_mix.h", "cq_dense.h")
 # the benchmark's plain-read yardstick kernel: a library of its own, not part of the C ABI
 BENCH_SOURCES = ["cq_bench.hip"]
+# the native host path of plain calls: a Python module over PyTorch's C++ interface, without device code
+HOST = os.path.join(HERE, "_host.so")
+HOST_SOURCE = "cq_host.cpp"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -90,7 +93,29 @@ def _build(groups, force: bool) -> None:
             os.replace(tmp, lib)
 
 
+def build_host(force: bool = False) -> str:
+    src = os.path.join(CSRC, HOST_SOURCE)
+    if not force and os.path.exists(HOST) and os.path.getmtime(HOST) > os.path.getmtime(src):
+        return HOST
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    libs = cpp_extension.library_paths()
+    inc = [*cpp_extension.include_paths(), os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    tmp = f"{HOST}.{os.getpid()}"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(f"-isystem{i}" for i in inc), "-Wall", src,
+           "-o", tmp, *(f"-L{p}" for p in libs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {HOST_SOURCE}:\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+    os.replace(tmp, HOST)
+    return HOST
+
+
 def build(force: bool = False) -> str:
+    build_host(force)
     _build(((LIB, SOURCES), (LIB_MIXER, MIXER_SOURCES), (LIB_BENCH, BENCH_SOURCES)), force)
     return LIB
 

