@@ -134,6 +134,8 @@ MIXER_SIGNATURES = {
                                                 _vp, _vp, _i64, _vp]),
     "cq_mix_delta_prep": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "cq_mix_delta_scan": (_int, [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
+    "cq_mix_delta_rows_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "cq_mix_delta_rows": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),
     "cq_mix_delta_step": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp]),
 }
 MIXER_SIGNATURES.update({

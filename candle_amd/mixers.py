@@ -435,14 +435,14 @@ class GeneralDelta(Mixer):
         ldp, ldw, ldo, bf = pad_to(self.w_in.n, 4), pad_to(w, 4), self.w_out.kp, int(rt.t_bf16)
         row = rt.scratch("projection", rows * ldp)
         low, wl = rt.typed("delta_low", rows * self.w2.kp), rt.scratch("delta_decay", rows * ldw)
-        packed = rt.scratch("delta_packed", rows * self.heads * (4 * L.cq_mix_state_pad(self.dim) + 1))
+        need = L.cq_mix_delta_rows_workspace_bytes(rows, self.heads, self.dim)
+        work = rt.scratch("delta_work", need // 4)
         raw, out = rt.scratch("mixer_raw", rows * w), rt.typed("mixer_out_typed", rows * ldo)
         self.w_in.rows(h.typed, ldh, row, ldp, rows, sp, x_bf16=bf)
         mix(rt, "tanh", rt.t_bf16)(row + 4 * self.low_off, ldp, low, self.w2.kp, rows, self.rank, sp)
         self.w2.rows(low, self.w2.kp, wl, ldw, rows, sp, x_bf16=bf)
-        check("cq_mix_delta_prep", L.cq_mix_delta_prep(row, ldp, self.r_off, self.k_off, self.a_off, wl, ldw, self.w0.data_ptr(), self.a_bias.data_ptr(), packed, rows,
-                                                       self.heads, self.dim, sp))
-        check("cq_mix_delta_scan", L.cq_mix_delta_scan(packed, row + 4 * self.v_off, ldp, kept.data_ptr(), raw, w, rows, self.heads, self.dim, sp))
+        check("cq_mix_delta_rows", L.cq_mix_delta_rows(row, ldp, self.r_off, self.k_off, self.v_off, self.a_off, wl, ldw, self.w0.data_ptr(), self.a_bias.data_ptr(),
+                                                       kept.data_ptr(), raw, w, rows, self.heads, self.dim, work, need, sp))
         mix(rt, "head_norm_gate", rt.t_bf16)(raw, w, row + 4 * self.g_off, ldp, self.norm.data_ptr(), SIGMOID, 1.0, out, ldo, rows, self.heads, self.dim, self.eps, sp)
         self.w_out.rows(out, ldo, x, ldx, rows, sp, accumulate=True, x_bf16=bf)
 

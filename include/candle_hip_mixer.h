@@ -169,6 +169,12 @@ int cq_mix_delta_prep(const float *row_dev, int64_t row_stride, int64_t r_off, i
                       const float *w0_dev, const float *a_bias_dev, float *packed_dev, int64_t rows, int64_t heads, int64_t dim, void *stream);
 int cq_mix_delta_scan(const float *packed_dev, const float *v_dev, int64_t v_stride, float *state_dev, float *out_dev, int64_t out_stride, int64_t rows,
                       int64_t heads, int64_t dim, void *stream);
+/* Both in one call (what a prompt takes): heads of up to 64 dimensions in chunks of 16 tokens on the matrix cores, in f32 like the scan; other heads and short
+ * calls by prep and scan.  v lies at v_off of the projection rows; workspace 16-byte aligned. */
+int64_t cq_mix_delta_rows_workspace_bytes(int64_t rows, int64_t heads, int64_t dim);
+int cq_mix_delta_rows(const float *row_dev, int64_t row_stride, int64_t r_off, int64_t k_off, int64_t v_off, int64_t a_off, const float *wl_dev, int64_t wl_stride,
+                      const float *w0_dev, const float *a_bias_dev, float *state_dev, float *out_dev, int64_t out_stride, int64_t rows, int64_t heads, int64_t dim,
+                      void *workspace_dev, int64_t workspace_bytes, void *stream);
 /* One token, one launch: the low-rank projection of the decay (w2 [heads * dim, rank] bfloat16 with row stride ldw2, applied to tanh of the
  * rank values at low_off), the recurrence, and out = weight * sigmoid(g) * o / rms(o). */
 int cq_mix_delta_step(const float *row_dev, int64_t r_off, int64_t k_off, int64_t v_off, int64_t g_off, int64_t a_off, int64_t low_off, const void *w2_dev,

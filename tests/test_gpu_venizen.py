@@ -393,6 +393,39 @@ def test_general_delta_portions(H, d, cuts):
     assert rel(out, o) < 2e-5 and not state[:, :, d:].any()
 
 
+@pytest.mark.parametrize("H,d", [(1, 8), (3, 20), (9, 48), (2, 64), (2, 100)])
+@pytest.mark.parametrize("kind", ["normal", "one key", "fast decay", "slow decay"])
+def test_general_delta_rows(H, d, kind):
+    """A prompt's call over portions at the edges of the chunks of 16 and on either side of the two ways: outputs and the state left against 64 bits.  The bound is
+    that of the packed scan above; a state that hardly decays adds up the roundings of all tokens."""
+    L, W, spd, cuts = _lib.mixer_lib(), H * d, _lib.mixer_lib().cq_mix_state_pad(d), (32, 31, 33, 1, 48, 63, 40)
+    T = sum(cuts)
+    rows, wl, w0, ab = rnd(11, T, 5 * W + 12), rnd(12, T, W), rnd(13, W, scale=1.5), rnd(14, W)
+    if kind == "one key":
+        rows[:, W:2 * W] = rows[:1, W:2 * W] + 0.01 * rows[:, W:2 * W]
+        ab += 4
+    w0 += {"fast decay": 8, "slow decay": -9}.get(kind, 0)
+    r64 = rows.astype(np.float64)
+    part = lambda i: r64[:, i * W:(i + 1) * W].reshape(T, H, d)
+    w = np.exp(-np.exp(-0.5) * vo.sigmoid(wl.astype(np.float64) + w0)).reshape(T, H, d)
+    a = vo.sigmoid(part(4) + ab.astype(np.float64).reshape(H, d))
+    want = vo.general_delta(part(0), part(1), part(2), w, a)
+    state, rd, wld, w0d, abd, ld, at = torch.zeros((H, d, spd), device=DEV), up(rows), up(wl), up(w0), up(ab), rows.shape[1], 0
+    for n in cuts:
+        need = L.cq_mix_delta_rows_workspace_bytes(n, H, d)
+        work, out = torch.full((need // 4,), float("nan"), device=DEV), torch.full((n, W + 1), 7.0, device=DEV)
+        _lib.check("r", L.cq_mix_delta_rows(rd.data_ptr() + 4 * at * ld, ld, 0, W, 2 * W, 4 * W, wld.data_ptr() + 4 * at * W, W, w0d.data_ptr(), abd.data_ptr(),
+                                            state.data_ptr(), out.data_ptr(), W + 1, n, H, d, work.data_ptr(), need, sp()))
+        assert rel(out[:, :W].reshape(n, H, d), want[at:at + n]) < 1e-5, at
+        assert (out[:, W] == 7.0).all()
+        at += n
+    S = np.zeros((H, d, d))
+    u = part(1) / np.sqrt(np.sum(part(1) ** 2, -1, keepdims=True) + 1e-6)
+    for t in range(T):
+        S = w[t][:, :, None] * S - (a[t] * u[t])[:, :, None] * np.einsum("hi,hij->hj", u[t], S)[:, None] + part(1)[t][:, :, None] * part(2)[t][:, None]
+    assert rel(state[:, :, :d].transpose(1, 2), S) < 1e-5 and not state[:, :, d:].any()
+
+
 # ---------------------------------------------------------------------------------------------- the decoder
 LIMIT = {"float32": 2e-5, "bfloat16": 2e-2}
 _built = {}

@@ -205,6 +205,10 @@ def test_mixer_argument_validation_codes_without_gpu():
     assert att(128, 2, 16, 16, 16, 4, 0, 0, 1, 8) == RANGE
     assert L.cq_mix_delta_scan(16, 16, 64, 16, 16, 64, 1, 2, 300, None) == SHAPE
     assert L.cq_mix_delta_scan(16, 16, 600, 16, 16, 600, 1, 2, 300, None) == RANGE
+    rows = lambda row=16, stride=640, state=16, n=40, dim=64, need=1 << 30: L.cq_mix_delta_rows(row, stride, 0, 128, 256, 512, 16, 128, 16, 16, state, 16, 128, n, 2, dim, 16, need, None)
+    assert rows(stride=639) == SHAPE and rows(n=-1) == SHAPE and rows(dim=65) == SHAPE
+    assert rows(row=None) == NULL and rows(state=8) == ALIGN and rows(n=0) == 0
+    assert rows(need=L.cq_mix_delta_rows_workspace_bytes(40, 2, 64) - 1) == WS
     g = _lib.MixHeads(heads=2, dim=8, dim_pad=4, dst_dev=16)
     assert L.cq_mix_pack_heads(16, 64, g, 1, 1e-5, None, 0, 1, None) == SHAPE
     g = _lib.MixHeads(heads=2, dim=8, dim_pad=8, dst_dev=16, rot_dims=6)
