@@ -571,6 +571,229 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(const float *__restrict_
     }
 }
 
+// The prompt's attention from 256 keys on (attn_by_planes): the two products on the bf16 matrix cores, from operands split into three bf16 parts that add up to the
+// f32 value (8 + 8 + 8 bits; of an infinity, NaN).  Of the nine products of parts the six above 2^-24 of the whole are formed, the scores' small ones apart from the
+// large one; sums are f32.  Six times 16 cycles for 16 x 16 x 32 stand against 8 x 32 of the f32 instruction, which bounds the kernel above; the error against 64 bits
+// is half of that kernel's, which rounds four keys or dimensions at a time (2-norm, 1000 rows: 1.64e-7 against 3.35e-7; scores four times as large 4.3e-7, 1.03e-6).
+// attn_planes_kernel splits the keys and values that are visible, once for all workgroups, into tiles of 32 keys laid out as the operands are read: keys
+// [part][32 dims c][16 keys y][lane], values [part][16 dims d][lane], 16 bytes a lane.  attn_planes_run_kernel: a workgroup has 64 (row, head) pairs, 16 a wave; of its
+// eight waves four take the even tiles of keys and four the odd ones (the last rows of a prompt see all keys, and are the longest chain of the launch).  Scores are formed
+// as k q^T: a lane then holds keys 16 y + 4 lk + e of its pair lr, which is an operand of the second product as it lies (the values' tiles have their keys in that
+// order); a maximum is taken across lanes only where a score exceeds the running one.  Values are summed four tiles at a time and the sums then added, as above.
+// Keys arrive an iteration ahead, values under the first product.  Bound by LDS: four waves read 48 KB a tile each, 1920 cycles with the copies, beside 1536 of products.
+// 32 heads, 8 kv heads, us (f32 kernel above -> this, splitting 5 - 20 of it): 300 rows 31 -> 25, 500: 48 -> 35, 1000: 145 -> 73, 2048: 450 -> 216, 300 behind 4000 keys:
+// 406 -> 191.
+constexpr int AT_K = 32, AT_PART = 8192, AT_TILE = 3 * AT_PART;      // keys of a tile; bytes of a part of its keys (or values), of all three
+typedef __bf16 at_bf8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void at_lds;
+
+__device__ __forceinline__ void at_split(const float (&x)[8], at_bf8 (&p)[3]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        p[0][i] = (__bf16)x[i];
+        const float r = x[i] - (float)p[0][i];
+        p[1][i] = (__bf16)r;
+        p[2][i] = (__bf16)(r - (float)p[1][i]);
+    }
+}
+
+__global__ __launch_bounds__(256) void attn_planes_kernel(const float *__restrict__ k_cache, const float *__restrict__ v_cache, uint8_t *__restrict__ planes,
+                                                          const int32_t *__restrict__ pos_dev, int pos0, int rows, int ctx, int tiles) {
+    const int i = blockIdx.x, kvh = blockIdx.y, n = min(pos0 + (pos_dev ? pos_dev[0] : 0) + rows, ctx);
+    if (i * AT_K >= n) return;
+    uint8_t *const to = planes + (((int64_t)kvh * tiles + i) * 2 + blockIdx.z) * AT_TILE;
+    const float *const from = (blockIdx.z ? v_cache : k_cache) + ((int64_t)kvh * ctx + i * AT_K) * 128;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int at = threadIdx.x + 256 * h, lr = at & 15, lk = at >> 4 & 3, y = at >> 6 & 1, c = at >> 7, d = at >> 6;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int key = blockIdx.z ? 16 * (j >> 2) + 4 * lk + (j & 3) : 16 * y + lr, dim = blockIdx.z ? 16 * d + lr : 32 * c + 8 * lk + j;
+            x[j] = i * AT_K + key < n ? from[key * 128 + dim] : 0.0f;
+        }
+        at_bf8 p[3];
+        at_split(x, p);
+#pragma unroll
+        for (int j = 0; j < 3; j++) *reinterpret_cast<at_bf8 *>(to + j * AT_PART + 16 * at) = p[j];
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(512, 2) void attn_planes_run_kernel(const float *__restrict__ q, int64_t q_stride, const uint8_t *__restrict__ planes, float *__restrict__ out,
+                                                                 const int32_t *__restrict__ pos_dev, int pos0, int rows, int n_head, int ctx, float scale, int tiles,
+                                                                 int groups) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
+    constexpr int HD = 128, R = 64 / G;              // pair 16 wv + lr = R * head of the group + row
+    __shared__ __attribute__((aligned(16))) uint8_t smem[6 * AT_TILE];     // of either set of waves: keys of two tiles, values of one
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), set = wave >> 2, wv = wave & 3, lr = lane & 15, lk = lane >> 4;
+    uint8_t *const lds = smem + 3 * AT_TILE * set;
+    const int n_kv = n_head / G, kvh = blockIdx.x % n_kv, t = blockIdx.x / n_kv;
+    const int group = groups - 1 - t;                // later rows see more keys: the long ones first
+    const int r0 = group * R, nr = min(R, rows - r0);     // valid rows of this workgroup (>= 1)
+    const int base_len = pos0 + (pos_dev ? pos_dev[0] : 0) + r0 + 1;
+    const int len_first = min(base_len, ctx), n_t = min((min(base_len + nr - 1, ctx) + AT_K - 1) / AT_K, tiles);
+    const int pair = 16 * wv + lr, row = min(pair % R, nr - 1), head = kvh * G + pair / R;
+    const int len = min(base_len + row, ctx);              // keys of this lane's row
+
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)(planes + (int64_t)kvh * tiles * 2 * AT_TILE), 0, -1, 0x00020000);
+    auto copy = [&](int it, int v) {                       // the keys (0) or values (1) of tile 2 it + set (past the last one: that one again)
+        uint8_t *const to = lds + (v ? 2 : it & 1) * AT_TILE + 1024 * wv;
+        const int i = min(2 * it + set, n_t - 1);
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (at_lds *)(to + 4096 * j), 16, 1024 * wv + 4096 * j + 16 * lane, (2 * i + v) * AT_TILE, 0, 0);
+        asm volatile("" ::: "memory");
+    };
+    copy(0, 0);
+    at_bf8 qp[4][3];                                       // dims 32 c + 8 lk .. of pair lr
+    {
+        const float *qr = q + (int64_t)(r0 + row) * q_stride + (int64_t)head * HD + 8 * lk;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[j] = qr[32 * c + j];
+            at_split(x, qp[c]);
+        }
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 o[8], os[8];                                     // dims 16 d + 4 lk + e of pair lr: all keys up to the last 128, and those since
+#pragma unroll
+    for (int d = 0; d < 8; d++) o[d] = os[d] = zero;
+    float m = -INFINITY, l = 0.0f, ls = 0.0f;              // l: this lane's keys only
+    copy(0, 1);
+    copy(1, 0);
+    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");
+    const int n_it = (n_t + 1) >> 1;
+    for (int it = 0; it < n_it; it++) {
+        const int key0 = (2 * it + set) * AT_K;            // (past the last tile none of them is visible)
+        const uint8_t *const kt = lds + (it & 1) * AT_TILE, *const vt = lds + 2 * AT_TILE;
+        f32x4 s[2] = {zero, zero}, sa[2] = {zero, zero}, sb[2] = {zero, zero};      // large products; two sums of small ones
+        at_bf8 kp[2][2][3];                                // a step's operands, one step ahead
+        auto keys = [&](int c) {
+#pragma unroll
+            for (int y = 0; y < 2; y++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) kp[c & 1][y][j] = *reinterpret_cast<const at_bf8 *>(kt + j * AT_PART + (2 * c + y) * 1024 + 16 * lane);
+        };
+        keys(0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (c < 3) keys(c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const auto &k = kp[c & 1];
+#define CQ_ATS(acc, a_, b_) _Pragma("unroll") for (int y = 0; y < 2; y++) acc[y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[y][a_], qp[c][b_], acc[y], 0, 0, 0)
+            CQ_ATS(sa, 2, 0);
+            CQ_ATS(sb, 1, 0);
+            CQ_ATS(s, 0, 0);
+            CQ_ATS(sa, 0, 2);
+            CQ_ATS(sb, 0, 1);
+            CQ_ATS(sa, 1, 1);
+#undef CQ_ATS
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float top = -INFINITY, p[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) p[j] = (s[j >> 2][j & 3] + (sa[j >> 2][j & 3] + sb[j >> 2][j & 3])) * scale;
+        if (key0 + AT_K > len_first) {                 // (some row of the workgroup does not see all keys)
+#pragma unroll
+            for (int j = 0; j < 8; j++) p[j] = key0 + 16 * (j >> 2) + 4 * lk + (j & 3) < len ? p[j] : -INFINITY;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) top = fmaxf(top, p[j]);
+        if (__any(top > m)) {
+            top = fmaxf(top, __shfl_xor(top, 16, 64));
+            top = fmaxf(top, __shfl_xor(top, 32, 64));
+            const float mn = fmaxf(m, top), f = m > -INFINITY ? __expf(m - mn) : 0.0f;
+            m = mn;
+            l *= f;
+            ls *= f;
+#pragma unroll
+            for (int d = 0; d < 8; d++) {
+                o[d] *= f;
+                os[d] *= f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            p[j] = p[j] == -INFINITY ? 0.0f : __expf(p[j] - m);
+            ls += p[j];
+        }
+        at_bf8 pp[3];
+        at_split(p, pp);
+        asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the values are there for everybody, the next keys need not be
+        at_bf8 vp[2][2][3];
+        auto values = [&](int d) {                         // of dims 16 d .. and 16 (d + 1) ..
+#pragma unroll
+            for (int y = 0; y < 2; y++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) vp[d >> 1 & 1][y][j] = *reinterpret_cast<const at_bf8 *>(vt + j * AT_PART + (d + y) * 1024 + 16 * lane);
+        };
+        values(0);
+#pragma unroll
+        for (int d = 0; d < 8; d += 2) {
+            if (d < 6) values(d + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            const auto &v = vp[d >> 1 & 1];
+#define CQ_ATV(a_, b_) _Pragma("unroll") for (int y = 0; y < 2; y++) os[d + y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[y][a_], pp[b_], os[d + y], 0, 0, 0)
+            CQ_ATV(2, 0);
+            CQ_ATV(0, 2);
+            CQ_ATV(1, 1);
+            CQ_ATV(1, 0);
+            CQ_ATV(0, 1);
+            CQ_ATV(0, 0);
+#undef CQ_ATV
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if ((it & 3) == 3 || it + 1 == n_it) {
+            l += ls;
+            ls = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 8; d++) {
+                o[d] += os[d];
+                os[d] = zero;
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the next keys are, and nobody reads this tile any more
+        copy(it + 1, 1);
+        copy(it + 2, 0);
+    }
+    // the second set's part of a pair joins the first one's (copies have all arrived first: they may not outlive the workgroup)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    f32x4 *const far = reinterpret_cast<f32x4 *>(smem) + 10 * 64 * wv + lane;      // eight of o, then m and l
+    if (set) {
+#pragma unroll
+        for (int d = 0; d < 8; d++) far[64 * d] = o[d];
+        far[512] = f32x4{m, l, 0.0f, 0.0f};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (set) return;
+    {
+        const f32x4 ml = far[512];
+        const float top = fmaxf(m, ml.x), f = m > -INFINITY ? __expf(m - top) : 0.0f, g = ml.x > -INFINITY ? __expf(ml.x - top) : 0.0f;
+        l = l * f + ml.y * g;
+#pragma unroll
+        for (int d = 0; d < 8; d++) {
+            const f32x4 x = far[64 * d];
+            o[d] = o[d] * f + x * g;
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (pair % R >= nr) return;
+    struct __attribute__((packed, aligned(4))) Out4 { f32x4 v; };      // (out has the alignment of a float)
+    float *const dst = out + ((int64_t)(r0 + row) * n_head + head) * HD + 4 * lk;
+#pragma unroll
+    for (int d = 0; d < 8; d++) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = o[d][e] / l;
+        reinterpret_cast<Out4 *>(dst + 16 * d)->v = x;
+    }
+#endif
+}
+
 // merge the splits of one (row, head): out = sum_s e^{m_s - M} acc_s / sum_s e^{m_s - M} l_s
 template <int HD>
 __global__ __launch_bounds__(HD) void attn_combine_kernel(const float *__restrict__ part, float *__restrict__ out, int splits) {
@@ -1328,6 +1551,29 @@ int launch_attn_mfma(int G, dim3 grid, hipStream_t s, const float *q, int64_t q_
     return (int)hipGetLastError();
 }
 
+// From 256 keys on the split operands win back what splitting them costs (300 rows: 25 us against 31, 64 rows behind 1000 keys: 59 against 69; 200 rows: 21.1 against
+// 19.1); they lie in the workspace that partial results would take, which holds them from 95 rows of four heads per kv head on.  (2^20 keys: offsets of 32 bits.)
+bool attn_by_planes(int64_t n_kv, int64_t max_kv_len, const void *workspace, int64_t workspace_bytes) {
+    return max_kv_len >= 256 && max_kv_len <= (1 << 20) && !misaligned(workspace, 16) && workspace_bytes >= n_kv * ((max_kv_len + AT_K - 1) / AT_K) * 2 * AT_TILE;
+}
+
+int launch_attn_planes(int G, hipStream_t s, const float *q, int64_t q_stride, const float *kc, const float *vc, float *out, const int32_t *pos_dev, int pos0, int rows,
+                       int n_head, int ctx, int max_kv_len, float scale, void *planes) {
+    const int tiles = (max_kv_len + AT_K - 1) / AT_K, groups = (rows + 64 / G - 1) / (64 / G), n_kv = n_head / G, wgs = groups * n_kv;
+    hipLaunchKernelGGL(attn_planes_kernel, dim3((unsigned)tiles, (unsigned)n_kv, 2), dim3(256), 0, s, kc, vc, (uint8_t *)planes, pos_dev, pos0, rows, ctx, tiles);
+#define CQ_ATT(GG)                                                                                                                                     \
+    case GG:                                                                                                                                           \
+        hipLaunchKernelGGL((attn_planes_run_kernel<GG>), dim3((unsigned)wgs), dim3(512), 0, s, q, q_stride, (const uint8_t *)planes, out, pos_dev, pos0, rows, \
+                           n_head, ctx, scale, tiles, groups);                                                                      \
+        break;
+    switch (G) {
+        CQ_ATT(1) CQ_ATT(2) CQ_ATT(4) CQ_ATT(8)
+        default: return CQ_ERR_RANGE;
+    }
+#undef CQ_ATT
+    return (int)hipGetLastError();
+}
+
 // rows per workgroup of attn_rows_kernel for a grouping of G query heads per kv head (G * R <= 16 pairs)
 inline int attn_rows_per_group(int G) { return G == 8 ? 2 : 4; }
 
@@ -1423,6 +1669,9 @@ int cq_nn_attention(const float *q_dev, int64_t q_stride, const float *k_cache_d
     int rc;
     if (rows >= CQ_ATTN_MFMA_MIN && head_dim == 128 && (G == 1 || G == 2 || G == 4 || G == 8)) {
         // prompts: 32 (row, head) pairs per workgroup on the f32 matrix cores, all splits in one pass (nothing to combine)
+        if (attn_by_planes(n_kv_head, max_kv_len, workspace_dev, workspace_bytes))
+            return launch_attn_planes(G, s, q_dev, q_stride, k_cache_dev, v_cache_dev, out_dev, pos_dev, (int)pos, (int)rows, (int)n_head, (int)ctx, (int)max_kv_len, scale,
+                                      workspace_dev);
         const int R = 32 / G;
         return launch_attn_mfma(G, dim3((unsigned)n_kv_head, (unsigned)((rows + R - 1) / R)), s, q_dev, q_stride, k_cache_dev, v_cache_dev,
                                 out_dev, pos_dev, (int)pos, (int)rows, (int)n_head, (int)ctx, scale);

@@ -132,6 +132,45 @@ def test_attention(H, KV, D, rows, pos, ctx):
         assert rel_l2(out.cpu().numpy(), attention_oracle(q, kc, vc, pos, H, KV, D)) <= TOL
 
 
+@pytest.mark.parametrize("H,KV", [(8, 1), (8, 2), (4, 2), (2, 2)])
+@pytest.mark.parametrize("rows,pos,max_kv", [(64, 192, 256), (64, 191, 255), (65, 192, 257), (97, 200, 320), (256, 0, 256), (64, 700, 1000), (300, 5, 305)])
+def test_attention_prompt_split_operands(H, KV, rows, pos, max_kv):
+    """Prompts on either side of 256 keys and at the edges of tiles (32 keys, 64 pairs), with a workspace for the split operands and without: outputs within the f32
+    bound, from a position on the device, to a row that is aligned like a float only; what lies behind the visible keys is not read into them."""
+    D, ctx = 128, max_kv + 3
+    q, kc, vc = normal(60, (rows, H * D), 1.0), normal(61, (KV, ctx, D), 1.0), normal(62, (KV, ctx, D), 1.0)
+    want = attention_oracle(q, kc, vc, pos, H, KV, D)
+    kc[:, pos + rows:], vc[:, pos + rows:] = np.nan, np.nan
+    lib, qd, kd, vd, pos_dev = L(), dev(q), dev(kc), dev(vc), torch.tensor([pos - 1], dtype=torch.int32, device="cuda")
+    need, fits = lib.cq_nn_attention_workspace_bytes(rows, H, D, max_kv), (max_kv + 31) // 32 * KV * 49152
+    scale, got = float(np.float32(1.0 / math.sqrt(D))), []
+    for nbytes in (max(need, fits), need):
+        ws, out = torch.full((max(nbytes, 16),), 255, dtype=torch.uint8, device="cuda"), torch.full((rows * H * D + 2,), 7.0, device="cuda")
+        ok(lib.cq_nn_attention(qd.data_ptr(), H * D, kd.data_ptr(), vd.data_ptr(), out.data_ptr() + 4, pos_dev.data_ptr(), 1, rows, H, KV, D, ctx, max_kv, scale,
+                               ws.data_ptr(), nbytes, None))
+        torch.cuda.synchronize()
+        got.append(out.cpu().numpy())
+        assert got[-1][0] == 7.0 and got[-1][-1] == 7.0
+        assert rel_l2(got[-1][1:-1].reshape(rows, H * D), want) <= TOL
+    assert np.array_equal(got[0], got[1]) == (max_kv < 256 or need >= fits)
+
+
+def test_attention_prompt_split_operands_of_all_sizes():
+    """Scores from -600 to 600 beside values from 1e-30 to 1e30: where one key outweighs all others, its value comes out as it went in."""
+    H, KV, D, rows, pos = 8, 2, 128, 64, 300
+    ctx = pos + rows
+    q, kc, vc = normal(63, (rows, H * D), 1.0), normal(64, (KV, ctx, D), 0.02), normal(65, (KV, ctx, D), 1.0)
+    vc *= np.float32(10.0) ** np.random.Generator(np.random.PCG64(66)).integers(-30, 31, vc.shape).astype(np.float32)
+    q[:, :] = 0.0
+    q[:, ::D] = 30.0                                      # only the first dimension counts, and key 17 is far ahead there
+    kc[:, :, 0], kc[:, 17, 0] = -20.0, 20.0
+    wsb = max(L().cq_nn_attention_workspace_bytes(rows, H, D, ctx), (ctx + 31) // 32 * KV * 49152)
+    ws, out, qd, kd, vd = torch.empty(wsb, dtype=torch.uint8, device="cuda"), torch.empty((rows, H, D), device="cuda"), dev(q), dev(kc), dev(vc)
+    ok(L().cq_nn_attention(qd.data_ptr(), H * D, kd.data_ptr(), vd.data_ptr(), out.data_ptr(), None, pos, rows, H, KV, D, ctx, ctx, 1.0, ws.data_ptr(), wsb, None))
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), np.broadcast_to(np.repeat(vc[:, 17], H // KV, 0), (rows, H, D)))
+
+
 @pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (8, 1, 128), (4, 4, 128), (32, 8, 128)])
 def test_attention_rows_share_keys_with_position_on_device(H, KV, D):
     """16 rows and more go several to a workgroup; the position may come from device memory (a captured graph)."""
