@@ -39,7 +39,17 @@ __device__ __forceinline__ int cq_round_sat_i8(float v) {
 //
 // cq_quantize_q8k_vals takes the lane's four values already in registers, so a caller can issue the
 // load early and overlap its latency with other work.
-__device__ __forceinline__ void cq_quantize_q8k_vals(const float v[4], int64_t blk, int lane, int8_t *qs, float *dout, int16_t *bsums) {
+struct Q8kBlock {                            // a lane's part of a quantized block: four elements, the sum of its group of 16, the scale
+    uint32_t packed;
+    int sum;
+    float d;
+    __device__ __forceinline__ void store(int64_t blk, int lane, int8_t *qs, float *dout, int16_t *bsums) const {
+        reinterpret_cast<uint32_t *>(qs)[blk * 64 + lane] = packed;
+        if ((lane & 3) == 0) bsums[blk * 16 + (lane >> 2)] = (int16_t)sum;
+        if (lane == 0) dout[blk] = d;
+    }
+};
+__device__ __forceinline__ Q8kBlock cq_quantize_q8k_regs(const float v[4], int lane) {
     // signed value of the first element with the largest magnitude (strict `<`: the first one wins)
     float amax = 0.0f;
     int idx = 0;
@@ -66,10 +76,10 @@ __device__ __forceinline__ void cq_quantize_q8k_vals(const float v[4], int64_t b
         }
         d = 1.0f / iscale;
     }
-    reinterpret_cast<uint32_t *>(qs)[blk * 64 + lane] = packed;
-    lsum = quad_sum(lsum);                   // 16-element sums: four neighbouring lanes
-    if ((lane & 3) == 0) bsums[blk * 16 + (lane >> 2)] = (int16_t)lsum;
-    if (lane == 0) dout[blk] = d;
+    return Q8kBlock{packed, quad_sum(lsum), d};      // 16-element sums: four neighbouring lanes
+}
+__device__ __forceinline__ void cq_quantize_q8k_vals(const float v[4], int64_t blk, int lane, int8_t *qs, float *dout, int16_t *bsums) {
+    cq_quantize_q8k_regs(v, lane).store(blk, lane, qs, dout, bsums);
 }
 
 template <int XDT>
@@ -85,7 +95,22 @@ __device__ __forceinline__ void cq_quantize_q8k_span(const void *x, int64_t blk,
 //   qs int8 [..]      ds {float d (f16-rounded), int32 sum} [1 per 32-element block]
 //
 // cq_quantize_q80_vals: the lane's four values (zeros when `valid` is false) are already in registers.
-__device__ __forceinline__ void cq_quantize_q80_vals(const float v[4], bool valid, int64_t base, int lane, int8_t *qs, float *ds) {
+struct Q80Block {                            // a lane's part of a quantized block: four elements, the block's sum, its scale
+    uint32_t packed;
+    int sum;
+    float d;
+    __device__ __forceinline__ void store(int64_t base, int lane, int8_t *qs, float *ds) const {
+        reinterpret_cast<uint32_t *>(qs)[base >> 2] = packed;
+        if ((lane & 7) == 0) {
+            // the CPU path stores d as f16 and multiplies by f16::to_f32(d) in vec_dot
+            u32x2 o;
+            o.x = __float_as_uint(h2f(f2h_bits(d)));
+            o.y = (uint32_t)sum;
+            reinterpret_cast<u32x2 *>(ds)[base >> 5] = o;
+        }
+    }
+};
+__device__ __forceinline__ Q80Block cq_quantize_q80_regs(const float v[4]) {
     float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
     amax = oct_max(amax);                    // a 32-element block = eight neighbouring lanes
     float d = amax / 127.0f;
@@ -98,17 +123,11 @@ __device__ __forceinline__ void cq_quantize_q80_vals(const float v[4], bool vali
         lsum += q;
         packed |= (uint32_t)(q & 0xff) << (8 * i);
     }
-    lsum = oct_sum(lsum);
-    if (!valid) return;
-    reinterpret_cast<uint32_t *>(qs)[base >> 2] = packed;
-    if ((lane & 7) == 0) {
-        // the CPU path stores d as f16 and multiplies by f16::to_f32(d) in vec_dot
-        float d16 = h2f(f2h_bits(d));
-        u32x2 o;
-        o.x = __float_as_uint(d16);
-        o.y = (uint32_t)lsum;
-        reinterpret_cast<u32x2 *>(ds)[base >> 5] = o;
-    }
+    return Q80Block{packed, oct_sum(lsum), d};
+}
+__device__ __forceinline__ void cq_quantize_q80_vals(const float v[4], bool valid, int64_t base, int lane, int8_t *qs, float *ds) {
+    const Q80Block q = cq_quantize_q80_regs(v);
+    if (valid) q.store(base, lane, qs, ds);
 }
 
 template <int XDT>

@@ -143,6 +143,8 @@ int cq_moe_pairs_launch(int w_dtype, const void *w, const float *x, float *out, 
 int cq_moe_pairs_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const float *x, float *out, const PairSource &ps, int64_t k,
                                int64_t n, hipStream_t s);
 
+int cq_quantize_act_spread_launch(int w_dtype, const float *x, const int *tokens, const int *place, int64_t topk, void *scratch, int64_t k, int64_t n_pairs,
+                                  int64_t rows_alloc, hipStream_t s);
 int cq_quantize_act_gather_launch(int w_dtype, const float *x, const int *row_map, void *scratch, int64_t k, int64_t rows, int64_t rows_alloc,
                                   hipStream_t s);
 int cq_quantize_act_swiglu_gather_launch(int w_dtype, const float *gate, const float *up, const int *row_map, const int *n_valid, const float *scale_in,

@@ -51,9 +51,9 @@ inline MoeWorkspace moe_workspace(int w_dtype, int64_t num_experts, int64_t n_pa
 // offsets[e] .. offsets[e+1] is expert e's segment of pair_in / pair_out / pair_scale.
 // LC: the per-expert counters live in LDS (up to GROUP_LDS_EXPERTS experts) instead of the global `cursor` array: the
 // two passes of atomics are then LDS atomics, not trips of one workgroup to the L2.
-// The first KEEP pairs of every thread stay in registers between the two passes.  Decoding a pair is two dependent loads.  MANY: all first ones are asked for
-// before any is used, then all second ones, whether a thread has that many pairs or not.  12000 pairs on 128 experts: 26 us, 30 pair by pair; but what threads
-// without pairs go through, divisions by topk above all, costs a call of 300 - 3000 pairs 2.3 us, one of 4800 1.1, one of 6000 0.4; 8000 gain 0.5.
+// (Lists of expert, token pairs: moe_group_wide_kernel, up to its number of experts.)
+// The first KEEP pairs of every thread stay in registers between the two passes.  MANY (indexed calls): the loads of all of them are asked for before any is used,
+// whether a thread has that many pairs or not, which pays from 6144 pairs on.
 constexpr int GROUP_LDS_EXPERTS = 4096, GROUP_MANY_PAIRS = 6144;
 template <bool LC, bool MANY>
 __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__restrict__ offsets, int *__restrict__ cursor,
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
     if (!MANY) {
 #pragma unroll
         for (int i = 0; i < KEEP; i++) kok[i] = tid + i * 1024 <= last && pair_decode(ps, tid + i * 1024, ke[i], kin[i], kout[i], ksc[i]);
-    } else if (ps.mode == MOE_INDEXED) {
+    } else {
 #pragma unroll
         for (int i = 0; i < KEEP; i++) ke[i] = (int)ps.ids_u32[min(tid + i * 1024, last)];
 #pragma unroll
@@ -85,19 +85,6 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
             kin[i] = ps.input_dim1 == 1 ? kout[i] / ps.topk : kout[i];
             ksc[i] = 1.0f;
             kok[i] = tid + i * 1024 <= last && (uint32_t)ke[i] < (uint32_t)E;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < KEEP; i++) {
-            ke[i] = ps.expert_ids[min(tid + i * 1024, last)];
-            kout[i] = ps.sorted_token_ids[min(tid + i * 1024, last)];
-        }
-#pragma unroll
-        for (int i = 0; i < KEEP; i++) ksc[i] = ps.topk_weights ? ps.topk_weights[min(max(kout[i], 0), last)] : 1.0f;
-#pragma unroll
-        for (int i = 0; i < KEEP; i++) {
-            kin[i] = ps.topk_weights ? kout[i] : kout[i] / ps.topk;
-            kok[i] = tid + i * 1024 <= last && ke[i] >= 0 && ke[i] < E && kout[i] >= 0 && kout[i] <= last && kin[i] < ps.x_rows;
         }
     }
 #pragma unroll
@@ -179,6 +166,91 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
         const bool ok = pair_decode(ps, p, e, in_row, out_row, scale);
         place(p, ok, e, in_row, out_row, scale);
     }
+}
+
+// The same with a workgroup per expert, for lists of (expert, token) pairs of up to GROUP_WIDE_EXPERTS experts: every workgroup counts the whole list in LDS, which
+// comes out of the L2, and then places the pairs of its own expert.  One workgroup for all of them takes 1.7 us per 1000 pairs: its loads, atomics and
+// stores wait for each other on one unit (12000 pairs of 128 experts 25.8 -> 9.6 us; a layer of 256 tokens 142 -> 138).
+// inverse: pair_in[p] is the place of pair p (-1: none) instead of the row at a place.
+constexpr int GROUP_WIDE_EXPERTS = 1024;
+__global__ __launch_bounds__(1024) void moe_group_wide_kernel(PairSource ps, int *__restrict__ offsets, int *__restrict__ pair_in, int *__restrict__ pair_out,
+                                                              float *__restrict__ pair_scale, int *__restrict__ chunks, int max_chunks, int chunk,
+                                                              int *__restrict__ extra, int inverse) {
+    __shared__ int cnt[GROUP_WIDE_EXPERTS], before[4], own;
+    const int tid = threadIdx.x, e = blockIdx.x, E = ps.num_experts, n = ps.n_pairs;
+    // tokens below this have a row and, where rows are weighed, a weight
+    const int limit = (int)min((int64_t)n, ps.topk_weights ? (int64_t)ps.x_rows : (int64_t)ps.x_rows * ps.topk);
+    for (int i = tid; i < E; i += 1024) cnt[i] = 0;
+    if (tid == 0) own = 0;
+    __syncthreads();
+    constexpr int U = 6;                       // pairs of a thread asked for at a time
+    auto each = [&](auto &&f) {
+        for (int p0 = tid; p0 < n; p0 += U * 1024) {
+            int ke[U], to[U];
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                ke[i] = ps.expert_ids[min(p0 + 1024 * i, n - 1)];
+                to[i] = ps.sorted_token_ids[min(p0 + 1024 * i, n - 1)];
+            }
+#pragma unroll
+            for (int i = 0; i < U; i++)
+                if (p0 + 1024 * i < n) f(p0 + 1024 * i, (uint32_t)ke[i] < (uint32_t)E && to[i] >= 0 && to[i] < limit, ke[i], to[i]);
+        }
+    };
+    each([&](int, bool ok, int x, int) {
+        if (ok) atomicAdd(&cnt[x], 1);
+    });
+    __syncthreads();
+    auto passes = [](int c) { return c > 32 ? (c + 31) / 32 - 1 : 0; };       // (of an expert's pairs beyond the first 32, for the batched matvecs)
+    if (tid < 64) {
+        int sum[4] = {0, 0, 0, 0};
+        for (int i = tid; i < E; i += 64) {
+            const int c = cnt[i];
+            sum[3] += c;
+            if (i < e) {
+                sum[0] += c;
+                sum[1] += (c + chunk - 1) / chunk;
+                sum[2] += passes(c);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            for (int o = 32; o; o >>= 1) sum[i] += __shfl_xor(sum[i], o, 64);
+            if (tid == 0) before[i] = sum[i];
+        }
+    }
+    __syncthreads();
+    const int c = cnt[e], start = before[0], n_chunks = (c + chunk - 1) / chunk, cb = before[1], n_extra = extra ? passes(c) : 0, eb = before[2], all = before[3];
+    if (tid == 0) {
+        offsets[e] = start;
+        if (e == E - 1) {
+            offsets[E] = all;
+            chunks[0] = cb + n_chunks;
+            if (extra) { extra[0] = eb + n_extra; extra[1] = 0; extra[2] = 0; }
+        }
+    }
+    for (int i = tid; i < n_chunks; i += 1024) {
+        chunks[1 + cb + i] = e;
+        chunks[1 + max_chunks + cb + i] = start + i * chunk;
+        chunks[1 + 2 * max_chunks + cb + i] = min(chunk, c - i * chunk);
+    }
+    for (int i = tid; i < n_extra; i += 1024) {
+        extra[CQ_MOE_EXTRA_HEADER + 2 * (eb + i)] = e;
+        extra[CQ_MOE_EXTRA_HEADER + 2 * (eb + i) + 1] = i + 1;
+    }
+    each([&](int p, bool ok, int x, int tok) {
+        if (ok && x == e) {
+            const int pos = start + atomicAdd(&own, 1);
+            if (inverse) pair_in[p] = pos;
+            else pair_in[pos] = ps.topk_weights ? tok : tok / ps.topk;
+            pair_out[pos] = tok;
+            pair_scale[pos] = ps.topk_weights ? ps.topk_weights[tok] : 1.0f;
+        }
+        if (!ok && inverse && e == 0) pair_in[p] = -1;
+    });
+    // places behind the last valid pair are in no chunk, but a gathering quantizer walks all of them
+    if (!inverse && e == 0)
+        for (int p = all + tid; p < n; p += 1024) pair_in[p] = 0;
 }
 
 // Workgroup (blockIdx.x = row tile, blockIdx.y = expert); 4 waves x R rows.  Pairs of the expert are
@@ -341,11 +413,19 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     // Hundreds of pairs per call: the expert-sorted rows go through the MFMA prefill kernel of the format in tiles of up to
     // 128 rows of one expert (integer-exact like the dense paths).  Otherwise 8 pairs per matvec pass.
     const int tile_rows = moe_tile_rows(a.n_pairs, a.num_experts);
-    const bool many = a.n_pairs > GROUP_MANY_PAIRS;
+    const bool many = a.mode == MOE_INDEXED && a.n_pairs > GROUP_MANY_PAIRS;
     auto *const group = a.num_experts <= GROUP_LDS_EXPERTS ? (many ? moe_group_kernel<true, true> : moe_group_kernel<true, false>)
                                                            : (many ? moe_group_kernel<false, true> : moe_group_kernel<false, false>);
-    hipLaunchKernelGGL(group, dim3(1), dim3(1024), 0, s, ps, offsets, cursor, pin, pout, pscale, a.out, (int)a.n, chunks, (int)ws.max_chunks,
-                       stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK, stream ? extra : nullptr);
+    const int chunk = stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK;
+    const bool wide = a.mode != MOE_INDEXED && a.num_experts <= GROUP_WIDE_EXPERTS;
+    // pairs of the gate / up products: the same row goes to all experts of a token
+    const bool spread = wide && mfma && !stream && !a.topk_weights && a.topk > 1;
+    if (wide)
+        hipLaunchKernelGGL(moe_group_wide_kernel, dim3((unsigned)a.num_experts), dim3(1024), 0, s, ps, offsets, pin, pout, pscale, chunks, (int)ws.max_chunks, chunk,
+                           stream ? extra : nullptr, (int)spread);
+    else
+        hipLaunchKernelGGL(group, dim3(1), dim3(1024), 0, s, ps, offsets, cursor, pin, pout, pscale, a.out, (int)a.n, chunks, (int)ws.max_chunks, chunk,
+                           stream ? extra : nullptr);
     if ((rc = (int)hipGetLastError())) return rc;
     if (stream) {
         // every expert a batched matvec over its own pairs: the weights of an expert are streamed once per 32 pairs
@@ -354,7 +434,9 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
         return cq_moe_stream_launch(a.w_dtype, a.w, a.w_b, a.out, a.out_b, b + ws.act_off, offsets, pout, pscale, extra, 0, a.num_experts, a.k, a.n, s);
     }
     if (mfma) {
-        if ((rc = cq_quantize_act_gather_launch(a.w_dtype, a.x, pin, b + ws.act_off, a.k, a.n_pairs, ws.rows_alloc, s))) return rc;
+        rc = spread ? cq_quantize_act_spread_launch(a.w_dtype, a.x, a.sorted_token_ids, pin, a.topk, b + ws.act_off, a.k, a.n_pairs, ws.rows_alloc, s)
+                    : cq_quantize_act_gather_launch(a.w_dtype, a.x, pin, b + ws.act_off, a.k, a.n_pairs, ws.rows_alloc, s);
+        if (rc) return rc;
         MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
         rc = cq_matmul_moe_launch(a.w_dtype, a.w, b + ws.act_off, ws.rows_alloc, a.out, mc, a.num_experts, a.k, a.n, tile_rows, s);
         if (!rc && a.w_b) rc = cq_matmul_moe_launch(a.w_dtype, a.w_b, b + ws.act_off, ws.rows_alloc, a.out_b, mc, a.num_experts, a.k, a.n, tile_rows, s);

@@ -69,3 +69,45 @@ def test_grouping_at_the_change_of_form(tokens, weights):
         t, s = np.nonzero(ids == e)
         assert rel_l2(got[t, s], oracle.matmul(oracle.Q8_0, x[t], blocks[e * len(blocks) // E:(e + 1) * len(blocks) // E], n)) <= 2e-6
     assert (got[ids == E] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [oracle.Q8_0, oracle.Q6K])
+@pytest.mark.parametrize("E,tokens,top,order", [(3, 2048, 3, "tokens"), (3, 2049, 3, "shuffled"), (1024, 700, 2, "tokens"), (1025, 700, 2, "tokens"), (1, 300, 2, "shuffled"),
+                                                (70, 30, 65, "tokens"), (9, 1025, 6, "twice")])
+def test_grouping_of_lists(dtype, E, tokens, top, order):
+    """Lists of pairs at the edges of what a thread takes at a time (6144 pairs), of the experts that get a workgroup each (1024) and of a wave's 64 pairs, in token order
+    (a row is quantized once for its pairs), shuffled, and with every entry of the first half listed again in place of one of the second: valid pairs get their
+    product, and pairs that name no expert or no token write nothing."""
+    import candle_amd as ca
+    n, k = 12, 256
+    blocks = oracle.from_float(dtype, normal(5, (E, n, k), 0.02).reshape(-1))
+    qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(dtype)), (E, n, k))
+    pairs, rng = tokens * top, np.random.default_rng(tokens)
+    experts, order_of = rng.integers(0, E, pairs).astype(np.int32), np.arange(pairs, dtype=np.int32)
+    if order == "shuffled":
+        order_of = rng.permutation(pairs).astype(np.int32)
+    if order == "twice":
+        half = pairs // 2
+        order_of[half:2 * half], experts[half:2 * half] = order_of[:half], experts[:half]
+    bad = rng.choice(pairs // 2, 9, replace=False)
+    if order != "twice":
+        experts[bad[:3]], experts[bad[3:5]] = -1, E
+        order_of[bad[5:7]], order_of[bad[7:]] = -1, pairs
+    x, L = normal(6, (tokens, k)), _lib.lib()
+    cuda = lambda a: torch.from_numpy(a).cuda()
+    xd, od, ed = cuda(x), cuda(order_of), cuda(experts)
+    out = torch.full((pairs, n), 7.0, device="cuda")
+    ws = torch.full((L.cq_moe_gemm_workspace_bytes(int(dtype), E, top, pairs, n, k, 0),), 255, dtype=torch.uint8, device="cuda")
+    _lib.check("cq_moe_gemm_gguf", L.cq_moe_gemm_gguf(int(dtype), xd.data_ptr(), qt.device_ptr(), od.data_ptr(), ed.data_ptr(), None, out.data_ptr(), E, top, pairs, n, k, 1,
+                                                      ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    got, want = out.cpu().numpy(), np.full((pairs, n), 7.0, np.float32)
+    valid = (experts >= 0) & (experts < E) & (order_of >= 0) & (order_of < pairs)
+    per = len(blocks) // E
+    for e in range(E):
+        rows = order_of[valid & (experts == e)]
+        if len(rows):
+            want[rows] = oracle.matmul(dtype, x[rows // top], blocks[e * per:(e + 1) * per], n)
+    hit = np.zeros(pairs, bool)
+    hit[order_of[valid]] = True
+    assert rel_l2(got[hit], want[hit]) <= 2e-6 and (got[~hit] == 7.0).all() and (~hit).any()
