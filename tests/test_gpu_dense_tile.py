@@ -74,3 +74,46 @@ def test_stages_on_their_way(k, splits):
     err = (y[1:m + 1, :n].double() - want).norm(dim=1) / want.norm(dim=1)
     assert float(err.max()) <= BOUND
     assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, n:] == 5).all()
+
+
+@pytest.mark.parametrize("m,n,k,pad", [(1100, 2500, 1024, 0), (1535, 2049, 1088, 64), (1500, 2817, 1024, 128), (1537, 2700, 4160, 0), (1290, 4485, 1024, 0), (1000, 5602, 1024, 0), (1500, 5633, 1088, 64)])
+@pytest.mark.parametrize("form", ["plain", "add", "swiglu", "bf16", "rows"])
+def test_ring_of_stages(m, n, k, pad, form):
+    """One workgroup to a unit: 128 rows (180 and 204 tiles), 192 (one round), 128 in two rounds, 192 in two; stages of k even and odd."""
+    print(f"case {m} {n} {k} {pad} {form}", flush=True)
+    if form == "swiglu":
+        n &= ~1
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = torch.randn((n, k + pad), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k + pad), generator=g, device="cuda").bfloat16()
+    x[:, k:], w[:, k:] = float("nan"), float("nan")
+    cols = n // 2 if form == "swiglu" else n
+    y = torch.full((m + 2, cols + 3), 5.0, device="cuda", dtype=torch.bfloat16 if form == "bf16" else torch.float32)
+    add = torch.randn((m, n), generator=g, device="cuda") if form == "add" else None
+    perm = torch.randperm(m, generator=g, device="cuda").int() if form == "rows" else None
+    scale = torch.rand(m, generator=g, device="cuda") + 0.5 if form == "swiglu" else None
+    a = DenseArgs(w_dev=w.data_ptr(), ldw=k + pad, x_dev=x.data_ptr(), ldx=k + pad, x_bf16=1, dst_dev=y[1].data_ptr(), ldd=cols + 3, m=m, n=n, k=k, batch=1,
+                  dst_bf16=int(form == "bf16"), act=2 if form == "swiglu" else 0, accumulate=int(form == "add"), add_dev=add.data_ptr() if form == "add" else None,
+                  ld_add=n if form == "add" else 0, dst_rows_dev=perm.data_ptr() if form == "rows" else None, row_scale_dev=scale.data_ptr() if form == "swiglu" else None)
+    L = _lib.mixer_lib()
+    nb = L.cq_dense_matmul_workspace_bytes(0, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    want = x[:, :k].double() @ w[:, :k].double().t()
+    size = want.norm(dim=1, keepdim=True)
+    if form == "add":
+        want += add + 5.0
+    if form == "swiglu":
+        want = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2] * scale[:, None]
+    got = y[1:m + 1, :cols].double()
+    if form == "rows":
+        got = got[perm.long()]
+    err = (got - want).abs()
+    if form == "bf16":
+        err = (err - want.abs() * 2.0 ** -8).clamp(min=0)
+    if form == "add":
+        err = (err - want.abs() * 2.0 ** -23).clamp(min=0)              # two more roundings
+    assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * (4 if form == "swiglu" else 1)
+    assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, cols:] == 5).all()
+
