@@ -1,6 +1,7 @@
 // Softmax attention whose scores are mixed across heads before the softmax, over a sliding window plus the first tokens of
 // the sequence.  Mixing couples the heads, so one workgroup holds the scores of all heads for its queries and keys.
 // f32 throughout (v_mfma_f32_16x16x4): scores, weights, caches.
+#include <algorithm>
 #include "cq_mix.h"
 
 namespace {
@@ -222,6 +223,188 @@ __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__
     }
 }
 
+// ---- several queries, heads of 128 dimensions in groups of R = 2, 4 or 8 on one kv head, H = 8 or 16 of them -----------------------------------
+// Workgroup: 16 query rows x all heads, one wave a head, keys in tiles of 16.  Above, every wave reads its queries, keys and values from the caches for every tile, 40 KB a
+// wave and 32 keys through a unit's 64 bytes a cycle, and three barriers separate that from the mixing.  Here the queries stay in registers, and copies that no
+// register sees bring keys and values to LDS two tiles ahead, once for the R heads that share them.  Per tile:
+//   mixing   wave w takes 16 / H queries of all heads, as above; running maxima and sums in its registers
+//   values   wave w: the weights of head w x V onto its outputs, then the scores of the next tile, which replace those weights when they are formed
+// so that only the mixing stands between two barriers.
+// LDS rows of 512 bytes in 32 16-byte chunks: keys' chunk c of row r at c ^ r, values as they are; both without bank conflicts.
+// 16 heads in us, above -> this: 2048 rows (window 1024) 327 -> 210, 500: 111 -> 53, 100: 65 -> 30; the error against 64 bits falls (2048 rows 4.9e-7 -> 4.0e-7: scores in two
+// sums).  Bound by the f32 matrix instructions, 68 of 32 cycles a wave and tile, four waves to a matrix core: 63 % of a unit's cycles, the rest barriers and
+// the mixing; and by the first rows, which see fewer keys than the last and leave a quarter of the units' time idle.
+typedef __attribute__((address_space(3))) void talk_lds;
+constexpr int TT_RS = 20, TT_HS = 16 * TT_RS + 16, TT_ROW = 512, TT_TILE = 16 * TT_ROW;      // floats of a query's weights, of a head's; bytes of a key, of a tile
+__host__ __device__ constexpr int talk_tile_lds(int H, int R) { return 4 * (H / R) * TT_TILE + (H * TT_HS + 3 * 256) * 4; }
+
+template <int H, int R, typename OT>
+__global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restrict__ q, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
+                                                           const float *__restrict__ talk, float scale, int window, int keep_first, float out_scale, OT *__restrict__ out,
+                                                           int64_t out_stride, float *__restrict__ part, int pos, int rows, int vdim, int ctx) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
+    constexpr int G = H / R, RW = 16 / H, NI = 8 / R, HALF = G * TT_TILE;       // queries of a wave in the mixing; copies of a wave for a tile of keys
+    extern __shared__ __attribute__((aligned(16))) uint8_t tt_smem[];
+    uint8_t *const kbuf = tt_smem, *const vbuf = tt_smem + 2 * HALF;
+    float *const S = reinterpret_cast<float *>(tt_smem + 4 * HALF), *const alpha = S + H * TT_HS, *const m_run = alpha + 256, *const l_run = m_run + 256;
+    const int lane = threadIdx.x & 63, h = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lk = lane >> 4;
+    const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 16, nr = min(16, rows - r0), p0 = pos + r0, last = p0 + nr - 1;      // (the long ones first)
+    // tiles of the kept first tokens, then of the window; the share of this split
+    const int t_lo = max(0, p0 - window + 1) / 16, n_keep = min((keep_first + 15) / 16, t_lo), n_tiles = n_keep + last / 16 - t_lo + 1, nz = gridDim.z, z = blockIdx.z;
+    const int it0 = n_tiles * z / nz, it1 = n_tiles * (z + 1) / nz;
+    auto first_key = [&](int it) { return 16 * (it < n_keep ? it : t_lo + it - n_keep); };
+
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)k_cache, 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void *)v_cache, 0, -1, 0x00020000);
+    // two rows an instruction, rows beyond the last visible key repeat it (past the last tile: that one again, for nobody)
+    auto copy = [&](auto values, int it) {
+        uint8_t *const to = (values ? vbuf : kbuf) + ((it - it0) & 1) * HALF;
+        const int j0 = first_key(min(it, it1 - 1));
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const int u = h + H * j, g = u >> 3, row = 2 * (u & 7) + (lane >> 5), c = values ? lane & 31 : (lane & 31) ^ row;
+            const uint32_t at = (uint32_t)(g * ctx + min(j0 + row, last)) * TT_ROW + 16 * c;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(values ? vrs : krs, (talk_lds *)(to + 1024 * u), 16, at, 0, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    };
+    constexpr std::integral_constant<bool, false> keys{};
+    constexpr std::integral_constant<bool, true> values{};
+    f32x4 qd[8];                                           // dims 16 c + 4 lk .. of query lr
+    float tf[H / 4], m[RW][4], l[RW][4];                   // mixing weights [head lr][4 s + lk]; of head 4 lk + e and the wave's queries (l: of this lane's keys)
+    {
+        const float *qr = q + ((int64_t)(r0 + min(lr, nr - 1)) * H + h) * 128 + 4 * lk;
+#pragma unroll
+        for (int c = 0; c < 8; c++) qd[c] = *reinterpret_cast<const f32x4 *>(qr + 16 * c);
+    }
+#pragma unroll
+    for (int s = 0; s < H / 4; s++) tf[s] = lr < H ? talk[min(lr, H - 1) * H + 4 * s + lk] * scale : 0.0f;
+#pragma unroll
+    for (int a = 0; a < RW; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            m[a][e] = -INFINITY;
+            l[a][e] = 0.0f;
+        }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 o[2][4];                                         // queries 4 lk .. of column 64 x + 4 lr + n
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int n = 0; n < 4; n++) o[x][n] = zero;
+    bool stale[RW];
+#pragma unroll
+    for (int a = 0; a < RW; a++) stale[a] = false;
+    float *const Sh = S + h * TT_HS;
+    auto scores = [&](int it) {                            // of the wave's head, into S
+        const uint8_t *const kt = kbuf + ((it - it0) & 1) * HALF + (h / R) * TT_TILE + lr * TT_ROW;
+        f32x4 sc[2] = {zero, zero};
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const f32x4 kf = *reinterpret_cast<const f32x4 *>(kt + 16 * ((4 * c + lk) ^ lr));
+#pragma unroll
+            for (int e = 0; e < 4; e++) sc[c & 1] = mfma4(qd[c][e], kf[e], sc[c & 1]);
+        }
+        const f32x4 s = sc[0] + sc[1];
+#pragma unroll
+        for (int e = 0; e < 4; e++) Sh[(4 * lk + e) * TT_RS + lr] = s[e];
+    };
+    if (it0 < it1) {
+        copy(keys, it0);
+        copy(values, it0);
+        copy(keys, it0 + 1);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NI) : "memory");
+        scores(it0);
+    }
+    for (int it = it0; it < it1; it++) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the scores of all heads are there
+        const int j = first_key(it) + lr;
+#pragma unroll
+        for (int a = 0; a < RW; a++) {
+            const int qi = RW * h + a, p = p0 + qi;
+            f32x4 acc = zero;
+#pragma unroll
+            for (int s = 0; s < H / 4; s++) acc = mfma4(tf[s], S[(4 * s + lk) * TT_HS + qi * TT_RS + lr], acc);
+            const bool vis = j <= p && (p - j < window || j < keep_first);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = vis ? acc[e] : -INFINITY;
+            const bool up = acc[0] > m[a][0] || acc[1] > m[a][1] || acc[2] > m[a][2] || acc[3] > m[a][3];
+            if (__any(up) || stale[a]) {                   // a new maximum, or one in the tile before
+                stale[a] = __any(up);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float top = fmaxf(m[a][e], row16_max(acc[e])), al = m[a][e] > -INFINITY ? __expf(m[a][e] - top) : 0.0f;
+                    m[a][e] = top;
+                    l[a][e] *= al;
+                    if (H == 16 || lk < 2) alpha[(4 * lk + e) * 16 + qi] = al;      // (the same value from 16 lanes)
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float w = vis ? __expf(acc[e] - m[a][e]) : 0.0f;
+                l[a][e] += w;
+                if (H == 16 || lk < 2) S[(4 * lk + e) * TT_HS + qi * TT_RS + lr] = w;
+            }
+        }
+        // the weights of all queries are there, and so are the values of this tile and the keys of the next
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        copy(values, it + 1);
+        copy(keys, it + 2);
+        const f32x4 al = *reinterpret_cast<const f32x4 *>(&alpha[h * 16 + 4 * lk]);
+        if (__any(al.x != 1.0f || al.y != 1.0f || al.z != 1.0f || al.w != 1.0f)) {
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int n = 0; n < 4; n++) o[x][n] *= al;
+        }
+        const uint8_t *const vt = vbuf + ((it - it0) & 1) * HALF + (h / R) * TT_TILE + lk * TT_ROW + 16 * lr;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const float w = Sh[lr * TT_RS + 4 * s + lk];
+#pragma unroll
+            for (int x = 0; x < 2; x++) {
+                const f32x4 vf = *reinterpret_cast<const f32x4 *>(vt + 4 * s * TT_ROW + 256 * x);
+#pragma unroll
+                for (int n = 0; n < 4; n++) o[x][n] = mfma4(w, vf[n], o[x][n]);
+            }
+        }
+        if (it + 1 < it1) scores(it + 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (copies may not outlive the workgroup)
+#pragma unroll
+    for (int a = 0; a < RW; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            l_run[(4 * lk + e) * 16 + RW * h + a] = row16_sum(l[a][e]);
+            m_run[(4 * lk + e) * 16 + RW * h + a] = m[a][e];
+        }
+    __syncthreads();
+    const f32x4 lh = *reinterpret_cast<const f32x4 *>(&l_run[h * 16 + 4 * lk]);
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int row = 4 * lk + e, col = 64 * x + 4 * lr;
+            if (row >= nr) continue;
+#pragma unroll
+            for (int n = 0; n < 4; n++) {
+                if (col + n >= vdim) continue;
+                if (nz == 1) out[(int64_t)(r0 + row) * out_stride + (int64_t)h * vdim + col + n] = (OT)(out_scale * o[x][n][e] / lh[e]);
+                else part[((int64_t)(z * rows + r0 + row) * H + h) * vdim + col + n] = o[x][n][e];
+            }
+        }
+    if (nz > 1) {
+        float *ml = part + (int64_t)nz * rows * H * vdim;                 // [split][row][head] of (m, l)
+        for (int i = threadIdx.x; i < nr * H; i += 64 * H) {
+            const int row = i / H, hh = i - row * H;
+            float *x = ml + 2 * ((int64_t)(z * rows + r0 + row) * H + hh);
+            x[0] = m_run[hh * 16 + row];
+            x[1] = l_run[hh * 16 + row];
+        }
+    }
+#endif
+}
+
 // one wave per (row, head)
 template <typename OT>
 __global__ __launch_bounds__(256) void talk_combine_kernel(const float *__restrict__ part, int nz, int64_t rows, int H, int vdim, float out_scale,
@@ -251,6 +434,19 @@ int talk_key_splits(int64_t rows, int64_t unit_blocks, int64_t max_keys) {
     n = n < tiles / 4 ? n : tiles / 4;
     return (int)(n < 1 ? 1 : (n > 16 ? 16 : n));
 }
+// The same for talk_tile_kernel, with at least two tiles of 16 keys each: 200 rows in one split 77.6 us, in six 37.1.  (More workgroups than units gain nothing: 2048
+// rows in two splits 210, in four 230.)
+int talk_tile_splits(int64_t rows, int64_t max_keys) {
+    int64_t n = 256 / ((rows + 15) / 16);
+    n = std::min(n, (max_keys + 15) / 32);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(n, 16));
+}
+// Which calls talk_tile_kernel takes: what it has instances for, LDS for up to four kv heads, offsets of 32 bits into the caches.  It is the faster one at all sizes
+// (16 heads: 20 rows 22.8 -> 21.0 us, 100: 65 -> 31, 500: 111 -> 54, 2048: 327 -> 210; 8 heads, 2048 rows 196 -> 132).
+bool talk_by_tiles(int64_t H, int64_t G, int64_t dim_pad, int64_t vdim_pad, int64_t ctx) {
+    const int64_t R = H / G;
+    return dim_pad == 128 && vdim_pad == 128 && (H == 8 || H == 16) && (R == 4 || R == 8 || (R == 2 && H == 8)) && G * ctx < (1LL << 23);
+}
 int talk_unit_blocks(int64_t H, int64_t vp) {               // units a launch takes: NW * U of the instance for H heads
     const int64_t per = H <= 8 ? 16 : (H <= 16 ? 32 : 64);
     return (int)((H * ((vp + 63) / 64) + per - 1) / per);
@@ -269,6 +465,20 @@ int talk_launch(const float *q, const float *kc, const float *vc, const float *t
     const int units = H * ((vp + 63) / 64);
     hipLaunchKernelGGL((talk_attention_kernel<NW, NHW, SHARED_K, U, VS, KT, OT>), dim3((rows + 15) / 16, (units + NW * U - 1) / (NW * U), nz), dim3(64 * NW), lds,
                        s, q, kc, vc, talk, scale, window, keep, out_scale, out, out_stride, part, pos, rows, H, G, dp, vdim, vp, ctx);
+    if (nz > 1)
+        hipLaunchKernelGGL(talk_combine_kernel<OT>, dim3((unsigned)rows, (unsigned)((H + 3) / 4)), dim3(256), 0, s, (const float *)part, nz, (int64_t)rows, H, vdim, out_scale,
+                           out, out_stride);
+    return (int)hipGetLastError();
+}
+
+template <int H, int R, typename OT>
+int talk_tile_launch(const float *q, const float *kc, const float *vc, const float *talk, float scale, int window, int keep, float out_scale, OT *out, int64_t out_stride,
+                     float *part, int nz, int pos, int rows, int vdim, int ctx, hipStream_t s) {
+    constexpr int lds = talk_tile_lds(H, R);
+    const int e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(talk_tile_kernel<H, R, OT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e) return e;
+    hipLaunchKernelGGL((talk_tile_kernel<H, R, OT>), dim3((rows + 15) / 16, 1, nz), dim3(64 * H), lds, s, q, kc, vc, talk, scale, window, keep, out_scale, out, out_stride, part,
+                       pos, rows, vdim, ctx);
     if (nz > 1)
         hipLaunchKernelGGL(talk_combine_kernel<OT>, dim3((unsigned)rows, (unsigned)((H + 3) / 4)), dim3(256), 0, s, (const float *)part, nz, (int64_t)rows, H, vdim, out_scale,
                            out, out_stride);
@@ -508,10 +718,12 @@ int talk_decode_launch(const float *row, const cq_mix_heads *g, float eps, const
     return (int)hipGetLastError();
 }
 
+int64_t talk_split_bytes(int64_t rows, int64_t H, int64_t vdim) { return rows * H * (vdim + 2) * 4; }
 int64_t talk_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos) {
     if (rows <= 0 || n_head <= 0 || vdim <= 0 || window < 1 || keep_first < 0 || pos < 0) return 0;
-    const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, (vdim + 15) / 16 * 16), talk_max_keys(window, keep_first, pos + rows));
-    return nz > 1 ? nz * rows * n_head * (vdim + 2) * 4 : 0;
+    const int64_t max_keys = talk_max_keys(window, keep_first, pos + rows), vp = (vdim + 15) / 16 * 16;
+    const int nz = std::max(talk_key_splits(rows, talk_unit_blocks(n_head, vp), max_keys), vp == 128 && (n_head == 8 || n_head == 16) ? talk_tile_splits(rows, max_keys) : 1);
+    return nz > 1 ? talk_split_bytes(rows, n_head, vdim) * nz : 0;
 }
 
 template <typename OT>
@@ -528,12 +740,28 @@ int talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_
     if (ctx * (dim_pad > vdim_pad ? dim_pad : vdim_pad) * 4 > 0x7fffffffLL) return CQ_ERR_RANGE;      // byte offsets inside a kv head are 32-bit
     const int w = (int)(window < ctx ? window : ctx), keep = (int)(keep_first < ctx ? keep_first : ctx);
     const int H = (int)n_head, G = (int)n_kv_head, R = H / G;
-    const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vdim_pad), talk_max_keys(window, keep_first, pos + rows));
-    if (nz > 1 && (!workspace_dev || workspace_bytes < talk_workspace_bytes(rows, n_head, vdim, window, keep_first, pos))) return CQ_ERR_WORKSPACE;
+    const bool by_tiles = talk_by_tiles(n_head, n_kv_head, dim_pad, vdim_pad, ctx);
+    const int64_t max_keys = talk_max_keys(window, keep_first, pos + rows);
+    const int64_t split_bytes = talk_split_bytes(rows, n_head, vdim);
+    int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vdim_pad), max_keys);
+    if (nz > 1 && (!workspace_dev || workspace_bytes < nz * split_bytes)) return CQ_ERR_WORKSPACE;
+    if (by_tiles)                                          // (as many of its splits as the workspace holds)
+        nz = (int)std::max<int64_t>(1, std::min<int64_t>(talk_tile_splits(rows, max_keys), workspace_dev ? workspace_bytes / split_bytes : 1));
     hipStream_t s = (hipStream_t)stream;
 #define CQ_TA(NW_, NHW_, SH_, U_, VS_, KT_)                                                                                                            \
     talk_launch<NW_, NHW_, SH_, U_, VS_, KT_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride,      \
                                               (float *)workspace_dev, nz, (int)pos, (int)rows, H, G, (int)dim_pad, (int)vdim, (int)vdim_pad, (int)ctx, s)
+    if (by_tiles) {
+#define CQ_TT(H_, R_)                                                                                                                                  \
+    talk_tile_launch<H_, R_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride, (float *)workspace_dev, nz, (int)pos, (int)rows, \
+                             (int)vdim, (int)ctx, s)
+        if (H == 16 && R == 4) return CQ_TT(16, 4);
+        if (H == 16 && R == 8) return CQ_TT(16, 8);
+        if (H == 8 && R == 2) return CQ_TT(8, 2);
+        if (H == 8 && R == 4) return CQ_TT(8, 4);
+        if (H == 8 && R == 8) return CQ_TT(8, 8);
+#undef CQ_TT
+    }
     if (H <= 8) return R % 2 ? CQ_TA(8, 1, true, 2, 1, 32) : CQ_TA(8, 1, true, 2, 2, 32);
     if (H <= 16) return R % 2 ? CQ_TA(16, 1, true, 2, 1, 32) : CQ_TA(16, 1, true, 2, 2, 32);
     if (H <= 32) return R % 2 ? CQ_TA(16, 2, false, 4, 1, 32) : (R % 4 ? CQ_TA(16, 2, true, 4, 2, 32) : CQ_TA(16, 2, true, 4, 4, 32));

@@ -212,6 +212,19 @@ def test_talk_attention(H, G, d, e, window, keep, pos, rows):
     assert rel(attend(q, k, v, talk, scale, window, keep, pos, rows, 0.6), 0.6 * want) < 5e-6
 
 
+@pytest.mark.parametrize("H,G", [(16, 4), (16, 2), (8, 4), (8, 2), (8, 1)])
+@pytest.mark.parametrize("e,window,keep,pos,rows", [(128, 1000, 0, 0, 1), (128, 16, 0, 0, 65), (128, 17, 1, 31, 33), (120, 40, 33, 70, 47), (113, 15, 16, 100, 16), (128, 300, 4, 5, 500),
+                                                    (128, 64, 200, 90, 150)])
+def test_talk_attention_tiles(H, G, e, window, keep, pos, rows):
+    """Heads of 128 dimensions: windows and kept tokens at the edges of tiles of 16 keys, rows that do not fill 16, value columns that do not fill 128, one split and several."""
+    T, d = pos + rows, 128
+    q, k, v, talk = rnd(1, T, H, d), rnd(2, T, G, d), rnd(3, T, G, e), np.eye(H, dtype=np.float32) + rnd(4, H, H, scale=0.4)
+    k[T // 2] *= 20.0                                   # a maximum that comes late and goes: scores of 150, whose last bit (2^-17) is the weights' error
+    scale = 1.5 * d ** -0.5
+    want = vo.talking_attention(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), talk.astype(np.float64), scale, vo.window_mask(T, window, keep))[pos:]
+    assert rel(attend(q, k, v, talk, scale, window, keep, pos, rows, 0.6), 0.6 * want) < 2e-5
+
+
 @pytest.mark.parametrize("window,keep,T", [(7, 0, 60), (32, 3, 150), (33, 32, 150), (64, 33, 300), (200, 1, 900)])
 def test_talk_attention_edges_stand_out(window, keep, T):
     """One key whose score and value stand out, just inside and just outside the window and the kept first tokens: head 0 returns its value
