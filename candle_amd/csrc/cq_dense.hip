@@ -113,6 +113,19 @@ __device__ __forceinline__ void tile_at(int t, int tiles_m, int tiles_n, int &tm
     tn = in / wide;
 }
 
+// Tile t of a grouped product's order: all tiles of a group (of those in the same sixteen of the table) side by side, column by column, so that its weights are
+// read once, and then the next group.  (By a fixed number of row tiles, as above, tiles of one group fall to two runs of workgroups: 1500 tokens, 64 experts of which the largest have three
+// times the mean, 1.06 GB come from behind the L2 for 740 MB of weights, and 0.86 so: 263 -> 245 us.)
+__device__ __forceinline__ void group_tile_at(const Src &s, int t, int tiles_m, int tiles_n, int lane, int &tm, int &tn) {
+    const int at = t / tiles_n, base = at & ~15, x = base + (lane & 15);
+    const int group = s.tiles[at].group;
+    const uint32_t same = (uint32_t)__ballot(x < tiles_m && s.tiles[min(x, tiles_m - 1)].group == group) & 0xffffu;
+    const int me = at - base, below = __builtin_clz(~(same << (31 - me))) - 1, above = __builtin_ctz(~(same >> me)) - 1;      // of the same group in a row before and after
+    const int first = at - below, wide = below + above + 1, in = t - first * tiles_n;
+    tm = first + in % wide;
+    tn = in / wide;
+}
+
 // ---- bf16 tiles: BM activation rows x BN weight rows, k in steps of 64, LDS double-buffered -----------------------------
 // The weights are the A operand, so a lane ends with four consecutive output columns of one row.  LDS rows are 128 bytes in
 // eight 16-byte chunks, chunk c of row r at c ^ (r / 2) % 8, without bank conflicts; c ^ r % 8, with two lanes to a bank, for the large tile of f32 activations,
@@ -134,7 +147,8 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
         if ((int)blockIdx.x >= tiles_m * tiles_n) return;
     }
     int tm, tn;
-    tile_at(xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
+    if (src.tiles) group_tile_at(src, xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, lane, tm, tn);
+    else tile_at(xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
     int64_t m0 = (int64_t)tm * BM;
     const uint16_t *w = src.w + blockIdx.z * src.w_batch;
     if (src.tiles) {
