@@ -292,6 +292,14 @@ class Attention:
 SHAPES = [(1, 8, 2, 8, 8, 70), (3, 24, 10, 40, 36, 140), (16, 72, 24, 56, 112, 150), (5, 128, 64, 128, 512, 130), (18, 40, 16, 20, 130, 90), (33, 16, 8, 12, 256, 70), (2, 250, 64, 250, 200, 80), (3, 32, 150, 24, 90, 100)]
 
 
+@pytest.mark.parametrize("H,d,r,e,rank", [(3, 128, 64, 128, 256), (8, 64, 32, 96, 128)])
+@pytest.mark.parametrize("cuts", [[65], [128], [129], [64, 1, 63, 65], [193, 3], [256, 1, 64], [321]])
+def test_expanded_attention_even_and_odd_tiles(H, d, r, e, rank, cuts):
+    """Two sets of waves on the even and the odd tiles of 64 keys: one tile and two, odd counts, rows that see nothing of a set's only tile."""
+    a = Attention(H, d, r, e, rank, sum(cuts), mixers.BF16)
+    assert rel(a.run(cuts, "expanded"), a.want()) < dict(TYPES)[mixers.BF16]
+
+
 @pytest.mark.parametrize("precision,tol", TYPES)
 @pytest.mark.parametrize("H,d,r,e,rank,T", SHAPES)
 def test_latent_attention_forms_and_portions(H, d, r, e, rank, T, precision, tol):
