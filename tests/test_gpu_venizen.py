@@ -353,6 +353,24 @@ def test_retention_portions(H, d, e, cuts):
     assert rel(state[:, :, :d], S.transpose(0, 2, 1)) < 1e-5 and not state[:, :, d:].any()
 
 
+@pytest.mark.parametrize("n,held", [(100, 0), (200, 2), (1000, 8)])
+def test_retention_with_less_workspace(n, held):
+    """A workspace that holds the states of segments of two chunks only (held of them; none for a call that is not cut so) gives the same within rounding, one with less
+    is refused."""
+    L, H, d, e = _lib.mixer_lib(), 3, 32, 64
+    q, k, v = rnd(1, n, H, d), rnd(2, n, H, d, scale=d ** -0.5), rnd(3, n, H * e)
+    need, small, outs = L.cq_mix_retention_workspace_bytes(n, H, d, e), H * held * d * 64 * 4, []
+    assert need > small
+    qd, kd, vd, l2 = up(q), up(k), up(v), up(np.log2(np.array([0.9, 0.97, 1.0])))
+    for nbytes in (need, small, small - 4):
+        state, out, ws = torch.zeros((H, e, 64), device=DEV), torch.zeros((n, H * e), device=DEV), torch.full((max(nbytes, 4) // 4,), float("nan"), device=DEV)
+        r = L.cq_mix_retention(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), H * e, l2.data_ptr(), state.data_ptr(), out.data_ptr(), H * e, n, H, d, d, e,
+                               ws.data_ptr() if nbytes > 0 else None, nbytes, sp())
+        assert r == (-5 if 0 < nbytes < small else 0)
+        outs.append(torch.cat([out.flatten(), state.flatten()]).double().cpu().numpy())
+    assert rel(outs[1], outs[0]) < 2e-6
+
+
 def test_retention_remembers_a_far_token():
     """A single value written hundreds of tokens ago, everything since orthogonal to it, read back at its decayed size."""
     L, H, d, e, T = _lib.mixer_lib(), 2, 16, 16, 900
