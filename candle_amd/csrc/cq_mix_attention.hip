@@ -294,7 +294,7 @@ __global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restri
         for (int n = 0; n < 4; n++) o[x][n] = zero;
     bool stale[RW];
 #pragma unroll
-    for (int a = 0; a < RW; a++) stale[a] = false;
+    for (int a = 0; a < RW; a++) stale[a] = true;          // (the first tile rescales, also for a query that sees nothing of it)
     float *const Sh = S + h * TT_HS;
     auto scores = [&](int it) {                            // of the wave's head, into S
         const uint8_t *const kt = kbuf + ((it - it0) & 1) * HALF + (h / R) * TT_TILE + lr * TT_ROW;

@@ -225,6 +225,18 @@ def test_talk_attention_tiles(H, G, e, window, keep, pos, rows):
     assert rel(attend(q, k, v, talk, scale, window, keep, pos, rows, 0.6), 0.6 * want) < 2e-5
 
 
+@pytest.mark.parametrize("H,G", [(16, 4), (16, 2), (8, 4), (8, 2), (8, 1)])
+def test_talk_attention_tiles_a_query_sees_nothing_of(H, G):
+    """Window 16: the last of 16 queries sees no key of the first of their two tiles.  Its result may not depend on what LDS held, here the NaN that infinite scores
+    leave as the rescaling of every query."""
+    T, d = 65, 128
+    huge = np.full((4112, H, d), 1e30, np.float32)
+    attend(huge, huge[:, :G], huge[:, :G], np.ones((H, H), np.float32), 1.0, 64, 0, 0, 4112)
+    q, k, v, talk = rnd(1, T, H, d), rnd(2, T, G, d), rnd(3, T, G, d), np.eye(H, dtype=np.float32) + rnd(4, H, H, scale=0.4)
+    want = vo.talking_attention(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), talk.astype(np.float64), 0.1, vo.window_mask(T, 16, 0))
+    assert rel(attend(q, k, v, talk, 0.1, 16, 0, 0, T), want) < 5e-6
+
+
 @pytest.mark.parametrize("window,keep,T", [(7, 0, 60), (32, 3, 150), (33, 32, 150), (64, 33, 300), (200, 1, 900)])
 def test_talk_attention_edges_stand_out(window, keep, T):
     """One key whose score and value stand out, just inside and just outside the window and the kept first tokens: head 0 returns its value
