@@ -231,27 +231,76 @@ __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__
 //   values   wave w: the weights of head w x V onto its outputs, then the scores of the next tile, which replace those weights when they are formed
 // so that only the mixing stands between two barriers.
 // LDS rows of 512 bytes in 32 16-byte chunks: keys' chunk c of row r at c ^ r, values as they are; both without bank conflicts.
-// 16 heads in us, above -> this: 2048 rows (window 1024) 327 -> 210, 500: 111 -> 53, 100: 65 -> 30; the error against 64 bits falls (2048 rows 4.9e-7 -> 4.0e-7: scores in two
+// 16 heads in us, above -> this: 2048 rows (window 1024) 327 -> 185, 500: 111 -> 43, 100: 65 -> 30; the error against 64 bits falls (2048 rows 4.9e-7 -> 4.0e-7: scores in two
 // sums).  Bound by the f32 matrix instructions, 68 of 32 cycles a wave and tile, four waves to a matrix core: 63 % of a unit's cycles, the rest barriers and
-// the mixing; and by the first rows, which see fewer keys than the last and leave a quarter of the units' time idle.
+// the mixing.
 typedef __attribute__((address_space(3))) void talk_lds;
+// The tiles of all blocks of 16 rows form one sequence, of which every workgroup takes `chunk`: the first rows see fewer keys than the last, and equal parts of each block left
+// a quarter of the units' time idle (2048 rows 210 -> 185 us, 6000 rows 730 -> 530, 8 heads and 2048 rows 132 -> 106).  A part costs 12 us beside its tiles of 5.5: the
+// queries and the first keys arrive, every tile at first brings new maxima, and its results go to the workspace.  So a block counts for `lead` tiles more than it has (with none
+// the workgroup that gets the six first blocks ended last, 256 us; with 1: 218, 2: 185, 3: 185, and 4096 rows 422, 371, 358), and where the chunks are of
+// few tiles (lead 0) none crosses into another block.
 constexpr int TT_RS = 20, TT_HS = 16 * TT_RS + 16, TT_ROW = 512, TT_TILE = 16 * TT_ROW;      // floats of a query's weights, of a head's; bytes of a key, of a tile
 __host__ __device__ constexpr int talk_tile_lds(int H, int R) { return 4 * (H / R) * TT_TILE + (H * TT_HS + 3 * 256) * 4; }
+
+// The tiles of keys that the 16 rows from r0 on see: those of the kept first tokens, then the window's from t_lo on.
+struct TalkTiles {
+    int t_lo, n_keep, n, last;
+};
+__host__ __device__ __forceinline__ TalkTiles talk_tiles_of(int r0, int rows, int pos, int window, int keep_first) {
+    TalkTiles t;
+    const int p0 = pos + r0, lo = p0 - window + 1, kt = (keep_first + 15) / 16;
+    t.last = pos + (r0 + 16 < rows ? r0 + 16 : rows) - 1;
+    t.t_lo = (lo > 0 ? lo : 0) / 16;
+    t.n_keep = kt < t.t_lo ? kt : t.t_lo;
+    t.n = t.n_keep + t.last / 16 - t.t_lo + 1;
+    return t;
+}
+// What a block of n tiles counts in the common sequence: `lead` more than it has, or for lead 0 whole chunks.
+__host__ __device__ __forceinline__ int talk_length(int n, int chunk, int lead) { return lead ? n + lead : (n + chunk - 1) / chunk * chunk; }
+__host__ __device__ constexpr int64_t talk_slot(int H) { return 16 * H * 130; }      // floats of a partial result: outputs [row][head][128], (m, l) [row][head]
 
 template <int H, int R, typename OT>
 __global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restrict__ q, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
                                                            const float *__restrict__ talk, float scale, int window, int keep_first, float out_scale, OT *__restrict__ out,
-                                                           int64_t out_stride, float *__restrict__ part, int pos, int rows, int vdim, int ctx) {
+                                                           int64_t out_stride, float *__restrict__ part, int2 *__restrict__ span, int chunk, int lead, int pos, int rows, int vdim,
+                                                           int ctx) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
     constexpr int G = H / R, RW = 16 / H, NI = 8 / R, HALF = G * TT_TILE;       // queries of a wave in the mixing; copies of a wave for a tile of keys
     extern __shared__ __attribute__((aligned(16))) uint8_t tt_smem[];
     uint8_t *const kbuf = tt_smem, *const vbuf = tt_smem + 2 * HALF;
     float *const S = reinterpret_cast<float *>(tt_smem + 4 * HALF), *const alpha = S + H * TT_HS, *const m_run = alpha + 256, *const l_run = m_run + 256;
     const int lane = threadIdx.x & 63, h = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lk = lane >> 4;
-    const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 16, nr = min(16, rows - r0), p0 = pos + r0, last = p0 + nr - 1;      // (the long ones first)
-    // tiles of the kept first tokens, then of the window; the share of this split
-    const int t_lo = max(0, p0 - window + 1) / 16, n_keep = min((keep_first + 15) / 16, t_lo), n_tiles = n_keep + last / 16 - t_lo + 1, nz = gridDim.z, z = blockIdx.z;
-    const int it0 = n_tiles * z / nz, it1 = n_tiles * (z + 1) / nz;
+    const int w = blockIdx.x, blocks = (rows + 15) / 16;
+    int b = blocks - 1 - w, first = 0, todo = 0;           // block of rows (whole ones: the long ones first), the tile of it to start with, tiles left
+    if (chunk) {
+        int before = 0;                                    // tiles of the blocks before b
+        for (int b0 = 0; b0 < blocks; b0 += 64) {
+            int sum = b0 + lane < blocks ? talk_length(talk_tiles_of(16 * (b0 + lane), rows, pos, window, keep_first).n, chunk, lead) : 0;
+#pragma unroll
+            for (int d = 1; d < 64; d *= 2) {
+                const int x = __shfl_up(sum, d);
+                if (lane >= d) sum += x;
+            }
+            const int skip = __popcll(__ballot(before + sum <= w * chunk));
+            b = b0 + skip;
+            if (skip < 64) {
+                if (skip) before += __shfl(sum, skip - 1);
+                break;
+            }
+            before += __shfl(sum, 63);
+        }
+        b = __builtin_amdgcn_readfirstlane(b);
+        first = __builtin_amdgcn_readfirstlane(w * chunk - before);
+        todo = chunk;
+    }
+    for (bool head = true; b < blocks; b++, first = 0, head = false) {
+    const int r0 = 16 * b, nr = min(16, rows - r0), p0 = pos + r0;
+    const TalkTiles tiles = talk_tiles_of(r0, rows, pos, window, keep_first);
+    const int t_lo = tiles.t_lo, n_keep = tiles.n_keep, last = tiles.last, it0 = max(first - lead, 0), it1 = chunk ? min(tiles.n, first - lead + todo) : tiles.n;
+    const bool whole = it0 == 0 && it1 == tiles.n;
+    todo -= it1 - (first - lead);
+    if (it1 <= 0) break;                                   // (nothing but the lead)
     auto first_key = [&](int it) { return 16 * (it < n_keep ? it : t_lo + it - n_keep); };
 
     const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void *)k_cache, 0, -1, 0x00020000);
@@ -273,7 +322,9 @@ __global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restri
     f32x4 qd[8];                                           // dims 16 c + 4 lk .. of query lr
     float tf[H / 4], m[RW][4], l[RW][4];                   // mixing weights [head lr][4 s + lk]; of head 4 lk + e and the wave's queries (l: of this lane's keys)
     {
-        const float *qr = q + ((int64_t)(r0 + min(lr, nr - 1)) * H + h) * 128 + 4 * lk;
+        int dim0 = 4 * lk;
+        asm("" : "+v"(dim0));
+        const float *qr = q + ((int64_t)(r0 + min(lr, nr - 1)) * H + h) * 128 + dim0;
 #pragma unroll
         for (int c = 0; c < 8; c++) qd[c] = *reinterpret_cast<const f32x4 *>(qr + 16 * c);
     }
@@ -294,7 +345,7 @@ __global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restri
         for (int n = 0; n < 4; n++) o[x][n] = zero;
     bool stale[RW];
 #pragma unroll
-    for (int a = 0; a < RW; a++) stale[a] = true;          // (the first tile rescales, also for a query that sees nothing of it)
+    for (int a = 0; a < RW; a++) stale[a] = true;                // (the first tile rescales, also for a query that sees nothing of it)
     float *const Sh = S + h * TT_HS;
     auto scores = [&](int it) {                            // of the wave's head, into S
         const uint8_t *const kt = kbuf + ((it - it0) & 1) * HALF + (h / R) * TT_TILE + lr * TT_ROW;
@@ -379,30 +430,69 @@ __global__ __launch_bounds__(64 * H) void talk_tile_kernel(const float *__restri
             m_run[(4 * lk + e) * 16 + RW * h + a] = m[a][e];
         }
     __syncthreads();
-    const f32x4 lh = *reinterpret_cast<const f32x4 *>(&l_run[h * 16 + 4 * lk]);
+    float *const slot = part + (2 * (int64_t)w + !head) * talk_slot(H);
+    int row0 = 4 * lk, col0 = 4 * lr;
+    asm("" : "+v"(row0), "+v"(col0));                    // (addresses made from these stay out of the loop's registers)
+    if (whole) {
+        const f32x4 lh = *reinterpret_cast<const f32x4 *>(&l_run[h * 16 + row0]);
 #pragma unroll
-    for (int x = 0; x < 2; x++)
+        for (int x = 0; x < 2; x++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int row = 4 * lk + e, col = 64 * x + 4 * lr;
-            if (row >= nr) continue;
+            for (int e = 0; e < 4; e++) {
+                const int row = row0 + e, col = 64 * x + col0;
+                if (row >= nr) continue;
 #pragma unroll
-            for (int n = 0; n < 4; n++) {
-                if (col + n >= vdim) continue;
-                if (nz == 1) out[(int64_t)(r0 + row) * out_stride + (int64_t)h * vdim + col + n] = (OT)(out_scale * o[x][n][e] / lh[e]);
-                else part[((int64_t)(z * rows + r0 + row) * H + h) * vdim + col + n] = o[x][n][e];
+                for (int n = 0; n < 4; n++)
+                    if (col + n < vdim) out[(int64_t)(r0 + row) * out_stride + (int64_t)h * vdim + col + n] = (OT)(out_scale * o[x][n][e] / lh[e]);
             }
-        }
-    if (nz > 1) {
-        float *ml = part + (int64_t)nz * rows * H * vdim;                 // [split][row][head] of (m, l)
-        for (int i = threadIdx.x; i < nr * H; i += 64 * H) {
+    } else {
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                *reinterpret_cast<f32x4 *>(&slot[((row0 + e) * H + h) * 128 + 64 * x + col0]) = f32x4{o[x][0][e], o[x][1][e], o[x][2][e], o[x][3][e]};
+        for (int i = threadIdx.x; i < 16 * H; i += 64 * H) {
             const int row = i / H, hh = i - row * H;
-            float *x = ml + 2 * ((int64_t)(z * rows + r0 + row) * H + hh);
-            x[0] = m_run[hh * 16 + row];
-            x[1] = l_run[hh * 16 + row];
+            slot[16 * H * 128 + 2 * i] = m_run[hh * 16 + row];
+            slot[16 * H * 128 + 2 * i + 1] = l_run[hh * 16 + row];
         }
     }
+    // the partial results of a block: the slot of its first part, the workgroup of its last; whole ones are done
+    if (chunk && threadIdx.x == 0) {
+        if (it0 == 0) span[b].x = whole ? -1 : 2 * w + !head;
+        if (it1 == tiles.n) span[b].y = w;
+    }
+    if (todo <= 0 || !lead) break;
+    }
 #endif
+}
+
+// The partial results of talk_tile_kernel; half a wave per (row, head).  2048 rows of 16 heads: 12.6 us, of which most is their memory.
+template <typename OT>
+__global__ __launch_bounds__(256) void talk_tile_combine_kernel(const float *__restrict__ part, const int2 *__restrict__ span, int H, int vdim, float out_scale,
+                                                                OT *__restrict__ out, int64_t out_stride) {
+    const int lane = threadIdx.x & 31, h = blockIdx.y * 8 + (threadIdx.x >> 5), r = blockIdx.x, i = (r & 15) * H + h;
+    const int2 sp = span[r >> 4];
+    if (sp.x < 0) return;
+    const int64_t step = talk_slot(H);
+    auto slot = [&](int z) { return part + (z ? 2 * ((sp.x >> 1) + z) : sp.x) * step; };      // the others are the first of their workgroups
+    auto stat = [&](int z) { return *reinterpret_cast<const float2 *>(slot(z) + 16 * H * 128 + 2 * i); };
+    const int nz = sp.y - (sp.x >> 1) + 1;
+    float m = -INFINITY, l = 0.0f;
+    for (int z = 0; z < nz; z++) m = fmaxf(m, stat(z).x);
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < nz; z++) {
+        const float2 ml = stat(z);
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(slot(z) + (int64_t)i * 128 + 4 * lane);
+        const float w = ml.x > -INFINITY ? __expf(ml.x - m) : 0.0f;
+        l = fmaf(w, ml.y, l);
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[e] = fmaf(w, v[e], a[e]);
+    }
+    OT *o = out + (int64_t)r * out_stride + (int64_t)h * vdim + 4 * lane;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (4 * lane + e < vdim) o[e] = (OT)(out_scale * a[e] / l);
 }
 
 // one wave per (row, head)
@@ -434,15 +524,34 @@ int talk_key_splits(int64_t rows, int64_t unit_blocks, int64_t max_keys) {
     n = n < tiles / 4 ? n : tiles / 4;
     return (int)(n < 1 ? 1 : (n > 16 ? 16 : n));
 }
-// The same for talk_tile_kernel, with at least two tiles of 16 keys each: 200 rows in one split 77.6 us, in six 37.1.  (More workgroups than units gain nothing: 2048
-// rows in two splits 210, in four 230.)
-int talk_tile_splits(int64_t rows, int64_t max_keys) {
-    int64_t n = 256 / ((rows + 15) / 16);
-    n = std::min(n, (max_keys + 15) / 32);
-    return (int)std::max<int64_t>(1, std::min<int64_t>(n, 16));
+constexpr int TALK_MAX_BLOCKS = 1024, TALK_LEAD = 3;
+// Tiles of keys of a workgroup of talk_tile_kernel when the workspace holds `slots` partial results; 0: one workgroup per 16 rows.  The balanced sequence pays from 8 tiles
+// a unit on (us balanced / whole chunks: 2048 rows 190 / 213, 1200: 90 / 96, 1000: 78 / 75, 700: 54 / 53); at most 17 parts a block, of two tiles and more; beyond TALK_MAX_BLOCKS
+// the order of the blocks balances as well (12000 rows 1054 us, one workgroup per block 1094).
+struct TalkPlan {
+    int chunk = 0, lead = 0, workgroups = 0;
+};
+TalkPlan talk_tile_plan(int64_t rows, int64_t window, int64_t keep_first, int64_t pos, int64_t slots) {
+    const int blocks = (int)((rows + 15) / 16);
+    TalkPlan plan{0, 0, blocks};
+    if (blocks > TALK_MAX_BLOCKS || slots < 2) return plan;
+    auto total = [&](int chunk, int lead) {
+        int64_t n = 0;
+        for (int b = 0; b < blocks; b++) n += talk_length(talk_tiles_of(16 * b, (int)rows, (int)pos, (int)window, (int)keep_first).n, chunk, lead);
+        return n;
+    };
+    int most = 0;
+    for (int b = 0; b < blocks; b++) most = std::max(most, talk_tiles_of(16 * b, (int)rows, (int)pos, (int)window, (int)keep_first).n);
+    const int64_t units = std::min<int64_t>(256, slots / 2), tiles = total(1, 0);
+    const int lead = tiles >= 8 * 256 ? TALK_LEAD : 0;
+    if (!lead && blocks > units) return plan;
+    int64_t chunk = std::max<int64_t>({(tiles + (int64_t)lead * blocks + units - 1) / units, 2, (most + 15) / 16});
+    while (!lead && total((int)chunk, 0) > units * chunk) chunk++;
+    if (chunk + lead < (int64_t)((blocks + 255) / 256) * (most + lead)) plan = {(int)chunk, lead, (int)((total((int)chunk, lead) + chunk - 1) / chunk)};
+    return plan;
 }
 // Which calls talk_tile_kernel takes: what it has instances for, LDS for up to four kv heads, offsets of 32 bits into the caches.  It is the faster one at all sizes
-// (16 heads: 20 rows 22.8 -> 21.0 us, 100: 65 -> 31, 500: 111 -> 54, 2048: 327 -> 210; 8 heads, 2048 rows 196 -> 132).
+// (16 heads: 20 rows 22.8 -> 20.7 us, 100: 65 -> 30, 500: 111 -> 43, 2048: 327 -> 185; 8 heads, 2048 rows 196 -> 106).
 bool talk_by_tiles(int64_t H, int64_t G, int64_t dim_pad, int64_t vdim_pad, int64_t ctx) {
     const int64_t R = H / G;
     return dim_pad == 128 && vdim_pad == 128 && (H == 8 || H == 16) && (R == 4 || R == 8 || (R == 2 && H == 8)) && G * ctx < (1LL << 23);
@@ -473,15 +582,15 @@ int talk_launch(const float *q, const float *kc, const float *vc, const float *t
 
 template <int H, int R, typename OT>
 int talk_tile_launch(const float *q, const float *kc, const float *vc, const float *talk, float scale, int window, int keep, float out_scale, OT *out, int64_t out_stride,
-                     float *part, int nz, int pos, int rows, int vdim, int ctx, hipStream_t s) {
+                     float *part, const TalkPlan &plan, int pos, int rows, int vdim, int ctx, hipStream_t s) {
     constexpr int lds = talk_tile_lds(H, R);
+    int2 *const span = reinterpret_cast<int2 *>(part + 2 * plan.workgroups * talk_slot(H));
     const int e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(talk_tile_kernel<H, R, OT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e) return e;
-    hipLaunchKernelGGL((talk_tile_kernel<H, R, OT>), dim3((rows + 15) / 16, 1, nz), dim3(64 * H), lds, s, q, kc, vc, talk, scale, window, keep, out_scale, out, out_stride, part,
-                       pos, rows, vdim, ctx);
-    if (nz > 1)
-        hipLaunchKernelGGL(talk_combine_kernel<OT>, dim3((unsigned)rows, (unsigned)((H + 3) / 4)), dim3(256), 0, s, (const float *)part, nz, (int64_t)rows, H, vdim, out_scale,
-                           out, out_stride);
+    hipLaunchKernelGGL((talk_tile_kernel<H, R, OT>), dim3(plan.workgroups), dim3(64 * H), lds, s, q, kc, vc, talk, scale, window, keep, out_scale, out, out_stride, part, span,
+                       plan.chunk, plan.lead, pos, rows, vdim, ctx);
+    if (plan.chunk)
+        hipLaunchKernelGGL(talk_tile_combine_kernel<OT>, dim3((unsigned)rows, H / 8), dim3(256), 0, s, (const float *)part, (const int2 *)span, H, vdim, out_scale, out, out_stride);
     return (int)hipGetLastError();
 }
 
@@ -719,11 +828,17 @@ int talk_decode_launch(const float *row, const cq_mix_heads *g, float eps, const
 }
 
 int64_t talk_split_bytes(int64_t rows, int64_t H, int64_t vdim) { return rows * H * (vdim + 2) * 4; }
+int64_t talk_plan_bytes(const TalkPlan &plan, int64_t rows, int H) { return 2 * plan.workgroups * talk_slot(H) * 4 + (rows + 15) / 16 * 8; }
 int64_t talk_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos) {
     if (rows <= 0 || n_head <= 0 || vdim <= 0 || window < 1 || keep_first < 0 || pos < 0) return 0;
     const int64_t max_keys = talk_max_keys(window, keep_first, pos + rows), vp = (vdim + 15) / 16 * 16;
-    const int nz = std::max(talk_key_splits(rows, talk_unit_blocks(n_head, vp), max_keys), vp == 128 && (n_head == 8 || n_head == 16) ? talk_tile_splits(rows, max_keys) : 1);
-    return nz > 1 ? talk_split_bytes(rows, n_head, vdim) * nz : 0;
+    const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vp), max_keys);
+    int64_t bytes = nz > 1 ? talk_split_bytes(rows, n_head, vdim) * nz : 0;
+    if (vp == 128 && (n_head == 8 || n_head == 16) && pos + rows <= 0x7fffffff) {
+        const TalkPlan plan = talk_tile_plan(rows, std::min<int64_t>(window, 0x7fffffff), std::min<int64_t>(keep_first, 0x7ffffff0), pos, 512);
+        if (plan.chunk) bytes = std::max(bytes, talk_plan_bytes(plan, rows, (int)n_head));
+    }
+    return bytes;
 }
 
 template <typename OT>
@@ -743,17 +858,18 @@ int talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_
     const bool by_tiles = talk_by_tiles(n_head, n_kv_head, dim_pad, vdim_pad, ctx);
     const int64_t max_keys = talk_max_keys(window, keep_first, pos + rows);
     const int64_t split_bytes = talk_split_bytes(rows, n_head, vdim);
-    int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vdim_pad), max_keys);
+    const int nz = talk_key_splits(rows, talk_unit_blocks(n_head, vdim_pad), max_keys);
     if (nz > 1 && (!workspace_dev || workspace_bytes < nz * split_bytes)) return CQ_ERR_WORKSPACE;
-    if (by_tiles)                                          // (as many of its splits as the workspace holds)
-        nz = (int)std::max<int64_t>(1, std::min<int64_t>(talk_tile_splits(rows, max_keys), workspace_dev ? workspace_bytes / split_bytes : 1));
+    TalkPlan plan;
+    if (by_tiles)                                          // (as many partial results as the workspace holds)
+        plan = talk_tile_plan(rows, w, keep, pos, workspace_dev && !mix_misaligned(workspace_dev, 16) ? std::max<int64_t>(0, workspace_bytes - (rows + 15) / 16 * 8) / (talk_slot(H) * 4) : 0);
     hipStream_t s = (hipStream_t)stream;
 #define CQ_TA(NW_, NHW_, SH_, U_, VS_, KT_)                                                                                                            \
     talk_launch<NW_, NHW_, SH_, U_, VS_, KT_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride,      \
                                               (float *)workspace_dev, nz, (int)pos, (int)rows, H, G, (int)dim_pad, (int)vdim, (int)vdim_pad, (int)ctx, s)
     if (by_tiles) {
 #define CQ_TT(H_, R_)                                                                                                                                  \
-    talk_tile_launch<H_, R_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride, (float *)workspace_dev, nz, (int)pos, (int)rows, \
+    talk_tile_launch<H_, R_>(q_dev, k_cache_dev, v_cache_dev, talk_dev, scale, w, keep, out_scale, out_dev, out_stride, (float *)workspace_dev, plan, (int)pos, (int)rows, \
                              (int)vdim, (int)ctx, s)
         if (H == 16 && R == 4) return CQ_TT(16, 4);
         if (H == 16 && R == 8) return CQ_TT(16, 8);

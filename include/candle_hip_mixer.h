@@ -120,8 +120,8 @@ int cq_mix_head_norm_gate_bf16(const float *o_dev, int64_t o_stride, const float
  * score_h = sum_g talk[h, g] * scale * (q_g . k_g), key j visible to position i when j <= i and (i - j < window or j < keep_first), softmax
  * over the visible keys, out[r, h * vdim + e] = out_scale * sum_j p_h(j) v(j).  Query head h uses kv head h / (n_head / n_kv_head).
  * q [rows, n_head, dim_pad], caches [n_kv_head, ctx, dim_pad] and [n_kv_head, ctx, vdim_pad]; dim_pad and vdim_pad are multiples of 16
- * (padding zero; vdim_pad the least one), at most CQ_MIX_MAX_DIM; n_head <= CQ_MIX_MAX_HEADS.  Calls with few rows split the keys over workgroups and merge
- * through the workspace (0 bytes when not split). */
+ * (padding zero; vdim_pad the least one), at most CQ_MIX_MAX_DIM; n_head <= CQ_MIX_MAX_HEADS.  Calls that do not fill the chip evenly split the keys
+ * over workgroups and merge through the workspace (0 bytes when not split). */
 #define CQ_MIX_MAX_HEADS 64
 int64_t cq_mix_talk_attention_workspace_bytes(int64_t rows, int64_t n_head, int64_t vdim, int64_t window, int64_t keep_first, int64_t pos);
 int cq_mix_talk_attention(const float *q_dev, const float *k_cache_dev, const float *v_cache_dev, const float *talk_dev, float scale, int64_t window,

@@ -181,8 +181,8 @@ def test_pack_heads(dim, rot):
 
 
 # ---------------------------------------------------------------------------------------------- attention
-def attend(q, k, v, talk, scale, window, keep, pos, rows, out_scale=1.0):
-    """cq_mix_talk_attention for the last `rows` of len(k) positions."""
+def attend(q, k, v, talk, scale, window, keep, pos, rows, out_scale=1.0, have=None, offset=0):
+    """cq_mix_talk_attention for the last `rows` of len(k) positions; `have` bytes of workspace, `offset` floats behind an aligned address."""
     L = _lib.mixer_lib()
     T, G, d = k.shape
     H, e = q.shape[1], v.shape[2]
@@ -191,8 +191,8 @@ def attend(q, k, v, talk, scale, window, keep, pos, rows, out_scale=1.0):
     kc[:, :T, :d], vc_[:, :T, :e], qd[..., :d] = up(k.transpose(1, 0, 2)), up(v.transpose(1, 0, 2)), up(q[pos:pos + rows])
     kc[:, T:], vc_[:, T:] = float("nan"), float("nan")          # positions that do not exist yet
     out = torch.zeros((rows, H * e + 5), device=DEV)
-    need = L.cq_mix_talk_attention_workspace_bytes(rows, H, e, window, keep, pos)
-    ws = torch.full((max(need, 4) // 4,), float("nan"), device=DEV)
+    need = L.cq_mix_talk_attention_workspace_bytes(rows, H, e, window, keep, pos) if have is None else have
+    ws = torch.full((max(need, 4) // 4 + offset,), float("nan"), device=DEV)[offset:]
     _lib.check("a", L.cq_mix_talk_attention(qd.data_ptr(), kc.data_ptr(), vc_.data_ptr(), ptr(talk), scale, window, keep, out_scale, out.data_ptr(), H * e + 5, pos,
                                             rows, H, G, dp, e, ep, ctx, ws.data_ptr(), need, sp()))
     assert not out[:, H * e:].any()
@@ -235,6 +235,29 @@ def test_talk_attention_tiles_a_query_sees_nothing_of(H, G):
     q, k, v, talk = rnd(1, T, H, d), rnd(2, T, G, d), rnd(3, T, G, d), np.eye(H, dtype=np.float32) + rnd(4, H, H, scale=0.4)
     want = vo.talking_attention(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), talk.astype(np.float64), 0.1, vo.window_mask(T, 16, 0))
     assert rel(attend(q, k, v, talk, 0.1, 16, 0, 0, T), want) < 5e-6
+
+
+@pytest.mark.parametrize("H,G,window,keep,pos,rows", [(16, 4, 5000, 0, 0, 1100), (8, 2, 300, 40, 900, 1137), (16, 2, 700, 4, 0, 1300), (8, 4, 90, 7, 33, 500), (16, 4, 5000, 0, 3000, 20),
+                                                      (8, 1, 100, 0, 0, 4250)])
+def test_talk_attention_tiles_in_chunks(H, G, window, keep, pos, rows):
+    """The tiles of all rows in one sequence: parts that cross from one block of rows into the next or not, more blocks than units, and less workspace than asked for:
+    half, what the least call needs, and one that is not aligned for the partial results."""
+    T, d, e, L = pos + rows, 128, 120, _lib.mixer_lib()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(rows)
+    q, k, v = (torch.randn((T, n, w), generator=g, device=DEV, dtype=torch.float32).cpu().numpy() for n, w in ((H, d), (G, d), (G, e)))
+    talk, scale = np.eye(H, dtype=np.float32) + rnd(4, H, H, scale=0.3), 1.5 * d ** -0.5
+    i, j = torch.arange(pos, T, device=DEV)[:, None], torch.arange(T, device=DEV)[None]
+    hidden = (j > i) | ((i - j >= window) & (j >= keep))
+    qt, kt, vt = (up(a).double().transpose(0, 1) for a in (q[pos:], k, v))
+    score = torch.stack([qt[h] @ kt[h * G // H].T for h in range(H)]) * scale
+    score = (up(talk).double() @ score.flatten(1)).reshape(score.shape).masked_fill_(hidden, float("-inf"))
+    want = torch.stack([torch.softmax(score[h], -1) @ vt[h * G // H] for h in range(H)]).transpose(0, 1).cpu().numpy()
+    need = L.cq_mix_talk_attention_workspace_bytes(rows, H, e, window, keep, pos)
+    tile = rows * H * (e + 2) * 4                       # of one split of the keys, in the kernel that takes any shape
+    least = min(need, tile * max(1, min(256 // ((rows + 15) // 16), min(T, window + keep + 16) // 128, 16)))
+    for have, offset in ((need, 0), (max(least, need // 2), 0), (least, 0), (need, 1)):
+        assert rel(attend(q, k, v, talk, scale, window, keep, pos, rows, have=have, offset=offset), want) < 1e-5, (have, offset)
 
 
 @pytest.mark.parametrize("window,keep,T", [(7, 0, 60), (32, 3, 150), (33, 32, 150), (64, 33, 300), (200, 1, 900)])
