@@ -401,21 +401,24 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
 // ---- bf16 tiles of BM activation rows x 128 weight rows, bfloat16 activations, one workgroup on a unit --------------------------------------
 // The 128 x 128 tile above, two workgroups to a unit, wants 512 of them: products of a few hundred tiles are cut along k instead, write their sums to memory and have
 // another launch add them, and each workgroup waits for stages that it has asked for one or three of its own short steps ago.  Here one workgroup has a unit's LDS.
-// 2048 x 2048 x 2048, cold weights: 39.2 -> 25.5 us (674 TFLOP/s), and the sums are nearer to 64 bits (1.86e-7 -> 1.31e-7).  Bound by LDS: a stage writes 32 KB and
-// reads 64, 768 cycles beside 512 of products (192 rows: 960 beside 768); of the 25 us about 6 are the way to the first products and the last sums.
-// Eight waves: two halves of a stage's 64 of k, each 2 x 2 waves of BM / 2 x 64 results, so that every result has two sums (four with CH = 2) that meet at the end.
-// LDS holds four stages; copies that no register sees bring them, four ahead of the products, and a stage's operands are read while those of the stage before are
-// multiplied: one barrier a stage, which waits for nothing that was asked for less than three stages ago.  Rows in LDS as above.
-template <int BM, int CH>
-__global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n) {
+// Results are those of that tile to the last bit, so that no choice made from them (of a token's experts, say) depends on which of the two a call takes: the same
+// instructions in the order of k, and for a product that would be cut along k (PARTS) one sum per part of k_split, added in order.
+// 2048 x 2048 x 2048, cold weights: 39.5 -> 27.2 us, of which about 7 are the way to the first products and the last sums.  A stage takes 0.62 us, 1490 cycles, of which
+// LDS has work for 1024 (32 KB written, 96 read) and the matrix cores for 512 (192 rows: 1216 and 768); 256 units then take 13.5 TB/s out of the L2s.
+// Eight waves, 4 x 2, of BM / 4 x 64 results each: four of BM / 2 x 64 read a third less from LDS, but have a matrix core to themselves and wait more (2048 x 2048 x 2048:
+// 31.0 us; 192 rows: 52 where eight take 33).  LDS holds four stages of 64 of k; copies that no register sees bring them, four ahead of the products, and the operands of
+// half a stage are read while those of the half before are multiplied: one barrier a stage, which waits for nothing that was asked for less than three stages ago.  Rows
+// in LDS as above.
+template <int BM, bool PARTS>
+__global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n, int k_split) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
-    constexpr int STAGE = (BM + 128) * 128, TM = BM / 32, TN = 4, NX = BM / 64, NW = 2;      // 16-row blocks of a wave; copies of a wave and stage
+    constexpr int STAGE = (BM + 128) * 128, TM = BM / 64, TN = 4, NX = BM / 64, NW = 2;      // 16-row blocks of a wave; copies of a wave and stage
     extern __shared__ __align__(16) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2, wv = wave & 3, lr = lane & 15, lk = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lk = lane >> 4;
     int tm, tn;
     tile_at(xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
     const int64_t m0 = (int64_t)tm * BM;
-    const int n0 = tn * 128, nst = K >> 6, wm = (wv >> 1) * (BM / 2), wn = (wv & 1) * 64;
+    const int n0 = tn * 128, nst = K >> 6, part = k_split >> 6, wm = (wv >> 1) * (BM / 4), wn = (wv & 1) * 64;
 
     // ---- copy i of a wave brings eight rows of a stage, one 16-byte chunk a lane; rows past the end repeat the last ----
     const uint8_t *const xbase = reinterpret_cast<const uint8_t *>(src.x) + m0 * src.ldx * 2;
@@ -424,16 +427,16 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
     uint32_t x_off[NX], w_off[NW];
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-        const int row = 8 * (wave + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        const int row = 8 * (wv + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
         x_off[i] = (uint32_t)min((int64_t)row, M - 1 - m0) * (uint32_t)(2 * src.ldx) + 16 * c;
     }
 #pragma unroll
     for (int i = 0; i < NW; i++) {
-        const int row = 8 * (wave + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        const int row = 8 * (wv + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
         w_off[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)(2 * src.ldw) + 16 * c;
     }
     auto copy = [&](int st) {                              // (past the last stage: that one again, into a place nobody reads)
-        uint8_t *const to = lds + (st & 3) * STAGE + 1024 * wave;
+        uint8_t *const to = lds + (st & 3) * STAGE + 1024 * wv;
         const int at = 128 * min(st, nst - 1);
 #pragma unroll
         for (int i = 0; i < NW; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (dt_lds *)(to + BM * 128 + 8192 * i), 16, w_off[i], at, 0, 0);
@@ -441,29 +444,27 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
         for (int i = 0; i < NX; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (dt_lds *)(to + 8192 * i), 16, x_off[i], at, 0, 0);
         asm volatile("" ::: "memory");
     };
-    f32x4 acc[CH][TM][TN];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[TM][TN], sum[TM][TN];                        // sum: of the parts before
 #pragma unroll
-    for (int c = 0; c < CH; c++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TN; j++) acc[i][j] = zero;
     bf16x8 fa[2][TM], fb[2][TN];
-    const uint32_t sw = 16 * ((4 * half + lk) ^ ((lr >> 1) & 7)), a_at = (wm + lr) * 128 + sw, b_at = (BM + wn + lr) * 128 + sw;
-    auto operands = [&](int st, auto set) {
-        const uint8_t *const from = lds + (st & 3) * STAGE;
+    const uint32_t sw = (lr >> 1) & 7, a_at = (wm + lr) * 128, b_at = (BM + wn + lr) * 128;
+    auto operands = [&](int st, auto half) {
+        const uint8_t *const from = lds + (st & 3) * STAGE + 16 * ((4 * half + lk) ^ sw);
 #pragma unroll
-        for (int j = 0; j < TN; j++) fb[set][j] = *reinterpret_cast<const bf16x8 *>(from + b_at + 2048 * j);
+        for (int j = 0; j < TN; j++) fb[half][j] = *reinterpret_cast<const bf16x8 *>(from + b_at + 2048 * j);
 #pragma unroll
-        for (int i = 0; i < TM; i++) fa[set][i] = *reinterpret_cast<const bf16x8 *>(from + a_at + 2048 * i);
+        for (int i = 0; i < TM; i++) fa[half][i] = *reinterpret_cast<const bf16x8 *>(from + a_at + 2048 * i);
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto multiply = [&](auto set) {
+    auto multiply = [&](auto half) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                acc[set % CH][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[set][j], fa[set][i], acc[set % CH][i][j], 0, 0, 0);
+            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[half][j], fa[half][i], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     constexpr int PER = NX + NW;
@@ -472,61 +473,59 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
     copy(2);
     copy(3);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * PER) : "memory");
-    constexpr std::integral_constant<int, 0> even{};
-    constexpr std::integral_constant<int, 1> odd{};
-    operands(0, even);
-    auto step = [&](int st, auto set, auto next) {
+    constexpr std::integral_constant<int, 0> low{};
+    constexpr std::integral_constant<int, 1> high{};
+    operands(0, low);
+    int left = part;                                       // stages to the end of the part
+    bool first = true;
+    for (int st = 0; st < nst; st++) {
+        operands(st, high);
+        multiply(low);
         // stage st + 1 is there for everybody, and everybody has the operands of stage st: stage st + 4 may take its place
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * PER) : "memory");
         copy(st + 4);
-        operands(st + 1, next);
-        multiply(set);
-    };
-    for (int st = 0; st < nst; st += 2) {
-        step(st, even, odd);
-        if (st + 1 < nst) step(st + 1, odd, even);
+        operands(st + 1, low);
+        multiply(high);
+        if (PARTS && --left == 0 && st + 1 < nst) {
+            left = part;
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    sum[i][j] = first ? acc[i][j] : sum[i][j] + acc[i][j];
+                    acc[i][j] = zero;
+                }
+            first = false;
+        }
     }
-    // ---- the halves' sums meet: each half of the waves ends with one half of the row blocks (no copy may be on its way) ----
-    if (CH == 2)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (copies may not outlive the workgroup)
+    if (PARTS)
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) acc[0][i][j] += acc[CH - 1][i][j];
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    f32x4 *const meet = reinterpret_cast<f32x4 *>(lds) + 64 * (TM / 2) * TN * wv + lane;
-    constexpr int FAR = 64 * (TM / 2) * TN * 4;
-    auto finish = [&](auto h) {
-        constexpr int lo = h * (TM / 2), other = (1 - h) * (TM / 2);
-        // what the sums are added to is asked for here, all at once (as each is stored, a load would have to wait for the store before it: 41 us for the 28 of
-        // 2048 x 2048 x 2048 onto a residual stream)
-        f32x4 old[TM / 2][TN];
-        Out o = out;
-        o.accumulate = 0;
+            for (int j = 0; j < TN; j++) acc[i][j] = sum[i][j] + acc[i][j];
+    // what the sums are added to is asked for here, all at once (as each is stored, a load would have to wait for the store before it, and the
+    // product would take half as long again)
+    f32x4 old[TM][TN];
+    Out o = out;
+    o.accumulate = 0;
+    if (out.accumulate)
 #pragma unroll
-        for (int i = 0; i < TM / 2; i++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                old[i][j] = out.accumulate ? present4(out, m0 + wm + 16 * (lo + i) + lr, n0 + wn + 16 * j + 4 * lk, M, N) : f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < TN; j++) old[i][j] = present4(out, m0 + wm + 16 * i + lr, n0 + wn + 16 * j + 4 * lk, M, N);
 #pragma unroll
-        for (int i = 0; i < TM / 2; i++)
+    for (int i = 0; i < TM; i++) {
+        const int64_t m = m0 + wm + 16 * i + lr;
+        if (m >= M) continue;
 #pragma unroll
-            for (int j = 0; j < TN; j++) meet[h * FAR + 64 * (i * TN + j)] = acc[0][other + i][j];
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-        for (int i = 0; i < TM / 2; i++) {
-            const int64_t m = m0 + wm + 16 * (lo + i) + lr;
-            if (m >= M) continue;
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int n = n0 + wn + 16 * j + 4 * lk;
-                f32x4 v = acc[0][lo + i][j] + meet[(1 - h) * FAR + 64 * (i * TN + j)];
-                if (out.accumulate) v += old[i][j];
-                if (n < N) emit4(o, v, m, n, M, N, 0);
-            }
+        for (int j = 0; j < TN; j++) {
+            const int n = n0 + wn + 16 * j + 4 * lk;
+            f32x4 v = acc[i][j];
+            if (out.accumulate) v += old[i][j];
+            if (n < N) emit4(o, v, m, n, M, N, 0);
         }
-    };
-    if (half) finish(odd);
-    else finish(even);
+    }
 #endif
 }
 
@@ -678,19 +677,21 @@ bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
     return rounds == 1 ? t >= 160 : 4 * t >= 3 * 256 * rounds;
 }
 
-// Where one workgroup to a unit with a ring of stages (128 or 192 rows; 0: neither) takes the place of two workgroups of 128 x 128 (products of bfloat16 rows).  One round
-// of 256 tiles takes 20 - 25 us at k = 2048 with 128 rows and 25 - 30 with 192; 512 tiles two to a unit take 46, and fewer tiles 37 - 50 in splits of k and their sum.
-//   up to 256 tiles of 128 (2048 x 2048 x 2048: 39.2 -> 25.5 us, 1500 x 2048 x 7168: 81.7 -> 62.3), unless more than four splits give shorter sums than the ring's four
-//     per result, or many splits of a long k more workgroups (1000 x 2048 x 7168 in four splits: 49.6 against 62.4);
-//   one round of 192 where 128 takes two (1500 x 3500 x 2048: 49.8 -> 29.6), else two rounds of 128 up to 384 tiles (1000 x 5632 x 2048: 53.1 -> 46.4; 448: 46.6 against 48.0);
-//   beyond one round of two to a unit, rounds of 192 that are two thirds full (1200 x 7168 x 2048: 63.9 -> 56.3, 2048 x 10368 x 2048: 119 -> 111; the 256 x 256 tile first).
+// Where one workgroup to a unit with a ring of stages (128 or 192 rows; 0: neither) takes the place of two workgroups of 128 x 128 (products of bfloat16 rows; the large
+// tile first where it would take the call).  At k = 2048, cold weights, one round of 256 tiles takes 23 - 27 us with 128 rows and 32 - 34 with 192; 512 tiles two to a
+// unit take 49 - 53, and fewer tiles 26 - 54 in parts of k and their sum.
+//   up to 256 tiles of 128 in up to three parts (2048 x 2048 x 2048: 39.5 -> 27.2 us, 1500 x 2048 x 7168: 86.5 -> 69.3), or four of a short k (1200 x 2048 x 2048: 37.4 ->
+//     24.5, 1000 x 2048 x 7168: 54.1 against 66.3); more parts bring more workgroups to a long k (700 x 2048 x 7168: 53.2 against 60.4);
+//   one round of 192 where 128 takes two (1500 x 3500 x 2048: 53.5 -> 34.2), else two rounds of 128 up to 384 tiles (1000 x 5632 x 2048: 57.2 -> 49.1; 448: 51.1 against 51.3);
+//   beyond one round of two to a unit, rounds of 192 that are two thirds full (1200 x 7168 x 2048: 68.4 -> 63.8, 2048 x 10368 x 2048: 130.5 -> 122.9).
 int ring_rows(const Plan &p, int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
     if (p.bm != 128 || ldw > (1 << 20) || ldx > (1 << 20)) return 0;       // (its offsets have 32 bits)
     const int64_t t128 = (int64_t)p.tiles_m * p.tiles_n, t192 = (m + 191) / 192 * p.tiles_n, rounds = (t192 + 255) / 256;
+    if (p.splits == 1 && large_tile(m, n, k, ldw, ldx)) return 0;
     if (t128 <= 256) return p.splits <= 3 || (p.splits == 4 && k <= 3072) ? 128 : 0;
     if (t192 <= 256) return 192;
     if (t128 <= 384) return 128;
-    return t128 > 512 && 3 * t192 >= 2 * 256 * rounds && !large_tile(m, n, k, ldw, ldx) ? 192 : 0;
+    return t128 > 512 && 3 * t192 >= 2 * 256 * rounds ? 192 : 0;
 }
 
 // ---- one row --------------------------------------------------------------------------------------------------------------
@@ -872,12 +873,13 @@ int cq_dense_product(int precision, const cq_dense_args *args, void *workspace_d
     const int ring = a.x_bf16 && a.batch == 1 && !a.tiles_dev && !a.src_rows_dev ? ring_rows(p, m, n, k, a.ldw, a.ldx) : 0;
     if (ring) {
         o.planes = nullptr;
-        auto *const fn = ring == 192 ? dense_ring_kernel<192, 1> : dense_ring_kernel<128, 2>;
+        auto *const fn = ring == 192 ? (p.splits > 1 ? dense_ring_kernel<192, true> : dense_ring_kernel<192, false>)
+                                     : (p.splits > 1 ? dense_ring_kernel<128, true> : dense_ring_kernel<128, false>);
         const int lds = 4 * (ring + 128) * 128;
         const hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return (int)e;
         const int tm = (int)((m + ring - 1) / ring), tn = (int)((n + 127) / 128);
-        hipLaunchKernelGGL(fn, dim3((unsigned)(tm * tn)), dim3(512), lds, s, src, o, m, (int)n, (int)k, tm, tn);
+        hipLaunchKernelGGL(fn, dim3((unsigned)(tm * tn)), dim3(512), lds, s, src, o, m, (int)n, (int)k, tm, tn, p.k_split);
         return (int)hipGetLastError();
     }
     if (precision == CQ_DENSE_F32) CQ_DM(dense_f32_kernel);

@@ -117,3 +117,22 @@ def test_ring_of_stages(m, n, k, pad, form):
     assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * (4 if form == "swiglu" else 1)
     assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, cols:] == 5).all()
 
+
+@pytest.mark.parametrize("m,n,k", [(2000, 2048, 1536), (1100, 2500, 1024), (1000, 1800, 2112), (1500, 2048, 7168), (1290, 4485, 1024), (1537, 2700, 4160), (1000, 5602, 1024),
+                                   (1535, 4481, 512), (1500, 5633, 1088), (1200, 7168, 2048), (100, 49100, 1024)])
+def test_ring_of_stages_keeps_bits(m, n, k):
+    """Bit for bit what the same rows in f32 give, which go through the 128 x 128 tile (or the large one): a choice made from a product, like that of a token's
+    experts, may not depend on the kernel.  One part of k, two to four, even and uneven; 128 rows and 192; a few rows of very many columns, where the large tile stays."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = torch.randn((n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k), generator=g, device="cuda").bfloat16()
+    L = _lib.mixer_lib()
+    nb = L.cq_dense_matmul_workspace_bytes(0, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    got = []
+    for rows in (x, x.float()):
+        y = torch.randn((m, n), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+        a = DenseArgs(w_dev=w.data_ptr(), ldw=k, x_dev=rows.data_ptr(), ldx=k, x_bf16=int(rows is x), dst_dev=y.data_ptr(), ldd=n, m=m, n=n, k=k, batch=1, accumulate=1)
+        _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got.append(y)
+    assert torch.equal(*got)
