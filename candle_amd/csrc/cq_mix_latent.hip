@@ -98,25 +98,18 @@ struct Expanded {
     int pos, rows, heads;
 };
 
-// SETS = 2: eight waves, of which four take the even tiles and four the odd ones, and meet at the end.  A workgroup of the last rows sees all keys and is the longest
-// chain of a launch that has all its workgroups on the chip at once: half as long so (16 heads: 1500 rows 43.8 -> 33.4 us, 500:
-// 17.2 -> 14.5, 100 behind 1500 keys 41.5 -> 32.7).
-template <typename T, int DK, int DV, int NQ, int SETS = 1>
-__global__ __launch_bounds__(256 * SETS) void latent_expanded_kernel(Expanded p) {
+template <typename T, int DK, int DV, int NQ>
+__global__ __launch_bounds__(256) void latent_expanded_kernel(Expanded p) {
     constexpr int CH = Chunk<T>::N, KT = Chunk<T>::KEYS, NT = KT / 16, NKF = DK / Chunk<T>::STEP, KC = DK / CH, NVF = DV / 16, BM = 64 * NQ;
     constexpr int KL = KT * KC / 256, VT = (KT / 4) * (DV / CH), VL = (VT + 255) / 256;
-    constexpr int TILE = KT * KC + DV * 8;                 // keys, then values
-    __shared__ u32x4 lds[SETS * TILE];
-    static_assert(SETS == 1 || (NQ == 1 && SETS * TILE >= 256 * (NVF + 1)), "room for the second set's outputs");
-    const int set = SETS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-    u32x4 *const ks = lds + set * TILE, *const vs = ks + KT * KC;
-    const int tid = threadIdx.x & 255, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lk = lane >> 4;
+    __shared__ u32x4 ks[KT * KC], vs[DV * 8];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lk = lane >> 4;
     // The longest rows first; where two workgroups per CU hold them all, the shortest join the longest.  With heads in eighths a head stays on one XCD, whose L2
     // then holds its keys and values.
     const int blocks = (p.rows + BM - 1) / BM, per = p.heads >> 3, total = blocks * p.heads;
     const bool split = (p.heads & 7) == 0;
     const int n = split ? total >> 3 : total, half = (n + 1) / 2, turn = split ? blockIdx.x >> 3 : blockIdx.x;
-    const int rank = SETS == 1 && NQ == 1 && total <= 512 && turn >= half ? n - 1 - (turn - half) : turn, heads = split ? per : p.heads;
+    const int rank = NQ == 1 && total <= 512 && turn >= half ? n - 1 - (turn - half) : turn, heads = split ? per : p.heads;
     const int h = (split ? (blockIdx.x & 7) * per : 0) + rank % heads, block = blocks - 1 - rank / heads;
     const int m0 = block * BM, mw = m0 + wv * 16 * NQ;
     const int last = p.pos + min(m0 + BM, p.rows) - 1, n_tiles = last / KT + 1, dk = p.d1 + p.d2;
@@ -184,14 +177,14 @@ __global__ __launch_bounds__(256 * SETS) void latent_expanded_kernel(Expanded p)
     // LDS slots of a lane: key chunks 4 k + lk of row lr by parity of k, value chunks 4 sp + lk of column lr by (n & 3) ^ 2 sp
     const int ka[2] = {lr * KC + (lk ^ (lr & 7)), lr * KC + ((4 + lk) ^ (lr & 7))}, vx = lk ^ (lr & 7) ^ (lr >> 3);
     const int va[4] = {lr * 8 + vx, lr * 8 + (vx ^ 2), lr * 8 + (vx ^ 4), lr * 8 + (vx ^ 6)};
-    fetch(set * KT);
-    for (int it = set; it < n_tiles + set; it += SETS) {   // (the second set's last one may lie behind the last tile: read as the last key, used by nobody)
+    fetch(0);
+    for (int it = 0; it < n_tiles; it++) {
         const int j0 = it * KT;
         __syncthreads();
         stage();
         __syncthreads();
-        if (it + SETS < n_tiles + set) fetch(j0 + SETS * KT);
-        if (j0 > p.pos + mw + 16 * NQ - 1 || (SETS > 1 && j0 > last)) continue;       // wave-uniform: nothing visible to this wave's rows
+        if (it + 1 < n_tiles) fetch(j0 + KT);
+        if (j0 > p.pos + mw + 16 * NQ - 1) continue;       // wave-uniform: nothing visible to this wave's rows
         f32x4 s[NQ][NT];
 #pragma unroll
         for (int i = 0; i < NQ; i++)
@@ -221,19 +214,18 @@ __global__ __launch_bounds__(256 * SETS) void latent_expanded_kernel(Expanded p)
 #pragma unroll
                 for (int e = 0; e < 4; e++) mx = fmaxf(mx, s[i][t][e]);
             if (__any(mx > m_run[i] + LAG)) {              // in the first tile for every row: it sees key 0
-                const float m = fmaxf(m_run[i], group_max(mx)), al = SETS > 1 && m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[i] - m);
+                const float m = fmaxf(m_run[i], group_max(mx)), al = __builtin_amdgcn_exp2f(m_run[i] - m);
 #pragma unroll
                 for (int n = 0; n < NVF; n++) o[i][n] *= al;
                 l_run[i] *= al;
                 m_run[i] = m;
             }
             float sum[2] = {0.0f, 0.0f};
-            const float base = SETS > 1 && m_run[i] == -INFINITY ? 0.0f : m_run[i];      // (an odd tile may show a row nothing)
 #pragma unroll
             for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    s[i][t][e] = __builtin_amdgcn_exp2f(s[i][t][e] - base);
+                    s[i][t][e] = __builtin_amdgcn_exp2f(s[i][t][e] - m_run[i]);
                     sum[e & 1] += s[i][t][e];
                 }
             l_run[i] += sum[0] + sum[1];
@@ -250,22 +242,6 @@ __global__ __launch_bounds__(256 * SETS) void latent_expanded_kernel(Expanded p)
                 for (int i = 0; i < NQ; i++) o[i][n] = mma<T>(a, for_block<T>(w[i], n >> 2), o[i][n]);
             }
         }
-    }
-    if constexpr (SETS == 2) {
-        f32x4 *const far = reinterpret_cast<f32x4 *>(lds) + 64 * (NVF + 1) * wv + lane;
-        __syncthreads();
-        if (set) {
-#pragma unroll
-            for (int n = 0; n < NVF; n++) far[64 * n] = o[0][n];
-            far[64 * NVF] = f32x4{m_run[0], l_run[0], 0.0f, 0.0f};
-        }
-        __syncthreads();
-        if (set) return;
-        const f32x4 ml = far[64 * NVF];                    // (the first set has seen key 0: its maximum is finite)
-        const float m = fmaxf(m_run[0], ml.x), f = __builtin_amdgcn_exp2f(m_run[0] - m), g = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
-        l_run[0] = l_run[0] * f + ml.y * g;
-#pragma unroll
-        for (int n = 0; n < NVF; n++) o[0][n] = o[0][n] * f + far[64 * n] * g;
     }
     const bool vec = p.vdim % 4 == 0 && p.out_row % 4 == 0;
 #pragma unroll
@@ -717,10 +693,10 @@ template <typename T> int absorbed_dispatch(const Absorbed &a, const AbsorbedPla
 #undef CQ_AB
 }
 
-template <typename T, int DK, int DV, int NQ, int SETS = 1> int expanded_launch(const Expanded &a, hipStream_t s) {
+template <typename T, int DK, int DV, int NQ> int expanded_launch(const Expanded &a, hipStream_t s) {
     const int64_t blocks = (int64_t)((a.rows + 64 * NQ - 1) / (64 * NQ)) * a.heads;
     if (blocks > 0x7fffffffLL) return CQ_ERR_RANGE;
-    hipLaunchKernelGGL((latent_expanded_kernel<T, DK, DV, NQ, SETS>), dim3((unsigned)blocks), dim3(256 * SETS), 0, s, a);
+    hipLaunchKernelGGL((latent_expanded_kernel<T, DK, DV, NQ>), dim3((unsigned)blocks), dim3(256), 0, s, a);
     return (int)hipGetLastError();
 }
 
@@ -783,12 +759,9 @@ int cq_mix_latent_expanded(const cq_latent *g, const void *q_dev, int64_t dim_pa
     const int dk = a.q_head;
     // 32 query rows per wave where that leaves two workgroups per CU
     const bool wide = (rows + 127) / 128 * g->heads >= 512;
-    // two sets of waves where that leaves two workgroups of one set per CU (2048 rows of 16 heads, 512 workgroups: 57 -> 49 us; 3000: 89 -> 104) and there is a second tile
-    const bool two = (rows + 63) / 64 * g->heads <= 512 && pos + rows > 64;
 #define CQ_EX(DK_, DV_)                                                                                                     \
     do {                                                                                                                    \
         if (!g->bf16) return expanded_launch<float, DK_, DV_, 1>(a, s);                                                     \
-        if (two) return expanded_launch<__bf16, DK_, DV_, 1, 2>(a, s);                                                      \
         return wide ? expanded_launch<__bf16, DK_, DV_, 2>(a, s) : expanded_launch<__bf16, DK_, DV_, 1>(a, s);              \
     } while (0)
     if (dk <= 128 && v_pad <= 128) CQ_EX(128, 128);

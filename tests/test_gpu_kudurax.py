@@ -295,9 +295,17 @@ SHAPES = [(1, 8, 2, 8, 8, 70), (3, 24, 10, 40, 36, 140), (16, 72, 24, 56, 112, 1
 @pytest.mark.parametrize("H,d,r,e,rank", [(3, 128, 64, 128, 256), (8, 64, 32, 96, 128)])
 @pytest.mark.parametrize("cuts", [[65], [128], [129], [64, 1, 63, 65], [193, 3], [256, 1, 64], [321]])
 def test_expanded_attention_even_and_odd_tiles(H, d, r, e, rank, cuts):
-    """Two sets of waves on the even and the odd tiles of 64 keys: one tile and two, odd counts, rows that see nothing of a set's only tile."""
+    """Even and odd counts of 64-key tiles, one and two of them, and portions that end with the first or the last row of one."""
     a = Attention(H, d, r, e, rank, sum(cuts), mixers.BF16)
     assert rel(a.run(cuts, "expanded"), a.want()) < dict(TYPES)[mixers.BF16]
+
+
+@pytest.mark.parametrize("H,d,r,e,rank,T,most", [(64, 16, 8, 16, 32, 400, 1000), (40, 128, 64, 128, 64, 496, 1700)])
+def test_expanded_attention_rows_do_not_depend_on_those_that_follow(H, d, r, e, rank, T, most):
+    """Bit for bit, across the calls of 16 and of 32 rows a wave: in a model a last bit in front of a router decides now and then which expert a token takes.
+    (Whole sixteens of rows: those of a wave are rescaled together.)"""
+    a = Attention(H, d, r, e, rank, most, mixers.BF16)
+    assert torch.equal(a.run([most], "expanded")[:T], a.run([T, most - T], "expanded")[:T])
 
 
 @pytest.mark.parametrize("precision,tol", TYPES)
