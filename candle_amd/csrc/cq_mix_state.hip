@@ -691,7 +691,9 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaRowsIn a, float *
 
 // Chunk after chunk.  Workgroup: 16 value columns of one head.  Of its eight waves the first four carry the state: wave wv keeps rows 16 wv .. as a result tile, which
 // is at the same time the operand of its quarter of P S; the quarters meet in LDS (one barrier a chunk), and their sum is again a result tile and the operand of the
-// update.  The other four form the outputs, a chunk later, from the states that the first ones leave in LDS.
+// update.  The other four form the outputs from the states that the first ones leave in LDS, each a quarter, and write the sums of the quarters one chunk later.  All
+// that waves hand to each other lies in LDS twice, for even and odd chunks: what is written between barriers c - 1 and c is read between c and c + 1, and its place written
+// again behind c + 1.
 struct DeltaPart {
     f32x4 a, u, b, v, w;                                   // a: P (state waves) or Ro (output waves)
     float qo;
@@ -709,7 +711,7 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     const float *const r0 = rec + (int64_t)h * KREC;
     const int64_t r_step = (int64_t)heads * KREC;
-    // barrier c: the quarters of P S and the state of chunk c are there, and the outputs of chunk c - 2 (__syncthreads would wait for the records on their way)
+    // barrier c: the quarters of P S and the state of chunk c are there, and those of the outputs of chunk c - 1 (__syncthreads would wait for the records on their way)
     auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     if (outputs) {
@@ -727,16 +729,15 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
             f32x4 o0 = zero, o1 = mfma4(x.qo, vs, zero);
             meet();
             const f32x4 s = ps[c & 1][wv][lane];
-            if (c > 1 && oc < dim) {                       // (whole chunks)
-                const float *p = src + (c & 1) * 1024;
-                dst[(int64_t)(KC * (c - 2) + ot) * out_stride] = (p[0] + p[256]) + (p[512] + p[768]);
+            if (c > 0 && oc < dim) {                       // (whole chunks)
+                const float *p = src + (~c & 1) * 1024;
+                dst[(int64_t)(KC * (c - 1) + ot) * out_stride] = (p[0] + p[256]) + (p[512] + p[768]);
             }
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 o0 = mfma4(x.a[e], s[e], o0);
                 o1 = mfma4(x.a[2 + e], s[2 + e], o1);
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the outputs of chunk c - 2 are read: those of c take their place
             po[c & 1][wv][lane] = o0 + o1;
         };
         DeltaPart x[4];
@@ -752,10 +753,9 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
             }
         }
         meet();
-        for (int c = max(chunks - 2, 0); c < chunks; c++) {
-            const float *p = src + (c & 1) * 1024;
-            if (KC * c + ot < rows && oc < dim) dst[(int64_t)(KC * c + ot) * out_stride] = (p[0] + p[256]) + (p[512] + p[768]);
-        }
+        const int c = chunks - 1;
+        const float *p = src + (c & 1) * 1024;
+        if (KC * c + ot < rows && oc < dim) dst[(int64_t)(KC * c + ot) * out_stride] = (p[0] + p[256]) + (p[512] + p[768]);
         return;
     }
 

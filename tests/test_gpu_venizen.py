@@ -492,6 +492,36 @@ def test_general_delta_rows(H, d, kind):
     assert rel(state[:, :, :d].transpose(1, 2), S) < 1e-5 and not state[:, :, d:].any()
 
 
+@pytest.mark.parametrize("H,d", [(5, 64), (40, 64), (600, 16)])
+def test_general_delta_long_calls(H, d):
+    """Chunks in every remainder of four, whole and cut last ones, many of them, and several workgroups to a unit: what the waves of a workgroup hand to each other
+    chunk by chunk is there when it is read, and still there.  The same bounds, the rule in 64 bits on the GPU."""
+    L, W, spd, cuts = _lib.mixer_lib(), H * d, _lib.mixer_lib().cq_mix_state_pad(d), (129, 145, 161, 177, 96, 1501)
+    T = sum(cuts)
+    g = torch.Generator(device=DEV).manual_seed(H + d)
+    rnd_dev = lambda *s: torch.randn(s, generator=g, device=DEV)
+    rows, wl, w0, ab = rnd_dev(T, 5 * W + 12), rnd_dev(T, W), 1.5 * rnd_dev(W), rnd_dev(W)
+    r, k, v, a = (rows[:, i * W:(i + 1) * W].double().reshape(T, H, d) for i in (0, 1, 2, 4))
+    w = torch.exp(-np.exp(-0.5) * torch.sigmoid(wl.double() + w0.double())).reshape(T, H, d)
+    au = torch.sigmoid(a + ab.double().reshape(H, d)) * k / (k.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+    u = k / (k.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+    S, want = torch.zeros((H, d, d), dtype=torch.float64, device=DEV), torch.zeros((T, H, d), dtype=torch.float64, device=DEV)
+    for t in range(T):
+        S = w[t, :, :, None] * S - au[t, :, :, None] * (u[t, :, :, None] * S).sum(1, keepdim=True) + k[t, :, :, None] * v[t, :, None]
+        want[t] = (r[t, :, :, None] * S).sum(1)
+    state, at = torch.zeros((H, d, spd), device=DEV), 0
+    for n in cuts:
+        need = L.cq_mix_delta_rows_workspace_bytes(n, H, d)
+        work, out = torch.full((need // 4,), float("nan"), device=DEV), torch.full((n, W + 1), 7.0, device=DEV)
+        _lib.check("r", L.cq_mix_delta_rows(rows[at:].data_ptr(), rows.shape[1], 0, W, 2 * W, 4 * W, wl[at:].data_ptr(), W, w0.data_ptr(), ab.data_ptr(),
+                                            state.data_ptr(), out.data_ptr(), W + 1, n, H, d, work.data_ptr(), need, sp()))
+        part = want[at:at + n]
+        assert float((out[:, :W].reshape(n, H, d) - part).abs().amax((1, 2)).max() / part.abs().max()) < 1e-5, at
+        assert (out[:, W] == 7.0).all()
+        at += n
+    assert float((state[:, :, :d].transpose(1, 2) - S).abs().max() / S.abs().max()) < 1e-5 and not state[:, :, d:].any()
+
+
 # ---------------------------------------------------------------------------------------------- the decoder
 LIMIT = {"float32": 2e-5, "bfloat16": 2e-2}
 _built = {}
