@@ -44,8 +44,8 @@ __device__ __forceinline__ void put(const Out &o, int64_t at, float v) {
     else reinterpret_cast<float *>(o.dst)[at] = v;
 }
 
-// four consecutive columns n .. n+3 of row m (n % 4 == 0)
-__device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, int64_t M, int N, int split) {
+// four consecutive columns n .. n+3 of row m (n % 4 == 0); present: what is already there, from a caller that has it
+__device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, int64_t M, int N, int split, const f32x4 *present = nullptr) {
     if (o.planes) {
         *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + m) * o.n4 + n) = v;
         return;
@@ -81,14 +81,14 @@ __device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, i
     float *d = reinterpret_cast<float *>(o.dst) + r * o.ldd + n;
     const float *a = o.add ? o.add + r * o.ld_add + n : nullptr;
     if (n + 4 <= N && ((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(a)) & 15) == 0) {
-        if (o.accumulate) v += *reinterpret_cast<const f32x4 *>(d);
+        if (o.accumulate) v += present ? *present : *reinterpret_cast<const f32x4 *>(d);
         if (a) v += *reinterpret_cast<const f32x4 *>(a);
         *reinterpret_cast<f32x4 *>(d) = v;
         return;
     }
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        if (n + i < N) d[i] = v[i] + (o.accumulate ? d[i] : 0.0f) + (a ? a[i] : 0.0f);
+        if (n + i < N) d[i] = v[i] + (o.accumulate ? (present ? (*present)[i] : d[i]) : 0.0f) + (a ? a[i] : 0.0f);
 }
 
 // What is already at those four columns (zero where there are none).
@@ -507,8 +507,6 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
     // what the sums are added to is asked for here, all at once (as each is stored, a load would have to wait for the store before it, and the
     // product would take half as long again)
     f32x4 old[TM][TN];
-    Out o = out;
-    o.accumulate = 0;
     if (out.accumulate)
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -521,9 +519,7 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int n = n0 + wn + 16 * j + 4 * lk;
-            f32x4 v = acc[i][j];
-            if (out.accumulate) v += old[i][j];
-            if (n < N) emit4(o, v, m, n, M, N, 0);
+            if (n < N) emit4(out, acc[i][j], m, n, M, N, 0, &old[i][j]);
         }
     }
 #endif

@@ -136,3 +136,25 @@ def test_ring_of_stages_keeps_bits(m, n, k):
         _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         got.append(y)
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("m,n,k", [(1500, 2048, 1024), (1290, 4485, 1024), (1000, 5602, 1024), (40, 516, 1024), (700, 517, 1024), (2300, 4610, 1088)])
+@pytest.mark.parametrize("x_bf16", [0, 1])
+def test_row_factors_of_sums(m, n, k, x_bf16):
+    """The factor of a row is the product's alone: y + factor * (x w) + add, whichever kernel the call takes (ring of 128 and of 192 rows, small tiles in one part and
+    in several, the large tile).  Three roundings more than the products alone."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = torch.randn((n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k), generator=g, device="cuda").bfloat16()
+    xd = x if x_bf16 else x.float()
+    scale, add, y = torch.rand(m, generator=g, device="cuda") * 4 - 2, torch.randn((m, n), generator=g, device="cuda"), torch.randn((m, n), generator=g, device="cuda")
+    product = x.double() @ w.double().t() * scale[:, None]
+    want = y + product + add
+    L = _lib.mixer_lib()
+    nb = L.cq_dense_matmul_workspace_bytes(0, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    a = DenseArgs(w_dev=w.data_ptr(), ldw=k, x_dev=xd.data_ptr(), ldx=k, x_bf16=x_bf16, dst_dev=y.data_ptr(), ldd=n, m=m, n=n, k=k, batch=1, accumulate=1,
+                  add_dev=add.data_ptr(), ld_add=n, row_scale_dev=scale.data_ptr())
+    _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    size = product.norm(dim=1) + want.norm(dim=1)
+    assert float(((y.double() - want).norm(dim=1) / size).max()) <= BOUND
