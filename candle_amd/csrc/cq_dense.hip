@@ -677,14 +677,15 @@ bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
 // tile first where it would take the call).  At k = 2048, cold weights, one round of 256 tiles takes 23 - 27 us with 128 rows and 32 - 34 with 192; 512 tiles two to a
 // unit take 49 - 53, and fewer tiles 26 - 54 in parts of k and their sum.
 //   up to 256 tiles of 128 in up to three parts (2048 x 2048 x 2048: 39.5 -> 27.2 us, 1500 x 2048 x 7168: 86.5 -> 69.3), or four of a short k (1200 x 2048 x 2048: 37.4 ->
-//     24.5, 1000 x 2048 x 7168: 54.1 against 66.3); more parts bring more workgroups to a long k (700 x 2048 x 7168: 53.2 against 60.4);
+//     24.5, 1000 x 2304 x 3072: 45.4 -> 33.9; 128 tiles in four parts just fill the chip, 1000 x 2048 x 2304: 28.2 -> 27.1, x 2560: 30.1 against 31.4, x 7168: 54.1
+//     against 66.3); more parts bring more workgroups to a long k (700 x 2048 x 7168: 53.2 against 60.4);
 //   one round of 192 where 128 takes two (1500 x 3500 x 2048: 53.5 -> 34.2), else two rounds of 128 up to 384 tiles (1000 x 5632 x 2048: 57.2 -> 49.1; 448: 51.1 against 51.3);
 //   beyond one round of two to a unit, rounds of 192 that are two thirds full (1200 x 7168 x 2048: 68.4 -> 63.8, 2048 x 10368 x 2048: 130.5 -> 122.9).
 int ring_rows(const Plan &p, int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
     if (p.bm != 128 || ldw > (1 << 20) || ldx > (1 << 20)) return 0;       // (its offsets have 32 bits)
     const int64_t t128 = (int64_t)p.tiles_m * p.tiles_n, t192 = (m + 191) / 192 * p.tiles_n, rounds = (t192 + 255) / 256;
     if (p.splits == 1 && large_tile(m, n, k, ldw, ldx)) return 0;
-    if (t128 <= 256) return p.splits <= 3 || (p.splits == 4 && k <= 3072) ? 128 : 0;
+    if (t128 <= 256) return p.splits <= 3 || (p.splits == 4 && k <= (t128 > 128 ? 3072 : 2304)) ? 128 : 0;
     if (t192 <= 256) return 192;
     if (t128 <= 384) return 128;
     return t128 > 512 && 3 * t192 >= 2 * 256 * rounds ? 192 : 0;
