@@ -572,7 +572,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(const float *__restrict_
 }
 
 // The prompt's attention from 256 keys on (attn_by_planes): the two products on the bf16 matrix cores, from operands split into three bf16 parts that add up to the
-// f32 value (8 + 8 + 8 bits; of an infinity, NaN).  Of the nine products of parts the six above 2^-24 of the whole are formed, the scores' small ones apart from the
+// f32 value (8 + 8 + 8 bits).  Of the nine products of parts the six above 2^-24 of the whole are formed, the scores' small ones apart from the
 // large one; sums are f32.  Six times 16 cycles for 16 x 16 x 32 stand against 8 x 32 of the f32 instruction, which bounds the kernel above; the error against 64 bits
 // is half of that kernel's, which rounds four keys or dimensions at a time (2-norm, 1000 rows: 1.64e-7 against 3.35e-7; scores four times as large 4.3e-7, 1.03e-6).
 // attn_planes_kernel splits the keys and values that are visible, once for all workgroups, into tiles of 32 keys laid out as the operands are read: keys
@@ -580,6 +580,8 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(const float *__restrict_
 // eight waves four take the even tiles of keys and four the odd ones (the last rows of a prompt see all keys, and are the longest chain of the launch).  Scores are formed
 // as k q^T: a lane then holds keys 16 y + 4 lk + e of its pair lr, which is an operand of the second product as it lies (the values' tiles have their keys in that
 // order); a maximum is taken across lanes only where a score exceeds the running one.  Values are summed four tiles at a time and the sums then added, as above.
+// The parts of an infinity, and of a finite value that bfloat16 rounds to one, are no numbers, and neither is any result that they reach: a pair with such a result is
+// formed again in f32, from the caches (attn_pair_again).
 // Keys arrive an iteration ahead, values under the first product.  Bound by LDS: four waves read 48 KB a tile each, 1920 cycles with the copies, beside 1536 of products.
 // 32 heads, 8 kv heads, us (f32 kernel above -> this, splitting 5 - 20 of it): 300 rows 31 -> 25, 500: 48 -> 35, 1000: 145 -> 73, 2048: 450 -> 216, 300 behind 4000 keys:
 // 406 -> 191.
@@ -619,10 +621,46 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(const float *__restric
     }
 }
 
+// One (row, head) pair by one wave, as the f32 kernels form it: keys k and values v [len][128] of the head, weights of zero where a score is not above -inf.  Rare, and
+// slow: 64 keys at a time, a lane forms the score of one and sums two dimensions of their values.
+__device__ __forceinline__ void attn_pair_again(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, float *__restrict__ out, int len,
+                                                float scale, int lane) {
+    auto score = [&](int j) {
+        float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const f32x4 *kr = reinterpret_cast<const f32x4 *>(k + (int64_t)min(j, len - 1) * 128);
+        for (int c = 0; c < 32; c++) {
+            const f32x4 x = kr[c];
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[e] = fmaf(q[4 * c + e], x[e], s[e]);
+        }
+        return j < len ? ((s[0] + s[1]) + (s[2] + s[3])) * scale : -INFINITY;
+    };
+    float m = -INFINITY, l = 0.0f, o[2] = {0.0f, 0.0f};
+    for (int j = lane; j < len + lane; j += 64) m = fmaxf(m, score(j));
+    m = wave_max(m);
+    for (int j0 = 0; j0 < len; j0 += 64) {
+        const float s = score(j0 + lane), p = s > -INFINITY ? __expf(s - m) : 0.0f;
+        float a[2] = {0.0f, 0.0f};
+        const int n = min(64, len - j0);
+        for (int j = 0; j < n; j++) {
+            const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
+            const float *x = v + (int64_t)(j0 + j) * 128 + 2 * lane;
+            a[0] = fmaf(w, x[0], a[0]);
+            a[1] = fmaf(w, x[1], a[1]);
+        }
+        l += p;
+        o[0] += a[0];
+        o[1] += a[1];
+    }
+    l = wave_sum(l);
+    out[2 * lane] = o[0] / l;
+    out[2 * lane + 1] = o[1] / l;
+}
+
 template <int G>
 __global__ __launch_bounds__(512, 2) void attn_planes_run_kernel(const float *__restrict__ q, int64_t q_stride, const uint8_t *__restrict__ planes, float *__restrict__ out,
                                                                  const int32_t *__restrict__ pos_dev, int pos0, int rows, int n_head, int ctx, float scale, int tiles,
-                                                                 int groups) {
+                                                                 int groups, const float *__restrict__ k_cache, const float *__restrict__ v_cache) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
     constexpr int HD = 128, R = 64 / G;              // pair 16 wv + lr = R * head of the group + row
     __shared__ __attribute__((aligned(16))) uint8_t smem[6 * AT_TILE];     // of either set of waves: keys of two tiles, values of one
@@ -781,15 +819,32 @@ __global__ __launch_bounds__(512, 2) void attn_planes_run_kernel(const float *__
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if (pair % R >= nr) return;
-    struct __attribute__((packed, aligned(4))) Out4 { f32x4 v; };      // (out has the alignment of a float)
-    float *const dst = out + ((int64_t)(r0 + row) * n_head + head) * HD + 4 * lk;
+    if (pair % R < nr) {
+        struct __attribute__((packed, aligned(4))) Out4 { f32x4 v; };      // (out has the alignment of a float)
+        float *const dst = out + ((int64_t)(r0 + row) * n_head + head) * HD + 4 * lk;
 #pragma unroll
-    for (int d = 0; d < 8; d++) {
-        f32x4 x;
+        for (int d = 0; d < 8; d++) {
+            f32x4 x;
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[e] = o[d][e] / l;
-        reinterpret_cast<Out4 *>(dst + 16 * d)->v = x;
+            for (int e = 0; e < 4; e++) x[e] = o[d][e] / l;
+            reinterpret_cast<Out4 *>(dst + 16 * d)->v = x;
+        }
+    }
+    f32x4 none = zero;                                     // zero where all are numbers
+#pragma unroll
+    for (int d = 0; d < 8; d++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) none[e] = fmaf(o[d][e], 0.0f, none[e]);
+    const uint64_t lanes = __ballot(!((none[0] + none[1]) + (none[2] + none[3]) == 0.0f));
+    if (!lanes) return;
+    const uint32_t again = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;      // pairs of the wave
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // what is there of them is overwritten
+    for (uint32_t left = again; left; left &= left - 1) {
+        const int i = 16 * wv + __builtin_ctz(left), r = i % R, h = kvh * G + i / R;
+        if (r >= nr) continue;
+        const int64_t at = (int64_t)kvh * ctx * HD;
+        attn_pair_again(q + (int64_t)(r0 + r) * q_stride + (int64_t)h * HD, k_cache + at, v_cache + at, out + ((int64_t)(r0 + r) * n_head + h) * HD, min(base_len + r, ctx),
+                        scale, lane);
     }
 #endif
 }
@@ -1564,7 +1619,7 @@ int launch_attn_planes(int G, hipStream_t s, const float *q, int64_t q_stride, c
 #define CQ_ATT(GG)                                                                                                                                     \
     case GG:                                                                                                                                           \
         hipLaunchKernelGGL((attn_planes_run_kernel<GG>), dim3((unsigned)wgs), dim3(512), 0, s, q, q_stride, (const uint8_t *)planes, out, pos_dev, pos0, rows, \
-                           n_head, ctx, scale, tiles, groups);                                                                      \
+                           n_head, ctx, scale, tiles, groups, kc, vc);                                                                      \
         break;
     switch (G) {
         CQ_ATT(1) CQ_ATT(2) CQ_ATT(4) CQ_ATT(8)

@@ -171,6 +171,57 @@ def test_attention_prompt_split_operands_of_all_sizes():
     assert np.array_equal(out.cpu().numpy(), np.broadcast_to(np.repeat(vc[:, 17], H // KV, 0), (rows, H, D)))
 
 
+@pytest.mark.parametrize("H,KV", [(8, 1), (8, 2), (4, 2), (2, 2)])
+@pytest.mark.parametrize("what", ["key far below", "key far above", "infinite value", "infinite query", "largest values", "largest keys", "largest queries"])
+def test_attention_prompt_beyond_split_operands(H, KV, what):
+    """Infinities, and finite values that bfloat16 rounds to one, in the split operands' call: what f32 arithmetic gives.  A key whose score is -inf has no weight, one
+    of +inf leaves no number; a value counts from its own row on.  (The call for few keys computes with f32 throughout.)"""
+    D, rows, pos, j = 128, 70, 230, 240                    # the marked key is the new row 10's
+    ctx, at = pos + rows, j - pos
+    q, kc, vc = normal(70, (rows, H, D), 1.0), normal(71, (KV, ctx, D), 1.0), normal(72, (KV, ctx, D), 1.0)
+    top, scale = np.float32(3.4e38), float(np.float32(1.0 / math.sqrt(D)))
+    q[:, :, 5] = np.abs(q[:, :, 5]) + 0.1
+    if what == "key far below":
+        kc[:, j, 5] = -np.inf
+    elif what == "key far above":
+        kc[:, j, 5] = np.inf
+    elif what == "infinite value":
+        vc[:, j, 7], vc[:, j, 8] = np.inf, -np.inf
+    elif what == "infinite query":
+        q[at, 0, 5] = np.inf
+        kc[:, :, 5] = -np.abs(kc[:, :, 5])
+        kc[:, 3, 5] = 0.0                                  # inf * 0: no number, and no weight
+        kc[:, 4, 5] = 2.0                                  # +inf
+    elif what == "largest values":
+        vc[:, j, 7:9] = top, -top
+    elif what == "largest keys":
+        kc[:, j, 5], q[:, :, 5] = top, 1e-38
+    else:
+        q[at, 0, 5], kc[:, :, 5] = -top, np.abs(kc[:, :, 5]) * 1e-38
+    k64, v64, G = kc.astype(np.float64), vc.astype(np.float64), H // KV
+    want = np.zeros((rows, H, D))
+    with np.errstate(all="ignore"):
+        for r in range(rows):
+            for h in range(H):
+                k, v = k64[h // G, :pos + r + 1], v64[h // G, :pos + r + 1]
+                z = (k * q[r, h].astype(np.float64)).sum(1) * scale
+                m = np.fmax.reduce(z)
+                p = np.where(z > -np.inf, np.exp(z - m), 0.0)
+                want[r, h] = (p[:, None] * v).sum(0) / p.sum()
+        want = want.astype(np.float32)
+    lib, qd, kd, vd = L(), dev(q), dev(kc), dev(vc)
+    need, fits = lib.cq_nn_attention_workspace_bytes(rows, H, D, ctx), (ctx + 31) // 32 * KV * 49152
+    ws, out = torch.full((max(need, fits),), 255, dtype=torch.uint8, device="cuda"), torch.full((rows, H, D), 7.0, device="cuda")
+    ok(lib.cq_nn_attention(qd.data_ptr(), H * D, kd.data_ptr(), vd.data_ptr(), out.data_ptr(), None, pos, rows, H, KV, D, ctx, ctx, scale, ws.data_ptr(), max(need, fits), None))
+    torch.cuda.synchronize()
+    got, fine = out.cpu().numpy(), np.isfinite(want)
+    assert {"key far below": fine.all(), "largest values": fine.all(), "largest keys": fine.all(), "largest queries": fine.all()}.get(what, not fine.all())
+    assert np.array_equal(np.where(fine, 0.0, want), np.where(fine, 0.0, got), equal_nan=True)
+    small = fine & (np.abs(want) < 1e30)
+    assert rel_l2(np.where(small, got, 0.0), np.where(small, want, 0.0)) <= TOL
+    assert np.allclose(got[fine & ~small], want[fine & ~small], rtol=1e-5)
+
+
 @pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (8, 1, 128), (4, 4, 128), (32, 8, 128)])
 def test_attention_rows_share_keys_with_position_on_device(H, KV, D):
     """16 rows and more go several to a workgroup; the position may come from device memory (a captured graph)."""
