@@ -659,13 +659,17 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaRowsIn a, float *
         const int j = 4 * lk + g;                          // Qo: [t = lr][s = 4 lk + g]
         float sum = 0.0f;
 #pragma unroll
-        for (int s = 0; s < KC; s++) sum = fmaf(mat[3 * MAT + lr * LD + s], mat[s * LD + j], sum);
+        for (int s = 0; s < KC; s++) {
+            const float more = fmaf(mat[3 * MAT + lr * LD + s], mat[s * LD + j], sum);
+            sum = s <= lr ? more : sum;
+        }
         r[KREC_Q + tid] = mat[2 * MAT + lr * LD + j] - sum;
     }
-    // Ro and U of the wave's own tokens (beyond the triangles the matrices are zero)
+    // Ro and U of the wave's own tokens (beyond the triangles the matrices are zero, but P and Q of a token that is no number are none either, and may not reach the
+    // tokens before it)
     float ro[4] = {0.f, 0.f, 0.f, 0.f};
     f32x4 lost = {0.f, 0.f, 0.f, 0.f};
-    for (int s4 = 0; s4 <= g; s4++) {
+    auto removed = [&](int s4, auto whole) {
         float p[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) p[e] = s_ut[(4 * s4 + e) * KLD + lane];
@@ -673,9 +677,12 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaRowsIn a, float *
         for (int i = 0; i < 4; i++) {
             const f32x4 l = *reinterpret_cast<const f32x4 *>(mat + 3 * MAT + (4 * g + i) * LD + 4 * s4);
 #pragma unroll
-            for (int e = 0; e < 4; e++) ro[i] = fmaf(l[e], p[e], ro[i]);
+            for (int e = 0; e < 4; e++)
+                if (whole || e <= i) ro[i] = fmaf(l[e], p[e], ro[i]);
         }
-    }
+    };
+    for (int s4 = 0; s4 < g; s4++) removed(s4, std::integral_constant<bool, true>{});
+    removed(g, std::integral_constant<bool, false>{});
     for (int t = 4 * g + 1; t < KC; t++) {
         const f32x4 q = *reinterpret_cast<const f32x4 *>(mat + t * LD + 4 * g);
         const float x = s_bt[t * KLD + lane];
@@ -724,9 +731,24 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
             x.v = reinterpret_cast<const f32x4 *>(r)[1024 + 64 * cb + lane];
             x.qo = r[KREC_Q + tid];
         };
-        auto step = [&](const DeltaPart &x, int c) {
-            const float vs = wv & 2 ? (wv & 1 ? x.v[3] : x.v[2]) : (wv & 1 ? x.v[1] : x.v[0]);
-            f32x4 o0 = zero, o1 = mfma4(x.qo, vs, zero);
+        auto value = [&](const DeltaPart &x) { return wv & 2 ? (wv & 1 ? x.v[3] : x.v[2]) : (wv & 1 ? x.v[1] : x.v[0]); };      // of token 4 lk + wv
+        auto marked = [&](const DeltaPart &x) { return __any(!(fabsf(value(x)) < INFINITY)) != 0; };
+        bool mark;                                         // one of the chunk's values is no number (found out a step ahead: in front of the products it costs 2 %)
+        auto step = [&](const DeltaPart &x, const DeltaPart &next, int c) {
+            const float vs = value(x);
+            f32x4 o0 = zero, o1 = zero;
+            if (!mark) o1 = mfma4(x.qo, vs, zero);
+            else {                                         // such a value counts from its own token on: zero times it is no number either
+#pragma unroll
+                for (int a = 0; a < 4; a++) {
+                    const float va = __shfl(vs, 16 * a + lr, 64);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float q = __shfl(x.qo, 16 * a + 4 * lk + e, 64), more = fmaf(q, va, o1[e]);
+                        o1[e] = 4 * a + wv <= 4 * lk + e ? more : o1[e];
+                    }
+                }
+            }
             meet();
             const f32x4 s = ps[c & 1][wv][lane];
             if (c > 0 && oc < dim) {                       // (whole chunks)
@@ -739,17 +761,19 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
                 o1 = mfma4(x.a[2 + e], s[2 + e], o1);
             }
             po[c & 1][wv][lane] = o0 + o1;
+            mark = marked(next);
         };
         DeltaPart x[4];
         load(x[0], 0);
         load(x[1], 1);
         load(x[2], 2);
+        mark = marked(x[0]);
         for (int c = 0; c < chunks; c += 4) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 if (c + j >= chunks) break;
                 load(x[(j + 3) & 3], c + j + 3);
-                step(x[j], c + j);
+                step(x[j], x[(j + 1) & 3], c + j);
             }
         }
         meet();

@@ -522,6 +522,43 @@ def test_general_delta_long_calls(H, d):
     assert float((state[:, :, :d].transpose(1, 2) - S).abs().max() / S.abs().max()) < 1e-5 and not state[:, :, d:].any()
 
 
+@pytest.mark.parametrize("H,d", [(2, 64), (3, 20)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("t", [0, 5, 18, 31, 46, 66])
+def test_general_delta_tokens_that_are_no_numbers(H, d, bad, t):
+    """A value, query, key, removal rate or decay of one token that is no number, in every quarter of a chunk: the outputs of the tokens before it, and those that it does
+    not reach, stay what they are without it (a query: its own token; a value: its column from there on; the others: everything from there on)."""
+    L, W, spd, T = _lib.mixer_lib(), H * d, _lib.mixer_lib().cq_mix_state_pad(d), 67
+    rows, wl, w0, ab = up(rnd(21, T, 5 * W + 12)), up(rnd(22, T, W)), up(rnd(23, W)), up(rnd(24, W))
+
+    def run(rows, wl):
+        state, out = torch.zeros((H, d, spd), device=DEV), torch.full((T, W), 7.0, device=DEV)
+        need = L.cq_mix_delta_rows_workspace_bytes(T, H, d)
+        work = torch.full((need // 4,), float("nan"), device=DEV)
+        _lib.check("r", L.cq_mix_delta_rows(rows.data_ptr(), rows.shape[1], 0, W, 2 * W, 4 * W, wl.data_ptr(), W, w0.data_ptr(), ab.data_ptr(), state.data_ptr(), out.data_ptr(),
+                                            W, T, H, d, work.data_ptr(), need, sp()))
+        return out.reshape(T, H, d), state[:, :, :d]
+
+    plain, plain_state = run(rows, wl)
+    for name, at in (("query", 0), ("key", W), ("value", 2 * W), ("rate", 4 * W), ("decay", None)):
+        if at in (4 * W, None) and bad == float("inf"):
+            continue                                       # a sigmoid of infinity is a number
+        r, w = rows.clone(), wl.clone()
+        (w if at is None else r)[t, (at or 0) + d + 3] = bad           # of the second head
+        got, state = run(r, w)
+        keep = torch.ones((T, H, d), dtype=torch.bool, device=DEV)
+        keep_state = torch.ones_like(state, dtype=torch.bool)
+        if name == "query":
+            keep[t, 1] = False
+        elif name == "value":
+            keep[t:, 1, 3], keep_state[1, 3] = False, False
+        else:
+            keep[t:, 1], keep_state[1] = False, False
+        assert torch.equal(got[keep], plain[keep]), name
+        assert not torch.isfinite(got[t, 1, 3]) and (name == "query" or not torch.isfinite(got[t:, 1, 3]).any()), name
+        assert torch.equal(state[keep_state], plain_state[keep_state]) and (name == "query" or not torch.isfinite(state[1, 3]).all()), name
+
+
 # ---------------------------------------------------------------------------------------------- the decoder
 LIMIT = {"float32": 2e-5, "bfloat16": 2e-2}
 _built = {}
