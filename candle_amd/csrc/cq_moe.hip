@@ -173,6 +173,10 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
 // stores wait for each other on one unit (12000 pairs of 128 experts 25.8 -> 9.6 us; a layer of 256 tokens 142 -> 138).
 // inverse: pair_in[p] is the place of pair p (-1: none) instead of the row at a place.
 constexpr int GROUP_WIDE_EXPERTS = 1024;
+// From here on the pairs of a token are quantized once: fewer take no longer by a wave for each row of a pair (a call of 600 Q8_0 pairs on 512 experts in us, once / pair by
+// pair: 40.6 / 39.8, on 128: 64.0 / 63.5, 1200: 65.7 / 67.4; sorted by expert 600 on 512: 42.8 / 39.8, 1200 on 128: 69.3 / 68.4, 2400: 76.5 / 74.3; 2400 in token order 72.2 /
+// 74.7, 12000: 161 / 174).
+constexpr int SPREAD_PAIRS = 2048;
 __global__ __launch_bounds__(1024) void moe_group_wide_kernel(PairSource ps, int *__restrict__ offsets, int *__restrict__ pair_in, int *__restrict__ pair_out,
                                                               float *__restrict__ pair_scale, int *__restrict__ chunks, int max_chunks, int chunk,
                                                               int *__restrict__ extra, int inverse) {
@@ -419,7 +423,7 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     const int chunk = stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK;
     const bool wide = a.mode != MOE_INDEXED && a.num_experts <= GROUP_WIDE_EXPERTS;
     // pairs of the gate / up products: the same row goes to all experts of a token
-    const bool spread = wide && mfma && !stream && !a.topk_weights && a.topk > 1;
+    const bool spread = wide && mfma && !stream && !a.topk_weights && a.topk > 1 && a.n_pairs > SPREAD_PAIRS;
     if (wide)
         hipLaunchKernelGGL(moe_group_wide_kernel, dim3((unsigned)a.num_experts), dim3(1024), 0, s, ps, offsets, pin, pout, pscale, chunks, (int)ws.max_chunks, chunk,
                            stream ? extra : nullptr, (int)spread);

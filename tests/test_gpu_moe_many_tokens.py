@@ -111,3 +111,34 @@ def test_grouping_of_lists(dtype, E, tokens, top, order):
     hit = np.zeros(pairs, bool)
     hit[order_of[valid]] = True
     assert rel_l2(got[hit], want[hit]) <= 2e-6 and (got[~hit] == 7.0).all() and (~hit).any()
+
+
+@pytest.mark.parametrize("dtype", [oracle.Q8_0, oracle.Q6K])
+@pytest.mark.parametrize("E,tokens,top", [(5, 128, 16), (5, 129, 16), (40, 160, 17), (40, 200, 20), (512, 700, 3), (513, 1365, 3), (513, 1366, 3), (1024, 600, 8), (1025, 800, 8)])
+def test_grouping_of_lists_in_any_order(dtype, E, tokens, top):
+    """A list in token order, sorted by expert and shuffled gives the same bits: on either side of the numbers of pairs and experts at which another kernel groups or
+    quantizes them, with groups of pairs that hold parts of two tokens, and with experts that have no pair."""
+    import candle_amd as ca
+    n, k, pairs = 12, 512, tokens * top
+    blocks = oracle.from_float(dtype, normal(5, (E, n, k), 0.02).reshape(-1))
+    qt = ca.QTensor.new(ca.QStorage.from_data(blocks, "cuda", ca.GgmlDType(dtype)), (E, n, k))
+    rng = np.random.default_rng(tokens)
+    experts = rng.integers(0, E, pairs).astype(np.int32)
+    experts[rng.choice(pairs, 5, replace=False)] = -1
+    x, L = normal(6, (tokens, k)), _lib.lib()
+    cuda = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    xd, got = cuda(x), []
+    ws = torch.full((L.cq_moe_gemm_workspace_bytes(int(dtype), E, top, pairs, n, k, 0),), 255, dtype=torch.uint8, device="cuda")
+    for order in (np.arange(pairs), np.argsort(experts, kind="stable"), rng.permutation(pairs)):
+        ed, od, out = cuda(experts[order]), cuda(order.astype(np.int32)), torch.full((pairs, n), 7.0, device="cuda")
+        _lib.check("cq_moe_gemm_gguf", L.cq_moe_gemm_gguf(int(dtype), xd.data_ptr(), qt.device_ptr(), od.data_ptr(), ed.data_ptr(), None, out.data_ptr(), E, top, pairs, n, k, 1,
+                                                          ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        got.append(out.cpu().numpy())
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    want, per = np.full((pairs, n), 7.0, np.float32), len(blocks) // E
+    for e in range(E):
+        p = np.flatnonzero(experts == e)
+        if len(p):
+            want[p] = oracle.matmul(dtype, x[p // top], blocks[e * per:(e + 1) * per], n)
+    assert rel_l2(got[0], want) <= 2e-6 and (got[0][experts < 0] == 7.0).all()
