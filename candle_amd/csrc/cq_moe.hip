@@ -170,9 +170,11 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(PairSource ps, int *__r
 
 // The same with a workgroup per expert, for lists of (expert, token) pairs of up to GROUP_WIDE_EXPERTS experts: every workgroup counts the whole list in LDS, which
 // comes out of the L2, and then places the pairs of its own expert.  One workgroup for all of them takes 1.7 us per 1000 pairs: its loads, atomics and
-// stores wait for each other on one unit (12000 pairs of 128 experts 25.8 -> 9.6 us; a layer of 256 tokens 142 -> 138).
+// stores wait for each other on one unit (12000 pairs of 128 experts 25.8 -> 9.6 us; a layer of 256 tokens 142 -> 138).  That every workgroup reads the whole list shows
+// where there are many: beyond 512 experts, one round of workgroups, up to 4096 pairs are grouped by one (a call of 1024 experts in us, by one / by all: 600 pairs 40.0 /
+// 44.3, 2400: 57.6 / 58.7, 5000: 69.4 / 66.1, 12000: 96.9 / 87.8; in a list sorted by expert 5000: 64.1 / 66.8, 12000: 85.8 / 89.3, 48000: 266 / 239).
 // inverse: pair_in[p] is the place of pair p (-1: none) instead of the row at a place.
-constexpr int GROUP_WIDE_EXPERTS = 1024;
+constexpr int GROUP_WIDE_EXPERTS = 1024, GROUP_WIDE_ROUND = 512, GROUP_WIDE_PAIRS = 4096;
 // From here on the pairs of a token are quantized once: fewer take no longer by a wave for each row of a pair (a call of 600 Q8_0 pairs on 512 experts in us, once / pair by
 // pair: 40.6 / 39.8, on 128: 64.0 / 63.5, 1200: 65.7 / 67.4; sorted by expert 600 on 512: 42.8 / 39.8, 1200 on 128: 69.3 / 68.4, 2400: 76.5 / 74.3; 2400 in token order 72.2 /
 // 74.7, 12000: 161 / 174).
@@ -201,8 +203,18 @@ __global__ __launch_bounds__(1024) void moe_group_wide_kernel(PairSource ps, int
                 if (p0 + 1024 * i < n) f(p0 + 1024 * i, (uint32_t)ke[i] < (uint32_t)E && to[i] >= 0 && to[i] < limit, ke[i], to[i]);
         }
     };
-    each([&](int, bool ok, int x, int) {
-        if (ok) atomicAdd(&cnt[x], 1);
+    // pairs of one expert in a row, as in a list sorted by expert, are counted by the first of them: one by one their lanes would wait for each other (48000 sorted pairs
+    // of 512 experts: a call of 207 us takes 161)
+    each([&](int, bool ok, int expert, int) {
+        const int lane = tid & 63, x = ok ? expert : -1;
+        const bool head = __builtin_amdgcn_update_dpp(-2, x, 0x138, 0xf, 0xf, false) != x;      // (the lane before; -2 in front of the first)
+        const uint64_t heads = __ballot(head), here = __ballot(1);
+        int count = 1;
+        if (heads != here) {
+            const uint64_t after = heads >> lane >> 1;
+            count = after ? __builtin_ctzll(after) + 1 : __popcll(here) - lane;
+        }
+        if (head && ok) atomicAdd(&cnt[x], count);
     });
     __syncthreads();
     auto passes = [](int c) { return c > 32 ? (c + 31) / 32 - 1 : 0; };       // (of an expert's pairs beyond the first 32, for the batched matvecs)
@@ -421,7 +433,7 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     auto *const group = a.num_experts <= GROUP_LDS_EXPERTS ? (many ? moe_group_kernel<true, true> : moe_group_kernel<true, false>)
                                                            : (many ? moe_group_kernel<false, true> : moe_group_kernel<false, false>);
     const int chunk = stream ? CQ_MOE_STREAM_CHUNK : mfma ? tile_rows : CQ_MOE_CHUNK;
-    const bool wide = a.mode != MOE_INDEXED && a.num_experts <= GROUP_WIDE_EXPERTS;
+    const bool wide = a.mode != MOE_INDEXED && (a.num_experts <= GROUP_WIDE_ROUND || (a.num_experts <= GROUP_WIDE_EXPERTS && a.n_pairs > GROUP_WIDE_PAIRS));
     // pairs of the gate / up products: the same row goes to all experts of a token
     const bool spread = wide && mfma && !stream && !a.topk_weights && a.topk > 1 && a.n_pairs > SPREAD_PAIRS;
     if (wide)
