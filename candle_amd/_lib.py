@@ -2,12 +2,15 @@
 include/candle_hip_nn.h) and of libcandle_hip_mixer.so (include/candle_hip_mixer.h, plus the glue of candle_hip_nn.h).
 
 The library must be built first (``python -m candle_amd.build`` or ``__graft_entry__.build()``);
-loading fails loudly when it is missing — there is no CPU or PyTorch fallback.
+loading fails loudly when it is missing — there is no CPU or PyTorch fallback.  The native host path of quantized
+products is a third file, without which the same launches are made from Python.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcandle_hip_quant.so")
@@ -182,19 +185,33 @@ def _load(path: str, signatures: dict) -> ctypes.CDLL:
     return L
 
 
-qmatmul = None                 # QTensor.fwd of an ordinary call (csrc/cq_host.cpp), once the library is loaded
+def host_path() -> str:
+    return os.path.join(_HERE, "_host.so")
+
+
+def _native_qmatmul(L: ctypes.CDLL):
+    path = host_path()
+    try:
+        spec = importlib.util.spec_from_file_location(f"{__package__}._host", path)
+        host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(host)
+    except ImportError as e:
+        warnings.warn(f"{path} is missing or does not load ({e}): quantized products take the slower host path in Python until it is built (python -m candle_amd.build)",
+                      RuntimeWarning, stacklevel=3)
+        return None
+    host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (L.cq_qmatmul_workspace_bytes, L.cq_qmatmul_forward)))
+    return host.qmatmul
+
+
+qmatmul = None                 # QTensor.fwd of an ordinary call (csrc/cq_host.cpp), once the library is loaded and where that was built
 
 
 def lib() -> ctypes.CDLL:
     global _lib, qmatmul
     if _lib is None:
         L = _load(LIB_PATH, SIGNATURES)
-        try:
-            from . import _host
-        except ImportError as e:
-            raise ImportError("candle_amd/_host.so is missing or does not fit this PyTorch: build it first (python -m candle_amd.build)") from e
-        _host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (L.cq_qmatmul_workspace_bytes, L.cq_qmatmul_forward)))
-        _lib, qmatmul = L, _host.qmatmul
+        qmatmul = _native_qmatmul(L)
+        _lib = L
     return _lib
 
 

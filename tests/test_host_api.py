@@ -215,3 +215,17 @@ def test_native_host_path_leaves_other_calls_to_python():
     for args in ((x, x, 12, (4, 256), q._workspaces), (x, x, "12", (4, 256), q._workspaces), (x, x, 12, [4, 256], q._workspaces), (x, x, 12, (4,), q._workspaces),
                  (x, x, 12, (4, 256), None), (None, x, 12, (4, 256), q._workspaces), (x,), (torch.nn.Parameter(x), x, 12, (4, 256), q._workspaces)):
         assert _lib.qmatmul(*args) is None
+
+
+@pytest.mark.parametrize("found", ["nothing", "another file"])
+def test_library_loads_without_the_native_host_path(found, monkeypatch, tmp_path):
+    """Where the module was not built for this Python and PyTorch, or does not load, the library does, says so, and leaves the calls to the Python path."""
+    path = tmp_path / "_host.so"
+    if found == "another file":
+        path.write_bytes(b"not a module")
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "qmatmul", None)
+    monkeypatch.setattr(_lib, "host_path", lambda: str(path))
+    with pytest.warns(RuntimeWarning, match="slower host path"):
+        L = _lib.lib()
+    assert _lib.qmatmul is None and L.cq_qmatmul_workspace_bytes(12, 1, 256, 4) >= 0
