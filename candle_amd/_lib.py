@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
 import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -186,7 +187,9 @@ def _load(path: str, signatures: dict) -> ctypes.CDLL:
 
 
 def host_path() -> str:
-    return os.path.join(_HERE, "_host.so")
+    """The native host path for the Python and PyTorch that run now: its code has their objects' layout built in, so each of them has a file of its own."""
+    import torch
+    return os.path.join(_HERE, f"_host.{sys.implementation.cache_tag}.torch-{torch.__version__}-{str(torch.version.git_version)[:10]}-abi{int(torch.compiled_with_cxx11_abi())}.so")
 
 
 def _native_qmatmul(L: ctypes.CDLL):

@@ -1,4 +1,4 @@
-"""Builds libcandle_hip_quant.so (gfx950) in-tree with hipcc, and the native host path (_host.so) with the host compiler.
+"""Builds libcandle_hip_quant.so (gfx950) in-tree with hipcc, and the native host path (_host....so) with the host compiler.
 
     python -m candle_amd.build            # compile what changed, link
     python -m candle_amd.build --force    # recompile everything
@@ -34,7 +34,6 @@ MIXER_HEADERS = ("candle_hip_mixer.h", "cq_mix.h", "cq_dense.h")
 # the benchmark's plain-read yardstick kernel: a library of its own, not part of the C ABI
 BENCH_SOURCES = ["cq_bench.hip"]
 # the native host path of plain calls: a Python module over PyTorch's C++ interface, without device code
-HOST = os.path.join(HERE, "_host.so")
 HOST_SOURCE = "cq_host.cpp"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -93,25 +92,33 @@ def _build(groups, force: bool) -> None:
             os.replace(tmp, lib)
 
 
+def host_is_current(path: str) -> bool:
+    """Whether the host path at `path` (the name says for which Python and PyTorch) was built from the present source by the present recipe."""
+    return os.path.exists(path) and os.path.getmtime(path) > max(os.path.getmtime(os.path.join(CSRC, HOST_SOURCE)), os.path.getmtime(os.path.abspath(__file__)))
+
+
 def build_host(force: bool = False) -> str:
-    src = os.path.join(CSRC, HOST_SOURCE)
-    if not force and os.path.exists(HOST) and os.path.getmtime(HOST) > os.path.getmtime(src):
-        return HOST
+    from ._lib import host_path
+    path = host_path()
+    if not force and host_is_current(path):
+        return path
     import sysconfig
 
+    import torch
     from torch.utils import cpp_extension
     libs = cpp_extension.library_paths()
     inc = [*cpp_extension.include_paths(), os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
-    tmp = f"{HOST}.{os.getpid()}"
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(f"-isystem{i}" for i in inc), "-Wall", src,
+    tmp = f"{path}.{os.getpid()}"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *(f"-isystem{i}" for i in inc), "-Wall", os.path.join(CSRC, HOST_SOURCE),
            "-o", tmp, *(f"-L{p}" for p in libs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"{cmd[0]} failed for {HOST_SOURCE}:\n{r.stderr}")
     if r.stderr.strip():
         sys.stderr.write(r.stderr)
-    os.replace(tmp, HOST)
-    return HOST
+    os.replace(tmp, path)
+    return path
 
 
 def build(force: bool = False) -> str:

@@ -229,3 +229,37 @@ def test_library_loads_without_the_native_host_path(found, monkeypatch, tmp_path
     with pytest.warns(RuntimeWarning, match="slower host path"):
         L = _lib.lib()
     assert _lib.qmatmul is None and L.cq_qmatmul_workspace_bytes(12, 1, 256, 4) >= 0
+
+
+@pytest.mark.parametrize("what", ["version", "source", "abi", "python"])
+def test_native_host_path_is_for_one_python_and_pytorch(what, monkeypatch):
+    """A module that was built for another one is never taken for this one's."""
+    import sys
+
+    import torch
+    before = _lib.host_path()
+    if what == "version":
+        monkeypatch.setattr(torch, "__version__", "9.9.9")
+    elif what == "source":
+        monkeypatch.setattr(torch.version, "git_version", "0123456789abcdef")
+    elif what == "abi":
+        monkeypatch.setattr(torch, "compiled_with_cxx11_abi", lambda: not torch._C._GLIBCXX_USE_CXX11_ABI)
+    else:
+        import types
+        monkeypatch.setattr(sys, "implementation", types.SimpleNamespace(cache_tag="cpython-399"))
+    assert _lib.host_path() != before and _lib.host_path().startswith(os.path.dirname(before)) and _lib.host_path().endswith(".so")
+
+
+def test_native_host_path_is_built_again_after_its_recipe(monkeypatch, tmp_path):
+    from candle_amd import build
+    path, source, recipe = tmp_path / "_host.so", tmp_path / build.HOST_SOURCE, tmp_path / "build.py"
+    for f in (path, source, recipe):
+        f.write_text("")
+    monkeypatch.setattr(build, "CSRC", str(tmp_path))
+    monkeypatch.setattr(build, "__file__", str(recipe))
+    for times, current in (((3, 1, 2), True), ((3, 4, 2), False), ((3, 1, 4), False)):
+        for f, t in zip((path, source, recipe), times):
+            os.utime(f, (t, t))
+        assert build.host_is_current(str(path)) == current
+    path.unlink()
+    assert not build.host_is_current(str(path))
