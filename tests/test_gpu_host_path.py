@@ -103,6 +103,24 @@ def test_the_python_path_takes_what_is_not_ordinary():
     assert torch.equal(got[0], want) and not slot.lock.locked()
 
 
+@pytest.mark.parametrize("fmt", [GgmlDType.Q8_0, GgmlDType.Q4K])
+def test_workspace_of_just_enough_bytes(fmt):
+    """A buffer of the stream that is missing or a byte too small is left to Python, unlocked; one of exactly the bytes that the library asks for is taken, and nothing
+    behind it is written."""
+    w, x = weight(fmt), torch.randn(200, K, device=DEV)
+    want, need = w.fwd(x), _lib.lib().cq_qmatmul_workspace_bytes(int(fmt), 200, K, N)
+    assert need > 1
+    slot, memory = q._Workspace(), torch.full((need + 4096,), 255, dtype=torch.uint8, device=DEV)
+    mine = {(0, torch.cuda.current_stream().cuda_stream): slot}
+    native = lambda: _lib.qmatmul(x, w.storage._data, w.storage._dtype, w._shape, mine)
+    for buf in (None, memory[:need - 1], memory[:0]):
+        slot.buf = buf
+        assert native() is None and not slot.lock.locked()
+    slot.buf = memory[:need]
+    assert torch.equal(native(), want) and not slot.lock.locked() and bool((memory[need:] == 255).all())
+    assert _lib.qmatmul(x, w.storage._data, w.storage._dtype, w._shape, {}) is None
+
+
 def test_threads_share_a_stream():
     """Several threads on one stream: calls of more than one launch do not get between each other's."""
     w = weight()
