@@ -115,7 +115,7 @@ __device__ __forceinline__ void tile_at(int t, int tiles_m, int tiles_n, int &tm
 
 // Tile t of a grouped product's order: all tiles of a group (of those in the same sixteen of the table) side by side, column by column, so that its weights are
 // read once, and then the next group.  (By a fixed number of row tiles, as above, tiles of one group fall to two runs of workgroups: 1500 tokens, 64 experts of which the largest have three
-// times the mean, 1.06 GB come from behind the L2 for 740 MB of weights, and 0.86 so: 263 -> 245 us.)
+// times the mean, 1.05 GB come from behind the L2 for 740 MB of weights, and 0.87 so: 264 -> 247 us.)
 __device__ __forceinline__ void group_tile_at(const Src &s, int t, int tiles_m, int tiles_n, int lane, int &tm, int &tn) {
     const int at = t / tiles_n, base = at & ~15, x = base + (lane & 15);
     const int group = s.tiles[at].group;
@@ -403,8 +403,8 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
 // another launch add them, and each workgroup waits for stages that it has asked for one or three of its own short steps ago.  Here one workgroup has a unit's LDS.
 // Results are those of that tile to the last bit, so that no choice made from them (of a token's experts, say) depends on which of the two a call takes: the same
 // instructions in the order of k, and for a product that would be cut along k (PARTS) one sum per part of k_split, added in order.
-// 2048 x 2048 x 2048, cold weights: 39.5 -> 27.2 us, of which about 7 are the way to the first products and the last sums.  A stage takes 0.62 us, 1490 cycles, of which
-// LDS has work for 1024 (32 KB written, 96 read) and the matrix cores for 512 (192 rows: 1216 and 768); 256 units then take 13.5 TB/s out of the L2s.
+// 2048 x 2048 x 2048, cold weights: 39.5 -> 27.2 us, of which about 7 are the way to the first products and the last sums.  A stage takes 0.62 us.  Of a unit's busy cycles
+// the matrix cores have 40 % (x 7168), reads of LDS 30, and waves wait for 36 % of theirs: for stages, of which 256 units bring 13.4 TB/s out of the L2s and 2.6 from behind.
 // Eight waves, 4 x 2, of BM / 4 x 64 results each: four of BM / 2 x 64 read a third less from LDS, but have a matrix core to themselves and wait more (2048 x 2048 x 2048:
 // 31.0 us; 192 rows: 52 where eight take 33).  LDS holds four stages of 64 of k; copies that no register sees bring them, four ahead of the products, and the operands of
 // half a stage are read while those of the half before are multiplied: one barrier a stage, which waits for nothing that was asked for less than three stages ago.  Rows

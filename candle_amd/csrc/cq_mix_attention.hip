@@ -232,7 +232,7 @@ __global__ __launch_bounds__(64 * NW) void talk_attention_kernel(const float *__
 // so that only the mixing stands between two barriers.
 // LDS rows of 512 bytes in 32 16-byte chunks: keys' chunk c of row r at c ^ r, values as they are; both without bank conflicts.
 // 16 heads in us, above -> this: 2048 rows (window 1024) 327 -> 185, 500: 111 -> 43, 100: 65 -> 30; the error against 64 bits falls (2048 rows 4.9e-7 -> 4.0e-7: scores in two
-// sums).  Bound by the f32 matrix instructions, 68 of 32 cycles a wave and tile, four waves to a matrix core: 63 % of a unit's cycles, the rest barriers and
+// sums).  Bound by the f32 matrix instructions, 68 of 32 cycles a wave and tile, four waves to a matrix core: 62 % of a unit's busy cycles, the rest barriers and
 // the mixing.
 typedef __attribute__((address_space(3))) void talk_lds;
 // The tiles of all blocks of 16 rows form one sequence, of which every workgroup takes `chunk`: the first rows see fewer keys than the last, and equal parts of each block left

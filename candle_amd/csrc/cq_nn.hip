@@ -582,7 +582,8 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(const float *__restrict_
 // order); a maximum is taken across lanes only where a score exceeds the running one.  Values are summed four tiles at a time and the sums then added, as above.
 // The parts of an infinity, and of a finite value that bfloat16 rounds to one, are no numbers, and neither is any result that they reach: a pair with such a result is
 // formed again in f32, from the caches (attn_pair_again).
-// Keys arrive an iteration ahead, values under the first product.  Bound by LDS: four waves read 48 KB a tile each, 1920 cycles with the copies, beside 1536 of products.
+// Keys arrive an iteration ahead, values under the first product.  Of a unit's busy cycles the matrix cores have 41 % (1000 rows; 2048: 46),
+// reads of LDS 22 - 24, and waves wait for 26 - 24 % of theirs: a wave's products, softmax and splitting of its weights follow each other, and two waves share a matrix core.
 // 32 heads, 8 kv heads, us (f32 kernel above -> this, splitting 5 - 20 of it): 300 rows 31 -> 25, 500: 48 -> 35, 1000: 145 -> 73, 2048: 450 -> 216, 300 behind 4000 keys:
 // 406 -> 191.
 constexpr int AT_K = 32, AT_PART = 8192, AT_TILE = 3 * AT_PART;      // keys of a tile; bytes of a part of its keys (or values), of all three

@@ -75,7 +75,7 @@ def test_grouping_at_the_change_of_form(tokens, weights):
 @pytest.mark.parametrize("E,tokens,top,order", [(3, 2048, 3, "tokens"), (3, 2049, 3, "shuffled"), (1024, 700, 2, "tokens"), (1025, 700, 2, "tokens"), (1, 300, 2, "shuffled"),
                                                 (70, 30, 65, "tokens"), (9, 1025, 6, "twice")])
 def test_grouping_of_lists(dtype, E, tokens, top, order):
-    """Lists of pairs at the edges of what a thread takes at a time (6144 pairs), of the experts that get a workgroup each (1024) and of a wave's 64 pairs, in token order
+    """Lists of pairs at the edges of what a thread takes at a time (6144 pairs), of hundreds of experts and of a wave's 64 pairs, in token order
     (a row is quantized once for its pairs), shuffled, and with every entry of the first half listed again in place of one of the second: valid pairs get their
     product, and pairs that name no expert or no token write nothing."""
     import candle_amd as ca
