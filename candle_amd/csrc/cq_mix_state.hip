@@ -199,10 +199,11 @@ __global__ __launch_bounds__(256) void retention_prefix_kernel(Retention a) {
     if (col < a.vdim) st[0] = s;
 }
 
-// Segments of at least `least` chunks: one where the workspace holds their states (8 heads in us, of two chunks -> of one: 2048 rows 56.6 -> 50.6, 1000: 51.4 -> 38.7,
-// 300: 64.5 -> 32.6), else two.
-void retention_plan(int64_t rows, int64_t heads, int64_t vdim, int64_t least, int *nseg, int *seg_len) {
-    const int64_t wg = heads * ((vdim + 63) / 64), chunks = (rows + RC - 1) / RC;
+// Segments of at least two chunks, or of one (`fine`, where the workspace holds their states: 8 heads of 128 in us, of two chunks -> of one: 2048 rows 55.2 -> 48.9, 1000: 52.7 ->
+// 38.0, 300: 64.7 -> 32.6, 100: 36.1 -> 30.9).  Two or three chunks stay one segment where the heads alone are many workgroups, whose states are then neither written nor
+// read (whole / cut to chunks: 64 heads of 64, 100 rows 23.1 / 24.3, 180: 32.0 / 26.0; 128 heads 23.5 / 29.2, 180: 32.1 / 35.8, 200: 40.3 / 35.8; 256 heads, 65: 23.8 / 41.4).
+void retention_plan(int64_t rows, int64_t heads, int64_t vdim, bool fine, int *nseg, int *seg_len) {
+    const int64_t wg = heads * ((vdim + 63) / 64), chunks = (rows + RC - 1) / RC, least = fine && chunks >= (wg <= 48 ? 2 : wg <= 64 ? 3 : 4) ? 1 : 2;
     int64_t n = 512 / wg;
     n = n < chunks / least ? n : chunks / least;
     n = n < 1 ? 1 : n;
@@ -915,7 +916,7 @@ int64_t cq_mix_state_pad(int64_t dim) { return dim > 0 && dim <= CQ_MIX_MAX_DIM 
 int64_t cq_mix_retention_workspace_bytes(int64_t rows, int64_t heads, int64_t dim, int64_t vdim) {
     if (rows <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
     int nseg, seg_len;
-    retention_plan(rows, heads, vdim, 1, &nseg, &seg_len);
+    retention_plan(rows, heads, vdim, true, &nseg, &seg_len);
     return retention_bytes(heads, dim, vdim, nseg);
 }
 
@@ -934,9 +935,9 @@ int cq_mix_retention(const float *q_dev, const float *k_dev, const float *v_dev,
     a.v_stride = v_stride; a.out_stride = out_stride;
     a.rows = (int)rows; a.heads = (int)heads; a.dp = (int)dim_pad; a.vdim = (int)vdim; a.sp = (int)cq_mix_state_pad(dim);
     a.nvb = (a.vdim + 63) / 64;
-    retention_plan(rows, heads, vdim, 1, &a.nseg, &a.seg_len);
+    retention_plan(rows, heads, vdim, true, &a.nseg, &a.seg_len);
     if (!workspace_dev || workspace_bytes < retention_bytes(heads, dim, vdim, a.nseg)) {
-        retention_plan(rows, heads, vdim, 2, &a.nseg, &a.seg_len);
+        retention_plan(rows, heads, vdim, false, &a.nseg, &a.seg_len);
         if (a.nseg > 1 && (!workspace_dev || workspace_bytes < retention_bytes(heads, dim, vdim, a.nseg))) return CQ_ERR_WORKSPACE;
     }
     hipStream_t s = (hipStream_t)stream;

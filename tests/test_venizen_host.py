@@ -180,6 +180,14 @@ def test_sequence_cache_keeps_states_in_order():
     only_kv.begin(1)                             # caches written by position may move back
 
 
+@pytest.mark.parametrize("heads,vdim,rows,segments", [(8, 128, 64, 1), (8, 128, 65, 2), (48, 64, 128, 2), (64, 64, 128, 1), (64, 64, 129, 3), (32, 128, 128, 1), (128, 64, 192, 1),
+                                                      (128, 64, 193, 4), (256, 64, 65, 1), (256, 64, 192, 1), (256, 64, 193, 2)])
+def test_retention_cuts_short_calls_only_where_that_pays(heads, vdim, rows, segments):
+    """The workspace holds a state per segment of a call that is cut: calls of a few chunks of 64 are not where the heads alone are many workgroups."""
+    blocks = (vdim + 63) // 64
+    assert _lib.mixer_lib().cq_mix_retention_workspace_bytes(rows, heads, 64, vdim) == (heads * blocks * segments * 64 * 64 * 4 if segments > 1 else 0)
+
+
 def test_mixer_argument_validation_codes_without_gpu():
     L = _lib.mixer_lib()
     OK, DTYPE, SHAPE, ALIGN, NULL, WS, RANGE = 0, -1, -2, -3, -4, -5, -6
