@@ -529,7 +529,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float *__restrict
 // A decay is at least exp(-exp(-1/2)) = 0.545, so W stays above 6e-5; it and the four products of rows are formed in 64 bits and rounded once, which leaves the
 // error of the whole against 64 bits where that of the scan is (2-norm, 32 heads of 64, 64 - 2048 tokens: outputs 1.20 - 1.33e-7 against 1.20 - 1.41e-7, states 1.00 -
 // 1.18e-7 against 1.03 - 1.30e-7).
-// 32 heads of 64 in us, packing and scan -> chunks and chain: 2048 tokens 25 + 223 -> 40 + 70, 200: 31.6 -> 21.1, 32: 14.1 -> 10.4; 16 heads, 1500 tokens 177 -> 71.
+// 32 heads of 64 in us, packing and scan -> chunks and chain: 2048 tokens 25 + 223 -> 40 + 70, 256: 37.1 -> 23.4, 100: 18.0 -> 14.3; 16 heads, 1500 tokens 177 -> 71.
 // The chunks are bound by the bytes of rows and records (64 + 89 MB of 2048 tokens) and the latencies between four barriers, with five workgroups on a CU; the chain
 // by the latencies of a chunk: eight products in a row (8 x 32 cycles) and a way through LDS.
 constexpr int KC = 16, KLD = 68;                     // chunk length; LDS row of 64 dimensions
@@ -831,9 +831,10 @@ __global__ __launch_bounds__(512, 2) void delta_chain_kernel(const float *__rest
     if (16 * cb + lr < dim) *reinterpret_cast<f32x4 *>(st) = s;
 }
 
-// Chunks from two whole ones on (10.4 us against 14.1 at 32 tokens), for heads of at most 64 dimensions: their operators have 64 rows.
-constexpr int64_t DELTA_MIN_ROWS = 32;
-bool delta_chunked(int64_t rows, int64_t heads, int64_t dim) { return dim <= 64 && heads <= 65535 && rows >= DELTA_MIN_ROWS; }
+// Chunks for heads of at most 64 dimensions (their operators have 64 rows) and from so many tokens on that they take no longer than packing and scan, whose time grows by the
+// token: with more heads a chunk's work fills the chip and shows (us, packing and scan / chunks: 32 heads of 64, 32 tokens 8.2 / 10.0, 48: 10.5 / 11.1, 56: 12.2 / 11.9,
+// 64 heads, 56: 13.6 / 13.2; 128 heads, 64: 18.9 / 19.0, 96: 25.8 / 23.0; 200 heads of 16, 64: 19.5 / 22.1, 96: 25.5 / 24.8; 400 heads of 16, 128: 41.3 / 43.7, 256: 73.3 / 73.0).
+bool delta_chunked(int64_t rows, int64_t heads, int64_t dim) { return dim <= 64 && heads <= 65535 && rows >= (heads <= 64 ? 56 : heads <= 200 ? 96 : 256); }
 
 struct DeltaStep {
     const float *row, *w0, *ab, *weight;

@@ -496,7 +496,7 @@ def test_general_delta_rows(H, d, kind):
 def test_general_delta_long_calls(H, d):
     """Chunks in every remainder of four, whole and cut last ones, many of them, and several workgroups to a unit: what the waves of a workgroup hand to each other
     chunk by chunk is there when it is read, and still there.  The same bounds, the rule in 64 bits on the GPU."""
-    L, W, spd, cuts = _lib.mixer_lib(), H * d, _lib.mixer_lib().cq_mix_state_pad(d), (129, 145, 161, 177, 96, 1501)
+    L, W, spd, cuts = _lib.mixer_lib(), H * d, _lib.mixer_lib().cq_mix_state_pad(d), (129, 145, 161, 177, 96, 56, 57, 63, 64, 65, 1501)
     T = sum(cuts)
     g = torch.Generator(device=DEV).manual_seed(H + d)
     rnd_dev = lambda *s: torch.randn(s, generator=g, device=DEV)

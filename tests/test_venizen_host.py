@@ -180,6 +180,15 @@ def test_sequence_cache_keeps_states_in_order():
     only_kv.begin(1)                             # caches written by position may move back
 
 
+@pytest.mark.parametrize("heads,dim,rows,chunked", [(32, 64, 32, False), (32, 64, 55, False), (32, 64, 56, True), (64, 8, 56, True), (65, 64, 95, False), (65, 64, 96, True),
+                                                    (200, 16, 96, True), (201, 16, 255, False), (201, 16, 256, True), (8, 65, 4096, False)])
+def test_delta_rule_goes_by_chunks_only_where_that_pays(heads, dim, rows, chunked):
+    """The workspace tells: records of chunks of 16 tokens, or the packed vectors of the scan."""
+    L = _lib.mixer_lib()
+    records, packed = (rows + 15) // 16 * heads * (5 * 1024 + 64 + 256) * 4, rows * heads * (4 * L.cq_mix_state_pad(dim) + 1) * 4
+    assert L.cq_mix_delta_rows_workspace_bytes(rows, heads, dim) == (records if chunked else packed)
+
+
 @pytest.mark.parametrize("heads,vdim,rows,segments", [(8, 128, 64, 1), (8, 128, 65, 2), (48, 64, 128, 2), (64, 64, 128, 1), (64, 64, 129, 3), (32, 128, 128, 1), (128, 64, 192, 1),
                                                       (128, 64, 193, 4), (256, 64, 65, 1), (256, 64, 192, 1), (256, 64, 193, 2)])
 def test_retention_cuts_short_calls_only_where_that_pays(heads, vdim, rows, segments):
