@@ -571,7 +571,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(const float *__restrict_
     }
 }
 
-// The prompt's attention from 256 keys on (attn_by_planes): the two products on the bf16 matrix cores, from operands split into three bf16 parts that add up to the
+// The prompt's attention beyond 256 keys (attn_by_planes): the two products on the bf16 matrix cores, from operands split into three bf16 parts that add up to the
 // f32 value (8 + 8 + 8 bits).  Of the nine products of parts the six above 2^-24 of the whole are formed, the scores' small ones apart from the
 // large one; sums are f32.  Six times 16 cycles for 16 x 16 x 32 stand against 8 x 32 of the f32 instruction, which bounds the kernel above; the error against 64 bits
 // is half of that kernel's, which rounds four keys or dimensions at a time (2-norm, 1000 rows: 1.64e-7 against 3.35e-7; scores four times as large 4.3e-7, 1.03e-6).
@@ -1607,10 +1607,10 @@ int launch_attn_mfma(int G, dim3 grid, hipStream_t s, const float *q, int64_t q_
     return (int)hipGetLastError();
 }
 
-// From 256 keys on the split operands win back what splitting them costs (300 rows: 25 us against 31, 64 rows behind 1000 keys: 59 against 69; 200 rows: 21.1 against
-// 19.1); they lie in the workspace that partial results would take, which holds them from 95 rows of four heads per kv head on.  (2^20 keys: offsets of 32 bits.)
+// Beyond 256 keys, two of the f32 kernel's splits, the split operands win back what splitting them costs (257 rows: 25.3 us against 29.0, 64 rows behind 1000 keys: 58 against
+// 78; 256 rows: 22.5 against 20.2, 200: 21.1 against 19.1); they lie in the workspace that partial results would take, which holds them from 95 rows of four heads per kv head on.  (2^20 keys: offsets of 32 bits.)
 bool attn_by_planes(int64_t n_kv, int64_t max_kv_len, const void *workspace, int64_t workspace_bytes) {
-    return max_kv_len >= 256 && max_kv_len <= (1 << 20) && !misaligned(workspace, 16) && workspace_bytes >= n_kv * ((max_kv_len + AT_K - 1) / AT_K) * 2 * AT_TILE;
+    return max_kv_len > 256 && max_kv_len <= (1 << 20) && !misaligned(workspace, 16) && workspace_bytes >= n_kv * ((max_kv_len + AT_K - 1) / AT_K) * 2 * AT_TILE;
 }
 
 int launch_attn_planes(int G, hipStream_t s, const float *q, int64_t q_stride, const float *kc, const float *vc, float *out, const int32_t *pos_dev, int pos0, int rows,

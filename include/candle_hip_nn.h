@@ -52,7 +52,7 @@ int cq_nn_rope_i_kv(float *q_dev, const float *k_dev, const float *v_dev, float 
 /* Causal grouped-query attention of `rows` new queries over the cache (quantized_llama.rs:246-261:
  * repeat_kv, q k^T / sqrt(d), mask, softmax_last_dim, . v, transpose back to [rows, n_head*head_dim]).
  * Query row r attends keys [0, pos + *pos_dev + r].  max_kv_len bounds pos + *pos_dev + rows and fixes
- * the launch geometry (keys are processed in splits of 128; more than one split needs the workspace).  64 rows and more of head_dim 128 with max_kv_len >= 256
+ * the launch geometry (keys are processed in splits of 128; more than one split needs the workspace).  64 rows and more of head_dim 128 with max_kv_len > 256
  * are computed from split operands that lie in the workspace if it is 16-byte aligned and holds ceil(max_kv_len / 32) * n_kv_head * 49152 bytes (f32 matrix
  * instructions otherwise: other last bits).
  * head_dim 64 or 128; n_head / n_kv_head in {1, 2, 4, 8}. */

@@ -152,7 +152,7 @@ def test_attention_prompt_split_operands(H, KV, rows, pos, max_kv):
         got.append(out.cpu().numpy())
         assert got[-1][0] == 7.0 and got[-1][-1] == 7.0
         assert rel_l2(got[-1][1:-1].reshape(rows, H * D), want) <= TOL
-    assert np.array_equal(got[0], got[1]) == (max_kv < 256 or need >= fits)
+    assert np.array_equal(got[0], got[1]) == (max_kv <= 256 or need >= fits)
 
 
 def test_attention_prompt_split_operands_of_all_sizes():
