@@ -114,14 +114,14 @@ __global__ __launch_bounds__(256) void layer_norm_rows_kernel(const float *__res
 }
 
 // sum over n = 1..3 of coef[n-1] z^n / rms(z^n), plus coef[3]: one workgroup per row.  The bound is memory: the first KEEP * 256 values are requested together and
-// stay in registers between the three sums and the result, so that a row is read once.
-template <typename T>
+// stay in registers between the three sums and the result, so that a row is read once.  KEEP follows the row: a thread goes through all of them, there or not (4096 rows of
+// 256: 12.1 us with 32, 5.8 with 4; 2048 rows of 2048: 8.7 with 32, 6.3 with 8).
+template <int KEEP, typename T>
 __global__ __launch_bounds__(256) void poly_norm_kernel(const float *z, int64_t z_stride, const float *__restrict__ coef, T *out, int64_t out_stride,
                                                         int dim, float eps) {
     __shared__ float red[4];
     const float *zr = z + (int64_t)blockIdx.x * z_stride;
     T *o = out + (int64_t)blockIdx.x * out_stride;
-    constexpr int KEEP = 32;
     float keep[KEEP], s2 = 0.0f, s4 = 0.0f, s6 = 0.0f;
     auto count = [&](float v) {
         const float q = v * v;
@@ -271,7 +271,8 @@ int poly_norm(const float *z, int64_t z_stride, const float *coef, T *out, int64
     if (rows == 0) return CQ_OK;
     if (!z || !coef || !out) return CQ_ERR_NULL;
     if (rows > 0x7fffffffLL || dim > (1 << 24)) return CQ_ERR_RANGE;
-    hipLaunchKernelGGL(poly_norm_kernel<T>, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, z, z_stride, coef, out, out_stride, (int)dim, eps);
+    auto *const fn = dim <= 4 * 256 ? poly_norm_kernel<4, T> : dim <= 8 * 256 ? poly_norm_kernel<8, T> : dim <= 16 * 256 ? poly_norm_kernel<16, T> : poly_norm_kernel<32, T>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, z, z_stride, coef, out, out_stride, (int)dim, eps);
     return (int)hipGetLastError();
 }
 

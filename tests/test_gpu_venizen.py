@@ -116,6 +116,16 @@ def test_row_norms(dim):
     assert rel(out[:, :dim], np.tanh(s)) < 1e-6
 
 
+@pytest.mark.parametrize("dim", [1, 255, 257, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193])
+def test_poly_norm_at_the_lengths_that_threads_keep(dim):
+    """Rows on either side of 4, 8, 16 and 32 values a thread, in place."""
+    L, ld, rows = _lib.mixer_lib(), dim + 3, 70
+    z, coef = rnd(1, rows, dim), np.array([0.5, -0.7, 0.9, -0.2], dtype=np.float32)
+    zd = up(padded(z, ld))
+    _lib.check("p", L.cq_mix_poly_norm(zd.data_ptr(), ld, ptr(coef), zd.data_ptr(), ld, rows, dim, EPS, sp()))
+    assert rel(zd[:, :dim], vo.poly_norm(z.astype(np.float64), coef.astype(np.float64), EPS)) < 3e-6 and not zd[:, dim:].any()
+
+
 @pytest.mark.parametrize("kind,weight", [(mixers.SILU, False), (mixers.SIGMOID, True)])
 @pytest.mark.parametrize("heads,dim", [(1, 5), (3, 64), (5, 200)])
 def test_head_norm_gate(heads, dim, kind, weight):
