@@ -6,27 +6,23 @@
 // 13 bits, so it goes through the int8 cores as two operands in two chains: Q4_K as scale % 8 * q and scale / 8 * q (S = lo + 8 hi), Q5_K and Q6_K as the
 // low byte less 128 and the high byte of scale * q + 128 (S = lo + 256 hi).
 //
-// What bounds it: at many rows matrix and vector instructions together, at the 1.9 GHz that the power limit leaves.  Of the SIMDs' cycles at 2048 rows the matrix
-// cores take 39 % with Q4_K and 35 % with Q5_K and Q6_K (16 + 1 MFMAs of 32 x 32 x 32 per 32 rows, super-block and wave), the vector units 43, 55 and 54 %
-// (conversion, and the sums of a super-block), and the two waves of a SIMD overlap them only in part.  At few rows the weights' way from memory, and
-// in unsplit small products the chain of one wave a SIMD.  So:
-//  - a workgroup is eight waves (or four: qtile_plan) side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
-//    multiplies it, straight into its operand registers (the kernels before this one staged converted weights in LDS, and the conversion
-//    of Q5_K and Q6_K was to f16, Q6_K as two f16 terms: twice the matrix time of int8);
-//  - weights go by copies to LDS into a ring of the wave's own, three stages of 64 elements ahead, with counted waits and no barrier; activations into a ring of
-//    three super-blocks shared by the workgroup, one barrier per super-block.  Q6_K blocks begin on 2 bytes: its pieces are brought from the dword below and
-//    shifted on reading, two half super-blocks at a time;
-//  - waves 4 - 7 (the second on each SIMD) run half a super-block behind, so that the vector work at the end of a super-block lies under the other wave's
-//    matrix work (Q6_K gains nothing from it and does without);
-//  - fragments, conversions and products of one step are interleaved by hand, the sums of a tile pinned before the next one's: left to itself the
-//    scheduler spills.
+// A workgroup is eight waves (or four: qtile_plan) side by side along n that share 32 MI rows of activations: each weight is converted once, by the one wave that
+// multiplies it, straight into its operand registers.  Weights go by copies to LDS, into a ring of the wave's own, with counted waits; activations into a ring
+// shared by the workgroup, one barrier per super-block.  Two kernels: qtile_kernel interleaves the conversion of one step with the products of the step before and scales the sums of
+// all tiles at the end of a super-block (Q4_K, Q5_K, tiles of up to 64 rows); qtile_wide_kernel converts a whole super-block and then multiplies it tile by tile.
+//
+// What bounds it: at many rows the power limit.  With all units busy the clock falls to 1.65 - 1.9 GHz (the int8 cores alone, on random operands, run at 1.65: 3300 TOP/s);
+// on an eighth of the units, or on zeros, the same workgroups take 185 us where they take 260 (Q4_K, 2048 rows of [4096 x 14336]).  In those 7900 cycles per super-block and pair of
+// waves the matrix cores are busy 4350; a matrix instruction also keeps the vector unit from issuing for ten cycles, whatever its shape, so that half as many of 32 x 32 x 32 leave it
+// more room than of 16 x 16 x 64 (282 us for 262).  At few rows the weights' way from memory, and in unsplit small products the chain of one wave a SIMD.
 // f16 / bf16 results are written by the product; the f32 copy and its conversion went (12 us of 154 for 512 rows of Q5_K).
 //
-// [4096 x 14336], us, before / now, quantizing the activations included:    17 rows   131 rows   512 rows   2048 rows
-//   Q4_K                                                                  20.9 18.3  59.3 45.2  113 95.5   386 305
-//   Q5_K                                                                  38.4 21.8  80.3 50.1  160 103    559 324
-//   Q6_K                                                                  38.8 28.6  87.0 55.5  175 112    619 368
-// 2048 rows of Q4_K are 790 TOP/s of products asked for and 1580 done.
+// [4096 x 14336], us, with Q4_K and Q5_K of 96- and 128-row tiles and Q6_K in qtile_kernel / now, quantizing the activations included:
+//              17 rows   131 rows   512 rows   2048 rows
+//   Q4_K     19.0 18.9  45.6 42.1  96.4 90.3   318 294
+//   Q5_K     22.5 22.5  50.6 48.1   105 100    375 361
+//   Q6_K     29.0 26.7  57.4 48.4   116 101    393 356
+// 2048 rows of Q4_K are 900 TOP/s of products asked for and 1800 done.
 #include "cq_qtile.h"
 
 #include <algorithm>
@@ -50,6 +46,9 @@ __device__ __forceinline__ uint32_t qt_pk_mad(uint32_t a, uint32_t b, uint32_t c
     return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
 }
 
+// the high bytes of both halves
+__device__ __forceinline__ uint32_t qt_pk_high(uint32_t a) { return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) >> 8)); }
+
 // The lane's number, worked out where it is asked for (what follows from threadIdx.x is kept in registers over the whole main loop, which needs all of them).
 __device__ __forceinline__ int qt_lane() {
     int l = 0;
@@ -64,25 +63,18 @@ __device__ __forceinline__ int qt_lane() {
 template <int DT> struct QTile;
 template <> struct QTile<CQ_Q4K> {
     static constexpr int EXTRA = 1, HI = 8, QS = 16;
-    static constexpr bool HAS_MIN = true;
 };
 template <> struct QTile<CQ_Q5K> {
     static constexpr int EXTRA = 2, HI = 256, QS = 48;
-    static constexpr bool HAS_MIN = true;
 };
 
-// Q6_K blocks (210 bytes) begin on 2 bytes: a lane brings the four dwords that its 16 bytes begin in and, separately, the one after them.
-// Its ring holds two half super-blocks of three pieces (ql[0 .. 31], ql[32 .. 63], qh of the half), and a piece of the scales with d behind them.
-template <> struct QTile<CQ_Q6K> {
-    static constexpr int EXTRA = 0, HI = 256, QS = 0;
-    static constexpr bool HAS_MIN = false;
-};
-
+// Weights: three stages of 64 elements ahead; activations: three super-blocks.  Waves 4 - 7 (the second on each SIMD) run half a super-block behind, so that the vector work at the
+// end of a super-block lies under the other wave's matrix work.  Fragments, conversions and products of one step are interleaved by hand, the sums of a tile pinned before the
+// next one's: left to itself the scheduler spills.
 constexpr int QT_R = 4, QT_L = QT_R - 1;                 // stages (64 elements) in a wave's ring of weights, stages requested ahead
 // RA: super-blocks in the ring of activations
 template <int DT, int MI, int NW> struct QtLds {
-    static constexpr int PIECE = 1024 + 256, RA = DT == CQ_Q6K ? 2 : 3;
-    static constexpr int A = MI * 8192, B = DT == CQ_Q6K ? 7 * PIECE : 1024 * (QT_R + QTile<DT>::EXTRA), AM = QTile<DT>::HAS_MIN ? MI * 1024 : 0, D8 = (MI + 1) / 2 * 256;
+    static constexpr int RA = 3, A = MI * 8192, B = 1024 * (QT_R + QTile<DT>::EXTRA), AM = MI * 1024, D8 = (MI + 1) / 2 * 256;
     static constexpr int A_OFF = 0, B_OFF = RA * A, AM_OFF = B_OFF + NW * B, D8_OFF = AM_OFF + RA * AM, BYTES = D8_OFF + RA * D8;
 };
 
@@ -113,9 +105,8 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     // ---- weights: rows past the end repeat the last one (their results are not stored) ----
     const int wbase = min(n0, n - 1);
     const uint8_t *const wrow = w + wbase * row_bytes;
-    const uint32_t w_odd = DT == CQ_Q6K ? (uint32_t)(uintptr_t)wrow & 2u : 0u;       // (the descriptor begins on a dword)
-    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(wrow - w_odd), 0, -1, 0x00020000);
-    const uint32_t w_off = (uint32_t)(min(nr, n - 1 - wbase) * row_bytes) + 16 * kg + w_odd;
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)wrow, 0, -1, 0x00020000);
+    const uint32_t w_off = (uint32_t)(min(nr, n - 1 - wbase) * row_bytes) + 16 * kg;
     // ---- activations: 64 bytes of 16 rows per instruction, piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
     // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + NW i of its 8 MI KB)
     const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
@@ -128,31 +119,14 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     }
     uint8_t *const myB = lds + LD::B_OFF + wv * LD::B;
     // ---- scales and 16-element sums of the activations: the first half of the waves brings the sums of 32 rows each, the others the scales of 64 ----
-    const bool x_sums = T::HAS_MIN && wv < NW / 2;
+    const bool x_sums = wv < NW / 2;
     const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = min(x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane, rows - 1 - m0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         x_sums ? (void *)(av.bsums + (int64_t)m0 * (k >> 4)) : (void *)(av.d + (int64_t)m0 * nsb_all), 0, -1, 0x00020000);
     const uint32_t x_off = x_sums ? (uint32_t)x_r * (uint32_t)(32 * nsb_all) + 16 * (lane & 1) : (uint32_t)x_r * (uint32_t)(4 * nsb_all);
     // weights of stage u = 4 (kb - kb0) + q into slot q of this wave's ring; past the end the last super-block again, into slots nobody reads
-    // (Q6_K: half q of the super-block)
     auto issue_w = [&](int kb, int q) {
         kb = min(kb, kb1 - 1);
-        if constexpr (DT == CQ_Q6K) {
-            const int at0 = kb * BB & ~3;                  // (210 kb is 2 past a dword for odd kb, and so are odd rows of an odd number of blocks)
-            const uint32_t off = (w_off + (uint32_t)(kb * BB & 2)) & ~2u;
-            auto piece = [&](int at, int slot) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::PIECE), 16, off, at0 + at, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::PIECE + 1024), 4, off, at0 + at + 16, 0, 0);
-            };
-            piece(64 * q, 3 * q);
-            piece(64 * q + 32, 3 * q + 1);
-            piece(128 + 32 * q, 3 * q + 2);
-            if (q == 0) {                                  // scales and d, for both halves of the wave
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 6 * LD::PIECE), 16, off - 16 * kg, at0 + 192, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 6 * LD::PIECE + 1024), 4, off - 16 * kg, at0 + 208, 0, 0);
-            }
-            return;
-        }
         if (q == 0) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 1024 * QT_R), 16, w_off, kb * BB, 0, 0);      // (the upper lanes bring the 16 bytes behind it)
             if constexpr (EX == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + 1024 * (QT_R + 1)), 16, w_off, kb * BB + 16, 0, 0);
@@ -183,11 +157,11 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     issue_x(0, 0);
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int t = 0; t < (DT == CQ_Q6K ? 1 : QT_L); t++) issue_w(kb0, t);
+    for (int t = 0; t < QT_L; t++) issue_w(kb0, t);
     const int nsb = kb1 - kb0;
     const int live = MOE ? (rows - m0 + 31) / 32 : MI;     // 32-row tiles that hold rows: an expert rarely fills its last ones
 
-    constexpr bool STAGGER = DT != CQ_Q6K && NW == 8;      // (four waves have a SIMD each)
+    constexpr bool STAGGER = NW == 8;      // (four waves have a SIMD each)
     auto body = [&](auto late) {
     constexpr bool LATE = decltype(late)::value;
     int slot = 0, slot1 = 1;                               // ring slots of super-blocks j and j + 1
@@ -196,21 +170,13 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
         issue_x(j1, sl1);
         asm volatile("" ::: "memory");
     };
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(DT == CQ_Q6K ? 0 : QT_L + EX) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(QT_L + EX) : "memory");
     if constexpr (LATE) request(1, 1);
     u32x4 hdr = u32x4{0, 0, 0, 0}, qh = u32x4{0, 0, 0, 0}, raw;
-    uint32_t shift = 0, d6 = 0;                            // Q6_K: bytes by which this super-block's pieces are off their dwords; d
     i32x4 af[MI], bl, bh;
     // operands of step s = 2 q + ks (32 elements): dword i of this lane's weights, tile t of the activations
     uint32_t m_lo, m_hi;
     auto scales = [&](int s) {
-        if constexpr (DT == CQ_Q6K) {
-            // int8 scale of the 16 elements 32 s + 16 kg (hdr is shifted by kg bytes)
-            const int sc = (int)(hdr[s >> 1] << (24 - 16 * (s & 1))) >> 24;
-            m_lo = __builtin_amdgcn_perm(0, (uint32_t)sc, 0x01000100u);
-            m_hi = __builtin_amdgcn_perm(0, (uint32_t)(128 - 32 * sc), 0x01000100u);
-            return;
-        }
         // 6-bit scale of sub-block s (utils.rs:50-60)
         const int sft = 8 * (s & 3);
         const uint32_t sc = s < 4 ? (hdr.y >> sft) & 63u : ((hdr.w >> sft) & 0xFu) | (((hdr.y >> sft) >> 2) & 0x30u);
@@ -218,14 +184,6 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
         else m_lo = sc * 0x00010001u;
     };
     auto convert = [&](int s, int i, i32x4 &lo, i32x4 &hi) {
-        if constexpr (DT == CQ_Q6K) {
-            // sc (q - 32) + 128 in 16 bits: high byte, and low byte less 128
-            const uint32_t v6 = ((s & 2 ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu) | (((qh[i] >> (2 * (s & 3))) & 0x03030303u) << 4);
-            const uint32_t e = qt_pk_mad(v6 & 0x00ff00ffu, m_lo, m_hi), o = qt_pk_mad((v6 >> 8) & 0x00ff00ffu, m_lo, m_hi);
-            lo[i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
-            hi[i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
-            return;
-        }
         uint32_t v = (s & 1 ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu;
         if constexpr (DT == CQ_Q4K) {
             lo[i] = (int)qt_pk_mul(v, m_lo);
@@ -241,46 +199,20 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     const int a_x0 = 16 * (kg ^ ((nr >> 2) & 3)), a_x1 = a_x0 ^ 32;
     auto a_frag = [&](int s, int t) { return *reinterpret_cast<const i32x4 *>(a_lane + slot * LD::A + (s >> 1) * (MI * 2048) + t * 2048 + (s & 1 ? a_x1 : a_x0)); };
     auto weights = [&](int q) { return *reinterpret_cast<const u32x4 *>(myB + 1024 * q + 16 * lane); };
-    // Q6_K: a piece, moved onto its dwords
-    auto piece6 = [&](int slot, uint32_t *last) {
-        u32x4 v = *reinterpret_cast<const u32x4 *>(myB + slot * LD::PIECE + 16 * lane);
-        const uint32_t behind = *reinterpret_cast<const uint32_t *>(myB + slot * LD::PIECE + 1024 + 4 * lane);
-#pragma unroll
-        for (int i = 0; i < 3; i++) v[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], shift);
-        v[3] = __builtin_amdgcn_alignbyte(behind, v[3], shift);
-        if (last) *last = behind >> (8 * shift);
-        return v;
-    };
-    auto weights6 = [&](int s) {                           // of step s
-        raw = piece6(3 * (s >> 2) + (s & 1), nullptr);
-        qh = piece6(3 * (s >> 2) + 2, nullptr);
-    };
     // what this wave has requested behind its weights of stage q when it asks for them
     constexpr int NX = NA + 1, W0[4] = {2, 2 + NX, 2 + NX + EX, 2 + EX}, W1[4] = {2 + NX, 2, 2 + EX, 2 + EX + NX};
     for (int j = 0; j < nsb; j++) {
         const int kb = kb0 + j;
         // ---- first step of a super-block: nothing of it is in registers yet ----
-        if constexpr (DT == CQ_Q6K) {
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LATE ? W1[0] : W0[0]) : "memory");
+        if constexpr (!LATE) {
             if (j > 0) asm volatile("s_barrier" ::: "memory");
-            issue_w(kb, 1);
             request(j + 1, slot1);
-            shift = (w_off + (uint32_t)(kb * BB)) & 2u;
-            hdr = piece6(6, &d6);
-#pragma unroll
-            for (int i = 0; i < 4; i++) hdr[i] >>= 8 * kg;
-            weights6(0);
-        } else {
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LATE ? W1[0] : W0[0]) : "memory");
-            if constexpr (!LATE) {
-                if (j > 0) asm volatile("s_barrier" ::: "memory");
-                request(j + 1, slot1);
-            }
-            issue_w(kb, 3);
-            hdr = *reinterpret_cast<const u32x4 *>(myB + 1024 * QT_R + 16 * (qt_lane() & 31));
-            if constexpr (EX == 2) qh = *reinterpret_cast<const u32x4 *>(myB + 1024 * (QT_R + 1) + 16 * lane);
-            raw = weights(0);
         }
+        issue_w(kb, 3);
+        hdr = *reinterpret_cast<const u32x4 *>(myB + 1024 * QT_R + 16 * (qt_lane() & 31));
+        if constexpr (EX == 2) qh = *reinterpret_cast<const u32x4 *>(myB + 1024 * (QT_R + 1) + 16 * lane);
+        raw = weights(0);
 #pragma unroll
         for (int t = 0; t < MI; t++) af[t] = a_frag(0, t);
         scales(0);
@@ -290,11 +222,7 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
         for (int s = 0; s < 8; s++) {
             const int q = s >> 1, ns = s + 1;
             i32x4 nl, nh;
-            if constexpr (DT == CQ_Q6K) {
-                if (s == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NX) : "memory");
-                if (s == 4) issue_w(kb + 1, 0);
-                if (ns < 8) weights6(ns);
-            } else if (s & 1) {
+            if (s & 1) {
                 if (q < 3) {
                     // the weights of the next stage, and a request for those three stages on
                     if (q == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATE ? W1[1] : W0[1]) : "memory");
@@ -334,37 +262,30 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
             }
             if (ns < 8) { bl = nl; bh = nh; }
             if (s == 7) {
-                const float d = h2f(DT == CQ_Q6K ? d6 : hdr.x), dmin = h2f(hdr.x >> 16);
-                half8 bm;
-                if (T::HAS_MIN) {
-                    const uint32_t mlo = hdr.z & 0x3f3f3f3fu, mhi = ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u);
-                    const uint32_t kmask = 0u - (uint32_t)(qt_lane() >> 5), mine = (mhi & kmask) | (mlo & ~kmask);
-                    u32x4 mv;
+                const float d = h2f(hdr.x), dmin = h2f(hdr.x >> 16);
+                const uint32_t mlo = hdr.z & 0x3f3f3f3fu, mhi = ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u);
+                const uint32_t kmask = 0u - (uint32_t)(qt_lane() >> 5), mine = (mhi & kmask) | (mlo & ~kmask);
+                u32x4 mv;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) mv[i] = qt_pk_add((0x6400u | ((mine >> (8 * i)) & 0xffu)) * 0x00010001u, 0xe400e400u);
-                    bm = __builtin_bit_cast(half8, mv);
-                }
+                for (int i = 0; i < 4; i++) mv[i] = qt_pk_add((0x6400u | ((mine >> (8 * i)) & 0xffu)) * 0x00010001u, 0xe400e400u);
+                const half8 bm = __builtin_bit_cast(half8, mv);
 #pragma unroll
                 for (int t = 0; t < MI; t++) {
                     if (MOE && t >= live) break;
                     __builtin_amdgcn_sched_barrier(0);
-                    f32x16 mt;
-                    if (T::HAS_MIN) {
-                        const s16x8 ai = *reinterpret_cast<const s16x8 *>(lds + LD::AM_OFF + slot * LD::AM + (t * 32 + nr) * 32 + 16 * kg);
-                        const half8 am = __builtin_convertvector(ai, half8);       // sums of 16 int8: exact
-                        f32x16 z;
+                    const s16x8 ai = *reinterpret_cast<const s16x8 *>(lds + LD::AM_OFF + slot * LD::AM + (t * 32 + nr) * 32 + 16 * kg);
+                    const half8 am = __builtin_convertvector(ai, half8);           // sums of 16 int8: exact
+                    f32x16 z;
 #pragma unroll
-                        for (int e = 0; e < 16; e++) z[e] = 0.0f;
-                        mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
-                    }
+                    for (int e = 0; e < 16; e++) z[e] = 0.0f;
+                    const f32x16 mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, z, 0, 0, 0);
 #pragma unroll
                     for (int e4 = 0; e4 < 4; e4++) {
                         const f32x4 d8 = *reinterpret_cast<const f32x4 *>(lds + LD::D8_OFF + slot * LD::D8 + 4 * (t * 32 + 8 * e4 + 4 * kg));
 #pragma unroll
                         for (int e1 = 0; e1 < 4; e1++) {
                             const int e = 4 * e4 + e1;
-                            float v = d * (float)(T::HI * sh[t][e] + sl[t][e]);
-                            if (T::HAS_MIN) v = fmaf(-dmin, mt[e], v);
+                            const float v = fmaf(-dmin, mt[e], d * (float)(T::HI * sh[t][e] + sl[t][e]));
                             acc[t][e] = fmaf(d8[e1], v, acc[t][e]);
                         }
                     }
@@ -381,6 +302,313 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     else if (wv < NW / 2) body(std::false_type{});
     else body(std::true_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    const int lane_out = qt_lane();
+    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
+#endif
+}
+
+// ---- the kernel of tiles of 96 and 128 rows (Q6_K: of all) ----------------------------------------------------------------------------------
+// A wave converts all weights of a super-block into registers, then multiplies 32 rows at a time: sixteen matrix instructions on two chains, under which the sums of the 32 rows before are
+// scaled and added.  Per tile only 32 registers of int32 sums and 32 of scaled ones are alive instead of 32 MI, which is what makes room for the operands.  The second wave of a SIMD
+// meets at the barrier before its conversion, the first behind it: one converts while the other multiplies.  (All of the conversion interleaved with the products of the last and first
+// tile instead, whichever wave: Q6_K 327 us for 271 of 2048 rows, since the vector work of a wave then waits behind matrix instructions that wait for the other wave's.  Products without any
+// vector work between them, and a raised priority for the wave that is among them: no difference.)
+// Tiles without rows are left out, of experts and of the end of a prompt.  Integers, and the order of the f32 sums, are those of qtile_kernel: the same bits.
+//
+// Blocks of a row as they lie in memory: PIECES 16-byte pieces, the quants from piece QS on (Q6_K: 13 pieces and the dword behind them, from the dword that the block
+// begins in).  HI: factor of the hi chain.
+template <int DT> struct QWide;
+template <> struct QWide<CQ_Q4K> {
+    static constexpr int PIECES = 9, QS = 1, HI = 8;
+    static constexpr bool HAS_MIN = true;
+};
+template <> struct QWide<CQ_Q5K> {
+    static constexpr int PIECES = 11, QS = 3, HI = 256;
+    static constexpr bool HAS_MIN = true;
+};
+template <> struct QWide<CQ_Q6K> {
+    static constexpr int PIECES = 13, QS = 0, HI = 256;
+    static constexpr bool HAS_MIN = false;
+};
+
+// AHEAD: super-blocks requested ahead, as many as the 160 KB of a unit hold (half of that for workgroups of four waves, of which two share a unit): the ring of
+// activations has one slot more, a wave's ring of weights as many
+template <int DT, int MI, int NW> struct QwLds {
+    static constexpr int A = MI * 8192, AM = QWide<DT>::HAS_MIN ? MI * 1024 : 0, D8 = (MI + 1) / 2 * 256;
+    static constexpr int NB = (32 * QWide<DT>::PIECES + 63) / 64, B = 1024 * NB + (DT == CQ_Q6K ? 256 : 0);
+    static constexpr int bytes(int ahead) { return (ahead + 1) * (A + AM + D8) + ahead * NW * B; }
+    static constexpr int ROOM = 20 * 1024 * NW, AHEAD = bytes(3) <= ROOM ? 3 : bytes(2) <= ROOM ? 2 : 1;
+    static constexpr int A_OFF = 0, AM_OFF = (AHEAD + 1) * A, D8_OFF = AM_OFF + (AHEAD + 1) * AM, B_OFF = D8_OFF + (AHEAD + 1) * D8, BYTES = bytes(AHEAD);
+};
+
+template <int DT, int MI, bool MOE, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
+                                                              int rows, int64_t stride_dst, MoeChunks mc, int64_t expert_bytes, float *__restrict__ planes) {
+#ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler has no use for the body, and does not know its buffer accesses)
+    typedef QWide<DT> T;
+    typedef QwLds<DT, MI, NW> LD;
+    static_assert(NW == 8 || (NW == 4 && MI <= 2), "two waves bring the sums and two the scales of 64 rows at most");
+    constexpr int BB = BlockInfo<DT>::bytes, BM = 32 * MI, BN = 32 * NW, AHEAD = LD::AHEAD, ROW = 16 * T::PIECES;
+    constexpr int NA = 8 * MI / NW, NX = NA + 1, NB = LD::NB + (DT == CQ_Q6K ? 1 : 0);      // copies per wave and super-block: activations, with scales or sums, weights
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nr = lane & 31, kg = lane >> 5;
+    int m0 = blockIdx.x * BM;
+    const int n0 = blockIdx.y * BN + 32 * wv;
+    if (MOE) {
+        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
+        m0 = mc.first[blockIdx.x];
+        rows = m0 + mc.count[blockIdx.x];
+        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+    }
+    const int nsb_all = k >> 8;
+    const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
+    const int64_t row_bytes = (int64_t)nsb_all * BB;
+
+    // ---- weights: piece p of a super-block is piece p % PIECES of row p / PIECES; rows past the end repeat the last one (their results are not stored),
+    // pieces past the end the last piece ----
+    const int wbase = min(n0, n - 1), wlast = min(31, n - 1 - wbase);
+    const uint8_t *const wrow = w + wbase * row_bytes;
+    const uint32_t w_odd = DT == CQ_Q6K ? (uint32_t)(uintptr_t)wrow & 2u : 0u;       // (the descriptor begins on a dword)
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc((void *)(wrow - w_odd), 0, -1, 0x00020000);
+    uint32_t w_off[NB];
+#pragma unroll
+    for (int i = 0; i < LD::NB; i++) {
+        const int p = min(64 * i + lane, 32 * T::PIECES - 1), r = p / T::PIECES;
+        w_off[i] = (uint32_t)(min(r, wlast) * row_bytes) + 16 * (p - r * T::PIECES) + w_odd;
+    }
+    if constexpr (DT == CQ_Q6K) w_off[NB - 1] = (uint32_t)(min(lane & 31, wlast) * row_bytes) + 208 + w_odd;
+    // ---- activations: 64 bytes of 16 rows per instruction, piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
+    // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + NW i of its 8 MI KB)
+    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
+    constexpr int NAO = NW == 2 * MI ? 1 : NA;             // (as many waves as row blocks: the instructions of a wave are whole stages apart)
+    uint32_t a_off[NAO];
+#pragma unroll
+    for (int i = 0; i < NAO; i++) {
+        const int blk = wv + NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
+        a_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)k + 64 * st + 16 * p;
+    }
+    uint8_t *const myB = lds + LD::B_OFF + wv * (AHEAD * LD::B);
+    // ---- scales and 16-element sums of the activations: the first half of the waves brings the sums of 32 rows each, the others the scales of 64 ----
+    const bool x_sums = T::HAS_MIN && wv < NW / 2;
+    const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = min(x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane, rows - 1 - m0);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        x_sums ? (void *)(av.bsums + (int64_t)m0 * (k >> 4)) : (void *)(av.d + (int64_t)m0 * nsb_all), 0, -1, 0x00020000);
+    const uint32_t x_off = x_sums ? (uint32_t)x_r * (uint32_t)(32 * nsb_all) + 16 * (lane & 1) : (uint32_t)x_r * (uint32_t)(4 * nsb_all);
+    // Super-block kb0 + j of this workgroup's range into slot `slot`; past the end the last one again, into slots nobody reads.
+    auto issue_w = [&](int j, int slot) {
+        const int at = min(kb0 + j, kb1 - 1) * BB, odd = DT == CQ_Q6K ? at & 2 : 0;      // (210 kb is 2 past a dword for odd kb, and so are odd rows of an odd number of blocks)
+#pragma unroll
+        for (int i = 0; i < LD::NB; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::B + 1024 * i), 16, DT == CQ_Q6K ? (w_off[i] + odd) & ~2u : w_off[i], at - odd, 0, 0);
+        if constexpr (DT == CQ_Q6K)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (cq_lds_void *)(myB + slot * LD::B + 1024 * LD::NB), 4, (w_off[NB - 1] + odd) & ~2u, at - odd, 0, 0);
+        asm volatile("" ::: "memory");
+    };
+    auto issue_a = [&](int j, int slot) {
+        const int kb = min(kb0 + j, kb1 - 1);
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (cq_lds_void *)(lds + LD::A_OFF + slot * LD::A + 1024 * (wv + NW * i)), 16, a_off[NAO == 1 ? 0 : i], kb * 256 + (NAO == 1 ? 64 * i : 0), 0, 0);
+        if (x_sums) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (cq_lds_void *)(lds + LD::AM_OFF + slot * LD::AM + 1024 * x_blk), 16, x_off, 32 * kb, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (cq_lds_void *)(lds + LD::D8_OFF + slot * LD::D8 + 256 * x_blk), 4, x_off, 4 * kb, 0, 0);
+        asm volatile("" ::: "memory");
+    };
+
+    f32x16 acc[MI];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
+    const int live = (min(rows - m0, BM) + 31) / 32;       // 32-row tiles that hold rows: an expert, or the end of a prompt, rarely fills its last ones
+
+    // ---- the weights of a super-block, as operands: lane (nr, kg) has elements 16 kg .. 16 kg + 15 of every 32-element sub-block s of row nr ----
+    i32x4 wl[8], wh[8];
+    float d;
+    uint32_t dm = 0;                                       // d and dmin as they are in the block
+    u32x4 bm;                                              // the mins of four sub-blocks as f16, each twice
+    const uint8_t *const b_lane = myB + nr * ROW;
+    auto convert = [&](int j, int slot) {
+        const uint8_t *const blk = b_lane + slot * LD::B, *const quants = blk + 16 * (T::QS + kg);
+        if constexpr (DT == CQ_Q6K) {
+            const uint32_t shift = (uint32_t)(min(nr, wlast) * row_bytes + w_odd + (kb0 + j) * BB) & 2u;      // bytes by which this super-block is off its dword
+            auto piece = [&](const uint8_t *at, uint32_t behind) {
+                u32x4 v = *reinterpret_cast<const u32x4 *>(at);
+#pragma unroll
+                for (int i = 0; i < 3; i++) v[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], shift);
+                v[3] = __builtin_amdgcn_alignbyte(behind, v[3], shift);
+                return v;
+            };
+            const uint32_t last = *reinterpret_cast<const uint32_t *>(myB + slot * LD::B + 1024 * LD::NB + 4 * nr);
+            const u32x4 hdr = piece(blk + 192, last);
+            d = h2f(last >> (8 * shift));
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                u32x4 qa = piece(quants + 128 + 32 * h, *reinterpret_cast<const uint32_t *>(quants + 144 + 32 * h)), qb;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {              // high bits of sub-blocks 4 h (low nibbles) and 4 h + 2, and of 4 h + 1 and 4 h + 3
+                    qb[i] = (qa[i] >> 2) & 0x33333333u;
+                    qa[i] &= 0x33333333u;
+                }
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    const u32x4 raw = piece(quants + 64 * h + 32 * g, *reinterpret_cast<const uint32_t *>(quants + 64 * h + 32 * g + 16));
+                    const u32x4 qh = g ? qb : qa;
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        const int s = 4 * h + g + 2 * u;
+                        // int8 scale of 16 elements; scale (q - 32) + 128 in 16 bits: high byte, and low byte less 128
+                        const int sc = (int)(hdr[s >> 1] << (24 - 16 * (s & 1) - 8 * kg)) >> 24;
+                        const uint32_t mul = __builtin_amdgcn_perm(0, (uint32_t)sc, 0x01000100u), add = __builtin_amdgcn_perm(0, (uint32_t)(128 - 32 * sc), 0x01000100u);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t v = u ? ((raw[i] >> 4) & 0x0f0f0f0fu) | (qh[i] & ~0x0f0f0f0fu) : (raw[i] & 0x0f0f0f0fu) | ((qh[i] << 4) & ~0x0f0f0f0fu);
+                            const uint32_t e = qt_pk_mad(v & 0x00ff00ffu, mul, add), o = qt_pk_mad(qt_pk_high(v), mul, add);
+                            wl[s][i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+                            wh[s][i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+                        }
+                    }
+                }
+            }
+        } else {
+            const u32x4 hdr = *reinterpret_cast<const u32x4 *>(blk);
+            dm = hdr.x;
+            d = h2f(hdr.x);
+            // 6-bit scales and mins of four sub-blocks each (utils.rs:50-60)
+            const uint32_t sc[2] = {hdr.y & 0x3f3f3f3fu, (hdr.w & 0x0f0f0f0fu) | ((hdr.y >> 2) & 0x30303030u)};
+            const uint32_t m = kg ? ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3f3f3f3fu;
+#pragma unroll
+            for (int i = 0; i < 4; i++) bm[i] = qt_pk_add((0x6400u | ((m >> (8 * i)) & 0xffu)) * 0x00010001u, 0xe400e400u);
+            u32x4 qh = u32x4{0, 0, 0, 0};
+            if constexpr (DT == CQ_Q5K) qh = *reinterpret_cast<const u32x4 *>(blk + 16 + 16 * kg);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const u32x4 raw = *reinterpret_cast<const u32x4 *>(quants + 32 * q);
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int s = 2 * q + u;
+                    const uint32_t twice = 0x0c000c00u + 0x00010001u * (s & 3), scs = sc[s >> 2];       // byte s % 4 of four scales in both halves
+                    if constexpr (DT == CQ_Q4K) {
+                        const uint32_t lo = __builtin_amdgcn_perm(0, scs & 0x07070707u, twice), hi = __builtin_amdgcn_perm(0, (scs >> 3) & 0x07070707u, twice);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t v = (u ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu;
+                            wl[s][i] = (int)qt_pk_mul(v, lo);
+                            wh[s][i] = (int)qt_pk_mul(v, hi);
+                        }
+                    } else {
+                        const uint32_t mul = __builtin_amdgcn_perm(0, scs, twice);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t q1 = (qh[i] >> (s & 3)) & 0x11111111u;              // fifth bits of sub-blocks s % 4 (in the low nibbles) and s % 4 + 4
+                            const uint32_t v = ((u ? raw[i] >> 4 : raw[i]) & 0x0f0f0f0fu) | ((s < 4 ? q1 << 4 : q1) & ~0x0f0f0f0fu);
+                            const uint32_t e = qt_pk_mad(v & 0x00ff00ffu, mul, 0x00800080u), o = qt_pk_mad(qt_pk_high(v), mul, 0x00800080u);
+                            wl[s][i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+                            wh[s][i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+                        }
+                    }
+                }
+            }
+        }
+    };
+
+    // ---- products of a super-block, 32 rows at a time; the sums of the 32 rows before are scaled and added meanwhile ----
+    const uint8_t *const a_lane = lds + LD::A_OFF + nr * 64;
+    const int a_x0 = 16 * (kg ^ ((nr >> 2) & 3)), a_x1 = a_x0 ^ 32;
+    auto multiply = [&](int slot) {
+        const uint8_t *const a0 = a_lane + slot * LD::A + a_x0, *const a1 = a_lane + slot * LD::A + a_x1;
+        const uint8_t *const d8_lane = lds + LD::D8_OFF + slot * LD::D8 + 16 * kg, *const am_lane = lds + LD::AM_OFF + slot * LD::AM + nr * 32 + 16 * kg;
+        auto a_frag = [&](int t, int s) { return *reinterpret_cast<const i32x4 *>((s & 1 ? a1 : a0) + (s >> 1) * (MI * 2048) + t * 2048); };
+        i32x4 af[4];
+        i32x16 sl, sh, zero;
+        f32x16 sum, mt, none;
+        f32x4 d8;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            zero[e] = 0;
+            none[e] = 0.0f;
+        }
+        // results 2 s, 2 s + 1 of the sixteen that a lane has of tile t
+        auto scale = [&](int t, int s) {
+            if (s % 2 == 0) d8 = *reinterpret_cast<const f32x4 *>(d8_lane + 4 * (32 * t + 4 * s));
+#pragma unroll
+            for (int e = 2 * s; e < 2 * s + 2; e++) {
+                float v = d * sum[e];
+                if (T::HAS_MIN) v = fmaf(-h2f(dm >> 16), mt[e], v);
+                acc[t][e] = fmaf(d8[e & 3], v, acc[t][e]);
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < 4; u++) af[u] = a_frag(0, u);
+#pragma unroll
+        for (int t = 0; t < MI; t++) {
+            if (t < live) {
+                s16x8 ai;
+                if (T::HAS_MIN) ai = *reinterpret_cast<const s16x8 *>(am_lane + 1024 * t);
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    sl = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[s & 3], wl[s], s ? sl : zero, 0, 0, 0);
+                    sh = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[s & 3], wh[s], s ? sh : zero, 0, 0, 0);
+                    if (s < 4) af[s & 3] = a_frag(t, s + 4);
+                    else if (t + 1 < MI) af[s & 3] = a_frag(t + 1, s - 4);
+                    if (t > 0) scale(t - 1, s);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (T::HAS_MIN) {
+                    const half8 am = __builtin_convertvector(ai, half8);               // sums of 16 int8: exact
+                    mt = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, __builtin_bit_cast(half8, bm), none, 0, 0, 0);
+                }
+#pragma unroll
+                for (int e = 0; e < 16; e++) sum[e] = (float)(T::HI * sh[e] + sl[e]);
+                __builtin_amdgcn_sched_barrier(0);
+            } else if (t == live) {
+#pragma unroll
+                for (int s = 0; s < 8; s++) scale(t - 1, s);
+            }
+        }
+        if (live == MI) {
+#pragma unroll
+            for (int s = 0; s < 8; s++) scale(MI - 1, s);
+        }
+    };
+
+    const bool late = NW == 8 && wv >= 4;
+    // (in the order of the main loop: the waits count what was asked for behind)
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+        if (late) issue_a(j, j);
+        issue_w(j, j);
+        if (!late) issue_a(j, j);
+    }
+    const int nsb = kb1 - kb0;
+    int slot_a = 0, slot_w = 0;
+    for (int j = 0; j < nsb; j++) {
+        // Barrier j: the activations of super-block j are there for everybody, and nobody reads those of j - 1 any more.
+        auto meet = [&]() {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AHEAD * NB + (AHEAD - 1) * NX) : "memory");
+        };
+        const int next_a = slot_a == 0 ? AHEAD : slot_a - 1;
+        if (late) {
+            meet();
+            issue_a(j + AHEAD, next_a);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD * NX + (AHEAD - 1) * NB) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        convert(j, slot_w);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue_w(j + AHEAD, slot_w);
+        if (!late) {
+            meet();
+            issue_a(j + AHEAD, next_a);
+        }
+        multiply(slot_a);
+        slot_a = slot_a == AHEAD ? 0 : slot_a + 1;
+        slot_w = slot_w == AHEAD - 1 ? 0 : slot_w + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (copies may not outlive the workgroup)
 
     const int lane_out = qt_lane();
     qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
@@ -426,12 +654,19 @@ __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first,
     }
 }
 
+// Q6_K always, Q4_K and Q5_K in tiles of 96 and 128 rows take qtile_wide_kernel, which converts a super-block's weights first and multiplies then; tiles of 32 and 64 rows, whose
+// conversions are not much shorter than their products, are faster with both interleaved (qtile_kernel; Q4_K [4096 x 4096], 200 / 300 / 1000 rows 26.6 / 31.8 / 57.8 us against 28.1 / 33.5 / 60.6)
 template <int DT>
 int qtile_mi(int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
              const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
-#define QT_GO(M, E, NW)                                                                                                                                \
-    static_assert(QtLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                               \
-    return qtile_go(qtile_kernel<DT, M, E, NW>, NW, QtLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+#define QT_GO(M, E, NW)                                                                                                                                          \
+    if constexpr (DT == CQ_Q6K || M > 2) {                                                                                                                       \
+        static_assert(QwLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                     \
+        return qtile_go(qtile_wide_kernel<DT, M, E, NW>, NW, QwLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
+    } else {                                                                                                                                                     \
+        static_assert(QtLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                     \
+        return qtile_go(qtile_kernel<DT, M, E, NW>, NW, QtLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
+    }
     if (moe) {
         if (mi == 1) { QT_GO(1, true, QT_NW); }
         QT_GO(4, true, QT_NW);

@@ -83,6 +83,20 @@ def test_workgroups_of_four_and_eight_waves(fmt, m, n, k):
     assert row_error(got, want, x, w.cpu().numpy(), k) <= BOUND
 
 
+@pytest.mark.parametrize("fmt", ["q4k", "q5k", "q6k"])
+@pytest.mark.parametrize("m,n,k", [(97, 14338, 256), (128, 14338, 512), (129, 14338, 768), (225, 14338, 2304), (417, 7170, 2560), (385, 9002, 1536)])
+def test_wide_tiles(fmt, m, n, k):
+    """Tiles of 96 and 128 rows, the last one with one to four 32-row tiles of rows; one, two, three and more super-blocks (the rings hold two to four), odd numbers of
+    them (Q6_K rows then begin on 2 bytes; below 1536 of k it takes the general kernel), columns that end inside a wave's 32.  Against 64 bits, bound as above."""
+    from perf import cases
+    name = {"q4k": "q4_k", "q5k": "q5_k", "q6k": "q6_k"}[fmt]
+    print(f"case {fmt} m={m} n={n} k={k}", flush=True)
+    b = cases.blocks(name, 4, "w", n, k)
+    w, x = cases.values(name, b, n, k), normal(11 + n, (m, k))
+    got = run(FMT[fmt][0], b.reshape(-1).cpu().numpy(), x, n)
+    assert row_error(got, cases.product(name, torch.from_numpy(x).cuda(), w).cpu().numpy(), x, w.cpu().numpy(), k) <= BOUND
+
+
 @pytest.mark.parametrize("fmt", FMT)
 @pytest.mark.parametrize("out", [1, 30])
 @pytest.mark.parametrize("n,k", [(130, 512), (260, 4096)])
