@@ -9,15 +9,17 @@
 //
 // A workgroup's eight waves lie side by side along n and share 32 MI rows of activations in LDS (two super-blocks of 256, swizzled so that fragments are read
 // without bank conflicts); a wave owns 32 weight rows, brings their blocks for itself by copies to LDS, half a super-block at a time, and converts each
-// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  (The kernel that this
-// replaces for these formats shared weights and activations between 2 x 2 waves, converted every weight twice or four times and waited at two barriers per 64
-// elements.)  K is split over grid.z where that fills the chip better; see qtile_plan.
+// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  The weights are the matrix instructions' first operand, so that a
+// lane has sixteen weight rows' results of one activation row: the sixteen scales of the weights, put into LDS as f32 by the wave itself, are read once per block for all
+// tiles and one scale of the activations per tile.  (The other way round four reads of 16 bytes per tile and block brought the activations' scales, right in front of their
+// use: Q8_0, 2048 rows of [4096 x 14336] 457 us for 421.)  Results go out four columns at a time, whatever n is a multiple of.  K is split over grid.z where that fills the
+// chip better; see qtile_plan.
 //
-// [14336 x 4096], us, before / now, quantizing the activations included:   17 rows   131 rows   512 rows   2048 rows
-//   Q4_0                                                                  27.7 23.7  84.5 57.0  155 111    548 415
-//   Q8_0                                                                  27.1 23.9  82.0 61.0  144 121    515 468
-// 2048 rows of Q4_0 are 580 TOP/s: the two vector instructions per result and block take 1.1 us per super-block and 32 rows, the matrix cores a quarter of that
-// (of the SIMDs' cycles the vector units are busy 55 %, the matrix cores 12 %; the rest is the conversion's LDS reads and waits).
+// us, with the activations first / now, quantizing the activations included:        17 rows   131 rows   512 rows   2048 rows
+//   Q4_0 [14336 x 4096]                                                           23.8 24.1  61.0 57.8  122 115    455 435
+//   Q8_0 [14336 x 4096]                                                           26.3 26.3  66.3 59.9  134 121    504 461
+// 2048 rows of Q4_0 are 550 TOP/s.  A block of 32 x 32 results takes 198 cycles of a SIMD where its 32 fmas and a matrix instruction take 138 (on an eighth of the units; with all of
+// them busy the clock falls by a sixth): beside them the conversion of the weights from LDS places on 2 bytes (27 of 296 us), the scales (20) and the fragments (13).
 #include "cq_qtile.h"
 
 namespace {
@@ -28,13 +30,56 @@ template <> struct Q0Tile<CQ_Q4_0> { static constexpr int BB = 18, PPR = 5; };
 template <> struct Q0Tile<CQ_Q8_0> { static constexpr int BB = 34, PPR = 9; };
 
 typedef u32x4 u32x4_at2 __attribute__((aligned(2)));       // (LDS reads on 2 bytes)
+typedef f32x4 f32x4_at4 __attribute__((aligned(4)));       // (rows of results begin on an element)
+typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
 
 constexpr uint32_t Q0_MAGIC = 0x4b400000u;                 // 12582912.0f
 template <int DT, int MI> struct Q0Lds {
     static constexpr int NI = (32 * Q0Tile<DT>::PPR + 63) / 64;          // copy instructions per wave and half of weights
-    static constexpr int A = MI * 8192, B = NI * 1024, D8 = 8 * 32 * MI * 4;
-    static constexpr int A_OFF = 0, B_OFF = 2 * A, D8_OFF = B_OFF + 2 * QT_NW * B, BYTES = D8_OFF + 2 * D8;
+    static constexpr int A = MI * 8192, B = NI * 1024, D8 = 8 * 32 * MI * 4, DW = 8 * 32 * 4;
+    static constexpr int A_OFF = 0, B_OFF = 2 * A, D8_OFF = B_OFF + 2 * QT_NW * B, DW_OFF = D8_OFF + 2 * D8, BYTES = DW_OFF + QT_NW * DW;
 };
+
+// Results of a wave: row m0 + 32 t + nr of each tile, columns n0 + 8 e4 + 4 kg .. + 3: four at a time.  MOE: rows of the expert-sorted list, scattered to their pairs' rows and
+// scaled.  Splits of K after the first write f32 planes [rows, n].
+template <int MI, bool MOE>
+__device__ __forceinline__ void q0_store(const f32x16 (&acc)[MI], void *dst, int dst_dtype, int m0, int rows, int nr, int n0, int n, int kg, int64_t stride_dst, float *planes,
+                                         const MoeChunks &mc) {
+    const bool plane = !MOE && blockIdx.z > 0;
+    if (plane) dst = planes + (int64_t)(blockIdx.z - 1) * rows * n;
+    const int64_t ld = plane ? n : stride_dst;
+#pragma unroll
+    for (int t = 0; t < MI; t++) {
+        const int mm = m0 + 32 * t + nr;
+        if (mm >= rows) break;
+        const int64_t at = (MOE ? mc.pair_out[mm] : mm) * ld;
+        const float by = MOE ? mc.pair_scale[mm] : 1.0f;
+#pragma unroll
+        for (int e4 = 0; e4 < 4; e4++) {
+            const int nn = n0 + 8 * e4 + 4 * kg;
+            f32x4 v = {acc[t][4 * e4], acc[t][4 * e4 + 1], acc[t][4 * e4 + 2], acc[t][4 * e4 + 3]};
+            if (MOE) v *= by;
+            if (MOE || plane || dst_dtype == CQ_F32) {
+                float *const out = (float *)dst + at + nn;
+                if (nn + 4 <= n) *reinterpret_cast<f32x4_at4 *>(out) = v;
+                else
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (nn + i < n) out[i] = v[i];
+            } else {
+                uint16_t *const out = (uint16_t *)dst + at + nn;
+                uint16_t h[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) h[i] = dst_dtype == CQ_F16 ? f2h_bits(v[i]) : f2bf_bits(v[i]);
+                if (nn + 4 <= n) *reinterpret_cast<u32x2_at2 *>(out) = u32x2{(uint32_t)h[0] | (uint32_t)h[1] << 16, (uint32_t)h[2] | (uint32_t)h[3] << 16};
+                else
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (nn + i < n) out[i] = h[i];
+            }
+        }
+    }
+}
 
 template <int DT, int MI, bool MOE>
 __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
@@ -121,23 +166,40 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
     issue_w(kb0, 0);
     const int nsb = kb1 - kb0;
     bool wild = false;
-    const int live = MOE ? (rows - m0 + 31) / 32 : MI;
+    const int live = (min(rows - m0, BM) + 31) / 32;       // 32-row tiles that hold rows
     const uint32_t nib = 4 - 4 * kg;                       // Q4_0: the lower lanes take the low nibbles
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // ---- scales of the weights: [8 blocks][32 rows] of f32 in LDS, since a lane has results of sixteen rows ----
+    uint8_t *const my_dw = lds + LD::DW_OFF + wv * LD::DW;
+    auto row_scales = [&](int h) {                         // of the half that has landed: blocks 4 h + 2 kg and the one behind it
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            float v = h2f(*reinterpret_cast<const uint16_t *>(lds + my_row + (h * (LD::B + 8) + i * BB) + 2 * kg * BB));
+            if (DT == CQ_Q4_0) v *= 0.0625f;
+            wild |= !(__builtin_fabsf(v) < __builtin_inff());
+            *reinterpret_cast<float *>(my_dw + 128 * (4 * h + i) + 256 * kg + 4 * nr) = v;
+        }
+        asm volatile("" ::: "memory");                     // (other lanes read them; a wave's LDS accesses keep their order)
+    };
+    auto scales_of = [&](int b, f32x4 (&d)[4]) {
+#pragma unroll
+        for (int e4 = 0; e4 < 4; e4++) d[e4] = *reinterpret_cast<const f32x4 *>(my_dw + 128 * b + 32 * e4 + 16 * kg);
+    };
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    row_scales(0);
+    f32x4 dw[4];
+    scales_of(0, dw);
     for (int j = 0; j < nsb; j++) {
         const int kb = kb0 + j, slot = j & 1;
-        if (j > 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         issue_w(kb, 1);
         request(j + 1);
-        const uint8_t *const Aj = lds + LD::A_OFF + slot * LD::A + nr * 64, *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 16 * kg;
-        // this lane's 16 weights of block b, and the block's scale
-        auto operand = [&](int b, i32x4 &op, float &dw) {
+        const uint8_t *const Aj = lds + LD::A_OFF + slot * LD::A + nr * 64, *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 4 * nr;
+        // this lane's 16 weights of block b
+        auto operand = [&](int b, i32x4 &op) {
             const uint8_t *const blk = lds + my_row + ((b >> 2) * (LD::B + 8) + (b & 3) * BB);
-            dw = h2f(*reinterpret_cast<const uint16_t *>(blk));
             if constexpr (DT == CQ_Q4_0) {
                 // nibbles as 16 (q - 8): the high ones where they are, the low ones moved up
                 const u32x4 q = *reinterpret_cast<const u32x4_at2 *>(blk + 2);
-                dw *= 0.0625f;
 #pragma unroll
                 for (int i = 0; i < 4; i++) op[i] = (int)(((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u);
             } else {
@@ -147,40 +209,57 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
         auto a_frag = [&](int b, int t) {
             return *reinterpret_cast<const i32x4 *>(Aj + (b >> 1) * (MI * 2048) + t * 2048 + 16 * ((2 * (b & 1) + kg) ^ ((nr >> 2) & 3)));
         };
+        auto d8_of = [&](int b, float (&d)[MI]) {
+#pragma unroll
+            for (int t = 0; t < MI; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
+        };
         // The sums of block b + 1 are on their way in the matrix cores while those of block b are scaled, tile by tile.
         i32x4 op;
-        float dw;
         i32x16 S[MI];
-        operand(0, op, dw);
+        float d8[MI];
+        operand(0, op);
+        d8_of(0, d8);
 #pragma unroll
         for (int t = 0; t < MI; t++)
-            if (!MOE || t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_frag(0, t), op, magic, 0, 0, 0);
+            if (t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, a_frag(0, t), magic, 0, 0, 0);
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
-            if (b == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+            if (b == 3) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+                row_scales(1);
+            }
             if (b == 4) issue_w(kb + 1, 0);
-            const float c = -12582912.0f * dw;
-            wild |= !(__builtin_fabsf(dw) < __builtin_inff());
+            if (b == 7) {                                  // the next super-block's first half
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                row_scales(0);
+            }
+            f32x4 c[4], dw_n[4];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) c[e4] = -12582912.0f * dw[e4];
+            scales_of(b == 7 ? 0 : b + 1, dw_n);
             i32x4 op_n;
-            float dw_n = 0.0f;
-            if (b < 7) operand(b + 1, op_n, dw_n);
+            float d8_n[MI];
+            if (b < 7) {
+                operand(b + 1, op_n);
+                d8_of(b + 1, d8_n);
+            }
 #pragma unroll
             for (int t = 0; t < MI; t++) {
-                if (MOE && t >= live) break;
-                f32x4 d8[4];
-#pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) d8[e4] = *reinterpret_cast<const f32x4 *>(Dj + 4 * (b * BM + t * 32 + 8 * e4));
+                if (t >= live) break;
                 i32x4 af;
                 if (b < 7) af = a_frag(b + 1, t);
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw, c), d8[e >> 2][e & 3], acc[t][e]);
+                for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
                 qt_pin(acc[t]);
-                if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, op_n, magic, 0, 0, 0);
+                if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op_n, af, magic, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
             op = op_n;
-            dw = dw_n;
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) dw[e4] = dw_n[e4];
+#pragma unroll
+            for (int t = 0; t < MI; t++) d8[t] = d8_n[t];
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -193,31 +272,33 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
             f32x16 a[1];
 #pragma unroll
             for (int e = 0; e < 16; e++) a[0][e] = 0.0f;
+            const int64_t mm = min(m0 + 32 * t + nr, rows - 1);
 #pragma unroll 1
             for (int g = 8 * kb0; g < 8 * kb1; g++) {
                 const uint8_t *const blk = wr + (int64_t)g * BB;
-                const float dg = h2f(ld_u<uint16_t>(blk)) * (DT == CQ_Q4_0 ? 0.0625f : 1.0f);
                 u32x4 q = ld_u<u32x4>(blk + 2 + (DT == CQ_Q4_0 ? 0 : 16 * kg));
                 if (DT == CQ_Q4_0) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) q[i] = ((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u;
                 }
-                const i32x4 af = *reinterpret_cast<const i32x4 *>(av.qs + (int64_t)min(m0 + 32 * t + nr, rows - 1) * k + 32 * g + 16 * kg);
+                const i32x4 af = *reinterpret_cast<const i32x4 *>(av.qs + mm * k + 32 * g + 16 * kg);
+                const float d8 = av.d[2 * (mm * (8 * nsb_all) + g)];
                 i32x16 S;
 #pragma unroll
                 for (int e = 0; e < 16; e++) S[e] = 0;
-                S = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(i32x4, q), S, 0, 0, 0);
+                S = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, q), af, S, 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    const int64_t mm = min(m0 + t * 32 + 8 * (e >> 2) + 4 * kg + (e & 3), rows - 1);
-                    a[0][e] = fmaf((float)S[e] * dg, av.d[2 * (mm * (8 * nsb_all) + g)], a[0][e]);
+                    const int64_t nn = min(n0 + 8 * (e >> 2) + 4 * kg + (e & 3), n - 1);
+                    const float dg = h2f(ld_u<uint16_t>(w + nn * row_bytes + (int64_t)g * BB)) * (DT == CQ_Q4_0 ? 0.0625f : 1.0f);
+                    a[0][e] = fmaf((float)S[e] * dg, d8, a[0][e]);
                 }
             }
-            qt_store<1, MOE>(a, dst, dst_dtype, m0 + 32 * t, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+            q0_store<1, MOE>(a, dst, dst_dtype, m0 + 32 * t, rows, nr, n0, n, kg, stride_dst, planes, mc);
         }
         return;
     }
-    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+    q0_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, nr, n0, n, kg, stride_dst, planes, mc);
 #endif
 }
 

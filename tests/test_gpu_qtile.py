@@ -104,6 +104,13 @@ def test_half_results(fmt, out, n, k):
     check(fmt, 67, n, k, out)                              # written by the product itself, and by the sum over the splits
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("out", [0, 1, 30])
+@pytest.mark.parametrize("m,n,k", [(33, 131, 512), (101, 70, 768), (70, 291, 2304)])
+def test_rows_of_results_off_four_columns(fmt, out, m, n, k):
+    check(fmt, m, n, k, out)                               # four columns at a time on any element, the last one to three alone
+
+
 @pytest.mark.parametrize("fmt", FMT)
 @pytest.mark.parametrize("out", [0, 1])
 @pytest.mark.parametrize("m,n,k,splits", [(67, 260, 1536, 1), (67, 260, 4096, 4)])
