@@ -720,21 +720,21 @@ __global__ __launch_bounds__(QS_NW * 64) void qms_rows2_kernel(const uint8_t *a_
 // Two weight tensors over the same activation row in one launch, tensor A on the streaming body; tensor B on the
 // streaming body as well (SB) or on qmv_body.  Workgroups [0, blocks_a) take tensor A.  NW waves per workgroup: 8, or
 // 16 where qmv_body needs one wave per activation span (its plane-merging prologue).
-// Arguments of the two-tensor launch, 60 bytes: tensor B and its output are given as distances from tensor A's.
+// Arguments of the two-tensor launch, 68 bytes: tensor B is given as its distance from tensor A.  (Outputs as pointers, since buffers of an allocator may lie anywhere: further
+// than a 32-bit distance apart, the two tensors took two launches, 10 us for 6.)
 struct Qs2Args {
-    const uint8_t *wa; const float *x, *aux, *extra; float *dsta;      // extra: partial sums (PRO_NORM) or planes (PRO_NORM_SPLIT)
+    const uint8_t *wa; const float *x, *aux, *extra; float *dsta, *dstb;      // extra: partial sums (PRO_NORM) or planes (PRO_NORM_SPLIT)
     int na, nb;
     uint32_t meta;            // bpr | blocks_a << 8 | blocks_b << 16 | n_planes << 24
     float eps;
     int wb_off16;             // (wb - wa) / 16
-    int dstb_off;             // dstb - dsta, in floats
 };
 // The arguments are scalars, ordered by first use, so that the fourteen dwords placed in SGPRs at wave launch are the ones
-// the first loads need; the output pointer, needed last, is read from the argument block.
+// the first loads need; the output pointers, needed last, are read from the argument block.
 template <int DTA, int DTB, int NW, int XS, int MAXB, bool SINGLE, int PRO, bool SB>
 __global__ __launch_bounds__(NW * 64) void qms2_kernel(const uint8_t *a_wa, const float *a_x, const float *a_aux, const float *a_extra, int a_na, int a_nb,
-                                                       uint32_t a_meta, int a_wb_off16, float a_eps, int a_dstb_off, float *a_dsta) {
-    const Qs2Args a{a_wa, a_x, a_aux, a_extra, a_dsta, a_na, a_nb, a_meta, a_eps, a_wb_off16, a_dstb_off};
+                                                       uint32_t a_meta, int a_wb_off16, float a_eps, float *a_dsta, float *a_dstb) {
+    const Qs2Args a{a_wa, a_x, a_aux, a_extra, a_dsta, a_dstb, a_na, a_nb, a_meta, a_eps, a_wb_off16};
     const int blocks_a = (a.meta >> 8) & 255, blocks_b = (a.meta >> 16) & 255, bpr = a.meta & 255;
     Fuse fz{a.aux, PRO == PRO_NORM ? a.extra : nullptr, a.eps, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, 0, PRO == PRO_NORM_SPLIT ? a.extra : nullptr,
             (int)(a.meta >> 24)};
@@ -754,7 +754,7 @@ __global__ __launch_bounds__(NW * 64) void qms2_kernel(const uint8_t *a_wa, cons
         } else if constexpr (SB) {
             g.step_bytes = g.step_rows * bpr * StreamFmt<DTB>::BB;
             g.w_bytes = (int64_t)n * (bpr * StreamFmt<DTB>::BB);
-            qms_body<DTB, NW, XS, MAXB, PRO, EPI_NONE>(a.wa + (int64_t)a.wb_off16 * 16, a.x, a.dsta + a.dstb_off, g, fz, blockIdx.x - blocks_a, blocks_b);
+            qms_body<DTB, NW, XS, MAXB, PRO, EPI_NONE>(a.wa + (int64_t)a.wb_off16 * 16, a.x, a.dstb, g, fz, blockIdx.x - blocks_a, blocks_b);
         }
     } else if constexpr (!SB) {
         // tensor B on qmv_body: its geometry as make_geom() lays it out for NW waves and blocks_b workgroups
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(NW * 64) void qms2_kernel(const uint8_t *a_wa, cons
         gb.lds_red_off = (int)L.total;
         gb.dst_dtype = CQ_F32; gb.stride_dst = n;
         ActSrc src{a.x, ActView{nullptr, nullptr, nullptr}};
-        qmv_body<DTB, 1, CQ_F32, SINGLE, PRO, EPI_NONE, false>(a.wa + (int64_t)a.wb_off16 * 16, src, a.dsta + a.dstb_off, gb, fz, blockIdx.x - blocks_a, blocks_b);
+        qmv_body<DTB, 1, CQ_F32, SINGLE, PRO, EPI_NONE, false>(a.wa + (int64_t)a.wb_off16 * 16, src, a.dstb, gb, fz, blockIdx.x - blocks_a, blocks_b);
     }
 }
 
@@ -1203,9 +1203,9 @@ int launch_pair_stream_xs(const void *wa, float *dsta, const void *wb, int64_t n
     const size_t lds_bytes = lds_a > lds_b ? lds_a : lds_b;
     if (lds_bytes + StreamAct<MAXB>::BYTES + 256 > (size_t)LDS_BUDGET) return CQ_ERR_RANGE;
     const bool single = k / 64 <= 64;
-    // tensor B and its output travel as 32-bit distances from tensor A's; a launch they do not fit takes qmv2_kernel
-    const int64_t wdist = (const uint8_t *)wb - (const uint8_t *)wa, ddist = dstb - dsta;
-    if (wdist % 16 || wdist / 16 > 0x7fffffffLL || wdist / 16 < -0x7fffffffLL || ddist > 0x7fffffffLL || ddist < -0x7fffffffLL) return CQ_ERR_RANGE;
+    // tensor B travels as a 32-bit distance from tensor A; a launch it does not fit takes qmv2_kernel
+    const int64_t wdist = (const uint8_t *)wb - (const uint8_t *)wa;
+    if (wdist % 16 || wdist / 16 > 0x7fffffffLL || wdist / 16 < -0x7fffffffLL) return CQ_ERR_RANGE;
     if (groups_a > 255 || groups_b > 255 || groups_b < 1 || fz.n_planes > 15) return CQ_ERR_RANGE;
     if (!sb) {
         // qmv_body's geometry is rebuilt in the kernel from (nb, blocks_b): it must be what make_geom() returned
@@ -1216,14 +1216,14 @@ int launch_pair_stream_xs(const void *wa, float *dsta, const void *wb, int64_t n
     a.wa = (const uint8_t *)wa; a.x = x; a.aux = fz.aux; a.extra = PRO == PRO_NORM ? fz.part_in : fz.planes; a.dsta = dsta;
     a.na = ga.n; a.nb = (int)nb;
     a.meta = (uint32_t)ga.bpr | ((uint32_t)groups_a << 8) | ((uint32_t)groups_b << 16) | ((uint32_t)fz.n_planes << 24);
-    a.eps = fz.eps; a.wb_off16 = (int)(wdist / 16); a.dstb_off = (int)ddist;
+    a.eps = fz.eps; a.wb_off16 = (int)(wdist / 16); a.dstb = dstb;
     dim3 grid((unsigned)(groups_a + groups_b)), block(64 * NW);
     auto go = [&](auto kern) {
         if (lds_bytes > 48 * 1024) {
             hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
             if (e != hipSuccess) return (int)e;
         }
-        hipLaunchKernelGGL(kern, grid, block, lds_bytes, s, a.wa, a.x, a.aux, a.extra, a.na, a.nb, a.meta, a.wb_off16, a.eps, a.dstb_off, a.dsta);
+        hipLaunchKernelGGL(kern, grid, block, lds_bytes, s, a.wa, a.x, a.aux, a.extra, a.na, a.nb, a.meta, a.wb_off16, a.eps, a.dsta, a.dstb);
         return (int)hipGetLastError();
     };
     // (the sixteen-wave launch exists for a tensor B that does not stream)
@@ -1276,8 +1276,8 @@ int launch_pair(const void *wa, int64_t na, float *dsta, const void *wb, int64_t
     if constexpr (qs_streams(DTA)) {
         int rc = launch_pair_stream<DTA, DTB, PRO>(wa, na, dsta, wb, nb, dstb, (const float *)src.x, k, s, fz_in);
         if (rc != CQ_ERR_RANGE) return rc;
-        // the two-tensor launch does not take this call (the tensors or their outputs lie further apart than its 32-bit
-        // distances, or a geometry it has no kernel for): when a single call would stream, two launches, each on the
+        // the two-tensor launch does not take this call (the tensors lie further apart than its 32-bit
+        // distance, or a geometry it has no kernel for): when a single call would stream, two launches, each on the
         // kernel a single call gets, so that the results do not depend on where the buffers happen to lie
         StreamGeom gt;
         if (stream_geom<DTA>(gt, k, na, CQ_F32) || stream_geom<DTB>(gt, k, nb, CQ_F32)) {

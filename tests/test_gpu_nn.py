@@ -675,6 +675,28 @@ def test_fused_norm_pair_matvec(dta, dtb, na, nb, k):
                                        dev(part).data_ptr(), dev(nw).data_ptr(), 1e-5, k, None) == -1
 
 
+def test_fused_norm_pair_outputs_far_apart():
+    """Outputs more than 2^31 floats apart, in either order: one launch writes both, with the bits of the single launches."""
+    import oracle
+    lib = L()
+    na, nb, k = 5120, 1024, 4096
+    x, nw = normal(74, (1, k), 1.0), np.ones(k, dtype=np.float32)
+    wa = dev(oracle.from_float(12, normal(75, (na, k), 0.03).reshape(-1)))
+    wb = dev(oracle.from_float(14, normal(76, (nb, k), 0.03).reshape(-1)))
+    part = np.zeros(256, dtype=np.float32)
+    part[0] = (x.astype(np.float64) ** 2).sum()
+    xd, pd, wd = dev(x), dev(part), dev(nw)
+    far = torch.empty((1 << 31) + 16384, device="cuda")
+    low, high = far[:na], far[(1 << 31) + 8192:]
+    za, zb = torch.empty(na, device="cuda"), torch.empty(nb, device="cuda")
+    ok(lib.cq_nn_qmatmul_norm(12, wa.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(), 1e-5, za.data_ptr(), k, na, None))
+    ok(lib.cq_nn_qmatmul_norm(14, wb.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(), 1e-5, zb.data_ptr(), k, nb, None))
+    for ya, yb in ((low, high[:nb]), (high[:na], low[:nb])):
+        far[:na], far[(1 << 31) + 8192:] = 77.0, 77.0
+        ok(lib.cq_nn_qmatmul_norm_pair(12, wa.data_ptr(), na, ya.data_ptr(), 14, wb.data_ptr(), nb, yb.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(), 1e-5, k, None))
+        assert torch.equal(ya, za) and torch.equal(yb, zb)
+
+
 def split_planes(dtype, k):
     """The fewest equal slices of whole blocks (2..4) that are at most one wave step long: 64 units of 64 elements for
     K-quants, of 32 elements for Q4_0 / Q8_0."""
