@@ -299,6 +299,23 @@ int cq_nn_qmatmul_swiglu_rows(int w_dtype, const void *w_dev, const float *gate_
     return forward_quantized(w_dtype, w_dev, dst_dev, CQ_F32, m, k, n, workspace_dev, workspace_bytes, s);
 }
 
+int cq_nn_qmatmul_swiglu_pair(int w_dtype, const void *w1_dev, const void *w3_dev, const float *x_dev, float *dst_dev, int64_t m, int64_t k, int64_t n,
+                              void *workspace_dev, int64_t workspace_bytes, void *stream) {
+    int rc = check_mm_shape(w_dtype, k, n, m);
+    if (rc || (rc = check_mm_shape(w_dtype, k, 2 * n, m))) return rc;
+    if (m == 0 || n == 0) return CQ_OK;
+    if ((rc = check_weight_ptr(w_dtype, w1_dev)) || (rc = check_weight_ptr(w_dtype, w3_dev))) return rc;
+    if (!x_dev || !dst_dev || !workspace_dev) return CQ_ERR_NULL;
+    if (!aligned(x_dev, 16) || !aligned(workspace_dev, 256) || !aligned(dst_dev, 4)) return CQ_ERR_ALIGN;
+    if (workspace_bytes < workspace_least(w_dtype, m, k, 2 * n)) return CQ_ERR_WORKSPACE;
+    if (m <= 64 || !cq_use_mfma(w_dtype, m, k)) return CQ_ERR_RANGE;                 // (up to 64 rows are the batched matvecs')
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t act = cq_act_layout(w_dtype, k, m).total, room = std::min(workspace_bytes, cq_qmatmul_workspace_bytes(w_dtype, m, k, 2 * n)) - act;
+    if (!cq_qtile_takes_swiglu(w_dtype, w1_dev, w3_dev, k, n, m, room)) return CQ_ERR_RANGE;
+    if ((rc = cq_quantize_act_launch(w_dtype, x_dev, CQ_F32, workspace_dev, k, m, s))) return rc;
+    return cq_qtile_swiglu_launch(w_dtype, w1_dev, w3_dev, cq_act_view(workspace_dev, w_dtype, k, m), dst_dev, k, n, m, room, s);
+}
+
 int64_t cq_indexed_moe_workspace_bytes(int w_dtype, int64_t num_experts, int64_t n, int64_t k, int64_t batch, int64_t topk,
                                        int64_t input_dim1) {
     if (!moe_weight_dtype(w_dtype) || check_mm_shape(w_dtype, k, n, batch) || num_experts <= 0 || topk <= 0) return -1;

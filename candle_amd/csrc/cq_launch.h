@@ -184,6 +184,10 @@ int cq_moe_stream_launch(int w_dtype, const void *w_a, const void *w_b, float *o
 // more than one large one)
 #define CQ_MOE_TILE_SMALL 32
 #define CQ_MOE_TILE_LARGE 128
+// silu(x w_gate^T) * x w_up^T in one launch, for the shapes that takes_swiglu names
+bool cq_qtile_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes);
+int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *dst, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes,
+                           hipStream_t s);
 int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s);
 int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,
                          int64_t n, int tile_rows, hipStream_t s);

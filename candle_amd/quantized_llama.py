@@ -379,7 +379,15 @@ class ModelWeights(GreedyDecoder):
                                                  cfg.hidden, cfg.rms_eps, sp))
             tap("ffn_norm", li)
             # w2(silu(w1 x) * w3 x)                                                       :56-63
-            w1, w3 = w["feed_forward_w1"], w["feed_forward_w3"]
+            w1, w3, w2 = w["feed_forward_w1"], w["feed_forward_w3"], w["feed_forward_w2"]
+            if rows > 64 and self.tap is None and w1.dtype == w3.dtype:
+                # prompts: silu(w1 x) * w3 x in one launch (-6, CQ_ERR_RANGE: not a shape of it)
+                rc = L.cq_nn_qmatmul_swiglu_pair(int(w1.dtype), w1.ptr, w3.ptr, xn.data_ptr(), h.data_ptr(), rows, w1.k, cfg.ffn, self.ws.data_ptr(),
+                                                 self.ws.numel(), sp)
+                if rc != -6:
+                    ck("cq_nn_qmatmul_swiglu_pair", rc)
+                    self._mm(w2, cfg.hidden, h, delta.data_ptr(), rows, sp)
+                    continue
             if w1.dtype == w3.dtype and w3.ptr == w1.ptr + w1.nbytes:
                 self._mm(w1, 2 * cfg.ffn, xn, gu.data_ptr(), rows, sp)
                 g_ptr, u_ptr, gs = gu.data_ptr(), gu.data_ptr() + 4 * cfg.ffn, 2 * cfg.ffn
@@ -388,7 +396,6 @@ class ModelWeights(GreedyDecoder):
                 self._mm(w3, cfg.ffn, xn, gu.data_ptr() + 4 * rows * cfg.ffn, rows, sp)
                 g_ptr, u_ptr, gs = gu.data_ptr(), gu.data_ptr() + 4 * rows * cfg.ffn, cfg.ffn
             tap("w13", li)
-            w2 = w["feed_forward_w2"]
             if rows > 2 and cfg.ffn % 256 == 0:
                 # silu(w1 x) * w3 x goes straight into the activation quantizer of w2
                 ck("cq_nn_qmatmul_swiglu_rows", L.cq_nn_qmatmul_swiglu_rows(int(w2.dtype), w2.ptr, g_ptr, u_ptr, gs, gs, delta.data_ptr(), rows,

@@ -106,6 +106,13 @@ int cq_nn_silu_mul(const float *gate_dev, const float *up_dev, float *out_dev, i
 int cq_nn_qmatmul_swiglu_rows(int w_dtype, const void *w_dev, const float *gate_dev, const float *up_dev, int64_t gate_stride, int64_t up_stride,
                               float *dst_dev, int64_t m, int64_t k, int64_t n, void *workspace_dev, int64_t workspace_bytes, void *stream);
 
+/* dst [m, n] = silu(QMatMul(w1).forward(x)) * QMatMul(w3).forward(x) for m rows of x: the first half of Mlp::forward (quantized_llama.rs:56-63) for prompts
+ * of K formats, without either product in memory.  Results are those of cq_qmatmul_forward with each of the two weights (w3 right behind w1: with both as one of 2 n
+ * rows) and cq_nn_silu_mul, bit for bit.  CQ_ERR_RANGE, with nothing enqueued: not a shape that gains by it, use these.  Workspace as
+ * cq_qmatmul_workspace_bytes(w_dtype, m, k, 2 n). */
+int cq_nn_qmatmul_swiglu_pair(int w_dtype, const void *w1_dev, const void *w3_dev, const float *x_dev, float *dst_dev, int64_t m, int64_t k, int64_t n,
+                              void *workspace_dev, int64_t workspace_bytes, void *stream);
+
 /* Single-row (decode) fusions of the glue into the quantized matvec kernel.  No counterpart in the reference,
  * which runs these as separate tensor ops; results equal the unfused sequence up to f32 summation order.
  *

@@ -17,6 +17,9 @@ from tests.util import normal, rel_l2
 pytestmark = pytest.mark.gpu
 BOUND = 4e-6
 FMT = {"q4_0": (2, oracle.Q4_0), "q8_0": (8, oracle.Q8_0), "q4k": (12, oracle.Q4K), "q5k": (13, oracle.Q5K), "q6k": (14, oracle.Q6K)}
+# shapes that the joint product, or one of two, would split or give narrower tiles
+REFUSED_PAIRS = {("q6k", 129, 14338, 256), ("q6k", 225, 14337, 1792), ("q4k", 300, 14336, 2560)} | {(f, 97, 7169, 1536) for f in FMT}
+REFUSED_APART = {(f, 400, 5632, 2048) for f in FMT}
 OUT = {0: torch.float32, 1: torch.float16, 30: torch.bfloat16}
 
 
@@ -95,6 +98,52 @@ def test_wide_tiles(fmt, m, n, k):
     w, x = cases.values(name, b, n, k), normal(11 + n, (m, k))
     got = run(FMT[fmt][0], b.reshape(-1).cpu().numpy(), x, n)
     assert row_error(got, cases.product(name, torch.from_numpy(x).cuda(), w).cpu().numpy(), x, w.cpu().numpy(), k) <= BOUND
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q5k", "q6k"])
+@pytest.mark.parametrize("gap", [0, 16])
+@pytest.mark.parametrize("m,n,k", [(97, 7169, 1536), (129, 14338, 256), (225, 14337, 1792), (300, 14336, 2560), (400, 5632, 2048)])
+def test_silu_of_a_pair(fmt, gap, m, n, k):
+    """cq_nn_qmatmul_swiglu_pair, the second weight right behind the first or not: bit for bit what the products and cq_nn_silu_mul give, canaries around it; rows and
+    columns that end inside a tile and one whose last tiles have no rows.  Whatever the shape, it is taken whole or refused."""
+    L = _lib.lib()
+    print(f"case {fmt} gap={gap} m={m} n={n} k={k}", flush=True)
+    from perf import cases
+    code, name = FMT[fmt][0], {"q4k": "q4_k", "q5k": "q5_k", "q6k": "q6_k"}[fmt]
+    w = cases.blocks(name, 6, "w", 2 * n, k).reshape(-1)
+    nb = w.numel() // 2
+    raw = torch.zeros(2 * nb + gap, dtype=torch.uint8, device="cuda")
+    raw[:nb], raw[nb + gap:] = w[:nb], w[nb:]
+    x = torch.from_numpy(normal(12 + n, (m, k))).cuda()
+    st = torch.cuda.current_stream().cuda_stream
+    wsb = L.cq_qmatmul_workspace_bytes(code, m, k, 2 * n)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    y = torch.full((m + 2, n), 77.0, device="cuda")
+    args = (code, raw.data_ptr(), raw.data_ptr() + nb + gap, x.data_ptr(), y[1].data_ptr(), m, k, n, ws.data_ptr())
+    rc = L.cq_nn_qmatmul_swiglu_pair(*args, wsb, st)
+    taken = rc == 0
+    assert taken or rc == -6
+    assert taken == ((fmt, m, n, k) not in REFUSED_PAIRS and (gap == 0 or (fmt, m, n, k) not in REFUSED_APART))
+    assert L.cq_nn_qmatmul_swiglu_pair(*args, 256, st) == -5
+    torch.cuda.synchronize()
+    if not taken:
+        assert (y == 77.0).all()
+        return
+    assert (y[0] == 77.0).all() and (y[m + 1] == 77.0).all()
+    want = torch.empty((m, n), device="cuda")
+    gate, up = torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
+    for at, to in ((0, gate), (nb + gap, up)):
+        _lib.check("cq_qmatmul_forward", L.cq_qmatmul_forward(code, raw.data_ptr() + at, x.data_ptr(), 0, to.data_ptr(), 0, m, k, n, ws.data_ptr(), wsb, st))
+    if gap == 0:                                           # (as one product of 2 n rows, which is not split where those of n may be)
+        both = torch.empty((m, 2 * n), device="cuda")
+        _lib.check("cq_qmatmul_forward", L.cq_qmatmul_forward(code, raw.data_ptr(), x.data_ptr(), 0, both.data_ptr(), 0, m, k, 2 * n, ws.data_ptr(), wsb, st))
+        gate, up = both[:, :n].contiguous(), both[:, n:].contiguous()
+    pad = (-n) % 4                                         # (cq_nn_silu_mul takes four elements at a time)
+    gate, up = (torch.nn.functional.pad(t, (0, pad)).contiguous() for t in (gate, up))
+    want = torch.empty_like(gate)
+    _lib.check("cq_nn_silu_mul", L.cq_nn_silu_mul(gate.data_ptr(), up.data_ptr(), want.data_ptr(), m, n + pad, n + pad, n + pad, st))
+    torch.cuda.synchronize()
+    assert torch.equal(y[1:m + 1], want[:, :n])
 
 
 @pytest.mark.parametrize("fmt", FMT)
