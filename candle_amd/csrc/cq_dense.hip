@@ -134,6 +134,8 @@ __device__ __forceinline__ void group_tile_at(const Src &s, int t, int tiles_m, 
 // on warm operands 1500 x 5632 x 2048 66 -> 63), one for the others: f32 activations and small tiles gain nothing from more (40 x 4096 x 4096: 13.3 -> 14.2), and
 // workgroups of up to 12 stages (a split of k, short rows) lose by it: the three past the end are brought all the same (700 x 2048 x 2048 in six splits 26.4 us
 // with one, 28.1 with three; 4 - 11 stages 4 % slower on average, 13 - 16 none, from 18 on faster).
+// Rows go by sixteens to the WGM waves that share the tile's rows, and the main loop of the large tile exists once per number of fragments that a wave then has: rows that are not there are neither brought
+// nor multiplied (an expert's last tile; 64 experts of 2048 x 1408 under 6000 pairs, tiles of 128, a Kudurax prompt of 1000: 1616 -> 1608 us, of 800: 1558 -> 1530, of 1500: 1977 -> 1963).
 // XB: the activations are bfloat16; PF: stages on their way.  With a table of tiles (grouped products) the rows of a tile share the weights of one group.
 template <int BM, int BN, int WGM, int WGN, bool XB, int PF = 1>
 __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n, int k_split) {
@@ -160,10 +162,8 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
     out.dst = out.bf16 ? (void *)(reinterpret_cast<uint16_t *>(out.dst) + blockIdx.z * out.batch) : (void *)(reinterpret_cast<float *>(out.dst) + blockIdx.z * out.batch);
     const int n0 = tn * BN;
     const int k_lo = blockIdx.y * k_split, k_hi = min(K, k_lo + k_split);
-    const int wm = (wv / WGN) * (BM / WGM), wn = (wv % WGN) * (BN / WGN);
+    const int wm = 16 * (wv / WGN), wn = (wv % WGN) * (BN / WGN);       // (sixteen rows to each of the WGM waves by turns)
 
-    u32x4 ra[PF][CA][XV];
-    u32x4 rb[PF][CB];
     const uint8_t *xp[CA];                                 // row starts, in bytes
     const uint16_t *wp[CB];
 #pragma unroll
@@ -178,88 +178,101 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
         const int c = tid + 256 * i;
         wp[i] = w + (int64_t)min(n0 + (c >> 3), N - 1) * src.ldw + (c & 7) * 8;
     }
-    auto fetch = [&](int k, auto set) {                    // (past the end: the last stage again, for nobody)
-        k = min(k, k_hi - 64);
-#pragma unroll
-        for (int i = 0; i < CB; i++) rb[set][i] = *reinterpret_cast<const u32x4 *>(wp[i] + k);
-#pragma unroll
-        for (int i = 0; i < CA; i++) {
-#pragma unroll
-            for (int j = 0; j < XV; j++) ra[set][i][j] = *reinterpret_cast<const u32x4 *>(xp[i] + (int64_t)k * (XB ? 2 : 4) + 16 * j);
-        }
-    };
-    auto stage = [&](int b, auto set) {
-#pragma unroll
-        for (int i = 0; i < CB; i++) {
-            const int c = tid + 256 * i, r = c >> 3;
-            lds[b][BM * 8 + r * 8 + ((c & 7) ^ ((r >> SW) & 7))] = __builtin_bit_cast(bf16x8, rb[set][i]);
-        }
-#pragma unroll
-        for (int i = 0; i < CA; i++) {
-            const int c = tid + 256 * i, r = c >> 3;
-            lds[b][r * 8 + ((c & 7) ^ ((r >> SW) & 7))] =
-                XB ? __builtin_bit_cast(bf16x8, ra[set][i][0]) : round_bf16(__builtin_bit_cast(f32x4, ra[set][i][0]), __builtin_bit_cast(f32x4, ra[set][i][XV - 1]));
-        }
-    };
     f32x4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    constexpr std::integral_constant<int, 0> first{};
-    constexpr std::integral_constant<int, PF == 3 ? 1 : 0> second{};
-    constexpr std::integral_constant<int, PF == 3 ? 2 : 0> third{};
-    fetch(k_lo, first);
-    if (PF == 3) {
-        fetch(k_lo + 64, second);
-        fetch(k_lo + 128, third);
-    }
-    stage(0, first);
-    if (PF > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else __syncthreads();
-    int cur = 0;
     const int lr = lane & 15, lk = lane >> 4;
-    auto step = [&](int k, auto set, auto next) {          // the stage at k, which came through `set`
-        const bool more = PF > 1 || k + 64 < k_hi;
-        if (more) fetch(k + 64 * PF, set);
+    auto run = [&](auto live) {                            // of each wave's fragments of sixteen rows the first `live` hold any
+        constexpr int LM = decltype(live)::value, LA = CA == TM ? LM : CA;
+        u32x4 ra[PF][LA][XV];
+        u32x4 rb[PF][CB];
+        auto fetch = [&](int k, auto set) {                    // (past the end: the last stage again, for nobody)
+            k = min(k, k_hi - 64);
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            bf16x8 fa[TM], fb[TN];
+            for (int i = 0; i < CB; i++) rb[set][i] = *reinterpret_cast<const u32x4 *>(wp[i] + k);
 #pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const int r = wm + 16 * i + lr;
-                fa[i] = lds[cur][r * 8 + ((4 * s + lk) ^ ((r >> SW) & 7))];
+            for (int i = 0; i < LA; i++) {
+#pragma unroll
+                for (int j = 0; j < XV; j++) ra[set][i][j] = *reinterpret_cast<const u32x4 *>(xp[i] + (int64_t)k * (XB ? 2 : 4) + 16 * j);
+            }
+        };
+        auto stage = [&](int b, auto set) {
+#pragma unroll
+            for (int i = 0; i < CB; i++) {
+                const int c = tid + 256 * i, r = c >> 3;
+                lds[b][BM * 8 + r * 8 + ((c & 7) ^ ((r >> SW) & 7))] = __builtin_bit_cast(bf16x8, rb[set][i]);
             }
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int r = wn + 16 * j + lr;
-                fb[j] = lds[cur][BM * 8 + r * 8 + ((4 * s + lk) ^ ((r >> SW) & 7))];
+            for (int i = 0; i < LA; i++) {
+                const int c = tid + 256 * i, r = c >> 3;
+                lds[b][r * 8 + ((c & 7) ^ ((r >> SW) & 7))] =
+                    XB ? __builtin_bit_cast(bf16x8, ra[set][i][0]) : round_bf16(__builtin_bit_cast(f32x4, ra[set][i][0]), __builtin_bit_cast(f32x4, ra[set][i][XV - 1]));
             }
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+        };
+        constexpr std::integral_constant<int, 0> first{};
+        constexpr std::integral_constant<int, PF == 3 ? 1 : 0> second{};
+        constexpr std::integral_constant<int, PF == 3 ? 2 : 0> third{};
+        fetch(k_lo, first);
+        if (PF == 3) {
+            fetch(k_lo + 64, second);
+            fetch(k_lo + 128, third);
         }
-        if (!more) return;
-        stage(cur ^ 1, next);
-        // (__syncthreads would wait for the stages on their way)
+        stage(0, first);
         if (PF > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         else __syncthreads();
-        cur ^= 1;
-    };
-    for (int k = k_lo; k < k_hi; k += 64 * PF) {
-        step(k, first, second);
-        if (PF == 3) {
-            if (k + 64 >= k_hi) break;
-            step(k + 64, second, third);
-            if (k + 128 >= k_hi) break;
-            step(k + 128, third, first);
+        int cur = 0;
+        auto step = [&](int k, auto set, auto next) {          // the stage at k, which came through `set`
+            const bool more = PF > 1 || k + 64 < k_hi;
+            if (more) fetch(k + 64 * PF, set);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                bf16x8 fa[LM], fb[TN];
+#pragma unroll
+                for (int i = 0; i < LM; i++) {
+                    const int r = wm + 16 * WGM * i + lr;
+                    fa[i] = lds[cur][r * 8 + ((4 * s + lk) ^ ((r >> SW) & 7))];
+                }
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const int r = wn + 16 * j + lr;
+                    fb[j] = lds[cur][BM * 8 + r * 8 + ((4 * s + lk) ^ ((r >> SW) & 7))];
+                }
+#pragma unroll
+                for (int i = 0; i < LM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+            }
+            if (!more) return;
+            stage(cur ^ 1, next);
+            // (__syncthreads would wait for the stages on their way)
+            if (PF > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else __syncthreads();
+            cur ^= 1;
+        };
+        for (int k = k_lo; k < k_hi; k += 64 * PF) {
+            step(k, first, second);
+            if (PF == 3) {
+                if (k + 64 >= k_hi) break;
+                step(k + 64, second, third);
+                if (k + 128 >= k_hi) break;
+                step(k + 128, third, first);
+            }
         }
+    };
+    // (the smaller tiles in one form: what two cost is more than what is left out, prompts of 20 to 100 through layers 1024 wide 1.012x - 1.028x slower)
+    const int frags = BM < 128 ? TM : (int)((min(M - m0, (int64_t)BM) + 16 * WGM - 1) / (16 * WGM));
+    if (frags >= TM) run(std::integral_constant<int, TM>{});
+    else if constexpr (BM == 128) {
+        if (frags == 3) run(std::integral_constant<int, 3>{});
+        else if (frags == 2) run(std::integral_constant<int, 2>{});
+        else run(std::integral_constant<int, 1>{});
     }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-        const int64_t m = m0 + wm + 16 * i + lr;
+        const int64_t m = m0 + wm + 16 * WGM * i + lr;
         if (m >= M) continue;
 #pragma unroll
         for (int j = 0; j < TN; j++) {

@@ -666,6 +666,21 @@ class GatedExperts(FeedForward):
         shared = self.shared_up.nbytes() + self.shared_down.nbytes() if self.shared_ff else 0
         return self.router.nbytes() + shared + 2 * self.top * (self.up[0].numel() + self.down[0].numel())
 
+    def tile_rows(self, pairs: int) -> int:
+        """Rows of a tile of bfloat16 products.  Weights are read once per tile of rows, and 32 rows of a tall tile that are not there cost little, so tall tiles are the better ones as soon as
+        their workgroups (tiles of 128 columns) are four rounds of two to a unit: from 20 pairs an expert on where rows are long enough for three stages on their way,
+        from 96 else; and for many pairs in any case.  Gate/up and down of unevenly loaded experts, us with 32 / 64 / 128 rows:
+            64 experts 2048 x 1408:  12 pairs an expert  210 204 209    24  231 228 224    40  272 258 246    64  333 297 281   140  533 438 366
+            64 experts 1024 x 704:   24  55 58 59    40  59 62 70    64  72 71 79   140  120 98 105
+            128 experts 1024 x 704:  28  118 119 127    48  139 136 142   100  211 182 174
+            64 experts 1536 x 1024:  40  139 135 136    64  171 151 158    94  210 180 177
+            16 experts 2048 x 1408:  20  52 48 58   140  119 96 102   200  151 120 103"""
+        per_expert, columns = pairs / self.experts, (2 * self.ff + self.width) / 128
+        filled = columns * max(self.experts, pairs / 128 + self.experts / 2) >= 2048
+        if per_expert >= 192 or (filled and per_expert >= (20 if self.kp >= 2048 else 96)):
+            return 128
+        return 64 if per_expert >= (40 if columns * self.experts >= 768 else 24) else 32
+
     def prefill(self, h, ldh, x, ldx, rows, sp):
         rt, L, E, top, bf = self.rt, self.rt.L, self.experts, self.top, int(self.rt.t_bf16)
         ldl, pairs = pad_to(self.router.n, 4), rows * top
@@ -678,8 +693,7 @@ class GatedExperts(FeedForward):
             z = rt.typed("shared_activation", rows * ld)
             self.shared_up.rows(h.typed, ldh, z, ld, rows, sp, act=ACT_SWIGLU, row_scale_dev=shared, x_bf16=bf, dst_bf16=bf)
             self.shared_down.rows(z, ld, x, ldx, rows, sp, accumulate=True, x_bf16=bf)
-        per_expert = pairs / E
-        tile = 64 if not bf else (128 if per_expert >= 96 else (64 if per_expert >= 24 else 32))
+        tile = self.tile_rows(pairs) if bf else 64
         max_tiles = L.cq_mix_moe_max_tiles(rows, E, top, tile)
         src, dst, scale = (rt.scratch("pair_" + n, pairs) for n in ("src", "dst", "scale"))
         tiles, n_tiles = rt.scratch("pair_tiles", 4 * max_tiles), rt.scratch("pair_n_tiles", 1)

@@ -209,6 +209,32 @@ def test_experts_single_token_and_rows(width, mlp):
         assert rel(xd[:, :width], want) < tol and not xd[:, width:].any()
 
 
+@pytest.mark.parametrize("tile,k", [(32, 192), (64, 192), (128, 192), (128, 1024)])
+def test_grouped_tiles_of_every_number_of_rows(tile, k):
+    """Rows at every edge of a tile's fragments, in any tile height: the sums are one chain in the order of k, so the results are the same bits as those of a full tile."""
+    rt, n = mixers.Runtime(DEV, mixers.BF16, 8), 132
+    counts = [c for c in (1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 95, 96, 97, 112, 127, 128) if c <= tile]
+    first = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    pairs, E = sum(counts), len(counts)
+    w, xs = kc.bf16(rnd(2, E, n, k)), kc.bf16(rnd(1, E, 128, k))
+    x = np.concatenate([xs[e, :c] for e, c in enumerate(counts)])
+    wd = up(w, torch.bfloat16)
+
+    def run(x, tiles, height):
+        xd, y = up(x, torch.bfloat16), torch.full((len(x) + 1, n), 7.0, device=DEV)
+        t, count = torch.tensor(tiles, dtype=torch.int32, device=DEV), torch.tensor([len(tiles)], dtype=torch.int32, device=DEV)
+        mixers.dense_product(rt, rt.precision, sp(), w_dev=wd.data_ptr(), ldw=k, w_batch=n * k, x_dev=xd.data_ptr(), ldx=k, dst_dev=y.data_ptr(), ldd=n, m=len(x), n=n, k=k, batch=1,
+                             tiles_dev=t.data_ptr(), n_tiles_dev=count.data_ptr(), max_tiles=len(tiles), tile_rows=height, x_bf16=1)
+        assert bool((y[-1] == 7.0).all())
+        return y[:-1].cpu().numpy()
+
+    got = run(x, [(e, int(first[e]), c, 0) for e, c in enumerate(counts)], tile)
+    full = run(xs.reshape(-1, k), [(e, 128 * e, 128, 0) for e in range(E)], 128).reshape(E, 128, n)
+    for e, c in enumerate(counts):
+        assert np.array_equal(got[first[e]:first[e] + c], full[e, :c]), c
+        assert rel(got[first[e]:first[e] + c], xs[e, :c].astype(np.float64) @ w[e].T) < 1e-5, c      # exact products, f32 sums of up to 1024
+
+
 # ---------------------------------------------------------------------------------------------- latent attention
 class Attention:
     """The attention of a latent mixer on given latents and queries: both forms and the single-token step, the cache filled with NaN where nothing may be read."""

@@ -195,3 +195,11 @@ def test_argument_validation_codes_without_gpu():
     assert L.cq_mix_moe_step_fits(_lib.Moe(**{**f, "kp": 65536, "up_stride": 2 * 40 * 65536})) == 0
     step = lambda norm=3, dim=64, **kw: L.cq_mix_moe_step(_lib.Moe(**{**f, **kw}), 16, norm, 16, 1e-5, dim, 16, 16, 16, None, None)
     assert step(0) == DTYPE and step(dim=65) == SHAPE and step(up_dev=None) == NULL and step(shared_ff=8, shared_ffp=64) == NULL and step(down_dev=8) == ALIGN
+
+
+@pytest.mark.parametrize("experts,width,ff,heights", [(8, 2048, 1408, {20: 32, 24: 64, 100: 64, 191: 64, 192: 128}), (64, 1024, 704, {39: 32, 40: 64, 140: 64, 192: 128}),
+                                                      (64, 2048, 1408, {19: 32, 20: 128, 140: 128}), (64, 1536, 1024, {39: 32, 40: 64, 95: 64, 96: 128})])
+def test_heights_of_expert_tiles(experts, width, ff, heights):
+    m = mixers.GatedExperts.__new__(mixers.GatedExperts)
+    m.experts, m.width, m.kp, m.ff = experts, width, width, ff
+    assert {p: m.tile_rows(p * experts) for p in heights} == heights
