@@ -111,7 +111,7 @@ class Latent(ctypes.Structure):
 class Moe(ctypes.Structure):
     """cq_moe of include/candle_hip_mixer.h."""
     _fields_ = [(n, _vp) for n in ("up_dev", "down_dev", "shared_up_dev", "shared_down_dev")] + [("up_stride", _i64), ("down_stride", _i64)] + \
-               [(n, ctypes.c_int32) for n in ("experts", "top", "kp", "ff", "ffp", "shared_ff", "shared_ffp", "reserved")]
+               [(n, ctypes.c_int32) for n in ("experts", "top", "kp", "ff", "ffp", "shared_ff", "shared_ffp", "up_ld")]
 
 
 _dense, _latent, _moe = ctypes.POINTER(DenseArgs), ctypes.POINTER(Latent), ctypes.POINTER(Moe)

@@ -187,30 +187,31 @@ __global__ __launch_bounds__(512) void moe_up_step_kernel(cq_moe g, const float 
     }
     __syncthreads();
 
-    const int total = g.top * g.ff + g.shared_ff, step = gridDim.x * 8;
+    const int total = g.top * g.ff + g.shared_ff, step = gridDim.x * 8, up_ld = g.up_ld ? g.up_ld : g.kp;
     int u = blockIdx.x * 8 + wv;
+    auto ld_of = [&](int p) { return p < g.top * g.ff ? up_ld : g.kp; };
     auto row_of = [&](int p) -> const uint16_t * {
         if (p < g.top * g.ff) {
             const int slot = p / g.ff;
-            return (const uint16_t *)g.up_dev + cid[slot] * g.up_stride + (int64_t)2 * (p - slot * g.ff) * g.kp;
+            return (const uint16_t *)g.up_dev + cid[slot] * g.up_stride + (int64_t)2 * (p - slot * g.ff) * up_ld;
         }
         return (const uint16_t *)g.shared_up_dev + (int64_t)2 * (p - g.top * g.ff) * g.kp;
     };
     u32x4 cur[2][UP_U], nxt[2][UP_U];
-    auto load = [&](const uint16_t *p, int kb, u32x4 (&d)[2][UP_U]) {
+    auto load = [&](const uint16_t *p, int ld, int kb, u32x4 (&d)[2][UP_U]) {
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int i = 0; i < UP_U; i++)
-                d[t][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p + (int64_t)t * g.kp + min(kb * UP_BLOCK + i * 512 + lane * 8, g.kp - 8)));
+                d[t][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p + (int64_t)t * ld + min(kb * UP_BLOCK + i * 512 + lane * 8, g.kp - 8)));
     };
-    if (u < total) load(row_of(u), 0, cur);
+    if (u < total) load(row_of(u), ld_of(u), 0, cur);
     for (; u < total; u += step) {
         float acc[2][2] = {};
         for (int kb = 0; kb < kb_n; kb++) {
             const bool last = kb + 1 == kb_n;
             const int next = last ? u + step : u;
-            if (next < total) load(row_of(next), last ? 0 : kb + 1, nxt);
+            if (next < total) load(row_of(next), ld_of(next), last ? 0 : kb + 1, nxt);
 #pragma unroll
             for (int i = 0; i < UP_U; i++) {
                 const f32x4 *xv = reinterpret_cast<const f32x4 *>(xs + kb * UP_BLOCK + i * 512 + lane * 8);
@@ -292,7 +293,8 @@ constexpr size_t STEP_LDS = 160 * 1024 - 4096;
 int check_moe(const cq_moe *g) {
     if (!g) return CQ_ERR_NULL;
     if (g->experts < 1 || g->top < 1 || g->top > g->experts || g->ff < 1 || g->ffp < g->ff || g->ffp % 64 || g->kp < 64 || g->kp % 64 || g->shared_ff < 0 ||
-        (g->shared_ff && (g->shared_ffp < g->shared_ff || g->shared_ffp % 64)) || g->up_stride < (int64_t)2 * g->ff * g->kp || g->up_stride % 8 || g->down_stride % 8)
+        (g->shared_ff && (g->shared_ffp < g->shared_ff || g->shared_ffp % 64)) || (g->up_ld && (g->up_ld < g->kp || g->up_ld % 8)) ||
+        g->up_stride < (int64_t)2 * g->ff * (g->up_ld ? g->up_ld : g->kp) || g->up_stride % 8 || g->down_stride % 8)
         return CQ_ERR_SHAPE;
     if (g->experts > MAX_EXPERTS || g->top > MAX_TOP) return CQ_ERR_RANGE;
     return CQ_OK;

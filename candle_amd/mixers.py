@@ -641,7 +641,10 @@ class GatedExperts(FeedForward):
         self.shared_ff = int(shared["ff"]) if shared else 0
         self.router = Dense(rt, [router] + ([get("shared.sg")] if shared else []))
         self.kp, self.ffp = pad_to(self.width, 64), pad_to(self.ff, 64)
-        self.up = torch.zeros((self.experts, 2 * self.ff, self.kp), dtype=torch.bfloat16, device=rt.device)
+        # Rows a multiple of 4096 bytes apart lie in one channel of an L2 for all of a tile: 128 bytes between them, where tiles of few rows wait for the weights (64
+        # experts of 2 * 1408 rows of 2048: 512 pairs 146 -> 131 us, 1536 pairs 151 -> 145, from 4096 on no difference; rows of 3072 bytes: none).
+        self.up_ld = self.kp + (64 if self.kp % 2048 == 0 else 0)
+        self.up = torch.zeros((self.experts, 2 * self.ff, self.up_ld), dtype=torch.bfloat16, device=rt.device)
         self.down = torch.zeros((self.experts, self.width, self.ffp), dtype=torch.bfloat16, device=rt.device)
         for e in range(self.experts):
             gate, up, down = (get(f"e{e}.{n}").to(rt.device) for n in ("gate", "up", "down"))
@@ -655,7 +658,7 @@ class GatedExperts(FeedForward):
             if self.shared_up.n != 2 * self.shared_ff or self.shared_down.k != self.shared_ff:
                 raise ValueError("shared expert sizes do not match the configuration")
         self.sizes = Moe(self.up.data_ptr(), self.down.data_ptr(), self.shared_up.w.data_ptr() if shared else None, self.shared_down.w.data_ptr() if shared else None,
-                         self.up[0].numel(), self.down[0].numel(), self.experts, self.top, self.kp, self.ff, self.ffp, self.shared_ff, self.shared_down.kp if shared else 0, 0)
+                         self.up[0].numel(), self.down[0].numel(), self.experts, self.top, self.kp, self.ff, self.ffp, self.shared_ff, self.shared_down.kp if shared else 0, self.up_ld)
         self.fused = bool(rt.L.cq_mix_moe_step_fits(self.sizes))
 
     def denses(self) -> List[Dense]:
@@ -664,7 +667,7 @@ class GatedExperts(FeedForward):
     def token_bytes(self) -> int:
         """Weight bytes of a single-token step."""
         shared = self.shared_up.nbytes() + self.shared_down.nbytes() if self.shared_ff else 0
-        return self.router.nbytes() + shared + 2 * self.top * (self.up[0].numel() + self.down[0].numel())
+        return self.router.nbytes() + shared + 2 * self.top * (2 * self.ff * self.kp + self.down[0].numel())
 
     def tile_rows(self, pairs: int) -> int:
         """Rows of a tile of bfloat16 products.  Weights are read once per tile of rows, and 32 rows of a tall tile that are not there cost little, so tall tiles are the better ones as soon as
@@ -701,7 +704,7 @@ class GatedExperts(FeedForward):
         z, ldy = rt.typed("expert_activation", pairs * self.ffp), pad_to(self.width, 4)
         y = rt.scratch("expert_out", pairs * ldy)
         grouped = dict(tiles_dev=tiles, n_tiles_dev=n_tiles, max_tiles=max_tiles, tile_rows=tile, m=pairs, batch=1)
-        dense_product(rt, rt.precision, sp, w_dev=self.up.data_ptr(), ldw=self.kp, w_batch=self.up[0].numel(), x_dev=h.typed, ldx=ldh, dst_dev=z, ldd=self.ffp,
+        dense_product(rt, rt.precision, sp, w_dev=self.up.data_ptr(), ldw=self.up_ld, w_batch=self.up[0].numel(), x_dev=h.typed, ldx=ldh, dst_dev=z, ldd=self.ffp,
                       n=2 * self.ff, k=self.kp, src_rows_dev=src, row_scale_dev=scale, act=ACT_SWIGLU, x_bf16=bf, dst_bf16=bf, **grouped)
         dense_product(rt, rt.precision, sp, w_dev=self.down.data_ptr(), ldw=self.ffp, w_batch=self.down[0].numel(), x_dev=z, ldx=self.ffp, dst_dev=y, ldd=ldy, n=self.width,
                       k=self.ffp, dst_rows_dev=dst, x_bf16=bf, **grouped)

@@ -235,12 +235,12 @@ int cq_mix_moe_plan(const int32_t *ids_dev, const float *weights_dev, int64_t ro
 int cq_mix_moe_add(const float *y_dev, int64_t ldy, int64_t top, float *x_dev, int64_t ldx, int64_t rows, int64_t dim, void *stream);
 /* One token: x += sum of weight_e W_down,e (silu(W_gate,e f(x)) * (W_up,e f(x))) over the chosen experts, plus sigmoid(logits[experts]) times the shared one
  * (shared_ff > 0), plus `add`, with f the norm CQ_DENSE_NORM or CQ_DENSE_LAYER_NORM (vec, eps).  Two launches; the choice is part of the first.
- * Weights bfloat16: up [2 ff][kp] per expert, rows alternating gate and up; down [dim][ffp]; zero beyond dim and ff.  act_dev: top * ffp + shared_ffp
+ * Weights bfloat16: up [2 ff][kp] per expert, rows alternating gate and up, up_ld apart (0: kp); down [dim][ffp]; zero beyond dim and ff.  act_dev: top * ffp + shared_ffp
  * floats, ids_dev: top ints of scratch.  cq_mix_moe_step_fits: whether the sizes fit the launches (else CQ_ERR_RANGE). */
 typedef struct cq_moe {
     const void *up_dev, *down_dev, *shared_up_dev, *shared_down_dev;
     int64_t up_stride, down_stride;          /* weights from one expert to the next */
-    int32_t experts, top, kp, ff, ffp, shared_ff, shared_ffp, reserved;
+    int32_t experts, top, kp, ff, ffp, shared_ff, shared_ffp, up_ld;
 } cq_moe;
 int cq_mix_moe_step_fits(const cq_moe *g);
 int cq_mix_moe_step(const cq_moe *g, float *x_dev, int norm, const float *vec_dev, float eps, int64_t dim, const float *logits_dev, float *act_dev, int32_t *ids_dev,

@@ -235,6 +235,11 @@ def test_grouped_tiles_of_every_number_of_rows(tile, k):
         assert rel(got[first[e]:first[e] + c], xs[e, :c].astype(np.float64) @ w[e].T) < 1e-5, c      # exact products, f32 sums of up to 1024
 
 
+def test_experts_with_rows_of_weights_apart():
+    """Rows of 4096 bytes have 128 bytes between them: the single token, with a shared expert whose rows have none, and several rows."""
+    test_experts_single_token_and_rows(2048, kc.moe(5, 2, 24, 40))
+
+
 # ---------------------------------------------------------------------------------------------- latent attention
 class Attention:
     """The attention of a latent mixer on given latents and queries: both forms and the single-token step, the cache filled with NaN where nothing may be read."""

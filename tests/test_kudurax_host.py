@@ -197,6 +197,14 @@ def test_argument_validation_codes_without_gpu():
     assert step(0) == DTYPE and step(dim=65) == SHAPE and step(up_dev=None) == NULL and step(shared_ff=8, shared_ffp=64) == NULL and step(down_dev=8) == ALIGN
 
 
+def test_moe_step_refuses_rows_of_weights_that_overlap():
+    L = _lib.mixer_lib()
+    f = dict(up_dev=16, down_dev=16, up_stride=2 * 40 * 72, down_stride=64 * 64, experts=4, top=2, kp=64, ff=40, ffp=64)
+    fits = lambda **kw: L.cq_mix_moe_step_fits(_lib.Moe(**{**f, **kw}))
+    assert fits() == 1 and fits(up_ld=64) == 1 and fits(up_ld=72) == 1
+    assert fits(up_ld=56) == 0 and fits(up_ld=68) == 0 and fits(up_ld=80) == 0 and fits(up_ld=-8) == 0
+
+
 @pytest.mark.parametrize("experts,width,ff,heights", [(8, 2048, 1408, {20: 32, 24: 64, 100: 64, 191: 64, 192: 128}), (64, 1024, 704, {39: 32, 40: 64, 140: 64, 192: 128}),
                                                       (64, 2048, 1408, {19: 32, 20: 128, 140: 128}), (64, 1536, 1024, {39: 32, 40: 64, 95: 64, 96: 128})])
 def test_heights_of_expert_tiles(experts, width, ff, heights):
