@@ -14,6 +14,9 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 constexpr int QT_NW = 8;                                 // waves of a workgroup, side by side along n
 constexpr int QT_NW_NARROW = 4;                          // of a narrow one
 
+// Floats from one row of a plane of split sums to the next: rows begin on 16 bytes whatever n is, so that four columns at a time are added up.
+__host__ __device__ constexpr int64_t qt_plane_ld(int64_t n) { return (n + 3) & ~(int64_t)3; }
+
 // everything that goes into these sums is worked out before what follows (the scheduler would rather work on all tiles at once, out of
 // registers that are not there)
 __device__ __forceinline__ void qt_pin(f32x16 &v) {
@@ -23,7 +26,7 @@ __device__ __forceinline__ void qt_pin(f32x16 &v) {
 }
 
 // Results of a wave: column nn of rows m0 .., in the layout of the 32 x 32 matrix instructions (row 8 (e / 4) + 4 kg + e % 4 of each tile).
-// MOE: rows of the expert-sorted list, scattered to their pairs' rows and scaled.  Splits of K after the first write f32 planes [rows, n].
+// MOE: rows of the expert-sorted list, scattered to their pairs' rows and scaled.  Splits of K after the first write f32 planes [rows, qt_plane_ld(n)].
 template <int MI, bool MOE>
 __device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int dst_dtype, int m0, int rows, int nn, int n, int kg, int64_t stride_dst, float *planes,
                                          const MoeChunks &mc) {
@@ -41,8 +44,8 @@ __device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int
         store([&](int mm, float v) { ((float *)dst)[(int64_t)mc.pair_out[mm] * stride_dst + nn] = v * mc.pair_scale[mm]; });
     } else {
         if (dst_dtype == CQ_F32 || blockIdx.z > 0) {
-            float *const out = (blockIdx.z > 0 ? planes + (int64_t)(blockIdx.z - 1) * rows * n : (float *)dst) + nn;
-            const int64_t ld = blockIdx.z > 0 ? n : stride_dst;
+            float *const out = (blockIdx.z > 0 ? planes + (int64_t)(blockIdx.z - 1) * rows * qt_plane_ld(n) : (float *)dst) + nn;
+            const int64_t ld = blockIdx.z > 0 ? qt_plane_ld(n) : stride_dst;
             store([&](int mm, float v) { out[mm * ld] = v; });
         } else if (dst_dtype == CQ_F16) store([&](int mm, float v) { ((uint16_t *)dst)[nn + mm * stride_dst] = f2h_bits(v); });
         else store([&](int mm, float v) { ((uint16_t *)dst)[nn + mm * stride_dst] = f2bf_bits(v); });

@@ -648,15 +648,17 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
 
 // The sum of the splits of K in a fixed order, in pairs and pairs of pairs: sixteen sums added one after the other round more than the chain of super-blocks
 // that they were cut from (Q6_K rows of 4096: 8.5e-8 of the results' norm against 6.2e-8 in four splits; in pairs 6.2e-8).  The first split comes from
-// `first` (dst itself or a plane), the others from planes; n % 4 == 0.  Bound by the latency of the reads at the sizes that are split: four planes are on their way at
-// a time, and a workgroup is small enough that 32 x 4096 results fill the chip.
+// `first` (dst itself or a plane), the others from planes, whose rows are qt_plane_ld(n) long.  Bound by the latency of the reads at the sizes that are split: four planes are on their way at
+// a time, and a workgroup is small enough that 32 x 4096 results fill the chip.  RAGGED: n is no multiple of four (with its bounds in every case the others took 0.2 - 0.5 us more, 2 - 4 %).
 constexpr int QT_RT = 128, QT_MAX_SPLITS = 16;
-template <int ODT>
+template <int ODT, bool RAGGED>
 __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first, int64_t ld_first, const float *__restrict__ planes, void *dst, int splits, int64_t n,
                                                              int64_t stride_dst, int64_t count) {
     const int64_t i = ((int64_t)blockIdx.x * QT_RT + threadIdx.x) * 4;
     if (i >= count) return;
-    const int64_t r = i / n, c0 = i - r * n, o = r * stride_dst + c0;
+    const int64_t ld_plane = RAGGED ? qt_plane_ld(n) : n;
+    const int64_t r = i / ld_plane, c0 = i - r * ld_plane, o = r * stride_dst + c0;
+    const int here = RAGGED ? (int)min((int64_t)4, n - c0) : 4;      // columns behind n are not there
     const float none = -0.0f;                              // (x + -0 is x)
     f32x4 sum[QT_MAX_SPLITS / 4];
 #pragma unroll
@@ -668,7 +670,7 @@ __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first,
         for (int u = 0; u < 4; u++) {
             if (4 * g + u == 0) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) b[u][c] = first[r * ld_first + c0 + c];
+                for (int c = 0; c < 4; c++) b[u][c] = c < here ? first[r * ld_first + c0 + c] : 0.0f;
             } else b[u] = *reinterpret_cast<const f32x4 *>(planes + (min(4 * g + u, splits - 1) - 1) * count + i);
         }
 #pragma unroll
@@ -679,6 +681,7 @@ __global__ __launch_bounds__(QT_RT) void qtile_reduce_kernel(const float *first,
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
+        if (c >= here) break;
         const float a = (sum[0][c] + sum[1][c]) + (sum[2][c] + sum[3][c]);
         if (ODT == CQ_F32) ((float *)dst)[o + c] = a;
         else ((uint16_t *)dst)[o + c] = ODT == CQ_F16 ? f2h_bits(a) : f2bf_bits(a);
@@ -740,8 +743,8 @@ bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
 // Bytes of split planes that a call may use, not falling with the rows.
 static constexpr int64_t QT_PLANE_FLOATS = 12 << 20;
 int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
-    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K && w_dtype != CQ_Q4_0 && w_dtype != CQ_Q8_0) || n % 4 || k < (w_dtype == CQ_Q6K ? QT_Q6K_MIN_K : 512) || k % 256) return 0;
-    return cq_align256(std::min<int64_t>(16 * rows * n, QT_PLANE_FLOATS) * 4);
+    if ((w_dtype != CQ_Q4K && w_dtype != CQ_Q5K && w_dtype != CQ_Q6K && w_dtype != CQ_Q4_0 && w_dtype != CQ_Q8_0) || k < (w_dtype == CQ_Q6K ? QT_Q6K_MIN_K : 512) || k % 256) return 0;
+    return cq_align256(std::min<int64_t>(16 * rows * qt_plane_ld(n), QT_PLANE_FLOATS) * 4);
 }
 
 // Rows of the tile (32 mi), waves of a workgroup and K splits: the choice for which the model
@@ -753,6 +756,8 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
 // is 0.2 - 0.7 % slower than the best on average, at most 11 %.  Q4_0 and Q8_0 (rounds that leave compute units idle run at a higher clock
 // there, and a workgroup has 1.3 us of its own): 3800 launches of 17 - 2048 rows, 0.2 - 1.2 %.
 // Only splits whose sums round no more than those of the general kernels (qt_roundings).
+// Any number of columns: while those that are no multiple of four were not split, their few workgroups walked all of k (26 rows of Q4_0 [2986 x 9984] 112 us, 19 in splits; 10 rows of
+// Q8_0 [1299 x 9728] 113 -> 18, 65 of Q6_K [1970 x 13568] 126 -> 28, 239 of Q8_0 [2818 x 13056] 152 -> 58; 1494 rows of Q8_0 [3987 x 6144] 154 -> 140).
 struct QtPlan { int mi, nw, splits; };
 // What the f32 sums of one result round, as twice a variance in units of one term's: a chain of c terms takes c fma's, which round partial sums of 1 .. c terms
 // (the first one, a product alone, like one and a half), and every addition of two splits rounds a sum of as many terms as both have.  in_pairs: as
@@ -779,7 +784,7 @@ static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_
     const bool kq = cq_is_kquant(w_dtype);
     const Cost &c = w_dtype == CQ_Q4K ? q4k : w_dtype == CQ_Q5K ? q5k : w_dtype == CQ_Q6K ? q6k : q0;
     const double plane = (double)rows * n * 4;
-    const int most = n % 4 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({QT_MAX_SPLITS, nsb, most_splits}));
+    const int most = (int)std::max<int64_t>(1, std::min<int64_t>({QT_MAX_SPLITS, nsb, most_splits}));
     const int terms = kq ? 1 : 8;
     const int general = std::min(most, cq_qmm_splits(k, n, rows));
     bool rounds_less[QT_MAX_SPLITS + 1];
@@ -805,22 +810,22 @@ int cq_qtile_launch(int w_dtype, const void *w, const ActView &av, void *dst, in
                     int64_t plane_bytes, hipStream_t s) {
     // an f32 dst takes the first split itself
     const bool f32 = dst_dtype == CQ_F32;
-    const QtPlan plan = qtile_plan(w_dtype, k, n, rows, planes ? (f32 ? 1 : 0) + plane_bytes / (4 * rows * n) : 1);
+    const QtPlan plan = qtile_plan(w_dtype, k, n, rows, planes ? (f32 ? 1 : 0) + plane_bytes / (4 * rows * qt_plane_ld(n)) : 1);
     const int splits = plan.splits;
     const dim3 grid((unsigned)((rows + 32 * plan.mi - 1) / (32 * plan.mi)), (unsigned)((n + 32 * plan.nw - 1) / (32 * plan.nw)), (unsigned)splits);
     if (grid.y > 65535) return CQ_ERR_RANGE;
-    const int64_t count = rows * n;
+    const int64_t ld_plane = qt_plane_ld(n), count = rows * ld_plane;
     const bool direct = splits == 1 || f32;
     void *const first = direct ? dst : planes;
-    const int64_t ld = direct ? stride_dst : n;
+    const int64_t ld = direct ? stride_dst : ld_plane;
     float *const others = direct ? (float *)planes : (float *)planes + count;
     const MoeChunks none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
     const int rc = qtile_any(w_dtype, plan.mi, plan.nw, false, grid, w, av, first, direct ? dst_dtype : CQ_F32, k, n, rows, ld, none, 0, others, s);
     if (rc || splits == 1) return rc;
     const dim3 rg((unsigned)((count / 4 + QT_RT - 1) / QT_RT));
-    if (f32) hipLaunchKernelGGL(qtile_reduce_kernel<CQ_F32>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
-    else if (dst_dtype == CQ_F16) hipLaunchKernelGGL(qtile_reduce_kernel<CQ_F16>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
-    else hipLaunchKernelGGL(qtile_reduce_kernel<CQ_BF16>, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
+    auto *const add_up = n % 4 ? (f32 ? qtile_reduce_kernel<CQ_F32, true> : dst_dtype == CQ_F16 ? qtile_reduce_kernel<CQ_F16, true> : qtile_reduce_kernel<CQ_BF16, true>)
+                               : (f32 ? qtile_reduce_kernel<CQ_F32, false> : dst_dtype == CQ_F16 ? qtile_reduce_kernel<CQ_F16, false> : qtile_reduce_kernel<CQ_BF16, false>);
+    hipLaunchKernelGGL(add_up, rg, dim3(QT_RT), 0, s, (const float *)first, ld, others, dst, splits, n, stride_dst, count);
     return (int)hipGetLastError();
 }
 
@@ -835,10 +840,10 @@ static int swiglu_go(int mi, dim3 grid, const void *w, const ActView &av, float 
 }
 static bool swiglu_plan(int w_dtype, const void *w_gate, const void *w_up, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes, QtPlan &plan) {
     if (!cq_is_kquant(w_dtype) || !cq_qtile_takes(w_dtype, w_gate, k, n) || !cq_qtile_takes(w_dtype, w_up, k, n) || (n + 16 * QT_NW - 1) / (16 * QT_NW) > 65535) return false;
-    plan = qtile_plan(w_dtype, k, 2 * n, rows, 1 + plane_bytes / (8 * rows * n));
+    plan = qtile_plan(w_dtype, k, 2 * n, rows, 1 + plane_bytes / (4 * rows * qt_plane_ld(2 * n)));
     if (plan.splits > 1 || plan.mi < 3 || plan.nw != QT_NW) return false;
     const bool adjacent = (const uint8_t *)w_up - (const uint8_t *)w_gate == n * (k / 256) * cq_type_size(w_dtype);
-    return adjacent || qtile_plan(w_dtype, k, n, rows, 1 + plane_bytes / (4 * rows * n)).splits == 1;
+    return adjacent || qtile_plan(w_dtype, k, n, rows, 1 + plane_bytes / (4 * rows * qt_plane_ld(n))).splits == 1;
 }
 bool cq_qtile_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes) {
     QtPlan plan;

@@ -41,13 +41,13 @@ template <int DT, int MI> struct Q0Lds {
 };
 
 // Results of a wave: row m0 + 32 t + nr of each tile, columns n0 + 8 e4 + 4 kg .. + 3: four at a time.  MOE: rows of the expert-sorted list, scattered to their pairs' rows and
-// scaled.  Splits of K after the first write f32 planes [rows, n].
+// scaled.  Splits of K after the first write f32 planes [rows, qt_plane_ld(n)].
 template <int MI, bool MOE>
 __device__ __forceinline__ void q0_store(const f32x16 (&acc)[MI], void *dst, int dst_dtype, int m0, int rows, int nr, int n0, int n, int kg, int64_t stride_dst, float *planes,
                                          const MoeChunks &mc) {
     const bool plane = !MOE && blockIdx.z > 0;
-    if (plane) dst = planes + (int64_t)(blockIdx.z - 1) * rows * n;
-    const int64_t ld = plane ? n : stride_dst;
+    if (plane) dst = planes + (int64_t)(blockIdx.z - 1) * rows * qt_plane_ld(n);
+    const int64_t ld = plane ? qt_plane_ld(n) : stride_dst;
 #pragma unroll
     for (int t = 0; t < MI; t++) {
         const int mm = m0 + 32 * t + nr;

@@ -67,7 +67,7 @@ def check(fmt, m, n, k, out=0, shift=0, room=None):
 @pytest.mark.parametrize("m,n,k", [(66, 256, 256), (65, 1, 512), (97, 257, 768), (128, 31, 2304), (129, 260, 1280), (70, 292, 14336), (300, 510, 512), (65, 2, 1536), (97, 257, 2048), (129, 260, 1792),
                                    (300, 512, 1536)])
 def test_tile_edges(fmt, m, n, k):
-    # one row past a 32-row tile, one column past a workgroup's 256, one super-block, odd numbers of them, k split over workgroups (n % 4 == 0) and not;
+    # one row past a 32-row tile, one column past a workgroup's 256, one super-block, odd numbers of them, k split over workgroups and not;
     # Q6_K of less than 1536 of k or with an odd number of blocks (n k / 256 odd) takes the general kernel
     check(fmt, m, n, k)
 
@@ -158,6 +158,16 @@ def test_half_results(fmt, out, n, k):
 @pytest.mark.parametrize("m,n,k", [(33, 131, 512), (101, 70, 768), (70, 291, 2304)])
 def test_rows_of_results_off_four_columns(fmt, out, m, n, k):
     check(fmt, m, n, k, out)                               # four columns at a time on any element, the last one to three alone
+
+
+@pytest.mark.parametrize("fmt", FMT)
+@pytest.mark.parametrize("out", [0, 1, 30])
+@pytest.mark.parametrize("m,n,k", [(17, 1, 4096), (70, 291, 9984), (33, 1026, 2304), (131, 515, 14336)])
+def test_split_sums_of_any_number_of_columns(fmt, out, m, n, k):
+    """Planes have rows of whole fours of columns, the result has not: nothing behind a row's last column is read or written."""
+    L = _lib.lib()
+    assert L.cq_qmatmul_workspace_bytes(FMT[fmt][0], m, k, n) > L.cq_act_scratch_bytes(FMT[fmt][0], k, m) + 4 * m * n
+    check(fmt, m, n, k, out)
 
 
 @pytest.mark.parametrize("fmt", FMT)
