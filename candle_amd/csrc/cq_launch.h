@@ -188,6 +188,8 @@ int cq_moe_stream_launch(int w_dtype, const void *w_a, const void *w_b, float *o
 bool cq_qtile_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes);
 int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *dst, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes,
                            hipStream_t s);
-int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s);
+// num_experts, pairs: what the number of tiles that hold rows follows from
+int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows,
+                        hipStream_t s);
 int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,
                          int64_t n, int tile_rows, hipStream_t s);

@@ -768,7 +768,7 @@ int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_
     // against 37.5, 800 on 128 of 768 x 2048 58.8 against 59.7; of 2048 x 768 it is the slower one, 64.8 against 53.9, and the other formats' at any: Q8_0
     // 33.9 against 30.2, 94.8 against 74.2)
     const bool narrow = w_dtype == CQ_Q4_0 && tile_rows == CQ_MOE_TILE_SMALL && n <= 1024;
-    if (!narrow && cq_qtile_takes(w_dtype, w, k, num_experts * n)) return cq_qtile_moe_launch(w_dtype, w, av, out, mc, k, n, tile_rows, s);
+    if (!narrow && cq_qtile_takes(w_dtype, w, k, num_experts * n)) return cq_qtile_moe_launch(w_dtype, w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
     switch (w_dtype) {
         case CQ_Q4_0: return launch_qmm_moe<CQ_Q4_0>(w, av, out, mc, k, n, tile_rows, s);
         case CQ_Q8_0: return launch_qmm_moe<CQ_Q8_0>(w, av, out, mc, k, n, tile_rows, s);

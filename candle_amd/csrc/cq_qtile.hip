@@ -718,6 +718,7 @@ int qtile_mi(int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &
 #undef QT_GO
 }
 
+// rows: of grouped products the tiles to be expected (their kernels have the rows from mc)
 int qtile_any(int w_dtype, int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows,
               int64_t stride_dst, const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
     switch (w_dtype) {
@@ -864,8 +865,11 @@ int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, co
 }
 
 // tile_rows: rows of one chunk of the table, 32 or 128
-int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s) {
+int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows,
+                        hipStream_t s) {
     const dim3 grid((unsigned)mc.max_chunks, (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)));
     if (grid.y > 65535) return CQ_ERR_RANGE;
-    return qtile_any(w_dtype, tile_rows / 32, QT_NW, true, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
+    // tiles to be expected: every expert's last one is half full, and few experts have none
+    const int64_t tiles = std::max(std::min(num_experts, pairs), pairs / tile_rows + num_experts / 2);
+    return qtile_any(w_dtype, tile_rows / 32, QT_NW, true, grid, w, av, out, CQ_F32, k, n, tiles, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
 }

@@ -9,16 +9,16 @@
 //
 // A workgroup's eight waves lie side by side along n and share 32 MI rows of activations in LDS (two super-blocks of 256, swizzled so that fragments are read
 // without bank conflicts); a wave owns 32 weight rows, brings their blocks for itself by copies to LDS, half a super-block at a time, and converts each
-// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  The weights are the matrix instructions' first operand, so that a
-// lane has sixteen weight rows' results of one activation row: the sixteen scales of the weights, put into LDS as f32 by the wave itself, are read once per block for all
-// tiles and one scale of the activations per tile.  (The other way round four reads of 16 bytes per tile and block brought the activations' scales, right in front of their
-// use: Q8_0, 2048 rows of [4096 x 14336] 457 us for 421.)  Results go out four columns at a time, whatever n is a multiple of.  K is split over grid.z where that fills the
-// chip better; see qtile_plan.
+// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  WF: the weights are the matrix instructions' first
+// operand, so that a lane has sixteen weight rows' results of one activation row: the sixteen scales of the weights, put into LDS as f32 by the wave itself, are read once per
+// block for all tiles and one scale of the activations per tile.  (The other way round four reads of 16 bytes per tile and block bring the activations' scales, right in front of
+// their use, but a weight row's scale comes with its weights: the better way for some tiles of 32 rows, see launch_mi.)  Results then go out four columns at a time, whatever n
+// is a multiple of.  K is split over grid.z where that fills the chip better; see qtile_plan.
 //
-// us, with the activations first / now, quantizing the activations included:        17 rows   131 rows   512 rows   2048 rows
-//   Q4_0 [14336 x 4096]                                                           23.8 24.1  61.0 57.8  122 115    455 435
-//   Q8_0 [14336 x 4096]                                                           26.3 26.3  66.3 59.9  134 121    504 461
-// 2048 rows of Q4_0 are 550 TOP/s.  A block of 32 x 32 results takes 198 cycles of a SIMD where its 32 fmas and a matrix instruction take 138 (on an eighth of the units; with all of
+// us on one card, the activations first in all tiles / now, quantizing the activations included:      17 rows   131 rows   512 rows   2048 rows
+//   Q4_0 [14336 x 4096]                                                                              23.5 23.7  57.6 53.7  108 103    412 393
+//   Q8_0 [14336 x 4096]                                                                              27.3 27.3  62.6 56.1  121 111    464 420
+// 2048 rows of Q4_0 are 610 TOP/s.  A block of 32 x 32 results takes 198 cycles of a SIMD where its 32 fmas and a matrix instruction take 138 (on an eighth of the units; with all of
 // them busy the clock falls by a sixth): beside them the conversion of the weights from LDS places on 2 bytes (27 of 296 us), the scales (20) and the fragments (13).
 #include "cq_qtile.h"
 
@@ -34,9 +34,9 @@ typedef f32x4 f32x4_at4 __attribute__((aligned(4)));       // (rows of results b
 typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
 
 constexpr uint32_t Q0_MAGIC = 0x4b400000u;                 // 12582912.0f
-template <int DT, int MI> struct Q0Lds {
+template <int DT, int MI, bool WF> struct Q0Lds {
     static constexpr int NI = (32 * Q0Tile<DT>::PPR + 63) / 64;          // copy instructions per wave and half of weights
-    static constexpr int A = MI * 8192, B = NI * 1024, D8 = 8 * 32 * MI * 4, DW = 8 * 32 * 4;
+    static constexpr int A = MI * 8192, B = NI * 1024, D8 = 8 * 32 * MI * 4, DW = WF ? 8 * 32 * 4 : 0;
     static constexpr int A_OFF = 0, B_OFF = 2 * A, D8_OFF = B_OFF + 2 * QT_NW * B, DW_OFF = D8_OFF + 2 * D8, BYTES = DW_OFF + QT_NW * DW;
 };
 
@@ -81,12 +81,14 @@ __device__ __forceinline__ void q0_store(const f32x16 (&acc)[MI], void *dst, int
     }
 }
 
-template <int DT, int MI, bool MOE>
+// WF: the weights are the first operand
+template <int DT, int MI, bool MOE, bool WF>
 __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__restrict__ w, ActView av, void *__restrict__ dst, int dst_dtype, int k, int n,
                                                                int rows, int64_t stride_dst, MoeChunks mc, int64_t expert_bytes, float *__restrict__ planes) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler has no use for the body, and does not know its buffer accesses)
     typedef Q0Tile<DT> T;
-    typedef Q0Lds<DT, MI> LD;
+    typedef Q0Lds<DT, MI, WF> LD;
+    static_assert(WF || MI == 1, "the other order is for tiles of 32 rows");
     constexpr int BB = T::BB, NI = LD::NI, RS = 16 * T::PPR, BM = 32 * MI, BN = 32 * QT_NW, NA = MI, ND = (8 * MI * 32 / 64 + QT_NW - 1) / QT_NW;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -168,98 +170,143 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
     bool wild = false;
     const int live = (min(rows - m0, BM) + 31) / 32;       // 32-row tiles that hold rows
     const uint32_t nib = 4 - 4 * kg;                       // Q4_0: the lower lanes take the low nibbles
-    // ---- scales of the weights: [8 blocks][32 rows] of f32 in LDS, since a lane has results of sixteen rows ----
-    uint8_t *const my_dw = lds + LD::DW_OFF + wv * LD::DW;
-    auto row_scales = [&](int h) {                         // of the half that has landed: blocks 4 h + 2 kg and the one behind it
+    // this lane's 16 weights of block b, and a block's fragment of the activations
+    auto operand = [&](int b, i32x4 &op) {
+        const uint8_t *const blk = lds + my_row + ((b >> 2) * (LD::B + 8) + (b & 3) * BB);
+        if constexpr (DT == CQ_Q4_0) {
+            // nibbles as 16 (q - 8): the high ones where they are, the low ones moved up
+            const u32x4 q = *reinterpret_cast<const u32x4_at2 *>(blk + 2);
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            float v = h2f(*reinterpret_cast<const uint16_t *>(lds + my_row + (h * (LD::B + 8) + i * BB) + 2 * kg * BB));
-            if (DT == CQ_Q4_0) v *= 0.0625f;
-            wild |= !(__builtin_fabsf(v) < __builtin_inff());
-            *reinterpret_cast<float *>(my_dw + 128 * (4 * h + i) + 256 * kg + 4 * nr) = v;
+            for (int i = 0; i < 4; i++) op[i] = (int)(((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u);
+        } else {
+            op = __builtin_bit_cast(i32x4, (u32x4)*reinterpret_cast<const u32x4_at2 *>(blk + 2 + 16 * kg));
         }
-        asm volatile("" ::: "memory");                     // (other lanes read them; a wave's LDS accesses keep their order)
     };
-    auto scales_of = [&](int b, f32x4 (&d)[4]) {
-#pragma unroll
-        for (int e4 = 0; e4 < 4; e4++) d[e4] = *reinterpret_cast<const f32x4 *>(my_dw + 128 * b + 32 * e4 + 16 * kg);
+    auto a_frag = [&](int slot, int b, int t) {
+        return *reinterpret_cast<const i32x4 *>(lds + LD::A_OFF + slot * LD::A + nr * 64 + (b >> 1) * (MI * 2048) + t * 2048 + 16 * ((2 * (b & 1) + kg) ^ ((nr >> 2) & 3)));
     };
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    row_scales(0);
-    f32x4 dw[4];
-    scales_of(0, dw);
-    for (int j = 0; j < nsb; j++) {
-        const int kb = kb0 + j, slot = j & 1;
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        issue_w(kb, 1);
-        request(j + 1);
-        const uint8_t *const Aj = lds + LD::A_OFF + slot * LD::A + nr * 64, *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 4 * nr;
-        // this lane's 16 weights of block b
-        auto operand = [&](int b, i32x4 &op) {
-            const uint8_t *const blk = lds + my_row + ((b >> 2) * (LD::B + 8) + (b & 3) * BB);
-            if constexpr (DT == CQ_Q4_0) {
-                // nibbles as 16 (q - 8): the high ones where they are, the low ones moved up
-                const u32x4 q = *reinterpret_cast<const u32x4_at2 *>(blk + 2);
+    if constexpr (!WF) {
+        // ---- a lane has results of one weight row, whose scale comes with its weights ----
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        for (int j = 0; j < nsb; j++) {
+            const int kb = kb0 + j, slot = j & 1;
+            if (j > 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            issue_w(kb, 1);
+            request(j + 1);
+            const uint8_t *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 16 * kg;
+            auto row_scale = [&](int b) {
+                const float v = h2f(*reinterpret_cast<const uint16_t *>(lds + my_row + ((b >> 2) * (LD::B + 8) + (b & 3) * BB)));
+                return DT == CQ_Q4_0 ? v * 0.0625f : v;
+            };
+            i32x4 op;
+            float dw = row_scale(0);
+            operand(0, op);
+            i32x16 S = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_frag(slot, 0, 0), op, magic, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) op[i] = (int)(((q[i] << nib) ^ 0x80808080u) & 0xf0f0f0f0u);
-            } else {
-                op = __builtin_bit_cast(i32x4, (u32x4)*reinterpret_cast<const u32x4_at2 *>(blk + 2 + 16 * kg));
-            }
-        };
-        auto a_frag = [&](int b, int t) {
-            return *reinterpret_cast<const i32x4 *>(Aj + (b >> 1) * (MI * 2048) + t * 2048 + 16 * ((2 * (b & 1) + kg) ^ ((nr >> 2) & 3)));
-        };
-        auto d8_of = [&](int b, float (&d)[MI]) {
+            for (int b = 0; b < 8; b++) {
+                // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
+                if (b == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+                if (b == 4) issue_w(kb + 1, 0);
+                const float c = -12582912.0f * dw;
+                wild |= !(__builtin_fabsf(dw) < __builtin_inff());
+                i32x4 op_n;
+                float dw_n = 0.0f;
+                if (b < 7) {
+                    dw_n = row_scale(b + 1);
+                    operand(b + 1, op_n);
+                }
+                f32x4 d8[4];
 #pragma unroll
-            for (int t = 0; t < MI; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
-        };
-        // The sums of block b + 1 are on their way in the matrix cores while those of block b are scaled, tile by tile.
-        i32x4 op;
-        i32x16 S[MI];
-        float d8[MI];
-        operand(0, op);
-        d8_of(0, d8);
-#pragma unroll
-        for (int t = 0; t < MI; t++)
-            if (t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, a_frag(0, t), magic, 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
-            if (b == 3) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
-                row_scales(1);
-            }
-            if (b == 4) issue_w(kb + 1, 0);
-            if (b == 7) {                                  // the next super-block's first half
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                row_scales(0);
-            }
-            f32x4 c[4], dw_n[4];
-#pragma unroll
-            for (int e4 = 0; e4 < 4; e4++) c[e4] = -12582912.0f * dw[e4];
-            scales_of(b == 7 ? 0 : b + 1, dw_n);
-            i32x4 op_n;
-            float d8_n[MI];
-            if (b < 7) {
-                operand(b + 1, op_n);
-                d8_of(b + 1, d8_n);
-            }
-#pragma unroll
-            for (int t = 0; t < MI; t++) {
-                if (t >= live) break;
+                for (int e4 = 0; e4 < 4; e4++) d8[e4] = *reinterpret_cast<const f32x4 *>(Dj + 4 * (b * BM + 8 * e4));
                 i32x4 af;
-                if (b < 7) af = a_frag(b + 1, t);
+                if (b < 7) af = a_frag(slot, b + 1, 0);
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
-                qt_pin(acc[t]);
-                if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op_n, af, magic, 0, 0, 0);
+                for (int e = 0; e < 16; e++) acc[0][e] = fmaf(fmaf(__int_as_float(S[e]), dw, c), d8[e >> 2][e & 3], acc[0][e]);
+                qt_pin(acc[0]);
+                if (b < 7) S = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, op_n, magic, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
+                dw = dw_n;
             }
-            op = op_n;
+        }
+    } else {
+        // ---- scales of the weights: [8 blocks][32 rows] of f32 in LDS, since a lane has results of sixteen rows ----
+        uint8_t *const my_dw = lds + LD::DW_OFF + wv * LD::DW;
+        auto row_scales = [&](int h) {                     // of the half that has landed: blocks 4 h + 2 kg and the one behind it
 #pragma unroll
-            for (int e4 = 0; e4 < 4; e4++) dw[e4] = dw_n[e4];
+            for (int i = 0; i < 2; i++) {
+                float v = h2f(*reinterpret_cast<const uint16_t *>(lds + my_row + (h * (LD::B + 8) + i * BB) + 2 * kg * BB));
+                if (DT == CQ_Q4_0) v *= 0.0625f;
+                wild |= !(__builtin_fabsf(v) < __builtin_inff());
+                *reinterpret_cast<float *>(my_dw + 128 * (4 * h + i) + 256 * kg + 4 * nr) = v;
+            }
+            asm volatile("" ::: "memory");                 // (other lanes read them; a wave's LDS accesses keep their order)
+        };
+        auto scales_of = [&](int b, f32x4 (&d)[4]) {
 #pragma unroll
-            for (int t = 0; t < MI; t++) d8[t] = d8_n[t];
+            for (int e4 = 0; e4 < 4; e4++) d[e4] = *reinterpret_cast<const f32x4 *>(my_dw + 128 * b + 32 * e4 + 16 * kg);
+        };
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        row_scales(0);
+        f32x4 dw[4];
+        scales_of(0, dw);
+        for (int j = 0; j < nsb; j++) {
+            const int kb = kb0 + j, slot = j & 1;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            issue_w(kb, 1);
+            request(j + 1);
+            const uint8_t *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 4 * nr;
+            auto d8_of = [&](int b, float (&d)[MI]) {
+#pragma unroll
+                for (int t = 0; t < MI; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
+            };
+            // The sums of block b + 1 are on their way in the matrix cores while those of block b are scaled, tile by tile.
+            i32x4 op;
+            i32x16 S[MI];
+            float d8[MI];
+            operand(0, op);
+            d8_of(0, d8);
+#pragma unroll
+            for (int t = 0; t < MI; t++)
+                if (t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, a_frag(slot, 0, t), magic, 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
+                if (b == 3) {
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+                    row_scales(1);
+                }
+                if (b == 4) issue_w(kb + 1, 0);
+                if (b == 7) {                                  // the next super-block's first half
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    row_scales(0);
+                }
+                f32x4 c[4], dw_n[4];
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) c[e4] = -12582912.0f * dw[e4];
+                scales_of(b == 7 ? 0 : b + 1, dw_n);
+                i32x4 op_n;
+                float d8_n[MI];
+                if (b < 7) {
+                    operand(b + 1, op_n);
+                    d8_of(b + 1, d8_n);
+                }
+#pragma unroll
+                for (int t = 0; t < MI; t++) {
+                    if (t >= live) break;
+                    i32x4 af;
+                    if (b < 7) af = a_frag(slot, b + 1, t);
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
+                    qt_pin(acc[t]);
+                    if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op_n, af, magic, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                op = op_n;
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) dw[e4] = dw_n[e4];
+#pragma unroll
+                for (int t = 0; t < MI; t++) d8[t] = d8_n[t];
+            }
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -298,22 +345,41 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
         }
         return;
     }
-    q0_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, nr, n0, n, kg, stride_dst, planes, mc);
+    if constexpr (!WF) qt_store<1, MOE>(acc, dst, dst_dtype, m0, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+    else q0_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, nr, n0, n, kg, stride_dst, planes, mc);
 #endif
 }
 
 }  // namespace
 
+// Which operand comes first in tiles of 32 rows (larger ones: the weights, see above).  us, activations / weights first:
+//  - Q4_0, activations: their form leaves room for two workgroups to a unit, the other for one (20 rows of [13824 x 5120] 28.0 / 31.4, of [4096 x 14336] 24.1 / 24.2).
+//    Experts whose workgroups are two full rounds are the exception, 800 pairs on 48 experts of 3072 x 1024 58.1 / 55.4 (588 to be expected), 600 on 32 of 4096 x 2048
+//    84.6 / 68.7 (544), 600 on 16 of 4096 x 4096 135 / 115 (416); but 520 there 103 / 113 (384), 600 on 64 of 1280 x 1024 37.7 / 39.6 (320), 2000 on 128 of
+//    2048 x 768 60.8 / 65.9 (1024), 2400 on 256 of 2048 x 512 74.8 / 89.6 (2048).
+//  - Q8_0, weights, whose results are stored four columns at a time (20 rows of [2048 x 2048] 11.4 / 11.3; 900 pairs on 64 experts of 1024 x 1024 30.8 / 29.1), as long as
+//    they come out of a cache: the scales of a super-block's first half are put into LDS at the end of the one before, and what comes from memory is not there yet
+//    (20 rows of [4096 x 14336] 28.1 / 28.6, of [13824 x 5120] 35.3 / 35.7; cold weights of 17 MB and less 0.3 - 1 % the other way).
+static constexpr int64_t Q0_ROUND_AND_HALF = 400, Q0_TWO_ROUNDS = 600, Q0_CACHED = 24 << 20;
 template <int DT>
 static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                      const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
-#define Q0_GO(M, E) return qtile_go(qtile0_kernel<DT, M, E>, QT_NW, Q0Lds<DT, M>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
-    if (moe) { if (mi == 1) Q0_GO(1, true); else Q0_GO(4, true); }
+#define Q0_GO(M, E, F) return qtile_go(qtile0_kernel<DT, M, E, F>, QT_NW, Q0Lds<DT, M, F>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+    if (moe) {
+        if (mi != 1) Q0_GO(4, true, true);
+        if constexpr (DT == CQ_Q4_0)
+            if (rows * grid.y <= Q0_ROUND_AND_HALF || rows * grid.y > Q0_TWO_ROUNDS) Q0_GO(1, true, false);
+        Q0_GO(1, true, true);
+    }
+    if (mi == 1) {
+        if constexpr (DT == CQ_Q8_0)
+            if (n * k <= Q0_CACHED) Q0_GO(1, false, true);
+        Q0_GO(1, false, false);
+    }
     switch (mi) {
-        case 1: Q0_GO(1, false);
-        case 2: Q0_GO(2, false);
-        case 3: Q0_GO(3, false);
-        default: Q0_GO(4, false);
+        case 2: Q0_GO(2, false, true);
+        case 3: Q0_GO(3, false, true);
+        default: Q0_GO(4, false, true);
     }
 #undef Q0_GO
 }

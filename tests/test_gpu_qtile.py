@@ -288,3 +288,71 @@ def test_matmul_of_quantized_rows(fmt, rows, n, k):
     y = y.cpu().numpy()
     assert (y[:, n:] == 77).all()
     assert row_error(y[:, :n], oracle.matmul(odt, x, blocks, n), x, w, k) <= BOUND
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("n,k", [(8197, 256), (8197, 2304), (16385, 1792)])
+def test_few_rows_keep_the_bits_of_many(fmt, n, k):
+    """Unsplit, a result is one chain of blocks: rows in a tile of 32 (whichever operand comes first there, which the size of the weights decides for Q8_0) have the bits they
+    have among 2000, in tiles of 128."""
+    from perf import cases
+    L = _lib.lib()
+    code = FMT[fmt][0]
+    w = cases.blocks(fmt, 8, "w", n, k).reshape(-1)
+    x = torch.from_numpy(normal(33 + n, (2000, k))).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+
+    def product(rows):
+        scratch = torch.empty(L.cq_act_scratch_bytes(code, k, rows), dtype=torch.uint8, device="cuda")
+        y = torch.full((rows + 1, n), 77.0, device="cuda")
+        _lib.check("cq_quantize_act", L.cq_quantize_act(code, x.data_ptr(), 0, scratch.data_ptr(), k, rows, s))
+        _lib.check("cq_matmul", L.cq_matmul(code, w.data_ptr(), scratch.data_ptr(), y.data_ptr(), k, n, rows, n, s))
+        assert bool((y[rows] == 77).all())
+        return y[:rows]
+
+    many = product(2000)
+    for rows in (9, 31, 32):
+        print(f"case {fmt} rows={rows} n={n} k={k}", flush=True)
+        assert torch.equal(product(rows), many[:rows])
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("E,n,pairs", [(16, 2052, 528), (16, 4100, 528), (16, 8196, 530), (40, 2052, 1200), (64, 2048, 1600), (33, 4097, 513)])
+def test_grouped_tiles_of_32_rows_keep_bits(fmt, E, n, pairs):
+    """Experts on either side of the limits between the two orders of operands (Q4_0): the bits of each expert's own product, which no other rows change."""
+    import candle_amd as ca
+    from perf import cases
+    L = _lib.lib()
+    code, k = FMT[fmt][0], 512
+    print(f"case {fmt} E={E} n={n} pairs={pairs}", flush=True)
+    b = cases.blocks(fmt, 9, "w", E * n, k).reshape(-1)
+    qt = ca.QTensor.new(ca.QStorage.from_data(b.cpu().numpy(), "cuda", ca.GgmlDType(FMT[fmt][1])), (E, n, k))
+    x = torch.from_numpy(normal(34, (pairs, 1, k))).cuda()
+    ids = torch.arange(pairs, dtype=torch.int32, device="cuda").reshape(-1, 1) % E
+    got = qt.indexed_moe_forward(x, ids)[:, 0]
+    per, s = b.numel() // E, torch.cuda.current_stream().cuda_stream
+    for e in (0, 1, E // 2, E - 1):
+        rows = x[e::E, 0].contiguous()
+        scratch = torch.empty(L.cq_act_scratch_bytes(code, k, len(rows)), dtype=torch.uint8, device="cuda")
+        y = torch.empty((len(rows), n), device="cuda")
+        _lib.check("cq_quantize_act", L.cq_quantize_act(code, rows.data_ptr(), 0, scratch.data_ptr(), k, len(rows), s))
+        _lib.check("cq_matmul", L.cq_matmul(code, b.data_ptr() + e * per, scratch.data_ptr(), y.data_ptr(), k, n, len(rows), n, s))
+        assert torch.equal(got[e::E], y), e
+
+
+@pytest.mark.parametrize("fmt,bb", [("q4_0", 18), ("q8_0", 34)])
+@pytest.mark.parametrize("d", [np.inf, np.nan, 65504.0])
+def test_extreme_block_scales_of_few_rows(fmt, bb, d):
+    """As test_extreme_block_scales, in one tile of 32 rows."""
+    code, odt = FMT[fmt]
+    n, k, m = 99, 512, 21
+    blocks = oracle.from_float(odt, normal(3, (n, k), 0.02).reshape(-1)).reshape(n, k // 32, bb)
+    blocks[[0, 40, 98], [0, 7, 15], :2] = np.frombuffer(np.float16(d).tobytes(), dtype=np.uint8)
+    x = normal(4, (m, k))
+    x[5, :32] = 0.0
+    want = oracle.matmul(odt, x, blocks.reshape(-1), n)
+    got = run(code, blocks.reshape(-1), x, n)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.array_equal(got[~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)])
+    assert rel_l2(got[ok], want[ok]) <= BOUND
