@@ -670,19 +670,26 @@ class GatedExperts(FeedForward):
         return self.router.nbytes() + shared + 2 * self.top * (2 * self.ff * self.kp + self.down[0].numel())
 
     def tile_rows(self, pairs: int) -> int:
-        """Rows of a tile of bfloat16 products.  Weights are read once per tile of rows, and 32 rows of a tall tile that are not there cost little, so tall tiles are the better ones as soon as
-        their workgroups (tiles of 128 columns) are four rounds of two to a unit: from 20 pairs an expert on where rows are long enough for three stages on their way,
-        from 96 else; and for many pairs in any case.  Gate/up and down of unevenly loaded experts, us with 32 / 64 / 128 rows:
-            64 experts 2048 x 1408:  12 pairs an expert  210 204 209    24  231 228 224    40  272 258 246    64  333 297 281   140  533 438 366
-            64 experts 1024 x 704:   24  55 58 59    40  59 62 70    64  72 71 79   140  120 98 105
-            128 experts 1024 x 704:  28  118 119 127    48  139 136 142   100  211 182 174
-            64 experts 1536 x 1024:  40  139 135 136    64  171 151 158    94  210 180 177
-            16 experts 2048 x 1408:  20  52 48 58   140  119 96 102   200  151 120 103"""
-        per_expert, columns = pairs / self.experts, (2 * self.ff + self.width) / 128
-        filled = columns * max(self.experts, pairs / 128 + self.experts / 2) >= 2048
-        if per_expert >= 192 or (filled and per_expert >= (20 if self.kp >= 2048 else 96)):
-            return 128
-        return 64 if per_expert >= (40 if columns * self.experts >= 768 else 24) else 32
+        """Rows of a tile of bfloat16 products.  Weights are read once per tile of rows, and 32-row parts of a tall tile that are not there are neither brought nor multiplied, so tall
+        tiles are the better ones soon: 128 rows from 32 pairs an expert on, 64 from 24.  Not so soon where rows are short (11 to 23 stages of 64, of which the beginning and
+        the end of a workgroup are more) or a row tile of every expert, in 128 columns, is less than 768 workgroups; where it is not one round of two to a unit, the more workgroups the better
+        until tall tiles fill that.  A layer of prompts, its router and sums included, us with 32 / 64 / 128 rows, experts evenly loaded, and by a router whose rows' lengths vary by 15 %:
+            experts x width x ff    pairs an expert
+            64 x 2048 x 1408        16  235 230 235, 241 232 236    24  247 240 242, 252 245 250    32  278 251 255, 275 255 259    40  301 261 264, 296 279 268    96  437 384 321, 433 398 363
+            8 x 4096 x 4096         24  184 186 186, 186 187 186    32  201 198 194, 237 193 192    56  264 248 205, 263 252 207    150  424 375 307, 419 377 288
+            256 x 2048 x 512        24  375 379 385, 381 393 394    32  415 395 406, 417 416 418    64  564 539 501, 568 538 524
+            64 x 1024 x 704         24  81 86 89, 85 88 91    32  91 91 95, 90 91 95    40  98 94 99, 99 102 101    56  109 111 109, 113 113 113    150  195 183 179, 198 179 175
+            16 x 2048 x 1408        24  77 79 82, 77 79 82    32  85 81 85, 81 81 86    48  96 84 89, 93 86 93    64  120 116 97, 121 120 98    150  170 170 140, 171 154 148
+            8 x 2048 x 1408         64  63 67 71, 63 64 71    96  71 69 81, 71 69 81    150  95 91 97, 93 91 97    220  111 100 99, 118 102 102
+        Seventeen shapes of experts, 8 to 220 pairs each: 0.3 % slower than the best of the three on average, 6 % at most."""
+        per_expert, workgroups = pairs / self.experts, (2 * self.ff + self.width) / 128 * self.experts
+        if workgroups < 512:
+            middle, tall = 90, 200
+        elif workgroups < 768 or self.kp < 1536:
+            middle, tall = 30, 56
+        else:
+            middle, tall = 24, 32
+        return 128 if per_expert >= tall else 64 if per_expert >= middle else 32
 
     def prefill(self, h, ldh, x, ldx, rows, sp):
         rt, L, E, top, bf = self.rt, self.rt.L, self.experts, self.top, int(self.rt.t_bf16)
