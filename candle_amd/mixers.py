@@ -641,9 +641,7 @@ class GatedExperts(FeedForward):
         self.shared_ff = int(shared["ff"]) if shared else 0
         self.router = Dense(rt, [router] + ([get("shared.sg")] if shared else []))
         self.kp, self.ffp = pad_to(self.width, 64), pad_to(self.ff, 64)
-        # Rows a multiple of 4096 bytes apart lie in one channel of an L2 for all of a tile: 128 bytes between them, where tiles of few rows wait for the weights (64
-        # experts of 2 * 1408 rows of 2048: 512 pairs 146 -> 131 us, 1536 pairs 151 -> 145, from 4096 on no difference; rows of 3072 bytes: none).
-        self.up_ld = self.kp + (64 if self.kp % 2048 == 0 else 0)
+        self.up_ld = self.row_distance(self.experts, self.kp, self.ff)
         self.up = torch.zeros((self.experts, 2 * self.ff, self.up_ld), dtype=torch.bfloat16, device=rt.device)
         self.down = torch.zeros((self.experts, self.width, self.ffp), dtype=torch.bfloat16, device=rt.device)
         for e in range(self.experts):
@@ -660,6 +658,14 @@ class GatedExperts(FeedForward):
         self.sizes = Moe(self.up.data_ptr(), self.down.data_ptr(), self.shared_up.w.data_ptr() if shared else None, self.shared_down.w.data_ptr() if shared else None,
                          self.up[0].numel(), self.down[0].numel(), self.experts, self.top, self.kp, self.ff, self.ffp, self.shared_ff, self.shared_down.kp if shared else 0, self.up_ld)
         self.fused = bool(rt.L.cq_mix_moe_step_fits(self.sizes))
+
+    @staticmethod
+    def row_distance(experts: int, kp: int, ff: int) -> int:
+        """Weights from one row of the gate and up weights to the next.  Rows a multiple of 4096 bytes apart lie in one channel of an L2 for all of a tile: 128 bytes between them, where
+        tiles wait for the weights (a layer of 16 experts of 4096 x 2048 with 20 pairs each 217 -> 188 us, of 64 of 2048 x 1408 246 -> 236, with 150 pairs no difference; rows of 3072 bytes:
+        none).  Not from 1 GB of weights on, where it is the other way round, for a cause not found (64 experts of 4096 x 1024, 20 / 64 / 100 pairs 322 387 440 -> 323 398 452, 256 of
+        2048 x 512 356 489 622 -> 362 497 627)."""
+        return kp + (64 if kp % 2048 == 0 and 4 * experts * ff * kp < 1 << 30 else 0)
 
     def denses(self) -> List[Dense]:
         return [self.router]

@@ -212,3 +212,8 @@ def test_heights_of_expert_tiles(experts, width, ff, heights):
     m = mixers.GatedExperts.__new__(mixers.GatedExperts)
     m.experts, m.width, m.kp, m.ff = experts, width, width, ff
     assert {p: m.tile_rows(p * experts) for p in heights} == heights
+
+
+@pytest.mark.parametrize("experts,width,ff,apart", [(8, 2048, 64, 2048 + 64), (2, 4096, 40, 4096 + 64), (64, 4096, 1023, 4096 + 64), (64, 4096, 1024, 4096), (256, 2048, 512, 2048), (4, 1536, 64, 1536), (4, 2047, 64, 2048 + 64)])
+def test_distance_of_expert_rows(experts, width, ff, apart):
+    assert mixers.GatedExperts.row_distance(experts, mixers.pad_to(width, 64), ff) == apart
