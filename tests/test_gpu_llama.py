@@ -371,3 +371,56 @@ def test_random_init_with_a_per_layer_format_override():
     tok = int(np.argmax(want))
     got = model.forward(torch.tensor([[tok]], dtype=torch.int32), 5).cpu().numpy()
     assert rel_l2(got, ref.forward([tok], 5)) <= TOL
+
+
+class Spy:
+    """The library, with what calls of the pair product returned."""
+
+    def __init__(self, lib):
+        self.lib, self.pairs = lib, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+        if name != "cq_nn_qmatmul_swiglu_pair":
+            return fn
+
+        def pair(*args):
+            self.pairs.append(fn(*args))
+            return self.pairs[-1]
+        return pair
+
+
+@pytest.mark.parametrize("gate,down,apart,rows", [(oracle.Q4K, oracle.Q6K, False, (150, 512)), (oracle.Q4K, oracle.Q8_0, True, (512,)), (oracle.Q6K, oracle.Q4K, False, (300,)),
+                                                  (oracle.Q5K, oracle.Q5K, True, (300,))])
+def test_prompt_with_gate_and_up_in_one_product(gate, down, apart, rows):
+    """A layer wide enough for silu(w1 x) * w3 x inside the product's tiles, w3 behind w1 or elsewhere: the logits and the cache have the bits of the forward that takes the
+    steps one by one (with a tap, as the op-by-op tests do)."""
+    from candle_amd.quantized import GgmlDType
+    from candle_amd.quantized_llama import Config, ModelWeights, _W
+    cfg = Config(n_layer=2, hidden=4096, n_head=32, n_kv_head=8, head_dim=128, ffn=14336, vocab=512, rope_theta=500000.0, rms_eps=1e-5, ctx=512)
+    dtypes = {n: GgmlDType(d) for n, d in dict(MIX, feed_forward_w1=gate, feed_forward_w3=gate, feed_forward_w2=down).items()}
+    model = ModelWeights.random_init(cfg, seed=9, dtypes=dtypes)
+    others = []
+    if apart:
+        for lw in model.layers:
+            w = lw.w["feed_forward_w3"]
+            at = w.ptr - model._slab.data_ptr()
+            others.append(torch.cat([model._slab.new_zeros(256), model._slab[at:at + w.nbytes]]))
+            lw.w["feed_forward_w3"] = _W(others[-1].data_ptr() + 256, w.dtype, w.n, w.k, w.nbytes)
+            model._slab[at:at + w.nbytes] = 0
+    model.L = Spy(model.L)
+    for n in rows:
+        print(f"case gate={gate} down={down} apart={apart} rows={n}", flush=True)
+        ids = torch.from_numpy(np.random.default_rng(n).integers(0, cfg.vocab, (1, n)).astype(np.int32))
+        model.L.pairs.clear()
+        got = model.forward(ids, 0)
+        assert model.L.pairs == [0, 0]
+        keys = [lw.k_cache[:, :n].clone() for lw in model.layers]
+        model.clear_kv_cache()
+        model.L.pairs.clear()
+        model.tap = lambda stage, li: None
+        want = model.forward(ids, 0)
+        model.tap = None
+        assert model.L.pairs == []
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+        assert all(torch.equal(a, lw.k_cache[:, :n]) for a, lw in zip(keys, model.layers))
