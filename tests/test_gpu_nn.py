@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import llama_oracle as lo
-from tests.util import normal, rel_l2
+from tests.util import launches, normal, rel_l2
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
@@ -693,8 +693,11 @@ def test_fused_norm_pair_outputs_far_apart():
     ok(lib.cq_nn_qmatmul_norm(14, wb.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(), 1e-5, zb.data_ptr(), k, nb, None))
     for ya, yb in ((low, high[:nb]), (high[:na], low[:nb])):
         far[:na], far[(1 << 31) + 8192:] = 77.0, 77.0
-        ok(lib.cq_nn_qmatmul_norm_pair(12, wa.data_ptr(), na, ya.data_ptr(), 14, wb.data_ptr(), nb, yb.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(), 1e-5, k, None))
+        pair = lambda st: ok(lib.cq_nn_qmatmul_norm_pair(12, wa.data_ptr(), na, ya.data_ptr(), 14, wb.data_ptr(), nb, yb.data_ptr(), xd.data_ptr(), pd.data_ptr(), wd.data_ptr(),
+                                                         1e-5, k, st))
+        pair(None)
         assert torch.equal(ya, za) and torch.equal(yb, zb)
+        assert launches(pair) == 1
 
 
 def split_planes(dtype, k):

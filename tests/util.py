@@ -24,3 +24,17 @@ def bits_equal_or_both_nan(a, b):
     same = a.view(u) == b.view(u)
     both_nan = np.isnan(a) & np.isnan(b)
     return bool(np.all(same | both_nan))
+
+
+def launches(enqueue) -> int:
+    """Nodes of the graph that enqueue(stream) is captured as, without running it: the launches it makes."""
+    import ctypes
+
+    import torch
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        enqueue(torch.cuda.current_stream().cuda_stream)
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
