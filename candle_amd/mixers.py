@@ -677,24 +677,28 @@ class GatedExperts(FeedForward):
 
     def tile_rows(self, pairs: int) -> int:
         """Rows of a tile of bfloat16 products.  Weights are read once per tile of rows, and 32-row parts of a tall tile that are not there are neither brought nor multiplied, so tall
-        tiles are the better ones soon: 128 rows from 32 pairs an expert on, 64 from 24.  Not so soon where rows are short (11 to 23 stages of 64, of which the beginning and
-        the end of a workgroup are more) or a row tile of every expert, in 128 columns, is less than 768 workgroups; where it is not one round of two to a unit, the more workgroups the better
-        until tall tiles fill that.  A layer of prompts, its router and sums included, us with 32 / 64 / 128 rows, experts evenly loaded, and by a router whose rows' lengths vary by 15 %:
-            experts x width x ff    pairs an expert
-            64 x 2048 x 1408        16  235 230 235, 241 232 236    24  247 240 242, 252 245 250    32  278 251 255, 275 255 259    40  301 261 264, 296 279 268    96  437 384 321, 433 398 363
-            8 x 4096 x 4096         24  184 186 186, 186 187 186    32  201 198 194, 237 193 192    56  264 248 205, 263 252 207    150  424 375 307, 419 377 288
-            256 x 2048 x 512        24  375 379 385, 381 393 394    32  415 395 406, 417 416 418    64  564 539 501, 568 538 524
-            64 x 1024 x 704         24  81 86 89, 85 88 91    32  91 91 95, 90 91 95    40  98 94 99, 99 102 101    56  109 111 109, 113 113 113    150  195 183 179, 198 179 175
-            16 x 2048 x 1408        24  77 79 82, 77 79 82    32  85 81 85, 81 81 86    48  96 84 89, 93 86 93    64  120 116 97, 121 120 98    150  170 170 140, 171 154 148
-            8 x 2048 x 1408         64  63 67 71, 63 64 71    96  71 69 81, 71 69 81    150  95 91 97, 93 91 97    220  111 100 99, 118 102 102
-        Seventeen shapes of experts, 8 to 220 pairs each: 0.3 % slower than the best of the three on average, 6 % at most."""
+        tiles are the better ones soon: from 20 pairs an expert on, from 36 where rows are shorter than 2048.  Later, with tiles of 64 between, where rows are short (11 and 16 stages of
+        64, of which the beginning and the end of a workgroup are more) or a row tile of every expert, in 128 columns, is less than 768 workgroups; and where it is not one round of two to
+        a unit, the more workgroups the better until tall tiles fill that.  A layer of prompts, its router and sums included, us with 32 / 64 / 128 rows, experts evenly loaded (the
+        standard deviation of their pairs an eighth of the mean), and unevenly (six tenths):
+            experts x width x ff   pairs an expert
+            64 x 2048 x 1408       16  235 230 235, 241 232 237   24  247 240 242, 252 242 249   40  301 261 264, 300 291 286   56  335 310 280, 350 316 318   96  437 384 321, 443 405 367
+            8 x 4096 x 4096        16  181 183 185, 182 184 184   24  184 186 186, 199 192 191   56  264 248 205, 265 250 208   150  424 375 307, 424 374 307
+            64 x 1536 x 1024       24  157 153 157, 158 167 159   40  182 167 169, 179 179 172   64  217 214 189, 221 208 201
+            64 x 1024 x 704        32  91 91 95, 88 95 99   48  103 105 103, 103 106 112   96  151 133 129, 151 134 145   120  167 161 158, 168 160 153
+            128 x 1024 x 704       32  162 156 162, 165 168 170   56  198 191 182, 204 196 200   80  243 234 214, 242 229 224
+            16 x 2048 x 1408       24  77 79 82, 76 80 84   40  93 83 87, 87 84 93   64  120 116 97, 120 111 103
+            8 x 2048 x 1408        64  63 67 71, 63 68 71   96  71 69 81, 71 69 81   150  95 91 97, 94 79 97   220  111 100 99, 112 101 101
+        Seventeen shapes of experts, 8 to 220 pairs each, four degrees of unevenness: 0.5 % slower than the best of the three on average."""
         per_expert, workgroups = pairs / self.experts, (2 * self.ff + self.width) / 128 * self.experts
         if workgroups < 512:
             middle, tall = 90, 200
-        elif workgroups < 768 or self.kp < 1536:
-            middle, tall = 30, 56
+        elif self.kp < 1536:
+            middle, tall = 40, 80 if workgroups >= 2048 else 104
+        elif workgroups < 768:
+            middle, tall = 30, 60
         else:
-            middle, tall = 24, 32
+            middle = tall = 20 if self.kp >= 2048 else 36
         return 128 if per_expert >= tall else 64 if per_expert >= middle else 32
 
     def prefill(self, h, ldh, x, ldx, rows, sp):
