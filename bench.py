@@ -256,7 +256,7 @@ def prefill_record(L, torch, fmt, n, k, m, steps=20, warmup=5, pmc=False):
     peak = MFMA_I8_PEAK_TOPS if i8 else MFMA_F16_PEAK_TFLOPS
     achieved = flops / (kern_us * 1e-6) / 1e12
     return {"fmt": fmt, "n": n, "k": k, "m": m, "steps": steps, "warmup": warmup, "forward_ms": round(ms, 5),
-            "forward_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1), "kernel": ("qtile_kernel<%s>" if fmt in ("q4k", "q5k", "q6k") else "qtile0_kernel<%s>" if fmt in ("q4_0", "q8_0") else "qmm_q0_i8_kernel<%s>" if i8 else "qmm_kernel<%s>") % fmt,
+            "forward_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1), "kernel": ("qtile_wide_kernel<%s>" if fmt == "q6k" else "qtile_kernel<%s>, or qtile_wide_kernel in tiles of 96 and 128 rows" if fmt in ("q4k", "q5k") else "qtile0_kernel<%s>" if fmt in ("q4_0", "q8_0") else "qmm_q0_i8_kernel<%s>" if i8 else "qmm_kernel<%s>") % fmt,
             "split_k": split_k, "quantize_us": round(q_us, 2),
             "kernel_us": round(kern_us, 2), "kernel_median_us": round(kst["median"], 2), "kernel_p10_us": round(kst["p10"], 2),
             "kernel_p90_us": round(kst["p90"], 2), "kernel_TFLOPs": round(achieved, 1), "mfma": "i8" if i8 else "f16", "peak": peak,

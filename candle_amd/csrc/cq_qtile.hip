@@ -11,18 +11,18 @@
 // shared by the workgroup, one barrier per super-block.  Two kernels: qtile_kernel interleaves the conversion of one step with the products of the step before and scales the sums of
 // all tiles at the end of a super-block (Q4_K, Q5_K, tiles of up to 64 rows); qtile_wide_kernel converts a whole super-block and then multiplies it tile by tile.
 //
-// What bounds it: at many rows the power limit.  With all units busy the clock falls to 1.65 - 1.9 GHz (the int8 cores alone, on random operands, run at 1.65: 3300 TOP/s);
-// on an eighth of the units, or on zeros, the same workgroups take 185 us where they take 260 (Q4_K, 2048 rows of [4096 x 14336]).  In those 7900 cycles per super-block and pair of
-// waves the matrix cores are busy 4350; a matrix instruction also keeps the vector unit from issuing for ten cycles, whatever its shape, so that half as many of 32 x 32 x 32 leave it
-// more room than of 16 x 16 x 64 (282 us for 262).  At few rows the weights' way from memory, and in unsplit small products the chain of one wave a SIMD.
+// What bounds it: at many rows, first the power limit's clock: 2048 rows of Q4_K [4096 x 14336], one workgroup to a unit, take 482 k cycles at 1.93 GHz (249 us), the same workgroups
+// on an eighth of the units 468 k at 2.46 (190 us).  Then what the two waves of a SIMD overlap: of a unit's 7960 busy cycles per super-block the matrix cores work 4350 (55 %; Q5_K and Q6_K 43 %)
+// and the vector units issue in 61 % (69, 68), waves wait in 30 % of theirs.  A matrix instruction also keeps the vector unit from issuing for ten cycles, whatever its shape, so that half as
+// many of 32 x 32 x 32 leave it more room than of 16 x 16 x 64 (282 us for 262).  At few rows the weights' way from memory, and in unsplit small products the chain of one wave a SIMD.
 // f16 / bf16 results are written by the product; the f32 copy and its conversion went (12 us of 154 for 512 rows of Q5_K).
 //
-// [4096 x 14336], us, with Q4_K and Q5_K of 96- and 128-row tiles and Q6_K in qtile_kernel / now, quantizing the activations included:
+// [4096 x 14336], us on one card, with Q4_K and Q5_K of 96- and 128-row tiles and Q6_K in qtile_kernel / now, quantizing the activations included:
 //              17 rows   131 rows   512 rows   2048 rows
-//   Q4_K     19.0 18.9  45.6 42.1  96.4 90.3   318 294
-//   Q5_K     22.5 22.5  50.6 48.1   105 100    375 361
-//   Q6_K     29.0 26.7  57.4 48.4   116 101    393 356
-// 2048 rows of Q4_K are 900 TOP/s of products asked for and 1800 done.
+//   Q4_K     19.6 19.5  46.5 43.5  96.7 90.3   307 283
+//   Q5_K     22.7 22.7  51.1 49.1   104 99.1   336 317
+//   Q6_K     30.7 27.9  57.8 49.2   115 99.9   374 318
+// 2048 rows of Q4_K are 930 TOP/s of products asked for and 1860 done.
 #include "cq_qtile.h"
 
 #include <algorithm>
@@ -735,9 +735,9 @@ static constexpr int64_t QT_Q6K_MIN_K = 1536;
 bool cq_qtile_takes(int w_dtype, const void *w, int64_t k, int64_t rows_of_w) {
     if (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K) return k % 256 == 0;
     if (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) return k % 256 == 0 && ((uintptr_t)w & 15) == 0;      // (rows are multiples of 16 bytes)
-    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one.  Its two half super-blocks in flight need some of k to pay (in eight
-    // waves 67 / 300 rows of [4096 x 768] took 17.6 / 18.9 us against 16.8 / 17.6 of the general kernel, of [8192 x 1024] 21.3 at 67 against 20.2).  From 1536 on it is
-    // the faster one whatever the rows (9 / 131 / 300 / 2048 rows of [4096 x 1536] 12.9 / 20.6 / 24.0 / 49.8 us against 26.9 / 25.5 / 26.3 / 77.3)
+    // Q6_K pieces are read by whole dwords: the tensor has to begin and end on one.  The limit of k is from a kernel with two half super-blocks in flight, which short rows did not pay; from
+    // 1536 on it was the faster one whatever the rows.  qtile_wide_kernel is faster below it too (k of 256 - 1280 by 1024 - 8192, 9 - 2048 rows: 0.57 - 0.85 of the general kernel's time,
+    // 131 rows of [4096 x 768] 12.2 us for 16.6); the limit has not been moved.
     return w_dtype == CQ_Q6K && k % 256 == 0 && k >= QT_Q6K_MIN_K && ((uintptr_t)w & 3) == 0 && (rows_of_w * (k / 256)) % 2 == 0;
 }
 
@@ -753,9 +753,10 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
 // is least.  A round is 256 workgroups, a the conversion of the weights, b the products and sums of 32 rows.  Workgroups of the K formats may have four waves
 // instead of eight if their rows are at most 64: each SIMD then converts and multiplies for one wave, and a small product takes up twice as many
 // compute units (131 rows of Q6_K [4096 x 4096] unsplit: 56 us in eight waves, 41 in four; 65 rows of Q4_K [4096 x 4096] 20.6 -> 17.5).
-// Costs of the K formats: fitted to the choice among 9000 forwards of 9 - 1200 rows against 90 shapes each of 1024 - 16384 by 1024 - 14336, cold weights; it
-// is 0.2 - 0.7 % slower than the best on average, at most 11 %.  Q4_0 and Q8_0 (rounds that leave compute units idle run at a higher clock
-// there, and a workgroup has 1.3 us of its own): 3800 launches of 17 - 2048 rows, 0.2 - 1.2 %.
+// Costs: fitted to earlier kernels (qtile_kernel for all tiles of K formats; the activations first in all of Q4_0 and Q8_0; rounds that leave compute units idle run at a higher clock
+// there, and a workgroup has 1.3 us of its own), which multiplied 32-row parts without rows as well: a part-filled tile still counts as a full one.  With the present kernels the choice is
+// slower than the best by 1.0 % on average for Q4_K, 0.6 for Q5_K, 1.0 for Q6_K, 1.3 for Q4_0 and 1.1 for Q8_0, by more than 5 % in 3 - 9 % of the calls, by 18 % at most (28 rows of Q6_K
+// [3667 x 3072] 16.7 us in twelve splits of eight waves, 14.1 in six of four): 1800 forwards of drawn sizes, 17 (Q4_K, Q5_K: 65) - 1600 rows, 1024 - 16384 by 1536 - 14336, cold weights, every choice timed.
 // Only splits whose sums round no more than those of the general kernels (qt_roundings).
 // Any number of columns: while those that are no multiple of four were not split, their few workgroups walked all of k (26 rows of Q4_0 [2986 x 9984] 112 us, 19 in splits; 10 rows of
 // Q8_0 [1299 x 9728] 113 -> 18, 65 of Q6_K [1970 x 13568] 126 -> 28, 239 of Q8_0 [2818 x 13056] 152 -> 58; 1494 rows of Q8_0 [3987 x 6144] 154 -> 140).
