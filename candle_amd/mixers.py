@@ -685,7 +685,7 @@ class GatedExperts(FeedForward):
             64 x 2048 x 1408       16  235 230 235, 241 232 237   24  247 240 242, 252 242 249   40  301 261 264, 300 291 286   56  335 310 280, 350 316 318   96  437 384 321, 443 405 367
             8 x 4096 x 4096        16  181 183 185, 182 184 184   24  184 186 186, 199 192 191   56  264 248 205, 265 250 208   150  424 375 307, 424 374 307
             64 x 1536 x 1024       24  157 153 157, 158 167 159   40  182 167 169, 179 179 172   64  217 214 189, 221 208 201
-            64 x 1024 x 704        32  91 91 95, 88 95 99   48  103 105 103, 103 106 112   96  151 133 129, 151 134 145   120  167 161 158, 168 160 153
+            64 x 1024 x 704        32  91 91 95, 88 95 99   48  103 105 103, 103 106 112   96  151 133 129, 151 134 145   150  195 183 179, 198 177 175   180  225 206 186, 221 203 188
             128 x 1024 x 704       32  162 156 162, 165 168 170   56  198 191 182, 204 196 200   80  243 234 214, 242 229 224
             16 x 2048 x 1408       24  77 79 82, 76 80 84   40  93 83 87, 87 84 93   64  120 116 97, 120 111 103
             8 x 2048 x 1408        64  63 67 71, 63 68 71   96  71 69 81, 71 69 81   150  95 91 97, 94 79 97   220  111 100 99, 112 101 101
@@ -694,7 +694,7 @@ class GatedExperts(FeedForward):
         if workgroups < 512:
             middle, tall = 90, 200
         elif self.kp < 1536:
-            middle, tall = 40, 80 if workgroups >= 2048 else 104
+            middle, tall = 40, 80 if workgroups >= 2048 else 160
         elif workgroups < 768:
             middle, tall = 30, 60
         else:

@@ -206,7 +206,7 @@ def test_moe_step_refuses_rows_of_weights_that_overlap():
 
 
 @pytest.mark.parametrize("experts,width,ff,heights", [(8, 2048, 1408, {20: 32, 89: 32, 90: 64, 199: 64, 200: 128}), (16, 2048, 1408, {29: 32, 30: 64, 59: 64, 60: 128}),
-                                                      (64, 1024, 704, {39: 32, 40: 64, 103: 64, 104: 128}), (128, 1024, 704, {39: 32, 40: 64, 79: 64, 80: 128}),
+                                                      (64, 1024, 704, {39: 32, 40: 64, 159: 64, 160: 128}), (128, 1024, 704, {39: 32, 40: 64, 79: 64, 80: 128}),
                                                       (64, 2048, 1408, {19: 32, 20: 128, 140: 128}), (8, 4096, 4096, {19: 32, 20: 128, 140: 128}), (64, 1536, 1024, {35: 32, 36: 128})])
 def test_heights_of_expert_tiles(experts, width, ff, heights):
     m = mixers.GatedExperts.__new__(mixers.GatedExperts)
