@@ -134,10 +134,11 @@ __device__ __forceinline__ void group_tile_at(const Src &s, int t, int tiles_m, 
 // on warm operands 1500 x 5632 x 2048 66 -> 63), one for the others: f32 activations and small tiles gain nothing from more (40 x 4096 x 4096: 13.3 -> 14.2), and
 // workgroups of up to 12 stages (a split of k, short rows) lose by it: the three past the end are brought all the same (700 x 2048 x 2048 in six splits 26.4 us
 // with one, 28.1 with three; 4 - 11 stages 4 % slower on average, 13 - 16 none, from 18 on faster).
-// Rows go by sixteens to the WGM waves that share the tile's rows, and the main loop of the large tile exists once per number of fragments that a wave then has: rows that are not there are neither brought
-// nor multiplied (an expert's last tile; 64 experts of 2048 x 1408 under 6000 pairs, tiles of 128, a Kudurax prompt of 1000: 1616 -> 1608 us, of 800: 1558 -> 1530, of 1500: 1977 -> 1963).
+// Rows go by sixteens to the WGM waves that share the tile's rows.  PARTS: the main loop exists once per number of fragments that a wave then has: rows that are not there are neither brought
+// nor multiplied (an expert's last tile: a layer of 64 experts of 2048 x 1408, tiles of 128, 120 / 150 / 220 pairs each 380 465 571 -> 377 448 534 us; a Kudurax prompt of 1500, whose
+// experts are loaded unevenly, 1 %, which is what two runs differ by).
 // XB: the activations are bfloat16; PF: stages on their way.  With a table of tiles (grouped products) the rows of a tile share the weights of one group.
-template <int BM, int BN, int WGM, int WGN, bool XB, int PF = 1>
+template <int BM, int BN, int WGM, int WGN, bool XB, int PF = 1, bool PARTS = false>
 __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n, int k_split) {
     constexpr int XV = XB ? 1 : 2;                         // 16-byte loads per eight activations
     constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, CA = BM * 8 / 256, CB = BN * 8 / 256;
@@ -263,9 +264,10 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
         }
     };
     // (the smaller tiles in one form: what two cost is more than what is left out, prompts of 20 to 100 through layers 1024 wide 1.012x - 1.028x slower)
-    const int frags = BM < 128 ? TM : (int)((min(M - m0, (int64_t)BM) + 16 * WGM - 1) / (16 * WGM));
-    if (frags >= TM) run(std::integral_constant<int, TM>{});
-    else if constexpr (BM == 128) {
+    static_assert(!PARTS || TM == 4, "a form for each number of fragments");
+    const int frags = PARTS ? (int)((min(M - m0, (int64_t)BM) + 16 * WGM - 1) / (16 * WGM)) : TM;
+    if (!PARTS || frags >= TM) run(std::integral_constant<int, TM>{});
+    else if constexpr (PARTS) {
         if (frags == 3) run(std::integral_constant<int, 3>{});
         else if (frags == 2) run(std::integral_constant<int, 2>{});
         else run(std::integral_constant<int, 1>{});
@@ -797,6 +799,12 @@ __global__ __launch_bounds__(512) void dense_matvec_kernel(const uint16_t *__res
     }
 }
 
+// Whether tiles of 128 rows have a form for each number of fragments (dense_bf16_kernel, PARTS).  Not where all of them are full, which lose 0.5 - 1 % by the longer code and eight
+// registers more (119 x 13184 x 4096 of bf16 rows 42 -> 46 us), nor where row tiles are many: the one that ends early saves little then, and no longer reads an operand when its neighbours do.
+// 2900 drawn products, last tile part-filled, forms for each against one: up to 6 row tiles, 10 of more than 12 stages, 0.967 of the time on average (two of them 0.957), more 1.000 and now and then
+// 1.05 - 1.11 (2241 x 3048 x 4736 of f32 rows 95 -> 106 us, 2329 x 676 x 6400 of bf16 rows 49 -> 53).  A few of the former lose as well (135 x 8272 x 7168 58 -> 62).
+bool part_tiles(const cq_dense_args &a, int64_t m, const Plan &p) { return a.tiles_dev || (p.tiles_m <= (p.k_split > 12 * 64 ? 10 : 6) && (m - 1) % 128 < 96); }
+
 template <int PRO>
 int matvec_launch(const uint16_t *w, int64_t ldw, const float *x, const float *vec, float eps, int dim, float *dst, const float *add, int accumulate, int n,
                   int k, hipStream_t s) {
@@ -900,9 +908,13 @@ int cq_dense_product(int precision, const cq_dense_args *args, void *workspace_d
         const int tm = (int)((m + DT_B - 1) / DT_B), tn = (int)((n + DT_B - 1) / DT_B);
         hipLaunchKernelGGL(fn, dim3((unsigned)(tm * tn)), dim3(512), 2 * DT_STAGE, s, src, o, m, (int)n, (int)k, tm, tn);
     }
-    else if (p.bm == 128 && a.x_bf16 && p.k_split > 12 * 64) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, true, 3>));
-    else if (p.bm == 128 && a.x_bf16) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, true>));
-    else if (p.bm == 128) CQ_DM((dense_bf16_kernel<128, 128, 2, 2, false>));
+    else if (p.bm == 128) {
+        const bool deep = p.k_split > 12 * 64;
+        auto *const fn = !a.x_bf16 ? (part_tiles(a, m, p) ? dense_bf16_kernel<128, 128, 2, 2, false, 1, true> : dense_bf16_kernel<128, 128, 2, 2, false, 1, false>)
+                         : deep    ? (part_tiles(a, m, p) ? dense_bf16_kernel<128, 128, 2, 2, true, 3, true> : dense_bf16_kernel<128, 128, 2, 2, true, 3, false>)
+                                   : (part_tiles(a, m, p) ? dense_bf16_kernel<128, 128, 2, 2, true, 1, true> : dense_bf16_kernel<128, 128, 2, 2, true, 1, false>);
+        CQ_DM(fn);
+    }
     else if (p.bm == 64 && a.x_bf16) CQ_DM((dense_bf16_kernel<64, 64, 2, 2, true>));
     else if (p.bm == 64) CQ_DM((dense_bf16_kernel<64, 64, 2, 2, false>));
     else if (a.x_bf16) CQ_DM((dense_bf16_kernel<32, 64, 1, 4, true>));

@@ -158,3 +158,33 @@ def test_row_factors_of_sums(m, n, k, x_bf16):
     _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
     size = product.norm(dim=1) + want.norm(dim=1)
     assert float(((y.double() - want).norm(dim=1) / size).max()) <= BOUND
+
+
+@pytest.mark.parametrize("x_bf16", [0, 1])
+@pytest.mark.parametrize("tiles,n,k", [(2, 1028, 8192), (3, 1028, 5120), (3, 4100, 5120), (6, 516, 5120), (7, 516, 5120)])
+def test_last_row_tile_of_any_height(tiles, n, k, x_bf16):
+    """128-row tiles, the last one with rows of one to four fragments: in the forms for each and in one form (7 row tiles), with one stage on its way and with three: the bits of the same
+    rows with all tiles full, which come as near to float64 as the products of this file do; nothing behind the last row is written."""
+    print(f"case {tiles} {n} {k} {x_bf16}", flush=True)
+    L, full = _lib.mixer_lib(), 128 * tiles
+    g = torch.Generator(device="cuda").manual_seed(tiles + n + k)
+    w = torch.randn((n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((full, k), generator=g, device="cuda").bfloat16()
+    xd = x if x_bf16 else x.float()
+    nb = L.cq_dense_matmul_workspace_bytes(0, full, n, k)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+
+    def product(m):
+        y = torch.full((m + 1, n), 5.0, device="cuda")
+        a = DenseArgs(w_dev=w.data_ptr(), ldw=k, x_dev=xd.data_ptr(), ldx=k, x_bf16=x_bf16, dst_dev=y.data_ptr(), ldd=n, m=m, n=n, k=k, batch=1)
+        assert L.cq_dense_matmul_workspace_bytes(0, m, n, k) == nb // full * m
+        _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert bool((y[m] == 5).all())
+        return y[:m]
+
+    all_rows = product(full)
+    want = x.double() @ w.double().t()
+    assert float(((all_rows - want).norm(dim=1) / want.norm(dim=1)).max()) <= BOUND
+    for last in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127):
+        m = full - 128 + last
+        assert torch.equal(product(m), all_rows[:m]), last
