@@ -353,14 +353,15 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
 }  // namespace
 
 // Which operand comes first in tiles of 32 rows (larger ones: the weights, see above).  us, activations / weights first:
-//  - Q4_0, activations: their form leaves room for two workgroups to a unit, the other for one (20 rows of [13824 x 5120] 28.0 / 31.4, of [4096 x 14336] 24.1 / 24.2).
-//    Experts whose workgroups are two full rounds are the exception, 800 pairs on 48 experts of 3072 x 1024 58.1 / 55.4 (588 to be expected), 600 on 32 of 4096 x 2048
-//    84.6 / 68.7 (544), 600 on 16 of 4096 x 4096 135 / 115 (416); but 520 there 103 / 113 (384), 600 on 64 of 1280 x 1024 37.7 / 39.6 (320), 2000 on 128 of
-//    2048 x 768 60.8 / 65.9 (1024), 2400 on 256 of 2048 x 512 74.8 / 89.6 (2048).
+//  - Q4_0, activations: their form leaves room for two workgroups to a unit, the other for one (20 rows of [13824 x 5120] 28.0 / 31.4, of [4096 x 14336] 24.1 / 24.2).  Experts, whose
+//    grid has workgroups without rows between those with, by the number that is expected to have rows (3900 drawn calls; the time with the weights first by the other, mean): up to 256
+//    0.79, since two come to lie on one unit while others have none (606 pairs on 16 experts of 1536 x 1024 36.9 / 26.5); 257 - 500 1.06; 501 - 640, about two full rounds, 1.00, with more
+//    to win than to lose where they are full (600 on 32 of 4096 x 2048 84.6 / 68.7, on 48 of 3072 x 1024 56.9 / 53.8); more 1.10 (2000 on 128 of 2048 x 768 60.8 / 65.9, 2400 on 256 of
+//    2048 x 512 74.8 / 89.6).
 //  - Q8_0, weights, whose results are stored four columns at a time (20 rows of [2048 x 2048] 11.4 / 11.3; 900 pairs on 64 experts of 1024 x 1024 30.8 / 29.1), as long as
 //    they come out of a cache: the scales of a super-block's first half are put into LDS at the end of the one before, and what comes from memory is not there yet
 //    (20 rows of [4096 x 14336] 28.1 / 28.6, of [13824 x 5120] 35.3 / 35.7; cold weights of 17 MB and less 0.3 - 1 % the other way).
-static constexpr int64_t Q0_ROUND_AND_HALF = 400, Q0_TWO_ROUNDS = 600, Q0_CACHED = 24 << 20;
+static constexpr int64_t Q0_ONE_ROUND = 256, Q0_TWO_ROUNDS[2] = {500, 640}, Q0_CACHED = 24 << 20;
 template <int DT>
 static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                      const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
@@ -368,7 +369,7 @@ static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &
     if (moe) {
         if (mi != 1) Q0_GO(4, true, true);
         if constexpr (DT == CQ_Q4_0)
-            if (rows * grid.y <= Q0_ROUND_AND_HALF || rows * grid.y > Q0_TWO_ROUNDS) Q0_GO(1, true, false);
+            if (const int64_t t = rows * grid.y; t > Q0_ONE_ROUND && (t <= Q0_TWO_ROUNDS[0] || t > Q0_TWO_ROUNDS[1])) Q0_GO(1, true, false);
         Q0_GO(1, true, true);
     }
     if (mi == 1) {
