@@ -358,10 +358,11 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
 //    0.79, since two come to lie on one unit while others have none (606 pairs on 16 experts of 1536 x 1024 36.9 / 26.5); 257 - 500 1.06; 501 - 640, about two full rounds, 1.00, with more
 //    to win than to lose where they are full (600 on 32 of 4096 x 2048 84.6 / 68.7, on 48 of 3072 x 1024 56.9 / 53.8); more 1.10 (2000 on 128 of 2048 x 768 60.8 / 65.9, 2400 on 256 of
 //    2048 x 512 74.8 / 89.6).
-//  - Q8_0, weights, whose results are stored four columns at a time (20 rows of [2048 x 2048] 11.4 / 11.3; 900 pairs on 64 experts of 1024 x 1024 30.8 / 29.1), as long as
-//    they come out of a cache: the scales of a super-block's first half are put into LDS at the end of the one before, and what comes from memory is not there yet
-//    (20 rows of [4096 x 14336] 28.1 / 28.6, of [13824 x 5120] 35.3 / 35.7; cold weights of 17 MB and less 0.3 - 1 % the other way).
-static constexpr int64_t Q0_ONE_ROUND = 256, Q0_TWO_ROUNDS[2] = {500, 640}, Q0_CACHED = 24 << 20;
+//  - Q8_0, weights, whose results are stored four columns at a time (900 pairs on 64 experts of 1024 x 1024 30.8 / 29.1), but for weights so large that a model's next call finds them in
+//    memory: the scales of a super-block's first half are put into LDS at the end of the one before, when what comes from memory is not there yet.  3500 drawn calls of 9 - 32 rows, the time
+//    with the weights first by the other, weights out of a cache and out of memory: up to 8 MB 0.993 and 0.996, 16 - 24 MB 0.987 and 1.007, 48 MB and more 0.993 and 1.015 (24 rows of
+//    [4096 x 14336] from memory 27.9 / 28.4).
+static constexpr int64_t Q0_ONE_ROUND = 256, Q0_TWO_ROUNDS[2] = {500, 640}, Q0_CACHED = 44 << 20;
 template <int DT>
 static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                      const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {

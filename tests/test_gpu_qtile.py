@@ -291,7 +291,7 @@ def test_matmul_of_quantized_rows(fmt, rows, n, k):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
-@pytest.mark.parametrize("n,k", [(8197, 256), (8197, 2304), (16385, 1792)])
+@pytest.mark.parametrize("n,k", [(8197, 256), (8197, 2304), (16385, 3072)])
 def test_few_rows_keep_the_bits_of_many(fmt, n, k):
     """Unsplit, a result is one chain of blocks: rows in a tile of 32 (whichever operand comes first there, which the size of the weights decides for Q8_0) have the bits they
     have among 2000, in tiles of 128."""
