@@ -44,17 +44,26 @@ __device__ __forceinline__ void put(const Out &o, int64_t at, float v) {
     else reinterpret_cast<float *>(o.dst)[at] = v;
 }
 
-// four consecutive columns n .. n+3 of row m (n % 4 == 0); present: what is already there, from a caller that has it
-__device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, int64_t M, int N, int split, const f32x4 *present = nullptr) {
+// Where row m of a product goes and its factor.
+struct Row {
+    int64_t m, at;
+    float scale;
+    bool there;
+};
+__device__ __forceinline__ Row row_of(const Out &o, int64_t m, int64_t M) {
+    const int64_t mm = min(m, M - 1);
+    return Row{m, o.rows ? o.rows[mm] : mm, o.row_scale ? o.row_scale[mm] : 1.0f, m < M};
+}
+
+// four consecutive columns n .. n+3 of a row (n % 4 == 0)
+__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split) {
     if (o.planes) {
-        *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + m) * o.n4 + n) = v;
+        *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + row.m) * o.n4 + n) = v;
         return;
     }
-    const int64_t r = o.rows ? o.rows[m] : m;
     if (o.act == CQ_DENSE_ACT_SWIGLU) {                    // columns are gate, up, gate, up
-        const float sc = o.row_scale ? o.row_scale[m] : 1.0f;
-        const float a = sc * dense_silu(v.x) * v.y, b = sc * dense_silu(v.z) * v.w;
-        const int64_t at = r * o.ldd + (n >> 1);
+        const float a = row.scale * dense_silu(v.x) * v.y, b = row.scale * dense_silu(v.z) * v.w;
+        const int64_t at = row.at * o.ldd + (n >> 1);
         put(o, at, a);
         if (n + 3 < N) put(o, at + 1, b);
         return;
@@ -63,9 +72,9 @@ __device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, i
 #pragma unroll
         for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.0f) * fmaxf(v[i], 0.0f);
     }
-    if (o.row_scale) v *= o.row_scale[m];
+    if (o.row_scale) v *= row.scale;
     if (o.bf16) {
-        __bf16 *d = reinterpret_cast<__bf16 *>(o.dst) + r * o.ldd + n;
+        __bf16 *d = reinterpret_cast<__bf16 *>(o.dst) + row.at * o.ldd + n;
         if (n + 4 <= N && (reinterpret_cast<uintptr_t>(d) & 7) == 0) {
             bf16x4 b;
 #pragma unroll
@@ -78,29 +87,139 @@ __device__ __forceinline__ void emit4(const Out &o, f32x4 v, int64_t m, int n, i
             if (n + i < N) d[i] = (__bf16)v[i];
         return;
     }
-    float *d = reinterpret_cast<float *>(o.dst) + r * o.ldd + n;
-    const float *a = o.add ? o.add + r * o.ld_add + n : nullptr;
+    float *d = reinterpret_cast<float *>(o.dst) + row.at * o.ldd + n;
+    const float *a = o.add ? o.add + row.at * o.ld_add + n : nullptr;
     if (n + 4 <= N && ((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(a)) & 15) == 0) {
-        if (o.accumulate) v += present ? *present : *reinterpret_cast<const f32x4 *>(d);
+        if (o.accumulate) v += *reinterpret_cast<const f32x4 *>(d);
         if (a) v += *reinterpret_cast<const f32x4 *>(a);
         *reinterpret_cast<f32x4 *>(d) = v;
         return;
     }
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        if (n + i < N) d[i] = v[i] + (o.accumulate ? (present ? (*present)[i] : d[i]) : 0.0f) + (a ? a[i] : 0.0f);
+        if (n + i < N) d[i] = v[i] + (o.accumulate ? d[i] : 0.0f) + (a ? a[i] : 0.0f);
 }
 
-// What is already at those four columns (zero where there are none).
-__device__ __forceinline__ f32x4 present4(const Out &o, int64_t m, int n, int64_t M, int N) {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (m >= M) return v;
-    const float *d = reinterpret_cast<const float *>(o.dst) + (o.rows ? o.rows[m] : m) * o.ldd + n;
-    if (n + 4 <= N && (reinterpret_cast<uintptr_t>(d) & 15) == 0) return *reinterpret_cast<const f32x4 *>(d);
+__device__ __forceinline__ uint32_t pair_bf16(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)a, (__bf16)b});
+}
+// a, b: of the four groups of sixteen lanes, a0 a1 a2 a3 and b0 b1 b2 b3 -> a0 a1 b0 b1 and a2 a3 b2 b3 (halves), a0 b0 a2 b2 and a1 b1 a3 b3 (rows)
+__device__ __forceinline__ void swap_halves(uint32_t &a, uint32_t &b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+#endif
+}
+__device__ __forceinline__ void swap_rows(uint32_t &a, uint32_t &b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+#endif
+}
+
+// Whether results of columns n .. n + wide - 1 lie on 16 bytes, in f32 without an activation: whole rows of them in one go.
+__device__ __forceinline__ bool plain_f32(const Out &o, int n, int wide, int N) {
+    return !o.planes && !o.bf16 && o.act == CQ_DENSE_ACT_NONE && n + wide <= N && ((o.ldd | (o.add ? o.ld_add : 0)) & 3) == 0 &&
+           ((reinterpret_cast<uintptr_t>(o.dst) | reinterpret_cast<uintptr_t>(o.add)) & 15) == 0;
+}
+// One row of them: NF times four columns, number f from column(f) on, added to what is there and to the addend.
+template <int NF, class At>
+__device__ __forceinline__ void sum_f32(const Out &o, const Row &row, f32x4 (&old)[NF], f32x4 (&more)[NF], At column) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (n + i < N) v[i] = d[i];
-    return v;
+    for (int f = 0; f < NF; f++) {
+        if (o.accumulate) old[f] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(o.dst) + row.at * o.ldd + column(f));
+        if (o.add) more[f] = *reinterpret_cast<const f32x4 *>(o.add + row.at * o.ld_add + column(f));
+    }
+}
+template <int NF, class At, class Of>
+__device__ __forceinline__ void store_f32(const Out &o, const Row &row, Of sums, const f32x4 (&old)[NF], const f32x4 (&more)[NF], At column) {
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        f32x4 v = sums(f);
+        if (o.row_scale) v *= row.scale;
+        if (o.accumulate) v += old[f];
+        if (o.add) v += more[f];
+        *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(o.dst) + row.at * o.ldd + column(f)) = v;
+    }
+}
+
+// The sums of a wave: of row m(i) of lane % 16 columns nw + 16 j + 4 (lane / 16) .. + 3.  Whatever memory holds beside them (where a row goes, its factor, what the sums are added to) is
+// asked for in front of the stores: a load behind a store waits for it, since both are counted in one order, and per four columns that was sixteen round trips a workgroup.
+// bfloat16 results change lanes first, so that four lanes write 64 bytes in a row; as two and eight bytes a lane they were as many instructions again.
+// Products of 1500 rows on 64 experts of 2048 x 1408, six a row (unevenly loaded), 240 -> 211 us (gate and up) and 138 -> 125 (down); 1500 x 5632 x 2048 with silu 65 -> 58; a prompt
+// of 1500 of such a model 1965 -> 1826.
+template <int TM, int TN, class At>
+__device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN], At m, int nw, int lk, int64_t M, int N, int split) {
+    Row row[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) row[i] = row_of(o, m(i), M);
+    auto column = [&](int j) { return nw + 16 * j + 4 * lk; };
+    if (plain_f32(o, nw, 16 * TN, N)) {
+        f32x4 old[2][TN], more[2][TN];                     // the next row's in front of this one's stores
+        if (row[0].there) sum_f32(o, row[0], old[0], more[0], column);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (i + 1 < TM && row[i + 1].there) sum_f32(o, row[i + 1], old[(i + 1) & 1], more[(i + 1) & 1], column);
+            if (row[i].there) store_f32(o, row[i], [&](int j) { return acc[i][j]; }, old[i & 1], more[i & 1], column);
+        }
+        return;
+    }
+    if constexpr (TN == 4) {
+        if (o.bf16 && !o.planes && nw + 64 <= N && o.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(o.dst) & 15) == 0) {
+            uint16_t *const dst = reinterpret_cast<uint16_t *>(o.dst);
+            if (o.act == CQ_DENSE_ACT_SWIGLU) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    uint32_t p[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const f32x4 v = acc[i][j];
+                        p[j] = pair_bf16(row[i].scale * dense_silu(v.x) * v.y, row[i].scale * dense_silu(v.z) * v.w);
+                    }
+                    swap_halves(p[0], p[2]);
+                    swap_halves(p[1], p[3]);
+                    swap_rows(p[0], p[1]);
+                    swap_rows(p[2], p[3]);
+                    if (row[i].there) *reinterpret_cast<u32x4 *>(dst + row[i].at * o.ldd + (nw >> 1) + 8 * lk) = u32x4{p[0], p[1], p[2], p[3]};
+                }
+                return;
+            }
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j += 2) {
+                    uint32_t p[2][2];
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        f32x4 v = acc[i][j + u];
+                        if (o.act == CQ_DENSE_ACT_RELU2) {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) v[e] = fmaxf(v[e], 0.0f) * fmaxf(v[e], 0.0f);
+                        }
+                        if (o.row_scale) v *= row[i].scale;
+                        p[u][0] = pair_bf16(v.x, v.y);
+                        p[u][1] = pair_bf16(v.z, v.w);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        swap_halves(p[0][e], p[1][e]);
+                        swap_rows(p[0][e], p[1][e]);
+                    }
+                    if (row[i].there) *reinterpret_cast<u32x4 *>(dst + row[i].at * o.ldd + nw + 16 * j + 8 * lk) = u32x4{p[0][0], p[0][1], p[1][0], p[1][1]};
+                }
+            return;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        if (!row[i].there) continue;
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            if (column(j) < N) emit4(o, acc[i][j], row[i], column(j), M, N, split);
+    }
 }
 
 // Tile t of the order that a run follows: GROUP row tiles wide, column by column, so that the workgroups running side by side on an XCD need
@@ -253,14 +372,17 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
             else __syncthreads();
             cur ^= 1;
         };
-        for (int k = k_lo; k < k_hi; k += 64 * PF) {
-            step(k, first, second);
-            if (PF == 3) {
-                if (k + 64 >= k_hi) break;
+        int k = k_lo;
+        if constexpr (PF == 3) {                               // (not left in the middle: the compiler would keep its sets in memory)
+            for (; k + 128 < k_hi; k += 192) {
+                step(k, first, second);
                 step(k + 64, second, third);
-                if (k + 128 >= k_hi) break;
                 step(k + 128, third, first);
             }
+            if (k < k_hi) step(k, first, second);
+            if (k + 64 < k_hi) step(k + 64, second, third);
+        } else {
+            for (; k < k_hi; k += 64) step(k, first, second);
         }
     };
     // (the smaller tiles in one form: what two cost is more than what is left out, prompts of 20 to 100 through layers 1024 wide 1.012x - 1.028x slower)
@@ -272,16 +394,7 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
         else if (frags == 2) run(std::integral_constant<int, 2>{});
         else run(std::integral_constant<int, 1>{});
     }
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-        const int64_t m = m0 + wm + 16 * WGM * i + lr;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn + 16 * j + 4 * lk;
-            if (n < N) emit4(out, acc[i][j], m, n, M, N, blockIdx.y);
-        }
-    }
+    put_sums(out, acc, [&](int i) { return m0 + wm + 16 * WGM * i + lr; }, n0 + wn, lk, M, N, blockIdx.y);
 }
 
 // ---- bf16 tiles of 256 activation rows x 256 weight rows, for products that fill the chip with them ------------------------------
@@ -398,16 +511,18 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
         multiply(3);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (copies may not outlive the workgroup)
+    Row row[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) row[i] = row_of(out, m0 + wm + 32 * i + lr, M);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int64_t m = m0 + wm + 32 * i + lr;
-        if (m >= M) continue;
+        if (!row[i].there) continue;
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int n = n0 + wn + 32 * j + 8 * v + 4 * kg;
-                if (n < N) emit4(out, f32x4{acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]}, m, n, M, N, 0);
+                if (n < N) emit4(out, f32x4{acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]}, row[i], n, M, N, 0);
             }
     }
 #endif
@@ -519,24 +634,7 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++) acc[i][j] = sum[i][j] + acc[i][j];
-    // what the sums are added to is asked for here, all at once (as each is stored, a load would have to wait for the store before it, and the
-    // product would take half as long again)
-    f32x4 old[TM][TN];
-    if (out.accumulate)
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) old[i][j] = present4(out, m0 + wm + 16 * i + lr, n0 + wn + 16 * j + 4 * lk, M, N);
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-        const int64_t m = m0 + wm + 16 * i + lr;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn + 16 * j + 4 * lk;
-            if (n < N) emit4(out, acc[i][j], m, n, M, N, 0, &old[i][j]);
-        }
-    }
+    put_sums(out, acc, [&](int i) { return m0 + wm + 16 * i + lr; }, n0 + wn, lk, M, N, 0);
 #endif
 }
 
@@ -624,16 +722,7 @@ __global__ __launch_bounds__(256) void dense_f32_kernel(Src src, Out out, int64_
             cur ^= 1;
         }
     }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int64_t m = m0 + wm + 16 * i + lr;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int n = n0 + wn + 16 * j + 4 * lk;
-            if (n < N) emit4(out, acc[i][j], m, n, M, N, blockIdx.y);
-        }
-    }
+    put_sums(out, acc, [&](int i) { return m0 + wm + 16 * i + lr; }, n0 + wn, lk, M, N, blockIdx.y);
 }
 
 // the planes of a k split, added in order
@@ -647,7 +736,7 @@ __global__ __launch_bounds__(256) void dense_planes_kernel(Out out, int64_t M, i
     for (int s = 1; s < splits; s++) v += *reinterpret_cast<const f32x4 *>(out.planes + ((int64_t)s * M + m) * out.n4 + n);
     Out o = out;
     o.planes = nullptr;
-    emit4(o, v, m, n, M, N, 0);
+    emit4(o, v, row_of(o, m, M), n, M, N, 0);
 }
 
 struct Plan {

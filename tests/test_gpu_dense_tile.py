@@ -188,3 +188,52 @@ def test_last_row_tile_of_any_height(tiles, n, k, x_bf16):
     for last in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127):
         m = full - 128 + last
         assert torch.equal(product(m), all_rows[:m]), last
+
+
+@pytest.mark.parametrize("m,n,k,tile_rows", [(1100, 2506, 1024, 0), (1500, 5634, 1088, 0), (2000, 3202, 832, 0), (2000, 3266, 512, 0), (2300, 4612, 1088, 0), (300, 2506, 1024, 128), (130, 190, 512, 128),
+                                             (130, 190, 512, 64), (70, 190, 512, 32)])
+@pytest.mark.parametrize("form", ["bf16", "relu2", "swiglu", "sum"])
+def test_results_on_and_off_16_bytes(m, n, k, tile_rows, form):
+    """Results that lie on 16 bytes go out by whole rows, four lanes 64 bytes (bfloat16) or row by row with what they are added to asked for ahead (f32); elsewhere, and in the last
+    columns, four at a time: the same bits.  Ring of 128 and of 192 rows, the 128 x 128 tile with three stages and with one, the large tile, tiles of a table with scattered rows and factors."""
+    print(f"case {m} {n} {k} {tile_rows} {form}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    groups = 3 if tile_rows else 1
+    w = torch.randn((groups, n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k), generator=g, device="cuda").bfloat16()
+    scale, perm, cols = torch.rand(m, generator=g, device="cuda") + 0.5, torch.randperm(m, generator=g, device="cuda").int(), n // 2 if form == "swiglu" else n
+    starts = [t for e in range(groups) for t in range(e * m // groups, (e + 1) * m // groups, tile_rows)] if tile_rows else []
+    of = [next(e for e in range(groups) if t < (e + 1) * m // groups) for t in starts]
+    tiles = torch.tensor([[e, t, min(tile_rows, (e + 1) * m // groups - t), 0] for e, t in zip(of, starts)], dtype=torch.int32, device="cuda")
+    n_tiles = torch.tensor([len(starts)], dtype=torch.int32, device="cuda")
+    L, got = _lib.mixer_lib(), []
+    nb = L.cq_dense_matmul_workspace_bytes(0, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    for ld, first in (((cols + 7) // 8 * 8 + 8, 0), ((cols + 7) // 8 * 8 + 3, 1)):
+        y = torch.full((m + 2, ld), 3.0, device="cuda", dtype=torch.float32 if form == "sum" else torch.bfloat16)
+        add = torch.randn((m, n), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+        add = torch.nn.functional.pad(add, (0, ld - n))
+        a = DenseArgs(w_dev=w.data_ptr(), ldw=k, w_batch=n * k, x_dev=x.data_ptr(), ldx=k, x_bf16=1, dst_dev=y[1].data_ptr() + first * y.element_size(), ldd=ld, m=m, n=n, k=k, batch=1,
+                      dst_bf16=int(form != "sum"), act={"relu2": 1, "swiglu": 2}.get(form, 0), row_scale_dev=scale.data_ptr(), dst_rows_dev=perm.data_ptr())
+        if tile_rows:
+            a.tiles_dev, a.n_tiles_dev, a.max_tiles, a.tile_rows = tiles.data_ptr(), n_tiles.data_ptr(), len(starts) + 2, tile_rows
+        elif form == "sum":
+            a.accumulate, a.add_dev, a.ld_add = 1, add.data_ptr(), ld
+        _lib.check("cq_dense_product", L.cq_dense_product(0, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        flat = y.flatten()[ld + first:]
+        got.append(flat[:m * ld].view(m, ld)[:, :cols].clone())
+        flat[:m * ld].view(m, ld)[:, :cols] = 3.0
+        assert bool((y == 3).all())
+    assert torch.equal(*got)
+    rows = torch.cat([x[t:t + c].double() @ w[e].double().t() for e, t, c, _ in tiles.tolist()]) if tile_rows else x.double() @ w[0].double().t()
+    size = rows.norm(dim=1, keepdim=True)
+    if form == "swiglu":
+        rows = torch.nn.functional.silu(rows[:, 0::2]) * rows[:, 1::2]
+    if form == "relu2":
+        rows, size = rows.clamp(min=0).square(), size * rows.abs().amax()      # (a square's slope: twice the value)
+    rows = rows * scale[:, None]
+    if form == "sum" and not tile_rows:
+        rows = rows + 3.0 + add[perm.long(), :n]
+    err = (got[0].double()[perm.long()] - rows).abs()
+    err = (err - rows.abs() * (2.0 ** -22 if form == "sum" else 2.0 ** -8)).clamp(min=0)
+    assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * 4
