@@ -158,6 +158,11 @@ struct MoeChunks {
     const float *pair_scale;
     int max_chunks;
 };
+// Tiles of tile_rows pairs that a list of `pairs` can have: whole ones, and one that is not for every expert.  A multiple of eight (qt_moe_tile).
+inline unsigned cq_moe_grid(const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t tile_rows) {
+    const int64_t most = pairs / tile_rows + (num_experts < pairs ? num_experts : pairs), t = most < mc.max_chunks ? most : mc.max_chunks;
+    return (unsigned)((t + 7) / 8 * 8);
+}
 int cq_moe_chunks_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t k,
                          int64_t n, hipStream_t s);
 

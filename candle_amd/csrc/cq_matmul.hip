@@ -741,9 +741,9 @@ int cq_convert_f32_launch(const float *src, void *dst, int dst_dtype, int64_t co
 
 namespace {
 template <int DT>
-int launch_qmm_moe(const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t k, int64_t n, int tile_rows, hipStream_t s) {
+int launch_qmm_moe(const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows, hipStream_t s) {
     const int bn = tile_rows == 32 ? 128 : 64;
-    dim3 grid((unsigned)mc.max_chunks, (unsigned)((n + bn - 1) / bn));
+    dim3 grid(cq_moe_grid(mc, num_experts, pairs, tile_rows), (unsigned)((n + bn - 1) / bn));
     if (grid.y > 65535) return CQ_ERR_RANGE;
     const int64_t expert_bytes = n * (k / BlockInfo<DT>::elems) * BlockInfo<DT>::bytes;
     if (tile_rows == 32)
@@ -770,11 +770,11 @@ int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_
     const bool narrow = w_dtype == CQ_Q4_0 && tile_rows == CQ_MOE_TILE_SMALL && n <= 1024;
     if (!narrow && cq_qtile_takes(w_dtype, w, k, num_experts * n)) return cq_qtile_moe_launch(w_dtype, w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
     switch (w_dtype) {
-        case CQ_Q4_0: return launch_qmm_moe<CQ_Q4_0>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q8_0: return launch_qmm_moe<CQ_Q8_0>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q6K: return launch_qmm_moe<CQ_Q6K>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q2K: return launch_qmm_moe<CQ_Q2K>(w, av, out, mc, k, n, tile_rows, s);
-        case CQ_Q3K: return launch_qmm_moe<CQ_Q3K>(w, av, out, mc, k, n, tile_rows, s);
+        case CQ_Q4_0: return launch_qmm_moe<CQ_Q4_0>(w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
+        case CQ_Q8_0: return launch_qmm_moe<CQ_Q8_0>(w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
+        case CQ_Q6K: return launch_qmm_moe<CQ_Q6K>(w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
+        case CQ_Q2K: return launch_qmm_moe<CQ_Q2K>(w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
+        case CQ_Q3K: return launch_qmm_moe<CQ_Q3K>(w, av, out, mc, num_experts, rows_alloc, k, n, tile_rows, s);
     }
     return CQ_ERR_DTYPE;
 }

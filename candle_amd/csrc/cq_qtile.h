@@ -25,11 +25,36 @@ __device__ __forceinline__ void qt_pin(f32x16 &v) {
 #endif
 }
 
+// Grouped products: which tile of the table, and which columns, a workgroup takes.  The grid (a multiple of eight wide) has room for more tiles than there are; taken along x first, the
+// workgroups without a tile would lie between those of one block of columns and of the next, and each of them waits for a whole unit's LDS.  Here they come last, and all column blocks of a
+// tile run on one XCD, so that its rows come to one L2.
+__device__ __forceinline__ void qt_moe_tile(int &tile, int &block) {
+    const uint32_t id = blockIdx.x + gridDim.x * blockIdx.y, at = id >> 3;
+    tile = 8 * (at / gridDim.y) + (id & 7);
+    block = at % gridDim.y;
+}
+// ... and where the rows of its tile go, with their factors, brought to LDS in front of everything else: read from memory where they are used they would be
+// waited for behind the stores, four rows at a time.
+template <int BM> struct QtPairs {
+    static constexpr int PARTS = (BM + 63) / 64, SCALES = 256 * PARTS, BYTES = 2 * SCALES;
+    static __device__ __forceinline__ void request(const MoeChunks &mc, int m0, int rows, uint8_t *to, int wv, int lane) {
+#ifdef __HIP_DEVICE_COMPILE__
+        if (wv >= 2 * PARTS) return;
+        const int part = wv % PARTS;
+        const bool scales = wv >= PARTS;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(scales ? (void *)(mc.pair_scale + m0) : (void *)(mc.pair_out + m0), 0, -1, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (cq_lds_void *)(to + 256 * wv), 4, 4 * min(64 * part + lane, rows - 1 - m0), 0, 0, 0);
+        asm volatile("" ::: "memory");
+#endif
+    }
+};
+
 // Results of a wave: column nn of rows m0 .., in the layout of the 32 x 32 matrix instructions (row 8 (e / 4) + 4 kg + e % 4 of each tile).
-// MOE: rows of the expert-sorted list, scattered to their pairs' rows and scaled.  Splits of K after the first write f32 planes [rows, qt_plane_ld(n)].
+// MOE: rows of the expert-sorted list, scattered to their pairs' rows and scaled; `to` and `by`: these rows' places and factors, in LDS.
+// Splits of K after the first write f32 planes [rows, qt_plane_ld(n)].
 template <int MI, bool MOE>
 __device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int dst_dtype, int m0, int rows, int nn, int n, int kg, int64_t stride_dst, float *planes,
-                                         const MoeChunks &mc) {
+                                         const uint8_t *to = nullptr, const uint8_t *by = nullptr) {
     auto store = [&](auto put) {
 #pragma unroll
         for (int t = 0; t < MI; t++)
@@ -41,7 +66,18 @@ __device__ __forceinline__ void qt_store(const f32x16 (&acc)[MI], void *dst, int
             }
     };
     if constexpr (MOE) {
-        store([&](int mm, float v) { ((float *)dst)[(int64_t)mc.pair_out[mm] * stride_dst + nn] = v * mc.pair_scale[mm]; });
+#pragma unroll
+        for (int t = 0; t < MI; t++)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) {
+                const int r = t * 32 + 8 * e4 + 4 * kg;
+                const i32x4 row = *reinterpret_cast<const i32x4 *>(to + 4 * r);
+                const f32x4 f = *reinterpret_cast<const f32x4 *>(by + 4 * r);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (m0 + r + i < rows && nn < n) ((float *)dst)[(int64_t)row[i] * stride_dst + nn] = acc[t][4 * e4 + i] * f[i];
+                __builtin_amdgcn_sched_barrier(0);
+            }
     } else {
         if (dst_dtype == CQ_F32 || blockIdx.z > 0) {
             float *const out = (blockIdx.z > 0 ? planes + (int64_t)(blockIdx.z - 1) * rows * qt_plane_ld(n) : (float *)dst) + nn;

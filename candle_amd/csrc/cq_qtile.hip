@@ -90,14 +90,17 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nr = lane & 31, kg = lane >> 5;
-    int m0 = blockIdx.x * BM;
-    const int n0 = blockIdx.y * BN + 32 * wv;
+    int m0 = blockIdx.x * BM, block = blockIdx.y;
     if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+        int tile;
+        qt_moe_tile(tile, block);
+        if (tile >= mc.n_chunks[0]) return;
+        m0 = mc.first[tile];
+        rows = m0 + mc.count[tile];
+        w += (int64_t)mc.expert[tile] * expert_bytes;
+        QtPairs<BM>::request(mc, m0, rows, lds + LD::BYTES, wv, lane);
     }
+    const int n0 = block * BN + 32 * wv;
     const int nsb_all = k >> 8;
     const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
     const int64_t row_bytes = (int64_t)nsb_all * BB;
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_kernel(const uint8_t *__rest
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     const int lane_out = qt_lane();
-    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
+    qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, lds + LD::BYTES, lds + LD::BYTES + QtPairs<BM>::SCALES);
 #endif
 }
 
@@ -360,15 +363,18 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nr = lane & 31, kg = lane >> 5;
-    int m0 = blockIdx.x * BM;
-    const int n0 = blockIdx.y * BN + 32 * (PAIR ? wv & 3 : wv);
+    int m0 = blockIdx.x * BM, block = blockIdx.y;
     if (PAIR && wv >= 4) w += expert_bytes;
     if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+        int tile;
+        qt_moe_tile(tile, block);
+        if (tile >= mc.n_chunks[0]) return;
+        m0 = mc.first[tile];
+        rows = m0 + mc.count[tile];
+        w += (int64_t)mc.expert[tile] * expert_bytes;
+        QtPairs<BM>::request(mc, m0, rows, lds + LD::BYTES, wv, lane);
     }
+    const int n0 = block * BN + 32 * (PAIR ? wv & 3 : wv);
     const int nsb_all = k >> 8;
     const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
     const int64_t row_bytes = (int64_t)nsb_all * BB;
@@ -639,9 +645,9 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
                 const float o = other[64 * (16 * u + e)], g = late ? o : half[u][e];
                 half[u][e] = g / (1.0f + expf(-g)) * (late ? half[u][e] : o);
             }
-        qt_store<2, false>(half, dst, CQ_F32, m0 + (late ? 64 : 0), min(rows, m0 + BM), n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
+        qt_store<2, false>(half, dst, CQ_F32, m0 + (late ? 64 : 0), min(rows, m0 + BM), n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes);
     } else {
-        qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, mc);
+        qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, lds + LD::BYTES, lds + LD::BYTES + QtPairs<BM>::SCALES);
     }
 #endif
 }
@@ -695,11 +701,13 @@ int qtile_mi(int mi, int nw, bool moe, dim3 grid, const void *w, const ActView &
              const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
 #define QT_GO(M, E, NW)                                                                                                                                          \
     if constexpr (DT == CQ_Q6K || M > 2) {                                                                                                                       \
-        static_assert(QwLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                     \
-        return qtile_go(qtile_wide_kernel<DT, M, E, NW>, NW, QwLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
+        constexpr int bytes = QwLds<DT, M, NW>::BYTES + (E ? QtPairs<32 * M>::BYTES : 0);                                                                        \
+        static_assert(bytes <= 160 * 1024, "LDS of a CU");                                                                                                       \
+        return qtile_go(qtile_wide_kernel<DT, M, E, NW>, NW, bytes, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
     } else {                                                                                                                                                     \
-        static_assert(QtLds<DT, M, NW>::BYTES <= 160 * 1024, "LDS of a CU");                                                                                     \
-        return qtile_go(qtile_kernel<DT, M, E, NW>, NW, QtLds<DT, M, NW>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
+        constexpr int bytes = QtLds<DT, M, NW>::BYTES + (E ? QtPairs<32 * M>::BYTES : 0);                                                                        \
+        static_assert(bytes <= 160 * 1024, "LDS of a CU");                                                                                                       \
+        return qtile_go(qtile_kernel<DT, M, E, NW>, NW, bytes, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s); \
     }
     if (moe) {
         if (mi == 1) { QT_GO(1, true, QT_NW); }
@@ -868,7 +876,7 @@ int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, co
 // tile_rows: rows of one chunk of the table, 32 or 128
 int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows,
                         hipStream_t s) {
-    const dim3 grid((unsigned)mc.max_chunks, (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)));
+    const dim3 grid(cq_moe_grid(mc, num_experts, pairs, tile_rows), (unsigned)((n + 32 * QT_NW - 1) / (32 * QT_NW)));
     if (grid.y > 65535) return CQ_ERR_RANGE;
     // tiles to be expected: every expert's last one is half full, and few experts have none
     const int64_t tiles = std::max(std::min(num_experts, pairs), pairs / tile_rows + num_experts / 2);

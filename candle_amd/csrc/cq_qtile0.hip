@@ -48,17 +48,25 @@ __device__ __forceinline__ void q0_store(const f32x16 (&acc)[MI], void *dst, int
     const bool plane = !MOE && blockIdx.z > 0;
     if (plane) dst = planes + (int64_t)(blockIdx.z - 1) * rows * qt_plane_ld(n);
     const int64_t ld = plane ? qt_plane_ld(n) : stride_dst;
+    int row[MI];                                           // (all of them in front of the stores, which they would be waited for behind)
+    float by[MI];
+    if constexpr (MOE) {
+#pragma unroll
+        for (int t = 0; t < MI; t++) {
+            row[t] = mc.pair_out[min(m0 + 32 * t + nr, rows - 1)];
+            by[t] = mc.pair_scale[min(m0 + 32 * t + nr, rows - 1)];
+        }
+    }
 #pragma unroll
     for (int t = 0; t < MI; t++) {
         const int mm = m0 + 32 * t + nr;
         if (mm >= rows) break;
-        const int64_t at = (MOE ? mc.pair_out[mm] : mm) * ld;
-        const float by = MOE ? mc.pair_scale[mm] : 1.0f;
+        const int64_t at = (MOE ? row[t] : mm) * ld;
 #pragma unroll
         for (int e4 = 0; e4 < 4; e4++) {
             const int nn = n0 + 8 * e4 + 4 * kg;
             f32x4 v = {acc[t][4 * e4], acc[t][4 * e4 + 1], acc[t][4 * e4 + 2], acc[t][4 * e4 + 3]};
-            if (MOE) v *= by;
+            if (MOE) v *= by[t];
             if (MOE || plane || dst_dtype == CQ_F32) {
                 float *const out = (float *)dst + at + nn;
                 if (nn + 4 <= n) *reinterpret_cast<f32x4_at4 *>(out) = v;
@@ -93,14 +101,17 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nr = lane & 31, kg = lane >> 5;
-    int m0 = blockIdx.x * BM;
-    const int n0 = blockIdx.y * BN + 32 * wv;
+    int m0 = blockIdx.x * BM, block = blockIdx.y;
     if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+        int tile;
+        qt_moe_tile(tile, block);
+        if (tile >= mc.n_chunks[0]) return;
+        m0 = mc.first[tile];
+        rows = m0 + mc.count[tile];
+        w += (int64_t)mc.expert[tile] * expert_bytes;
+        if constexpr (!WF) QtPairs<BM>::request(mc, m0, rows, lds + LD::BYTES, wv, lane);
     }
+    const int n0 = block * BN + 32 * wv;
     const int nsb_all = k >> 8;
     const int kb0 = (uint32_t)nsb_all * blockIdx.z / gridDim.z, kb1 = (uint32_t)nsb_all * (blockIdx.z + 1) / gridDim.z;
     const int64_t row_bytes = (int64_t)nsb_all * (8 * BB);
@@ -345,7 +356,7 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
         }
         return;
     }
-    if constexpr (!WF) qt_store<1, MOE>(acc, dst, dst_dtype, m0, rows, n0 + nr, n, kg, stride_dst, planes, mc);
+    if constexpr (!WF) qt_store<1, MOE>(acc, dst, dst_dtype, m0, rows, n0 + nr, n, kg, stride_dst, planes, lds + LD::BYTES, lds + LD::BYTES + QtPairs<BM>::SCALES);
     else q0_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, nr, n0, n, kg, stride_dst, planes, mc);
 #endif
 }
@@ -366,7 +377,7 @@ static constexpr int64_t Q0_ONE_ROUND = 256, Q0_TWO_ROUNDS[2] = {500, 640}, Q0_C
 template <int DT>
 static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &av, void *dst, int dst_dtype, int64_t k, int64_t n, int64_t rows, int64_t stride_dst,
                      const MoeChunks &mc, int64_t expert_bytes, float *planes, hipStream_t s) {
-#define Q0_GO(M, E, F) return qtile_go(qtile0_kernel<DT, M, E, F>, QT_NW, Q0Lds<DT, M, F>::BYTES, grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
+#define Q0_GO(M, E, F) return qtile_go(qtile0_kernel<DT, M, E, F>, QT_NW, Q0Lds<DT, M, F>::BYTES + (E && !F ? QtPairs<32 * M>::BYTES : 0), grid, w, av, dst, dst_dtype, k, n, rows, stride_dst, mc, expert_bytes, planes, s)
     if (moe) {
         if (mi != 1) Q0_GO(4, true, true);
         if constexpr (DT == CQ_Q4_0)
