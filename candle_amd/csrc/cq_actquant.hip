@@ -130,7 +130,8 @@ int launch_quantize_act(int w_dtype, const void *x, void *scratch, int64_t k, in
 }
 
 // Scratch row i = quantized silu(gate[row_map[i]]) * up[row_map[i]] (rows of k contiguous floats), and scale_out[i] =
-// scale_in[row_map[i]], for i < *n_valid: the down projection of an expert MLP over pairs that an earlier call has bucketed by expert.
+// scale_in[row_map[i]], for i < *n_valid: the down projection of an expert MLP over pairs that an earlier call has bucketed by expert.  PLAIN: of gate alone.
+template <bool PLAIN>
 __global__ __launch_bounds__(256) void quantize_q8k_swiglu_gather_kernel(const float *__restrict__ gate, const float *__restrict__ up,
                                                                          const int *__restrict__ row_map, const int *__restrict__ n_valid,
                                                                          const float *__restrict__ scale_in, float *__restrict__ scale_out, int kb,
@@ -143,7 +144,8 @@ __global__ __launch_bounds__(256) void quantize_q8k_swiglu_gather_kernel(const f
     const int src = row < *n_valid ? row_map[row] : 0;          // (rows behind the last valid pair are in no tile: any valid source)
     const int64_t off = ((int64_t)src * kb + b) * 256 + lane * 4;
     float v[4];
-    cq_load_swiglu4(gate, up, off, off, v);
+    if constexpr (PLAIN) cq_load4<CQ_F32>(gate, off, v);
+    else cq_load_swiglu4(gate, up, off, off, v);
     cq_quantize_q8k_vals(v, blk, lane, qs, dout, bsums);
     if (b == 0 && lane == 0) scale_out[row] = scale_in[src];
 }
@@ -210,7 +212,7 @@ int cq_quantize_act_spread_launch(int w_dtype, const float *x, const int *tokens
     return (int)hipGetLastError();
 }
 
-// Scratch rows [0, rows) = quantized silu(gate[row_map[i]]) * up[row_map[i]], scale_out[i] = scale_in[row_map[i]].
+// Scratch rows [0, rows) = quantized silu(gate[row_map[i]]) * up[row_map[i]] (without up, of K formats: gate[row_map[i]]), scale_out[i] = scale_in[row_map[i]].
 int cq_quantize_act_swiglu_gather_launch(int w_dtype, const float *gate, const float *up, const int *row_map, const int *n_valid, const float *scale_in,
                                          float *scale_out, void *scratch, int64_t k, int64_t rows, int64_t rows_alloc, hipStream_t s) {
     if (k % 256) return CQ_ERR_SHAPE;
@@ -220,8 +222,9 @@ int cq_quantize_act_swiglu_gather_launch(int w_dtype, const float *gate, const f
     const int64_t spans = rows * (k / 256);
     const int64_t grid = (spans + 3) / 4;
     if (grid > 0x7fffffffLL) return CQ_ERR_RANGE;
+    if (!up && !cq_is_kquant(w_dtype)) return CQ_ERR_DTYPE;
     if (cq_is_kquant(w_dtype))
-        hipLaunchKernelGGL(quantize_q8k_swiglu_gather_kernel, dim3((unsigned)grid), dim3(256), 0, s, gate, up, row_map, n_valid, scale_in, scale_out, (int)(k / 256),
+        hipLaunchKernelGGL(up ? quantize_q8k_swiglu_gather_kernel<false> : quantize_q8k_swiglu_gather_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, gate, up, row_map, n_valid, scale_in, scale_out, (int)(k / 256),
                            (int8_t *)(b + L.qs_off), (float *)(b + L.d_off), (int16_t *)(b + L.bs_off), spans);
     else
         hipLaunchKernelGGL(quantize_q80_swiglu_gather_kernel, dim3((unsigned)grid), dim3(256), 0, s, gate, up, row_map, n_valid, scale_in, scale_out, (int)(k / 256),

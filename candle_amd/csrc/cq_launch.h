@@ -82,13 +82,15 @@ struct MoeArgs {
     // optional second grouped matmul over the same x and pairs (gate and up of an expert MLP): out_b = x W_b^T
     const void *w_b = nullptr;
     float *out_b = nullptr;
+    // out = silu(x W^T) * (x W_b^T), in one launch (or CQ_ERR_RANGE)
+    bool swiglu = false;
 };
 int64_t cq_moe_workspace_bytes_impl(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t x_rows, int64_t k);
 int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s);
 // The down projection of an expert MLP right after a grouped gate / up call (cq_moe_launch with w_b, more pairs than the per-pair
 // kernels take) on the same workspace and pair list: out[pair] = topk_weights[pair] * W_down[e] . quantize(silu(gate[pair]) * up[pair]),
 // with the grouping that call left in the workspace.  CQ_ERR_RANGE when that call did not group on the matrix-core path or the
-// quantized rows of this one do not fit in front of its tables.
+// quantized rows of this one do not fit in front of its tables.  up == nullptr: after a call with swiglu, whose out gate is.
 int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *gate, const float *up, const float *topk_weights, float *out,
                                   int64_t num_experts, int64_t topk, int64_t n_pairs, int64_t n, int64_t k, int64_t k_pair, void *workspace,
                                   hipStream_t s);
@@ -157,6 +159,7 @@ struct MoeChunks {
     const int *pair_out;
     const float *pair_scale;
     int max_chunks;
+    int64_t up = 0;      // bytes from the gate weights to the up weights, where a launch multiplies by both
 };
 // Tiles of tile_rows pairs that a list of `pairs` can have: whole ones, and one that is not for every expert.  A multiple of eight (qt_moe_tile).
 inline unsigned cq_moe_grid(const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t tile_rows) {
@@ -169,6 +172,7 @@ int cq_moe_chunks_launch(int w_dtype, const void *w, const void *scratch, int64_
 // Q4_K experts hit by a few dozen pairs each as batched matvecs (cq_matvec_batch.hip): the expert-sorted pairs of an expert are the
 // batch rows, in sets of 16 whose quantized rows sit in operand tiles.
 bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);      // ... by shape alone
+bool cq_moe_wants_aligned(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);
 bool cq_moe_stream_takes(int w_dtype, const void *w, const void *w_b, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);
 int64_t cq_moe_stream_operand_bytes(int64_t num_experts, int64_t n_pairs, int64_t k);
 #define CQ_MOE_STREAM_CHUNK 16
@@ -194,6 +198,9 @@ bool cq_qtile_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, in
 int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *dst, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes,
                            hipStream_t s);
 // num_experts, pairs: what the number of tiles that hold rows follows from
+bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n, int tile_rows);
+int cq_qtile_moe_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k,
+                               int64_t n, int tile_rows, hipStream_t s);
 int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows,
                         hipStream_t s);
 int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,

@@ -727,7 +727,7 @@ struct QmeArgs {
     int extra_parts;              // parts per expert and tensor that a listed pass is cut into (a multiple of parts: finer than a workgroup's own share)
 };
 constexpr int QME_NS = 2;         // sets of 16 pairs per pass over the weights
-constexpr int QME_MAX_AVG_PAIRS = 64;   // pairs per expert on average up to which a call takes this form
+constexpr int QME_MAX_AVG_PAIRS = 27;   // pairs per expert on average up to which a call takes this form
 constexpr int QME_DEPTH = 4;      // tiles of the ring where LDS holds them
 
 template <int CW, int CPW, int DEPTH, bool Q5 = false>
@@ -1109,12 +1109,19 @@ int cq_matvec_batch_swiglu_launch(int w_dtype, const void *w, const float *gate,
 
 // ---- MoE: experts as batched matvecs (see qme_q4k_kernel) ----
 // Q4_K or Q5_K experts of rows up to 16 super-blocks (two columns per wave: three do not fit the registers next to two operand sets),
-// 16-byte aligned, and on average at most 64 pairs per expert: beyond that a pass over the weights per 32 pairs loses to the
-// tiles that reuse a weight 32 or 128 times.
-bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
+// 16-byte aligned, and on average at most 27 pairs per expert: beyond that a pass over the weights per 32 pairs loses to the
+// tiles that reuse a weight 128 times.  us of a layer, batched matvecs / tiles: 64 experts of 2048 x 1024, 6 each, 230 / 330 / 430 / 640 tokens Q4_K 109 112, 145 126, 178 136, 230 157,
+// Q5_K 119 131, 157 144, 192 155, 249 174; 128 of 2048 x 768, 8 each, 400 / 600 / 1000 Q4_K 168 174, 248 200, 336 237, Q5_K 184 203, 266 228, 362 264; 64 of 1024 x 512, 4 each,
+// 400 / 900 Q4_K 70 54, 110 70, Q5_K 71 60, 113 78.
+static bool qme_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n, int64_t pairs_each) {
     return qb_weights(w_dtype) && k % 256 == 0 && k / 256 <= 2 * QB_NW && n >= 1 && n <= 0x7ffffff0 / 16 && num_experts >= 1 && num_experts <= 65535 &&
-           n_pairs <= QME_MAX_AVG_PAIRS * num_experts && n * (k / 256) * qb_bb(w_dtype == CQ_Q5K) < 0x7fffffffLL;
+           n_pairs <= pairs_each * num_experts && n * (k / 256) * qb_bb(w_dtype == CQ_Q5K) < 0x7fffffffLL;
 }
+bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
+    return qme_shape(w_dtype, num_experts, n_pairs, k, n, QME_MAX_AVG_PAIRS);
+}
+// Up to 64 pairs an expert a gate / up call, and a down projection on its grouping, ask for 16-byte aligned experts, whichever form they take.
+bool cq_moe_wants_aligned(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) { return qme_shape(w_dtype, num_experts, n_pairs, k, n, 64); }
 bool cq_moe_stream_takes(int w_dtype, const void *w, const void *w_b, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
     return cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)w_b & 15) == 0;
 }

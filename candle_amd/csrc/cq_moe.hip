@@ -14,7 +14,7 @@
 // hit expert's rows once: workgroup (row tile, expert) keeps the decoded weight registers and loops
 // over that expert's pairs — unlike the reference kernels, which re-read the expert's weights for
 // every pair routed to it.  (Few pairs skip steps 1 and 2: a fused matvec per pair.  Hundreds of pairs take step 3 on the matrix
-// cores: Q4_K experts with up to 64 pairs each as batched matvecs over their pairs, cq_matvec_batch.hip, the rest as tiles of
+// cores: Q4_K and Q5_K experts with up to 27 pairs each as batched matvecs over their pairs, cq_matvec_batch.hip, the rest as tiles of
 // expert-sorted rows through the prefill kernel of the format.)
 #include <algorithm>
 #include "cq_device.h"
@@ -364,7 +364,17 @@ static bool moe_takes_mfma(int w_dtype, const void *w, const void *w_b, int64_t 
     const bool q0_ok = (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) && ((uintptr_t)w & 7) == 0 && (!w_b || ((uintptr_t)w_b & 7) == 0);
     return k % 256 == 0 && (cq_is_kquant(w_dtype) || q0_ok) && cq_has_mfma(w_dtype) && n_pairs >= CQ_MOE_MFMA_MIN_PAIRS;
 }
-static int moe_tile_rows(int64_t n_pairs, int64_t num_experts) { return n_pairs < 40 * num_experts ? CQ_MOE_TILE_SMALL : CQ_MOE_TILE_LARGE; }
+// Rows of a tile of one expert's pairs: 128 (of which parts of 32 rows that are not there are left out) from 19 pairs an expert on, so that most experts convert and read their weights once.
+// n: rows of an expert's weights (of a gate / up call, whose grouping the down projection takes over: of that call).  Experts of 32-element blocks have room for more workgroups a unit
+// in tiles of 32 rows; where those of 128 leave much of a second round empty (128 experts of 768 rows: 384 workgroups), from 30 on.  us of a layer, limit at 8 / 20 / 40 pairs an expert:
+//   Q6_K 64 experts of 2048 x 1024, 6 each, 170 tokens 184 181 181, 205: 189 225 225, 400: 214 214 314; 128 of 1024 x 512, 8 each, 310: 189 193 193, 620: 221 221 326
+//   Q8_0 64 of 2048 x 1024, 170: 163 150 150, 205: 169 195 195, 400: 189 189 239; 128 of 2048 x 768, 310: 269 244 244, 420: 287 287 262, 500: 299 299 327
+//   Q4_0 64 of 2048 x 1024, 170: 140 156 156, 205: 149 185 185; 128 of 2048 x 768, 250: 230 195 195, 310: 236 222 222
+static int moe_tile_rows(int w_dtype, int64_t n_pairs, int64_t num_experts, int64_t n) {
+    const int64_t wgs = num_experts * ((n + 255) / 256), rounds = (wgs + 255) / 256;
+    const bool gaps = !cq_is_kquant(w_dtype) && rounds > 1 && 5 * wgs < 4 * 256 * rounds;
+    return n_pairs < (gaps ? 30 : 19) * num_experts ? CQ_MOE_TILE_SMALL : CQ_MOE_TILE_LARGE;
+}
 
 int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *gate, const float *up, const float *topk_weights, float *out,
                                   int64_t num_experts, int64_t topk, int64_t n_pairs, int64_t n, int64_t k, int64_t k_pair, void *workspace,
@@ -379,6 +389,7 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
     // the pair call ran its experts as batched matvecs (chunks of 16 pairs): this one must be able to as well
     // (n of the pair call = this call's k; its expert tensors were 16-byte aligned or it returned CQ_ERR_ALIGN)
     if (cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k_pair, k)) {
+        if (!up) return CQ_ERR_RANGE;                      // (such calls have no swiglu form)
         if (!cq_moe_stream_takes(w_dtype, w_down, nullptr, num_experts, n_pairs, k, n)) return CQ_ERR_RANGE;
         if (cq_align256(cq_moe_stream_operand_bytes(num_experts, n_pairs, k)) > ws.offsets_off) return CQ_ERR_RANGE;
         uint8_t *b = (uint8_t *)workspace;
@@ -391,6 +402,7 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
         return cq_moe_stream_launch(w_dtype, w_down, nullptr, out, nullptr, b + ws.act_off, offsets, pout, pscale, (int *)(b + ws.extra_off), 1,
                                     num_experts, k, n, s);
     }
+    if (cq_moe_wants_aligned(w_dtype, num_experts, n_pairs, k_pair, k) && ((uintptr_t)w_down & 15)) return CQ_ERR_RANGE;
     // the rows of this call are quantized into the front of the workspace: they must end before that call's tables begin
     if (cq_act_layout(w_dtype, k, ws.rows_alloc).total > ws.offsets_off) return CQ_ERR_RANGE;
     uint8_t *b = (uint8_t *)workspace;
@@ -402,7 +414,7 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
     int rc = cq_quantize_act_swiglu_gather_launch(w_dtype, gate, up, pout, n_valid, topk_weights, pscale, b + ws.act_off, k, n_pairs, ws.rows_alloc, s);
     if (rc) return rc;
     MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
-    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, num_experts, k, n, moe_tile_rows(n_pairs, num_experts), s);
+    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, num_experts, k, n, moe_tile_rows(w_dtype, n_pairs, num_experts, k), s);
 }
 
 int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
@@ -412,6 +424,12 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     const bool stream = stream_shape && cq_moe_stream_takes(a.w_dtype, a.w, a.w_b, a.num_experts, a.n_pairs, a.k, a.n);
     // (a later cq_moe_down_after_pair_launch tells from the shape alone how this call chunked its pairs)
     if (a.w_b && stream_shape && !stream) return CQ_ERR_ALIGN;
+    if (a.w_b && !a.swiglu && mfma && !cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) && cq_moe_wants_aligned(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n) &&
+        (((uintptr_t)a.w | (uintptr_t)a.w_b) & 15))
+        return CQ_ERR_ALIGN;
+    if (a.swiglu && (!mfma || stream_shape || cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) ||
+                     !cq_qtile_moe_takes_swiglu(a.w_dtype, a.w, a.w_b, a.num_experts, a.k, a.n, moe_tile_rows(a.w_dtype, a.n_pairs, a.num_experts, a.n))))
+        return CQ_ERR_RANGE;
     if (a.w_b && !mfma) {
         // only the MFMA path shares its grouping pass and quantized activations between two weight tensors
         MoeArgs one = a;
@@ -441,7 +459,7 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     int *extra = (int *)(b + ws.extra_off);
     // Hundreds of pairs per call: the expert-sorted rows go through the MFMA prefill kernel of the format in tiles of up to
     // 128 rows of one expert (integer-exact like the dense paths).  Otherwise 8 pairs per matvec pass.
-    const int tile_rows = moe_tile_rows(a.n_pairs, a.num_experts);
+    const int tile_rows = moe_tile_rows(a.w_dtype, a.n_pairs, a.num_experts, a.n);
     const bool many = a.n_pairs > GROUP_MANY_PAIRS;
     auto *const group = a.num_experts <= GROUP_LDS_EXPERTS ? (many ? moe_group_kernel<true, true> : moe_group_kernel<true, false>)
                                                            : (many ? moe_group_kernel<false, true> : moe_group_kernel<false, false>);
@@ -467,6 +485,8 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
                     : cq_quantize_act_gather_launch(a.w_dtype, a.x, pin, b + ws.act_off, a.k, a.n_pairs, ws.rows_alloc, s);
         if (rc) return rc;
         MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
+        if (a.swiglu)
+            return cq_qtile_moe_swiglu_launch(a.w_dtype, a.w, a.w_b, cq_act_view(b + ws.act_off, a.w_dtype, a.k, ws.rows_alloc), a.out, mc, a.num_experts, ws.rows_alloc, a.k, a.n, tile_rows, s);
         rc = cq_matmul_moe_launch(a.w_dtype, a.w, b + ws.act_off, ws.rows_alloc, a.out, mc, a.num_experts, a.k, a.n, tile_rows, s);
         if (!rc && a.w_b) rc = cq_matmul_moe_launch(a.w_dtype, a.w_b, b + ws.act_off, ws.rows_alloc, a.out_b, mc, a.num_experts, a.k, a.n, tile_rows, s);
         return rc;

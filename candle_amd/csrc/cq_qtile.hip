@@ -345,7 +345,7 @@ template <int DT, int MI, int NW> struct QwLds {
     static constexpr int A_OFF = 0, AM_OFF = (AHEAD + 1) * A, D8_OFF = AM_OFF + (AHEAD + 1) * AM, B_OFF = D8_OFF + (AHEAD + 1) * D8, BYTES = bytes(AHEAD);
 };
 
-// PAIR: rows of two tensors, the second pair bytes behind the first: waves 0 .. 3 multiply by 128 rows of the first, waves 4 .. 7 by the same rows of the second, and the
+// PAIR: rows of two tensors, the second expert_bytes (of experts: mc.up) behind the first: waves 0 .. 3 multiply by 128 rows of the first, waves 4 .. 7 by the same rows of the second, and the
 // results are silu(first) * second (Mlp::forward, quantized_llama.rs:56-63).  At the end the two waves of a SIMD, which have the same rows and columns of both, hand each other
 // half of their tiles through LDS, so that both compute and store.  What it saves is a write and a read of both products where one result does, and what it costs is
 // that the silu of a workgroup's results has no other workgroup to hide behind (1000 rows of two Q4_K [14336 x 4096]: 309 us and 30.5 of the quantizer that took both products,
@@ -357,14 +357,14 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
     typedef QWide<DT> T;
     typedef QwLds<DT, MI, NW> LD;
     static_assert(NW == 8 || (NW == 4 && MI <= 2), "two waves bring the sums and two the scales of 64 rows at most");
-    static_assert(!PAIR || (NW == 8 && MI > 2 && !MOE), "tiles of four pairs of waves");
+    static_assert(!PAIR || (NW == 8 && MI > 2), "tiles of four pairs of waves");
     constexpr int BB = BlockInfo<DT>::bytes, BM = 32 * MI, BN = PAIR ? 16 * NW : 32 * NW, AHEAD = LD::AHEAD, ROW = 16 * T::PIECES;
     constexpr int NA = 8 * MI / NW, NX = NA + 1, NB = LD::NB + (DT == CQ_Q6K ? 1 : 0);      // copies per wave and super-block: activations, with scales or sums, weights
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nr = lane & 31, kg = lane >> 5;
     int m0 = blockIdx.x * BM, block = blockIdx.y;
-    if (PAIR && wv >= 4) w += expert_bytes;
+    if (PAIR && wv >= 4) w += MOE ? mc.up : expert_bytes;
     if (MOE) {
         int tile;
         qt_moe_tile(tile, block);
@@ -645,7 +645,8 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
                 const float o = other[64 * (16 * u + e)], g = late ? o : half[u][e];
                 half[u][e] = g / (1.0f + expf(-g)) * (late ? half[u][e] : o);
             }
-        qt_store<2, false>(half, dst, CQ_F32, m0 + (late ? 64 : 0), min(rows, m0 + BM), n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes);
+        const uint8_t *const to = lds + LD::BYTES + (late ? 256 : 0);
+        qt_store<2, MOE>(half, dst, CQ_F32, m0 + (late ? 64 : 0), min(rows, m0 + BM), n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, to, to + QtPairs<BM>::SCALES);
     } else {
         qt_store<MI, MOE>(acc, dst, dst_dtype, m0, rows, n0 + (lane_out & 31), n, lane_out >> 5, stride_dst, planes, lds + LD::BYTES, lds + LD::BYTES + QtPairs<BM>::SCALES);
     }
@@ -881,4 +882,29 @@ int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *ou
     // tiles to be expected: every expert's last one is half full, and few experts have none
     const int64_t tiles = std::max(std::min(num_experts, pairs), pairs / tile_rows + num_experts / 2);
     return qtile_any(w_dtype, tile_rows / 32, QT_NW, true, grid, w, av, out, CQ_F32, k, n, tiles, n, mc, n * (k / cq_block_size(w_dtype)) * cq_type_size(w_dtype), nullptr, s);
+}
+
+// silu(gate) * up of experts in tiles of 128 rows, K formats.  1500 tokens, 128 Q4_K experts of 2048 x 768, 8 each: 131 us, and 15 of the quantizer behind; a launch of 1.5 rounds for
+// each of the two took 79 and 79, and the quantizer that multiplied them 22.
+bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n, int tile_rows) {
+    return tile_rows == 128 && (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K || w_dtype == CQ_Q6K) && cq_qtile_takes(w_dtype, w_gate, k, num_experts * n) &&
+           cq_qtile_takes(w_dtype, w_up, k, num_experts * n) && (n + 16 * QT_NW - 1) / (16 * QT_NW) <= 65535;
+}
+template <int DT>
+static int moe_swiglu_go(dim3 grid, const void *w, const ActView &av, float *out, int64_t k, int64_t n, const MoeChunks &mc, hipStream_t s) {
+    constexpr int bytes = QwLds<DT, 4, QT_NW>::BYTES + QtPairs<128>::BYTES;
+    return qtile_go(qtile_wide_kernel<DT, 4, true, QT_NW, true>, QT_NW, bytes, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / 256) * cq_type_size(DT), nullptr, s);
+}
+int cq_qtile_moe_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k,
+                               int64_t n, int tile_rows, hipStream_t s) {
+    if (!cq_qtile_moe_takes_swiglu(w_dtype, w_gate, w_up, num_experts, k, n, tile_rows)) return CQ_ERR_RANGE;
+    MoeChunks both = mc;
+    both.up = (const uint8_t *)w_up - (const uint8_t *)w_gate;
+    const dim3 grid(cq_moe_grid(mc, num_experts, pairs, tile_rows), (unsigned)((n + 16 * QT_NW - 1) / (16 * QT_NW)));
+    switch (w_dtype) {
+        case CQ_Q4K: return moe_swiglu_go<CQ_Q4K>(grid, w_gate, av, out, k, n, both, s);
+        case CQ_Q5K: return moe_swiglu_go<CQ_Q5K>(grid, w_gate, av, out, k, n, both, s);
+        case CQ_Q6K: return moe_swiglu_go<CQ_Q6K>(grid, w_gate, av, out, k, n, both, s);
+    }
+    return CQ_ERR_RANGE;
 }

@@ -118,6 +118,17 @@ class FusedMoeGGUF:
             if fused != -6:
                 ck("cq_moe_gemm_gguf_swiglu", fused)
         down_done = False
+        if fused == -6 and self.share_grouping:
+            # hundreds of pairs of K-quant experts: gate, up and the activation in the tiles of one launch, the down projection on its grouping
+            fused = L.cq_moe_gemm_gguf_pair_swiglu(dt, x2.data_ptr(), self.gate_experts.device_ptr(), self.up_experts.device_ptr(), sti_ptr, eid_ptr,
+                                                   self.down_in.data_ptr(), E, topk, pairs, self.inter, hidden, self.ws.data_ptr(), self.ws.numel(), sp)
+            if fused != -6:
+                ck("cq_moe_gemm_gguf_pair_swiglu", fused)
+                rc = L.cq_moe_gemm_gguf_down_after_swiglu(dt, self.down_in.data_ptr(), self.down_experts.device_ptr(), self.topk_weights.data_ptr(), self.down_out.data_ptr(),
+                                                          E, topk, pairs, hidden, self.inter, hidden, self.ws.data_ptr(), self.ws.numel(), sp)
+                if rc != -6:
+                    ck("cq_moe_gemm_gguf_down_after_swiglu", rc)
+                    down_done = True
         if fused == -6:                                          # CQ_ERR_RANGE: not a shape of the fused launch
             # gate and up share x and the pairs: one grouping pass and one activation quantization for both
             ck("cq_moe_gemm_gguf_pair", L.cq_moe_gemm_gguf_pair(dt, x2.data_ptr(), self.gate_experts.device_ptr(), self.up_experts.device_ptr(),

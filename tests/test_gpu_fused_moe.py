@@ -234,6 +234,50 @@ def test_down_projection_on_the_grouping_of_gate_and_up(dtype, tokens, E, topk):
     assert rel_l2(shared, ref.forward(x)) <= 1e-3
 
 
+@pytest.mark.parametrize("dtype", [oracle.Q4K, oracle.Q5K, oracle.Q6K])
+@pytest.mark.parametrize("counts", [[300, 0, 1, 33, 64, 65, 127, 130], [28] * 24, [19, 20, 18, 19] * 6])
+@pytest.mark.parametrize("inter,hidden", [(256, 512), (768, 256), (512, 2048)])
+def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
+    """silu(gate) * up in the tiles of one launch, and the down projection behind it: bit for bit what the two products, cq_nn_silu_mul and the down projection of their own give.  Pairs that
+    name no expert are left alone."""
+    from candle_amd import _lib
+    from tests.test_gpu_moe import make_experts
+    lib, E, topk = L(), len(counts), 2
+    eid = np.repeat(np.arange(E, dtype=np.int32), counts)
+    rng = np.random.Generator(np.random.PCG64(hidden + inter))
+    pairs = eid.size
+    assert pairs % topk == 0
+    eid[rng.integers(0, pairs, 3)] = E + 5
+    sti = rng.permutation(pairs).astype(np.int32)
+    sti, eid = torch.from_numpy(sti).cuda(), torch.from_numpy(eid).cuda()
+    (_, g), (_, u), (_, d) = (make_experts(dtype, E, n, k, seed=s) for n, k, s in ((inter, hidden, 1), (inter, hidden, 2), (hidden, inter, 3)))
+    x, tw = torch.from_numpy(normal(4, (pairs // topk, hidden), 1.0)).cuda(), torch.from_numpy(rng.uniform(0.1, 1.0, pairs).astype(np.float32)).cuda()
+    nb = max(lib.cq_moe_gemm_workspace_bytes(int(dtype), E, topk, pairs, inter, hidden, 0), lib.cq_moe_gemm_workspace_bytes(int(dtype), E, topk, pairs, hidden, inter, 1))
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    h, out = torch.full((pairs, inter), 7.0, device="cuda"), torch.full((pairs, hidden), 7.0, device="cuda")
+    swiglu = lib.cq_moe_gemm_gguf_pair_swiglu(int(dtype), x.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), h.data_ptr(), E, topk, pairs, inter, hidden,
+                                              ws.data_ptr(), nb, None)
+    batched = dtype in (oracle.Q4K, oracle.Q5K) and pairs <= 27 * E
+    short = dtype == oracle.Q6K and hidden < 1536                     # (left to the general kernels)
+    if batched or short or pairs < 19 * E:
+        assert swiglu == -6 and bool((h == 7).all())                  # CQ_ERR_RANGE: nothing enqueued
+        return
+    _lib.check("cq_moe_gemm_gguf_pair_swiglu", swiglu)
+    down = lib.cq_moe_gemm_gguf_down_after_swiglu(int(dtype), h.data_ptr(), d.device_ptr(), tw.data_ptr(), out.data_ptr(), E, topk, pairs, hidden, inter, hidden, ws.data_ptr(), nb, None)
+    assert down == (0 if inter <= hidden else -6)                     # longer rows than the first call's do not fit in front of its tables: nothing enqueued
+    a, b, both, want = (torch.full((pairs, c), 7.0, device="cuda") for c in (inter, inter, inter, hidden))
+    _lib.check("pair", lib.cq_moe_gemm_gguf_pair(int(dtype), x.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), a.data_ptr(), b.data_ptr(), E, topk, pairs, inter,
+                                                 hidden, 1, ws.data_ptr(), nb, None))
+    named = torch.zeros(pairs, dtype=torch.bool, device="cuda")
+    named[sti[eid < E].long()] = True
+    assert bool((h[~named] == 7).all()) and bool((out[~named] == 7).all())
+    _lib.check("silu", lib.cq_nn_silu_mul(a.data_ptr(), b.data_ptr(), both.data_ptr(), pairs, inter, inter, inter, None))
+    assert torch.equal(h[named], both[named])
+    _lib.check("down", lib.cq_moe_gemm_gguf(int(dtype), both.data_ptr(), d.device_ptr(), sti.data_ptr(), eid.data_ptr(), tw.data_ptr(), want.data_ptr(), E, topk, pairs, hidden, inter, 1,
+                                            ws.data_ptr(), nb, None))
+    assert torch.equal(out[named], want[named]) if down == 0 else bool((out == 7).all())
+
+
 def test_down_after_pair_refuses_what_it_cannot_reuse():
     lib = L()
     p = 256          # an aligned non-null address: the calls below return before anything is enqueued

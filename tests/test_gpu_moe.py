@@ -91,7 +91,7 @@ def test_moe_gemm_gguf_gate_and_down(dtype, tokens, is_prefill):
 @pytest.mark.parametrize("k,n", [(256, 64), (512, 40), (768, 203), (1024, 130), (1792, 50), (2048, 96), (2304, 33), (4096, 72)])
 @pytest.mark.parametrize("with_weights", [False, True])
 def test_moe_gemm_gguf_experts_as_batched_matvecs(wdt, k, n, with_weights):
-    """Q4_K or Q5_K experts hit by at most 64 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
+    """Q4_K or Q5_K experts hit by at most 27 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
     over the weights).  Expert loads on every edge: none, one pair, 15 / 16 / 17, 31 / 32 / 33 (a second pass), 47 .. 49, 65 (a
     third pass); rows of 1 .. 16 super-blocks (one to eight waves per row block, columns without a wave's second column), ragged
     n, several workgroups per expert."""
@@ -143,6 +143,31 @@ def test_moe_gemm_gguf_mfma_tile_sizes(dtype, E, n):
     assert err <= TIGHT, err
 
 
+@pytest.mark.parametrize("wdt", [oracle.Q4_0, oracle.Q8_0, oracle.Q4K, oracle.Q5K, oracle.Q6K], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("k,n", [(256, 260), (1536, 203), (2304, 130)])
+def test_moe_gemm_gguf_tiles_of_uneven_experts(wdt, k, n):
+    """Tiles of 128 pairs on every edge of their 32-row parts and with no pair at all, beside workgroups of the grid that have no tile; ragged n in one block of columns and in two; pair by pair,
+    since a row sent to another pair's place would hide in the norm."""
+    import candle_amd as ca
+    counts = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 0, 161, 257, 3]
+    E, topk = len(counts), 2
+    n_pairs = sum(counts)
+    assert n_pairs % topk == 0 and n_pairs >= 64 * E
+    blocks, qt = make_experts(wdt, E, n, k, seed=191)
+    rng = np.random.Generator(np.random.PCG64(192))
+    expert_ids = np.repeat(np.arange(E, dtype=np.int32), counts)
+    sorted_token_ids = rng.permutation(n_pairs).astype(np.int32)
+    x = normal(193, (n_pairs, k), 1.0)
+    tw = rng.uniform(0.1, 1.0, n_pairs).astype(np.float32)
+    got = ca.moe_gemm_gguf(torch.from_numpy(x).cuda(), qt, torch.from_numpy(tw).cuda(), torch.from_numpy(sorted_token_ids).cuda(), torch.from_numpy(expert_ids).cuda(), topk, True)
+    torch.cuda.synchronize()
+    want = oracle.moe_gemm_gguf(wdt, x, blocks, (E, n, k), sorted_token_ids, expert_ids, tw, topk)
+    got = got.cpu().numpy()
+    assert rel_l2(got, want) <= TIGHT
+    for p in range(n_pairs):
+        assert rel_l2(got[p], want[p]) <= 1e-5, p
+
+
 @pytest.mark.parametrize("wdt", [oracle.Q4K, oracle.Q5K], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("k,n", [(2048, 96), (768, 203)])
 def test_moe_gemm_gguf_one_expert_draws_most_pairs(wdt, k, n):
@@ -174,7 +199,7 @@ def test_moe_gemm_gguf_one_expert_draws_most_pairs(wdt, k, n):
 
 def test_moe_gemm_gguf_q4k_rows_too_long_for_the_batched_form():
     """Q4_K experts with rows of more than 16 super-blocks do not run as batched matvecs: 25 pairs per expert go through the
-    32-row tiles of the Q4_K matrix-core kernel."""
+    tiles of the Q4_K matrix-core kernel."""
     import candle_amd as ca
     E, n, k, topk, tokens = 16, 96, 4352, 4, 100
     blocks, qt = make_experts(oracle.Q4K, E, n, k, seed=75)
