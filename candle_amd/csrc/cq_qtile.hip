@@ -763,7 +763,8 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
 // instead of eight if their rows are at most 64: each SIMD then converts and multiplies for one wave, and a small product takes up twice as many
 // compute units (131 rows of Q6_K [4096 x 4096] unsplit: 56 us in eight waves, 41 in four; 65 rows of Q4_K [4096 x 4096] 20.6 -> 17.5).
 // Costs: fitted to earlier kernels (qtile_kernel for all tiles of K formats; the activations first in all of Q4_0 and Q8_0; rounds that leave compute units idle run at a higher clock
-// there, and a workgroup has 1.3 us of its own), which multiplied 32-row parts without rows as well: a part-filled tile still counts as a full one.  With the present kernels the choice is
+// there, and a workgroup has 1.3 us of its own), which multiplied 32-row parts without rows as well: a part-filled tile still counts as a full one.  Of Q4_0 tiles of 160 rows as well, by
+// the same costs (54.4 us predicted 54.9 for 131 rows of [13824 x 5120] in four splits, 94.8 predicted 96.7 for 300 in two; where 128 rows or less are chosen they measured best as well).  With the kernels before those the choice is
 // slower than the best by 1.0 % on average for Q4_K, 0.6 for Q5_K, 1.0 for Q6_K, 1.3 for Q4_0 and 1.1 for Q8_0, by more than 5 % in 3 - 9 % of the calls, by 18 % at most (28 rows of Q6_K
 // [3667 x 3072] 16.7 us in twelve splits of eight waves, 14.1 in six of four): 1800 forwards of drawn sizes, 17 (Q4_K, Q5_K: 65) - 1600 rows, 1024 - 16384 by 1536 - 14336, cold weights, every choice timed.
 // Only splits whose sums round no more than those of the general kernels (qt_roundings).
@@ -803,8 +804,9 @@ static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_
         rounds_less[sp] = sp == general || qt_roundings(nsb, terms, sp, true) < qt_roundings(nsb, terms, general, false);
     QtPlan best{4, QT_NW, general};
     double least = 1e30;
+    const int tallest = w_dtype == CQ_Q4_0 ? 5 : 4;           // (160 rows of Q8_0 do not fit LDS, of K formats the registers)
     for (int nw : {QT_NW, QT_NW_NARROW})
-        for (int mi = 1; mi <= (nw == QT_NW ? 4 : 2); mi++)
+        for (int mi = 1; mi <= (nw == QT_NW ? tallest : 2); mi++)
             for (int sp = 1; sp <= most; sp++) {
                 const int64_t wgs = (rows + 32 * mi - 1) / (32 * mi) * ((n + 32 * nw - 1) / (32 * nw)) * sp, rounds = (wgs + 255) / 256;
                 const bool narrow = nw == QT_NW_NARROW;

@@ -9,18 +9,25 @@
 //
 // A workgroup's eight waves lie side by side along n and share 32 MI rows of activations in LDS (two super-blocks of 256, swizzled so that fragments are read
 // without bank conflicts); a wave owns 32 weight rows, brings their blocks for itself by copies to LDS, half a super-block at a time, and converts each
-// weight once for 32 MI rows.  The products of block b + 1 run on the matrix cores while those of block b are scaled.  WF: the weights are the matrix instructions' first
+// weight once for 32 MI rows.  The products of the next tile run on the matrix cores while those of one are scaled.  WF: the weights are the matrix instructions' first
 // operand, so that a lane has sixteen weight rows' results of one activation row: the sixteen scales of the weights, put into LDS as f32 by the wave itself, are read once per
 // block for all tiles and one scale of the activations per tile.  (The other way round four reads of 16 bytes per tile and block bring the activations' scales, right in front of
 // their use, but a weight row's scale comes with its weights: the better way for some tiles of 32 rows, see launch_mi.)  Results then go out four columns at a time, whatever n
 // is a multiple of.  K is split over grid.z where that fills the chip better; see qtile_plan.
 //
-// us on one card, the activations first in all tiles / now, quantizing the activations included:      17 rows   131 rows   512 rows   2048 rows
+// Only the sums of two tiles are in registers at a time, those of the one that is scaled and of the next, and the main loop exists for each number of 32-row tiles that hold rows, which is
+// what makes that known where registers are given out.  (The sums of all tiles before: 16 registers a tile more, so that tiles end at 128 rows.)  Q4_0 has tiles of 160 rows for it, whose weights are
+// converted once where two tiles of 96 did it twice and left a sixth of the work to one of them: 131 rows of [13824 x 5120] 59.5 -> 51.7 us with f16 results.  Two tiles' sums alone, us:
+//   2048 rows of Q4_0 [14336 x 4096] 393 -> 353, 700 of [11008 x 4096] 124 -> 119; Q8_0 2048 of [4096 x 4096] 106 -> 104; 60 rows of Q4_0 [1536 x 2048] 12.1 -> 12.3 (the longer code)
+//
+// us on one card, the activations first in all tiles / the weights first from 64 rows on, quantizing the activations included:      17 rows   131 rows   512 rows   2048 rows
 //   Q4_0 [14336 x 4096]                                                                              23.5 23.7  57.6 53.7  108 103    412 393
 //   Q8_0 [14336 x 4096]                                                                              27.3 27.3  62.6 56.1  121 111    464 420
-// 2048 rows of Q4_0 are 610 TOP/s.  A block of 32 x 32 results takes 198 cycles of a SIMD where its 32 fmas and a matrix instruction take 138 (on an eighth of the units; with all of
-// them busy the clock falls by a sixth): beside them the conversion of the weights from LDS places on 2 bytes (27 of 296 us), the scales (20) and the fragments (13).
+// 2048 rows of Q4_0 are 680 TOP/s.  What a block of 32 x 32 results takes beyond its 32 fmas and a matrix instruction (138 cycles of a SIMD): the conversion of the weights from LDS places
+// on 2 bytes, the scales and the fragments.
 #include "cq_qtile.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -260,63 +267,83 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
         row_scales(0);
         f32x4 dw[4];
         scales_of(0, dw);
-        for (int j = 0; j < nsb; j++) {
-            const int kb = kb0 + j, slot = j & 1;
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            issue_w(kb, 1);
-            request(j + 1);
-            const uint8_t *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 4 * nr;
-            auto d8_of = [&](int b, float (&d)[MI]) {
+        // the main loop, for each number of tiles that hold rows
+        auto run = [&](auto tiles) {
+            constexpr int LIVE = decltype(tiles)::value, NS = LIVE > 1 ? 2 : 1;
+            for (int j = 0; j < nsb; j++) {
+                const int kb = kb0 + j, slot = j & 1;
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                issue_w(kb, 1);
+                request(j + 1);
+                const uint8_t *const Dj = lds + LD::D8_OFF + slot * LD::D8 + 4 * nr;
+                auto d8_of = [&](int b, float (&d)[LIVE]) {
 #pragma unroll
-                for (int t = 0; t < MI; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
-            };
-            // The sums of block b + 1 are on their way in the matrix cores while those of block b are scaled, tile by tile.
-            i32x4 op;
-            i32x16 S[MI];
-            float d8[MI];
-            operand(0, op);
-            d8_of(0, d8);
+                    for (int t = 0; t < LIVE; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
+                };
+                // The sums of the next tile, or of the first one of the next block, are on their way in the matrix cores while those of a tile are scaled; its fragment was asked for
+                // another tile before.
+                i32x4 op, af;
+                i32x16 S[NS];
+                float d8[LIVE];
+                auto ahead = [&](int u) { if (u < 8 * LIVE) af = a_frag(slot, u / LIVE, u % LIVE); };
+                operand(0, op);
+                d8_of(0, d8);
+                ahead(0);
+                S[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, af, magic, 0, 0, 0);
+                ahead(1);
 #pragma unroll
-            for (int t = 0; t < MI; t++)
-                if (t < live) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, a_frag(slot, 0, t), magic, 0, 0, 0);
+                for (int b = 0; b < 8; b++) {
+                    // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
+                    if (b == 3) {
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
+                        row_scales(1);
+                    }
+                    if (b == 4) issue_w(kb + 1, 0);
+                    if (b == 7) {                              // the next super-block's first half
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                        row_scales(0);
+                    }
+                    f32x4 c[4], dw_n[4];
 #pragma unroll
-            for (int b = 0; b < 8; b++) {
-                // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
-                if (b == 3) {
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + ND) : "memory");
-                    row_scales(1);
+                    for (int e4 = 0; e4 < 4; e4++) c[e4] = -12582912.0f * dw[e4];
+                    scales_of(b == 7 ? 0 : b + 1, dw_n);
+                    i32x4 op_n;
+                    float d8_n[LIVE];
+                    if (b < 7) {
+                        operand(b + 1, op_n);
+                        d8_of(b + 1, d8_n);
+                    }
+#pragma unroll
+                    for (int t = 0; t < LIVE; t++) {
+                        const int u = b * LIVE + t;
+                        auto next = [&]() {
+                            if (u + 1 < 8 * LIVE) S[(u + 1) % NS] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t + 1 < LIVE ? op : op_n, af, magic, 0, 0, 0);
+                            ahead(u + 2);
+                        };
+                        if (NS > 1) next();
+#pragma unroll
+                        for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[u % NS][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
+                        qt_pin(acc[t]);
+                        if (NS == 1) next();
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    op = op_n;
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; e4++) dw[e4] = dw_n[e4];
+#pragma unroll
+                    for (int t = 0; t < LIVE; t++) d8[t] = d8_n[t];
                 }
-                if (b == 4) issue_w(kb + 1, 0);
-                if (b == 7) {                                  // the next super-block's first half
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    row_scales(0);
+            }
+        };
+        if (live == MI) run(std::integral_constant<int, MI>{});
+        else if constexpr (MI > 1) {
+            if (live == 1) run(std::integral_constant<int, 1>{});
+            else if constexpr (MI > 2) {
+                if (live == 2) run(std::integral_constant<int, 2>{});
+                else if constexpr (MI > 3) {
+                    if (live == 3) run(std::integral_constant<int, 3>{});
+                    else if constexpr (MI > 4) run(std::integral_constant<int, 4>{});
                 }
-                f32x4 c[4], dw_n[4];
-#pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) c[e4] = -12582912.0f * dw[e4];
-                scales_of(b == 7 ? 0 : b + 1, dw_n);
-                i32x4 op_n;
-                float d8_n[MI];
-                if (b < 7) {
-                    operand(b + 1, op_n);
-                    d8_of(b + 1, d8_n);
-                }
-#pragma unroll
-                for (int t = 0; t < MI; t++) {
-                    if (t >= live) break;
-                    i32x4 af;
-                    if (b < 7) af = a_frag(slot, b + 1, t);
-#pragma unroll
-                    for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[t][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
-                    qt_pin(acc[t]);
-                    if (b < 7) S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op_n, af, magic, 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                op = op_n;
-#pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) dw[e4] = dw_n[e4];
-#pragma unroll
-                for (int t = 0; t < MI; t++) d8[t] = d8_n[t];
             }
         }
     }
@@ -392,7 +419,9 @@ static int launch_mi(int mi, bool moe, dim3 grid, const void *w, const ActView &
     switch (mi) {
         case 2: Q0_GO(2, false, true);
         case 3: Q0_GO(3, false, true);
-        default: Q0_GO(4, false, true);
+        case 4: Q0_GO(4, false, true);
+        case 5: if constexpr (DT == CQ_Q4_0) Q0_GO(5, false, true);
+        default: return CQ_ERR_RANGE;
     }
 #undef Q0_GO
 }

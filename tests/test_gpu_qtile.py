@@ -146,6 +146,13 @@ def test_silu_of_a_pair(fmt, gap, m, n, k):
     assert torch.equal(y[1:m + 1], want[:, :n])
 
 
+@pytest.mark.parametrize("out", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(129, 5632, 2048), (150, 5633, 2304), (290, 3585, 4096), (300, 7681, 2048), (449, 4609, 2048)])
+def test_tiles_of_160_rows(m, n, k, out):
+    """Q4_0 in tiles of five parts of 32 rows, the last one with one to five of them; ragged columns, K split and not."""
+    check("q4_0", m, n, k, out)
+
+
 @pytest.mark.parametrize("fmt", FMT)
 @pytest.mark.parametrize("out", [1, 30])
 @pytest.mark.parametrize("n,k", [(130, 512), (260, 4096)])
