@@ -1190,7 +1190,7 @@ static int qme_launch(QmeArgs &a, int w_dtype, int64_t num_experts, int tensors,
 // scaling the results)
 bool cq_matvec_batch_mid_takes(int w_dtype, const void *w, const void *x, int x_dtype, int dst_dtype, int64_t k, int64_t n, int64_t rows) {
     return qb_weights(w_dtype) && x_dtype == CQ_F32 && dst_dtype == CQ_F32 && rows > 16 && rows <= 64 &&
-           cq_moe_stream_takes(w_dtype, w, nullptr, 1, rows, k, n) && ((uintptr_t)x & 15) == 0;
+           qme_shape(w_dtype, 1, rows, k, n, 64) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0;
 }
 int64_t cq_matvec_batch_mid_workspace(int w_dtype, int64_t k, int64_t rows) {
     return qb_weights(w_dtype) && rows > 16 && rows <= 64 && k % 256 == 0 && k / 256 <= 2 * QB_NW ? cq_align256(((rows + 15) / 16) * (k / 256) * QME_TILE_COL_BYTES) : 0;

@@ -147,6 +147,17 @@ def test_q4k_rows_in_sets_of_16_vs_oracle(wdt, k, n, rows):
         assert rel_l2(got[r], want[r]) <= TIGHT, r
 
 
+@pytest.mark.parametrize("wdt", [oracle.Q4K, oracle.Q5K], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("k", [1024, 4096])
+def test_q4k_rows_in_sets_of_16_do_not_depend_on_their_number(wdt, k):
+    """17 .. 64 rows take one form, whose results of a row are the same bits whichever rows are beside it (the limit of pairs an expert is another one)."""
+    blocks, qmm = make_weight(wdt, 300, k, seed=183)
+    x = normal(184, (64, k), 1.0)
+    few = forward(qmm, x[:17])
+    for rows in (27, 28, 40, 64):
+        assert np.array_equal(forward(qmm, x[:rows])[:17], few), rows
+
+
 def test_cfg1_q8_0_4096x4096():
     # BASELINE configs[0]: Q8_0 weight [4096 x 4096], activation 1 x 4096
     blocks, qmm = make_weight(oracle.Q8_0, 4096, 4096, seed=1)
