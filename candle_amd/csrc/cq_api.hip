@@ -312,8 +312,33 @@ int cq_nn_qmatmul_swiglu_pair(int w_dtype, const void *w1_dev, const void *w3_de
     hipStream_t s = (hipStream_t)stream;
     const int64_t act = cq_act_layout(w_dtype, k, m).total, room = std::min(workspace_bytes, cq_qmatmul_workspace_bytes(w_dtype, m, k, 2 * n)) - act;
     if (!cq_qtile_takes_swiglu(w_dtype, w1_dev, w3_dev, k, n, m, room)) return CQ_ERR_RANGE;
-    if ((rc = cq_quantize_act_launch(w_dtype, x_dev, CQ_F32, workspace_dev, k, m, s))) return rc;
+    if ((const void *)x_dev != workspace_dev && (rc = cq_quantize_act_launch(w_dtype, x_dev, CQ_F32, workspace_dev, k, m, s))) return rc;
     return cq_qtile_swiglu_launch(w_dtype, w1_dev, w3_dev, cq_act_view(workspace_dev, w_dtype, k, m), dst_dev, k, n, m, room, s);
+}
+
+int cq_nn_rms_norm_quantized(int w_dtype, const float *x_dev, const float *delta_dev, const float *weight_dev, float *sum_out_dev, int64_t rows, int64_t dim, float eps,
+                             void *workspace_dev, int64_t workspace_bytes, void *stream) {
+    if (!cq_is_kquant(w_dtype)) return CQ_ERR_DTYPE;
+    if (rows < 0 || dim <= 0 || dim % 256) return CQ_ERR_SHAPE;
+    if (rows == 0) return CQ_OK;
+    if (!x_dev || !weight_dev || !workspace_dev) return CQ_ERR_NULL;
+    if (!aligned(x_dev, 16) || !aligned(delta_dev, 16) || !aligned(weight_dev, 16) || !aligned(sum_out_dev, 16) || !aligned(workspace_dev, 256)) return CQ_ERR_ALIGN;
+    if (workspace_bytes < cq_act_layout(w_dtype, dim, rows).total) return CQ_ERR_WORKSPACE;
+    return cq_quantize_norm_launch(x_dev, delta_dev, weight_dev, sum_out_dev, workspace_dev, dim, rows, eps, (hipStream_t)stream);
+}
+
+int cq_qmatmul_quantized(int w_dtype, const void *w_dev, void *dst_dev, int dst_dtype, int64_t m, int64_t k, int64_t n, void *workspace_dev, int64_t workspace_bytes,
+                         void *stream) {
+    int rc = check_mm_shape(w_dtype, k, n, m);
+    if (rc) return rc;
+    if (!float_dtype(dst_dtype) || !cq_is_kquant(w_dtype)) return CQ_ERR_DTYPE;
+    if (m == 0 || n == 0) return CQ_OK;
+    if ((rc = check_weight_ptr(w_dtype, w_dev))) return rc;
+    if (!dst_dev || !workspace_dev) return CQ_ERR_NULL;
+    if (!aligned(workspace_dev, 256) || !aligned(dst_dev, float_size(dst_dtype))) return CQ_ERR_ALIGN;
+    if (workspace_bytes < workspace_least(w_dtype, m, k, n)) return CQ_ERR_WORKSPACE;
+    if (m <= 64 || !cq_use_mfma(w_dtype, m, k)) return CQ_ERR_RANGE;                 // (such calls of cq_qmatmul_forward quantize in another layout, or within their kernel)
+    return forward_quantized(w_dtype, w_dev, dst_dev, dst_dtype, m, k, n, workspace_dev, workspace_bytes, (hipStream_t)stream);
 }
 
 int64_t cq_indexed_moe_workspace_bytes(int w_dtype, int64_t num_experts, int64_t n, int64_t k, int64_t batch, int64_t topk,

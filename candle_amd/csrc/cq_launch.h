@@ -5,6 +5,7 @@
 
 int cq_dequantize_launch(int dtype, const void *blocks, void *out, int64_t elems, int out_dtype, hipStream_t s);
 int cq_quantize_launch(int dtype, const float *x, void *blocks, int64_t elems, hipStream_t s);
+int cq_quantize_norm_launch(const float *x, const float *delta, const float *w, float *sum_out, void *scratch, int64_t dim, int64_t rows, float eps, hipStream_t s);
 int cq_quantize_act_launch(int w_dtype, const void *x, int x_dtype, void *scratch, int64_t k, int64_t rows, hipStream_t s);
 int cq_quantize_act_swiglu_launch(int w_dtype, const float *gate, const float *up, int64_t gate_stride, int64_t up_stride, void *scratch, int64_t k,
                                   int64_t rows, hipStream_t s);

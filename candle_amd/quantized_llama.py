@@ -56,6 +56,7 @@ def precomput_freqs_cis(head_dim: int, freq_base: float, max_seq_len: int):
 
 
 # tensor order inside one layer's slab: pairs that can be fused are adjacent
+_K_FORMATS = (GgmlDType.Q2K, GgmlDType.Q3K, GgmlDType.Q4K, GgmlDType.Q5K, GgmlDType.Q6K)      # (their rows are quantized alike)
 _LAYER_ORDER = ("attention_wq", "attention_wk", "attention_wv", "attention_wo", "feed_forward_w1", "feed_forward_w3", "feed_forward_w2")
 
 
@@ -329,6 +330,23 @@ class ModelWeights(GreedyDecoder):
         _lib.check("cq_qmatmul_forward", L.cq_qmatmul_forward(int(w.dtype), w.ptr, src.data_ptr(), 0, dst_ptr, 0, rows, w.k, n,
                                                               self.ws.data_ptr(), self.ws.numel(), sp))
 
+    def _product(self, w: _W, n: int, src: Optional[torch.Tensor], dst_ptr: int, rows: int, sp):
+        """_mm, or (src None) the product over the rows that the workspace holds quantized."""
+        if src is not None:
+            return self._mm(w, n, src, dst_ptr, rows, sp)
+        _lib.check("cq_qmatmul_quantized", self.L.cq_qmatmul_quantized(int(w.dtype), w.ptr, dst_ptr, 0, rows, w.k, n, self.ws.data_ptr(), self.ws.numel(), sp))
+
+    def _norm_rows(self, readers: Sequence[_W], add: bool, norm_w: torch.Tensor, rows: int, sp) -> Optional[torch.Tensor]:
+        """x (+= delta) and its norm: f32 rows for `readers`, or None where all of them take the quantized form of a prompt's rows, which then lies in the workspace."""
+        cfg, x, delta = self.cfg, self.x.data_ptr(), self.delta.data_ptr() if add else None
+        into = self.x.data_ptr() if add else None
+        if rows > 64 and self.tap is None and cfg.hidden % 256 == 0 and cfg.hidden <= 8192 and all(w.dtype in _K_FORMATS for w in readers):
+            _lib.check("cq_nn_rms_norm_quantized", self.L.cq_nn_rms_norm_quantized(int(readers[0].dtype), x, delta, norm_w.data_ptr(), into, rows, cfg.hidden, cfg.rms_eps,
+                                                                                  self.ws.data_ptr(), self.ws.numel(), sp))
+            return None
+        _lib.check("cq_nn_rms_norm", self.L.cq_nn_rms_norm(x, delta, norm_w.data_ptr(), into, self.xn.data_ptr(), rows, cfg.hidden, cfg.rms_eps, sp))
+        return self.xn
+
     def _enqueue(self, ids_ptr: Optional[int], rows: int, pos: int, pos_dev_ptr: Optional[int], max_kv_len: int, sp) -> None:
         """All kernels of ModelWeights::forward (quantized_llama.rs:568-596) for `rows` new tokens; logits of the last.
         ids_ptr None (fused single-token step only): the token's embedding row and its partial sums of squares are already in
@@ -347,20 +365,19 @@ class ModelWeights(GreedyDecoder):
         tap("embedding", -1)
         for li, lw in enumerate(self.layers):
             w = lw.w
-            # x (+= mlp output of the previous layer); xn = attention_norm(x)          :579-583, :590-592
-            ck("cq_nn_rms_norm", L.cq_nn_rms_norm(x.data_ptr(), delta.data_ptr() if li else None, lw.attention_norm.data_ptr(),
-                                                 x.data_ptr() if li else None, xn.data_ptr(), rows, cfg.hidden, cfg.rms_eps, sp))
+            # x (+= mlp output of the previous layer); attention_norm(x)               :579-583, :590-592
+            wq, wk, wv = w["attention_wq"], w["attention_wk"], w["attention_wv"]
+            normed = self._norm_rows((wq, wk, wv), li > 0, lw.attention_norm, rows, sp)
             tap("attention_norm", li)
             # q, k, v projections                                                         :200-202
-            wq, wk, wv = w["attention_wq"], w["attention_wk"], w["attention_wv"]
             if wq.dtype == wk.dtype and wk.ptr == wq.ptr + wq.nbytes:
-                self._mm(wq, qd + kvd, xn, qk.data_ptr(), rows, sp)
+                self._product(wq, qd + kvd, normed, qk.data_ptr(), rows, sp)
                 q_ptr, k_ptr, qs, ks = qk.data_ptr(), qk.data_ptr() + 4 * qd, qd + kvd, qd + kvd
             else:
-                self._mm(wq, qd, xn, qk.data_ptr(), rows, sp)
-                self._mm(wk, kvd, xn, qk.data_ptr() + 4 * rows * qd, rows, sp)
+                self._product(wq, qd, normed, qk.data_ptr(), rows, sp)
+                self._product(wk, kvd, normed, qk.data_ptr() + 4 * rows * qd, rows, sp)
                 q_ptr, k_ptr, qs, ks = qk.data_ptr(), qk.data_ptr() + 4 * rows * qd, qd, kvd
-            self._mm(wv, kvd, xn, v.data_ptr(), rows, sp)
+            self._product(wv, kvd, normed, v.data_ptr(), rows, sp)
             tap("qkv", li)
             # rope on q and k, append k and v to the cache                                :217-233
             ck("cq_nn_rope_i_kv", L.cq_nn_rope_i_kv(q_ptr, k_ptr, v.data_ptr(), lw.k_cache.data_ptr(), lw.v_cache.data_ptr(),
@@ -374,26 +391,25 @@ class ModelWeights(GreedyDecoder):
             tap("attention", li)
             self._mm(w["attention_wo"], cfg.hidden, att, delta.data_ptr(), rows, sp)    # :264
             tap("attention_wo", li)
-            # x += attn; xn = ffn_norm(x)                                                 :584-589
-            ck("cq_nn_rms_norm", L.cq_nn_rms_norm(x.data_ptr(), delta.data_ptr(), lw.ffn_norm.data_ptr(), x.data_ptr(), xn.data_ptr(), rows,
-                                                 cfg.hidden, cfg.rms_eps, sp))
+            # x += attn; ffn_norm(x)                                                      :584-589
+            w1, w3, w2 = w["feed_forward_w1"], w["feed_forward_w3"], w["feed_forward_w2"]
+            normed = self._norm_rows((w1, w3), True, lw.ffn_norm, rows, sp)
             tap("ffn_norm", li)
             # w2(silu(w1 x) * w3 x)                                                       :56-63
-            w1, w3, w2 = w["feed_forward_w1"], w["feed_forward_w3"], w["feed_forward_w2"]
             if rows > 64 and self.tap is None and w1.dtype == w3.dtype:
                 # prompts: silu(w1 x) * w3 x in one launch (-6, CQ_ERR_RANGE: not a shape of it)
-                rc = L.cq_nn_qmatmul_swiglu_pair(int(w1.dtype), w1.ptr, w3.ptr, xn.data_ptr(), h.data_ptr(), rows, w1.k, cfg.ffn, self.ws.data_ptr(),
-                                                 self.ws.numel(), sp)
+                src = self.ws if normed is None else normed           # (the workspace itself: the rows that it holds quantized)
+                rc = L.cq_nn_qmatmul_swiglu_pair(int(w1.dtype), w1.ptr, w3.ptr, src.data_ptr(), h.data_ptr(), rows, w1.k, cfg.ffn, self.ws.data_ptr(), self.ws.numel(), sp)
                 if rc != -6:
                     ck("cq_nn_qmatmul_swiglu_pair", rc)
                     self._mm(w2, cfg.hidden, h, delta.data_ptr(), rows, sp)
                     continue
             if w1.dtype == w3.dtype and w3.ptr == w1.ptr + w1.nbytes:
-                self._mm(w1, 2 * cfg.ffn, xn, gu.data_ptr(), rows, sp)
+                self._product(w1, 2 * cfg.ffn, normed, gu.data_ptr(), rows, sp)
                 g_ptr, u_ptr, gs = gu.data_ptr(), gu.data_ptr() + 4 * cfg.ffn, 2 * cfg.ffn
             else:
-                self._mm(w1, cfg.ffn, xn, gu.data_ptr(), rows, sp)
-                self._mm(w3, cfg.ffn, xn, gu.data_ptr() + 4 * rows * cfg.ffn, rows, sp)
+                self._product(w1, cfg.ffn, normed, gu.data_ptr(), rows, sp)
+                self._product(w3, cfg.ffn, normed, gu.data_ptr() + 4 * rows * cfg.ffn, rows, sp)
                 g_ptr, u_ptr, gs = gu.data_ptr(), gu.data_ptr() + 4 * rows * cfg.ffn, cfg.ffn
             tap("w13", li)
             if rows > 2 and cfg.ffn % 256 == 0:

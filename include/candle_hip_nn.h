@@ -113,6 +113,16 @@ int cq_nn_qmatmul_swiglu_rows(int w_dtype, const void *w_dev, const float *gate_
 int cq_nn_qmatmul_swiglu_pair(int w_dtype, const void *w1_dev, const void *w3_dev, const float *x_dev, float *dst_dev, int64_t m, int64_t k, int64_t n,
                               void *workspace_dev, int64_t workspace_bytes, void *stream);
 
+/* What several products over the same normed rows share, for prompts of K formats (more than 64 rows): cq_nn_rms_norm whose rows go to the front of the workspace in the form that
+ * cq_qmatmul_forward makes of them (sum_out, which may be x, gets x + delta; the normed f32 rows are not written), and the product over the rows that lie there: the
+ * values of cq_qmatmul_forward, which quantizes them anew.  cq_nn_qmatmul_swiglu_pair takes them where its x_dev is the workspace itself.  One workspace, of at least what each of
+ * those calls asks for; every K format reads the same rows.  dim: a multiple of 256 up to 8192 (CQ_ERR_RANGE beyond).  CQ_ERR_DTYPE: other formats; CQ_ERR_RANGE of the product:
+ * up to 64 rows. */
+int cq_nn_rms_norm_quantized(int w_dtype, const float *x_dev, const float *delta_dev, const float *weight_dev, float *sum_out_dev, int64_t rows, int64_t dim, float eps,
+                             void *workspace_dev, int64_t workspace_bytes, void *stream);
+int cq_qmatmul_quantized(int w_dtype, const void *w_dev, void *dst_dev, int dst_dtype, int64_t m, int64_t k, int64_t n, void *workspace_dev, int64_t workspace_bytes,
+                         void *stream);
+
 /* Single-row (decode) fusions of the glue into the quantized matvec kernel.  No counterpart in the reference,
  * which runs these as separate tensor ops; results equal the unfused sequence up to f32 summation order.
  *

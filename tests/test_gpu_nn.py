@@ -52,6 +52,42 @@ def test_embedding_rows_and_out_of_range():
     assert np.all(got[4:] == 0.0)
 
 
+@pytest.mark.parametrize("dim,rows", [(256, 1), (512, 67), (4096, 65), (4352, 70), (5120, 3), (8192, 66)])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_rms_norm_quantized(dim, rows, with_delta):
+    """The quantized rows, and x + delta, that cq_nn_rms_norm and cq_quantize_act give, bit for bit; and the products over them those of cq_qmatmul_forward over the normed rows."""
+    import oracle
+    lib = L()
+    x, d, w = normal(2, (rows, dim), 1.0), normal(3, (rows, dim), 0.5), normal(4, (dim,), 1.0)
+    x[rows - 1, 7] = 300.0
+    xs, ds, ws = dev(x), dev(d), dev(w)
+    normed, sums = torch.empty((rows, dim), device="cuda"), torch.empty((rows, dim), device="cuda")
+    delta = ds.data_ptr() if with_delta else None
+    ok(lib.cq_nn_rms_norm(xs.data_ptr(), delta, ws.data_ptr(), sums.data_ptr(), normed.data_ptr(), rows, dim, 1e-5, None))
+    nb = lib.cq_act_scratch_bytes(12, dim, rows)
+    want, got = (torch.full((nb + 256,), 173, dtype=torch.uint8, device="cuda") for _ in range(2))
+    ok(lib.cq_quantize_act(12, normed.data_ptr(), 0, want.data_ptr(), dim, rows, None))
+    ok(lib.cq_nn_rms_norm_quantized(12, xs.data_ptr(), delta, ws.data_ptr(), xs.data_ptr(), rows, dim, 1e-5, got.data_ptr(), nb, None))
+    assert torch.equal(got, want) and torch.equal(xs, sums)
+    assert lib.cq_nn_rms_norm_quantized(12, xs.data_ptr(), delta, ws.data_ptr(), None, rows, dim, 1e-5, got.data_ptr(), nb - 1, None) == -5
+    assert lib.cq_nn_rms_norm_quantized(8, xs.data_ptr(), delta, ws.data_ptr(), None, rows, dim, 1e-5, got.data_ptr(), nb, None) == -1
+    assert lib.cq_nn_rms_norm_quantized(12, xs.data_ptr(), delta, ws.data_ptr(), None, rows, dim - 128, 1e-5, got.data_ptr(), nb, None) == -2
+    assert lib.cq_nn_rms_norm_quantized(12, xs.data_ptr(), delta, ws.data_ptr(), None, 1, 8448, 1e-5, got.data_ptr(), 1 << 40, None) == -6
+    for code, n in ((12, 130), (13, 257), (14, 256), (14, 131)):
+        blocks = dev(oracle.from_float(code, normal(5, (n * dim,), 0.02)))
+        full = lib.cq_qmatmul_workspace_bytes(code, rows, dim, n)
+        room = torch.empty(full, dtype=torch.uint8, device="cuda")
+        a, b = torch.empty((rows, n), device="cuda"), torch.full((rows, n), 7.0, device="cuda")
+        ok(lib.cq_qmatmul_forward(code, blocks.data_ptr(), normed.data_ptr(), 0, a.data_ptr(), 0, rows, dim, n, room.data_ptr(), full, None))
+        room[:nb] = want[:nb]
+        rc = lib.cq_qmatmul_quantized(code, blocks.data_ptr(), b.data_ptr(), 0, rows, dim, n, room.data_ptr(), full, None)
+        if rows <= 64:
+            assert rc == -6 and bool((b == 7).all())
+        else:
+            ok(rc)
+            assert torch.equal(a, b) and torch.equal(room[:nb], want[:nb])      # (the rows are still there for the next product)
+
+
 @pytest.mark.parametrize("dim", [64, 256, 4096, 5120, 14336])
 @pytest.mark.parametrize("with_delta", [False, True])
 def test_rms_norm(dim, with_delta):
