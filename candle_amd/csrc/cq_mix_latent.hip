@@ -83,6 +83,15 @@ __device__ __forceinline__ float group_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
+// over aligned groups of four lanes, in every lane
+__device__ __forceinline__ float quad_sum(float v) {
+#define CQ_ADD(ctrl) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true))
+    CQ_ADD(CQ_DPP_QUAD_XOR1);
+    CQ_ADD(CQ_DPP_QUAD_XOR2);
+#undef CQ_ADD
+    return v;
+}
+
 // ---- expanded: causal attention head by head ---------------------------------------------------------------------------------------------
 // Workgroup: four waves of 16 NQ query rows of one head; tiles of keys through LDS, the next one on its way in registers.  Scores come out
 // transposed (key x query), so a lane holds one query's keys and its weights are the operand of the value product as they are; the outputs
@@ -617,6 +626,221 @@ __global__ __launch_bounds__(256) void latent_absorb_step_kernel(cq_latent g, co
         for (int i = threadIdx.x; i < g.rot_pad; i += 256) d[g.rank_pad + i] = i < g.rot_dim ? (T)(query_factor(g) * turned<T>(g, s + g.dim, p, i)) : (T)0.0f;
 }
 
+// One token over few keys: workgroup (head, tile of keys) takes W_uk to the query itself and attends to its tile; the record goes to latent_merge_step_kernel.  Every tile of a head reads
+// W_uk of it again (128 KB of 512 x 128; the tiles of a head run on one XCD and share its L2), which is what bounds it: with its keys a unit takes 200 KB at 43 bytes a ns, whether they come
+// from the L2 or not (pulled there by the launch before: no difference).  Three launches before, of 4.6 + 6.6 + 5.0 us, now 9.3 + 4.9 (16 heads, 150 keys; with W_uk on the vector units 0.9 more).
+// The workgroups whose tile holds the token's own position work its cache row out for themselves; those of head 0 store it.
+struct Attend {
+    const float *row;
+    const uint16_t *w_ukt;
+    float *part;
+    const int32_t *pos_dev;
+    int64_t kv_off;
+    int ldw, pos, tiles;
+};
+template <typename T>
+__global__ __launch_bounds__(512) void latent_attend_step_kernel(cq_latent g, Attend in, T *cache) {
+    constexpr int CH = Chunk<T>::N, KT = Chunk<T>::KEYS, LPK = 512 / KT, MAX_LD = CQ_LATENT_MAX_RANK + 64, NP = MAX_LD / (LPK * CH), NG = CQ_LATENT_MAX_RANK / CH, PARTS = 512 / NG;
+    static_assert(KT == 8 * PARTS && NP * LPK * CH == MAX_LD, "eight keys a group of threads");
+    extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+    __shared__ __attribute__((aligned(16))) float sums[PARTS * CQ_LATENT_MAX_RANK], scores[2][KT];
+    __shared__ __attribute__((aligned(16))) T q[MAX_LD];
+    __shared__ __attribute__((aligned(16))) uint16_t planes[3][128];
+    __shared__ float red[4];
+    T *const tile = reinterpret_cast<T *>(lds);            // [key][row]
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.x, z = blockIdx.y, j0 = z * KT;
+    const int ld = g.rank_pad + g.rot_pad, stride = ld + CH;       // rows in LDS begin four banks apart
+    const float *const row = in.row;
+    const int64_t kv_off = in.kv_off;
+    float *const part = in.part;
+    const int ldw = in.ldw;
+    const int64_t rec = (int64_t)z * g.heads + h;
+    float *const ml = part + (int64_t)in.tiles * g.heads * g.rank_pad + 2 * rec;
+    // (by a vector load: the wait for a scalar one would be in front of the loads of everything else)
+    int zero = 0, p_dev = 0;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+v"(zero));
+#endif
+    if (in.pos_dev) p_dev = in.pos_dev[zero];
+    const int key = tid / LPK, sub = tid % LPK;
+    const T *const krow = cache + (int64_t)min(j0 + key, g.ctx - 1) * ld;
+    // of the token's own row: a thread's share of the latent, twice (for its sum and for its result), and of the rotated parts of key and query
+    const float *const s = row + (int64_t)h * (g.dim + g.rot_dim), *const src = row + max(kv_off, (int64_t)0), fq = query_factor(g);
+    const int at = min(tid, g.rank - 1), turn = min(tid, max(g.rot_dim - 1, 0));
+    float lat = 0.0f, more = 0.0f, norm = 0.0f, kx = 0.0f, ky = 0.0f, qx = 0.0f, qy = 0.0f, cs = 0.0f, sn = 0.0f;
+    if (kv_off >= 0) {
+        lat = src[at];
+        more = src[min(tid + 256, g.rank - 1)];
+        norm = g.norm_dev[at];
+    }
+    if (g.rot_dim) {
+        if (kv_off >= 0) {
+            kx = src[g.rank + turn];
+            ky = src[g.rank + (turn ^ 1)];
+        }
+        qx = s[g.dim + turn];
+        qy = s[g.dim + (turn ^ 1)];
+    }
+    float sv = tid < min(g.dim, 128) ? s[tid] : 0.0f;
+    // W_uk, then the keys: everything is on its way before the first wait
+    const uint16_t *const w = in.w_ukt + (int64_t)h * g.rank * ldw;
+    u32x4 wr[4][4], kr[NP];
+    auto weights = [&](int c0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int r = 16 * (wv + 8 * i), c = c0 + 32 * t + 8 * lk;
+                wr[i][t] = c < ldw && r < g.rank ? *reinterpret_cast<const u32x4 *>(w + (int64_t)min(r + lr, g.rank - 1) * ldw + c) : u32x4{0, 0, 0, 0};
+            }
+    };
+    weights(0);
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int c = (i * LPK + sub) * CH;
+        kr[i] = c < ld ? *reinterpret_cast<const u32x4 *>(krow + c) : u32x4{0, 0, 0, 0};
+    }
+    const int p = in.pos + __builtin_amdgcn_readfirstlane(p_dev);
+    if (p >= g.ctx || j0 > p) {
+        if (p < g.ctx && tid == 0) {
+            ml[0] = -INFINITY;
+            ml[1] = 0.0f;
+        }
+        return;
+    }
+    if (g.rot_dim) {
+        cs = g.cos_dev[(int64_t)p * (g.rot_dim >> 1) + (turn >> 1)];
+        sn = g.sin_dev[(int64_t)p * (g.rot_dim >> 1) + (turn >> 1)];
+    }
+    auto turned_here = [&](float x, float y) { return turn & 1 ? x * cs + y * sn : x * cs - y * sn; };
+    // ---- the query in the latents' space: W_uk on the matrix cores, by the three bfloat16 planes that the query's f32 values are the sum of, a column each ----
+    {
+        f32x4 acc[4] = {};
+        for (int c0 = 0; c0 < g.dim; c0 += 128) {
+            if (c0) __syncthreads();
+            if (tid < 128) {
+                const uint32_t bits = __builtin_bit_cast(uint32_t, sv);
+                const bool finite = (bits & 0x7f800000u) != 0x7f800000u;
+                const float r = sv - __builtin_bit_cast(float, bits & 0xffff0000u);
+                const uint32_t mid = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+                planes[0][tid] = finite ? (uint16_t)(bits >> 16) : f2bf_bits(sv);
+                planes[1][tid] = finite ? (uint16_t)(mid >> 16) : (uint16_t)0;
+                planes[2][tid] = finite ? (uint16_t)(__builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, mid)) >> 16) : (uint16_t)0;
+                sv = c0 + 128 + tid < g.dim ? s[c0 + 128 + tid] : 0.0f;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                    // (the weights may still be on their way)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                u32x4 x = *reinterpret_cast<const u32x4 *>(&planes[min(lr, 2)][32 * t + 8 * lk]);
+                if (lr > 2) x = u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = mma<__bf16>(wr[i][t], x, acc[i]);
+            }
+            if (c0 + 128 < g.dim) weights(c0 + 128);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int j = 16 * (wv + 8 * i) + 4 * lk + e;
+                const float v = quad_sum(acc[i][e]);
+                if (lr == 0 && j < g.rank) q[j] = (T)(fq * v);
+            }
+        if (tid >= g.rank && tid < g.rank_pad) q[tid] = (T)0.0f;
+        if (tid < g.rot_pad) q[g.rank_pad + tid] = tid < g.rot_dim ? (T)(fq * turned_here(qx, qy)) : (T)0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int c = (i * LPK + sub) * CH;
+        if (c < ld) *reinterpret_cast<u32x4 *>(tile + key * stride + c) = j0 + key > p ? u32x4{0, 0, 0, 0} : kr[i];
+    }
+    // ---- the token's own row (append_row's sums) ----
+    const bool own = kv_off >= 0 && p - j0 < KT;
+    if (own && wv < 4) {
+        float t = tid < g.rank ? lat * lat : 0.0f;
+        t = wave_sum(tid + 256 < g.rank ? fmaf(more, more, t) : t);
+        if (lane == 0) red[wv] = t;
+    }
+    __syncthreads();
+    if (own) {
+        const float m = sqrtf((((red[0] + red[1]) + red[2]) + red[3]) / (float)g.rank + g.eps);
+        T *const mine = tile + (p - j0) * stride, *const kept = cache + (int64_t)p * ld;
+        if (tid < g.rank) {
+            const T v = (T)(lat / m * norm);
+            mine[tid] = v;
+            if (h == 0) kept[tid] = v;
+        }
+        if (tid < g.rot_dim) {
+            const T v = (T)turned_here(kx, ky);
+            mine[g.rank_pad + tid] = v;
+            if (h == 0) kept[g.rank_pad + tid] = v;
+        }
+        __syncthreads();
+    }
+    // ---- scores ----
+    auto value = [](const u32x4 &x, int e) {
+        if constexpr (sizeof(T) == 2) return e & 1 ? bf_hi(x[e >> 1]) : bf_lo(x[e >> 1]);
+        else return __builtin_bit_cast(f32x4, x)[e];
+    };
+    if constexpr (sizeof(T) == 2) {                        // a wave: 16 keys, every other step of 32 columns; the query is the first column
+        const int t = wv & 3, half = wv >> 2;
+        f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < MAX_LD / 64; i++) {
+            const int c = 64 * i + 32 * half + 8 * lk;
+            if (64 * i >= ld) break;
+            const u32x4 a = *reinterpret_cast<const u32x4 *>(tile + (16 * t + lr) * stride + min(c, ld - 8));
+            u32x4 x = *reinterpret_cast<const u32x4 *>(q + min(c, ld - 8));
+            if (lr > 0 || c >= ld) x = u32x4{0, 0, 0, 0};
+            d = mma<T>(a, x, d);
+        }
+        if (lr == 0)
+#pragma unroll
+            for (int e = 0; e < 4; e++) scores[half][16 * t + 4 * lk + e] = d[e];
+    } else {                                               // LPK lanes a key
+        float sc[2] = {};
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int c = (i * LPK + sub) * CH;
+            if (c >= ld) continue;
+            const u32x4 x = *reinterpret_cast<const u32x4 *>(tile + key * stride + c);
+#pragma unroll
+            for (int e = 0; e < CH; e++) sc[e & 1] = fmaf(value(x, e), q[c + e], sc[e & 1]);
+        }
+        const float score = row16_sum(sc[0] + sc[1]);
+        if (sub == 0) {
+            scores[0][key] = score;
+            scores[1][key] = 0.0f;
+        }
+    }
+    __syncthreads();
+    // ---- weights of all keys in every wave, values: 8 keys and a chunk of the latent a thread ----
+    const float mine = lane < KT && j0 + lane <= p ? scores[0][lane & (KT - 1)] + scores[1][lane & (KT - 1)] : -INFINITY, mx = wave_max(mine), weight = __builtin_amdgcn_exp2f(mine - mx), total = wave_sum(weight);
+    const int grp = tid % NG, k0 = __builtin_amdgcn_readfirstlane(8 * (tid / NG));
+    const T *const column = tile + k0 * stride + min(grp * CH, g.rank_pad - CH);       // (sums of columns beyond the latent are not stored)
+    float o[CH] = {};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), k0 + i));
+        const u32x4 x = *reinterpret_cast<const u32x4 *>(column + i * stride);
+#pragma unroll
+        for (int e = 0; e < CH; e++) o[e] = fmaf(f, value(x, e), o[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < CH; e += 4) *reinterpret_cast<f32x4 *>(sums + k0 / 8 * CQ_LATENT_MAX_RANK + grp * CH + e) = f32x4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+    __syncthreads();
+    if (tid < g.rank_pad) {
+        float t = sums[tid];
+#pragma unroll
+        for (int i = 1; i < PARTS; i++) t += sums[i * CQ_LATENT_MAX_RANK + tid];
+        part[rec * g.rank_pad + tid] = t;
+    }
+    if (tid == 0) {
+        ml[0] = mx;
+        ml[1] = total;
+    }
+}
+
 // One token: workgroup (head, 16 value rows) merges the records of the head's splits and takes W_uv to the latent.
 __global__ __launch_bounds__(256) void latent_merge_step_kernel(const float *__restrict__ part, int nz, int heads, int rank_pad, const uint16_t *__restrict__ w_uv, int ldw,
                                                                 const float *__restrict__ gate, float *__restrict__ out, int vdim) {
@@ -691,6 +915,23 @@ template <typename T> int absorbed_dispatch(const Absorbed &a, const AbsorbedPla
     if (a.rank_pad <= 256) CQ_AB(256, 64);
     CQ_AB(512, 64);
 #undef CQ_AB
+}
+
+// Tiles of keys of the one launch that does query and attention, 0 where two do.  Up to a workgroup for every unit; beyond that units would read W_uk more than once.  A step's
+// launches, three and now two: 16 heads, rank 512: 15.7 -> 14.4 us (150 keys), 16.0 -> 14.6 (1024, 256 workgroups); f32 17.9 -> 13.9 (150), 18.1 -> 14.2 (512); 8 heads 14.8 -> 14.6;
+// rank 256 with 64 dimensions 12.5 -> 10.9.
+int attend_tiles(const cq_latent &g) {
+    const int kt = g.bf16 ? 64 : 32;
+    const int64_t tiles = ((int64_t)g.ctx + kt - 1) / kt;
+    return g.heads * tiles <= 256 ? (int)tiles : 0;
+}
+template <typename T> int attend_step_launch(const cq_latent &g, const Attend &a, void *cache, hipStream_t s) {
+    const size_t lds = (size_t)Chunk<T>::KEYS * ((g.rank_pad + g.rot_pad) * sizeof(T) + 16);
+    constexpr int MOST = Chunk<T>::KEYS * ((CQ_LATENT_MAX_RANK + 64) * (int)sizeof(T) + 16);
+    const int e = (int)hipFuncSetAttribute(reinterpret_cast<const void *>(latent_attend_step_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize, MOST);
+    if (e) return e;
+    hipLaunchKernelGGL(latent_attend_step_kernel<T>, dim3((unsigned)g.heads, (unsigned)a.tiles), dim3(512), lds, s, g, a, (T *)cache);
+    return (int)hipGetLastError();
 }
 
 template <typename T, int DK, int DV, int NQ> int expanded_launch(const Expanded &a, hipStream_t s) {
@@ -823,26 +1064,32 @@ int cq_mix_latent_step(const cq_latent *g, const float *row_dev, int64_t kv_off,
     const AbsorbedPlan plan = absorbed_plan(g->bf16, g->heads, g->ctx);
     const int nz = plan.splits;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)(g->heads * ((g->rank + 63) / 64) + 1));
-    if (g->bf16)
-        hipLaunchKernelGGL(latent_absorb_step_kernel<__bf16>, grid, dim3(256), 0, s, *g, row_dev, kv_off, (__bf16 *)cache_dev, (const uint16_t *)w_ukt_dev, (int)ld_ukt,
-                           (__bf16 *)q_dev, pos_dev, (int)pos);
-    else
-        hipLaunchKernelGGL(latent_absorb_step_kernel<float>, grid, dim3(256), 0, s, *g, row_dev, kv_off, (float *)cache_dev, (const uint16_t *)w_ukt_dev, (int)ld_ukt,
-                           (float *)q_dev, pos_dev, (int)pos);
-    Absorbed a = {};
-    a.q = q_dev;
-    a.cache = cache_dev;
-    a.ld = g->rank_pad + g->rot_pad;
-    a.rank_pad = g->rank_pad;
-    a.heads = g->heads;
-    a.rows = 1;
-    a.pos = (int)pos;
-    a.ctx = g->ctx;
-    a.pos_dev = pos_dev;
-    a.part = (float *)workspace_dev;
-    const int r = g->bf16 ? absorbed_dispatch<__bf16>(a, plan, s) : absorbed_dispatch<float>(a, plan, s);
-    if (r) return r;
+    if (attend_tiles(*g) == nz) {
+        const Attend a = {row_dev, (const uint16_t *)w_ukt_dev, (float *)workspace_dev, pos_dev, kv_off, (int)ld_ukt, (int)pos, nz};
+        const int r = g->bf16 ? attend_step_launch<__bf16>(*g, a, cache_dev, s) : attend_step_launch<float>(*g, a, cache_dev, s);
+        if (r) return r;
+    } else {
+        const dim3 grid((unsigned)(g->heads * ((g->rank + 63) / 64) + 1));
+        if (g->bf16)
+            hipLaunchKernelGGL(latent_absorb_step_kernel<__bf16>, grid, dim3(256), 0, s, *g, row_dev, kv_off, (__bf16 *)cache_dev, (const uint16_t *)w_ukt_dev, (int)ld_ukt,
+                               (__bf16 *)q_dev, pos_dev, (int)pos);
+        else
+            hipLaunchKernelGGL(latent_absorb_step_kernel<float>, grid, dim3(256), 0, s, *g, row_dev, kv_off, (float *)cache_dev, (const uint16_t *)w_ukt_dev, (int)ld_ukt,
+                               (float *)q_dev, pos_dev, (int)pos);
+        Absorbed a = {};
+        a.q = q_dev;
+        a.cache = cache_dev;
+        a.ld = g->rank_pad + g->rot_pad;
+        a.rank_pad = g->rank_pad;
+        a.heads = g->heads;
+        a.rows = 1;
+        a.pos = (int)pos;
+        a.ctx = g->ctx;
+        a.pos_dev = pos_dev;
+        a.part = (float *)workspace_dev;
+        const int r = g->bf16 ? absorbed_dispatch<__bf16>(a, plan, s) : absorbed_dispatch<float>(a, plan, s);
+        if (r) return r;
+    }
     hipLaunchKernelGGL(latent_merge_step_kernel, dim3((unsigned)g->heads, (unsigned)((g->vdim + 15) / 16)), dim3(256), 0, s,
                        (const float *)workspace_dev, nz, g->heads, g->rank_pad, (const uint16_t *)w_uv_dev, (int)ld_uv, row_dev + gate_off, out_dev, g->vdim);
     return (int)hipGetLastError();

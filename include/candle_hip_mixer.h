@@ -213,7 +213,7 @@ int cq_mix_latent_expanded(const cq_latent *g, const void *q_dev, int64_t dim_pa
 int64_t cq_mix_latent_absorbed_workspace_bytes(const cq_latent *g, int64_t rows, int64_t pos, int step);
 int cq_mix_latent_absorbed(const cq_latent *g, const void *q_dev, const void *cache_dev, const float *gate_dev, int64_t gate_row, float *out_dev, int64_t pos, int64_t rows,
                            void *workspace_dev, int64_t workspace_bytes, void *stream);
-/* One new token from its projection row to the gated head outputs [heads * vdim], three launches: w_ukt [heads][rank][ld_ukt] (W_uk transposed head by head) and
+/* One new token from its projection row to the gated head outputs [heads * vdim], two launches or three: w_ukt [heads][rank][ld_ukt] (W_uk transposed head by head) and
  * w_uv [heads * vdim][ld_uv] bfloat16, zero beyond dim and rank; gate at row + gate_off; q_dev: scratch of heads * (rank_pad + rot_pad) T, zero-initialized once. */
 int cq_mix_latent_step(const cq_latent *g, const float *row_dev, int64_t kv_off, void *cache_dev, const void *w_ukt_dev, int64_t ld_ukt, const void *w_uv_dev, int64_t ld_uv,
                        int64_t gate_off, void *q_dev, float *out_dev, const int32_t *pos_dev, int64_t pos, void *workspace_dev, int64_t workspace_bytes, void *stream);

@@ -349,6 +349,19 @@ def test_latent_attention_forms_and_portions(H, d, r, e, rank, T, precision, tol
 
 
 @pytest.mark.parametrize("precision,tol", TYPES)
+@pytest.mark.parametrize("H,d,r,e,rank,keys", [(32, 16, 8, 16, 40, 8), (32, 16, 8, 16, 40, 9), (16, 130, 64, 24, 512, 2), (4, 257, 0, 12, 64, 3), (5, 24, 150, 16, 250, 3), (257, 8, 2, 8, 16, 1)])
+def test_single_tokens_of_as_many_heads_and_key_tiles_as_units_and_more(H, d, r, e, rank, keys, precision, tol):
+    """Query and attention in one launch and in two; cache rows have the bits that those of a prompt have."""
+    tile = 64 if precision == mixers.BF16 else 32
+    a = Attention(H, d, r, e, rank, tile * keys - 3, precision)           # (the context has three positions more)
+    want, got = a.want(), a.run([1] * a.T, "step")
+    kept = a.kept[:a.T].clone()
+    assert rel(got, want) < tol
+    a.run([a.T], "absorbed")
+    assert torch.equal(kept, a.kept[:a.T])
+
+
+@pytest.mark.parametrize("precision,tol", TYPES)
 @pytest.mark.parametrize("T", [66, 130, 700])
 def test_one_key_stands_out(T, precision, tol):
     """One position whose score for the last query and whose value stand out, at the first tokens, around the borders of key tiles and splits, at the query
