@@ -66,6 +66,8 @@ SIGNATURES = {
     "cq_nn_moe_route": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "cq_nn_moe_sort": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "cq_nn_moe_sum": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
+    "cq_nn_moe_route_typed": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
+    "cq_nn_moe_sum_typed": (_int, [_vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "cq_nn_rms_norm": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp]),
     "cq_nn_rope_i_kv": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
     "cq_nn_attention_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),

@@ -5,6 +5,7 @@
 // 222-301): router + softmax + top-k, the sort of the pairs by expert, the sum over top-k.  All f32, like the reference's CPU path.  Token ids and the
 // decode position can be read from device memory so that a whole decode step (including "pick the next
 // token, advance the position") can be captured in a HIP graph and replayed without host round trips.
+#include "cq_actquant.h"
 #include "cq_device.h"
 #include "../../include/candle_hip_nn.h"
 
@@ -1379,19 +1380,34 @@ constexpr int ROUTE_MAX_EXPERTS = 1024, ROUTE_MAX_TOPK = 64;
 // 1 MB: walked chunk by chunk with a wait per chunk it took eight dependent memory trips, 5.2 us for one token).
 // <1, 8>: few tokens, one row per wave, a 2048-element row is one trip; <4, 2>: many tokens, the token's row is loaded once
 // per four experts.  Per lane the products are added in the same order in both, so the logits do not depend on the variant.
+// The sums go out in one store, lane i with the i-th (one at a time, 64 of them took as long as a quarter of the products).
 // T: tokens per wave (blockIdx.y is a group of T tokens): with hundreds of tokens the router rows a wave has loaded serve T
-// tokens instead of one (one token per wave re-reads the 1 MB router matrix once per token: 14 us for 256 tokens).  What bounds it there is the L2: <4, 2, 2>
-// asks for 48 KB of a 2048-element row set per eight logits, <8, 1, 8> for 128 KB per 64 (1500 tokens, 128 experts: 45 -> 24 us).  That one needs 1024 waves'
-// worth of logits, 65536 of them, to fill the chip, and of short rows some more (rows of 1024: 76800 logits 14.2 -> 15.1 us, 96000 16.0 -> 15.1).
-template <int R, int C, int T = 1>
-__global__ __launch_bounds__(256) void moe_logits_kernel(const float *__restrict__ x, const float *__restrict__ router_w, float *__restrict__ logits,
-                                                         int hidden, int n_experts, int tokens) {
+// tokens instead of one (one token per wave re-reads the 1 MB router matrix once per token: 14 us for 256 tokens).
+// X: half-precision tokens are read as they are, and the first wave of a group of tokens leaves them in f32 for the launches behind (routing, with the conversion that was a launch of its
+// own: 16 rows or fewer of 2048, 128 experts, 8.4 -> 6.7 us, 200 rows 16.8 -> 14.4, 1500 rows 37.3 -> 29.0).
+template <int T, int R>
+__device__ __forceinline__ void store_logits(const float (&acc)[T][R], float *__restrict__ logits, int t0, int e0, int n_experts, int tokens, int lane) {
+    float mine = 0.0f;
+#pragma unroll
+    for (int j = 0; j < T; j++)
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            const float v = wave_sum(acc[j][i]);
+            mine = lane == j * R + i ? v : mine;
+        }
+    const int j = lane / R, i = lane % R;
+    if (j < T && e0 + i < n_experts && t0 + j < tokens) logits[(int64_t)(t0 + j) * n_experts + e0 + i] = mine;
+}
+template <int R, int C, int T, int X>
+__global__ __launch_bounds__(256) void moe_logits_kernel(const void *__restrict__ x, const float *__restrict__ router_w, float *__restrict__ logits,
+                                                         int hidden, int n_experts, int tokens, float *__restrict__ x_f32) {
     const int t0 = blockIdx.y * T, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int e0 = (blockIdx.x * 4 + wv) * R;
     if (e0 >= n_experts) return;
-    const float *xr[T];
+    const char *xr[T];
 #pragma unroll
-    for (int j = 0; j < T; j++) xr[j] = x + (int64_t)min(t0 + j, tokens - 1) * hidden;
+    for (int j = 0; j < T; j++) xr[j] = (const char *)x + (int64_t)min(t0 + j, tokens - 1) * hidden * (X == CQ_F32 ? 4 : 2);
+    const bool keeps = X != CQ_F32 && e0 == 0;
     const float *w[R];
 #pragma unroll
     for (int i = 0; i < R; i++) w[i] = router_w + (int64_t)min(e0 + i, n_experts - 1) * hidden;
@@ -1406,13 +1422,21 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const float *__restrict
         for (int c = 0; c < C; c++) {
             const int kc = min(k0 + 256 * c, hidden - 4);          // past the end: re-read the last vector, not used below
 #pragma unroll
-            for (int j = 0; j < T; j++) a[j][c] = *reinterpret_cast<const f32x4 *>(xr[j] + kc);
+            for (int j = 0; j < T; j++) {
+                float v[4];
+                cq_load4<X>(xr[j], kc, v);
+                a[j][c] = f32x4{v[0], v[1], v[2], v[3]};
+            }
 #pragma unroll
             for (int i = 0; i < R; i++) b[i][c] = *reinterpret_cast<const f32x4 *>(w[i] + kc);
         }
 #pragma unroll
         for (int c = 0; c < C; c++) {
             if (k0 + 256 * c < hidden) {
+                if (keeps)
+#pragma unroll
+                    for (int j = 0; j < T; j++)
+                        if (t0 + j < tokens) *reinterpret_cast<f32x4 *>(x_f32 + (int64_t)(t0 + j) * hidden + k0 + 256 * c) = a[j][c];
 #pragma unroll
                 for (int j = 0; j < T; j++)
 #pragma unroll
@@ -1425,13 +1449,69 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const float *__restrict
             }
         }
     }
+    store_logits<T, R>(acc, logits, t0, e0, n_experts, tokens, lane);
+}
+
+// The same for thousands of tokens: a wave takes 8 experts of 8 tokens, whose rows the four waves of a workgroup share through LDS, 256 columns at a time, the next ones on their way.
+// Per lane the products are added in the order above: the same logits.  Bound by the vector units (393 M products of 1500 tokens and 128 experts take 10 us at their rate, the sums over lanes
+// 3) and the way from the L2, which one group of columns ahead does not hide where a SIMD has one wave.  Needs 1024 waves' worth of logits, 65536 of them, to fill the chip, and of short rows
+// some more (rows of 1024: 76800 logits 14.2 -> 15.1 us, 96000 16.0 -> 15.1).  Routing of f32 rows, every wave with rows of its own -> this: 1500 of 2048 29.0 -> 27.7 us, 3000 47.4 -> 45.6,
+// 1500 of 1024 19.3 -> 18.7, 520 to 1030 of 2048 19 - 21 -> 19.5 - 21.7.
+template <int X>
+__global__ __launch_bounds__(256, 3) void moe_logits_tile_kernel(const void *__restrict__ x, const float *__restrict__ router_w, float *__restrict__ logits,
+                                                                 int hidden, int n_experts, int tokens, float *__restrict__ x_f32) {
+    constexpr int T = 8, R = 8;
+    __shared__ f32x4 rows[2][T][64];
+    const int t0 = blockIdx.y * T, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), e0 = (blockIdx.x * 4 + wv) * R;
+    const float *w[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) w[i] = router_w + (int64_t)min(e0 + i, n_experts - 1) * hidden;
+    // this thread's share of the tokens: those of its wave's number and of four more
+    const int64_t own[2] = {(int64_t)min(t0 + wv, tokens - 1) * hidden, (int64_t)min(t0 + wv + 4, tokens - 1) * hidden};
+    float acc[T][R], a[2][4];
+    f32x4 cur[R], next[R];
 #pragma unroll
     for (int j = 0; j < T; j++)
 #pragma unroll
-        for (int i = 0; i < R; i++) {
-            const float v = wave_sum(acc[j][i]);
-            if (lane == 0 && e0 + i < n_experts && t0 + j < tokens) logits[(int64_t)(t0 + j) * n_experts + e0 + i] = v;
+        for (int i = 0; i < R; i++) acc[j][i] = 0.0f;
+    auto fetch = [&](int k0) {                             // past the end: the last vector again, not used below
+        const int k = min(k0 + 4 * lane, hidden - 4);
+#pragma unroll
+        for (int j = 0; j < 2; j++) cq_load4<X>(x, own[j] + k, a[j]);
+#pragma unroll
+        for (int i = 0; i < R; i++) next[i] = *reinterpret_cast<const f32x4 *>(w[i] + k);
+    };
+    auto stage = [&](int k0, int slot) {
+        const bool keeps = X != CQ_F32 && (k0 >> 8) % gridDim.x == blockIdx.x && k0 + 4 * lane < hidden;      // (the groups of experts take turns)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const f32x4 v = {a[j][0], a[j][1], a[j][2], a[j][3]};
+            rows[slot][wv + 4 * j][lane] = v;
+            if (keeps && t0 + wv + 4 * j < tokens) *reinterpret_cast<f32x4 *>(x_f32 + own[j] + k0 + 4 * lane) = v;
         }
+#pragma unroll
+        for (int i = 0; i < R; i++) cur[i] = next[i];
+    };
+    fetch(0);
+    stage(0, 0);
+    for (int k0 = 0, slot = 0; k0 < hidden; k0 += 256, slot ^= 1) {
+        if (k0 + 256 < hidden) fetch(k0 + 256);
+        __syncthreads();                                   // the rows are there, and nobody reads the other slot any more
+        if (k0 + 4 * lane < hidden)
+#pragma unroll
+            for (int j = 0; j < T; j++) {
+                const f32x4 v = rows[slot][j][lane];
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    acc[j][i] = fmaf(v.x, cur[i].x, acc[j][i]);
+                    acc[j][i] = fmaf(v.y, cur[i].y, acc[j][i]);
+                    acc[j][i] = fmaf(v.z, cur[i].z, acc[j][i]);
+                    acc[j][i] = fmaf(v.w, cur[i].w, acc[j][i]);
+                }
+            }
+        if (k0 + 256 < hidden) stage(k0 + 256, slot ^ 1);
+    }
+    store_logits<T, R>(acc, logits, t0, e0, n_experts, tokens, lane);
 }
 
 // One workgroup per token: softmax over the experts (:235-236), the topk largest probabilities in descending order
@@ -1561,7 +1641,8 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t *__restri
 }
 
 // ys.reshape((tokens, topk, dim)).sum(-2) (fused_moe.rs:296): the topk rows of a token added in slot order
-__global__ __launch_bounds__(256) void moe_sum_kernel(const float *__restrict__ y, float *__restrict__ out, int topk, int dim) {
+template <int OUT>
+__global__ __launch_bounds__(256) void moe_sum_kernel(const float *__restrict__ y, void *__restrict__ out, int topk, int dim) {
     const int t = blockIdx.y;
     const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (c >= dim) return;
@@ -1571,7 +1652,25 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float *__restrict__ 
         const f32x4 v = *reinterpret_cast<const f32x4 *>(src + (int64_t)j * dim);
         acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
     }
-    *reinterpret_cast<f32x4 *>(out + (int64_t)t * dim + c) = acc;
+    const int64_t at = (int64_t)t * dim + c;
+    if (OUT == CQ_F32) *reinterpret_cast<f32x4 *>((float *)out + at) = acc;
+    else {
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = OUT == CQ_BF16 ? f2bf_bits(acc[e]) : f2h_bits(acc[e]);
+        *reinterpret_cast<u32x2 *>((uint16_t *)out + at) = u32x2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+    }
+}
+
+// Logits of all tokens; which of them a wave takes depends on their number alone.
+template <int X>
+void moe_logits_launch(const void *x, const float *w, float *logits, int hidden, int experts, int tokens, float *x_f32, hipStream_t s) {
+    const int64_t n = (int64_t)tokens * experts;
+    auto grid = [&](int r, int t) { return dim3((unsigned)((experts + 4 * r - 1) / (4 * r)), (unsigned)((tokens + t - 1) / t)); };
+    if (n <= 4096) hipLaunchKernelGGL((moe_logits_kernel<1, 8, 1, X>), grid(1, 1), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
+    else if (n <= 16384) hipLaunchKernelGGL((moe_logits_kernel<4, 2, 1, X>), grid(4, 1), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
+    else if (n < (hidden < 2048 ? 90112 : 65536)) hipLaunchKernelGGL((moe_logits_kernel<4, 2, 2, X>), grid(4, 2), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
+    else hipLaunchKernelGGL(moe_logits_tile_kernel<X>, grid(8, 8), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
 }
 
 inline bool misaligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; }
@@ -1886,25 +1985,23 @@ int cq_nn_argmax_embed(const float *logits_dev, int64_t n, int32_t *token_out_de
 
 int cq_nn_moe_route(const float *x_dev, const float *router_w_dev, uint32_t *topk_ids_dev, float *topk_weights_dev, float *logits_dev,
                     int64_t tokens, int64_t hidden, int64_t num_experts, int64_t topk, int norm_topk_prob, void *stream) {
+    return cq_nn_moe_route_typed(x_dev, CQ_F32, nullptr, router_w_dev, topk_ids_dev, topk_weights_dev, logits_dev, tokens, hidden, num_experts, topk, norm_topk_prob, stream);
+}
+
+int cq_nn_moe_route_typed(const void *x_dev, int x_dtype, float *x_f32_dev, const float *router_w_dev, uint32_t *topk_ids_dev, float *topk_weights_dev, float *logits_dev,
+                          int64_t tokens, int64_t hidden, int64_t num_experts, int64_t topk, int norm_topk_prob, void *stream) {
     if (tokens < 0 || hidden <= 0 || hidden % 4 || num_experts <= 0 || topk <= 0 || topk > num_experts) return CQ_ERR_SHAPE;
+    if (x_dtype != CQ_F32 && x_dtype != CQ_F16 && x_dtype != CQ_BF16) return CQ_ERR_DTYPE;
     if (num_experts > ROUTE_MAX_EXPERTS || topk > ROUTE_MAX_TOPK || tokens > 65535 || hidden > 0x7fffffffLL) return CQ_ERR_RANGE;
     if (tokens == 0) return CQ_OK;
-    if (!x_dev || !router_w_dev || !topk_ids_dev || !topk_weights_dev || !logits_dev) return CQ_ERR_NULL;
-    if (misaligned(x_dev, 16) || misaligned(router_w_dev, 16) || misaligned(topk_ids_dev, 4) || misaligned(topk_weights_dev, 4) ||
-        misaligned(logits_dev, 4))
+    if (!x_dev || !router_w_dev || !topk_ids_dev || !topk_weights_dev || !logits_dev || (x_dtype != CQ_F32 && !x_f32_dev)) return CQ_ERR_NULL;
+    if (misaligned(x_dev, x_dtype == CQ_F32 ? 16 : 8) || misaligned(x_f32_dev, 16) || misaligned(router_w_dev, 16) || misaligned(topk_ids_dev, 4) ||
+        misaligned(topk_weights_dev, 4) || misaligned(logits_dev, 4))
         return CQ_ERR_ALIGN;
-    if (tokens * num_experts <= 4096)
-        hipLaunchKernelGGL((moe_logits_kernel<1, 8>), dim3((unsigned)((num_experts + 3) / 4), (unsigned)tokens), dim3(256), 0, (hipStream_t)stream, x_dev,
-                           router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
-    else if (tokens * num_experts <= 16384)
-        hipLaunchKernelGGL((moe_logits_kernel<4, 2>), dim3((unsigned)((num_experts + 15) / 16), (unsigned)tokens), dim3(256), 0, (hipStream_t)stream, x_dev,
-                           router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
-    else if (tokens * num_experts < (hidden < 2048 ? 90112 : 65536))
-        hipLaunchKernelGGL((moe_logits_kernel<4, 2, 2>), dim3((unsigned)((num_experts + 15) / 16), (unsigned)((tokens + 1) / 2)), dim3(256), 0,
-                           (hipStream_t)stream, x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
-    else
-        hipLaunchKernelGGL((moe_logits_kernel<8, 1, 8>), dim3((unsigned)((num_experts + 31) / 32), (unsigned)((tokens + 7) / 8)), dim3(256), 0,
-                           (hipStream_t)stream, x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens);
+    hipStream_t s = (hipStream_t)stream;
+    if (x_dtype == CQ_F32) moe_logits_launch<CQ_F32>(x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens, nullptr, s);
+    else if (x_dtype == CQ_F16) moe_logits_launch<CQ_F16>(x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens, x_f32_dev, s);
+    else moe_logits_launch<CQ_BF16>(x_dev, router_w_dev, logits_dev, (int)hidden, (int)num_experts, (int)tokens, x_f32_dev, s);
     if (num_experts <= 256)
         hipLaunchKernelGGL(moe_topk_wave_kernel, dim3((unsigned)tokens), dim3(64), 0, (hipStream_t)stream, (const float *)logits_dev, topk_ids_dev,
                            topk_weights_dev, (int)num_experts, (int)topk, norm_topk_prob);
@@ -1927,13 +2024,22 @@ int cq_nn_moe_sort(const uint32_t *topk_ids_dev, int32_t *expert_ids_dev, int32_
 }
 
 int cq_nn_moe_sum(const float *y_dev, float *out_dev, int64_t tokens, int64_t topk, int64_t dim, void *stream) {
+    return cq_nn_moe_sum_typed(y_dev, out_dev, CQ_F32, tokens, topk, dim, stream);
+}
+
+int cq_nn_moe_sum_typed(const float *y_dev, void *out_dev, int out_dtype, int64_t tokens, int64_t topk, int64_t dim, void *stream) {
     if (tokens < 0 || topk <= 0 || dim <= 0 || dim % 4) return CQ_ERR_SHAPE;
+    if (out_dtype != CQ_F32 && out_dtype != CQ_F16 && out_dtype != CQ_BF16) return CQ_ERR_DTYPE;
     if (tokens > 65535 || topk > 0x7fffffffLL || dim > 0x7fffffffLL) return CQ_ERR_RANGE;
     if (tokens == 0) return CQ_OK;
     if (!y_dev || !out_dev) return CQ_ERR_NULL;
-    if (misaligned(y_dev, 16) || misaligned(out_dev, 16)) return CQ_ERR_ALIGN;
-    hipLaunchKernelGGL(moe_sum_kernel, dim3((unsigned)((dim / 4 + 255) / 256), (unsigned)tokens), dim3(256), 0, (hipStream_t)stream, y_dev, out_dev,
-                       (int)topk, (int)dim);
+    if (misaligned(y_dev, 16) || misaligned(out_dev, out_dtype == CQ_F32 ? 16 : 8)) return CQ_ERR_ALIGN;
+    const dim3 grid((unsigned)((dim / 4 + 255) / 256), (unsigned)tokens);
+#define CQ_SUM(T_) hipLaunchKernelGGL(moe_sum_kernel<T_>, grid, dim3(256), 0, (hipStream_t)stream, y_dev, out_dev, (int)topk, (int)dim)
+    if (out_dtype == CQ_F32) CQ_SUM(CQ_F32);
+    else if (out_dtype == CQ_F16) CQ_SUM(CQ_F16);
+    else CQ_SUM(CQ_BF16);
+#undef CQ_SUM
     return (int)hipGetLastError();
 }
 

@@ -14,6 +14,9 @@ import torch
 from . import _lib
 from .quantized import GgmlDType, QTensor
 
+F32 = int(GgmlDType.F32)
+HALF_TYPES = {torch.float16: int(GgmlDType.F16), torch.bfloat16: int(GgmlDType.BF16)}
+
 
 class FusedMoeGGUF:
     """fused_moe.rs:163-175.  gate: router weight f32 [num_experts, hidden] (``ffn_gate_inp``, dequantized at load time
@@ -79,10 +82,14 @@ class FusedMoeGGUF:
             raise ValueError("xs must be on the GPU")
         batch, seq_len, hidden = xs.shape
         original_dtype = xs.dtype
-        x2 = xs.reshape(-1, hidden).to(torch.float32).contiguous()
+        rows = xs.reshape(-1, hidden).contiguous()
+        # half-precision rows go in and out as they are: the router leaves their f32 copy, the sum rounds its results
+        typed = HALF_TYPES.get(original_dtype) if rows.data_ptr() % 8 == 0 else None
+        x2 = torch.empty(rows.shape, dtype=torch.float32, device=xs.device) if typed is not None else rows.to(torch.float32)
         tokens, topk = x2.shape[0], self.num_experts_per_tok
         pairs = tokens * topk
-        ys = out if out is not None else torch.empty((tokens, hidden), dtype=torch.float32, device=xs.device)
+        ys = out if out is not None else torch.empty((tokens, hidden), dtype=torch.float32 if typed is None else original_dtype, device=xs.device)
+        ys_type = F32 if typed is None or out is not None else typed
         if tokens == 0:
             return ys.reshape(batch, seq_len, hidden).to(original_dtype)
         self._reserve(tokens)
@@ -90,9 +97,11 @@ class FusedMoeGGUF:
         sp = torch.cuda.current_stream(xs.device).cuda_stream
         for t0 in range(0, tokens, 65535):
             t = min(65535, tokens - t0)
-            ck("cq_nn_moe_route", L.cq_nn_moe_route(x2.data_ptr() + 4 * t0 * hidden, self.gate.data_ptr(), self.topk_ids.data_ptr() + 4 * t0 * topk,
-                                                    self.topk_weights.data_ptr() + 4 * t0 * topk, self.router_logits.data_ptr() + 4 * t0 * E,
-                                                    t, hidden, E, topk, 1 if self.norm_topk_prob else 0, sp))
+            x2_at = x2.data_ptr() + 4 * t0 * hidden
+            x_at, x_type, copy_at = (x2_at, F32, None) if typed is None else (rows.data_ptr() + 2 * t0 * hidden, typed, x2_at)
+            ck("cq_nn_moe_route", L.cq_nn_moe_route_typed(x_at, x_type, copy_at, self.gate.data_ptr(), self.topk_ids.data_ptr() + 4 * t0 * topk,
+                                                          self.topk_weights.data_ptr() + 4 * t0 * topk, self.router_logits.data_ptr() + 4 * t0 * E,
+                                                          t, hidden, E, topk, 1 if self.norm_topk_prob else 0, sp))
         # (expert_ids, sorted_token_ids) of fused_moe.rs:249-260.  Every path of the expert matmuls gives each pair a row of its
         # own whatever the order of the pair list (decode-sized calls run each pair as its own matvec launch block, larger ones
         # bucket the pairs by expert themselves), so the layer does not sort: the pairs are taken in token order
@@ -152,6 +161,6 @@ class FusedMoeGGUF:
             gemm(self.down_in.data_ptr(), self.down_experts, self.topk_weights.data_ptr(), self.down_out, hidden, self.inter)
         for t0 in range(0, tokens, 65535):
             t = min(65535, tokens - t0)
-            ck("cq_nn_moe_sum", L.cq_nn_moe_sum(self.down_out.data_ptr() + 4 * t0 * topk * hidden, ys.data_ptr() + 4 * t0 * hidden, t, topk, hidden, sp))
-        ys = ys.reshape(batch, seq_len, hidden)
-        return ys if original_dtype == torch.float32 else ys.to(original_dtype)
+            ck("cq_nn_moe_sum", L.cq_nn_moe_sum_typed(self.down_out.data_ptr() + 4 * t0 * topk * hidden, ys.data_ptr() + ys.element_size() * t0 * hidden, ys_type, t, topk, hidden,
+                                                      sp))
+        return ys.reshape(batch, seq_len, hidden).to(original_dtype)

@@ -245,6 +245,11 @@ int cq_nn_moe_route(const float *x_dev, const float *router_w_dev, uint32_t *top
 int cq_nn_moe_sort(const uint32_t *topk_ids_dev, int32_t *expert_ids_dev, int32_t *sorted_token_ids_dev, int64_t n_pairs, int64_t num_experts,
                    void *stream);
 int cq_nn_moe_sum(const float *y_dev, float *out_dev, int64_t tokens, int64_t topk, int64_t dim, void *stream);
+/* The same for tokens in another type (CQ_F32, CQ_F16, CQ_BF16; the latter two 8-byte aligned): route leaves them in f32 as well, x_f32 [tokens, hidden], 16-byte aligned
+ * (NULL for CQ_F32), which the expert products take; sum rounds its results to nearest even. */
+int cq_nn_moe_route_typed(const void *x_dev, int x_dtype, float *x_f32_dev, const float *router_w_dev, uint32_t *topk_ids_dev, float *topk_weights_dev, float *logits_dev,
+                          int64_t tokens, int64_t hidden, int64_t num_experts, int64_t topk, int norm_topk_prob, void *stream);
+int cq_nn_moe_sum_typed(const float *y_dev, void *out_dev, int out_dtype, int64_t tokens, int64_t topk, int64_t dim, void *stream);
 
 #ifdef __cplusplus
 }

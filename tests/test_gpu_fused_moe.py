@@ -278,6 +278,47 @@ def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
     assert torch.equal(out[named], want[named]) if down == 0 else bool((out == 7).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,E,hidden,topk", [(1, 16, 256, 2), (33, 128, 2304, 4), (129, 128, 256, 2), (515, 130, 2048, 2), (705, 130, 1028, 3)])      # every logits kernel
+def test_half_precision_rows_in_the_router_and_the_sum(dtype, tokens, E, hidden, topk):
+    """Rows of either type give the logits, copies and choices that their f32 values give; sums are those of f32, rounded."""
+    kind = {torch.float16: 1, torch.bfloat16: 30}[dtype]
+    xd, rd = torch.from_numpy(normal(1, (tokens, hidden), 1.0)).cuda().to(dtype), torch.from_numpy(normal(2, (E, hidden), 0.1)).cuda()
+    wide = xd.float()
+
+    def route(x, kind, copy):
+        ids, w, lg = (torch.empty((tokens, n), dtype=t, device="cuda") for n, t in ((topk, torch.int32), (topk, torch.float32), (E, torch.float32)))
+        assert L().cq_nn_moe_route_typed(x.data_ptr(), kind, copy, rd.data_ptr(), ids.data_ptr(), w.data_ptr(), lg.data_ptr(), tokens, hidden, E, topk, 1, None) == 0
+        return ids, w, lg
+
+    copy = torch.full((tokens + 1, hidden), 7.0, device="cuda")
+    for a, b in zip(route(xd, kind, copy.data_ptr()), route(wide, 0, None)):
+        assert torch.equal(a, b)
+    assert torch.equal(copy[:tokens], wide) and bool((copy[tokens] == 7.0).all())
+    y = torch.from_numpy(normal(3, (tokens, topk, hidden), 1.0)).cuda()
+    y[0, 0, :4] = torch.tensor([float("inf"), -float("inf"), 7e4, 1e-41])
+    out, ref = torch.full((tokens + 1, hidden), 7.0, device="cuda", dtype=dtype), torch.empty((tokens, hidden), device="cuda")
+    assert L().cq_nn_moe_sum_typed(y.data_ptr(), out.data_ptr(), kind, tokens, topk, hidden, None) == 0
+    assert L().cq_nn_moe_sum(y.data_ptr(), ref.data_ptr(), tokens, topk, hidden, None) == 0
+    assert torch.equal(out[:tokens], ref.to(dtype)) and bool((out[tokens] == 7.0).all())
+    assert L().cq_nn_moe_route_typed(xd.data_ptr(), kind, None, rd.data_ptr(), out.data_ptr(), ref.data_ptr(), ref.data_ptr(), tokens, hidden, E, topk, 1, None) != 0
+    assert L().cq_nn_moe_sum_typed(y.data_ptr(), out.data_ptr() + 2, kind, tokens, topk, hidden, None) != 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("seq", [1, 40, 300])
+def test_fused_moe_layer_of_half_precision_rows(dtype, seq):
+    layer, _ = build_layer(oracle.Q4K, 16, 512, 256, 4, True, seed=20)
+    x = torch.from_numpy(normal(30, (1, seq, 512), 1.0)).cuda().to(dtype)
+    want = layer.forward(x.float(), True).to(dtype)
+    odd = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")[1:].view(1, seq, 512)           # rows that begin off 8 bytes
+    odd.copy_(x)
+    given = torch.empty((seq, 512), device="cuda")
+    for got in (layer.forward(x, True), layer.forward(odd, True), layer.forward(x, True, given)):
+        assert got.dtype == dtype and torch.equal(got, want)
+    assert torch.equal(given.view(1, seq, 512).to(dtype), want)
+
+
 def test_down_after_pair_refuses_what_it_cannot_reuse():
     lib = L()
     p = 256          # an aligned non-null address: the calls below return before anything is enqueued
