@@ -161,6 +161,7 @@ struct MoeChunks {
     const float *pair_scale;
     int max_chunks;
     int64_t up = 0;      // bytes from the gate weights to the up weights, where a launch multiplies by both
+    const int *src = nullptr;      // ... and the rows of the quantized activations that its pairs have (else: the pairs' own)
 };
 // Tiles of tile_rows pairs that a list of `pairs` can have: whole ones, and one that is not for every expert.  A multiple of eight (qt_moe_tile).
 inline unsigned cq_moe_grid(const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t tile_rows) {

@@ -394,21 +394,25 @@ __global__ __launch_bounds__(NW * 64, 2) void qtile_wide_kernel(const uint8_t *_
     if constexpr (DT == CQ_Q6K) w_off[NB - 1] = (uint32_t)(min(lane & 31, wlast) * row_bytes) + 208 + w_odd;
     // ---- activations: 64 bytes of 16 rows per instruction, piece p of row r in slot p ^ (r / 4) % 4 of its 64 bytes ----
     // (a super-block is [4 stages][32 MI rows][64 bytes]; instruction i of a wave brings block wv + NW i of its 8 MI KB)
-    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + (int64_t)m0 * k), 0, -1, 0x00020000);
+    // (experts' gate and up: of the tokens' rows, each of which several pairs share, those that the tile's pairs name)
+    constexpr bool NAMED = MOE && PAIR;
+    const int64_t a_first = NAMED ? 0 : m0;
+    auto a_row = [&](int r) { return NAMED ? (uint32_t)mc.src[m0 + min(r, rows - 1 - m0)] : (uint32_t)min(r, rows - 1 - m0); };
+    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void *)(av.qs + a_first * k), 0, -1, 0x00020000);
     constexpr int NAO = NW == 2 * MI ? 1 : NA;             // (as many waves as row blocks: the instructions of a wave are whole stages apart)
     uint32_t a_off[NAO];
 #pragma unroll
     for (int i = 0; i < NAO; i++) {
         const int blk = wv + NW * i, st = blk / (2 * MI), r = 16 * (blk - st * 2 * MI) + (lane >> 2), p = (lane & 3) ^ ((r >> 2) & 3);
-        a_off[i] = (uint32_t)min(r, rows - 1 - m0) * (uint32_t)k + 64 * st + 16 * p;
+        a_off[i] = a_row(r) * (uint32_t)k + 64 * st + 16 * p;
     }
     uint8_t *const myB = lds + LD::B_OFF + wv * (AHEAD * LD::B);
     // ---- scales and 16-element sums of the activations: the first half of the waves brings the sums of 32 rows each, the others the scales of 64 ----
     const bool x_sums = T::HAS_MIN && wv < NW / 2;
-    const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = min(x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane, rows - 1 - m0);
+    const int x_blk = x_sums ? min(wv, MI - 1) : min(wv & 1, (MI - 1) / 2), x_r = x_sums ? 32 * x_blk + (lane >> 1) : 64 * x_blk + lane;
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        x_sums ? (void *)(av.bsums + (int64_t)m0 * (k >> 4)) : (void *)(av.d + (int64_t)m0 * nsb_all), 0, -1, 0x00020000);
-    const uint32_t x_off = x_sums ? (uint32_t)x_r * (uint32_t)(32 * nsb_all) + 16 * (lane & 1) : (uint32_t)x_r * (uint32_t)(4 * nsb_all);
+        x_sums ? (void *)(av.bsums + a_first * (k >> 4)) : (void *)(av.d + a_first * nsb_all), 0, -1, 0x00020000);
+    const uint32_t x_off = x_sums ? a_row(x_r) * (uint32_t)(32 * nsb_all) + 16 * (lane & 1) : a_row(x_r) * (uint32_t)(4 * nsb_all);
     // Super-block kb0 + j of this workgroup's range into slot `slot`; past the end the last one again, into slots nobody reads.
     auto issue_w = [&](int j, int slot) {
         const int at = min(kb0 + j, kb1 - 1) * BB, odd = DT == CQ_Q6K ? at & 2 : 0;      // (210 kb is 2 past a dword for odd kb, and so are odd rows of an odd number of blocks)
