@@ -167,10 +167,10 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
         }
         return;
     }
-    if constexpr (TN == 4) {
-        if (o.bf16 && !o.planes && nw + 64 <= N && o.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(o.dst) & 15) == 0) {
+    if constexpr (TN % 2 == 0) {
+        if (o.bf16 && !o.planes && nw + 16 * TN <= N && (TN == 4 || o.act != CQ_DENSE_ACT_SWIGLU) && o.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(o.dst) & 15) == 0) {
             uint16_t *const dst = reinterpret_cast<uint16_t *>(o.dst);
-            if (o.act == CQ_DENSE_ACT_SWIGLU) {
+            if constexpr (TN == 4) if (o.act == CQ_DENSE_ACT_SWIGLU) {
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     uint32_t p[4];
@@ -190,7 +190,7 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j += 2) {
+                for (int j = 0; j < TN; j += 2) {
                     uint32_t p[2][2];
 #pragma unroll
                     for (int u = 0; u < 2; u++) {
@@ -528,13 +528,15 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
 #endif
 }
 
-// ---- bf16 tiles of BM activation rows x 128 weight rows, bfloat16 activations, one workgroup on a unit --------------------------------------
+// ---- bf16 tiles of BM (64, 96, 128, 192) activation rows x 128 weight rows, bfloat16 activations, one workgroup on a unit --------------------------------------
 // The 128 x 128 tile above, two workgroups to a unit, wants 512 of them: products of a few hundred tiles are cut along k instead, write their sums to memory and have
 // another launch add them, and each workgroup waits for stages that it has asked for one or three of its own short steps ago.  Here one workgroup has a unit's LDS.
 // Results are those of that tile to the last bit, so that no choice made from them (of a token's experts, say) depends on which of the two a call takes: the same
 // instructions in the order of k, and for a product that would be cut along k (PARTS) one sum per part of k_split, added in order.
 // 2048 x 2048 x 2048, cold weights: 39.5 -> 27.2 us, of which about 7 are the way to the first products and the last sums.  A stage takes 0.62 us.  Of a unit's busy cycles
 // the matrix cores have 40 % (x 7168), reads of LDS 30, and waves wait for 36 % of theirs: for stages, of which 256 units bring 13.4 TB/s out of the L2s and 2.6 from behind.
+// Tiles of 64 and 96 rows, 2 x 4 waves of BM / 2 x 32 results, for products that larger ones leave units without (1500 x 2048 x 2048 in 256 workgroups instead of 192 25.4 -> 23.6 us, 1000 x
+// 2048 x 2048 in 256 instead of four parts of 128 22.7 -> 16.3).
 // Eight waves, 4 x 2, of BM / 4 x 64 results each: four of BM / 2 x 64 read a third less from LDS, but have a matrix core to themselves and wait more (2048 x 2048 x 2048:
 // 31.0 us; 192 rows: 52 where eight take 33).  LDS holds four stages of 64 of k; copies that no register sees bring them, four ahead of the products, and the operands of
 // half a stage are read while those of the half before are multiplied: one barrier a stage, which waits for nothing that was asked for less than three stages ago.  Rows
@@ -542,13 +544,14 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
 template <int BM, bool PARTS>
 __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, int64_t M, int N, int K, int tiles_m, int tiles_n, int k_split) {
 #ifdef __HIP_DEVICE_COMPILE__                             // (the host compiler does not know the buffer accesses)
-    constexpr int STAGE = (BM + 128) * 128, TM = BM / 64, TN = 4, NX = BM / 64, NW = 2;      // 16-row blocks of a wave; copies of a wave and stage
+    constexpr int WN = BM < 128 ? 4 : 2, STAGE = (BM + 128) * 128, TM = BM / (128 / WN), TN = 8 / WN, NX = (BM + 63) / 64, NW = 2;      // 16-row blocks of a wave; copies of a wave and stage
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lk = lane >> 4;
     int tm, tn;
     tile_at(xcd_tile(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
     const int64_t m0 = (int64_t)tm * BM;
-    const int n0 = tn * 128, nst = K >> 6, part = k_split >> 6, wm = (wv >> 1) * (BM / 4), wn = (wv & 1) * 64;
+    const int n0 = tn * 128, nst = K >> 6, part = k_split >> 6, wm = wv / WN * (16 * TM), wn = wv % WN * (16 * TN);
+    const bool fewer = BM % 64 && wv >= 4;                 // (the last copy of activations is one of the first four waves')
 
     // ---- copy i of a wave brings eight rows of a stage, one 16-byte chunk a lane; rows past the end repeat the last ----
     const uint8_t *const xbase = reinterpret_cast<const uint8_t *>(src.x) + m0 * src.ldx * 2;
@@ -571,7 +574,8 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
 #pragma unroll
         for (int i = 0; i < NW; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (dt_lds *)(to + BM * 128 + 8192 * i), 16, w_off[i], at, 0, 0);
 #pragma unroll
-        for (int i = 0; i < NX; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (dt_lds *)(to + 8192 * i), 16, x_off[i], at, 0, 0);
+        for (int i = 0; i < NX; i++)
+            if (i + 1 < NX || !fewer) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (dt_lds *)(to + 8192 * i), 16, x_off[i], at, 0, 0);
         asm volatile("" ::: "memory");
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -602,7 +606,9 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
     copy(1);
     copy(2);
     copy(3);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * PER) : "memory");
+    if (fewer) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PER - 3) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PER) : "memory");
+    asm volatile("s_barrier" ::: "memory");
     constexpr std::integral_constant<int, 0> low{};
     constexpr std::integral_constant<int, 1> high{};
     operands(0, low);
@@ -612,7 +618,9 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
         operands(st, high);
         multiply(low);
         // stage st + 1 is there for everybody, and everybody has the operands of stage st: stage st + 4 may take its place
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * PER) : "memory");
+        if (fewer) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * PER - 2) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * PER) : "memory");
+        asm volatile("s_barrier" ::: "memory");
         copy(st + 4);
         operands(st + 1, low);
         multiply(high);
@@ -785,10 +793,14 @@ bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
 //     against 66.3); more parts bring more workgroups to a long k (700 x 2048 x 7168: 53.2 against 60.4);
 //   one round of 192 where 128 takes two (1500 x 3500 x 2048: 53.5 -> 34.2), else two rounds of 128 up to 384 tiles (1000 x 5632 x 2048: 57.2 -> 49.1; 448: 51.1 against 51.3);
 //   beyond one round of two to a unit, rounds of 192 that are two thirds full (1200 x 7168 x 2048: 68.4 -> 63.8, 2048 x 10368 x 2048: 130.5 -> 122.9).
-int ring_rows(const Plan &p, int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
+//   64 rows where they are one round, of a long k only if that is more than half of one (350 .. 1000 x 2048 x 2048: 21 - 29 -> 15 - 16, 850 x 2048 x 7168: 55.5 -> 39, 512 rows 34.3 against
+//     36.4, 260 rows 27.8 against 36.4), else 96 (1500 x 2048 x 2048: 25.4 -> 23.6, x 7168 65.5 -> 57.6, 1200 x 2048 x 7168 68.3 -> 52); silu results want waves of four columns of 16 (small).
+int ring_rows(const Plan &p, int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx, bool small) {
     if (p.bm != 128 || ldw > (1 << 20) || ldx > (1 << 20)) return 0;       // (its offsets have 32 bits)
-    const int64_t t128 = (int64_t)p.tiles_m * p.tiles_n, t192 = (m + 191) / 192 * p.tiles_n, rounds = (t192 + 255) / 256;
+    const int64_t t64 = (m + 63) / 64 * p.tiles_n, t96 = (m + 95) / 96 * p.tiles_n, t128 = (int64_t)p.tiles_m * p.tiles_n, t192 = (m + 191) / 192 * p.tiles_n, rounds = (t192 + 255) / 256;
     if (p.splits == 1 && large_tile(m, n, k, ldw, ldx)) return 0;
+    if (t64 <= 256 && small && (t64 > 128 || k <= 4096)) return 64;
+    if (t96 <= 256 && t64 > 256 && small) return 96;
     if (t128 <= 256) return p.splits <= 3 || (p.splits == 4 && k <= (t128 > 128 ? 3072 : 2304)) ? 128 : 0;
     if (t192 <= 256) return 192;
     if (t128 <= 384) return 128;
@@ -977,10 +989,12 @@ int cq_dense_product(int precision, const cq_dense_args *args, void *workspace_d
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.splits, (unsigned)a.batch);
 #define CQ_DM(K_) hipLaunchKernelGGL(K_, grid, dim3(256), 0, s, src, o, m, (int)n, (int)k, p.tiles_m, p.tiles_n, p.k_split)
-    const int ring = a.x_bf16 && a.batch == 1 && !a.tiles_dev && !a.src_rows_dev ? ring_rows(p, m, n, k, a.ldw, a.ldx) : 0;
+    const int ring = a.x_bf16 && a.batch == 1 && !a.tiles_dev && !a.src_rows_dev ? ring_rows(p, m, n, k, a.ldw, a.ldx, a.act != CQ_DENSE_ACT_SWIGLU) : 0;
     if (ring) {
         o.planes = nullptr;
         auto *const fn = ring == 192 ? (p.splits > 1 ? dense_ring_kernel<192, true> : dense_ring_kernel<192, false>)
+                         : ring == 64 ? (p.splits > 1 ? dense_ring_kernel<64, true> : dense_ring_kernel<64, false>)
+                         : ring == 96 ? (p.splits > 1 ? dense_ring_kernel<96, true> : dense_ring_kernel<96, false>)
                                      : (p.splits > 1 ? dense_ring_kernel<128, true> : dense_ring_kernel<128, false>);
         const int lds = 4 * (ring + 128) * 128;
         const hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);

@@ -237,3 +237,13 @@ def test_results_on_and_off_16_bytes(m, n, k, tile_rows, form):
     err = (got[0].double()[perm.long()] - rows).abs()
     err = (err - rows.abs() * (2.0 ** -22 if form == "sum" else 2.0 ** -8)).clamp(min=0)
     assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * 4
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 2048, 2048), (961, 2049, 1024), (260, 3500, 1088), (513, 2047, 2112), (850, 1024, 3584), (1024, 2500, 1024), (1153, 2178, 1088), (1536, 2048, 4160), (577, 4481, 1024)])
+def test_ring_of_64_and_of_96_rows(m, n, k):
+    """Last tiles of one row and of all but one, one part of k and up to ten: the bits of the 128 x 128 tile, and results of every kind."""
+    test_ring_of_stages_keeps_bits(m, n, k)
+    for form in ("add", "bf16", "rows"):
+        test_ring_of_stages(m, n, k, 64, form)
+    for form in ("bf16", "relu2", "sum"):
+        test_results_on_and_off_16_bytes(m, n // 2 * 2, k, 0, form)
