@@ -153,6 +153,17 @@ __device__ __forceinline__ void store_f32(const Out &o, const Row &row, Of sums,
 // of 1500 of such a model 1965 -> 1826.
 template <int TM, int TN, class At>
 __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN], At m, int nw, int lk, int64_t M, int N, int split) {
+    if (o.planes) {                                        // a part of k: nothing to look up (70 to 350 rows of small products lost 1 - 2 % on the way past the questions below)
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            float *const at = o.planes + ((int64_t)split * M + m(i)) * o.n4 + nw + 4 * lk;
+            if (m(i) < M)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    if (nw + 16 * j + 4 * lk < N) *reinterpret_cast<f32x4 *>(at + 16 * j) = acc[i][j];
+        }
+        return;
+    }
     Row row[TM];
 #pragma unroll
     for (int i = 0; i < TM; i++) row[i] = row_of(o, m(i), M);
