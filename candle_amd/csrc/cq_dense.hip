@@ -55,8 +55,18 @@ __device__ __forceinline__ Row row_of(const Out &o, int64_t m, int64_t M) {
     return Row{m, o.rows ? o.rows[mm] : mm, o.row_scale ? o.row_scale[mm] : 1.0f, m < M};
 }
 
-// four consecutive columns n .. n+3 of a row (n % 4 == 0)
-__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split) {
+// Four consecutive columns from column n of f32 values at p, those of them that there are.
+__device__ __forceinline__ f32x4 some4(const float *p, int n, int N) {
+    if (n + 4 <= N && (reinterpret_cast<uintptr_t>(p) & 15) == 0) return *reinterpret_cast<const f32x4 *>(p);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (n + i < N) v[i] = p[i];
+    return v;
+}
+
+// four consecutive columns n .. n+3 of a row (n % 4 == 0); old, more: what is there already and the addend, from a caller that has them
+__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split, const f32x4 *old = nullptr, const f32x4 *more = nullptr) {
     if (o.planes) {
         *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + row.m) * o.n4 + n) = v;
         return;
@@ -88,16 +98,15 @@ __device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int
         return;
     }
     float *d = reinterpret_cast<float *>(o.dst) + row.at * o.ldd + n;
-    const float *a = o.add ? o.add + row.at * o.ld_add + n : nullptr;
-    if (n + 4 <= N && ((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(a)) & 15) == 0) {
-        if (o.accumulate) v += *reinterpret_cast<const f32x4 *>(d);
-        if (a) v += *reinterpret_cast<const f32x4 *>(a);
+    if (o.accumulate) v += old ? *old : some4(d, n, N);
+    if (o.add) v += more ? *more : some4(o.add + row.at * o.ld_add + n, n, N);
+    if (n + 4 <= N && (reinterpret_cast<uintptr_t>(d) & 15) == 0) {
         *reinterpret_cast<f32x4 *>(d) = v;
         return;
     }
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        if (n + i < N) d[i] = v[i] + (o.accumulate ? d[i] : 0.0f) + (a ? a[i] : 0.0f);
+        if (n + i < N) d[i] = v[i];
 }
 
 __device__ __forceinline__ uint32_t pair_bf16(float a, float b) {
@@ -223,6 +232,28 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
                 }
             return;
         }
+    }
+    // Sums off 16 bytes, or in the last columns: the next row's in front of this one's stores here too (1125 x 4114 x 832 added to what is there 33.7 -> 26.4 us, 1103 x 960 x 5824 with rows an
+    // odd number of floats apart 42.6 -> 40.6, 2184 x 4686 x 1664 97.3 -> 78.9).
+    if (o.accumulate || o.add) {
+        f32x4 old[2][TN], more[2][TN];
+        auto ask = [&](int i) {
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if (!row[i].there || column(j) >= N) continue;
+                if (o.accumulate) old[i & 1][j] = some4(reinterpret_cast<const float *>(o.dst) + row[i].at * o.ldd + column(j), column(j), N);
+                if (o.add) more[i & 1][j] = some4(o.add + row[i].at * o.ld_add + column(j), column(j), N);
+            }
+        };
+        ask(0);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (i + 1 < TM) ask(i + 1);
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                if (row[i].there && column(j) < N) emit4(o, acc[i][j], row[i], column(j), M, N, split, &old[i & 1][j], &more[i & 1][j]);
+        }
+        return;
     }
 #pragma unroll
     for (int i = 0; i < TM; i++) {

@@ -247,3 +247,36 @@ def test_ring_of_64_and_of_96_rows(m, n, k):
         test_ring_of_stages(m, n, k, 64, form)
     for form in ("bf16", "relu2", "sum"):
         test_results_on_and_off_16_bytes(m, n // 2 * 2, k, 0, form)
+
+
+@pytest.mark.parametrize("precision,x_bf16,m,n,k", [(0, 1, 1100, 2506, 1024), (0, 1, 2000, 2046, 1088), (0, 1, 1500, 5634, 1088), (0, 1, 961, 2050, 1024), (0, 1, 1000, 2046, 2048), (0, 1, 2000, 3202, 832), (0, 0, 2000, 3203, 512),
+                                                    (0, 1, 2300, 4610, 1088), (0, 1, 50, 190, 512), (0, 0, 50, 189, 512), (0, 1, 20, 66, 256), (1, 0, 70, 190, 192), (1, 0, 70, 62, 192)])
+@pytest.mark.parametrize("accumulate,addend", [(1, 0), (0, 1), (1, 1)])
+def test_sums_off_16_bytes(precision, x_bf16, m, n, k, accumulate, addend):
+    """Results added to what is there, to an addend and to both, off 16 bytes (what they are added to is asked for a row ahead, column by column) and on them: the same bits, in every kernel,
+    and nothing beside them changes."""
+    print(f"case {precision} {x_bf16} {m} {n} {k} {accumulate} {addend}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = torch.randn((n, k), generator=g, device="cuda").mul_(0.02).bfloat16()
+    x = torch.randn((m, k), generator=g, device="cuda")
+    x = x.bfloat16() if x_bf16 else x
+    there, more = (torch.randn((m, n), generator=g, device="cuda") for _ in range(2))
+    L, got = _lib.mixer_lib(), []
+    nb = L.cq_dense_matmul_workspace_bytes(precision, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    for ld, first in (((n + 3) // 4 * 4 + 4, 0), ((n + 3) // 4 * 4 + 5, 1)):
+        y, add = (torch.nn.functional.pad(t, (0, ld - n, 1, 1), value=3.0).flatten().contiguous() for t in (there, more))
+        y, add = (torch.cat([t.new_full((first,), 3.0), t]) for t in (y, add))
+        a = DenseArgs(w_dev=w.data_ptr(), ldw=k, x_dev=x.data_ptr(), ldx=k, x_bf16=x_bf16, dst_dev=y.data_ptr() + 4 * (first + ld), ldd=ld, m=m, n=n, k=k, batch=1, accumulate=accumulate,
+                      add_dev=add.data_ptr() + 4 * (first + ld) if addend else None, ld_add=ld if addend else 0)
+        _lib.check("cq_dense_product", L.cq_dense_product(precision, ctypes.byref(a), ws.data_ptr(), nb, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        rows = y[first:].view(m + 2, ld)
+        got.append(rows[1:m + 1, :n].clone())
+        rows[1:m + 1, :n] = 3.0
+        assert bool((y == 3.0).all())
+    assert torch.equal(*got)
+    want = (x if precision else x.bfloat16()).double() @ w.double().t()
+    size = want.norm(dim=1, keepdim=True)
+    want = want + accumulate * there + addend * more
+    err = ((got[0] - want).abs() - want.abs() * 2.0 ** -22).clamp(min=0)       # (up to three roundings of the sums themselves)
+    assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND
