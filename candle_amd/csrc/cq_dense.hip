@@ -55,7 +55,7 @@ __device__ __forceinline__ Row row_of(const Out &o, int64_t m, int64_t M) {
     return Row{m, o.rows ? o.rows[mm] : mm, o.row_scale ? o.row_scale[mm] : 1.0f, m < M};
 }
 
-// Four consecutive columns from column n of f32 values at p, those of them that there are.
+// Four consecutive columns from column n on of f32 values at p, those of them that there are.
 __device__ __forceinline__ f32x4 some4(const float *p, int n, int N) {
     if (n + 4 <= N && (reinterpret_cast<uintptr_t>(p) & 15) == 0) return *reinterpret_cast<const f32x4 *>(p);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -64,9 +64,18 @@ __device__ __forceinline__ f32x4 some4(const float *p, int n, int N) {
         if (n + i < N) v[i] = p[i];
     return v;
 }
+__device__ __forceinline__ void store4(float *p, const f32x4 &v, int n, int N) {
+    if (n + 4 <= N && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+        *reinterpret_cast<f32x4 *>(p) = v;
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (n + i < N) p[i] = v[i];
+}
 
-// four consecutive columns n .. n+3 of a row (n % 4 == 0); old, more: what is there already and the addend, from a caller that has them
-__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split, const f32x4 *old = nullptr, const f32x4 *more = nullptr) {
+// four consecutive columns n .. n+3 of a row (n % 4 == 0)
+__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split) {
     if (o.planes) {
         *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + row.m) * o.n4 + n) = v;
         return;
@@ -98,15 +107,9 @@ __device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int
         return;
     }
     float *d = reinterpret_cast<float *>(o.dst) + row.at * o.ldd + n;
-    if (o.accumulate) v += old ? *old : some4(d, n, N);
-    if (o.add) v += more ? *more : some4(o.add + row.at * o.ld_add + n, n, N);
-    if (n + 4 <= N && (reinterpret_cast<uintptr_t>(d) & 15) == 0) {
-        *reinterpret_cast<f32x4 *>(d) = v;
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (n + i < N) d[i] = v[i];
+    if (o.accumulate) v += some4(d, n, N);
+    if (o.add) v += some4(o.add + row.at * o.ld_add + n, n, N);
+    store4(d, v, n, N);
 }
 
 __device__ __forceinline__ uint32_t pair_bf16(float a, float b) {
@@ -233,9 +236,10 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
             return;
         }
     }
-    // Sums off 16 bytes, or in the last columns: the next row's in front of this one's stores here too (1125 x 4114 x 832 added to what is there 33.7 -> 26.4 us, 1103 x 960 x 5824 with rows an
-    // odd number of floats apart 42.6 -> 40.6, 2184 x 4686 x 1664 97.3 -> 78.9).
-    if (o.accumulate || o.add) {
+    // Sums off 16 bytes, or in the last columns: the next row's in front of this one's stores here too (1125 x 4114 x 832 added to what is there 33.7 -> 26.6 us, 1103 x 960 x 5824 with rows an
+    // odd number of floats apart 42.6 -> 40.6).  (bf16 first: the others are arguments that nobody has asked for yet, and a trip to memory that results in
+    // bfloat16 need not wait for: half a microsecond.)
+    if (!o.bf16 && (o.accumulate || o.add)) {
         f32x4 old[2][TN], more[2][TN];
         auto ask = [&](int i) {
 #pragma unroll
@@ -250,8 +254,14 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
         for (int i = 0; i < TM; i++) {
             if (i + 1 < TM) ask(i + 1);
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                if (row[i].there && column(j) < N) emit4(o, acc[i][j], row[i], column(j), M, N, split, &old[i & 1][j], &more[i & 1][j]);
+            for (int j = 0; j < TN; j++) {
+                if (!row[i].there || column(j) >= N) continue;
+                f32x4 v = acc[i][j];
+                if (o.row_scale) v *= row[i].scale;
+                if (o.accumulate) v += old[i & 1][j];
+                if (o.add) v += more[i & 1][j];
+                store4(reinterpret_cast<float *>(o.dst) + row[i].at * o.ldd + column(j), v, column(j), N);
+            }
         }
         return;
     }
@@ -383,8 +393,10 @@ __global__ __launch_bounds__(256, 2) void dense_bf16_kernel(Src src, Out out, in
             fetch(k_lo + 128, third);
         }
         stage(0, first);
-        if (PF > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        else __syncthreads();
+        if (PF > 1) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);                // (one that the compiler sees: see dense_ring_kernel)
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else __syncthreads();
         int cur = 0;
         auto step = [&](int k, auto set, auto next) {          // the stage at k, which came through `set`
             const bool more = PF > 1 || k + 64 < k_hi;
@@ -653,6 +665,7 @@ __global__ __launch_bounds__(512, 2) void dense_ring_kernel(Src src, Out out, in
     asm volatile("s_barrier" ::: "memory");
     constexpr std::integral_constant<int, 0> low{};
     constexpr std::integral_constant<int, 1> high{};
+    __builtin_amdgcn_s_waitcnt(0xc07f);                    // scalar loads that only the results want: on their way into the loop they would turn its waits for single operands into waits for all
     operands(0, low);
     int left = part;                                       // stages to the end of the part
     bool first = true;
