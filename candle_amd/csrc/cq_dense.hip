@@ -840,7 +840,7 @@ bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
     return rounds == 1 ? t >= 160 : 4 * t >= 3 * 256 * rounds;
 }
 
-// Where one workgroup to a unit with a ring of stages (128 or 192 rows; 0: neither) takes the place of two workgroups of 128 x 128 (products of bfloat16 rows; the large
+// Where one workgroup to a unit with a ring of stages (64, 96, 128 or 192 rows; 0: none of them) takes the place of two workgroups of 128 x 128 (products of bfloat16 rows; the large
 // tile first where it would take the call).  At k = 2048, cold weights, one round of 256 tiles takes 23 - 27 us with 128 rows and 32 - 34 with 192; 512 tiles two to a
 // unit take 49 - 53, and fewer tiles 26 - 54 in parts of k and their sum.
 //   up to 256 tiles of 128 in up to three parts (2048 x 2048 x 2048: 39.5 -> 27.2 us, 1500 x 2048 x 7168: 86.5 -> 69.3), or four of a short k (1200 x 2048 x 2048: 37.4 ->
@@ -848,13 +848,15 @@ bool large_tile(int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx) {
 //     against 66.3); more parts bring more workgroups to a long k (700 x 2048 x 7168: 53.2 against 60.4);
 //   one round of 192 where 128 takes two (1500 x 3500 x 2048: 53.5 -> 34.2), else two rounds of 128 up to 384 tiles (1000 x 5632 x 2048: 57.2 -> 49.1; 448: 51.1 against 51.3);
 //   beyond one round of two to a unit, rounds of 192 that are two thirds full (1200 x 7168 x 2048: 68.4 -> 63.8, 2048 x 10368 x 2048: 130.5 -> 122.9).
-//   64 rows where they are one round, of a long k only if that is more than half of one (350 .. 1000 x 2048 x 2048: 21 - 29 -> 15 - 16, 850 x 2048 x 7168: 55.5 -> 39, 512 rows 34.3 against
-//     36.4, 260 rows 27.8 against 36.4), else 96 (1500 x 2048 x 2048: 25.4 -> 23.6, x 7168 65.5 -> 57.6, 1200 x 2048 x 7168 68.3 -> 52); silu results want waves of four columns of 16 (small).
+//   64 rows where they are one round, of a k that is no longer than their number pays for, since each brings its 128 weight rows of all of k by itself where parts of k share that: 350 .. 1000 x
+//     2048 x 2048 21 - 29 -> 15 - 16, 850 x 2048 x 7168 55.5 -> 39.  220 drawn products of up to 128 tiles, time with 64 rows by the time in parts: up to 112 tiles and k of 2816 0.80, of 3072 to
+//     4096 0.95 on average and up to 1.17 (241 x 3200 x 3776 24.2 against 28.4); 113 - 128 tiles 0.86 up to k of 4096; 129 - 136 tiles 0.85 up to 4992, 1.08 - 1.09 beyond (1084 x 960 x 6272 38.4
+//     against 42); more 0.79.  Else 96 (1500 x 2048 x 2048: 25.4 -> 23.6, x 7168 65.5 -> 57.6, 1200 x 2048 x 7168 68.3 -> 52).  Silu results want waves of four columns of 16 (small).
 int ring_rows(const Plan &p, int64_t m, int64_t n, int64_t k, int64_t ldw, int64_t ldx, bool small) {
     if (p.bm != 128 || ldw > (1 << 20) || ldx > (1 << 20)) return 0;       // (its offsets have 32 bits)
     const int64_t t64 = (m + 63) / 64 * p.tiles_n, t96 = (m + 95) / 96 * p.tiles_n, t128 = (int64_t)p.tiles_m * p.tiles_n, t192 = (m + 191) / 192 * p.tiles_n, rounds = (t192 + 255) / 256;
     if (p.splits == 1 && large_tile(m, n, k, ldw, ldx)) return 0;
-    if (t64 <= 256 && small && (t64 > 128 || k <= 4096)) return 64;
+    if (t64 <= 256 && small && (t64 > 136 || k <= (t64 > 128 ? 4992 : t64 > 112 ? 4096 : 2816))) return 64;
     if (t96 <= 256 && t64 > 256 && small) return 96;
     if (t128 <= 256) return p.splits <= 3 || (p.splits == 4 && k <= (t128 > 128 ? 3072 : 2304)) ? 128 : 0;
     if (t192 <= 256) return 192;

@@ -76,10 +76,10 @@ def test_stages_on_their_way(k, splits):
     assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, n:] == 5).all()
 
 
-@pytest.mark.parametrize("m,n,k,pad", [(1100, 2500, 1024, 0), (1535, 2049, 1088, 64), (1500, 2817, 1024, 128), (1537, 2700, 4160, 0), (1290, 4485, 1024, 0), (1000, 5602, 1024, 0), (1500, 5633, 1088, 64)])
+@pytest.mark.parametrize("m,n,k,pad", [(1100, 2500, 1024, 0), (2000, 2046, 1088, 64), (1535, 2049, 1088, 64), (1500, 2817, 1024, 128), (1537, 2700, 4160, 0), (1290, 4485, 1024, 0), (1000, 5602, 1024, 0), (1500, 5633, 1088, 64)])
 @pytest.mark.parametrize("form", ["plain", "add", "swiglu", "bf16", "rows"])
 def test_ring_of_stages(m, n, k, pad, form):
-    """One workgroup to a unit: 128 rows (180 and 204 tiles), 192 (one round), 128 in two rounds, 192 in two; stages of k even and odd."""
+    """One workgroup to a unit: 96 rows (of silu results 128), 128, 192 (one round), 128 in two rounds, 192 in two; stages of k even and odd."""
     print(f"case {m} {n} {k} {pad} {form}", flush=True)
     if form == "swiglu":
         n &= ~1
@@ -239,9 +239,9 @@ def test_results_on_and_off_16_bytes(m, n, k, tile_rows, form):
     assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * 4
 
 
-@pytest.mark.parametrize("m,n,k", [(1000, 2048, 2048), (961, 2049, 1024), (260, 3500, 1088), (513, 2047, 2112), (850, 1024, 3584), (1024, 2500, 1024), (1153, 2178, 1088), (1536, 2048, 4160), (577, 4481, 1024)])
+@pytest.mark.parametrize("m,n,k", [(1000, 2048, 2048), (961, 2049, 1024), (260, 3500, 2112), (513, 2047, 2112), (850, 1024, 2560), (961, 1024, 4096), (1024, 2500, 1024), (1153, 2178, 1088), (1536, 2048, 4160), (577, 4481, 1024)])
 def test_ring_of_64_and_of_96_rows(m, n, k):
-    """Last tiles of one row and of all but one, one part of k and up to ten: the bits of the 128 x 128 tile, and results of every kind."""
+    """Last tiles of one row and of all but one, three parts of k and up to ten: the bits of the 128 x 128 tile, and results of every kind.  (64 rows: the first, and the third to the sixth; 96: the others.)"""
     test_ring_of_stages_keeps_bits(m, n, k)
     for form in ("add", "bf16", "rows"):
         test_ring_of_stages(m, n, k, 64, form)
