@@ -15,10 +15,13 @@
 // their use, but a weight row's scale comes with its weights: the better way for some tiles of 32 rows, see launch_mi.)  Results then go out four columns at a time, whatever n
 // is a multiple of.  K is split over grid.z where that fills the chip better; see qtile_plan.
 //
-// Only the sums of two tiles are in registers at a time, those of the one that is scaled and of the next, and the main loop exists for each number of 32-row tiles that hold rows, which is
-// what makes that known where registers are given out.  (The sums of all tiles before: 16 registers a tile more, so that tiles end at 128 rows.)  Q4_0 has tiles of 160 rows for it, whose weights are
-// converted once where two tiles of 96 did it twice and left a sixth of the work to one of them: 131 rows of [13824 x 5120] 59.5 -> 51.7 us with f16 results.  Two tiles' sums alone, us:
-//   2048 rows of Q4_0 [14336 x 4096] 393 -> 353, 700 of [11008 x 4096] 124 -> 119; Q8_0 2048 of [4096 x 4096] 106 -> 104; 60 rows of Q4_0 [1536 x 2048] 12.1 -> 12.3 (the longer code)
+// The main loop exists for each number of 32-row tiles that hold rows, which makes that known where registers are given out.  The product that follows a tile's goes into the registers of the
+// sums that have just been scaled, a block ahead; or (TWO) only the sums of two tiles are there at a time, those of the one that is scaled and of the next: 16 registers a tile less, so that Q4_0
+// has tiles of 160 rows, whose weights are converted once where two tiles of 96 did it twice and left a sixth of the work to one of them (131 rows of [13824 x 5120] 59.5 -> 51.6 us with f16
+// results), and faster for two tiles of Q8_0 (700 rows of [11008 x 4096] 138 -> 133, a block ahead 136), slower for the others.  us, one loop for any number of tiles / two tiles' sums / now:
+//   Q4_0   2048 rows of [14336 x 4096] in tiles of 128 388 387 364   512 of [4096 x 14336] 105.9 103.7 99.6   700 of [11008 x 4096] in tiles of 64 128.3 130.6 129.4
+//   Q8_0   2048 rows of [14336 x 4096]                 409 396 393   512 of [4096 x 14336] 110.4 107.5 106.6
+// 600 drawn calls, time by that of the one loop, two tiles' sums / now: Q4_0 in tiles of 64 1.013 1.004, of 96 0.993 0.962, of 128 1.004 0.958; Q8_0 0.973 0.973, 0.985 0.979, 0.976 0.965.
 //
 // us on one card, the activations first in all tiles / the weights first from 64 rows on, quantizing the activations included:      17 rows   131 rows   512 rows   2048 rows
 //   Q4_0 [14336 x 4096]                                                                              23.5 23.7  57.6 53.7  108 103    412 393
@@ -269,7 +272,9 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
         scales_of(0, dw);
         // the main loop, for each number of tiles that hold rows
         auto run = [&](auto tiles) {
-            constexpr int LIVE = decltype(tiles)::value, NS = LIVE > 1 ? 2 : 1;
+            constexpr int LIVE = decltype(tiles)::value;
+            constexpr bool TWO = LIVE > 1 && (MI == 5 || (DT == CQ_Q8_0 && LIVE == 2));
+            constexpr int NS = TWO ? 2 : LIVE, LEAD = TWO ? 1 : NS;
             for (int j = 0; j < nsb; j++) {
                 const int kb = kb0 + j, slot = j & 1;
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -280,8 +285,7 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
 #pragma unroll
                     for (int t = 0; t < LIVE; t++) d[t] = *reinterpret_cast<const float *>(Dj + 4 * (b * BM + t * 32));
                 };
-                // The sums of the next tile, or of the first one of the next block, are on their way in the matrix cores while those of a tile are scaled; its fragment was asked for
-                // another tile before.
+                // The product LEAD tiles ahead, in this block or the next, is on its way in the matrix cores while the sums of a tile are scaled; its fragment was asked for another tile before.
                 i32x4 op, af;
                 i32x16 S[NS];
                 float d8[LIVE];
@@ -289,8 +293,11 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
                 operand(0, op);
                 d8_of(0, d8);
                 ahead(0);
-                S[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, af, magic, 0, 0, 0);
-                ahead(1);
+#pragma unroll
+                for (int u = 0; u < LEAD; u++) {
+                    S[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, af, magic, 0, 0, 0);
+                    ahead(u + 1);
+                }
 #pragma unroll
                 for (int b = 0; b < 8; b++) {
                     // the second half has landed (behind it only the next super-block's activations were asked for); the first one's place is free
@@ -315,16 +322,16 @@ __global__ __launch_bounds__(QT_NW * 64, 2) void qtile0_kernel(const uint8_t *__
                     }
 #pragma unroll
                     for (int t = 0; t < LIVE; t++) {
-                        const int u = b * LIVE + t;
+                        const int u = b * LIVE + t, v = u + LEAD;
                         auto next = [&]() {
-                            if (u + 1 < 8 * LIVE) S[(u + 1) % NS] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t + 1 < LIVE ? op : op_n, af, magic, 0, 0, 0);
-                            ahead(u + 2);
+                            if (v < 8 * LIVE) S[v % NS] = __builtin_amdgcn_mfma_i32_32x32x32_i8(v / LIVE == b ? op : op_n, af, magic, 0, 0, 0);
+                            ahead(v + 1);
                         };
-                        if (NS > 1) next();
+                        if (TWO) next();
 #pragma unroll
                         for (int e = 0; e < 16; e++) acc[t][e] = fmaf(fmaf(__int_as_float(S[u % NS][e]), dw[e >> 2][e & 3], c[e >> 2][e & 3]), d8[t], acc[t][e]);
                         qt_pin(acc[t]);
-                        if (NS == 1) next();
+                        if (!TWO) next();
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     op = op_n;

@@ -363,3 +363,29 @@ def test_extreme_block_scales_of_few_rows(fmt, bb, d):
     ok = np.isfinite(want)
     assert np.array_equal(got[~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)])
     assert rel_l2(got[ok], want[ok]) <= BOUND
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+def test_every_last_tile_keeps_the_bits(fmt):
+    """Tiles of 32 to 128 rows (Q4_0: 160), the last one with each number of parts of 32 rows: one chain of blocks a result, so the bits of the rows among 2000; and those against 64 bits."""
+    from perf import cases
+    L = _lib.lib()
+    code, n, k = FMT[fmt][0], 16384, 768
+    w = cases.blocks(fmt, 8, "w", n, k).reshape(-1)
+    x = torch.from_numpy(normal(36, (2000, k))).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+
+    def product(rows):
+        print(f"case {fmt} rows={rows}", flush=True)
+        scratch = torch.empty(L.cq_act_scratch_bytes(code, k, rows), dtype=torch.uint8, device="cuda")
+        y = torch.full((rows + 1, n), 77.0, device="cuda")
+        _lib.check("cq_quantize_act", L.cq_quantize_act(code, x.data_ptr(), 0, scratch.data_ptr(), k, rows, s))
+        _lib.check("cq_matmul", L.cq_matmul(code, w.data_ptr(), scratch.data_ptr(), y.data_ptr(), k, n, rows, n, s))
+        assert bool((y[rows] == 77).all())
+        return y[:rows]
+
+    many = product(2000)
+    values = cases.values(fmt, w.reshape(-1, cases.BLOCK_BYTES[fmt][1]), n, k)
+    assert row_error(many.cpu().numpy(), cases.product(fmt, x, values).cpu().numpy(), x.cpu().numpy(), values.cpu().numpy(), k) <= BOUND
+    for rows in (33, 64, 129, 160, 161, 193, 257, 288, 289, 321, 352, 385, 417, 449, 481, 512, 513, 545, 577, 609):
+        assert torch.equal(product(rows), many[:rows]), rows
