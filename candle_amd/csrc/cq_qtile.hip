@@ -767,8 +767,10 @@ int64_t cq_qtile_plane_bytes(int w_dtype, int64_t k, int64_t n, int64_t rows) {
 // instead of eight if their rows are at most 64: each SIMD then converts and multiplies for one wave, and a small product takes up twice as many
 // compute units (131 rows of Q6_K [4096 x 4096] unsplit: 56 us in eight waves, 41 in four; 65 rows of Q4_K [4096 x 4096] 20.6 -> 17.5).
 // Costs: fitted to earlier kernels (qtile_kernel for all tiles of K formats; the activations first in all of Q4_0 and Q8_0; rounds that leave compute units idle run at a higher clock
-// there, and a workgroup has 1.3 us of its own), which multiplied 32-row parts without rows as well: a part-filled tile still counts as a full one.  Of Q4_0 tiles of 160 rows as well, by
-// the same costs (54.4 us predicted 54.9 for 131 rows of [13824 x 5120] in four splits, 94.8 predicted 96.7 for 300 in two; where 128 rows or less are chosen they measured best as well).  With the kernels before those the choice is
+// there, and a workgroup has 1.3 us of its own), which multiplied 32-row parts without rows as well: a part-filled tile still counts as a full one.  Tiles of 160 rows (Q4_0) have these costs as well,
+// but are only taken where that makes a tenth less: those of 96 and 128 rows are 4 % faster by now than the costs say, and 160 rows in several splits slower.  180 drawn calls for which they would
+// be the least, time by that of the best other choice: predicted below 0.9 0.79 - 1.01, mean 0.90 (131 rows of [13824 x 5120] in four splits 0.95, 2048 of [14336 x 4096] 0.96); 0.9 - 1 unsplit
+// 0.95 - 1.04, in splits 0.98 - 1.27 (139 rows of [4032 x 2816] 22.5 us, 28.6 in eleven splits of 160).  With the kernels before those the choice is
 // slower than the best by 1.0 % on average for Q4_K, 0.6 for Q5_K, 1.0 for Q6_K, 1.3 for Q4_0 and 1.1 for Q8_0, by more than 5 % in 3 - 9 % of the calls, by 18 % at most (28 rows of Q6_K
 // [3667 x 3072] 16.7 us in twelve splits of eight waves, 14.1 in six of four): 1800 forwards of drawn sizes, 17 (Q4_K, Q5_K: 65) - 1600 rows, 1024 - 16384 by 1536 - 14336, cold weights, every choice timed.
 // Only splits whose sums round no more than those of the general kernels (qt_roundings).
@@ -818,7 +820,8 @@ static QtPlan qtile_plan(int w_dtype, int64_t k, int64_t n, int64_t rows, int64_
                 const double load = kq ? (double)rounds : 1.1 * (rounds - 1) + 1.0 + 0.1 * (double)(wgs - 256 * (rounds - 1)) / 256;
                 const double block = narrow ? c.a_narrow + c.b_narrow * mi : c.a + c.b * mi;
                 const double t = load * ((double)((nsb + sp - 1) / sp) * block + c.start) + (sp > 1 ? c.split + (sp + 1) * plane / c.rate : 0.0);
-                if (t < least) { least = t; best = {mi, nw, sp}; }
+                const double as = mi == 5 ? t / 0.9 : t;
+                if (as < least) { least = as; best = {mi, nw, sp}; }
             }
     return best;
 }
