@@ -1449,14 +1449,23 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const void *__restrict_
             }
         }
     }
-    store_logits<T, R>(acc, logits, t0, e0, n_experts, tokens, lane);
+    if constexpr (T * R == 64) {                           // (one at a time: their selection for one store took a quarter longer than the whole kernel does)
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+                const float v = wave_sum(acc[j][i]);
+                if (lane == 0 && e0 + i < n_experts && t0 + j < tokens) logits[(int64_t)(t0 + j) * n_experts + e0 + i] = v;
+            }
+    } else store_logits<T, R>(acc, logits, t0, e0, n_experts, tokens, lane);
 }
 
 // The same for thousands of tokens: a wave takes 8 experts of 8 tokens, whose rows the four waves of a workgroup share through LDS, 256 columns at a time, the next ones on their way.
 // Per lane the products are added in the order above: the same logits.  Bound by the vector units (393 M products of 1500 tokens and 128 experts take 10 us at their rate, the sums over lanes
 // 3) and the way from the L2, which one group of columns ahead does not hide where a SIMD has one wave.  Needs 1024 waves' worth of logits, 65536 of them, to fill the chip, and of short rows
-// some more (rows of 1024: 76800 logits 14.2 -> 15.1 us, 96000 16.0 -> 15.1).  Routing of f32 rows, every wave with rows of its own -> this: 1500 of 2048 29.0 -> 27.7 us, 3000 47.4 -> 45.6,
-// 1500 of 1024 19.3 -> 18.7, 520 to 1030 of 2048 19 - 21 -> 19.5 - 21.7.
+// some more (rows of 1024: 76800 logits 14.2 -> 15.1 us, 96000 16.0 -> 15.1).  Up to 131072 logits, two of its waves a SIMD, the waits at its barriers are longer than what the shared rows save of
+// f32 tokens of 2048 columns and more, for which every wave keeps rows of its own, <8, 1, 8>.  Routing of f32 rows, us, rows of its own / shared: 515 tokens and 128 experts of 2048 columns 19.1 20.0,
+// 1000 20.4 21.2, of 3072 24.8 25.9, of 4096 28.9 31.2, 1000 of 1024 16.4 16.0; 1171 of 2048 26.6 24.7, 1500 27.9 26.6, 3000 47.4 45.2.  Half-precision rows: shared, 1000 of 2048 23.6 22.6.
 template <int X>
 __global__ __launch_bounds__(256, 3) void moe_logits_tile_kernel(const void *__restrict__ x, const float *__restrict__ router_w, float *__restrict__ logits,
                                                                  int hidden, int n_experts, int tokens, float *__restrict__ x_f32) {
@@ -1670,7 +1679,8 @@ void moe_logits_launch(const void *x, const float *w, float *logits, int hidden,
     if (n <= 4096) hipLaunchKernelGGL((moe_logits_kernel<1, 8, 1, X>), grid(1, 1), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
     else if (n <= 16384) hipLaunchKernelGGL((moe_logits_kernel<4, 2, 1, X>), grid(4, 1), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
     else if (n < (hidden < 2048 ? 90112 : 65536)) hipLaunchKernelGGL((moe_logits_kernel<4, 2, 2, X>), grid(4, 2), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
-    else hipLaunchKernelGGL(moe_logits_tile_kernel<X>, grid(8, 8), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
+    else if (X != CQ_F32 || hidden < 2048 || n > 131072) hipLaunchKernelGGL(moe_logits_tile_kernel<X>, grid(8, 8), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
+    else if constexpr (X == CQ_F32) hipLaunchKernelGGL((moe_logits_kernel<8, 1, 8, X>), grid(8, 8), dim3(256), 0, s, x, w, logits, hidden, experts, tokens, x_f32);
 }
 
 inline bool misaligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; }
