@@ -227,9 +227,21 @@ template <int NH> __device__ __forceinline__ void lds_write_h(_Float16 *dstrow, 
     for (int i = 0; i < NH / 8; i++) p[i] = u32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
 }
 
+// MOE: which tile of the chunk table, and which block of columns, a workgroup takes; false where it has none.  The grid has room for more tiles than there are: the
+// workgroups with work are the first ones, tile by tile within a block of columns, so that they come to the XCDs and their CUs evenly whatever the number of tiles
+// (with blockIdx.x as the tile the ones without work lie between them: Q2_K, 720 pairs on 12 experts of 2560 x 4096 103 us where the grid was the whole table, 130
+// where its width was a multiple of eight and 87 so; 1600 on 16 of 768 x 4096 70, 90, 66; Q3_K, 2400 on 12 of 4096 x 1280 100, 134, 99)
+__device__ __forceinline__ bool moe_tile(const MoeChunks &mc, int &tile, int &block) {
+    const uint32_t id = blockIdx.x + gridDim.x * blockIdx.y, tiles = (uint32_t)mc.n_chunks[0];
+    if (id >= (uint64_t)tiles * gridDim.y) return false;
+    tile = id % tiles;
+    block = id / tiles;
+    return true;
+}
+
 // NJ = 32-column MFMA tiles per wave: block tile 128 x (64 * NJ).  NJ = 1 halves the accumulators so that two
 // workgroups share a CU and one converts operands while the other feeds the matrix cores.
-// MOE: blockIdx.x is a tile of the chunk table: up to BMT expert-sorted activation rows [first, first + count) of
+// MOE: a tile of the chunk table (moe_tile): up to BMT expert-sorted activation rows [first, first + count) of
 // expert e; the weights are that expert's [n, k] matrix and output rows are scattered through pair_out with pair_scale.
 // SM (experts with few rows each): the block tile is 32 (m) x 128 (n) (one workgroup per CU for a two-term format, whose
 // two weight tiles fill the LDS), the four waves side by side along n, so that a
@@ -254,13 +266,14 @@ __global__ __launch_bounds__(256, NJ == 1 && !(SM && Stage<DT>::TERMS == 2) ? 2 
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int wm = SM ? 0 : wv >> 1, wn = SM ? wv : wv & 1;
-    int m0 = blockIdx.x * BMT;
-    const int n0 = blockIdx.y * BN;
+    int m0 = blockIdx.x * BMT, n0 = blockIdx.y * BN;
     if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;           // uniform over the workgroup
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+        int tile, block;
+        if (!moe_tile(mc, tile, block)) return;                  // uniform over the workgroup
+        m0 = mc.first[tile];
+        n0 = block * BN;
+        rows = m0 + mc.count[tile];
+        w += (int64_t)mc.expert[tile] * expert_bytes;
     }
     // every thread stages NW = 64 / TPR weights of one row per stage (16 when the tile has 64 weight rows, else 32), so
     // that all waves carry the same conversion work and the loop body has no wave-dependent branch
@@ -492,7 +505,7 @@ template <> struct Q0Info<CQ_Q8_0> { static constexpr int QS = 2, QH = -1, MIN =
 template <> struct Q0Info<CQ_Q4_1> { static constexpr int QS = 4, QH = -1, MIN = 2; static constexpr uint32_t BIAS = 0; };
 template <> struct Q0Info<CQ_Q5_0> { static constexpr int QS = 6, QH = 2, MIN = -1; static constexpr uint32_t BIAS = 0x70707070u; };
 template <> struct Q0Info<CQ_Q5_1> { static constexpr int QS = 8, QH = 4, MIN = 2; static constexpr uint32_t BIAS = 0; };
-// MOE: blockIdx.x is a tile of the chunk table, as in the kernels above.
+// MOE: a tile of the chunk table, as in the kernels above.
 template <int DT, int NJ, bool MOE = false, bool SM = false>
 __global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void qmm_q0_i8_kernel(const uint8_t *__restrict__ w, ActView av, float *__restrict__ dst,
                                                                            int k, int n, int rows, int64_t stride_dst, MoeChunks mc,
@@ -513,13 +526,14 @@ __global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void qmm_q0_i8_kernel(const u
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int wm = SM ? 0 : wv >> 1, wn = SM ? wv : wv & 1;
-    int m0 = blockIdx.x * BMT;
-    const int n0 = blockIdx.y * BN;
+    int m0 = blockIdx.x * BMT, n0 = blockIdx.y * BN;
     if (MOE) {
-        if ((int)blockIdx.x >= mc.n_chunks[0]) return;           // uniform over the workgroup
-        m0 = mc.first[blockIdx.x];
-        rows = m0 + mc.count[blockIdx.x];
-        w += (int64_t)mc.expert[blockIdx.x] * expert_bytes;
+        int tile, block;
+        if (!moe_tile(mc, tile, block)) return;                  // uniform over the workgroup
+        m0 = mc.first[tile];
+        n0 = block * BN;
+        rows = m0 + mc.count[tile];
+        w += (int64_t)mc.expert[tile] * expert_bytes;
     }
     // split-K over spans of 256 elements, like the other kernels; a stage is half a span
     const int nsb_all = k >> 8;
