@@ -191,8 +191,7 @@ int cq_moe_stream_launch(int w_dtype, const void *w_a, const void *w_b, float *o
 // kernel's 32-row tiles against 427-644 us on the 8-pairs-per-pass matvec (the prefill kernels that most formats have now: 800 pairs of Q6_K 121 -> 84 us, of
 // Q8_0 95 -> 74 per product).
 #define CQ_MOE_MFMA_MIN_PAIRS 257
-// rows of one MFMA tile of an expert: the small tile while experts average fewer than 40 rows (two small tiles cost
-// more than one large one)
+// rows of one MFMA tile of an expert; which of the two: moe_tile_rows (cq_moe.hip)
 #define CQ_MOE_TILE_SMALL 32
 #define CQ_MOE_TILE_LARGE 128
 // silu(x w_gate^T) * x w_up^T in one launch, for the shapes that takes_swiglu names
@@ -200,9 +199,9 @@ bool cq_qtile_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, in
 int cq_qtile_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *dst, int64_t k, int64_t n, int64_t rows, int64_t plane_bytes,
                            hipStream_t s);
 // num_experts, pairs: what the number of tiles that hold rows follows from
-bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n, int tile_rows);
+bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n);
 int cq_qtile_moe_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k,
-                               int64_t n, int tile_rows, hipStream_t s);
+                               int64_t n, hipStream_t s);
 int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k, int64_t n, int tile_rows,
                         hipStream_t s);
 int cq_matmul_moe_launch(int w_dtype, const void *w, const void *scratch, int64_t rows_alloc, float *out, const MoeChunks &mc, int64_t num_experts, int64_t k,

@@ -364,16 +364,33 @@ static bool moe_takes_mfma(int w_dtype, const void *w, const void *w_b, int64_t 
     const bool q0_ok = (w_dtype == CQ_Q4_0 || w_dtype == CQ_Q8_0) && ((uintptr_t)w & 7) == 0 && (!w_b || ((uintptr_t)w_b & 7) == 0);
     return k % 256 == 0 && (cq_is_kquant(w_dtype) || q0_ok) && cq_has_mfma(w_dtype) && n_pairs >= CQ_MOE_MFMA_MIN_PAIRS;
 }
-// Rows of a tile of one expert's pairs: 128 (of which parts of 32 rows that are not there are left out) from 19 pairs an expert on, so that most experts convert and read their weights once.
-// n: rows of an expert's weights (of a gate / up call, whose grouping the down projection takes over: of that call).  Experts of 32-element blocks have room for more workgroups a unit
-// in tiles of 32 rows; where those of 128 leave much of a second round empty (128 experts of 768 rows: 384 workgroups), from 30 on.  us of a layer, limit at 8 / 20 / 40 pairs an expert:
-//   Q6_K 64 experts of 2048 x 1024, 6 each, 170 tokens 184 181 181, 205: 189 225 225, 400: 214 214 314; 128 of 1024 x 512, 8 each, 310: 189 193 193, 620: 221 221 326
-//   Q8_0 64 of 2048 x 1024, 170: 163 150 150, 205: 169 195 195, 400: 189 189 239; 128 of 2048 x 768, 310: 269 244 244, 420: 287 287 262, 500: 299 299 327
-//   Q4_0 64 of 2048 x 1024, 170: 140 156 156, 205: 149 185 185; 128 of 2048 x 768, 250: 230 195 195, 310: 236 222 222
-static int moe_tile_rows(int w_dtype, int64_t n_pairs, int64_t num_experts, int64_t n) {
-    const int64_t wgs = num_experts * ((n + 255) / 256), rounds = (wgs + 255) / 256;
-    const bool gaps = !cq_is_kquant(w_dtype) && rounds > 1 && 5 * wgs < 4 * 256 * rounds;
-    return n_pairs < (gaps ? 30 : 19) * num_experts ? CQ_MOE_TILE_SMALL : CQ_MOE_TILE_LARGE;
+// Rows of a tile of one expert's pairs, 32, or 128 of which parts of 32 rows that are not there are left out.  A tile of 128 reads and converts an expert's weights once where those of 32 do it
+// for every 32 pairs, but takes 5 - 20 % longer for the same rows: which is better depends on whether the second tiles of experts with more than 32 pairs fit into the rounds of workgroups that
+// the first ones leave part-filled.  With p pairs an expert on average about (p - 18) / 22 of them have a second tile (between even and as uneven as those of a model), so:
+// time in tiles of 128 over that in tiles of 32, p = 20, 24, 28, 33, 38 with even loads and, behind the bar, uneven ones:
+//   Q8_0 16 experts of 2048 x 1024 (64 workgroups)  1.08 1.17 1.17 1.16 1.17 | 1.08 1.17 1.19 1.18 1.19      40 of 2048 x 1024 (160)  1.07 1.09 1.14 1.11 0.73 | 1.14 1.14 1.14 1.28 1.28
+//   Q8_0 64 experts of 2048 x 1024 (256)  1.05 0.73 0.74 0.76 0.76 | 0.75 0.76 0.77 0.84 0.84      128 of 2048 x 768 (384)  1.08 1.09 1.11 0.88 0.89 | 1.13 1.20 0.94 0.94 0.93
+//   Q6_K as Q8_0 (the first 1.09 1.09 1.16 1.16 1.15, the last 1.04 1.05 1.06 0.84 0.85), Q4_0 of more than 1024 columns too (24 of 4096 x 1280, 120: 1.06 1.06 1.19 1.19 1.18; 32 of 4096 x 2048,
+//   256: 1.08 1.07 0.78 0.79 0.80).  Q4_K and Q5_K (what is not batched matvecs): a second tile pays up to 64 pairs
+//   (32 rows by the batched matvecs 0.8 where 128 take 0.9 - 1.15 of their time, 64 and 96 workgroups).
+// General kernels, whose tiles of 32 rows are 128 columns wide and those of 128 rows 64, over 780 shapes of 8 to 160 experts, time against the better of the two with the limit below (and without
+// a split by workgroups): Q2_K 1.008 (at 27 1.026, at 60 1.017); Q3_K 1.026 (at 18 1.033, at 39 1.055), where 39 is the better one for few workgroups; Q6_K of rows below 1536 1.024 (1.027, 1.085);
+// Q4_0 of up to 1024 columns 1.044 (at 18 1.034, but up to 1.11 of what tiles of 32 rows took where this is at most 1.08; at 39 1.106).
+// n, k: columns and rows' length of the weights (of a gate / up call, whose grouping the down projection takes over: of that call).
+static int moe_tile_rows(int w_dtype, int64_t n_pairs, int64_t num_experts, int64_t n, int64_t k) {
+    const int64_t wide = num_experts * ((n + 255) / 256), narrow = num_experts * ((n + 127) / 128), room = (wide + 255) / 256 * 256;
+    int64_t small = 18 + 22 * (room - wide) / wide;        // pairs an expert up to which tiles of 32 rows are taken
+    small = std::min<int64_t>(std::max<int64_t>(small, 18), w_dtype == CQ_Q4K || w_dtype == CQ_Q5K ? 64 : 39);
+    if (w_dtype == CQ_Q4_0 && n <= 1024) small = narrow <= 64 ? 30 : 24;
+    if (w_dtype == CQ_Q2K) small = 39;
+    if (w_dtype == CQ_Q3K) small = narrow <= 64 ? 39 : 27;
+    if (w_dtype == CQ_Q6K && k < 1536) small = narrow <= 224 ? 30 : 21;
+    return n_pairs < (small + 1) * num_experts ? CQ_MOE_TILE_SMALL : CQ_MOE_TILE_LARGE;
+}
+
+// Gate and up in one launch, which has tiles of 128 rows whatever their number (twice as many workgroups as a launch for one of them): from 19 pairs an expert on, beyond the batched matvecs.
+static bool moe_swiglu_pairs(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
+    return n_pairs >= 19 * num_experts && !cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n);
 }
 
 int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *gate, const float *up, const float *topk_weights, float *out,
@@ -388,8 +405,8 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
     const MoeWorkspace ws = moe_workspace(w_dtype, num_experts, n_pairs, n_pairs / topk, k_pair);
     // the pair call ran its experts as batched matvecs (chunks of 16 pairs): this one must be able to as well
     // (n of the pair call = this call's k; its expert tensors were 16-byte aligned or it returned CQ_ERR_ALIGN)
-    if (cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k_pair, k)) {
-        if (!up) return CQ_ERR_RANGE;                      // (such calls have no swiglu form)
+    if (!up && !moe_swiglu_pairs(w_dtype, num_experts, n_pairs, k_pair, k)) return CQ_ERR_RANGE;
+    if (up && cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k_pair, k)) {
         if (!cq_moe_stream_takes(w_dtype, w_down, nullptr, num_experts, n_pairs, k, n)) return CQ_ERR_RANGE;
         if (cq_align256(cq_moe_stream_operand_bytes(num_experts, n_pairs, k)) > ws.offsets_off) return CQ_ERR_RANGE;
         uint8_t *b = (uint8_t *)workspace;
@@ -414,7 +431,8 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
     int rc = cq_quantize_act_swiglu_gather_launch(w_dtype, gate, up, pout, n_valid, topk_weights, pscale, b + ws.act_off, k, n_pairs, ws.rows_alloc, s);
     if (rc) return rc;
     MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
-    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, num_experts, k, n, moe_tile_rows(w_dtype, n_pairs, num_experts, k), s);
+    const int tile_rows = up ? moe_tile_rows(w_dtype, n_pairs, num_experts, k, k_pair) : CQ_MOE_TILE_LARGE;
+    return cq_matmul_moe_launch(w_dtype, w_down, b + ws.act_off, ws.rows_alloc, out, mc, num_experts, k, n, tile_rows, s);
 }
 
 int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
@@ -427,9 +445,9 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     if (a.w_b && !a.swiglu && mfma && !cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) && cq_moe_wants_aligned(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n) &&
         (((uintptr_t)a.w | (uintptr_t)a.w_b) & 15))
         return CQ_ERR_ALIGN;
-    if (a.swiglu && (!mfma || stream_shape || cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) ||
+    if (a.swiglu && (!mfma || cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) || !moe_swiglu_pairs(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n) ||
                      a.x_rows * a.k > 0x7fffffffLL ||                          // (tokens' rows are named by 32-bit offsets)
-                     !cq_qtile_moe_takes_swiglu(a.w_dtype, a.w, a.w_b, a.num_experts, a.k, a.n, moe_tile_rows(a.w_dtype, a.n_pairs, a.num_experts, a.n))))
+                     !cq_qtile_moe_takes_swiglu(a.w_dtype, a.w, a.w_b, a.num_experts, a.k, a.n)))
         return CQ_ERR_RANGE;
     if (a.w_b && !mfma) {
         // only the MFMA path shares its grouping pass and quantized activations between two weight tensors
@@ -460,7 +478,7 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     int *extra = (int *)(b + ws.extra_off);
     // Hundreds of pairs per call: the expert-sorted rows go through the MFMA prefill kernel of the format in tiles of up to
     // 128 rows of one expert (integer-exact like the dense paths).  Otherwise 8 pairs per matvec pass.
-    const int tile_rows = moe_tile_rows(a.w_dtype, a.n_pairs, a.num_experts, a.n);
+    const int tile_rows = a.swiglu ? CQ_MOE_TILE_LARGE : moe_tile_rows(a.w_dtype, a.n_pairs, a.num_experts, a.n, a.k);
     const bool many = a.n_pairs > GROUP_MANY_PAIRS;
     auto *const group = a.num_experts <= GROUP_LDS_EXPERTS ? (many ? moe_group_kernel<true, true> : moe_group_kernel<true, false>)
                                                            : (many ? moe_group_kernel<false, true> : moe_group_kernel<false, false>);
@@ -491,7 +509,7 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
         MoeChunks mc{chunks, chunks + 1, chunks + 1 + ws.max_chunks, chunks + 1 + 2 * ws.max_chunks, pout, pscale, (int)ws.max_chunks};
         if (a.swiglu) {
             mc.src = pin;
-            return cq_qtile_moe_swiglu_launch(a.w_dtype, a.w, a.w_b, cq_act_view(b + ws.act_off, a.w_dtype, a.k, a.x_rows), a.out, mc, a.num_experts, a.n_pairs, a.k, a.n, tile_rows, s);
+            return cq_qtile_moe_swiglu_launch(a.w_dtype, a.w, a.w_b, cq_act_view(b + ws.act_off, a.w_dtype, a.k, a.x_rows), a.out, mc, a.num_experts, a.n_pairs, a.k, a.n, s);
         }
         rc = cq_matmul_moe_launch(a.w_dtype, a.w, b + ws.act_off, ws.rows_alloc, a.out, mc, a.num_experts, a.k, a.n, tile_rows, s);
         if (!rc && a.w_b) rc = cq_matmul_moe_launch(a.w_dtype, a.w_b, b + ws.act_off, ws.rows_alloc, a.out_b, mc, a.num_experts, a.k, a.n, tile_rows, s);

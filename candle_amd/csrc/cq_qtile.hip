@@ -895,8 +895,8 @@ int cq_qtile_moe_launch(int w_dtype, const void *w, const ActView &av, float *ou
 
 // silu(gate) * up of experts in tiles of 128 rows, K formats.  1500 tokens, 128 Q4_K experts of 2048 x 768, 8 each: 131 us, and 15 of the quantizer behind; a launch of 1.5 rounds for
 // each of the two took 79 and 79, and the quantizer that multiplied them 22.
-bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n, int tile_rows) {
-    return tile_rows == 128 && (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K || w_dtype == CQ_Q6K) && cq_qtile_takes(w_dtype, w_gate, k, num_experts * n) &&
+bool cq_qtile_moe_takes_swiglu(int w_dtype, const void *w_gate, const void *w_up, int64_t num_experts, int64_t k, int64_t n) {
+    return (w_dtype == CQ_Q4K || w_dtype == CQ_Q5K || w_dtype == CQ_Q6K) && cq_qtile_takes(w_dtype, w_gate, k, num_experts * n) &&
            cq_qtile_takes(w_dtype, w_up, k, num_experts * n) && (n + 16 * QT_NW - 1) / (16 * QT_NW) <= 65535;
 }
 template <int DT>
@@ -905,11 +905,11 @@ static int moe_swiglu_go(dim3 grid, const void *w, const ActView &av, float *out
     return qtile_go(qtile_wide_kernel<DT, 4, true, QT_NW, true>, QT_NW, bytes, grid, w, av, out, CQ_F32, k, n, 0, n, mc, n * (k / 256) * cq_type_size(DT), nullptr, s);
 }
 int cq_qtile_moe_swiglu_launch(int w_dtype, const void *w_gate, const void *w_up, const ActView &av, float *out, const MoeChunks &mc, int64_t num_experts, int64_t pairs, int64_t k,
-                               int64_t n, int tile_rows, hipStream_t s) {
-    if (!cq_qtile_moe_takes_swiglu(w_dtype, w_gate, w_up, num_experts, k, n, tile_rows)) return CQ_ERR_RANGE;
+                               int64_t n, hipStream_t s) {
+    if (!cq_qtile_moe_takes_swiglu(w_dtype, w_gate, w_up, num_experts, k, n)) return CQ_ERR_RANGE;
     MoeChunks both = mc;
     both.up = (const uint8_t *)w_up - (const uint8_t *)w_gate;
-    const dim3 grid(cq_moe_grid(mc, num_experts, pairs, tile_rows), (unsigned)((n + 16 * QT_NW - 1) / (16 * QT_NW)));
+    const dim3 grid(cq_moe_grid(mc, num_experts, pairs, CQ_MOE_TILE_LARGE), (unsigned)((n + 16 * QT_NW - 1) / (16 * QT_NW)));
     switch (w_dtype) {
         case CQ_Q4K: return moe_swiglu_go<CQ_Q4K>(grid, w_gate, av, out, k, n, both, s);
         case CQ_Q5K: return moe_swiglu_go<CQ_Q5K>(grid, w_gate, av, out, k, n, both, s);

@@ -332,9 +332,10 @@ def test_few_rows_keep_the_bits_of_many(fmt, n, k):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
-@pytest.mark.parametrize("E,n,pairs", [(16, 2052, 528), (16, 4100, 528), (16, 8196, 530), (40, 2052, 1200), (64, 2048, 1600), (33, 4097, 513)])
+@pytest.mark.parametrize("E,n,pairs", [(16, 2052, 528), (16, 4100, 528), (16, 8196, 448), (33, 2052, 513), (33, 4097, 513), (40, 4100, 600), (64, 2048, 1100)])
 def test_grouped_tiles_of_32_rows_keep_bits(fmt, E, n, pairs):
-    """Experts on either side of the limits between the two orders of operands (Q4_0): the bits of each expert's own product, which no other rows change."""
+    """Experts on either side of the limits between the two orders of operands (Q4_0: the activations first in the second, third, fourth and sixth case, of 408, 726, 297 and 680 expected
+    workgroups): the bits of each expert's own product, which no other rows change."""
     import candle_amd as ca
     from perf import cases
     L = _lib.lib()
