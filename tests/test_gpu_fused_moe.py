@@ -195,11 +195,12 @@ def _qwen3_layer():
     return _QWEN3["v"]
 
 
-@pytest.mark.parametrize("tokens,is_prefill", [(16, False), (16, True), (40, True), (256, True), (256, False), (600, True)])
+@pytest.mark.parametrize("tokens,is_prefill", [(16, False), (16, True), (40, True), (256, True), (256, False), (380, True), (400, True), (600, True)])
 def test_fused_moe_layer_qwen3_shape_token_batches(tokens, is_prefill):
     """16 to 600 tokens through the Qwen3-30B-A3B-shape layer: 128 (token, expert) pairs on the per-pair kernels; 320, 2048 and
-    4800 pairs with every expert as a batched matvec over its own pairs (2.5, 16 and 37.5 pairs per expert on average: one
-    sparse set, two sets, a second pass over the weights), against the CPU restatement of FusedMoeGGUF::forward."""
+    3040 pairs with every expert as a batched matvec over its own pairs (2.5, 16 and 23.75 pairs per expert on average: one
+    sparse set, two sets, a second pass over the weights of some); 3200 and 4800 in tiles, gate and up in one launch (25 and 37.5:
+    one and two parts of 32 rows), against the CPU restatement of FusedMoeGGUF::forward."""
     layer, ref = _qwen3_layer()
     x = normal(70 + tokens, (1, tokens, 2048), 1.0)
     got = layer.forward(torch.from_numpy(x).cuda(), is_prefill).cpu().numpy()
@@ -235,7 +236,7 @@ def test_down_projection_on_the_grouping_of_gate_and_up(dtype, tokens, E, topk):
 
 
 @pytest.mark.parametrize("dtype", [oracle.Q4K, oracle.Q5K, oracle.Q6K])
-@pytest.mark.parametrize("counts", [[300, 0, 1, 33, 64, 65, 127, 130], [28] * 24, [19, 20, 18, 19] * 6])
+@pytest.mark.parametrize("counts", [[300, 0, 1, 33, 64, 65, 127, 130], [28] * 66, [25] * 66, [19, 20, 18, 19] * 6])
 @pytest.mark.parametrize("inter,hidden", [(256, 512), (768, 256), (512, 2048)])
 def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
     """silu(gate) * up in the tiles of one launch, and the down projection behind it: bit for bit what the two products, cq_nn_silu_mul and the down projection of their own give.  Pairs that
@@ -257,7 +258,8 @@ def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
     h, out = torch.full((pairs, inter), 7.0, device="cuda"), torch.full((pairs, hidden), 7.0, device="cuda")
     swiglu = lib.cq_moe_gemm_gguf_pair_swiglu(int(dtype), x.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), h.data_ptr(), E, topk, pairs, inter, hidden,
                                               ws.data_ptr(), nb, None)
-    batched = dtype in (oracle.Q4K, oracle.Q5K) and pairs <= 27 * E
+    few = E * -(-min(inter, hidden) // 256)
+    batched = pairs <= {oracle.Q4K: 64 if few <= 24 else 30 if few <= 48 else 24, oracle.Q5K: 64 if few <= 64 else 25}.get(dtype, 0) * E
     short = dtype == oracle.Q6K and hidden < 1536                     # (left to the general kernels)
     if batched or short or pairs < 19 * E:
         assert swiglu == -6 and bool((h == 7).all())                  # CQ_ERR_RANGE: nothing enqueued

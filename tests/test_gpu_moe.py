@@ -91,7 +91,7 @@ def test_moe_gemm_gguf_gate_and_down(dtype, tokens, is_prefill):
 @pytest.mark.parametrize("k,n", [(256, 64), (512, 40), (768, 203), (1024, 130), (1792, 50), (2048, 96), (2304, 33), (4096, 72)])
 @pytest.mark.parametrize("with_weights", [False, True])
 def test_moe_gemm_gguf_experts_as_batched_matvecs(wdt, k, n, with_weights):
-    """Q4_K or Q5_K experts hit by at most 27 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
+    """Few Q4_K or Q5_K experts hit by at most 64 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
     over the weights).  Expert loads on every edge: none, one pair, 15 / 16 / 17, 31 / 32 / 33 (a second pass), 47 .. 49, 65 (a
     third pass); rows of 1 .. 16 super-blocks (one to eight waves per row block, columns without a wave's second column), ragged
     n, several workgroups per expert."""
