@@ -1109,11 +1109,11 @@ int cq_matvec_batch_swiglu_launch(int w_dtype, const void *w, const float *gate,
 // ---- MoE: experts as batched matvecs (see qme_q4k_kernel) ----
 // Q4_K or Q5_K experts of rows up to 16 super-blocks (two columns per wave: three do not fit the registers next to two operand sets), 16-byte aligned, and few pairs per expert: a pass over
 // the weights per 32 pairs loses to the tiles that reuse a weight 128 times where those fill the chip.  Where few workgroups (of 256 columns) have the weights to themselves, a tile's longer
-// chain through k is what a call takes.  Counted by the shorter side of the weights, so that the gate / up and the down projections of a layer take one form.  Pairs an expert on average
-// up to which a call is batched, from 1170 single products and layers of 8 - 160 experts with 18 - 62 pairs each, both forms timed: geometric mean of the time against that with 64 everywhere, and
-// how many of them take more than 1.05 of it
-//   Q4_K  64 up to 24 workgroups, 30 up to 48, else 24: 0.805, 4 of 593 (27 throughout: 0.823, 9 and up to 1.57; 64 up to 40: 0.810, 5)
-//   Q5_K  64 up to 64, else 25: 0.866, 3 of 580 (27 throughout: 0.874, 30 and up to 1.58; 64 up to 56, else 22: 0.850, 8)
+// chain through k is what a call takes: up to 64 pairs an expert then.  Time of one product in tiles over batched, 26 - 62 pairs an expert (456 products of 6 - 32 experts):
+//   k 2048: 12 - 16 workgroups Q4_K 0.86 - 1.08, Q5_K 1.07 - 1.38; 24 - 32 0.74 - 1.08, 0.87 - 1.38; 48 0.69 - 0.95, 0.82 - 1.14; 64 0.66 - 0.88, 0.76 - 1.08
+//   k 2560: 24 1.05 - 1.17, 1.16 - 1.39; 32 0.94 - 1.15, 1.07 - 1.32; 48 0.80 - 0.99, 0.92 - 1.16; 64 0.82 - 0.99, 0.91 - 1.13
+//   k 4096: 30 - 60 1.16 - 1.52, 1.24 - 1.84;      k 1280, n 4096: 0.53 - 0.71, 0.56 - 0.79;      k up to 1024: 0.72 and 0.83 on average
+// With the limits below they take 0.72 (Q4_K) and 0.82 of the time batched, 4 and 6 of 228 each more than 1.05 of it and 1.16 at most; at 27 throughout 0.89 and 0.98, 38 and 78, 1.84.
 // us of a layer, batched matvecs / tiles: 64 experts of 2048 x 1024, 6 each, 230 / 330 / 430 / 640 tokens Q4_K 109 112, 145 126, 178 136, 230 157, Q5_K 119 131, 157 144, 192 155, 249 174;
 // 128 of 2048 x 768, 8 each, 400 / 600 / 1000 Q4_K 168 174, 248 200, 336 237, Q5_K 184 203, 266 228, 362 264; 64 of 1024 x 512, 4 each, 400 / 900 Q4_K 70 54, 110 70, Q5_K 71 60, 113 78.
 static bool qme_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n, int64_t pairs_each) {
@@ -1121,9 +1121,9 @@ static bool qme_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t
            n_pairs <= pairs_each * num_experts && n * (k / 256) * qb_bb(w_dtype == CQ_Q5K) < 0x7fffffffLL;
 }
 bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
-    const int64_t wgs = num_experts * ((std::min(n, k) + 255) / 256);
-    const int64_t pairs_each = w_dtype == CQ_Q5K ? (wgs <= 64 ? 64 : 25) : (wgs <= 24 ? 64 : wgs <= 48 ? 30 : 24);
-    return qme_shape(w_dtype, num_experts, n_pairs, k, n, pairs_each);
+    const int64_t wgs = num_experts * ((n + 255) / 256);
+    const bool few = w_dtype == CQ_Q5K ? k >= 2048 && wgs <= std::min<int64_t>(64, k / 48) : k > 2048 && wgs <= std::min<int64_t>(64, k / 64);
+    return qme_shape(w_dtype, num_experts, n_pairs, k, n, few ? 64 : w_dtype == CQ_Q5K ? 25 : 24);
 }
 // Up to 64 pairs an expert a gate / up call, and a down projection on its grouping, ask for 16-byte aligned experts, whichever form they take.
 bool cq_moe_wants_aligned(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) { return qme_shape(w_dtype, num_experts, n_pairs, k, n, 64); }

@@ -14,7 +14,7 @@
 // hit expert's rows once: workgroup (row tile, expert) keeps the decoded weight registers and loops
 // over that expert's pairs — unlike the reference kernels, which re-read the expert's weights for
 // every pair routed to it.  (Few pairs skip steps 1 and 2: a fused matvec per pair.  Hundreds of pairs take step 3 on the matrix
-// cores: Q4_K and Q5_K experts with up to two dozen pairs each (few experts: 64) as batched matvecs over their pairs, cq_matvec_batch.hip, the rest as tiles of
+// cores: Q4_K and Q5_K experts with up to two dozen pairs each (few of long rows: 64) as batched matvecs over their pairs, cq_matvec_batch.hip, the rest as tiles of
 // expert-sorted rows through the prefill kernel of the format.)
 #include <algorithm>
 #include "cq_device.h"
@@ -388,9 +388,12 @@ static int moe_tile_rows(int w_dtype, int64_t n_pairs, int64_t num_experts, int6
     return n_pairs < (small + 1) * num_experts ? CQ_MOE_TILE_SMALL : CQ_MOE_TILE_LARGE;
 }
 
-// Gate and up in one launch, which has tiles of 128 rows whatever their number (twice as many workgroups as a launch for one of them): from 19 pairs an expert on, beyond the batched matvecs.
+// Gate and up in one launch, which has tiles of 128 rows whatever their number (twice as many workgroups as a launch for one of them): from 19 pairs an expert on where a
+// product is not batched matvecs, and from 28 where it is: a layer gains more by the one launch.  us of a layer, each product batched / gate and up in one launch: 12 experts of 2560 x 1024, 28 each,
+// Q4_K 85 65, Q5_K 90 77, 16 and 50 each 106 71, 111 84, 6 and 50 76 64, 79 76; 8 of 2048 x 512, 50 each, 56 53, 58 63 (few and short ones of Q5_K are what loses: 150 layers of 6 - 32 experts
+// 0.90 on average, 11 of them above 1.04, 1.21 at most; Q4_K 0.81 and 1.04).
 static bool moe_swiglu_pairs(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
-    return n_pairs >= 19 * num_experts && !cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n);
+    return n_pairs >= 19 * num_experts && (n_pairs > 27 * num_experts || !cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n));
 }
 
 int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *gate, const float *up, const float *topk_weights, float *out,
@@ -438,7 +441,7 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
 int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     if (a.n_pairs > 0x7fffffffLL || a.x_rows > 0x7fffffffLL) return CQ_ERR_RANGE;
     const bool mfma = moe_takes_mfma(a.w_dtype, a.w, a.w_b, a.n_pairs, a.k);
-    const bool stream_shape = mfma && !cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) && cq_moe_stream_shape(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n);
+    const bool stream_shape = mfma && !a.swiglu && !cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) && cq_moe_stream_shape(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n);
     const bool stream = stream_shape && cq_moe_stream_takes(a.w_dtype, a.w, a.w_b, a.num_experts, a.n_pairs, a.k, a.n);
     // (a later cq_moe_down_after_pair_launch tells from the shape alone how this call chunked its pairs)
     if (a.w_b && stream_shape && !stream) return CQ_ERR_ALIGN;

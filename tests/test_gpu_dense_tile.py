@@ -76,10 +76,10 @@ def test_stages_on_their_way(k, splits):
     assert (y[0] == 5).all() and (y[m + 1] == 5).all() and (y[:, n:] == 5).all()
 
 
-@pytest.mark.parametrize("m,n,k,pad", [(1100, 2500, 1024, 0), (2000, 2046, 1088, 64), (1535, 2049, 1088, 64), (1500, 2817, 1024, 128), (1537, 2700, 4160, 0), (1290, 4485, 1024, 0), (1000, 5602, 1024, 0), (1500, 5633, 1088, 64)])
+@pytest.mark.parametrize("m,n,k,pad", [(1100, 2500, 1024, 0), (1535, 2049, 1088, 64), (1500, 2817, 1024, 128), (1537, 2700, 4160, 0), (1290, 4485, 1024, 0), (1000, 5602, 1024, 0), (1500, 5633, 1088, 64)])
 @pytest.mark.parametrize("form", ["plain", "add", "swiglu", "bf16", "rows"])
 def test_ring_of_stages(m, n, k, pad, form):
-    """One workgroup to a unit: 96 rows (of silu results 128), 128, 192 (one round), 128 in two rounds, 192 in two; stages of k even and odd."""
+    """One workgroup to a unit: 128 rows (180 and 204 tiles), 192 (one round), 128 in two rounds, 192 in two; stages of k even and odd."""
     print(f"case {m} {n} {k} {pad} {form}", flush=True)
     if form == "swiglu":
         n &= ~1
@@ -239,14 +239,24 @@ def test_results_on_and_off_16_bytes(m, n, k, tile_rows, form):
     assert float((err.norm(dim=1, keepdim=True) / size).max()) <= BOUND * 4
 
 
-@pytest.mark.parametrize("m,n,k", [(1000, 2048, 2048), (961, 2049, 1024), (260, 3500, 2112), (513, 2047, 2112), (850, 1024, 2560), (961, 1024, 4096), (1024, 2500, 1024), (1153, 2178, 1088), (1536, 2048, 4160), (577, 4481, 1024)])
+@pytest.mark.parametrize("m,n,k", [(1000, 2048, 2048), (961, 2049, 1024), (260, 3500, 1088), (513, 2047, 2112), (850, 1024, 3584), (1024, 2500, 1024), (1153, 2178, 1088), (1536, 2048, 4160), (577, 4481, 1024)])
 def test_ring_of_64_and_of_96_rows(m, n, k):
-    """Last tiles of one row and of all but one, three parts of k and up to ten: the bits of the 128 x 128 tile, and results of every kind.  (64 rows: the first, and the third to the sixth; 96: the others.)"""
+    """Last tiles of one row and of all but one, one part of k and up to ten: the bits of the 128 x 128 tile, and results of every kind."""
     test_ring_of_stages_keeps_bits(m, n, k)
     for form in ("add", "bf16", "rows"):
         test_ring_of_stages(m, n, k, 64, form)
     for form in ("bf16", "relu2", "sum"):
         test_results_on_and_off_16_bytes(m, n // 2 * 2, k, 0, form)
+
+
+@pytest.mark.parametrize("form", ["plain", "add", "swiglu", "bf16", "rows"])
+def test_ring_of_96_rows_or_of_128_of_silu_results(form):
+    test_ring_of_stages(2000, 2046, 1088, 64, form)
+
+
+@pytest.mark.parametrize("m,n,k", [(260, 3500, 2112), (850, 1024, 2560), (961, 1024, 4096)])
+def test_ring_of_64_rows_in_three_parts_of_k_and_more(m, n, k):
+    test_ring_of_64_and_of_96_rows(m, n, k)
 
 
 @pytest.mark.parametrize("precision,x_bf16,m,n,k", [(0, 1, 1100, 2506, 1024), (0, 1, 2000, 2046, 1088), (0, 1, 1500, 5634, 1088), (0, 1, 961, 2050, 1024), (0, 1, 1000, 2046, 2048), (0, 1, 2000, 3202, 832), (0, 0, 2000, 3203, 512),

@@ -195,12 +195,11 @@ def _qwen3_layer():
     return _QWEN3["v"]
 
 
-@pytest.mark.parametrize("tokens,is_prefill", [(16, False), (16, True), (40, True), (256, True), (256, False), (380, True), (400, True), (600, True)])
+@pytest.mark.parametrize("tokens,is_prefill", [(16, False), (16, True), (40, True), (256, True), (256, False), (600, True)])
 def test_fused_moe_layer_qwen3_shape_token_batches(tokens, is_prefill):
     """16 to 600 tokens through the Qwen3-30B-A3B-shape layer: 128 (token, expert) pairs on the per-pair kernels; 320, 2048 and
-    3040 pairs with every expert as a batched matvec over its own pairs (2.5, 16 and 23.75 pairs per expert on average: one
-    sparse set, two sets, a second pass over the weights of some); 3200 and 4800 in tiles, gate and up in one launch (25 and 37.5:
-    one and two parts of 32 rows), against the CPU restatement of FusedMoeGGUF::forward."""
+    4800 pairs with every expert as a batched matvec over its own pairs (2.5, 16 and 37.5 pairs per expert on average: one
+    sparse set, two sets, a second pass over the weights), against the CPU restatement of FusedMoeGGUF::forward."""
     layer, ref = _qwen3_layer()
     x = normal(70 + tokens, (1, tokens, 2048), 1.0)
     got = layer.forward(torch.from_numpy(x).cuda(), is_prefill).cpu().numpy()
@@ -236,7 +235,7 @@ def test_down_projection_on_the_grouping_of_gate_and_up(dtype, tokens, E, topk):
 
 
 @pytest.mark.parametrize("dtype", [oracle.Q4K, oracle.Q5K, oracle.Q6K])
-@pytest.mark.parametrize("counts", [[300, 0, 1, 33, 64, 65, 127, 130], [28] * 66, [25] * 66, [19, 20, 18, 19] * 6])
+@pytest.mark.parametrize("counts", [[300, 0, 1, 33, 64, 65, 127, 130], [28] * 24, [19, 20, 18, 19] * 6])
 @pytest.mark.parametrize("inter,hidden", [(256, 512), (768, 256), (512, 2048)])
 def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
     """silu(gate) * up in the tiles of one launch, and the down projection behind it: bit for bit what the two products, cq_nn_silu_mul and the down projection of their own give.  Pairs that
@@ -258,8 +257,7 @@ def test_gate_and_up_in_one_launch(dtype, counts, inter, hidden):
     h, out = torch.full((pairs, inter), 7.0, device="cuda"), torch.full((pairs, hidden), 7.0, device="cuda")
     swiglu = lib.cq_moe_gemm_gguf_pair_swiglu(int(dtype), x.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), h.data_ptr(), E, topk, pairs, inter, hidden,
                                               ws.data_ptr(), nb, None)
-    few = E * -(-min(inter, hidden) // 256)
-    batched = pairs <= {oracle.Q4K: 64 if few <= 24 else 30 if few <= 48 else 24, oracle.Q5K: 64 if few <= 64 else 25}.get(dtype, 0) * E
+    batched = dtype in (oracle.Q4K, oracle.Q5K) and pairs <= 27 * E
     short = dtype == oracle.Q6K and hidden < 1536                     # (left to the general kernels)
     if batched or short or pairs < 19 * E:
         assert swiglu == -6 and bool((h == 7).all())                  # CQ_ERR_RANGE: nothing enqueued
@@ -357,3 +355,40 @@ def test_fused_moe_argument_errors():
     assert lib.cq_nn_moe_route(256, 256, 256, 256, None, 1, 8, 4, 2, 1, None) == -4
     assert lib.cq_nn_moe_sort(None, 256, 256, 4, 8, None) == -4
     assert lib.cq_nn_moe_sum(256, 256, 1, 2, 6, None) == -2
+
+
+@pytest.mark.parametrize("tokens", [380, 400])
+def test_fused_moe_layer_qwen3_shape_on_either_side_of_the_batched_form(tokens):
+    """3040 pairs, 23.75 an expert, as batched matvecs with a second pass over the weights of some; 3200 in tiles, gate and up in one launch."""
+    test_fused_moe_layer_qwen3_shape_token_batches(tokens, True)
+
+
+@pytest.mark.parametrize("dtype", [oracle.Q4K, oracle.Q5K, oracle.Q6K])
+@pytest.mark.parametrize("inter,hidden", [(256, 512), (768, 256), (512, 2048)])
+def test_gate_and_up_of_66_experts_in_one_launch(dtype, inter, hidden):
+    test_gate_and_up_in_one_launch(dtype, [28] * 66, inter, hidden)
+
+
+@pytest.mark.parametrize("dtype", [oracle.Q4K, oracle.Q5K])
+@pytest.mark.parametrize("tokens", [130, 148, 256])
+def test_few_experts_of_long_rows(dtype, tokens):
+    """32 to 64 pairs an expert of eight: each product on its own runs as batched matvecs, a layer has gate, up and silu in one launch, which agree with those to rounding."""
+    from candle_amd import _lib
+    from tests.test_gpu_moe import make_experts
+    lib, E, topk, inter, hidden = L(), 8, 2, 512, 2304
+    pairs = tokens * topk
+    layer, ref = build_layer(dtype, E, hidden, inter, topk, True, seed=520)
+    x = normal(521 + tokens, (1, tokens, hidden), 1.0)
+    xd = torch.from_numpy(x).cuda()
+    assert rel_l2(layer.forward(xd, True).cpu().numpy(), ref.forward(x)) <= 1e-3
+    (_, g), (_, u) = (make_experts(dtype, E, inter, hidden, seed=s) for s in (1, 2))
+    sti, eid = torch.arange(pairs, dtype=torch.int32, device="cuda"), (torch.arange(pairs, dtype=torch.int32, device="cuda") % E).contiguous()
+    nb = lib.cq_moe_gemm_workspace_bytes(int(dtype), E, topk, pairs, inter, hidden, 0)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    h, a, b = (torch.full((pairs, inter), 7.0, device="cuda") for _ in range(3))
+    _lib.check("swiglu", lib.cq_moe_gemm_gguf_pair_swiglu(int(dtype), xd.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), h.data_ptr(), E, topk, pairs, inter,
+                                                          hidden, ws.data_ptr(), nb, None))
+    _lib.check("pair", lib.cq_moe_gemm_gguf_pair(int(dtype), xd.data_ptr(), g.device_ptr(), u.device_ptr(), sti.data_ptr(), eid.data_ptr(), a.data_ptr(), b.data_ptr(), E, topk, pairs, inter,
+                                                 hidden, 1, ws.data_ptr(), nb, None))
+    a, b = a.double(), b.double()
+    assert rel_l2(h.cpu().numpy(), (a / (1 + torch.exp(-a)) * b).cpu().numpy()) <= 1e-5

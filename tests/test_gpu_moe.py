@@ -91,7 +91,7 @@ def test_moe_gemm_gguf_gate_and_down(dtype, tokens, is_prefill):
 @pytest.mark.parametrize("k,n", [(256, 64), (512, 40), (768, 203), (1024, 130), (1792, 50), (2048, 96), (2304, 33), (4096, 72)])
 @pytest.mark.parametrize("with_weights", [False, True])
 def test_moe_gemm_gguf_experts_as_batched_matvecs(wdt, k, n, with_weights):
-    """Few Q4_K or Q5_K experts hit by at most 64 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
+    """Q4_K or Q5_K experts hit by at most 27 pairs on average run as batched matvecs over their own pairs (sets of 16, two sets per pass
     over the weights).  Expert loads on every edge: none, one pair, 15 / 16 / 17, 31 / 32 / 33 (a second pass), 47 .. 49, 65 (a
     third pass); rows of 1 .. 16 super-blocks (one to eight waves per row block, columns without a wave's second column), ragged
     n, several workgroups per expert."""
@@ -423,3 +423,41 @@ def test_more_than_256_pairs_on_short_rows(tokens):
     assert L.cq_moe_direct_pairs(oracle.Q4K, E, tokens * topk, 2048) == (1 if tokens * topk <= 384 else 0)
     assert L.cq_moe_direct_pairs(oracle.Q4K, E, tokens * topk, 4096) == 0
     assert L.cq_moe_direct_pairs(oracle.Q4K, 8, 256, 4096) == 1
+
+
+def check_pair_by_pair(wdt, counts, k, n, seed):
+    """Pairs of experts with these loads, in any order, against the oracle, with and without weights: all of them in norm, and each one, since a row in another's place would hide there."""
+    import candle_amd as ca
+    E, topk, n_pairs = len(counts), 2, sum(counts)
+    assert n_pairs % topk == 0 and n_pairs >= 257
+    print(f"case {NAMES[wdt]} E={E} pairs={n_pairs} k={k} n={n}", flush=True)
+    blocks, qt = make_experts(wdt, E, n, k, seed=seed)
+    rng = np.random.Generator(np.random.PCG64(seed + 1))
+    expert_ids = np.repeat(np.arange(E, dtype=np.int32), counts)
+    sorted_token_ids = rng.permutation(n_pairs).astype(np.int32)
+    sti, eid = torch.from_numpy(sorted_token_ids).cuda(), torch.from_numpy(expert_ids).cuda()
+    for tw in (None, rng.uniform(0.1, 1.0, n_pairs).astype(np.float32)):
+        x = normal(seed + 2, (n_pairs if tw is not None else n_pairs // topk, k), 1.0)
+        got = ca.moe_gemm_gguf(torch.from_numpy(x).cuda(), qt, torch.from_numpy(tw).cuda() if tw is not None else None, sti, eid, topk, True).cpu().numpy()
+        want = oracle.moe_gemm_gguf(wdt, x, blocks, (E, n, k), sorted_token_ids, expert_ids, tw, topk)
+        assert rel_l2(got, want) <= TIGHT
+        for p in range(n_pairs):
+            assert rel_l2(got[p], want[p]) <= 1e-5, p
+
+
+@pytest.mark.parametrize("wdt,k,n", [(oracle.Q4K, 4352, 130), (oracle.Q5K, 4352, 260), (oracle.Q6K, 1536, 203), (oracle.Q6K, 2304, 260), (oracle.Q6K, 512, 130), (oracle.Q2K, 768, 203), (oracle.Q3K, 768, 203),
+                                     (oracle.Q4_0, 768, 203), (oracle.Q4_0, 512, 2052), (oracle.Q8_0, 768, 260)], ids=lambda v: NAMES.get(v, str(v)))
+@pytest.mark.parametrize("counts", [[0, 1, 31, 32, 33, 2, 3, 0, 12, 17, 5, 40, 7, 6, 8, 9, 4, 10, 11, 13, 14, 15, 16, 1, 0, 1], [8, 9] * 17, [18] * 16], ids=["uneven", "8-9", "18"])
+def test_tiles_of_32_pairs_of_uneven_experts(wdt, k, n, counts):
+    """Up to 18 pairs an expert: tiles of 32 rows of every kernel that has them (rows of Q4_K and Q5_K that the batched matvecs do not take), part-filled, whole and more than one of an expert."""
+    counts = counts + [sum(counts) % 2]
+    assert sum(counts) <= 18 * len(counts)
+    check_pair_by_pair(wdt, counts, k, n, 291)
+
+
+@pytest.mark.parametrize("wdt", [oracle.Q4K, oracle.Q5K], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("k,n,counts", [(2048, 96, [290, 20, 20, 0, 0, 7, 0, 1, 0, 12, 0, 0, 0, 3, 0, 29]), (768, 203, [290, 20, 20, 0, 0, 7, 0, 1, 0, 12, 0, 0, 0, 3, 0, 29]),
+                                        (2304, 130, [40, 64, 0, 65, 97, 110]), (4096, 72, [64, 63, 62, 67, 64])])
+def test_few_experts_of_many_pairs_as_batched_matvecs(wdt, k, n, counts):
+    """Loads up to the limit of the batched form, one expert with most pairs and, of long rows, up to 64 pairs an expert."""
+    check_pair_by_pair(wdt, counts, k, n, 391)
