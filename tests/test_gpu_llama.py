@@ -424,3 +424,23 @@ def test_prompt_with_gate_and_up_in_one_product(gate, down, apart, rows):
         assert model.L.pairs == []
         assert torch.isfinite(want).all() and torch.equal(got, want)
         assert all(torch.equal(a, lw.k_cache[:, :n]) for a, lw in zip(keys, model.layers))
+
+
+@pytest.mark.parametrize("dtypes", [Q3_K_M, Q2_K_MIX, UNFUSED, dict(Q2_K_MIX, attention_wv=oracle.Q4_0, feed_forward_w3=oracle.Q8_0)], ids=["q3_k_m", "q2k-q3k", "q5k-q6k-q4k", "not-all-k"])
+@pytest.mark.parametrize("rows", [64, 65, 131])
+def test_prompt_rows_quantized_by_the_norm(dtypes, rows):
+    """Projections of any K formats over the rows that the norm has quantized, and, where one of them is not of those, over its f32 rows: the bits of the forward that takes the steps one by
+    one, and of up to 64 rows too."""
+    from candle_amd.quantized import GgmlDType
+    from candle_amd.quantized_llama import Config, ModelWeights
+    cfg = Config(**dict(WIDE, n_layer=2))
+    model = ModelWeights.random_init(cfg, seed=12, dtypes={n: GgmlDType(d) for n, d in dtypes.items()})
+    ids = torch.from_numpy(np.random.default_rng(rows).integers(0, cfg.vocab, (1, rows)).astype(np.int32))
+    got = model.forward(ids, 0)
+    keys = [lw.k_cache[:, :rows].clone() for lw in model.layers]
+    model.clear_kv_cache()
+    model.tap = lambda stage, li: None
+    want = model.forward(ids, 0)
+    model.tap = None
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+    assert all(torch.equal(a, lw.k_cache[:, :rows]) for a, lw in zip(keys, model.layers))

@@ -876,3 +876,28 @@ def test_argument_validation():
     assert lib.cq_nn_attention(16, 256, 16, 16, 16, None, 0, 1, 4, 2, 64, 1024, 600, 0.1, None, 0, None) == -5   # splits need a workspace
     assert lib.cq_nn_silu_mul(16, 16, 16, 1, 8, 4, 8, None) == -2
     assert lib.cq_nn_rope_i_kv(16, 16, 16, 16, 16, 16, 16, None, 7, 2, 4, 2, 64, 8, 256, 128, 128, None) == -6   # pos + rows > ctx
+
+
+@pytest.mark.parametrize("code", [10, 11])
+@pytest.mark.parametrize("dim,rows,n", [(256, 65, 130), (2304, 67, 257), (8192, 66, 131)])
+def test_rms_norm_quantized_of_the_small_k_formats(code, dim, rows, n):
+    """Q2_K and Q3_K: the quantized rows of the norm and cq_quantize_act, and the products over them those of cq_qmatmul_forward, bit for bit; gate and up in one launch is not for them."""
+    import oracle
+    lib = L()
+    xs, ds, ws = dev(normal(2, (rows, dim), 1.0)), dev(normal(3, (rows, dim), 0.5)), dev(normal(4, (dim,), 1.0))
+    normed, sums = torch.empty((rows, dim), device="cuda"), torch.empty((rows, dim), device="cuda")
+    ok(lib.cq_nn_rms_norm(xs.data_ptr(), ds.data_ptr(), ws.data_ptr(), sums.data_ptr(), normed.data_ptr(), rows, dim, 1e-5, None))
+    nb, full = lib.cq_act_scratch_bytes(code, dim, rows), lib.cq_qmatmul_workspace_bytes(code, rows, dim, 2 * n)
+    rowed = torch.full((nb,), 173, dtype=torch.uint8, device="cuda")
+    ok(lib.cq_quantize_act(code, normed.data_ptr(), 0, rowed.data_ptr(), dim, rows, None))
+    room = torch.full((full,), 173, dtype=torch.uint8, device="cuda")
+    blocks = dev(oracle.from_float(code, normal(5, (n * dim,), 0.02)))
+    a, b = torch.empty((rows, n), device="cuda"), torch.full((rows, n), 7.0, device="cuda")
+    ok(lib.cq_qmatmul_forward(code, blocks.data_ptr(), normed.data_ptr(), 0, a.data_ptr(), 0, rows, dim, n, room.data_ptr(), full, None))
+    room.fill_(173)
+    ok(lib.cq_nn_rms_norm_quantized(code, xs.data_ptr(), ds.data_ptr(), ws.data_ptr(), xs.data_ptr(), rows, dim, 1e-5, room.data_ptr(), full, None))
+    assert torch.equal(room[:nb], rowed) and torch.equal(xs, sums)
+    assert lib.cq_nn_qmatmul_swiglu_pair(code, blocks.data_ptr(), blocks.data_ptr(), room.data_ptr(), b.data_ptr(), rows, dim, n, room.data_ptr(), full, None) == -6
+    assert bool((b == 7).all()) and torch.equal(room[:nb], rowed)
+    ok(lib.cq_qmatmul_quantized(code, blocks.data_ptr(), b.data_ptr(), 0, rows, dim, n, room.data_ptr(), full, None))
+    assert torch.equal(a, b) and torch.equal(room[:nb], rowed)
