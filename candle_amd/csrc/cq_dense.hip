@@ -46,13 +46,13 @@ __device__ __forceinline__ void put(const Out &o, int64_t at, float v) {
 
 // Where row m of a product goes and its factor.
 struct Row {
-    int64_t m, at;
+    int64_t at;
     float scale;
     bool there;
 };
 __device__ __forceinline__ Row row_of(const Out &o, int64_t m, int64_t M) {
     const int64_t mm = min(m, M - 1);
-    return Row{m, o.rows ? o.rows[mm] : mm, o.row_scale ? o.row_scale[mm] : 1.0f, m < M};
+    return Row{o.rows ? o.rows[mm] : mm, o.row_scale ? o.row_scale[mm] : 1.0f, m < M};
 }
 
 // Four consecutive columns from column n on of f32 values at p, those of them that there are.
@@ -75,11 +75,7 @@ __device__ __forceinline__ void store4(float *p, const f32x4 &v, int n, int N) {
 }
 
 // four consecutive columns n .. n+3 of a row (n % 4 == 0)
-__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int64_t M, int N, int split) {
-    if (o.planes) {
-        *reinterpret_cast<f32x4 *>(o.planes + ((int64_t)split * M + row.m) * o.n4 + n) = v;
-        return;
-    }
+__device__ __forceinline__ void emit4(const Out &o, f32x4 v, const Row &row, int n, int N) {
     if (o.act == CQ_DENSE_ACT_SWIGLU) {                    // columns are gate, up, gate, up
         const float a = row.scale * dense_silu(v.x) * v.y, b = row.scale * dense_silu(v.z) * v.w;
         const int64_t at = row.at * o.ldd + (n >> 1);
@@ -134,7 +130,7 @@ __device__ __forceinline__ void swap_rows(uint32_t &a, uint32_t &b) {
 
 // Whether results of columns n .. n + wide - 1 lie on 16 bytes, in f32 without an activation: whole rows of them in one go.
 __device__ __forceinline__ bool plain_f32(const Out &o, int n, int wide, int N) {
-    return !o.planes && !o.bf16 && o.act == CQ_DENSE_ACT_NONE && n + wide <= N && ((o.ldd | (o.add ? o.ld_add : 0)) & 3) == 0 &&
+    return !o.bf16 && o.act == CQ_DENSE_ACT_NONE && n + wide <= N && ((o.ldd | (o.add ? o.ld_add : 0)) & 3) == 0 &&
            ((reinterpret_cast<uintptr_t>(o.dst) | reinterpret_cast<uintptr_t>(o.add)) & 15) == 0;
 }
 // One row of them: NF times four columns, number f from column(f) on, added to what is there and to the addend.
@@ -191,7 +187,7 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
         return;
     }
     if constexpr (TN % 2 == 0) {
-        if (o.bf16 && !o.planes && nw + 16 * TN <= N && (TN == 4 || o.act != CQ_DENSE_ACT_SWIGLU) && o.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(o.dst) & 15) == 0) {
+        if (o.bf16 && nw + 16 * TN <= N && (TN == 4 || o.act != CQ_DENSE_ACT_SWIGLU) && o.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(o.dst) & 15) == 0) {
             uint16_t *const dst = reinterpret_cast<uint16_t *>(o.dst);
             if constexpr (TN == 4) if (o.act == CQ_DENSE_ACT_SWIGLU) {
 #pragma unroll
@@ -270,7 +266,7 @@ __device__ __forceinline__ void put_sums(const Out &o, const f32x4 (&acc)[TM][TN
         if (!row[i].there) continue;
 #pragma unroll
         for (int j = 0; j < TN; j++)
-            if (column(j) < N) emit4(o, acc[i][j], row[i], column(j), M, N, split);
+            if (column(j) < N) emit4(o, acc[i][j], row[i], column(j), N);
     }
 }
 
@@ -576,7 +572,7 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(Src src, Out out, in
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int n = n0 + wn + 32 * j + 8 * v + 4 * kg;
-                if (n < N) emit4(out, f32x4{acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]}, row[i], n, M, N, 0);
+                if (n < N) emit4(out, f32x4{acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]}, row[i], n, N);
             }
     }
 #endif
@@ -797,9 +793,7 @@ __global__ __launch_bounds__(256) void dense_planes_kernel(Out out, int64_t M, i
     const int n = (int)(i - m * groups) * 4;
     f32x4 v = *reinterpret_cast<const f32x4 *>(out.planes + m * out.n4 + n);
     for (int s = 1; s < splits; s++) v += *reinterpret_cast<const f32x4 *>(out.planes + ((int64_t)s * M + m) * out.n4 + n);
-    Out o = out;
-    o.planes = nullptr;
-    emit4(o, v, row_of(o, m, M), n, M, N, 0);
+    emit4(out, v, row_of(out, m, M), n, N);
 }
 
 struct Plan {
