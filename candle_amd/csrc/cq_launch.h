@@ -174,7 +174,6 @@ int cq_moe_chunks_launch(int w_dtype, const void *w, const void *scratch, int64_
 // Q4_K experts hit by a few dozen pairs each as batched matvecs (cq_matvec_batch.hip): the expert-sorted pairs of an expert are the
 // batch rows, in sets of 16 whose quantized rows sit in operand tiles.
 bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);      // ... by shape alone
-bool cq_moe_wants_aligned(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);
 bool cq_moe_stream_takes(int w_dtype, const void *w, const void *w_b, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n);
 int64_t cq_moe_stream_operand_bytes(int64_t num_experts, int64_t n_pairs, int64_t k);
 #define CQ_MOE_STREAM_CHUNK 16

@@ -1125,8 +1125,6 @@ bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int6
     const bool few = w_dtype == CQ_Q5K ? k >= 2048 && wgs <= std::min<int64_t>(64, k / 48) : k > 2048 && wgs <= std::min<int64_t>(64, k / 64);
     return qme_shape(w_dtype, num_experts, n_pairs, k, n, few ? 64 : w_dtype == CQ_Q5K ? 25 : 24);
 }
-// Up to 64 pairs an expert a gate / up call, and a down projection on its grouping, ask for 16-byte aligned experts, whichever form they take.
-bool cq_moe_wants_aligned(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) { return qme_shape(w_dtype, num_experts, n_pairs, k, n, 64); }
 bool cq_moe_stream_takes(int w_dtype, const void *w, const void *w_b, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
     return cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)w_b & 15) == 0;
 }

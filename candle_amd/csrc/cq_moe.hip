@@ -422,7 +422,6 @@ int cq_moe_down_after_pair_launch(int w_dtype, const void *w_down, const float *
         return cq_moe_stream_launch(w_dtype, w_down, nullptr, out, nullptr, b + ws.act_off, offsets, pout, pscale, (int *)(b + ws.extra_off), 1,
                                     num_experts, k, n, s);
     }
-    if (cq_moe_wants_aligned(w_dtype, num_experts, n_pairs, k_pair, k) && ((uintptr_t)w_down & 15)) return CQ_ERR_RANGE;
     // the rows of this call are quantized into the front of the workspace: they must end before that call's tables begin
     if (cq_act_layout(w_dtype, k, ws.rows_alloc).total > ws.offsets_off) return CQ_ERR_RANGE;
     uint8_t *b = (uint8_t *)workspace;
@@ -445,9 +444,6 @@ int cq_moe_launch(const MoeArgs &a, void *workspace, hipStream_t s) {
     const bool stream = stream_shape && cq_moe_stream_takes(a.w_dtype, a.w, a.w_b, a.num_experts, a.n_pairs, a.k, a.n);
     // (a later cq_moe_down_after_pair_launch tells from the shape alone how this call chunked its pairs)
     if (a.w_b && stream_shape && !stream) return CQ_ERR_ALIGN;
-    if (a.w_b && !a.swiglu && mfma && !cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) && cq_moe_wants_aligned(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n) &&
-        (((uintptr_t)a.w | (uintptr_t)a.w_b) & 15))
-        return CQ_ERR_ALIGN;
     if (a.swiglu && (!mfma || cq_moe_direct(a.w_dtype, a.num_experts, a.n_pairs, a.k) || !moe_swiglu_pairs(a.w_dtype, a.num_experts, a.n_pairs, a.k, a.n) ||
                      a.x_rows * a.k > 0x7fffffffLL ||                          // (tokens' rows are named by 32-bit offsets)
                      !cq_qtile_moe_takes_swiglu(a.w_dtype, a.w, a.w_b, a.num_experts, a.k, a.n)))

@@ -208,8 +208,8 @@ int cq_moe_gemm_gguf(int w_dtype, const float *x_dev, const void *w_dev, const i
  * grouped by expert and the activations quantized once for both (Q4_K / Q5_K experts that see at most 24 / 25 pairs each on average, or 64 where k is
  * above / at least 2048 and num_experts * ceil(n / 256) at most 64 and k / 64 or k / 48, rows up to 4096 elements: both tensors in one launch, every expert a batched matvec over its own pairs);
  * otherwise it is the two calls.  w_a / w_b [num_experts, n, k] of one format; workspace as cq_moe_gemm_workspace_bytes(..., has_topk_weights = 0).
- * CQ_ERR_ALIGN when such experts, of up to 64 pairs each, are not 16-byte aligned (a later cq_moe_gemm_gguf_down_after_pair tells from the shape
- * alone how this call grouped its pairs). */
+ * CQ_ERR_ALIGN when Q4_K or Q5_K experts are not 16-byte aligned (a later cq_moe_gemm_gguf_down_after_pair tells from the shape alone how this call
+ * grouped its pairs). */
 int cq_moe_gemm_gguf_pair(int w_dtype, const float *x_dev, const void *w_a_dev, const void *w_b_dev, const int32_t *sorted_token_ids_dev,
                           const int32_t *expert_ids_dev, float *out_a_dev, float *out_b_dev, int64_t num_experts, int64_t topk, int64_t size_m,
                           int64_t n, int64_t k, int is_prefill, void *workspace_dev, int64_t workspace_bytes, void *stream);
