@@ -1114,16 +1114,21 @@ int cq_matvec_batch_swiglu_launch(int w_dtype, const void *w, const float *gate,
 //   k 2560: 24 1.05 - 1.17, 1.16 - 1.39; 32 0.94 - 1.15, 1.07 - 1.32; 48 0.80 - 0.99, 0.92 - 1.16; 64 0.82 - 0.99, 0.91 - 1.13
 //   k 4096: 30 - 60 1.16 - 1.52, 1.24 - 1.84;      k 1280, n 4096: 0.53 - 0.71, 0.56 - 0.79;      k up to 1024: 0.72 and 0.83 on average
 // With the limits below they take 0.72 (Q4_K) and 0.82 of the time batched, 4 and 6 of 228 each more than 1.05 of it and 1.16 at most; at 27 throughout 0.89 and 0.98, 38 and 78, 1.84.
+// Else up to 24 and 25, and up to 27 where the experts' weights are so many that the tiles' rounds are full.  Time of a layer with gate and up in the tiles of one launch over batched, 25.2 - 27 pairs:
+//   of 64 Mi weights (gate) and fewer Q4_K 0.75 - 0.9, Q5_K 0.8 - 0.95; 128 experts of 1024 x 1024 0.99, 1.10; of 2048 x 512 0.97, 1.07; of 1536 x 1024 0.98, 1.06; of 2048 x 768 1.05, 1.11; of
+//   2048 x 1024 1.11, 1.15; 64 of 2048 x 1536 0.99, 1.07; of 4096 x 768 1.08, 1.15; 32 of 4096 x 1536 1.03, 1.13.
 // us of a layer, batched matvecs / tiles: 64 experts of 2048 x 1024, 6 each, 230 / 330 / 430 / 640 tokens Q4_K 109 112, 145 126, 178 136, 230 157, Q5_K 119 131, 157 144, 192 155, 249 174;
 // 128 of 2048 x 768, 8 each, 400 / 600 / 1000 Q4_K 168 174, 248 200, 336 237, Q5_K 184 203, 266 228, 362 264; 64 of 1024 x 512, 4 each, 400 / 900 Q4_K 70 54, 110 70, Q5_K 71 60, 113 78.
 static bool qme_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n, int64_t pairs_each) {
     return qb_weights(w_dtype) && k % 256 == 0 && k / 256 <= 2 * QB_NW && n >= 1 && n <= 0x7ffffff0 / 16 && num_experts >= 1 && num_experts <= 65535 &&
            n_pairs <= pairs_each * num_experts && n * (k / 256) * qb_bb(w_dtype == CQ_Q5K) < 0x7fffffffLL;
 }
+// (up to 27 pairs alike for [n, k] and [k, n], so that a layer's down projection follows its gate and up in their form)
 bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
-    const int64_t wgs = num_experts * ((n + 255) / 256);
-    const bool few = w_dtype == CQ_Q5K ? k >= 2048 && wgs <= std::min<int64_t>(64, k / 48) : k > 2048 && wgs <= std::min<int64_t>(64, k / 64);
-    return qme_shape(w_dtype, num_experts, n_pairs, k, n, few ? 64 : w_dtype == CQ_Q5K ? 25 : 24);
+    const bool q5 = w_dtype == CQ_Q5K;
+    auto few = [&](int64_t k, int64_t n) { return k >= (q5 ? 2048 : 2049) && num_experts * ((n + 255) / 256) <= std::min<int64_t>(64, k / (q5 ? 48 : 64)); };
+    const bool big = num_experts * n * k >= (q5 ? 128LL : 192LL) << 20 && (q5 || std::max(n, k) >= 2048);
+    return qme_shape(w_dtype, num_experts, n_pairs, k, n, few(k, n) ? 64 : few(n, k) || big ? 27 : q5 ? 25 : 24);
 }
 bool cq_moe_stream_takes(int w_dtype, const void *w, const void *w_b, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
     return cq_moe_stream_shape(w_dtype, num_experts, n_pairs, k, n) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)w_b & 15) == 0;

@@ -176,7 +176,7 @@ int cq_qmatmul_forward_static(int w_dtype, const void *w_dev, const void *x_dev,
  *   out[b, t, :] = W[ids[b, t]] . x[b, input_dim1 == 1 ? 0 : t, :].
  * Up to 256 pairs (512 for short rows, see cq_moe_direct_pairs) each pair is its own fused matvec; beyond, pairs are grouped by expert on the device and an expert's
  * rows are streamed once per 32 of its pairs as a batched matvec (Q4K / Q5K experts with rows of up to 4096 elements that see at
- * most 24 / 25 pairs each on average, few of long rows 64: see cq_moe_gemm_gguf_pair), once per tile of 32 or 128 pairs on the matrix cores (K-quant experts; integer-exact) or once per
+ * most 24 to 27 pairs each on average, few of long rows 64: see cq_moe_gemm_gguf_pair), once per tile of 32 or 128 pairs on the matrix cores (K-quant experts; integer-exact) or once per
  * 8 pairs by the matvec kernel (the other formats).  The reference takes Q2K-Q6K and Q8_0 experts (cuda.rs:543-548).
  * An id >= num_experts leaves its output row zero-filled.
  * ------------------------------------------------------------------------------------------- */
@@ -205,7 +205,7 @@ int cq_moe_gemm_gguf(int w_dtype, const float *x_dev, const void *w_dev, const i
 /* Two moe_gemm_gguf calls without topk_weights over the same x and the same pairs — the gate and up matmuls of
  * FusedMoeGGUF::forward (candle-transformers/src/fused_moe.rs:263-276) — as one call: out_a = x W_a^T, out_b = x W_b^T per
  * pair, results identical to two cq_moe_gemm_gguf calls.  With more than 256 pairs on K-quant experts the pairs are
- * grouped by expert and the activations quantized once for both (Q4_K / Q5_K experts that see at most 24 / 25 pairs each on average, or 64 where k is
+ * grouped by expert and the activations quantized once for both (Q4_K / Q5_K experts that see at most 24 / 25 pairs each on average, 27 of many weights or few long rows or columns, or 64 where k is
  * above / at least 2048 and num_experts * ceil(n / 256) at most 64 and k / 64 or k / 48, rows up to 4096 elements: both tensors in one launch, every expert a batched matvec over its own pairs);
  * otherwise it is the two calls.  w_a / w_b [num_experts, n, k] of one format; workspace as cq_moe_gemm_workspace_bytes(..., has_topk_weights = 0).
  * CQ_ERR_ALIGN when Q4_K or Q5_K experts are not 16-byte aligned (a later cq_moe_gemm_gguf_down_after_pair tells from the shape alone how this call

@@ -357,9 +357,9 @@ def test_fused_moe_argument_errors():
     assert lib.cq_nn_moe_sum(256, 256, 1, 2, 6, None) == -2
 
 
-@pytest.mark.parametrize("tokens", [380, 400])
+@pytest.mark.parametrize("tokens", [425, 440])
 def test_fused_moe_layer_qwen3_shape_on_either_side_of_the_batched_form(tokens):
-    """3040 pairs, 23.75 an expert, as batched matvecs with a second pass over the weights of some; 3200 in tiles, gate and up in one launch."""
+    """3400 pairs, 26.6 an expert, as batched matvecs with a second pass over the weights of some; 3520 in tiles, gate and up in one launch."""
     test_fused_moe_layer_qwen3_shape_token_batches(tokens, True)
 
 
