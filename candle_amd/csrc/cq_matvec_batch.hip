@@ -1123,7 +1123,8 @@ static bool qme_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t
     return qb_weights(w_dtype) && k % 256 == 0 && k / 256 <= 2 * QB_NW && n >= 1 && n <= 0x7ffffff0 / 16 && num_experts >= 1 && num_experts <= 65535 &&
            n_pairs <= pairs_each * num_experts && n * (k / 256) * qb_bb(w_dtype == CQ_Q5K) < 0x7fffffffLL;
 }
-// (up to 27 pairs alike for [n, k] and [k, n], so that a layer's down projection follows its gate and up in their form)
+// (Up to 27 pairs alike for [n, k] and [k, n], so that a layer's down projection follows its gate and up in their form.  Beyond, the limit of [k, n] with n <= k, a down projection that fits
+// into the gate / up call's workspace, is never the higher one: behind tiles a call of its own would be tiles too, and has the same bits.)
 bool cq_moe_stream_shape(int w_dtype, int64_t num_experts, int64_t n_pairs, int64_t k, int64_t n) {
     const bool q5 = w_dtype == CQ_Q5K;
     auto few = [&](int64_t k, int64_t n) { return k >= (q5 ? 2048 : 2049) && num_experts * ((n + 255) / 256) <= std::min<int64_t>(64, k / (q5 ? 48 : 64)); };

@@ -230,7 +230,7 @@ int cq_moe_gemm_gguf_swiglu(int w_dtype, const float *x_dev, const void *w_gate_
  * call left in the workspace is used again (no second grouping pass), and silu(gate) * up is evaluated inside the activation
  * quantizer (the f32 product is never written).  out[p, :] = topk_weights[p] * W_down[e_p] . quantize(silu(gate[p]) * up[p]) for
  * pair p; gate / up: [size_m, k] f32 as the pair call wrote them (k = its n), k_pair = the pair call's k.  Bit-identical to
- * cq_nn_silu_mul + cq_moe_gemm_gguf.  CQ_ERR_RANGE (nothing enqueued) when the pair call did not bucket its pairs for the
+ * cq_nn_silu_mul + cq_moe_gemm_gguf, but to rounding where k_pair > 4096 >= k and that would run batched matvecs.  CQ_ERR_RANGE (nothing enqueued) when the pair call did not bucket its pairs for the
  * matrix-core kernels or this call's quantized rows do not fit in front of that call's tables: the caller then takes the two
  * separate calls.  Nothing else may use the workspace between the two calls.  No counterpart in the reference, which sorts the
  * pairs once on the host side (fused_moe.rs:249-260) and passes the sorted list to all three calls. */
@@ -245,7 +245,8 @@ int cq_moe_gemm_gguf_down_after_pair(int w_dtype, const float *gate_dev, const f
 int cq_moe_gemm_gguf_pair_swiglu(int w_dtype, const float *x_dev, const void *w_gate_dev, const void *w_up_dev, const int32_t *sorted_token_ids_dev,
                                  const int32_t *expert_ids_dev, float *out_dev, int64_t num_experts, int64_t topk, int64_t size_m, int64_t n, int64_t k,
                                  void *workspace_dev, int64_t workspace_bytes, void *stream);
-/* cq_moe_gemm_gguf_down_after_pair behind that call, on its workspace and its out [size_m, k]: out[p, :] = topk_weights[p] * W_down[e_p] . quantize(x[p]). */
+/* cq_moe_gemm_gguf_down_after_pair behind that call, on its workspace and its out [size_m, k]: out[p, :] = topk_weights[p] * W_down[e_p] . quantize(x[p]),
+ * in tiles, also where a cq_moe_gemm_gguf call of its own would run batched matvecs. */
 int cq_moe_gemm_gguf_down_after_swiglu(int w_dtype, const float *x_dev, const void *w_down_dev, const float *topk_weights_dev, float *out_dev, int64_t num_experts,
                                        int64_t topk, int64_t size_m, int64_t n, int64_t k, int64_t k_pair, void *workspace_dev, int64_t workspace_bytes,
                                        void *stream);
