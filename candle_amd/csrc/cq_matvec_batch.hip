@@ -1113,7 +1113,7 @@ int cq_matvec_batch_swiglu_launch(int w_dtype, const void *w, const float *gate,
 //   k 2048: 12 - 16 workgroups Q4_K 0.86 - 1.08, Q5_K 1.07 - 1.38; 24 - 32 0.74 - 1.08, 0.87 - 1.38; 48 0.69 - 0.95, 0.82 - 1.14; 64 0.66 - 0.88, 0.76 - 1.08
 //   k 2560: 24 1.05 - 1.17, 1.16 - 1.39; 32 0.94 - 1.15, 1.07 - 1.32; 48 0.80 - 0.99, 0.92 - 1.16; 64 0.82 - 0.99, 0.91 - 1.13
 //   k 4096: 30 - 60 1.16 - 1.52, 1.24 - 1.84;      k 1280, n 4096: 0.53 - 0.71, 0.56 - 0.79;      k up to 1024: 0.72 and 0.83 on average
-// With the limits below they take 0.72 (Q4_K) and 0.82 of the time batched, 4 and 6 of 228 each more than 1.05 of it and 1.16 at most; at 27 throughout 0.89 and 0.98, 38 and 78, 1.84.
+// With the limits below they take 0.73 (Q4_K) and 0.83 of the time batched, 4 and 5 of 228 each more than 1.05 of it and 1.16 at most; at 27 throughout 0.89 and 0.98, 38 and 78, 1.84.
 // Else up to 24 and 25, and up to 27 where the experts' weights are so many that the tiles' rounds are full.  Time of a layer with gate and up in the tiles of one launch over batched, 25.2 - 27 pairs:
 //   of 64 Mi weights (gate) and fewer Q4_K 0.75 - 0.9, Q5_K 0.8 - 0.95; 128 experts of 1024 x 1024 0.99, 1.10; of 2048 x 512 0.97, 1.07; of 1536 x 1024 0.98, 1.06; of 2048 x 768 1.05, 1.11; of
 //   2048 x 1024 1.11, 1.15; 64 of 2048 x 1536 0.99, 1.07; of 4096 x 768 1.08, 1.15; 32 of 4096 x 1536 1.03, 1.13.
